@@ -200,6 +200,18 @@ def load() -> C.CDLL:
     return lib
 
 
+def load_native():
+    """The native half of the torch binding (``csrc/torch_binding.cpp``), bound to the library ``load`` opened."""
+    lib = load()
+    try:
+        from . import _oxq_torch
+    except ImportError as e:
+        raise ImportError(f"oxydllm_amd/_oxq_torch is missing or does not load ({e}): build it with "
+                          "`python -m oxydllm_amd.build`") from e
+    _oxq_torch.bind(lib._handle, OxqError, OxqTensor)
+    return _oxq_torch
+
+
 def check(rc: int):
     if rc != 0:
         msg = load().oxq_last_error()

@@ -1,13 +1,15 @@
-"""Compiles the HIP sources into ``oxydllm_amd/liboxq_hip.so`` for gfx950.
+"""Compiles the HIP sources into ``oxydllm_amd/liboxq_hip.so`` for gfx950, and the torch binding's native
+half into ``oxydllm_amd/_oxq_torch.so`` (host code, linked against torch and not against the library).
 
-hipcc cross-compiles without a GPU.  The library is built in-tree so it
-travels with the source snapshot; nothing is JIT-compiled at import time.
+hipcc cross-compiles without a GPU.  Both are built in-tree so they
+travel with the source snapshot; nothing is JIT-compiled at import time.
 """
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -25,6 +27,27 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-x", "hip",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument", "-Wno-unknown-attributes",
          f"-I{INCLUDE}", f"-I{CSRC}"]
+
+
+TORCH_SOURCE = "torch_binding.cpp"
+TORCH_LIB = os.path.join(HERE, "_oxq_torch.so")
+
+
+def _build_torch_binding(force: bool) -> None:
+    src = os.path.join(CSRC, TORCH_SOURCE)
+    newest = max(os.path.getmtime(p) for p in (src, os.path.join(INCLUDE, "oxq.h")))
+    if not force and os.path.exists(TORCH_LIB) and os.path.getmtime(TORCH_LIB) >= newest:
+        return
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", "-I/opt/rocm/include",
+           f"-I{sysconfig.get_paths()['include']}", src, "-o", TORCH_LIB, f"-L{root}/lib", "-ltorch_python", "-ltorch_hip",
+           "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10", "-ldl"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for {TORCH_SOURCE}:\n{res.stderr}")
 
 
 def _deps():
@@ -51,7 +74,9 @@ def _compile(src: str, force: bool) -> str:
 def build(force: bool = False, jobs: int = 6) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        binding = ex.submit(_build_torch_binding, force)
         objs = list(ex.map(lambda s: _compile(s, force), SOURCES))
+        binding.result()
     newest = max(os.path.getmtime(o) for o in objs)
     if force or not os.path.exists(LIB) or os.path.getmtime(LIB) < newest:
         cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs

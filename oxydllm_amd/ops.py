@@ -3,9 +3,12 @@
 ``src/common/mxfp4.rs``).
 
 torch is plumbing only: it owns device memory and the current stream.  All
-validation, routing and compute happen behind the C ABI; this module builds
-descriptors, allocates the output the reference op would have allocated, and
-raises :class:`OxqError` with the library's message on failure.
+validation, routing and compute happen behind the C ABI.  What an engine calls
+on every step (the products, the layers' forward, the expert layer's glue) goes
+through the native module ``_oxq_torch``, which builds the descriptors, allocates
+the output the reference op would have allocated, and raises :class:`OxqError`
+with the library's message on failure; the load-time calls do the same here
+through ctypes.
 """
 from __future__ import annotations
 
@@ -18,6 +21,8 @@ from . import _lib
 from ._lib import (BF16, F16, F32, GGUF_Q2_K, GGUF_Q3_K, GGUF_Q4_0, GGUF_Q4_1, GGUF_Q4_K, GGUF_Q5_0,
                    GGUF_Q5_1, GGUF_Q5_K, GGUF_Q6_K, GGUF_Q8_0, I32, I64, PACK_IN, PACK_OUT, U8, U32,
                    OxqError, OxqPlan, OxqTensor)
+
+_native = _lib.load_native()
 
 _DTYPES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16, torch.uint8: U8,
            torch.int32: I32, torch.int64: I64}
@@ -67,9 +72,11 @@ class Context:
         _lib.check(self._lib.oxq_ctx_create(dev, C.byref(self.handle)))
         self.device = dev
         self.plan_only = plan_only
+        self.native = _native.Handle(self.handle.value, _native.KIND_PLAIN, 0, plan_only)
 
     def close(self):
         if self.handle:
+            self.native = _native.Handle(0, _native.KIND_PLAIN, 0, self.plan_only)
             self._lib.oxq_ctx_destroy(self.handle)
             self.handle = C.c_void_p()
 
@@ -119,6 +126,10 @@ _default_ctx: dict = {}
 
 
 def default_context() -> Context:
+    if _default_ctx:
+        ctx = _default_ctx.get(_native.current_device())
+        if ctx is not None:
+            return ctx
     dev = torch.cuda.current_device()
     if dev not in _default_ctx:
         _default_ctx[dev] = Context(dev)
@@ -129,9 +140,7 @@ def _ctx(ctx: Optional[Context]) -> Context:
     return ctx if ctx is not None else default_context()
 
 
-def _out_for(x: torch.Tensor, n: int, out, ctx):
-    if out is not None:
-        return out
+def _out_for(x: torch.Tensor, n: int):
     return torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
 
 
@@ -177,11 +186,7 @@ def grid_barrier(workgroups: int, threads: int, state, spin_limit: int = 1 << 18
 
 def w4a16_matmul(x, qweight, qzeros, scales, *, out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:1821.  x [m,K] (m in 1..=8) -> [m,N] in x's dtype."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, scales.shape[1], out, ctx)
-    _lib.check(ctx._lib.oxq_w4a16_matmul(ctx.handle, ctx.stream(), desc(x), desc(qweight),
-                                         desc(qzeros), desc(scales), desc(out)))
-    return out
+    return _native.w4a16_matmul(_ctx(ctx).native, x, out, scales.shape[1], qweight, qzeros, scales)
 
 
 def w4a16_matmul_static(x, qweight, qzeros, scales, *, out, ctx: Optional[Context] = None):
@@ -196,20 +201,12 @@ def w4a16_matmul_static(x, qweight, qzeros, scales, *, out, ctx: Optional[Contex
 
 def w8a16_matmul(x, qweight, qzeros, scales, *, out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:1835."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, scales.shape[1], out, ctx)
-    _lib.check(ctx._lib.oxq_w8a16_matmul(ctx.handle, ctx.stream(), desc(x), desc(qweight),
-                                         desc(qzeros), desc(scales), desc(out)))
-    return out
+    return _native.w8a16_matmul(_ctx(ctx).native, x, out, scales.shape[1], qweight, qzeros, scales)
 
 
 def gptq_matmul(x, qweight, qzeros, scales, bits: int, *, out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:2281."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, scales.shape[1], out, ctx)
-    _lib.check(ctx._lib.oxq_gptq_matmul(ctx.handle, ctx.stream(), desc(x), desc(qweight),
-                                        desc(qzeros), desc(scales), bits, desc(out)))
-    return out
+    return _native.gptq_matmul(_ctx(ctx).native, x, out, scales.shape[1], qweight, qzeros, scales, bits)
 
 
 def _dequant_out(qweight, scales, bits, pack_dim, out):
@@ -251,18 +248,14 @@ def dequantize_gptq_packed(qweight, qzeros, scales, bits: int, *, out=None,
 def mpp_quant_matmul(x, qweight, qzeros, scales, bits: int, pack_dim: int, *, out=None,
                      ctx: Optional[Context] = None):
     """metal_ops.rs:2748: tile GEMM on the matrix cores, any m."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, scales.shape[1], out, ctx)
-    _lib.check(ctx._lib.oxq_mpp_quant_matmul(ctx.handle, ctx.stream(), desc(x), desc(qweight),
-                                             desc(qzeros), desc(scales), bits, pack_dim, desc(out)))
-    return out
+    return _native.mpp_quant_matmul(_ctx(ctx).native, x, out, scales.shape[1], qweight, qzeros, scales, bits, pack_dim)
 
 
 def maybe_mpp_quant_matmul(x, qweight, qzeros, scales, bits: int, pack_dim: int, *,
                            ctx: Optional[Context] = None):
     """metal_ops.rs:2771: returns None when the op declines (small m, wrong dtype...)."""
     ctx = _ctx(ctx)
-    out = _out_for(x, scales.shape[1], None, ctx)
+    out = _out_for(x, scales.shape[1])
     taken = C.c_int(0)
     _lib.check(ctx._lib.oxq_maybe_mpp_quant_matmul(ctx.handle, ctx.stream(), desc(x), desc(qweight),
                                                    desc(qzeros), desc(scales), bits, pack_dim,
@@ -346,18 +339,12 @@ def f8_block_dequant_bf16(bytes_, scales, *, ctx: Optional[Context] = None):
 
 def f8_gemv(x, bytes_, scales, *, out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:5788: x BF16 [m <= 8, in] times the block-scaled F8 weight [out, in]."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, bytes_.shape[0], out, ctx)
-    _lib.check(ctx._lib.oxq_f8_gemv(ctx.handle, ctx.stream(), desc(x), desc(bytes_), desc(scales), desc(out)))
-    return out
+    return _native.f8_gemv(_ctx(ctx).native, x, out, bytes_.shape[0], bytes_, scales)
 
 
 def f8_matmul(x, bytes_, scales, *, out=None, ctx: Optional[Context] = None):
     """moe.rs:106-113 (Fp8Cached::forward): any m."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, bytes_.shape[0], out, ctx)
-    _lib.check(ctx._lib.oxq_f8_matmul(ctx.handle, ctx.stream(), desc(x), desc(bytes_), desc(scales), desc(out)))
-    return out
+    return _native.f8_matmul(_ctx(ctx).native, x, out, bytes_.shape[0], bytes_, scales)
 
 
 # ---------------------------------------------------------------- GGUF
@@ -370,21 +357,13 @@ def gguf_block_layout(quant: int):
 def gguf_quant_matmul(x, weight_bytes, in_features: int, out_features: int, quant: int, *,
                       out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:5819 (1 <= m <= 8)."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, out_features, out, ctx)
-    _lib.check(ctx._lib.oxq_gguf_quant_matmul(ctx.handle, ctx.stream(), desc(x), desc(weight_bytes),
-                                              in_features, out_features, quant, desc(out)))
-    return out
+    return _native.gguf_quant_matmul(_ctx(ctx).native, x, out, out_features, weight_bytes, in_features, quant)
 
 
 def gguf_quant_mul_mm(x, weight_bytes, in_features: int, out_features: int, quant: int, *,
                       out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:5973 (any m)."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, out_features, out, ctx)
-    _lib.check(ctx._lib.oxq_gguf_quant_mul_mm(ctx.handle, ctx.stream(), desc(x), desc(weight_bytes),
-                                              in_features, out_features, quant, desc(out)))
-    return out
+    return _native.gguf_quant_mul_mm(_ctx(ctx).native, x, out, out_features, weight_bytes, in_features, quant)
 
 
 def gguf_dequantize(weight_bytes, in_features: int, out_features: int, quant: int, *,
@@ -399,11 +378,7 @@ def gguf_dequantize(weight_bytes, in_features: int, out_features: int, quant: in
 # ---------------------------------------------------------------- MXFP4
 def mxfp4_matmul(x, blocks, scales, k: int, n: int, *, out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:6197."""
-    ctx = _ctx(ctx)
-    out = _out_for(x, n, out, ctx)
-    _lib.check(ctx._lib.oxq_mxfp4_matmul(ctx.handle, ctx.stream(), desc(x), desc(blocks),
-                                         desc(scales), k, n, desc(out)))
-    return out
+    return _native.mxfp4_matmul(_ctx(ctx).native, x, out, n, blocks, scales, k)
 
 
 def mxfp4_dequantize(blocks, scales, k: int, n: int, *, ctx: Optional[Context] = None):
@@ -417,15 +392,7 @@ def mxfp4_dequantize(blocks, scales, k: int, n: int, *, ctx: Optional[Context] =
 def mxfp4_moe_matmul(x, blocks, scales, bias, expert_offsets, token_ids, k: int, n: int, *,
                      out=None, ctx: Optional[Context] = None):
     """Grouped expert GEMV: out[p] = x[row(p)] . W_e^T + bias_e for every routed pair."""
-    ctx = _ctx(ctx)
-    gather = token_ids is not None
-    n_pairs = token_ids.numel() if gather else x.shape[0]
-    if out is None:
-        out = torch.empty((n_pairs, n), dtype=x.dtype, device=x.device)
-    _lib.check(ctx._lib.oxq_mxfp4_moe_matmul(ctx.handle, ctx.stream(), desc(x), desc(blocks),
-                                             desc(scales), desc(bias), desc(expert_offsets),
-                                             desc(token_ids), 1 if gather else 0, k, n, desc(out)))
-    return out
+    return _native.moe_matmul(_ctx(ctx).native, x, out, blocks, scales, bias, expert_offsets, token_ids, k, n)
 
 
 # ---------------------------------------------------------------- mixture-of-experts glue
@@ -437,15 +404,8 @@ def mxfp4_moe_gate_up_swiglu(x, blocks, scales, bias, expert_offsets, token_ids,
     """gate_up projection of the routed pairs + GPT-OSS SwiGLU (moe.rs:152-173) -> [n_pairs, n / 2].  One
     launch where the decode kernel runs; otherwise the two calls it stands for (same bits either way)."""
     ctx = _ctx(ctx)
-    gather = token_ids is not None
-    n_pairs = token_ids.numel() if gather else x.shape[0]
-    if out is None:
-        out = torch.empty((n_pairs, n // 2), dtype=x.dtype, device=x.device)
-    fused = C.c_int()
-    _lib.check(ctx._lib.oxq_mxfp4_moe_gate_up_swiglu(ctx.handle, ctx.stream(), desc(x), desc(blocks), desc(scales),
-                                                     desc(bias), desc(expert_offsets), desc(token_ids),
-                                                     1 if gather else 0, k, n, float(limit), desc(out), C.byref(fused)))
-    if not fused.value:
+    out, fused = _native.moe_gate_up_swiglu(ctx.native, x, out, blocks, scales, bias, expert_offsets, token_ids, k, n, limit)
+    if not fused:
         gu = mxfp4_moe_matmul(x, blocks, scales, bias, expert_offsets, token_ids, k, n, ctx=ctx)
         gated_activation(gu, ACT_GPT_OSS_SWIGLU, limit, out=out, ctx=ctx)
     return out
@@ -463,6 +423,7 @@ class Mxfp4Experts:
         self.handle = C.c_void_p()
         _lib.check(self.ctx._lib.oxq_mxfp4_experts_new(self.ctx.handle, desc(blocks), desc(scales), desc(bias),
                                                        n_experts, k, n, C.byref(self.handle)))
+        self._native = _native.Handle(self.handle.value, _native.KIND_PLAIN, n, self.ctx.plan_only)
 
     @property
     def resident(self) -> bool:
@@ -471,25 +432,11 @@ class Mxfp4Experts:
         return bool(r.value)
 
     def matmul(self, x, expert_offsets, token_ids, *, out=None):
-        gather = token_ids is not None
-        n_pairs = token_ids.numel() if gather else x.shape[0]
-        if out is None:
-            out = torch.empty((n_pairs, self.n), dtype=x.dtype, device=x.device)
-        _lib.check(self.ctx._lib.oxq_mxfp4_experts_matmul(self.handle, self.ctx.stream(), desc(x), desc(expert_offsets),
-                                                          desc(token_ids), 1 if gather else 0, desc(out)))
-        return out
+        return _native.experts_matmul(self._native, x, out, expert_offsets, token_ids)
 
     def gate_up_swiglu(self, x, expert_offsets, token_ids, limit: float, *, out=None):
-        gather = token_ids is not None
-        n_pairs = token_ids.numel() if gather else x.shape[0]
-        if out is None:
-            out = torch.empty((n_pairs, self.n // 2), dtype=x.dtype, device=x.device)
-        fused = C.c_int()
-        _lib.check(self.ctx._lib.oxq_mxfp4_experts_gate_up_swiglu(self.handle, self.ctx.stream(), desc(x),
-                                                                  desc(expert_offsets), desc(token_ids),
-                                                                  1 if gather else 0, float(limit), desc(out),
-                                                                  C.byref(fused)))
-        if not fused.value:
+        out, fused = _native.experts_gate_up_swiglu(self._native, x, out, expert_offsets, token_ids, limit)
+        if not fused:
             gu = self.matmul(x, expert_offsets, token_ids)
             gated_activation(gu, ACT_GPT_OSS_SWIGLU, limit, out=out, ctx=self.ctx)
         return out
@@ -501,6 +448,7 @@ class Mxfp4Experts:
 
     def close(self):
         if self.handle:
+            self._native = _native.Handle(0, _native.KIND_PLAIN, self.n, self.ctx.plan_only)
             self.ctx._lib.oxq_mxfp4_experts_free(self.handle)
             self.handle = C.c_void_p()
 
@@ -513,65 +461,28 @@ class Mxfp4Experts:
 
 def moe_route(logits, top_k: int, norm_topk: bool = True, *, ctx: Optional[Context] = None):
     """moe.rs:466-486: softmax, stable descending top-k, optional renormalisation."""
-    ctx = _ctx(ctx)
-    T = logits.shape[0]
-    idx = torch.empty((T, top_k), dtype=torch.int32, device=logits.device)
-    vals = torch.empty((T, top_k), dtype=torch.float32, device=logits.device)
-    _lib.check(ctx._lib.oxq_moe_route(ctx.handle, ctx.stream(), desc(logits), top_k, 1 if norm_topk else 0,
-                                      desc(idx), desc(vals)))
-    return idx, vals
+    return _native.moe_route(_ctx(ctx).native, logits, top_k, 1 if norm_topk else 0)
 
 
 def moe_group(top_idx, top_vals, n_experts: int, *, ctx: Optional[Context] = None):
     """moe.rs:563-590: (expert_offsets [E+1], token_ids [P], pair_weights [P], pair_pos [T,k])."""
-    ctx = _ctx(ctx)
-    T, k = top_idx.shape
-    dev = top_idx.device
-    offsets = torch.empty((n_experts + 1,), dtype=torch.int32, device=dev)
-    tokens = torch.empty((T * k,), dtype=torch.int32, device=dev)
-    weights = torch.empty((T * k,), dtype=torch.float32, device=dev)
-    pos = torch.empty((T, k), dtype=torch.int32, device=dev)
-    _lib.check(ctx._lib.oxq_moe_group(ctx.handle, ctx.stream(), desc(top_idx), desc(top_vals), n_experts,
-                                      desc(offsets), desc(tokens), desc(weights), desc(pos)))
-    return offsets, tokens, weights, pos
+    return _native.moe_group(_ctx(ctx).native, top_idx, top_vals, n_experts)
 
 
 def moe_route_group(logits, top_k: int, norm_topk: bool = True, *, ctx: Optional[Context] = None):
     """moe_route + moe_group in one call (one launch for decode sizes): returns (top_idx, top_vals,
     expert_offsets, token_ids, pair_weights, pair_pos)."""
-    ctx = _ctx(ctx)
-    T, E = logits.shape
-    dev = logits.device
-    idx = torch.empty((T, top_k), dtype=torch.int32, device=dev)
-    vals = torch.empty((T, top_k), dtype=torch.float32, device=dev)
-    offsets = torch.empty((E + 1,), dtype=torch.int32, device=dev)
-    tokens = torch.empty((T * top_k,), dtype=torch.int32, device=dev)
-    weights = torch.empty((T * top_k,), dtype=torch.float32, device=dev)
-    pos = torch.empty((T, top_k), dtype=torch.int32, device=dev)
-    _lib.check(ctx._lib.oxq_moe_route_group(ctx.handle, ctx.stream(), desc(logits), top_k, 1 if norm_topk else 0,
-                                            desc(idx), desc(vals), desc(offsets), desc(tokens), desc(weights),
-                                            desc(pos)))
-    return idx, vals, offsets, tokens, weights, pos
+    return _native.moe_route_group(_ctx(ctx).native, logits, top_k, 1 if norm_topk else 0)
 
 
 def gated_activation(gate_up, kind: int, limit: float = 0.0, *, out=None, ctx: Optional[Context] = None):
     """ffn_kernels.metal gated SiLU / GeLU-tanh over [.., gate | up]; moe.rs:152-173 GPT-OSS SwiGLU."""
-    ctx = _ctx(ctx)
-    if out is None:
-        out = torch.empty(tuple(gate_up.shape[:-1]) + (gate_up.shape[-1] // 2,), dtype=gate_up.dtype,
-                          device=gate_up.device)
-    _lib.check(ctx._lib.oxq_gated_activation(ctx.handle, ctx.stream(), desc(gate_up), kind, float(limit),
-                                             desc(out)))
-    return out
+    return _native.gated_activation(_ctx(ctx).native, gate_up, out, kind, limit)
 
 
 def activation_mul(gate, up, kind: int, *, out=None, ctx: Optional[Context] = None):
     """metal_ops.rs:1252 silu_mul_fused / :1271 gelu_tanh_mul_fused: act(gate) * up over two tensors."""
-    ctx = _ctx(ctx)
-    if out is None:
-        out = torch.empty_like(gate)
-    _lib.check(ctx._lib.oxq_activation_mul(ctx.handle, ctx.stream(), desc(gate), desc(up), kind, desc(out)))
-    return out
+    return _native.activation_mul(_ctx(ctx).native, gate, up, out, kind)
 
 
 def silu_mul(gate, up, *, out=None, ctx: Optional[Context] = None):
@@ -584,13 +495,7 @@ def gelu_tanh_mul(gate, up, *, out=None, ctx: Optional[Context] = None):
 
 def moe_combine(expert_out, pair_pos, top_vals, *, out=None, ctx: Optional[Context] = None):
     """moe.rs:592-605: out[t] = sum_s top_vals[t, s] * expert_out[pair_pos[t, s]]."""
-    ctx = _ctx(ctx)
-    if out is None:
-        out = torch.empty((pair_pos.shape[0], expert_out.shape[1]), dtype=expert_out.dtype,
-                          device=expert_out.device)
-    _lib.check(ctx._lib.oxq_moe_combine(ctx.handle, ctx.stream(), desc(expert_out), desc(pair_pos),
-                                        desc(top_vals), desc(out)))
-    return out
+    return _native.moe_combine(_ctx(ctx).native, expert_out, pair_pos, top_vals, out)
 
 
 # ---------------------------------------------------------------- layers
@@ -621,16 +526,12 @@ class PackedQuantLinear:
         flag = C.c_int()
         self.ctx._lib.oxq_packed_quant_linear_is_prepacked(self.handle, C.byref(flag))
         self.prepacked = bool(flag.value)
+        self._forward = _native.Handle(self.handle.value, _LINEAR_KINDS[PackedQuantLinear], self.out_features, self.ctx.plan_only)
         if self.prepacked:          # the layer owns a tile-major copy; bias is still referenced
             self._keep = (bias,)
 
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
-        if out is None:
-            out = torch.empty(tuple(x.shape[:-1]) + (self.out_features,), dtype=x.dtype,
-                              device=x.device)
-        _lib.check(self.ctx._lib.oxq_packed_quant_linear_forward(self.handle, self.ctx.stream(),
-                                                                 desc(x), desc(out)))
-        return out
+        return self._forward(x, out)
 
     def dequantize(self, out=None) -> torch.Tensor:
         """Dense [in, out] weights in the layer dtype (linear.rs:510-523)."""
@@ -672,14 +573,10 @@ class QLinear:
             _lib.check(self.ctx._lib.oxq_qlinear_new_gate_up(
                 self.ctx.handle, quant, desc(weight_bytes), in_features, out_features, desc(bias), gate_up_act,
                 _DTYPES[out_dtype], C.byref(self.handle)))
+        self._forward = _native.Handle(self.handle.value, _LINEAR_KINDS[QLinear], self.out_features, self.ctx.plan_only)
 
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
-        if out is None:
-            out = torch.empty(tuple(x.shape[:-1]) + (self.out_features,), dtype=x.dtype,
-                              device=x.device)
-        _lib.check(self.ctx._lib.oxq_qlinear_forward(self.handle, self.ctx.stream(), desc(x),
-                                                     desc(out)))
-        return out
+        return self._forward(x, out)
 
     @property
     def resident(self) -> bool:
@@ -716,14 +613,10 @@ class Mxfp4Linear:
         _lib.check(self.ctx._lib.oxq_mxfp4_linear_new(
             self.ctx.handle, desc(blocks), desc(scales), desc(bias), in_features, out_features,
             C.byref(self.handle)))
+        self._forward = _native.Handle(self.handle.value, _LINEAR_KINDS[Mxfp4Linear], out_features, self.ctx.plan_only)
 
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
-        if out is None:
-            out = torch.empty(tuple(x.shape[:-1]) + (self.out_features,), dtype=x.dtype,
-                              device=x.device)
-        _lib.check(self.ctx._lib.oxq_mxfp4_linear_forward(self.handle, self.ctx.stream(), desc(x),
-                                                          desc(out)))
-        return out
+        return self._forward(x, out)
 
     def __del__(self):
         try:
@@ -765,6 +658,7 @@ class FeedForward:
         self.ctx._lib.oxq_mlp_in_features(self.handle, C.byref(k))
         self.ctx._lib.oxq_mlp_out_features(self.handle, C.byref(n))
         self.in_features, self.out_features = k.value, n.value
+        self._forward = _native.Handle(self.handle.value, _native.KIND_MLP, self.out_features, self.ctx.plan_only)
         self.gate_up_kind, self.intermediate_size, self.activation = gate_up_kind, intermediate_size, activation
 
     def scratch_elems(self, rows: int) -> int:
@@ -773,13 +667,7 @@ class FeedForward:
         return e.value
 
     def forward(self, x: torch.Tensor, out=None, scratch=None) -> torch.Tensor:
-        rows = x.numel() // max(x.shape[-1], 1)
-        if scratch is None:
-            scratch = torch.empty(max(self.scratch_elems(rows), 1), dtype=x.dtype, device=x.device)
-        if out is None:
-            out = torch.empty(tuple(x.shape[:-1]) + (self.out_features,), dtype=x.dtype, device=x.device)
-        _lib.check(self.ctx._lib.oxq_mlp_forward(self.handle, self.ctx.stream(), desc(x), desc(scratch), desc(out)))
-        return out
+        return self._forward(x, out, scratch)
 
     def __del__(self):
         try:
