@@ -429,10 +429,11 @@ int oxq_moe_combine(oxq_ctx *ctx, void *stream, const oxq_tensor *expert_out, co
  * in the runtime dtype (`dtype`), as after the cast at linear.rs:437.
  *
  * Like the reference's constructor, `new` is the load-time step: for layers
- * with in_features and group size multiples of 128, out_features a multiple
- * of 64 and at most 128 groups it builds a tile-major copy of qweight/qzeros/scales in device memory owned by
+ * with out_features a multiple of 8 and in_features and group size multiples of 32 (in_features and group size
+ * multiples of 128 and out_features a multiple of 64, or at least 2^18 weights)
+ * it builds a tile-major copy of qweight/qzeros/scales in device memory owned by
  * the layer (same size as the checkpoint tensors, plus 1.5 bytes per column
- * and 128 rows; strips of 64 output columns, or of 16 for 4-bit layers of at
+ * and group, filled up to whole blocks of 128 rows x 64 columns; strips of 64 output columns, or of 16 for 4-bit layers of at
  * most 8192 columns and 4096 - 14336 rows, such as attention and down projections) and forward never reads the caller's tensors again; it
  * synchronises the null stream once.  Other layers keep descriptors of the
  * caller-owned tensors.  OXQ_PREPACK=0 in the environment disables the copy. */

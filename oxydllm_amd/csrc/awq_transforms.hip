@@ -87,6 +87,17 @@ __global__ __launch_bounds__(256) void copy2d_u32_kernel(const uint32_t *__restr
     dst[(size_t)r * dst_pitch + dst_col + c] = src[i];
 }
 
+// n 16-bit elements between addresses of any (element) alignment
+__global__ __launch_bounds__(256) void copy_u16_kernel(const uint16_t *__restrict__ src, uint16_t *__restrict__ dst, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) dst[i] = src[i];
+}
+int launch_copy_u16(hipStream_t s, const void *src, void *dst, int64_t n) {
+    const int64_t blocks = std::min<int64_t>(ceil_div(n, 256), 4096);
+    hipLaunchKernelGGL(copy_u16_kernel, dim3((unsigned)std::max<int64_t>(blocks, 1)), dim3(256), 0, s, (const uint16_t *)src, (uint16_t *)dst, n);
+    OXQ_HIP_CHECK(hipGetLastError());
+    return OXQ_OK;
+}
+
 int launch_copy2d_u32(oxq_ctx *ctx, hipStream_t s, const void *src, void *dst, int64_t rows, int64_t width,
                       int64_t dst_pitch, int64_t dst_col) {
     if (ctx->plan_only || rows * width == 0) return OXQ_OK;

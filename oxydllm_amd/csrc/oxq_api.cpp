@@ -796,7 +796,7 @@ static bool wcache_forward(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p, i
             (void)hipGetLastError();
             return false;
         }
-        const size_t bytes = (pk4_weight_bytes(p.K, p.N, p.bits) + 255) & ~(size_t)255;
+        const size_t bytes = (pk4_weight_bytes(p.K, p.N, p.bits, pk4_sets(p.group_shift)) + 255) & ~(size_t)255;
         if (!wcache_make_room(ctx, bytes)) return false;
         void *mem = nullptr;
         if (hipMalloc(&mem, bytes) != hipSuccess) {
@@ -805,7 +805,7 @@ static bool wcache_forward(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p, i
         }
         oxq_weight_cache::Entry e{p.qweight, p.qzeros, p.scales, p.K, p.N, p.group_shift, p.dtype, p.bits, p.pack_dim,
                                   Pk4Weights{(uint32_t *)mem, nullptr, p.K, p.N, p.group_shift, p.dtype, p.bits, 0,
-                                             p.pack_dim == OXQ_PACK_IN ? 32 : 16, pk4_choose_strip(ctx, p.K, p.N, p.bits, 0)},
+                                             p.pack_dim == OXQ_PACK_IN ? 32 : 16, pk4_choose_strip(ctx, p.K, p.N, p.bits, 0, pk4_sets(p.group_shift))},
                                   bytes, 0, false};
         const int prc = launch_pk4_prepack(ctx, s, p, e.w);  // on the caller's stream, ahead of the matmul
         if (prc != OXQ_OK) {
@@ -1986,7 +1986,7 @@ static int prepack_layer(oxq_packed_quant_linear *l) {
     if (check_wna16(ctx, "PackedQuantLinear", KIND_DEQUANT, nullptr, &l->qweight, &l->qzeros, &l->scales,
                     l->bits, l->pack_dim, &shape_only, &src) != OXQ_OK)
         return OXQ_OK;
-    if (!pk4_eligible(src)) return OXQ_OK;
+    if (!pk4_eligible(src) || (l->act && src.N % 64 != 0) || (l->has_bias && ((uintptr_t)l->bias.data & 7))) return OXQ_OK;  // a strip pairs 32 gate with 32 up columns
     l->pk.K = src.K;
     l->pk.N = src.N;
     l->pk.group_shift = src.group_shift;
@@ -1994,7 +1994,7 @@ static int prepack_layer(oxq_packed_quant_linear *l) {
     l->pk.bits = src.bits;
     l->pk.gate_half = l->act ? src.N / 2 : 0;
     l->pk.gemv_rows = src.pack_dim == OXQ_PACK_IN ? 32 : 16;
-    l->pk.strip = pk4_choose_strip(l->ctx, src.K, src.N, src.bits, l->pk.gate_half);
+    l->pk.strip = pk4_choose_strip(l->ctx, src.K, src.N, src.bits, l->pk.gate_half, pk4_sets(src.group_shift));
     if (ctx->plan_only) {
         l->prepacked = true;
         return OXQ_OK;
@@ -2003,7 +2003,7 @@ static int prepack_layer(oxq_packed_quant_linear *l) {
     (void)hipGetDevice(&prev);
     OXQ_HIP_CHECK(hipSetDevice(ctx->device));
     int rc = OXQ_OK;
-    hipError_t e = hipMalloc((void **)&l->pk.pw, pk4_weight_bytes(src.K, src.N, src.bits));
+    hipError_t e = hipMalloc((void **)&l->pk.pw, pk4_weight_bytes(src.K, src.N, src.bits, pk4_sets(src.group_shift)));
     l->pk.pzs = nullptr;  // the zero/scale pairs live inside the blocks of pw
     if (e != hipSuccess) {
         rc = fail(OXQ_ERR_RUNTIME, "PackedQuantLinear: repack allocation failed: %s", hipGetErrorString(e));
@@ -2125,8 +2125,8 @@ static int new_packed_layer(const char *op, oxq_ctx *ctx, uint32_t bits, int pac
     int rc = prepack_layer(l);
     if (rc == OXQ_OK && act && !l->prepacked)
         rc = fail(OXQ_ERR_UNSUPPORTED,
-                  "%s: the fused activation needs a resident layer (in_features and group size multiples of 128, "
-                  "out_features a multiple of 64, at most 128 groups, OXQ_PREPACK not 0); build a plain layer and "
+                  "%s: the fused activation needs a resident layer (in_features and group size multiples of 128 - or of 32 "
+                  "with at least 2^18 weights -, out_features a multiple of 64, OXQ_PREPACK not 0); build a plain layer and "
                   "call oxq_gated_activation on its output instead",
                   op);
     if (rc != OXQ_OK) {
@@ -2154,6 +2154,27 @@ int oxq_packed_quant_linear_new_gate_up(oxq_ctx *ctx, uint32_t bits, int pack_di
 }
 
 // linear.rs:482-533 PackedQuantLinear::forward
+static int packed_forward_staged(oxq_packed_quant_linear *l, hipStream_t s, const Pk4Problem &p) {
+    oxq_ctx *ctx = l->ctx;
+    const int64_t in = l->in_features, out = l->act ? l->out_features / 2 : l->out_features;
+    const int64_t x_row = (in + 7) & ~(int64_t)7, y_row = (out + 7) & ~(int64_t)7;  // eligible layers: both already multiples of 8
+    const int64_t rows = std::min<int64_t>(p.M, (int64_t)(ctx->workspace_bytes / 2) / (x_row + y_row));
+    if (rows < 1) return fail(OXQ_ERR_WORKSPACE, "PackedQuantLinear: a row needs more than the ctx workspace");
+    uint16_t *xs = (uint16_t *)ctx->workspace, *ys = xs + rows * x_row;
+    uint32_t launches = 0;
+    for (int64_t m0 = 0; m0 < p.M; m0 += rows) {
+        Pk4Problem q = p;
+        q.M = std::min<int64_t>(rows, p.M - m0);
+        q.x = xs, q.y = ys, q.no_split = 1;  // the workspace holds the copies
+        OXQ_TRY(launch_copy_u16(s, (const uint16_t *)p.x + m0 * in, xs, q.M * in));
+        OXQ_TRY(launch_pk4_forward(ctx, s, q));
+        launches += ctx->plan.launches + 2;
+        OXQ_TRY(launch_copy_u16(s, ys, (uint16_t *)p.y + m0 * out, q.M * out));
+    }
+    ctx->plan.launches = launches;
+    return OXQ_OK;
+}
+
 int oxq_packed_quant_linear_forward(oxq_packed_quant_linear *l, void *stream, const oxq_tensor *x,
                                     const oxq_tensor *out) {
     const char *op = "PackedQuantLinear";
@@ -2180,6 +2201,9 @@ int oxq_packed_quant_linear_forward(oxq_packed_quant_linear *l, void *stream, co
         q.act = l->act;
         q.no_split = 0;
         q.w = l->pk;
+        // the kernels' 16-byte accesses: rows at other addresses (a view that starts inside a row) go through aligned
+        // copies in the ctx workspace
+        if (!l->ctx->plan_only && (((uintptr_t)q.x | (uintptr_t)q.y) & 15)) return packed_forward_staged(l, (hipStream_t)stream, q);
         return launch_pk4_forward(l->ctx, (hipStream_t)stream, q);
     }
     Wna16Problem p;

@@ -178,7 +178,7 @@ struct F8Problem {
 
 // A resident 4- or 8-bit layer repacked tile-major at load (layout: pk4.hip).
 struct Pk4Weights {
-    uint32_t *pw;           // [N/64][K/128]{[4][bits/4][64][4] weights, [16][4] {-(bias + z), s} pairs}
+    uint32_t *pw;           // [N/64][K/128]{[4][bits/4][64][4] weights, [sets][16][4] {-(bias + z), s} pairs}
     uint32_t *pzs;          // unused (the pairs live inside the blocks of pw); kept null
     int64_t K, N;
     int group_shift;
@@ -207,12 +207,16 @@ bool pk4_eligible(const Wna16Problem &p);
 // resident 4-bit layers at prefill sizes: 64 rows x eight strips a workgroup (pk4_gemm.hip)
 bool pk4_gemm_takes(const oxq_ctx *ctx, const Pk4Problem &p);
 int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p);
-size_t pk4_weight_bytes(int64_t K, int64_t N, int bits);
-int pk4_choose_strip(const oxq_ctx *ctx, int64_t K, int64_t N, int bits, int64_t gate_half);
+int pk4_sets(int group_shift);  // zero/scale pairs a column has in a block of 128 rows: 1, 2 (groups of 64) or 4 (of 32)
+size_t pk4_weight_bytes(int64_t K, int64_t N, int bits, int sets);
+int pk4_choose_strip(const oxq_ctx *ctx, int64_t K, int64_t N, int bits, int64_t gate_half, int sets);
 size_t pk4_zs_bytes(int64_t K, int64_t N, int group_shift);
 int launch_pk4_prepack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &src, const Pk4Weights &dst);
 int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p);
 int launch_pk4_dequant(oxq_ctx *ctx, hipStream_t s, const Pk4Weights &w, void *out_kn);
+// groups of 32 or 64 rows (pk4_fine.hip): the ring kernel of launch_pk4_forward and the prefill kernel
+int launch_pk4_fine(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p, int bslice, int mt, bool fold);
+int launch_pk4_gemm_fine(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows, int ks, int NG, int RT);
 // 49 - 64 rows on a 4-bit layer in 64-column strips (pk4_tile.hip)
 bool pk4_tile64_takes(const Pk4Problem &p, int ks);
 int launch_pk4_tile64(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p);
@@ -249,6 +253,7 @@ int launch_gguf_mm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);
 int launch_compressed_to_awq(oxq_ctx *ctx, hipStream_t s, const uint32_t *ct, const void *scale_ct,
                              int scale_elem_bytes, uint32_t *qweight, uint32_t *qzeros, void *scales,
                              int64_t out_f, int64_t in_f, int64_t groups);
+int launch_copy_u16(hipStream_t s, const void *src, void *dst, int64_t n);
 int launch_copy2d_u32(oxq_ctx *ctx, hipStream_t s, const void *src, void *dst, int64_t rows, int64_t width,
                       int64_t dst_pitch, int64_t dst_col);
 int launch_gguf_depermute_rows(oxq_ctx *ctx, hipStream_t s, const uint8_t *src, uint8_t *dst, int64_t rows,

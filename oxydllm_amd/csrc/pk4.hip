@@ -22,15 +22,16 @@
 // whole share before it waits), pk4n_mfma_kernel / pk4n_front_kernel (the same pair for layers stored in
 // 16-column strips), the load-time repacks and the dense dequants that pin them.
 //
-// Layout (K % 128 == 0, N % 64 == 0, group size a multiple of 128).  A strip is a run of
-// K/128 self-contained blocks; a block covers 128 rows of K and holds its weights followed by the
+// Layout (N % 8 == 0; K and the group size multiples of 32; a last strip or block is filled up with zero weights of
+// scale zero).  A strip is a run of K/128 self-contained blocks; a block covers 128 rows of K and holds its weights followed by the
 // zeros and scales that apply to them:
 //
 //   pw  [N/64 strips][K/128 blocks]{ [4 steps][bits/4][64 lanes][4 words] , [16 column quads][4 words] }
 //
 // i.e. 4 KB (4-bit) or 8 KB (8-bit) of weights and 256 bytes of {-(bias_f + z), s} pairs, two 16-bit
 // floats of the layer's dtype per column (z already includes GPTQ's +1; a group larger than 128 rows
-// repeats its pair in each of its blocks).  With the pairs inside the stream a wave's loads for a
+// repeats its pair in each of its blocks; groups of 64 or 32 rows have two or four such sets of pairs, one after
+// another, pk4_fine.hip).  With the pairs inside the stream a wave's loads for a
 // block are one contiguous run, nothing is staged through LDS before the first multiply, and any
 // wave can take any block.
 //
@@ -54,6 +55,7 @@
 #include "oxq_internal.hpp"
 #include "oxq_mfma.hpp"
 #include "pk4_common.hpp"
+#include "pk4_mfma.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -76,25 +78,27 @@ __device__ __forceinline__ uint32_t src_q(const uint32_t *__restrict__ qw, int k
 }
 
 // one thread per word of the resident copy
-template <typename TT, bool GPTQ, int BITS>
+template <typename TT, bool GPTQ, int BITS, int SETS>
 __global__ __launch_bounds__(256) void pk4_prepack_kernel(const uint32_t *__restrict__ qw,
                                                           const uint32_t *__restrict__ qz,
                                                           const uint16_t *__restrict__ sc,
                                                           uint32_t *__restrict__ pw, int K, int N, int gshift,
                                                           int half) {
-    constexpr int PF = 32 / BITS, WL = BITS / 4, BW = pk4_block_words(BITS);
+    constexpr int PF = 32 / BITS, WL = BITS / 4, BW = pk4_block_words(BITS, SETS);
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const int NB = K >> 7;
-    if (idx >= (size_t)(N >> 6) * NB * BW) return;
+    const int NB = (K + 127) >> 7;
+    if (idx >= (size_t)((N + 63) >> 6) * NB * BW) return;
     const int w = (int)(idx % BW);
     const int b = (int)((idx / BW) % NB), j = (int)(idx / ((size_t)BW * NB));
     if (w < 1024 * WL) {
         const int pp = w & 3, l = (w >> 2) & 63, sh = w >> 8;
         const int h = sh % WL, st = sh / WL;
         const int ni = l & 15, kb = l >> 4;
-        const int k = pk4_kk(4 * b + st, kb) + 2 * pp;
+        const int k = pk4_kk<SETS>(4 * b + st, kb) + 2 * pp;
         uint32_t v = 0;
-        if (BITS == 4) {
+        if (k >= K || pk4_src_col(64 * j + 4 * ni, half) >= N) {
+            // rows past K, columns past N (whole quads: N is a multiple of 8): zero weights with zero scales
+        } else if (BITS == 4) {
 #pragma unroll
             for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -109,9 +113,13 @@ __global__ __launch_bounds__(256) void pk4_prepack_kernel(const uint32_t *__rest
         }
         pw[idx] = v;
     } else {
-        const int q = w - 1024 * WL, ni = q >> 2, f = q & 3;
-        const int g = (b << 7) >> gshift;
+        const int q = (w - 1024 * WL) & 63, ni = q >> 2, f = q & 3;
+        const int row = (b << 7) + ((w - 1024 * WL) >> 6) * (128 / SETS), g = row >> gshift;
         const int col = pk4_src_col(64 * j + 4 * ni + f, half);
+        if (row >= K || col >= N) {
+            pw[idx] = 0;
+            return;
+        }
         const int c = col % PF;
         const int slot = (GPTQ || BITS == 8) ? c : ((c >> 1) | ((c & 1) << 2));
         const uint32_t z = ((qz[(size_t)g * (N / PF) + col / PF] >> (BITS * slot)) & ((1u << BITS) - 1u)) + (GPTQ ? 1u : 0u);
@@ -125,26 +133,28 @@ __global__ __launch_bounds__(256) void pk4_prepack_kernel(const uint32_t *__rest
 // dense dequant of a resident layer -> [K, N] (linear.rs:510-523 fallback);
 // the same arithmetic as the matmul kernel's B fragments.
 // ---------------------------------------------------------------------------
-template <typename TT, int BITS>
+template <typename TT, int BITS, int SETS>
 __global__ __launch_bounds__(256) void pk4_dequant_kernel(const uint32_t *__restrict__ pw,
                                                           uint16_t *__restrict__ out, int K, int N, int half) {
-    constexpr int WL = BITS / 4, BW = pk4_block_words(BITS);
+    constexpr int WL = BITS / 4, BW = pk4_block_words(BITS, SETS);
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;  // over the weight words only
-    const int NB = K >> 7;
-    if (idx >= (size_t)(N >> 6) * NB * 1024 * WL) return;
+    const int NB = (K + 127) >> 7;
+    if (idx >= (size_t)((N + 63) >> 6) * NB * 1024 * WL) return;
     const int w = (int)(idx % (1024 * WL));
     const int b = (int)((idx / (1024 * WL)) % NB), j = (int)(idx / ((size_t)1024 * WL * NB));
     const uint32_t *blk = pw + ((size_t)j * NB + b) * BW;
     const int pp = w & 3, l = (w >> 2) & 63, sh = w >> 8;
     const int h = sh % WL, st = sh / WL;
     const int ni = l & 15, kb = l >> 4;
-    const int k = pk4_kk(4 * b + st, kb) + 2 * pp;
+    const int k = pk4_kk<SETS>(4 * b + st, kb) + 2 * pp;
+    if (k >= K || pk4_src_col(64 * j + 4 * ni, half) >= N) return;
+    const int set = SETS == 4 ? st : SETS == 2 ? st >> 1 : 0;
     const uint32_t wd = blk[w];
     const NibbleMasks nm = nibble_masks();
 #pragma unroll
     for (int c = 0; c < (BITS == 4 ? 4 : 2); ++c) {
         const int f = BITS == 4 ? c : 2 * h + c;
-        const uint32_t zs = blk[1024 * WL + ni * 4 + f];
+        const uint32_t zs = blk[1024 * WL + 64 * set + ni * 4 + f];
         uint32_t c0, c1;
         Pk4T<TT>::prep(zs, c0, c1);
         const uint32_t pair = BITS == 4 ? TT::unpack1(wd, f, nm) : TT::unpack_bytes(c ? (wd >> 8) : wd);
@@ -153,330 +163,6 @@ __global__ __launch_bounds__(256) void pk4_dequant_kernel(const uint32_t *__rest
         out[(size_t)k * N + col] = (uint16_t)(d & 0xFFFFu);
         out[(size_t)(k + 1) * N + col] = (uint16_t)(d >> 16);
     }
-}
-
-// ---------------------------------------------------------------------------
-// y[M, N] = x[M, K] . W   on the repacked layout
-//
-// grid.x = strip (64 output columns), grid.z = block of 16*MT rows of x,
-// grid.y = K slice (1 unless the layer has few strips and a long K, see the
-// launcher); the 8 waves deal the slice's blocks of 128 rows (4 MFMA steps) out
-// round-robin, so that at any moment the workgroup reads one contiguous stretch of
-// its strip (a plain read of the same bytes is 4 % faster that way than with one
-// contiguous eighth per wave).  With more than one slice the workgroup writes its
-// f32 partial tile to the workspace and a second launch adds the slices in order.
-//
-// Weights: one 1 KB wave load per step, issued one block (4 steps) ahead; the block's
-// zero/scale pairs ride in the same ring (one 16-byte load per lane and block).
-// Activations: the matrix-core fragment pattern (16 rows x 64 bytes per load)
-// is served by L2 at a third of the rate of 256-byte row reads, so a wave
-// fetches its next 16*MT x 128 block of x with 4-rows-x-256-bytes loads one
-// block ahead, parks it in its private LDS slot (16-byte chunks XOR-swizzled by
-// row, so both the row-wise write and the fragment read are conflict-free)
-// and reads fragments from there.  Rows past M are never fetched (out-of-range
-// lane offset: the buffer unit returns zero without touching memory).
-// All vector loads are issued unconditionally - steps past the end of a
-// wave's share also use the out-of-range offset - so the compiler can count
-// exactly how many loads are younger than the one it waits for; a conditionally
-// issued load makes it wait for all of them, which serialises the pipeline.
-// The 8 partial 16*MT x 64 tiles meet in LDS (each wave's slot is its own
-// activation slot) and are added in wave order, which fixes the summation order.
-//
-// Two arithmetic forms, both with f32 accumulation:
-//  * GS = false (m > 16, the reference's tile-GEMM range): B = T((q - z) * s),
-//    bit-identical to the dense dequant, fed to the matrix cores.
-//  * GS = true (m <= 16, the reference's fused-GEMV range, which never rounds
-//    the dequantized weight: quant_kernels.metal w4a16 GEMV keeps (q - z) * s in
-//    f32): the matrix cores multiply x by the exact integers bias + q, one
-//    extra MFMA against a fragment of ones yields the row sums of x in the
-//    accumulator layout, and once per block
-//        y += s * (acc_b - (bias + z) * rowsum_b(x))            (all f32).
-// ---------------------------------------------------------------------------
-// Ring depth: weights WD steps (1 KB wave loads).  One block of weights in flight per wave is
-// the measured optimum (4096 x 14336, f16, M = 1 / 16): 2 steps equal, 8 steps 5 - 10 % slower,
-// 16 steps 17 % slower.  A CU takes only so many vector loads in flight: what the first waves
-// issue beyond their next block keeps the other waves' first loads waiting.
-template <int MT, int BITS> struct Pk4Ring {
-    static constexpr int WD = 4;
-};
-
-// XQ: activation loads per block and lane that can hold rows below M (4 rows each); the
-// launcher passes 4 * MT, or fewer for a short single tile, whose other rows stay zero in LDS.
-// NBLK > 0: every wave has exactly NBLK blocks and the block loop is straight-line code.
-template <typename TT, int BITS, int MT, bool GS, int WD, int XQ, bool PLZ = false, int NBLK = 0>
-__global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restrict__ x,
-                                                       const uint32_t *__restrict__ pw,
-                                                       const uint16_t *__restrict__ bias,
-                                                       uint16_t *__restrict__ y, float *__restrict__ ws,
-                                                       int M, int K, int N, int bslice, int contiguous, int act) {
-    typedef MfmaOps<TT> Ops;
-    constexpr int NW = 8;                      // waves per workgroup (4 and 16 waves measured 30 % slower)
-    constexpr int ROWS = 16 * MT;
-    constexpr int AQ = XQ;                     // activation loads per block and lane
-    constexpr int SLOT = ROWS * 256;           // bytes of one wave's LDS slot (= its partial tile)
-    constexpr int OOB = 0x7FFFFF00;
-    constexpr int WL = BITS / 4;               // 1 KB weight loads per step
-    constexpr int BB = pk4_block_words(BITS) * 4;  // bytes of one block: weights, then the zero/scale pairs
-    // Up to 48 rows there is one row tile, so every weight is read once per launch: nontemporal
-    // loads (cache policy bit 1), which a bare read of the same 30 MB also gains 7 % from.
-    // From 49 rows on several row tiles may share a strip through L2, so those keep the default - except the
-    // forms that are only launched with one row-tile workgroup a strip (NBLK, PLZ).  64 rows, same box, default ->
-    // nontemporal: 4096 x 14336 f16 15.93 -> 15.45 us, bf16 17.48 -> 17.02; 5120 x 13824 f16 19.33 -> 18.54, 8-bit 24.14 ->
-    // 22.60; 8192 x 28672 51.7 -> 50.8.  (4096 x 11008 measures 14.44 -> 14.60: its 12 rotated copies, 270 MB, are
-    // partly still in the 256 MB memory-side cache when their turn comes again, which a decoder's layers are not.)
-    constexpr int WNT = (MT < 4 || NBLK > 0 || PLZ) ? 2 : 0;
-    // Hand-placed memory operations (the three places marked PLACED below) instead of the compiler's own order,
-    // where that measured faster - same box, 48 / 64 / 128 rows: 8-bit f16 5120 x 13824 21.8 / 27.3 / 42.5 ->
-    // 20.6 / 24.3 / 41.0 us; 4-bit bf16 4096 x 14336 at 33 / 48 rows 16.4 / 16.7 -> 15.2 / 15.9 us.  The 4-bit f16
-    // kernels and bf16 at four row tiles are as fast or faster as the compiler orders them (f16 at 64 / 128
-    // rows 16.9 / 29.4 against 16.6 / 30.8; bf16 19.6 / 33.8 against 18.7 / 34.3).
-    // PLZ: the 4-bit kernel at four row tiles when a strip has one row-tile workgroup and the tile is (nearly)
-    // full, 57 - 64 rows: placed it is 1.5 - 5 % faster there (same box, 64 rows: f16 16.48 -> 16.24, bf16 19.39 ->
-    // 18.43, 5120 x 13824 f16 20.3 -> 19.9 us), slower at 49 rows (f16 15.33 -> 15.71) and when two or more
-    // row-tile workgroups share a strip's weights through L2 (128 rows: f16 29.4 -> 30.8).
-    constexpr bool PLACED = PLZ || (MT >= 3 && (BITS == 8 || (TT::DTYPE == BF16Traits::DTYPE && MT == 3)));
-    extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ni = lane & 15, kb = lane >> 4;
-    const int j = blockIdx.x;
-    const int m0 = blockIdx.z * ROWS;
-    const int NB = K >> 7;
-    // K slice of this workgroup: blocks [sb0, sb0 + SB).  The wave's blocks inside it, by local index
-    // i: every 8th block starting at its own number (the default), or one contiguous run (a tuning
-    // switch; the shares differ by at most one block either way).
-    const int sb0 = blockIdx.y * bslice;
-    const int SB = min(NB, sb0 + bslice) - sb0;
-    const int cbase = SB / NW, crem = SB % NW;
-    const int nloc = contiguous ? cbase + (wave < crem ? 1 : 0) : (SB > wave ? (SB - wave + NW - 1) / NW : 0);
-    const int cb0 = sb0 + wave * cbase + min(wave, crem);
-    auto blk_of = [&](int i) { return contiguous ? cb0 + i : sb0 + i * NW + wave; };
-    unsigned char *slot = pk4_lds + wave * SLOT;
-
-    const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(pw + (size_t)j * NB * (BB / 4), (uint32_t)NB * (uint32_t)BB);
-    const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x, (uint32_t)M * (uint32_t)K * 2u);
-    const int voff_w = lane * 16;
-    // The block's zero/scale pairs: lane (ni, kb) fetches word kb of column quad ni (one 4-byte load a lane,
-    // 256 contiguous bytes a wave: a quarter of what a 16-byte load costs the address unit, which is the
-    // busiest unit from 32 rows on) and the four lane groups then exchange their words (zs_words).
-    const int voff_z = 1024 * WL * 4 + (ni * 4 + kb) * 4;
-    // activation load q of a block: row 4q + lane/16, 16-byte chunk lane%16 of the row's 256 bytes; rows
-    // past M get an offset beyond any buffer, for which the buffer unit returns zeros without touching
-    // memory (the scalar offset of a buffer load is not part of its bounds check, so the lane offset
-    // has to carry the row)
-    // Up to two row tiles every load keeps its own offset register; the larger kernels are at their
-    // register budget and derives them from the first one (a row past M then lies beyond the end of x by
-    // its lane offset alone, which the bounds check does cover).
-    constexpr bool VA1 = MT >= 3;
-    int voff_a[VA1 ? 1 : AQ];
-#pragma unroll
-    for (int q = 0; q < (VA1 ? 1 : AQ); ++q) {
-        const int r = m0 + 4 * q + kb;
-        voff_a[q] = r < M ? (r * K * 2 + ni * 16) : OOB;
-    }
-    uint32_t rowstep = 4u * (uint32_t)K * 2u;
-    // LDS position of (row = 4q + kb, chunk ni): chunk index XORed with row % 16 = kb | (q % 4) << 2
-    int a_wr[4];
-#pragma unroll
-    for (int qq = 0; qq < 4; ++qq) a_wr[qq] = kb * 256 + (((ni ^ kb) ^ (qq << 2)) << 4);  // + 1024 q
-    // fragment read of step s (0..3), row tile mt: row 16mt + ni, chunk 8*(s/2) + 2kb + (s%2)
-    int a_rd[4];
-#pragma unroll
-    for (int st = 0; st < 4; ++st) a_rd[st] = ni * 256 + (((8 * (st >> 1) + 2 * kb + (st & 1)) ^ ni) << 4);
-    const NibbleMasks nm = nibble_masks();
-    // rows no load covers: zero once, no block writes them again
-#pragma unroll
-    for (int q = AQ; q < 4 * MT; ++q) {
-        const int row = 4 * q + kb;
-        *(u32x4_t *)(slot + row * 256 + ((ni ^ (row & 15)) << 4)) = u32x4_t{0u, 0u, 0u, 0u};
-    }
-
-    static_assert(WD == 4, "the ring holds exactly one block");
-    u32x4_t aring[AQ], wring[WD][WL];
-    uint32_t zring;
-    // Past the end of the wave's share the loads go through an empty descriptor: a scalar select,
-    // no vector instruction, and the buffer unit returns zero without touching memory.
-    const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);
-    auto load_a = [&](int i, u32x4_t (&a)[AQ]) {
-        const __amdgpu_buffer_rsrc_t rs = i < nloc ? rs_x : rs_none;  // wave-uniform
-        const int blk = blk_of(i);
-#pragma unroll
-        for (int q = 0; q < AQ; ++q) {
-            if (VA1) {
-                if (q == 0) asm volatile("" : "+s"(rowstep));  // recomputed per block: 15 registers less to hold
-                // no wrap-around: 15 row steps stay below 2^31 (K <= 2^24, checked on the host), so a row
-                // past M - from the first offset or by the steps - lies beyond x (< 2 GiB) and reads zeros
-                a[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)((uint32_t)voff_a[0] + (uint32_t)q * rowstep), blk * 256, 0);
-            } else {
-                a[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff_a[q], blk * 256, 0);
-            }
-        }
-    };
-    auto load_w = [&](int i, int st, u32x4_t (&w)[WL]) {
-        const __amdgpu_buffer_rsrc_t rs = i < nloc ? rs_w : rs_none;
-#pragma unroll
-        for (int h = 0; h < WL; ++h)
-            w[h] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff_w, blk_of(i) * BB + (st * WL + h) * 1024, WNT);
-    };
-    auto load_z = [&](int i) {
-        const __amdgpu_buffer_rsrc_t rs = i < nloc ? rs_w : rs_none;
-        zring = __builtin_amdgcn_raw_buffer_load_b32(rs, voff_z, blk_of(i) * BB, WNT);
-    };
-    // zv[f] = the word that lane group f fetched, in every lane group: the lane-swap instructions
-    // exchange 16-lane rows between two registers (odd rows of one with even rows of the other, then
-    // the upper half of one with the lower half of the other).
-    auto zs_words = [&](uint32_t z, uint32_t (&zv)[4]) {
-        const auto p16 = __builtin_amdgcn_permlane16_swap(z, z, false, false);  // {r0 r0 r2 r2}, {r1 r1 r3 r3}
-        const uint32_t even = p16[0], odd = p16[1];
-        const auto pe = __builtin_amdgcn_permlane32_swap(even, even, false, false);  // {r0 x4}, {r2 x4}
-        const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);    // {r1 x4}, {r3 x4}
-        zv[0] = pe[0], zv[2] = pe[1], zv[1] = po[0], zv[3] = po[1];
-    };
-    auto store_a = [&](const u32x4_t (&a)[AQ]) {
-#pragma unroll
-        for (int q = 0; q < AQ; ++q) *(u32x4_t *)(slot + q * 1024 + a_wr[q & 3]) = a[q];
-    };
-
-    // issue order = consumption order.  The tile form needs the pairs before its first B fragment,
-    // the folded form after the block's last step.
-    u32x4_t afirst[AQ];
-    load_a(0, afirst);
-    if (!GS) load_z(0);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) load_w(0, g, wring[g]);
-    if (GS) load_z(0);
-    load_a(1, aring);
-
-    float4_t acc[MT][4];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int f = 0; f < 4; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
-    uint32_t negzb[4], sp[4];          // GS = false: the two Pk4T constants per column
-    const uint32_t ones[4] = {TT::ONES, TT::ONES, TT::ONES, TT::ONES};
-    const float4_t zero4 = float4_t{0.f, 0.f, 0.f, 0.f};
-
-    store_a(afirst);
-
-    // PLACED (1).  The counter a wave waits on counts its loads in issue order, and what the loop waits for at
-    // its top is the stricter of what its two entries require.  From three row tiles on the compiler requests
-    // the second x block before the first pairs and weights here, but after them inside the loop: coming from
-    // here the pairs have 4 younger loads, so the loop would wait with "at most 4 outstanding" - that is, for
-    // 12 of the 16 x loads it has just issued - in every iteration.  With block 0's pairs and weights
-    // complete before the loop, only the loop's own order counts.
-    if constexpr (PLACED) {
-        asm volatile("" ::"v"(zring));
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int h = 0; h < WL; ++h) asm volatile("" ::"v"(wring[g][h]));
-    }
-    // Two blocks an iteration where placed by hand: the ring registers a block loads are copied to the ones
-    // the loop carries at the loop's end, which waits for those loads; twice as rarely this way.
-    // With the block count known (NBLK) there is no loop at all (figures where it is launched).
-    constexpr int UF = NBLK > 0 ? 1 : PLACED ? 2 : 1;
-    const int trip = NBLK > 0 ? NBLK : nloc;
-    constexpr int UNROLL = NBLK > 0 ? NBLK : 1;
-#pragma unroll UNROLL
-    for (int i0 = 0; i0 < trip; i0 += UF)
-#pragma unroll
-    for (int u = 0; u < UF; ++u) {
-        const int i = i0 + u;
-        if (u > 0 && i >= nloc) break;
-        float4_t tmp[GS ? MT : 1][4], tmps[GS ? MT : 1];  // per-block integer sums of the GS form
-        if (!GS) {
-            uint32_t zv[4];
-            zs_words(zring, zv);
-#pragma unroll
-            for (int f = 0; f < 4; ++f) Pk4T<TT>::prep(zv[f], negzb[f], sp[f]);
-            load_z(i + 1);
-        }
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            u32x4_t wv[WL];
-#pragma unroll
-            for (int h = 0; h < WL; ++h) wv[h] = wring[st][h];
-            uint32_t wp[WL][4];
-#pragma unroll
-            for (int h = 0; h < WL; ++h) {
-                const uint32_t w0 = wv[h][0], w1 = wv[h][1], w2 = wv[h][2], w3 = wv[h][3];
-                wp[h][0] = w0, wp[h][1] = w1, wp[h][2] = w2, wp[h][3] = w3;
-            }
-            // row pair pp of column f as two exact 16-bit floats bias + q
-            auto pair = [&](int pp, int f) -> uint32_t {
-                if (BITS == 4) return TT::unpack1(wp[0][pp], f, nm);
-                const uint32_t word = wp[(f >> 1) % WL][pp];
-                return TT::unpack_bytes((f & 1) ? (word >> 8) : word);
-            };
-            uint32_t a[MT][4];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const u32x4_t av = *(const u32x4_t *)(slot + mt * 4096 + a_rd[st]);
-                const uint32_t a0 = av[0], a1 = av[1], a2 = av[2], a3 = av[3];
-                a[mt][0] = a0, a[mt][1] = a1, a[mt][2] = a2, a[mt][3] = a3;
-            }
-            if (GS) {
-                const bool fresh = st == 0;  // the block's sums start from zero: no clearing
-#pragma unroll
-                for (int f = 0; f < 4; ++f) {
-                    uint32_t b[4];
-#pragma unroll
-                    for (int pp = 0; pp < 4; ++pp) b[pp] = pair(pp, f);
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        tmp[mt][f] = Ops::mfma(a[mt], b, fresh ? zero4 : tmp[mt][f]);
-                }
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) tmps[mt] = Ops::mfma(a[mt], ones, fresh ? zero4 : tmps[mt]);
-            } else {
-#pragma unroll
-                for (int f = 0; f < 4; ++f) {
-                    uint32_t b[4];
-#pragma unroll
-                    for (int pp = 0; pp < 4; ++pp) b[pp] = Pk4T<TT>::deq(pair(pp, f), negzb[f], sp[f]);
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) acc[mt][f] = Ops::mfma(a[mt], b, acc[mt][f]);
-                }
-            }
-            // PLACED (2).  Vector-memory requests, LDS writes and MFMAs stay inside their step (vector and
-            // scalar arithmetic and LDS reads may move across): the ring refill above is then issued a block
-            // ahead of its use, as written, instead of at the block's end with the other three.
-            // Refill this ring slot after its last use, so that the new block can land in the same registers
-            // (requested while the old value is live it lands in others, copied at the loop's end behind a wait
-            // for the request): 17 / 33 / 48 rows f16 9.96 / 12.76 / 13.57 -> 9.85 / 12.57 / 13.44 us.
-            load_w(i + 1, st, wring[st]);
-            if constexpr (PLACED) __builtin_amdgcn_sched_barrier(0x106);
-        }
-        if (GS) {  // fold the block in: y += s * (sum - (bias + z) * rowsum), all f32
-            uint32_t zv[4];
-            zs_words(zring, zv);
-            load_z(i + 1);
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                const float sf = TT::to_f32((uint16_t)(zv[f] >> 16));
-                const float nszb = sf * TT::to_f32((uint16_t)(zv[f] & 0xFFFFu));  // -s * (bias_f + z)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        acc[mt][f][e] = fmaf(sf, tmp[mt][f][e], fmaf(nszb, tmps[mt][e], acc[mt][f][e]));
-            }
-        }
-        // the next block's activations replace this one's (same wave: LDS accesses stay in order)
-        // PLACED (3).  The x block stays in its registers until here: hoisted to the block's start (with all 16
-        // fragments of the current block held in registers instead), its reload comes late in the block and
-        // is waited for at the next block's start.
-        if constexpr (PLACED) __builtin_amdgcn_sched_barrier(0);
-        store_a(aring);
-        load_a(i + 2, aring);
-        // two and four row tiles as straight-line code: the requests for the block after next stay at the block's
-        // end (four tiles at 64 rows, same box: f16 16.54 -> 16.37 us, bf16 18.42 -> 17.90; three tiles the same
-        // either way)
-        if constexpr (NBLK > 0 && (MT == 2 || MT == 4)) __builtin_amdgcn_sched_barrier(0);
-    }
-
-    pk4_epilogue<TT, MT>(acc, bias, y, ws, M, N, j, m0, act, wave, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1018,23 +704,29 @@ __global__ __launch_bounds__(1024) void pk4n_front_kernel(const uint16_t *__rest
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-size_t pk4_weight_bytes(int64_t K, int64_t N, int bits) {
-    return (size_t)(N / 64) * (size_t)(K / 128) * (size_t)pk4_block_words(bits) * 4;
+int pk4_sets(int group_shift) { return group_shift >= 7 ? 1 : group_shift == 6 ? 2 : 4; }
+size_t pk4_weight_bytes(int64_t K, int64_t N, int bits, int sets) {
+    return (size_t)ceil_div(N, 64) * (size_t)ceil_div(K, 128) * (size_t)pk4_block_words(bits, sets) * 4;
 }
 size_t pk4_zs_bytes(int64_t, int64_t, int) { return 0; }  // the pairs live inside the blocks
 
 bool pk4_eligible(const Wna16Problem &p) {
     if (p.bits != 4 && p.bits != 8) return false;
-    if (p.K % 128 != 0 || p.N % 64 != 0 || p.group_size % 128 != 0) return false;
+    if (p.N % 8 != 0 || p.K % 32 != 0 || p.group_size % 32 != 0) return false;
+    const int sets = pk4_sets(p.group_shift);
+    // Groups of 32 or 64 rows, or columns that end inside a strip: from 2^18 weights on.  Below, the checkpoint-layout
+    // kernels take a launch's time as well (512 x 512 at 1 - 8 rows: 4.5 - 6 us either way), and the copy would only cost memory.
+    if ((sets > 1 || p.N % 64 != 0) && p.K * p.N < (1 << 18)) return false;
     // 32-bit offsets inside a strip and in x; one launch of the repack covers the copy
-    if ((uint64_t)(p.K / 128) * pk4_block_words(p.bits) * 4 >= (1ull << 31) || p.K > (1 << 24)) return false;
-    if (pk4_weight_bytes(p.K, p.N, p.bits) / 4 >= (1ull << 31) * 256) return false;
+    if ((uint64_t)ceil_div(p.K, 128) * pk4_block_words(p.bits, sets) * 4 >= (1ull << 31) || p.K > (1 << 24)) return false;
+    if (pk4_weight_bytes(p.K, p.N, p.bits, sets) / 4 >= (1ull << 31) * 256) return false;
     return true;
 }
 
 int launch_pk4_prepack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &src, const Pk4Weights &dst) {
     const int K = (int)src.K, N = (int)src.N;
-    const size_t words = pk4_weight_bytes(K, N, src.bits) / 4;
+    const int sets = pk4_sets(src.group_shift);
+    const size_t words = pk4_weight_bytes(K, N, src.bits, sets) / 4;
     const bool gptq = src.pack_dim == OXQ_PACK_IN;
     dim3 grid((unsigned)ceil_div((int64_t)words, 256)), block(256);
     char name[64];
@@ -1052,9 +744,13 @@ int launch_pk4_prepack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &src, con
         return OXQ_OK;
     }
     const int half = (int)dst.gate_half;
-#define OXQ_PP(TTv, Gv, Bv)                                                                                     \
-    hipLaunchKernelGGL((pk4_prepack_kernel<TTv, Gv, Bv>), grid, block, 0, s, src.qweight, src.qzeros,           \
+#define OXQ_PPS(TTv, Gv, Bv, Sv)                                                                                \
+    hipLaunchKernelGGL((pk4_prepack_kernel<TTv, Gv, Bv, Sv>), grid, block, 0, s, src.qweight, src.qzeros,       \
                        (const uint16_t *)src.scales, dst.pw, K, N, src.group_shift, half)
+#define OXQ_PP(TTv, Gv, Bv)                                                                                     \
+    do {                                                                                                        \
+        if (sets == 1) OXQ_PPS(TTv, Gv, Bv, 1); else if (sets == 2) OXQ_PPS(TTv, Gv, Bv, 2); else OXQ_PPS(TTv, Gv, Bv, 4); \
+    } while (0)
     if (src.dtype == OXQ_F16) {
         if (src.bits == 4) { if (gptq) OXQ_PP(F16Traits, true, 4); else OXQ_PP(F16Traits, false, 4); }
         else { if (gptq) OXQ_PP(F16Traits, true, 8); else OXQ_PP(F16Traits, false, 8); }
@@ -1063,12 +759,14 @@ int launch_pk4_prepack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &src, con
         else { if (gptq) OXQ_PP(BF16Traits, true, 8); else OXQ_PP(BF16Traits, false, 8); }
     }
 #undef OXQ_PP
+#undef OXQ_PPS
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
 
 int launch_pk4_dequant(oxq_ctx *ctx, hipStream_t s, const Pk4Weights &w, void *out_kn) {
-    const size_t words = (size_t)w.K * w.N * w.bits / 32;
+    const int sets = pk4_sets(w.group_shift);
+    const size_t words = (size_t)ceil_div(w.N, 64) * (size_t)ceil_div(w.K, 128) * 256 * (size_t)w.bits;  // weights of whole blocks
     dim3 grid((unsigned)ceil_div((int64_t)words, 256)), block(256);
     char name[64];
     snprintf(name, sizeof name, "pk%d_dequant_%s", w.bits, w.dtype == OXQ_F16 ? "f16" : "bf16");
@@ -1082,15 +780,20 @@ int launch_pk4_dequant(oxq_ctx *ctx, hipStream_t s, const Pk4Weights &w, void *o
         OXQ_HIP_CHECK(hipGetLastError());
         return OXQ_OK;
     }
-#define OXQ_DQ(TTv, Bv)                                                                           \
-    hipLaunchKernelGGL((pk4_dequant_kernel<TTv, Bv>), grid, block, 0, s, w.pw, (uint16_t *)out_kn, \
+#define OXQ_DQS(TTv, Bv, Sv)                                                                          \
+    hipLaunchKernelGGL((pk4_dequant_kernel<TTv, Bv, Sv>), grid, block, 0, s, w.pw, (uint16_t *)out_kn, \
                        (int)w.K, (int)w.N, (int)w.gate_half)
+#define OXQ_DQ(TTv, Bv)                                                                               \
+    do {                                                                                              \
+        if (sets == 1) OXQ_DQS(TTv, Bv, 1); else if (sets == 2) OXQ_DQS(TTv, Bv, 2); else OXQ_DQS(TTv, Bv, 4); \
+    } while (0)
     if (w.dtype == OXQ_F16) {
         if (w.bits == 4) OXQ_DQ(F16Traits, 4); else OXQ_DQ(F16Traits, 8);
     } else {
         if (w.bits == 4) OXQ_DQ(BF16Traits, 4); else OXQ_DQ(BF16Traits, 8);
     }
 #undef OXQ_DQ
+#undef OXQ_DQS
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
@@ -1103,19 +806,6 @@ static int pk4_front_go(hipStream_t s, dim3 grid, const Pk4Problem &p, int bslic
     hipLaunchKernelGGL((pk4_front_kernel<TT, BITS, NBLK, XQ, NW, WIN>), grid, dim3(NW * 64), lds, s, (const uint16_t *)p.x, p.w.pw,
                        (const uint16_t *)p.bias, (uint16_t *)p.y, (float *)p.ws, (int)p.M, (int)p.w.K, (int)p.w.N,
                        bslice, p.act);
-    OXQ_HIP_CHECK(hipGetLastError());
-    return OXQ_OK;
-}
-
-// one instantiation of pk4_mfma_kernel: its LDS grant, the launch, the error check
-template <typename TT, int BITS, int MT, bool GS, int WD, int XQ, bool PLZ = false, int NBLK = 0>
-static int pk4_mfma_go(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p, int bslice) {
-    const size_t lds = (size_t)8 * MT * 4096;
-    static LdsGrant lds_grant;
-    OXQ_HIP_CHECK(lds_grant.ensure((const void *)pk4_mfma_kernel<TT, BITS, MT, GS, WD, XQ, PLZ, NBLK>, lds));
-    hipLaunchKernelGGL((pk4_mfma_kernel<TT, BITS, MT, GS, WD, XQ, PLZ, NBLK>), grid, dim3(512), lds, s,
-                       (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias, (uint16_t *)p.y, (float *)ctx->workspace,
-                       (int)p.M, (int)p.w.K, (int)p.w.N, bslice, tune(ctx, OXQ_TUNE_PK4_CONTIGUOUS, 1), p.act);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
@@ -1223,7 +913,7 @@ static int pk4_by_mt(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p
 // Strip width of a layer's resident copy: 16 columns for 4-bit layers of at most 128 64-column strips and a
 // K of 32 - 112 blocks, or at most 80 strips and 16 - 31 blocks (the shapes that otherwise leave CUs idle or need
 // K slices and a second launch), 64 otherwise.
-int pk4_choose_strip(const oxq_ctx *ctx, int64_t K, int64_t N, int bits, int64_t gate_half) {
+int pk4_choose_strip(const oxq_ctx *ctx, int64_t K, int64_t N, int bits, int64_t gate_half, int sets) {
     // Measured (f16; 64-column strips, with K slices where few -> 16-column strips, one launch up to 8 rows),
     // at 1 / 4 / 16 / 64 rows of x:
     //    4096 x  4096   5.85 / -    / -     / -      ->  3.64 /  3.95 /  5.24 / 11.5 us
@@ -1237,7 +927,7 @@ int pk4_choose_strip(const oxq_ctx *ctx, int64_t K, int64_t N, int bits, int64_t
     // 16.4; 5120 x 13824 and 8192 x 28672 alike), and on a very long K every strip's pass over x outweighs
     // the saved launch from 4 rows on (28672 x 8192: 23.2 / 23.4 us wide, 21.3 / 26.6 narrow).
     const int mode = tune(ctx, OXQ_TUNE_PK4_STRIP16, 1);  // 0 never, 1 by shape, 2 wherever the layout applies
-    if (!mode || bits != 4 || gate_half || N % 64 != 0) return 64;
+    if (!mode || bits != 4 || gate_half || N % 64 != 0 || sets != 1) return 64;
     if (mode == 2) return 16;
     // Shorter K (16 - 31 blocks: hidden sizes of 2048 - 3968) gains on layers up to 5120 columns, whose 64-column
     // strips leave most CUs idle (3584 x 3584 at 1 / 8 / 16 / 64 rows 5.79 / 6.08 / 6.80 / 13.6 -> 3.57 / 4.08 / 5.05 /
@@ -1390,13 +1080,14 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (p.w.strip == 16) return launch_pk4n_forward(ctx, s, p);
     const int64_t M = p.M;
     const int mt = M > 48 ? 4 : (int)ceil_div(M, 16);
-    const int NB = (int)(p.w.K / 128);
+    const int NB = (int)ceil_div(p.w.K, 128), sets = pk4_sets(p.w.group_shift);
+    const int64_t strips = ceil_div(p.w.N, 64);
     // Few column strips and a long K (a down projection: N = 4096 is 64 strips for 256 CUs):
     // K is also cut into slices, at least one block per wave, so that up to one workgroup per CU
     // runs; the slices' f32 partial tiles are added in slice order by a second launch.  Measured
     // (f16, M = 1 / 16): 14336 x 4096 16.9 / 19.1 us unsplit, 9.0 / 10.0 us in 4 slices, 9.5 - 10.2 /
     // 11.4 - 12.1 us in 3, 6 or 8; a 4096 x 4096 layer 6.4 / 7.4 us unsplit, 5.7 / 6.6 us in 4 slices.
-    const int64_t tiles = (p.w.N / 64) * ceil_div(M, 16 * mt);
+    const int64_t tiles = strips * ceil_div(M, 16 * mt);
     int ks = 1;
     if (tiles <= 96 && NB >= 32) ks = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tiles, NB / 8));
     // Half a round of workgroups and a long K: two slices.  Measured (f16, 1 / 16 / 64 rows): 8192 x 8192
@@ -1413,7 +1104,7 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     ks = (int)ceil_div(NB, bslice);  // no empty slice
     if (ceil_div(M, 16 * mt) > 65535)
         return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid limit (65535 row tiles)", (long long)M);
-    dim3 grid((unsigned)(p.w.N / 64), (unsigned)ks, (unsigned)ceil_div(M, 16 * mt));
+    dim3 grid((unsigned)strips, (unsigned)ks, (unsigned)ceil_div(M, 16 * mt));
     char name[64];
     // A single row tile (up to 16 rows) runs straight-line kernels (pk4_front_kernel) where one exists for the
     // slice: no loop, so no loop-carried ring registers to copy (and wait for) at its end, and every request
@@ -1441,14 +1132,14 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const int front_mode = tune(ctx, OXQ_TUNE_PK4_FRONT, 1);  // 0: the ring kernel, 2: never 16 waves
     const int share8 = (bslice + 7) / 8;
     int front = 0;
-    if (mt == 1 && front_mode != 0) {
+    if (mt == 1 && front_mode != 0 && sets == 1) {
         if (p.w.bits == 4)
             front = (front_mode != 2 && bslice == 32 && front_xq <= 2) ? 1 : share8 <= 8 ? 2 : 0;
         else
             front = (front_mode != 2 && bslice == 32 && ks == 1) ? 1 : (bslice % 8 == 0 && share8 <= 8 && share8 != 7) ? 2 : 0;
     }
-    snprintf(name, sizeof name, "pk%d_mfma_%s_mt%d%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", mt,
-             pk4_folds(ctx, p, mt) ? "_gs" : "", front == 1 ? "_front" : front == 2 ? "_line" : "",
+    snprintf(name, sizeof name, "pk%d_mfma_%s_mt%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", mt,
+             pk4_folds(ctx, p, mt) ? "_gs" : "", sets == 2 ? "_g64" : sets == 4 ? "_g32" : "", front == 1 ? "_front" : front == 2 ? "_line" : "",
              p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(front == 1 ? 1024 : 512), ks, 1, ks > 1 ? (size_t)ks * M * p.w.N * 4 : 0);
     if (ctx->plan_only) {
@@ -1461,6 +1152,11 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
         return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: x and y must be 16-byte aligned");
     const bool f16 = p.w.dtype == OXQ_F16;
     int rc;
+    if (sets > 1) {
+        rc = launch_pk4_fine(ctx, s, grid, p, bslice, mt, pk4_folds(ctx, p, mt));
+        if (rc != OXQ_OK || ks == 1) return rc;
+        return launch_splitk_reduce(ctx, s, (const float *)ctx->workspace, p.bias, p.y, M, p.w.N, ks, p.w.dtype);
+    }
     if (tune(ctx, OXQ_TUNE_PK4_T64, 1) && pk4_tile64_takes(p, ks)) {
         Pk4Problem q = p;
         q.ws = ctx->workspace;

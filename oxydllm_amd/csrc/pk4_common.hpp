@@ -127,7 +127,16 @@ template <> struct Pk4N<BF16Traits> {
     __device__ __forceinline__ void odd_from_even() {}
 };
 
-__device__ __forceinline__ int pk4_kk(int t, int kb) { return ((t >> 1) << 6) + (kb << 4) + ((t & 1) << 3); }
+// First row of lane group kb's eight in step t.  Groups of 64 rows and more: two steps cover 16 consecutive rows per
+// lane group (the matching activation loads are then 32 contiguous bytes a row).  Groups of 32 rows (SETS = 4): a
+// step's rows are one group, in order.
+template <int SETS = 1> __device__ __forceinline__ int pk4_kk(int t, int kb) {
+    return SETS == 4 ? (t << 5) + (kb << 3) : ((t >> 1) << 6) + (kb << 4) + ((t & 1) << 3);
+}
+// 16-byte chunk of a 128-element row of x that holds those rows' activations (step st of a block)
+template <int SETS> __device__ __forceinline__ int pk4_x_chunk(int st, int kb) {
+    return SETS == 4 ? 4 * st + kb : 8 * (st >> 1) + 2 * kb + (st & 1);
+}
 
 // Resident column -> checkpoint column.  A fused gate|up layer (half = N/2) keeps, in every strip
 // of 64, 32 gate columns followed by the 32 up columns they are multiplied with, so that one
@@ -138,8 +147,9 @@ __device__ __forceinline__ int pk4_src_col(int c, int half) {
     return cc < 32 ? 32 * j + cc : half + 32 * j + (cc - 32);
 }
 
-// words of one block: weights, then the 64 words of zero/scale pairs
-__host__ __device__ constexpr int pk4_block_words(int bits) { return 1024 * (bits / 4) + 64; }
+// words of one block: weights, then `sets` times the 64 words of zero/scale pairs (groups of 128 rows and more: one
+// set, groups of 64: two, groups of 32: four)
+__host__ __device__ constexpr int pk4_block_words(int bits, int sets = 1) { return 1024 * (bits / 4) + 64 * sets; }
 
 // The 8 waves' partial 16*MT x 64 tiles meet in LDS and are added in wave order; then either the
 // fused gate|up activation, the K slice's f32 partial, or the result in the layer dtype.
@@ -226,6 +236,7 @@ __device__ __forceinline__ void pk4_epilogue(const float4_t (&acc)[MT][4], const
             }
         }
         const int n = 64 * j + c0;
+        if (n >= N) continue;  // the last strip of a layer whose columns (a multiple of 8) end inside it
         if (gridDim.y > 1) {  // this K slice's f32 partial; a second kernel adds the slices in order
             float *dst = ws + ((size_t)blockIdx.y * M + (m0 + ml)) * N + n;
             if (CP == 2) {
@@ -278,6 +289,7 @@ __device__ __forceinline__ void pk4_epilogue_lanes(const float4_t (&acc)[MT][4],
     constexpr int PER = PLANES >= NW ? PLANES / NW : 1;
     if (PLANES < NW && wave >= PLANES) return;
     const int ni = lane & 15, kb = lane >> 4;
+    if (64 * j + 4 * ni >= N) return;
     float4_t bv = float4_t{0.f, 0.f, 0.f, 0.f};
     if (bias) {
         const uint2 b = *(const uint2 *)(bias + 64 * j + 4 * ni);

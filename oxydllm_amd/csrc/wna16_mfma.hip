@@ -696,9 +696,10 @@ bool awq4_mfma_ok(const Wna16Problem &p) {
 // is one pass over the weights: about 45 us at 5120 x 13824, 4-bit).  A caller that holds the layer should hold a
 // PackedQuantLinear, which repacks once.
 static bool transient_repack_fits(const oxq_ctx *ctx, const Wna16Problem &p) {
+    if ((((uintptr_t)p.x | (uintptr_t)p.y) & 15) || ((uintptr_t)p.bias & 7)) return false;
     return p.M > 8 && pk4_eligible(p) && !ctx->plan_only && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
            !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0) &&
-           ((pk4_weight_bytes(p.K, p.N, p.bits) + 255) & ~(size_t)255) <= ctx->workspace_bytes;
+           ((pk4_weight_bytes(p.K, p.N, p.bits, pk4_sets(p.group_shift)) + 255) & ~(size_t)255) <= ctx->workspace_bytes;
 }
 static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     Pk4Weights w{(uint32_t *)ctx->workspace, nullptr, p.K, p.N, p.group_shift, p.dtype, p.bits, 0,
