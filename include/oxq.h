@@ -494,13 +494,17 @@ int oxq_qlinear_forward(oxq_qlinear *layer, void *stream, const oxq_tensor *x,
  * builds a layer-owned copy of the blocks in strips of 16 rows (the file's bytes per weight; Q3_K: 112 for
  * 110 bytes a super-block; so twice the
  * layer's bytes while the caller keeps weight_bytes); forward then runs 1 - 4 rows of x on that copy (f32
- * rows up to 8, in two passes of four) and everything else on weight_bytes as before.  A BF16 layer of Q4_0,
- * Q4_1, Q5_0, Q5_1, Q8_0, Q4_K, Q5_K or Q6_K holds the copy in the matrix-core layout instead (the same size), on
- * which one launch takes 1 - 32 rows with the GEMV's arithmetic at every
- * row count: integer sums, one f32 scale per sub-block, the weights never rounded to bf16 (the reference's
- * prefill tiles round them above 8 rows).  The tuning switch OXQ_PREPACK=0 turns the copy off, OXQ_GGUF_MFMA=0
- * keeps the first layout for BF16 layers too.
- * *resident = 1 if the layer holds the copy. */
+ * rows up to 8, in two passes of four) and everything else on weight_bytes.  A BF16 layer of Q4_0,
+ * Q4_1, Q5_0, Q5_1, Q8_0, Q4_K, Q5_K or Q6_K holds the copy in the matrix-core layout instead (the same size; from
+ * 2^20 weights also where out_features ends inside a strip), on which one launch takes 1 - 32 rows with the GEMV's
+ * arithmetic at every row count: integer sums, one f32 scale per sub-block, the weights never rounded to bf16 (the
+ * reference's prefill tiles round them above 8 rows).  More rows run on the same copy too where a kernel on it is the
+ * cheapest (from 2^20 weights: always): tiles of bf16-rounded weights, or the integer kernel in row tiles.  An F32
+ * layer of those formats with at least 2^20 weights holds both copies (three times the layer's bytes with
+ * weight_bytes): from three rows on - fewer on some shapes - the matrix cores multiply each f32 as the sum of three bf16
+ * pieces, exact products in f32 sums, at any row count.  The tuning switch OXQ_PREPACK=0 turns the copies off,
+ * OXQ_GGUF_MFMA=0 keeps the first layout alone.
+ * *resident = 1 if the layer holds a copy. */
 int oxq_qlinear_is_resident(const oxq_qlinear *layer, int *resident);
 /* Dense f32 [out_features, in_features] of the layer's weights, read from the copy when there is one:
  * bit for bit what oxq_gguf_dequantize returns for weight_bytes. */

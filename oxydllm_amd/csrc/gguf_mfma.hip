@@ -84,9 +84,20 @@ __global__ __launch_bounds__(256) void ggm_repack_kernel(const uint8_t *__restri
     typedef GgmLayout<FMT> L;
     const int nch = K >> 7;
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (size_t)(N >> 4) * nch * 64) return;
+    if (idx >= (size_t)((N + 15) >> 4) * nch * 64) return;
     const int lane = (int)(idx & 63), c = (int)((idx >> 6) % nch), strip = (int)((idx >> 6) / nch);
     const int ni = lane & 15, kb = lane >> 4;
+    if (16 * strip + ni >= N) {  // the last strip of a layer whose rows end inside it: zero weights, zero scales
+        uint8_t *zb = pw + ((size_t)strip * (nch / F::CH) + c / F::CH) * L::BLKB, *zc = zb + (c % F::CH) * L::CHB;
+#pragma unroll
+        for (int pl = 0; pl < F::WQ; ++pl) *(u32x4_t *)(zc + pl * 1024 + lane * 16) = u32x4_t{0u, 0u, 0u, 0u};
+        if constexpr (FMT == OXQ_GGUF_Q6_K) *(uint2 *)(zc + L::H_OFF + lane * 8) = uint2{0u, 0u};
+        if constexpr (ggm_fifth_bit<FMT>) *(uint32_t *)(zc + L::H_OFF + lane * 4) = 0u;
+        for (int b = kb; b < F::UH; b += 4) zc[L::UH_OFF + ni * F::UH + b] = 0;
+        if (c % F::CH == 0)
+            for (int b = kb; b < F::BH; b += 4) zb[L::BH_OFF + ni * F::BH + b] = 0;
+        return;
+    }
     const size_t row_bytes = (size_t)(K / GgufFmt<FMT>::BE) * GgufFmt<FMT>::BB;
     const uint8_t *row = w + (size_t)ggm_src_row(16 * strip + ni, half) * row_bytes;
     uint8_t *blk = pw + ((size_t)strip * (nch / F::CH) + c / F::CH) * L::BLKB;
@@ -206,9 +217,10 @@ __global__ __launch_bounds__(256) void ggm_dequant_kernel(const uint8_t *__restr
     typedef GgmLayout<FMT> L;
     const int nch = K >> 7;
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (size_t)(N >> 4) * nch * 64) return;
+    if (idx >= (size_t)((N + 15) >> 4) * nch * 64) return;
     const int lane = (int)(idx & 63), c = (int)((idx >> 6) % nch), strip = (int)((idx >> 6) / nch);
     const int ni = lane & 15, kb = lane >> 4;
+    if (16 * strip + ni >= N) return;
     const uint8_t *blk = pw + ((size_t)strip * (nch / F::CH) + c / F::CH) * L::BLKB;
     const uint8_t *chunk = blk + (c % F::CH) * L::CHB;
     const size_t orow = (size_t)ggm_src_row(16 * strip + ni, half);
@@ -400,6 +412,41 @@ template <int FMT> struct GgmChunk {
     }
 };
 
+// The B operand with the smallest bias that leaves the integers exact, for f32 activations: 16 + q (4-bit formats), 32 + q
+// (5-bit), 64 + q (Q6_K).  The bias and the format's offset come out in the same f32 accumulator, and what is taken out
+// there costs precision in proportion to its size: with 128 + q the sums carry seven times the rounding of the integers'
+// own products.  Bytes (Q8_0) have no bias.  A pair is built as for 128 + q, with the bits moved to the mantissa position
+// that the exponent asks for: as many instructions.
+template <int FMT> struct GgmSmallBias {
+    static constexpr bool NIB = FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q4_K;
+    static constexpr float BIAS = NIB ? 16.f : ggm_fifth_bit<FMT> ? 32.f : FMT == OXQ_GGUF_Q6_K ? 64.f : 0.f;
+    // the constant that takes bias and offset out (the minimum's term divides by it)
+    static constexpr float NEG = -(BIAS + (FMT == OXQ_GGUF_Q4_0 ? 8.f : FMT == OXQ_GGUF_Q5_0 ? 16.f : FMT == OXQ_GGUF_Q6_K ? 32.f : FMT == OXQ_GGUF_Q8_0 ? 128.f : 0.f));
+    static constexpr uint32_t NEG_PAIR = (__builtin_bit_cast(uint32_t, NEG) >> 16) | (__builtin_bit_cast(uint32_t, NEG) & 0xFFFF0000u);
+    static constexpr int AT = NIB ? 3 : ggm_fifth_bit<FMT> ? 2 : 1;  // mantissa bit of the nibble's lowest
+    static constexpr uint32_t EXP = NIB ? 0x41804180u : ggm_fifth_bit<FMT> ? 0x42004200u : 0x42804280u;
+    static constexpr uint32_t M0 = (0xFu << AT) * 0x10001u, M1 = (ggm_fifth_bit<FMT> ? 0x40u : 0x60u) * 0x10001u;
+    __device__ static __forceinline__ uint32_t move(uint32_t v, int left) { return left >= 0 ? v << left : v >> -left; }
+    __device__ static __forceinline__ void operand(const GgmChunk<FMT> &w, int st, uint32_t (&b)[4], const NibbleMasks &nm) {
+        if constexpr (NIB) {
+#pragma unroll
+            for (int pp = 0; pp < 4; ++pp) b[pp] = (move(w.q[0][st], AT - 4 * pp) & nm.m0) | EXP;
+        } else if constexpr (ggm_fifth_bit<FMT>) {  // the bit of pair pp: bit 4 st + pp -> 6
+#pragma unroll
+            for (int pp = 0; pp < 4; ++pp)
+                b[pp] = (move(w.qh[0], 6 - 4 * st - pp) & nm.m1) | ((move(w.q[0][st], AT - 4 * pp) & nm.m0) | EXP);
+        } else if constexpr (FMT == OXQ_GGUF_Q6_K) {  // the bit pair of field f: bits 2 f, 2 f + 1 -> 5, 6
+#pragma unroll
+            for (int pr = 0; pr < 2; ++pr)
+                b[pr] = (move(w.qh[st >> 2], 5 - 2 * (2 * (st & 3) + pr)) & nm.m1) |
+                        ((move(w.q[0][st >> 1], AT - 4 * (2 * (st & 1) + pr)) & nm.m0) | EXP);
+            b[2] = b[3] = 0u;
+        } else {
+            w.operand(st, b, nm);
+        }
+    }
+};
+
 typedef short short4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float4_t ggm_mfma16(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4_t, u32x2_t{a0, a1}),
@@ -449,10 +496,66 @@ __device__ __forceinline__ void ggm_epilogue_act(const float4_t (&acc)[MT][NS], 
     }
 }
 
-template <int FMT, int MT, int XQ, int NW, int NS>
+// Epilogue of the f32 form: tile row 4 p + m holds piece p of row m of x.  The waves' partial tiles meet in LDS; a wave
+// takes a row of x, lane (p, ni) adds piece p's sums over the waves in order, and the three pieces' lanes meet, the
+// smallest piece first.
+template <int MT, int NS, int NW>
+__device__ __forceinline__ void ggm_epilogue_f32(const float4_t (&acc)[MT][NS], const float *__restrict__ bias, float *__restrict__ y,
+                                                 int M, int N, int j, int m0, int wave, int lane) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float *dst = (float *)(pk4_lds + (size_t)wave * MT * 4096) + ((mt * 4 + e) * 64 + lane) * NS;
+#pragma unroll
+            for (int f = 0; f < NS; ++f) dst[f] = acc[mt][f][e];
+        }
+    __syncthreads();
+    for (int ml = wave; ml < 4 * MT && m0 + ml < M; ml += NW)
+#pragma unroll
+        for (int f = 0; f < NS; ++f) {
+            float v = 0.f;
+#pragma unroll
+            for (int s = 0; s < NW; ++s) v += ((const float *)(pk4_lds + (size_t)s * MT * 4096))[(ml * 64 + lane) * NS + f];
+            const float v1 = __shfl_down(v, 16), v2 = __shfl_down(v, 32);
+            const int n = 16 * (NS * j + f) + lane;
+            if (lane < 16 && n < N) {
+                const float tot = (v2 + v1) + v;
+                y[(size_t)(m0 + ml) * N + n] = bias ? tot + bias[n] : tot;
+            }
+        }
+}
+// Eight f32 as three bf16 pieces whose sum they are, exactly: truncated to 8 significant bits, the rest truncated, the
+// rest of that (at most 8 bits).
+__device__ __forceinline__ void ggm_split3_pair(uint32_t a, uint32_t b, uint32_t (&p)[3]) {
+    const float ra = __builtin_bit_cast(float, a) - __builtin_bit_cast(float, a & 0xFFFF0000u);
+    const float rb = __builtin_bit_cast(float, b) - __builtin_bit_cast(float, b & 0xFFFF0000u);
+    const uint32_t am = __builtin_bit_cast(uint32_t, ra), bm = __builtin_bit_cast(uint32_t, rb);
+    const float sa = ra - __builtin_bit_cast(float, am & 0xFFFF0000u), sb = rb - __builtin_bit_cast(float, bm & 0xFFFF0000u);
+    p[0] = pack_hi16(a, b), p[1] = pack_hi16(am, bm);
+    p[2] = pack_hi16(__builtin_bit_cast(uint32_t, sa), __builtin_bit_cast(uint32_t, sb));
+}
+__device__ __forceinline__ void ggm_split3(const u32x4_t &v0, const u32x4_t &v1, u32x4_t (&p)[3]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t t[3];
+        ggm_split3_pair(i < 2 ? v0[2 * i] : v1[2 * i - 4], i < 2 ? v0[2 * i + 1] : v1[2 * i - 3], t);
+        p[0][i] = t[0], p[1][i] = t[1], p[2][i] = t[2];
+    }
+}
+
+// XF32: f32 activations and results.  An f32 value is the sum of three bf16 pieces, so four rows of x are twelve rows of
+// a matrix-core tile (piece p of row m in tile row 4 p + m) and the products stay exact; MT tiles take 4 MT rows of x,
+// XQ = 2 MT loads bring them.  The vector-ALU kernel on the rotated copy does the same work once per row.  XQ = 1: a single
+// row, whose chunk the whole wave fetches and splits, two elements a lane.
+template <int FMT, int MT, int XQ, int NW, int NS, bool XF32 = false>
 __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw,
                                                       const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                       float *__restrict__ ws, int M, int K, int N, int cslice, int act) {
+    constexpr bool ONE = XF32 && XQ == 1;
+    static_assert(!XF32 || XQ == 2 * MT || (ONE && MT == 1), "two loads a lane bring four rows' chunk of f32");
+    constexpr int TROWS = XF32 ? 4 * MT : 16 * MT;  // rows of x a tile takes
     typedef BF16Traits TT;
     typedef MfmaOps<TT> Ops;
     typedef GgmFmt<FMT> F;
@@ -469,7 +572,7 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ni = lane & 15, kb = lane >> 4;
     const int j = blockIdx.x;
-    const int m0 = blockIdx.z * ROWS;
+    const int m0 = blockIdx.z * TROWS;
     const int NC = K >> 7;
     const int sc0 = blockIdx.y * cslice;
     const int SC = min(NC, sc0 + cslice) - sc0;
@@ -481,14 +584,16 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
     // the workgroup's NS neighbouring strips behind one descriptor (NS * strip_bytes < 2^31: checked on the host)
     const uint32_t strip_bytes = (uint32_t)(NC / F::CH) * (uint32_t)L::BLKB;
     const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(pw + (size_t)j * NS * strip_bytes, NS * strip_bytes);
-    const int xrows = min(M - m0, ROWS);
-    const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x + (size_t)m0 * K, (uint32_t)xrows * (uint32_t)K * 2u);
+    const int xrows = min(M - m0, TROWS);
+    constexpr int XB = XF32 ? 4 : 2;  // bytes of an element of x
+    const __amdgpu_buffer_rsrc_t rs_x = make_rsrc((const uint8_t *)x + (size_t)m0 * K * XB, (uint32_t)xrows * (uint32_t)K * XB);
     const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);
     int voff_a[AQ];
 #pragma unroll
     for (int q = 0; q < AQ; ++q) {
-        const int r = 4 * q + kb;
-        voff_a[q] = r < xrows ? (r * K * 2 + ni * 16) : OOB;
+        const int r = ONE ? 0 : XF32 ? 4 * (q >> 1) + kb : 4 * q + kb;
+        const int at = ONE ? ni * 32 + kb * 8 : XF32 ? r * K * 4 + ni * 32 + (q & 1) * 16 : r * K * 2 + ni * 16;
+        voff_a[q] = r < xrows ? at : OOB;
     }
     // x in LDS: row r of the tile at r * 256, its sixteen 16-byte pieces XOR-swizzled by the row
     int a_wr[4];
@@ -500,10 +605,11 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
     for (int st = 0; st < NSTEP; ++st)
         a_rd[st] = K16 ? ni * 256 + (((2 * st + (kb >> 1)) ^ ni) << 4) + (kb & 1) * 8 : ni * 256 + (((4 * st + kb) ^ ni) << 4);
     // both masks in registers: v_and_or_b32 takes one literal, and the exponent pattern is it
-    const NibbleMasks nm = FMT == OXQ_GGUF_Q6_K ? NibbleMasks{vgpr_const(0x000F000Fu), vgpr_const(0x00300030u)}
+    const NibbleMasks nm = XF32 ? NibbleMasks{vgpr_const(GgmSmallBias<FMT>::M0), vgpr_const(GgmSmallBias<FMT>::M1)} : FMT == OXQ_GGUF_Q6_K ? NibbleMasks{vgpr_const(0x000F000Fu), vgpr_const(0x00300030u)}
                            : ggm_fifth_bit<FMT> ? NibbleMasks{vgpr_const(0x000F000Fu), vgpr_const(0x00100010u)} : nibble_masks();
 #pragma unroll
-    for (int q = AQ; q < 4 * MT; ++q) {  // rows no call of this instantiation brings stay zero
+    for (int q = XF32 ? 0 : AQ; q < 4 * MT; ++q) {  // rows no call of this instantiation brings stay zero
+        if (XF32 && !ONE && (q & 3) != 3) continue;
         const int row = 4 * q + kb;
         *(u32x4_t *)(slot + row * 256 + ((ni ^ (row & 15)) << 4)) = u32x4_t{0u, 0u, 0u, 0u};
     }
@@ -515,7 +621,14 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
         const __amdgpu_buffer_rsrc_t rx = live ? rs_x : rs_none, rw = live ? rs_w : rs_none;
         const int c = cc0 + i;
 #pragma unroll
-        for (int q = 0; q < AQ; ++q) a[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, voff_a[q], c * 256, 0);
+        for (int q = 0; q < AQ; ++q) {
+            if constexpr (ONE) {
+                const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rx, voff_a[0], c * 512, 0);
+                a[0][0] = v[0], a[0][1] = v[1];
+            } else {
+                a[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, voff_a[q], c * (128 * XB), 0);
+            }
+        }
 #pragma unroll
         for (int f = 0; f < NS; ++f) w[f].request(rw, lane, ni, c, (int)(f * strip_bytes));
         __builtin_amdgcn_sched_barrier(0);  // chunks are requested in the order they are used
@@ -528,7 +641,14 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int f = 0; f < NS; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
-    const uint32_t neg[4] = {F::NEG, F::NEG, F::NEG, F::NEG};
+    constexpr uint32_t NEGP = XF32 ? GgmSmallBias<FMT>::NEG_PAIR : F::NEG;
+    const uint32_t neg[4] = {NEGP, NEGP, NEGP, NEGP};
+    // the minimum's factor is per 128 (factors()); here the bias term is smaller
+    constexpr float MINF = XF32 && C::HAS_MIN ? 128.0f / -GgmSmallBias<FMT>::NEG : 1.0f;
+    auto operand = [&](const C &w, int st, uint32_t (&b)[4], const NibbleMasks &k) {
+        if constexpr (XF32) GgmSmallBias<FMT>::operand(w, st, b, k);
+        else w.operand(st, b, k);
+    };
     const float4_t zero4 = float4_t{0.f, 0.f, 0.f, 0.f};
 
     // A operand of step st, row tile mt
@@ -548,8 +668,23 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 
     auto chunk = [&](int i, auto cur_c, bool more) {
         constexpr int CUR = decltype(cur_c)::value;
+        if constexpr (ONE) {
+            uint32_t part[3];
+            ggm_split3_pair(ar[CUR][0][0], ar[CUR][0][1], part);
 #pragma unroll
-        for (int q = 0; q < AQ; ++q) *(u32x4_t *)(slot + q * 1024 + a_wr[q & 3]) = ar[CUR][q];
+            for (int p = 0; p < 3; ++p) *(uint32_t *)(slot + p * 1024 + ((ni ^ (4 * p)) << 4) + kb * 4) = part[p];
+        } else if constexpr (XF32) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                u32x4_t part[3];
+                ggm_split3(ar[CUR][2 * t], ar[CUR][2 * t + 1], part);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) *(u32x4_t *)(slot + (4 * t + p) * 1024 + a_wr[p]) = part[p];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < AQ; ++q) *(u32x4_t *)(slot + q * 1024 + a_wr[q & 3]) = ar[CUR][q];
+        }
         float f0[NSTEP], f1[NSTEP];
         if constexpr (MT == 1) {
             // what depends on x alone first (x is requested ahead of the chunk's quants): the operands and the
@@ -571,12 +706,12 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 #pragma unroll
                         for (int s4 = 0; s4 < 4; ++s4)
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) acc[0][f][e] = fmaf(f1[g + s4], tn[s4][e], acc[0][f][e]);
+                            for (int e = 0; e < 4; ++e) acc[0][f][e] = fmaf(f1[g + s4] * MINF, tn[s4][e], acc[0][f][e]);
                     }
 #pragma unroll
                     for (int s4 = 0; s4 < 4; ++s4) {
                         uint32_t b[4];
-                        w.operand(g + s4, b, nm);
+                        operand(w, g + s4, b, nm);
                         const float4_t t = mma(a[s4], b, tn[s4]);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) acc[0][f][e] = fmaf(f0[g + s4], t[e], acc[0][f][e]);
@@ -592,7 +727,7 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 #pragma unroll
                 for (int st = 0; st < NSTEP; ++st) {
                     uint32_t b[4];
-                    w.operand(st, b, nm);
+                    operand(w, st, b, nm);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) {
                         uint32_t a[4];
@@ -602,7 +737,7 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             acc[mt][f][e] = fmaf(f0[st], t[e], acc[mt][f][e]);
-                            if constexpr (C::HAS_MIN) acc[mt][f][e] = fmaf(f1[st], tn[e], acc[mt][f][e]);
+                            if constexpr (C::HAS_MIN) acc[mt][f][e] = fmaf(f1[st] * MINF, tn[e], acc[mt][f][e]);
                         }
                     }
                 }
@@ -630,8 +765,9 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
             if (i + 1 < nloc) chunk(i + 1, std::integral_constant<int, 1>{}, false);
         }
     }
-    if (act) ggm_epilogue_act<MT, NS, NW>(acc, bias, y, M, N, j, m0, act, wave, lane);
-    else pk4n_epilogue<TT, MT, NS, NW>(acc, bias, y, ws, M, N, j, m0, wave, lane);
+    if constexpr (XF32) ggm_epilogue_f32<MT, NS, NW>(acc, (const float *)bias, (float *)y, M, N, j, m0, wave, lane);
+    else if (act) ggm_epilogue_act<MT, NS, NW>(acc, bias, y, M, N, j, m0, act, wave, lane);
+    else pk4n_epilogue<TT, MT, NS, NW, true>(acc, bias, y, ws, M, N, j, m0, wave, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -646,11 +782,15 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 // fma each (two where a five-bit format has a minimum) from the integer kernel's own factors, and keeps the whole
 // K in its accumulators: one launch, no partial tiles.
 // KS = 4: two waves of 64 columns a workgroup and the four waves of a column group take every fourth chunk, as in
-// pk4_gemm_kernel - the form for 33 to a few hundred rows of a wide layer.
+// pk4_gemm_kernel - the form for 33 to a few hundred rows of a wide layer.  A layer of few columns does not fill the chip
+// with such workgroups: gridDim.y slices of `cslice` chunks each then write their f32 tiles to `part` and a second
+// launch adds them in slice order.  half: a fused gate|up layer without its activation - columns go back to the
+// file's order (ggm_src_row).
 template <int FMT, int MT, int KS>
 __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw,
                                                        const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
-                                                       int M, int K, int N, int NG, int RT, int act) {
+                                                       float *__restrict__ part, int M, int K, int N, int NG, int RT, int act,
+                                                       int cslice, int half) {
     typedef BF16Traits TT;
     typedef MfmaOps<TT> Ops;
     typedef GgmFmt<FMT> F;
@@ -675,14 +815,17 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         rt = (int)blockIdx.x / NG, g = (int)blockIdx.x % NG;
     }
     const int j = g * SPW + ws;  // the wave's 64 columns: strips 4 j .. 4 j + 3
-    const bool live = j < (N >> 6);
+    const int strips = (N + 15) >> 4;
+    const bool live = 4 * j < strips;
     const int m0 = rt * ROWS;
-    const int NC = K >> 7, NR = (NC + KS - 1) / KS;  // chunks; rounds of KS chunks
+    const int NC = K >> 7;
+    const int cbeg = (int)blockIdx.y * cslice, cend = min(NC, cbeg + cslice);  // the slice's chunks
+    const int NR = (cend - cbeg + KS - 1) / KS;                                // rounds of KS chunks
     const int xrows = min(M - m0, ROWS);
 
     const uint32_t strip_bytes = (uint32_t)(NC / F::CH) * (uint32_t)L::BLKB;
     const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);
-    const __amdgpu_buffer_rsrc_t rs_wl = make_rsrc(pw + (size_t)(live ? 4 * j : 0) * strip_bytes, 4u * strip_bytes);
+    const __amdgpu_buffer_rsrc_t rs_wl = make_rsrc(pw + (size_t)(live ? 4 * j : 0) * strip_bytes, (uint32_t)min(4, live ? strips - 4 * j : 4) * strip_bytes);
     const __amdgpu_buffer_rsrc_t rs_w = live ? rs_wl : rs_none;
     const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x + (size_t)m0 * K, (uint32_t)xrows * (uint32_t)K * 2u);
     // x: load q of a wave brings rows 4 (XV wave + q) .. + 3 of the chunk, lane l the 16 bytes that belong at
@@ -705,21 +848,21 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
 
     C wr[2][4];
     auto dma_x = [&](int r) {  // round r: the wave's chunk is KS r + kq, its tile of x at kq ROWS 256 of the round's buffer
-        const int i = KS * r + kq;
-        const __amdgpu_buffer_rsrc_t rs = i < NC ? rs_x : rs_none;
+        const int i = cbeg + KS * r + kq;
+        const __amdgpu_buffer_rsrc_t rs = i < cend ? rs_x : rs_none;
 #pragma unroll
         for (int q = 0; q < XV; ++q)
             pk4g_load_lds16(rs, pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256) + (ws * XV + q) * 1024, xo[q], i * 256);
     };
     auto request = [&](int i, C (&w)[4]) {
-        const __amdgpu_buffer_rsrc_t rs = i < NC ? rs_w : rs_none;
+        const __amdgpu_buffer_rsrc_t rs = i < cend ? rs_w : rs_none;
 #pragma unroll
         for (int f = 0; f < 4; ++f) w[f].request(rs, lane, ni, i, (int)(f * strip_bytes));
     };
 
     dma_x(0);
     __builtin_amdgcn_sched_barrier(0);  // requests keep this order: the wait counts rely on it
-    request(kq, wr[0]);
+    request(cbeg + kq, wr[0]);
     __builtin_amdgcn_sched_barrier(0);
     float4_t acc[MT][4];
 #pragma unroll
@@ -731,7 +874,7 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
 
     auto chunk = [&](int r, auto cur_c) {
         constexpr int CUR = decltype(cur_c)::value;
-        const int i = KS * r + kq;  // past NC (a ragged last round): zeros from both streams
+        const int i = cbeg + KS * r + kq;  // past the slice (a ragged last round): zeros from both streams
         dma_x(r + 1);
         __builtin_amdgcn_sched_barrier(0);
         request(i + KS, wr[CUR ^ 1]);
@@ -846,12 +989,12 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         // Fused gate|up layer (ggm_src_row): strip 4 j + f holds gate columns 8 (4 j + f) .. + 7 in lanes ni < 8 and
         // the up columns they meet in lanes ni + 8.  The two lanes of a pair exchange their four values (row_ror:8)
         // and finish two outputs each; both factors rounded to bf16 first, as in ggm_epilogue_act.  y is [M, N / 2].
-        const int half = N >> 1, p = ni & 7;
+        const int hc = N >> 1, p = ni & 7;
         const bool low = ni < 8;
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
         if (bias) {
 #pragma unroll
-            for (int f = 0; f < 4; ++f) bv[f] = TT::to_f32(bias[(low ? 0 : half) + 8 * (4 * j + f) + p]);
+            for (int f = 0; f < 4; ++f) bv[f] = TT::to_f32(bias[(low ? 0 : hc) + 8 * (4 * j + f) + p]);
         }
 #pragma unroll
         for (int t = 0; t < FT; ++t)
@@ -869,16 +1012,35 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
                     const int f = low ? q : 2 + q;
                     const float gq = low ? mine[q] : other[2 + q], uq = low ? other[q] : mine[2 + q];
                     const uint16_t o = TT::from_f32(mul_f32_rn(act == 1 ? silu_f32(gq) : gelu_tanh_f32(gq), uq));
-                    if (row < M) y[(size_t)row * half + 8 * (4 * j + f) + p] = o;
+                    if (row < M) y[(size_t)row * hc + 8 * (4 * j + f) + p] = o;
                 }
             }
         return;
     }
-    // row 16 mt + 4 kb + e, column 64 j + 16 f + ni
+    // row 16 mt + 4 kb + e, column 64 j + 16 f + ni (of the copy)
+    int col[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        const int c = 64 * j + 16 * f + ni;
+        col[f] = c < N ? ggm_src_row(c, half) : -1;
+    }
+    if (gridDim.y > 1) {
+#pragma unroll
+        for (int t = 0; t < FT; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
+                if (row >= M) continue;
+#pragma unroll
+                for (int f = 0; f < 4; ++f)
+                    if (col[f] >= 0) part[((size_t)blockIdx.y * M + row) * N + col[f]] = fin[t][f][e];
+            }
+        return;
+    }
     float bv[4] = {0.f, 0.f, 0.f, 0.f};
     if (bias) {
 #pragma unroll
-        for (int f = 0; f < 4; ++f) bv[f] = TT::to_f32(bias[64 * j + 16 * f + ni]);
+        for (int f = 0; f < 4; ++f) bv[f] = col[f] >= 0 ? TT::to_f32(bias[col[f]]) : 0.f;
     }
 #pragma unroll
     for (int t = 0; t < FT; ++t)
@@ -887,7 +1049,8 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
             const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
             if (row >= M) continue;
 #pragma unroll
-            for (int f = 0; f < 4; ++f) y[(size_t)row * N + 64 * j + 16 * f + ni] = TT::from_f32(fin[t][f][e] + bv[f]);
+            for (int f = 0; f < 4; ++f)
+                if (col[f] >= 0) y[(size_t)row * N + col[f]] = TT::from_f32(fin[t][f][e] + bv[f]);
         }
 }
 
@@ -913,12 +1076,29 @@ static const char *ggm_name(int q) {
 
 bool gguf_mfma_eligible(const oxq_ctx *ctx, int quant, int64_t K, int64_t N) {
     if (!ggm_format(quant) || tune(ctx, OXQ_TUNE_GGUF_MFMA, 1) == 0) return false;
-    return gguf_res_eligible(quant, K, N);  // the same strips, chunks and 32-bit offsets
+    // Rows that end inside a strip of 16 (a tensor-parallel shard, a padded vocabulary): from 2^20 weights on; below
+    // the file-layout kernels take a launch's time as well.
+    if (N % 16 != 0 && N * K < (1 << 20)) return false;
+    return gguf_res_eligible(quant, K, (N + 15) & ~(int64_t)15);  // the same strips, chunks and 32-bit offsets
 }
+// Whether a layer of these activations holds the matrix-core copy.  bf16: always where it exists.  f32: from 2^20
+// weights, beside the rotated copy of the vector GEMV; on smaller layers that one takes a launch's time.
+bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int act_dtype) {
+    return gguf_mfma_eligible(ctx, quant, K, N) && (act_dtype == OXQ_BF16 || (act_dtype == OXQ_F32 && N * K >= (1 << 20)));
+}
+// f32 rows of a layer that has both copies: the vector GEMV's arithmetic grows with the rows and is slow on many short
+// strips; the matrix cores take four rows as one.  us on the rotated / the matrix-core copy, Q4_K, 1 / 2 / 4 / 8 rows:
+// 4096 x 4096 4.2 / 5.0 / 6.5 / 12.7 against 4.5 / 5.2 / 5.5 / 7.8, 14336 x 4096 10.7 / 13.3 / 17.8 / 35.2 against 10.0 / 11.7 /
+// 11.7 / 19.2, 2048 x 8192 6.5 / 8.0 / 10.9 / 21.2 against 4.7 / 5.1 / 5.3 / 7.2 (Q6_K: 7.1 / 8.7 against 7.2 / 7.3).
+bool gguf_f32_on_mfma(const oxq_ctx *ctx, int64_t M, int64_t K, int64_t N) {
+    const bool many = ceil_div(N, (int64_t)16) > (ctx->num_cus > 0 ? ctx->num_cus : 256);
+    return M >= 3 || (M == 2 ? many || K >= 8192 : many && K <= 2048);
+}
+size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N) { return gguf_res_bytes(quant, K, (N + 15) & ~(int64_t)15); }
 
 int launch_gguf_mfma_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_t *w, void *pw, int64_t K, int64_t N,
                             int64_t gate_half) {
-    const size_t threads = (size_t)(N / 16) * (K / 128) * 64;
+    const size_t threads = (size_t)ceil_div(N, 16) * (K / 128) * 64;
     dim3 grid((unsigned)ceil_div((int64_t)threads, 256)), block(256);
     char name[64];
     snprintf(name, sizeof name, "gguf_%s_mfma_repack", ggm_name(quant));
@@ -941,7 +1121,7 @@ int launch_gguf_mfma_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_
 
 int launch_gguf_mfma_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void *pw, int64_t K, int64_t N, float *out_nk,
                              int64_t gate_half) {
-    const size_t threads = (size_t)(N / 16) * (K / 128) * 64;
+    const size_t threads = (size_t)ceil_div(N, 16) * (K / 128) * 64;
     dim3 grid((unsigned)ceil_div((int64_t)threads, 256)), block(256);
     char name[64];
     snprintf(name, sizeof name, "gguf_%s_mfma_dequant", ggm_name(quant));
@@ -972,6 +1152,26 @@ static int ggm_go(hipStream_t s, dim3 grid, const GgufProblem &p, float *ws, int
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
+template <int FMT, int MT, int XQ, int NW, int NS>
+static int ggm_f32_go(hipStream_t s, dim3 grid, const GgufProblem &p, int cslice) {
+    static LdsGrant lds_grant;
+    const size_t lds = (size_t)NW * MT * 4096;
+    OXQ_HIP_CHECK(lds_grant.ensure((const void *)ggm_kernel<FMT, MT, XQ, NW, NS, true>, lds));
+    hipLaunchKernelGGL((ggm_kernel<FMT, MT, XQ, NW, NS, true>), grid, dim3(NW * 64), lds, s, (const uint16_t *)p.x, p.w,
+                       (const uint16_t *)p.bias, (uint16_t *)p.y, nullptr, (int)p.M, (int)p.K, (int)p.N, cslice, 0);
+    OXQ_HIP_CHECK(hipGetLastError());
+    return OXQ_OK;
+}
+template <int FMT>
+static int ggm_f32_by_shape(hipStream_t s, dim3 grid, const GgufProblem &p, int cslice, int mt, int ns) {
+    if (ns == 4) {
+        if (p.M == 1) return ggm_f32_go<FMT, 1, 1, 8, 4>(s, grid, p, cslice);
+        return mt == 2 ? ggm_f32_go<FMT, 2, 4, 8, 4>(s, grid, p, cslice) : ggm_f32_go<FMT, 1, 2, 8, 4>(s, grid, p, cslice);
+    }
+    if (mt == 2) return ggm_f32_go<FMT, 2, 4, 8, 1>(s, grid, p, cslice);
+    return p.M == 1 ? ggm_f32_go<FMT, 1, 1, 8, 1>(s, grid, p, cslice) : ggm_f32_go<FMT, 1, 2, 8, 1>(s, grid, p, cslice);
+}
+
 template <int FMT>
 static int ggm_by_shape(hipStream_t s, dim3 grid, const GgufProblem &p, float *ws, int cslice, int mt, int xq, int nw, int ns) {
     if (ns == 4) {  // 8 waves: four strips' quants in flight take the registers of two waves of a 16-wave workgroup
@@ -996,13 +1196,15 @@ static int ggm_by_shape(hipStream_t s, dim3 grid, const GgufProblem &p, float *w
 // as 896 of 16 do not (three and a half rounds).
 static int ggm_strips(const oxq_ctx *ctx, int64_t N) {
     const int v = tune(ctx, OXQ_TUNE_GGUF_MFMA_NS, 0);
-    if (v == 1 || v == 4) return (N / 16) % v == 0 ? v : 1;
-    return (N / 16 >= 768 && (N / 16) % 4 == 0) ? 4 : 1;
+    const int64_t strips = ceil_div(N, 16);
+    if (v == 1 || v == 4) return strips % v == 0 ? v : 1;
+    return (strips >= 768 && strips % 4 == 0) ? 4 : 1;
 }
 
 // rows of x a launch of the matrix-core kernel takes (more go to the tile matmul on the file layout)
 bool gguf_mfma_takes(const oxq_ctx *ctx, int64_t M, int64_t, int act_dtype) {
-    return act_dtype == OXQ_BF16 && M >= 1 && M <= std::min<int64_t>(32, tune(ctx, OXQ_TUNE_GGUF_MFMA_MAX_M, 32));
+    if (act_dtype == OXQ_F32) return M >= 1;  // row tiles of eight: there is no other kernel for more f32 rows
+    return act_dtype == OXQ_BF16 && M >= 1 && M <= tune(ctx, OXQ_TUNE_GGUF_MFMA_MAX_M, 32);
 }
 
 // p.w is the matrix-core copy; p.act: 0, or 1 + the gated activation of a fused gate|up layer, whose y is [M, N / 2].
@@ -1010,118 +1212,197 @@ bool gguf_mfma_takes(const oxq_ctx *ctx, int64_t M, int64_t, int act_dtype) {
 // callers send such calls elsewhere where they can).
 
 int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
+    const bool f32 = p.act_dtype == OXQ_F32;
+    const int tile = f32 ? 4 : 16;  // rows of x a matrix-core tile takes
     const int ns = ggm_strips(ctx, p.N);
-    const int mt = p.M > 16 ? 2 : 1;
-    const int rows = (int)std::min<int64_t>(p.M, 16 * mt);
+    const int mt = p.M > tile ? 2 : 1;
+    const int rows = (int)std::min<int64_t>(p.M, tile * mt);
     const int xq = rows <= 4 ? 1 : rows <= 8 ? 2 : 4;
     // 16 waves split a strip's chunks where that leaves a wave two to three of them; from 64 chunks on 8 waves with
     // twice the run each measured 3 - 8 % faster (8192 x 4096 at one row, Q4_0 / Q4_K / Q6_K: 5.38 / 5.89 / 7.61
     // against 5.87 / 6.30 / 8.11 us).  Two row tiles or four strips need more than the 128 registers a wave of a
     // 16-wave workgroup has.
     const int64_t chunks = p.K / 128;
-    const int nw = (chunks < 16 || chunks >= 64 || mt == 2 || ns == 4 || tune(ctx, OXQ_TUNE_GGR_WAVES, 16) == 8) ? 8 : 16;
-    dim3 grid((unsigned)(p.N / (16 * ns)), 1, (unsigned)ceil_div(p.M, (int64_t)16 * mt));
+    // 16-wave workgroups are one a CU: more strips than CUs would take a second round of them (2048 x 8192 at one row
+    // of bf16 / f32, Q4_K: 6.3 / 6.1 -> 4.4 / 4.7 us).  f32 rows: 8 waves are as fast or faster everywhere.
+    const bool one_round = ceil_div(p.N, (int64_t)16) <= (ctx->num_cus > 0 ? ctx->num_cus : 256);
+    const int nw = (chunks < 16 || chunks >= 64 || mt == 2 || ns == 4 || f32 || !one_round || tune(ctx, OXQ_TUNE_GGR_WAVES, 16) == 8) ? 8 : 16;
+    dim3 grid((unsigned)ceil_div(p.N, (int64_t)16 * ns), 1, (unsigned)ceil_div(p.M, (int64_t)tile * mt));
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_mfma_bf16_mt%d%s%s", ggm_name(p.quant), mt, ns == 4 ? "_n64" : "", p.act ? "_act" : "");
+    if (f32) snprintf(name, sizeof name, "gguf_%s_res_gemv_f32_mfma_mt%d%s", ggm_name(p.quant), mt, ns == 4 ? "_n64" : "");
+    else if (p.M > 32 && !p.act) snprintf(name, sizeof name, "gguf_%s_mul_mm_bf16_mt%d_res_int%s", ggm_name(p.quant), mt, ns == 4 ? "_n64" : "");
+    else snprintf(name, sizeof name, "gguf_%s_mfma_bf16_mt%d%s%s", ggm_name(p.quant), mt, ns == 4 ? "_n64" : "", p.act ? "_act" : "");
     set_plan(ctx, name, grid, dim3(nw * 64), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
-    if (p.act_dtype != OXQ_BF16) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: activations must be BF16");
+    if (!f32 && p.act_dtype != OXQ_BF16) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: activations must be BF16 or F32");
+    if (f32 && p.act) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: a fused activation needs BF16");
     if ((uintptr_t)p.x & 15) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: x must be 16-byte aligned");
     if ((uint64_t)16 * mt * (uint64_t)p.K * 2 >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: K too large");
+    if (grid.z > 65535) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: m = %lld exceeds the grid", (long long)p.M);
     if (gguf_res_bytes(p.quant, p.K, 16) * (uint64_t)ns >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: K too large");
     const int cslice = (int)(p.K / 128);
+#define OXQ_GGM(F) \
+    case F: return f32 ? ggm_f32_by_shape<F>(s, grid, p, cslice, mt, ns) : ggm_by_shape<F>(s, grid, p, nullptr, cslice, mt, xq, nw, ns)
     switch (p.quant) {
-    case OXQ_GGUF_Q4_0: return ggm_by_shape<OXQ_GGUF_Q4_0>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
-    case OXQ_GGUF_Q8_0: return ggm_by_shape<OXQ_GGUF_Q8_0>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
-    case OXQ_GGUF_Q4_K: return ggm_by_shape<OXQ_GGUF_Q4_K>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
-    case OXQ_GGUF_Q6_K: return ggm_by_shape<OXQ_GGUF_Q6_K>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
-    case OXQ_GGUF_Q4_1: return ggm_by_shape<OXQ_GGUF_Q4_1>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
-    case OXQ_GGUF_Q5_0: return ggm_by_shape<OXQ_GGUF_Q5_0>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
-    case OXQ_GGUF_Q5_1: return ggm_by_shape<OXQ_GGUF_Q5_1>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
-    case OXQ_GGUF_Q5_K: return ggm_by_shape<OXQ_GGUF_Q5_K>(s, grid, p, nullptr, cslice, mt, xq, nw, ns);
+        OXQ_GGM(OXQ_GGUF_Q4_0);
+        OXQ_GGM(OXQ_GGUF_Q8_0);
+        OXQ_GGM(OXQ_GGUF_Q4_K);
+        OXQ_GGM(OXQ_GGUF_Q6_K);
+        OXQ_GGM(OXQ_GGUF_Q4_1);
+        OXQ_GGM(OXQ_GGUF_Q5_0);
+        OXQ_GGM(OXQ_GGUF_Q5_1);
+        OXQ_GGM(OXQ_GGUF_Q5_K);
     default: return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: format %d", p.quant);
     }
+#undef OXQ_GGM
 }
 
-// Rows from which a bf16 layer's matrix-core copy runs the prefill kernel instead of the tile matmul on the file
-// layout (gguf_mm: a workgroup of 64 rows x 64 columns with K slices), and in which form: 1 = eight waves of 64
-// columns a workgroup, 4 = two, with K split across the waves inside (0: the file layout).  Costs in rounds of 256
-// workgroups of 64 rows x 512 columns (one a CU: 154 - 210 registers), as for the packed layers (pk4_gemm_form): a
-// last round that fills at most three quarters of the CUs costs 0.95; a round of the two-wave form GGM_MID_ROUND
-// (25 - 35 us against 82 - 120 at K = 4096); the file-layout tile matmul 0.17 + 1.45 w (1.3 w for the five- and
-// six-bit formats, whose conversion weighs on the prefill kernel too): two launches or a latency floor, then about
-// two thirds of a full round's rate.  Fitted to 4096 x 4096, 4096 x 14336 and 14336 x 4096 at
-// 64 - 4096 rows.  OXQ_GGUF_GEMM_MIN_M: unset = by cost, 0 = never, n = the eight-wave form from n rows on whatever
-// the cost; OXQ_GGUF_GEMM_KS = 4 | 1: always | never the two-wave form.
-constexpr double GGM_MID_ROUND = 0.31;
-static int gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int64_t N, int act_dtype) {
-    const int64_t v = tune(ctx, OXQ_TUNE_GGUF_GEMM_MIN_M, -1);
-    if (v == 0 || act_dtype != OXQ_BF16 || !ggm_format(quant) || M <= 32 || N % 64 != 0) return 0;
-    const int ks = tune(ctx, OXQ_TUNE_GGUF_GEMM_KS, 0);
-    if (ks == 4) return 4;
-    if (v > 0) return M >= v ? 1 : 0;
-    const bool light = quant == OXQ_GGUF_Q4_0 || quant == OXQ_GGUF_Q4_1 || quant == OXQ_GGUF_Q4_K || quant == OXQ_GGUF_Q8_0;
-    const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-    const int64_t row_tiles = ceil_div(M, (int64_t)64);
-    const double w64 = (double)(ceil_div(N / 64, (int64_t)8) * row_tiles) / cus;
-    const double whole = std::floor(w64), rest = w64 - whole;
-    const double c64 = whole + (rest <= 0.0 ? 0.0 : rest <= 0.75 ? 0.95 : 1.0);
-    const double c_mid = ks == 1 ? 1e30 : std::ceil((double)(ceil_div(N / 64, (int64_t)2) * row_tiles) / cus) * GGM_MID_ROUND;
-    // (Q8_0's 34-byte blocks make the file layout's matmul 1.2 - 1.35 x the 4-bit formats' at the same shape)
-    const double c_file = 0.17 + (quant == OXQ_GGUF_Q8_0 ? 1.75 : light ? 1.45 : 1.3) * w64;
-    if (c_file <= c64 && c_file <= c_mid) return 0;
-    return c_mid < c64 ? 4 : 1;
+// How a bf16 layer's matrix-core copy runs more rows than one launch of the integer kernel's two row tiles takes (33 and
+// more): ks = 1 | 4: the prefill kernel, eight | two waves of 64 columns a workgroup (4: K split inside it, and over
+// `slices` workgroups); ks = -1: the integer kernel in row tiles of 32; 0: the tile matmul on the file layout (gguf_mm).
+//
+// From 2^20 weights the cheapest of these by estimate, in us (fitted on one box to 4096 x 4096, 14336 x 4096, 5120 x
+// 1408, 3072 x 7424, 2048 x 1024, 4096 x 14336 and 4096 x 28672 at 33 - 512 rows in Q4_K, Q6_K and Q8_0):
+//   integer row tiles   2.6 + chunks a wave x `chunk` x rounds of 256 workgroups (four strips each: 2.5 x).  Ahead where the
+//                       tiles fit one round: 2048 x 1024 at 128 rows 9.7 -> 5.3 us, 5120 x 1408 at 64 rows 12.0 -> 10.5
+//   two waves           rounds of workgroups x (4.5 + K rounds of four chunks x `round`), and with K slices a second launch of
+//                       3.5 us + the partials' bytes at 4.2 TB/s.  14336 x 4096 Q4_K at 33 / 128 / 256 rows 31.8 / 57.8 / 86 ->
+//                       20.9 / 30.7 / 53 us (7, 4 and 2 slices), 4096 x 14336 at 64 rows 28.5 -> 23.5 (2 slices)
+//   eight waves         rounds of workgroups (a last one on at most three quarters of the CUs 0.95) x chunks x `wide` + 5
+// The file layout's matmul is not ahead of all of these there.  Smaller layers compare it with the unsliced forms only, in
+// rounds of 256 workgroups of 64 rows x 512 columns: 0.17 + 1.45 w (1.3 w for the five- and six-bit formats).
+// OXQ_GGUF_GEMM_MIN_M: unset = by cost, 0 = never, n = the eight-wave form from n rows on whatever the cost;
+// OXQ_GGUF_GEMM_KS = 4 | 1: always | never the two-wave form; OXQ_GGUF_GEMM_SLICES = n: that many slices of it.
+struct GgmGemmForm {
+    int ks, slices;
+};
+struct GgmCost {
+    double chunk, round, wide;
+};
+static GgmCost ggm_cost(int quant) {
+    switch (quant) {
+    case OXQ_GGUF_Q4_0: case OXQ_GGUF_Q4_1: case OXQ_GGUF_Q4_K: return {1.45, 2.9, 2.6};
+    case OXQ_GGUF_Q8_0: return {1.6, 2.9, 2.9};
+    case OXQ_GGUF_Q6_K: return {1.75, 4.0, 3.75};
+    default: return {1.6, 4.1, 4.0};  // Q5_0, Q5_1, Q5_K
+    }
 }
-bool gguf_gemm_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
-    (void)K;
-    return gguf_gemm_form(ctx, quant, M, N, act_dtype) != 0;
+static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
+    const int64_t v = tune(ctx, OXQ_TUNE_GGUF_GEMM_MIN_M, -1);
+    if (v == 0 || act_dtype != OXQ_BF16 || !ggm_format(quant) || M <= 32) return {0, 1};
+    const int ks = tune(ctx, OXQ_TUNE_GGUF_GEMM_KS, 0);
+    if (ks == 4) return {N % 64 == 0 ? 4 : 0, 1};
+    if (v > 0) return {N % 64 == 0 && M >= v ? 1 : 0, 1};
+    const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    const int64_t row_tiles = ceil_div(M, (int64_t)64), groups = ceil_div(N, (int64_t)64), chunks = K / 128;
+    const double w64 = (double)(ceil_div(groups, (int64_t)8) * row_tiles) / cus;
+    const double whole = std::floor(w64), rest = w64 - whole;
+    const double r64 = whole + (rest <= 0.0 ? 0.0 : rest <= 0.75 ? 0.95 : 1.0);
+    const int64_t mid_wgs = ceil_div(groups, (int64_t)2) * row_tiles;
+    if (N * K < (1 << 20)) {
+        if (N % 64 != 0) return {0, 1};
+        const bool light = quant == OXQ_GGUF_Q4_0 || quant == OXQ_GGUF_Q4_1 || quant == OXQ_GGUF_Q4_K || quant == OXQ_GGUF_Q8_0;
+        const double c_mid = ks == 1 ? 1e30 : std::ceil((double)mid_wgs / cus) * 0.31;
+        // (Q8_0's 34-byte blocks make the file layout's matmul 1.2 - 1.35 x the 4-bit formats' at the same shape)
+        const double c_file = 0.17 + (quant == OXQ_GGUF_Q8_0 ? 1.75 : light ? 1.45 : 1.3) * w64;
+        if (c_file <= std::min(r64, c_mid)) return {0, 1};
+        return {c_mid < r64 ? 4 : 1, 1};
+    }
+    const GgmCost c = ggm_cost(quant);
+    GgmGemmForm best = {1, 1};
+    double least = r64 * ((double)chunks * c.wide + 5.0);
+    if (ks != 1) {
+        const int64_t given = tune(ctx, OXQ_TUNE_GGUF_GEMM_SLICES, 0);
+        const int64_t most = N % 4 == 0 ? std::min<int64_t>(ceil_div(chunks, (int64_t)4), 64) : 1;  // (the second launch adds four columns a thread)
+        for (int64_t S = 1; S <= most; ++S) {
+            if (given > 0 && S != std::min(given, most)) continue;
+            const int64_t rounds = ceil_div(ceil_div(chunks, S), (int64_t)4);
+            if (ceil_div(chunks, 4 * rounds) != S || (S > 1 && (uint64_t)(S * M) * (uint64_t)N * 4 > ctx->workspace_bytes)) continue;
+            double t = std::ceil((double)(mid_wgs * S) / cus) * (4.5 + (double)rounds * c.round);
+            if (S > 1) t += 3.5 + ((double)S * 8.0 + 2.0) * (double)M * (double)N / 4.2e6;
+            if (t < least || given > 0) least = given > 0 ? 0.0 : t, best = {4, (int)S};
+        }
+    }
+    const int ns = ggm_strips(ctx, N);
+    const double int_wgs = (double)(ceil_div(N, (int64_t)16 * ns) * ceil_div(M, (int64_t)32));
+    const double int_rounds = std::ceil(int_wgs / cus);
+    if (2.6 + (double)ceil_div(chunks, (int64_t)8) * c.chunk * (ns == 4 ? 2.5 : 1.0) * (int_rounds > 1.0 ? 1.15 * int_rounds : 1.0) < least) best = {-1, 1};
+    return best;
+}
+// sliced: whether the caller can take the form whose partial sums a second launch adds (a fused activation cannot)
+bool gguf_gemm_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype, bool sliced) {
+    const GgmGemmForm f = gguf_gemm_form(ctx, quant, M, K, N, act_dtype);
+    return f.ks > 0 && (sliced || f.slices == 1);
+}
+// rows beyond gguf_mfma_takes that the integer kernel takes in row tiles
+bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
+    return gguf_gemm_form(ctx, quant, M, K, N, act_dtype).ks < 0;
 }
 
 template <int FMT, int KS>
-static int ggm_gemm_go(hipStream_t s, dim3 grid, const GgufProblem &p, int NG, int RT) {
+static int ggm_gemm_go(hipStream_t s, dim3 grid, const GgufProblem &p, float *part, int NG, int RT, int cslice) {
     static LdsGrant grant;  // one per instantiation
     constexpr int MT = 4;
     const size_t lds = (size_t)2 * KS * 16 * MT * 256;
     OXQ_HIP_CHECK(grant.ensure((const void *)ggm_gemm_kernel<FMT, MT, KS>, lds));
     hipLaunchKernelGGL((ggm_gemm_kernel<FMT, MT, KS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w, (const uint16_t *)p.bias,
-                       (uint16_t *)p.y, (int)p.M, (int)p.K, (int)p.N, NG, RT, p.act);
+                       (uint16_t *)p.y, part, (int)p.M, (int)p.K, (int)p.N, NG, RT, p.act, cslice, (int)p.gate_half);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
 template <int FMT>
-static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, int NG, int RT, int ks) {
-    return ks == 4 ? ggm_gemm_go<FMT, 4>(s, grid, p, NG, RT) : ggm_gemm_go<FMT, 1>(s, grid, p, NG, RT);
+static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, float *part, int NG, int RT, int ks, int cslice) {
+    return ks == 4 ? ggm_gemm_go<FMT, 4>(s, grid, p, part, NG, RT, cslice) : ggm_gemm_go<FMT, 1>(s, grid, p, part, NG, RT, cslice);
 }
 
-// p.w is the matrix-core copy; p.act as for launch_gguf_mfma
+// p.w is the matrix-core copy; p.act as for launch_gguf_mfma; p.gate_half: the copy of a fused gate|up layer whose
+// activation this call leaves out
 int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     const int rows = 64;
-    int ks = gguf_gemm_form(ctx, p.quant, p.M, p.N, p.act_dtype);
-    if (ks == 0) ks = 1;  // a caller that asks for this kernel gets it
-    const int spw = 8 / ks;
-    const int64_t NG = ceil_div(p.N / 64, (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows);
+    GgmGemmForm form = gguf_gemm_form(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);
+    if (form.ks <= 0) form = {1, 1};  // a caller that asks for this kernel gets it
+    if (p.act) form.slices = 1;
+    const int ks = form.ks, spw = 8 / ks;
+    const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)64), (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows);
     const int64_t wgs = ks == 1 ? (RT / 8) * ceil_div(NG, (int64_t)8) * 64 + (RT % 8) * NG : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: m = %lld exceeds the grid", (long long)p.M);
-    dim3 grid((unsigned)wgs);
+    const int64_t chunks = p.K / 128;
+    const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)4) * 4) : (int)chunks;
+    dim3 grid((unsigned)wgs, (unsigned)form.slices);
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%d%s%s", ggm_name(p.quant), rows, spw, ks > 1 ? "k4" : "",
-             p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
-    set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
-    if (ctx->plan_only) return OXQ_OK;
+    if (form.slices > 1 && p.M <= 128)  // the rows of the file layout's tile matmul
+        snprintf(name, sizeof name, "gguf_%s_mul_mm_bf16_mt4_res_x%dk4s%d", ggm_name(p.quant), spw, form.slices);
+    else if (form.slices > 1)
+        snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%dk4_s%d", ggm_name(p.quant), rows, spw, form.slices);
+    else
+        snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%d%s%s", ggm_name(p.quant), rows, spw, ks > 1 ? "k4" : "",
+                 p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
+    set_plan(ctx, name, grid, dim3(512), form.slices, 1, form.slices > 1 ? (size_t)form.slices * p.M * p.N * 4 : 0);
+    if (ctx->plan_only) {
+        if (form.slices > 1) add_launch(ctx);
+        return OXQ_OK;
+    }
     if (p.act_dtype != OXQ_BF16) return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: activations must be BF16");
     if ((uint64_t)rows * (uint64_t)p.K * 2 >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: K too large");
     if (((uintptr_t)p.x & 15) || ((uintptr_t)p.y & 1)) return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: x must be 16-byte aligned");
+    float *part = (float *)ctx->workspace;
+    int rc;
+#define OXQ_GGM(F) \
+    case F: rc = ggm_gemm_go_form<F>(s, grid, p, part, (int)NG, (int)RT, ks, cslice); break
     switch (p.quant) {
-    case OXQ_GGUF_Q4_0: return ggm_gemm_go_form<OXQ_GGUF_Q4_0>(s, grid, p, (int)NG, (int)RT, ks);
-    case OXQ_GGUF_Q8_0: return ggm_gemm_go_form<OXQ_GGUF_Q8_0>(s, grid, p, (int)NG, (int)RT, ks);
-    case OXQ_GGUF_Q4_K: return ggm_gemm_go_form<OXQ_GGUF_Q4_K>(s, grid, p, (int)NG, (int)RT, ks);
-    case OXQ_GGUF_Q6_K: return ggm_gemm_go_form<OXQ_GGUF_Q6_K>(s, grid, p, (int)NG, (int)RT, ks);
-    case OXQ_GGUF_Q4_1: return ggm_gemm_go_form<OXQ_GGUF_Q4_1>(s, grid, p, (int)NG, (int)RT, ks);
-    case OXQ_GGUF_Q5_0: return ggm_gemm_go_form<OXQ_GGUF_Q5_0>(s, grid, p, (int)NG, (int)RT, ks);
-    case OXQ_GGUF_Q5_1: return ggm_gemm_go_form<OXQ_GGUF_Q5_1>(s, grid, p, (int)NG, (int)RT, ks);
-    case OXQ_GGUF_Q5_K: return ggm_gemm_go_form<OXQ_GGUF_Q5_K>(s, grid, p, (int)NG, (int)RT, ks);
+        OXQ_GGM(OXQ_GGUF_Q4_0);
+        OXQ_GGM(OXQ_GGUF_Q8_0);
+        OXQ_GGM(OXQ_GGUF_Q4_K);
+        OXQ_GGM(OXQ_GGUF_Q6_K);
+        OXQ_GGM(OXQ_GGUF_Q4_1);
+        OXQ_GGM(OXQ_GGUF_Q5_0);
+        OXQ_GGM(OXQ_GGUF_Q5_1);
+        OXQ_GGM(OXQ_GGUF_Q5_K);
     default: return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: format %d has no matrix-core layout", p.quant);
     }
+#undef OXQ_GGM
+    if (rc != OXQ_OK || form.slices == 1) return rc;
+    return launch_splitk_reduce(ctx, s, part, p.bias, p.y, p.M, p.N, form.slices, OXQ_BF16);
 }
 
 }  // namespace oxq

@@ -841,10 +841,14 @@ static bool wcache_forward(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p, i
 // GEMV for f32 (1 - 8 rows).  Entry fields: qw = the block bytes, bits = the ggml format, pack_dim = -1 (rotated) or -2
 // (matrix-core), w.pw = the copy.
 static bool wcache_forward_gguf(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, int *rc) {
-    if (!ctx->wcache_limit || ctx->plan_only || !gguf_res_eligible(p.quant, p.K, p.N)) return false;
-    const bool mfma = p.act_dtype == OXQ_BF16 && gguf_mfma_eligible(ctx, p.quant, p.K, p.N);
+    if (!ctx->wcache_limit || ctx->plan_only) return false;
+    const bool rotated = gguf_res_eligible(p.quant, p.K, p.N);
+    const bool mfma = gguf_mfma_layer(ctx, p.quant, p.K, p.N, p.act_dtype) &&
+                      !(p.act_dtype == OXQ_F32 && rotated && !gguf_f32_on_mfma(ctx, p.M, p.K, p.N));
+    if (!mfma && !rotated) return false;
     const bool gemm = mfma && gguf_gemm_takes(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);  // prefill sizes, same copy
-    if (!gemm && !(mfma ? gguf_mfma_takes(ctx, p.M, p.N, p.act_dtype) : gguf_res_takes(p.K, p.M, p.act_dtype))) return false;
+    const bool tiles = mfma && gguf_mfma_tiles(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);
+    if (!gemm && !tiles && !(mfma ? gguf_mfma_takes(ctx, p.M, p.N, p.act_dtype) : gguf_res_takes(p.K, p.M, p.act_dtype))) return false;
     const int kind = mfma ? -2 : -1;
     if (((uintptr_t)p.x & 15) || ((uintptr_t)p.w & 1)) return false;
     if (!ctx->wcache) {
@@ -866,7 +870,7 @@ static bool wcache_forward_gguf(oxq_ctx *ctx, hipStream_t s, const GgufProblem &
             (void)hipGetLastError();
             return false;
         }
-        const size_t bytes = (gguf_res_bytes(p.quant, p.K, p.N) + 255) & ~(size_t)255;
+        const size_t bytes = ((mfma ? gguf_mfma_bytes(p.quant, p.K, p.N) : gguf_res_bytes(p.quant, p.K, p.N)) + 255) & ~(size_t)255;
         if (!wcache_make_room(ctx, bytes)) return false;
         void *mem = nullptr;
         if (hipMalloc(&mem, bytes) != hipSuccess) {
@@ -1082,9 +1086,9 @@ int oxq_gguf_quant_matmul(oxq_ctx *ctx, void *stream, const oxq_tensor *x,
     // blocks: 10 us for 4096 x 4096 Q4_K), then its prefill kernel, which runs at 1.5 - 1.8 x the tile matmul on the
     // file layout - ahead from about a thousand rows.  Two launches.
     if (!ctx->plan_only && p.act_dtype == OXQ_BF16 && p.M >= 1024 && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
-        gguf_mfma_eligible(ctx, quant, p.K, p.N) && gguf_gemm_takes(ctx, quant, p.M, p.K, p.N, p.act_dtype) &&
+        gguf_mfma_eligible(ctx, quant, p.K, p.N) && gguf_gemm_takes(ctx, quant, p.M, p.K, p.N, p.act_dtype, false) &&
         ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 1) == 0 &&
-        ((gguf_res_bytes(quant, p.K, p.N) + 255) & ~(size_t)255) <= ctx->workspace_bytes) {
+        ((gguf_mfma_bytes(quant, p.K, p.N) + 255) & ~(size_t)255) <= ctx->workspace_bytes) {
         rc = launch_gguf_mfma_repack(ctx, (hipStream_t)stream, quant, p.w, ctx->workspace, p.K, p.N);
         if (rc != OXQ_OK) return rc;
         GgufProblem q = p;
@@ -1109,9 +1113,9 @@ int oxq_gguf_quant_mul_mm(oxq_ctx *ctx, void *stream, const oxq_tensor *x,
     // blocks: 10 us for 4096 x 4096 Q4_K), then its prefill kernel, which runs at 1.5 - 1.8 x the tile matmul on the
     // file layout - ahead from about a thousand rows.  Two launches.
     if (!ctx->plan_only && p.act_dtype == OXQ_BF16 && p.M >= 1024 && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
-        gguf_mfma_eligible(ctx, quant, p.K, p.N) && gguf_gemm_takes(ctx, quant, p.M, p.K, p.N, p.act_dtype) &&
+        gguf_mfma_eligible(ctx, quant, p.K, p.N) && gguf_gemm_takes(ctx, quant, p.M, p.K, p.N, p.act_dtype, false) &&
         ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 1) == 0 &&
-        ((gguf_res_bytes(quant, p.K, p.N) + 255) & ~(size_t)255) <= ctx->workspace_bytes) {
+        ((gguf_mfma_bytes(quant, p.K, p.N) + 255) & ~(size_t)255) <= ctx->workspace_bytes) {
         rc = launch_gguf_mfma_repack(ctx, (hipStream_t)stream, quant, p.w, ctx->workspace, p.K, p.N);
         if (rc != OXQ_OK) return rc;
         GgufProblem q = p;
@@ -2024,20 +2028,25 @@ struct oxq_qlinear {
     int64_t in_features, out_features;
     int quant;
     int out_dtype;
-    void *res = nullptr;    // layer-owned strip-major copy of the blocks
+    void *res = nullptr;    // layer-owned strip-major copies of the blocks, one allocation
     bool resident = false;
-    bool mfma = false;      // the copy is the matrix-core layout (bf16 layers), else the rotated one of the vector GEMV
+    void *rot = nullptr;    // the rotated copy of the vector GEMV, or null
+    void *mm = nullptr;     // the copy in the matrix-core layout, or null (large f32 layers hold both)
+    bool rotated = false, mfma = false;
     int act = 0;            // 0, or 1 + oxq_gated_act of a fused gate|up layer (matrix-core copy only)
 };
 
 // linear.rs:225-240: the fast path copies the block bytes at build; here the copy is strip-major
 static int build_resident_gguf(oxq_qlinear *l) {
     if (tune(l->ctx, OXQ_TUNE_PREPACK, 1) == 0) return OXQ_OK;
-    if (!gguf_res_eligible(l->quant, l->in_features, l->out_features)) return OXQ_OK;
     if (((uintptr_t)l->weight_bytes.data & 1) != 0) return OXQ_OK;
     oxq_ctx *ctx = l->ctx;
-    // a bf16 layer (the reference's GPU path: bf16 x and y) of a format that has it takes the matrix-core layout
-    l->mfma = l->out_dtype == OXQ_BF16 && gguf_mfma_eligible(ctx, l->quant, l->in_features, l->out_features);
+    // a bf16 layer (the reference's GPU path: bf16 x and y) of a format that has it takes the matrix-core layout, an
+    // f32 layer where it is large
+    l->mfma = gguf_mfma_layer(ctx, l->quant, l->in_features, l->out_features, l->out_dtype) &&
+              !(l->act && (l->out_features % 16 != 0 || l->out_dtype != OXQ_BF16));
+    l->rotated = !(l->mfma && l->out_dtype == OXQ_BF16) && gguf_res_eligible(l->quant, l->in_features, l->out_features);
+    if (!l->mfma && !l->rotated) return OXQ_OK;
     if (l->act && !l->mfma) return OXQ_OK;  // the caller reports it
     if (ctx->plan_only) {
         l->resident = true;
@@ -2047,15 +2056,22 @@ static int build_resident_gguf(oxq_qlinear *l) {
     (void)hipGetDevice(&prev);
     OXQ_HIP_CHECK(hipSetDevice(ctx->device));
     int rc = OXQ_OK;
-    hipError_t e = hipMalloc(&l->res, gguf_res_bytes(l->quant, l->in_features, l->out_features));
+    const size_t rot_bytes = l->rotated ? (gguf_res_bytes(l->quant, l->in_features, l->out_features) + 255) & ~(size_t)255 : 0;
+    hipError_t e = hipMalloc(&l->res, rot_bytes + (l->mfma ? gguf_mfma_bytes(l->quant, l->in_features, l->out_features) : 0));
     if (e != hipSuccess) {
         l->res = nullptr;
         rc = fail(OXQ_ERR_RUNTIME, "QLinear: repack allocation failed: %s", hipGetErrorString(e));
     } else {
         const uint8_t *src = (const uint8_t *)l->weight_bytes.data;
-        rc = l->mfma ? launch_gguf_mfma_repack(ctx, nullptr, l->quant, src, l->res, l->in_features, l->out_features,
-                                               l->act ? l->out_features / 2 : 0)
-                     : launch_gguf_res_repack(ctx, nullptr, l->quant, src, l->res, l->in_features, l->out_features);
+        if (l->rotated) {
+            l->rot = l->res;
+            rc = launch_gguf_res_repack(ctx, nullptr, l->quant, src, l->rot, l->in_features, l->out_features);
+        }
+        if (rc == OXQ_OK && l->mfma) {
+            l->mm = (uint8_t *)l->res + rot_bytes;
+            rc = launch_gguf_mfma_repack(ctx, nullptr, l->quant, src, l->mm, l->in_features, l->out_features,
+                                         l->act ? l->out_features / 2 : 0);
+        }
         if (rc == OXQ_OK && (e = hipStreamSynchronize(nullptr)) != hipSuccess)
             rc = fail(OXQ_ERR_RUNTIME, "QLinear: repack failed: %s", hipGetErrorString(e));
     }
@@ -2347,45 +2363,55 @@ int oxq_qlinear_forward(oxq_qlinear *l, void *stream, const oxq_tensor *x, const
                            l->quant, &full, &p));
         if ((uintptr_t)p.x & 15) return fail(OXQ_ERR_UNSUPPORTED, "%s: x must be 16-byte aligned", op);
         p.bias = l->has_bias ? l->bias.data : nullptr;
-        p.w = (const uint8_t *)l->res;
+        p.w = (const uint8_t *)l->mm;
         p.act = l->act;
-        if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype)) return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p);
+        if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype, false) && p.N % 64 == 0)
+            return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p);
         return launch_gguf_mfma(l->ctx, (hipStream_t)stream, p);
     }
     OXQ_TRY(check_gguf(l->ctx, decode ? "GgufQuantMatmul" : "GgufQuantMulMM", decode, false, &x2,
                        &l->weight_bytes, l->in_features, l->out_features, l->quant, &o2, &p));
     p.bias = l->has_bias ? l->bias.data : nullptr;
-    if (l->resident && l->mfma) {
-        if (gguf_mfma_takes(l->ctx, p.M, p.N, p.act_dtype) && ((uintptr_t)p.x & 15) == 0) {
-            p.w = (const uint8_t *)l->res;
-            return launch_gguf_mfma(l->ctx, (hipStream_t)stream, p);
+    if (l->resident && ((uintptr_t)p.x & 15) == 0) {
+        const bool f32_rotated = p.act_dtype == OXQ_F32 && l->rotated && gguf_res_takes(p.K, p.M, p.act_dtype) &&
+                                 !(l->mfma && gguf_f32_on_mfma(l->ctx, p.M, p.K, p.N));
+        if (l->mfma && !f32_rotated) {
+            GgufProblem q = p;
+            q.w = (const uint8_t *)l->mm;
+            if (gguf_mfma_takes(l->ctx, p.M, p.N, p.act_dtype) || gguf_mfma_tiles(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype))
+                return launch_gguf_mfma(l->ctx, (hipStream_t)stream, q);
+            if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype)) return launch_gguf_gemm(l->ctx, (hipStream_t)stream, q);
+        } else if (l->rotated && gguf_res_takes(p.K, p.M, p.act_dtype)) {
+            p.w = (const uint8_t *)l->rot;
+            return launch_gguf_res_gemv(l->ctx, (hipStream_t)stream, p);
         }
-        if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype) && ((uintptr_t)p.x & 15) == 0) {
-            p.w = (const uint8_t *)l->res;
-            return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p);
-        }
-    } else if (l->resident && gguf_res_takes(p.K, p.M, p.act_dtype) && ((uintptr_t)p.x & 15) == 0) {
-        p.w = (const uint8_t *)l->res;
-        return launch_gguf_res_gemv(l->ctx, (hipStream_t)stream, p);
     }
     return qlinear_forward_file_layout(l, stream, p);
 }
 
-// The projection of a fused gate|up layer without its activation, [m, out_features], from the file layout: for
-// callers that hold scratch for it (FeedForward at more rows than the fused kernel should take).
+// The projection of a fused gate|up layer without its activation, [m, out_features], on the kernel the plain layer
+// takes at these rows: for callers that hold scratch for it (FeedForward at more rows than the fused kernel should take).
 static int qlinear_forward_unfused(oxq_qlinear *l, void *stream, const oxq_tensor *x2, const oxq_tensor *gu) {
     GgufProblem p;
     const bool decode = x2->dims[0] >= 1 && x2->dims[0] <= 8;
     OXQ_TRY(check_gguf(l->ctx, decode ? "GgufQuantMatmul" : "GgufQuantMulMM", decode, false, x2, &l->weight_bytes,
                        l->in_features, l->out_features, l->quant, gu, &p));
     p.bias = l->has_bias ? l->bias.data : nullptr;
+    if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype) && ((uintptr_t)p.x & 15) == 0) {  // as the plain layer
+        p.w = (const uint8_t *)l->mm;
+        p.gate_half = p.N / 2;
+        return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p);
+    }
     return qlinear_forward_file_layout(l, stream, p);
 }
 
-// whether `rows` rows of a bf16 layer run the prefill kernel on its matrix-core copy (a fused gate|up layer then
-// keeps its activation in that kernel's epilogue, and the plain layer takes the same kernel: the same bits)
+// whether `rows` rows of a bf16 layer run whole sums on its matrix-core copy, in the prefill kernel or in row tiles of the
+// integer kernel (a fused gate|up layer then keeps its activation in that kernel's epilogue, and the plain layer takes
+// the same kernel: the same bits)
 static bool qlinear_prefill_on_copy(const oxq_qlinear *l, int64_t rows) {
-    return l->resident && l->mfma && gguf_gemm_takes(l->ctx, l->quant, rows, l->in_features, l->out_features, l->out_dtype);
+    if (l->resident && l->mfma && gguf_mfma_tiles(l->ctx, l->quant, rows, l->in_features, l->out_features, l->out_dtype)) return true;
+    return l->resident && l->mfma && l->out_features % 64 == 0 &&
+           gguf_gemm_takes(l->ctx, l->quant, rows, l->in_features, l->out_features, l->out_dtype, false);
 }
 
 int oxq_qlinear_is_resident(const oxq_qlinear *l, int *resident) {
@@ -2402,11 +2428,11 @@ int oxq_qlinear_dequantize(oxq_qlinear *l, void *stream, const oxq_tensor *out) 
         return fail(OXQ_ERR_SHAPE, "%s: out must be F32 [%lld, %lld]", op, (long long)l->out_features,
                     (long long)l->in_features);
     if (!out->contiguous) return fail(OXQ_ERR_CONTIGUOUS, "%s: out must be contiguous", op);
-    if (l->resident && l->mfma)
-        return launch_gguf_mfma_dequant(l->ctx, (hipStream_t)stream, l->quant, l->res, l->in_features, l->out_features,
+    if (l->resident && !l->rotated)
+        return launch_gguf_mfma_dequant(l->ctx, (hipStream_t)stream, l->quant, l->mm, l->in_features, l->out_features,
                                         (float *)out->data, l->act ? l->out_features / 2 : 0);
     if (l->resident)
-        return launch_gguf_res_dequant(l->ctx, (hipStream_t)stream, l->quant, l->res, l->in_features, l->out_features,
+        return launch_gguf_res_dequant(l->ctx, (hipStream_t)stream, l->quant, l->rot, l->in_features, l->out_features,
                                        (float *)out->data);
     GgufProblem p{};
     p.w = (const uint8_t *)l->weight_bytes.data;

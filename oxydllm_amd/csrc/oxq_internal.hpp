@@ -18,7 +18,7 @@
 // call costs no getenv and two engine threads cannot race on the process environment.
 #define OXQ_TUNE_LIST(X)                                                                                      \
     X(ACT_VEC) X(F8_MM_KS) X(F8_MM_MIN_M) X(F8_MM_MT) X(FORCE_GENERIC) X(GEMV_CFG) X(GEMV_GPW) X(GEMV_TILE)   \
-    X(GGR_GRID) X(GGR_WAVES) X(GGUF_BIG_LDS) X(GGUF_GEMM_KS) X(GGUF_GEMM_MIN_M) X(GGUF_MFMA)                  \
+    X(GGR_GRID) X(GGR_WAVES) X(GGUF_BIG_LDS) X(GGUF_GEMM_KS) X(GGUF_GEMM_MIN_M) X(GGUF_GEMM_SLICES) X(GGUF_MFMA)                  \
     X(GGUF_MFMA_MAX_M) X(GGUF_MFMA_NS) X(GGUF_MM_KS) X(GGUF_MM_MIN_M) X(GGUF_MM_MT) X(GGUF_PW) X(GGUF_RPWG)   \
     X(GPTQ_TILE) X(GPTQ_TILE_KS) X(MFMA_MT) X(MFMA_SPLITK) X(MFMA_VARIANT) X(MXFP4_FR) X(MXFP4_GEMM_MIN_PAIRS) \
     X(MXFP4_GEMM_ROWS) X(MXFP4_MM)      \
@@ -144,6 +144,7 @@ struct GgufProblem {
     int quant;
     int act_dtype;          // OXQ_BF16 or OXQ_F32
     int act = 0;            // matrix-core copy of a fused gate|up layer: 1 + the gated activation (y is [M, N / 2])
+    int64_t gate_half = 0;  // such a copy without its activation: N / 2 (y is [M, N] in the file's column order)
 };
 
 struct Mxfp4Problem {
@@ -238,6 +239,10 @@ int launch_gguf_res_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void *
 int launch_gguf_res_gemv(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);  // p.w = the copy
 // matrix-core copy of a GGUF weight for 16-bit activations and its matmul (gguf_mfma.hip)
 bool gguf_mfma_eligible(const oxq_ctx *ctx, int quant, int64_t K, int64_t N);
+bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int act_dtype);
+size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N);
+bool gguf_f32_on_mfma(const oxq_ctx *ctx, int64_t M, int64_t K, int64_t N);
+bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);
 bool gguf_mfma_takes(const oxq_ctx *ctx, int64_t M, int64_t N, int act_dtype);
 int launch_gguf_mfma_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_t *w, void *pw, int64_t K, int64_t N,
                             int64_t gate_half = 0);
@@ -245,7 +250,7 @@ int launch_gguf_mfma_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void 
                              int64_t gate_half = 0);
 int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);  // p.w = the copy
 // the prefill kernel on the same copy (csrc/gguf_mfma.hip: ggm_gemm_kernel)
-bool gguf_gemm_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);
+bool gguf_gemm_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype, bool sliced = true);
 int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);  // p.w = the copy
 bool gguf_mm_eligible(const oxq_ctx *ctx, const GgufProblem &p);
 int launch_gguf_mm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);

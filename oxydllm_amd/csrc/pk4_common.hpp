@@ -317,7 +317,8 @@ __device__ __forceinline__ void pk4_epilogue_lanes(const float4_t (&acc)[MT][4],
 // Strips of 16 columns (the narrow form of pk4.hip, the GGUF matrix-core kernels): the waves' partial tiles meet
 // in LDS as in the wide form; a thread then owns (row, column ni of every strip of the workgroup) and adds the
 // waves in order.
-template <typename TT, int MT, int NS, int NW>
+// RAGGED: columns may end inside the last strip (the narrow form's never do).
+template <typename TT, int MT, int NS, int NW, bool RAGGED = false>
 __device__ __forceinline__ void pk4n_epilogue(const float4_t (&acc)[MT][NS], const uint16_t *__restrict__ bias,
                                               uint16_t *__restrict__ y, float *__restrict__ ws, int M, int N, int j,
                                               int m0, int wave, int lane) {
@@ -353,6 +354,7 @@ __device__ __forceinline__ void pk4n_epilogue(const float4_t (&acc)[MT][NS], con
 #pragma unroll
         for (int f = 0; f < NS; ++f) {
             const int n = 16 * (NS * j + f) + ni;
+            if (RAGGED && n >= N) continue;
             if (gridDim.y > 1) {  // this K slice's f32 partial; a second kernel adds the slices in order
                 ws[((size_t)blockIdx.y * M + (m0 + ml)) * N + n] = v[f];
             } else {

@@ -1,0 +1,91 @@
+"""The matrix-core copy of GGUF layers beyond bf16 decode: f32 activations (three bf16 pieces a value), prefill rows of
+layers of few columns (K slices over workgroups, added by a second launch) and rows that end inside a strip of 16.
+
+f32: against the product in float64.  A value, a weight's integer and their product are exact; what rounds is f32
+addition, at most K / 32 sub-block sums of magnitude amplified by the operand's bias (below 2 x the sums' own), so the
+2-norm error stays under 1e-5 of the result's, which is also what two summation orders of plain f32 may differ by.
+bf16: 2e-3 relative / 1e-2 absolute against the oracle with the weights rounded as the prefill tiles round them."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from oxydllm_amd import ops, synth
+from tests.helpers import assert_close, bits_of, round_x, to_dev, tune
+
+pytestmark = pytest.mark.gpu
+FMTS = [synth.GGUF_Q4_0, synth.GGUF_Q8_0, synth.GGUF_Q4_K, synth.GGUF_Q6_K, synth.GGUF_Q4_1, synth.GGUF_Q5_0,
+        synth.GGUF_Q5_1, synth.GGUF_Q5_K]
+
+
+def say(msg):
+    print(f"[case] {msg}", flush=True)
+    sys.stdout.flush()
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("N,K", [(1024, 1024), (1032, 2304), (144, 8192), (12296, 256)])
+def test_f32_rows_on_the_matrix_core_copy(fmt, N, K):
+    data = synth.gguf_weight(fmt, N, K, seed=N + K + fmt)
+    w = oracle.dequantize_gguf(fmt, data, N, K)
+    bias = np.random.default_rng(N).standard_normal(N).astype(np.float32)
+    layer = ops.QLinear(fmt, to_dev(data), K, N, to_dev(bias), torch.float32)
+    assert layer.resident
+    assert np.array_equal(layer.dequantize().cpu().numpy().view(np.uint32), w.view(np.uint32)), "repack changed a weight"
+    for m in (1, 3, 4, 5, 8, 9, 21):
+        say(f"gguf f32 matrix cores {synth.GGUF_NAMES[fmt]} N={N} K={K} m={m}")
+        x = np.random.default_rng(K + m).standard_normal((m, K)).astype(np.float32)
+        y = layer.forward(to_dev(x))
+        kernel = ops.default_context().last_plan()["kernel"]
+        assert ("_res_gemv_f32_mfma" if m >= 3 or N % 16 else "_res_gemv_f32") in kernel, kernel
+        ref = x.astype(np.float64) @ w.astype(np.float64).T + bias
+        err = np.linalg.norm(y.cpu().numpy() - ref) / np.linalg.norm(ref)
+        assert err < 1e-5, f"{synth.GGUF_NAMES[fmt]} m={m}: {err:.2e}"
+        assert np.array_equal(bits_of(layer.forward(to_dev(x))), bits_of(y)), "run to run"
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("N,K", [(256, 4096), (1032, 2304), (640, 14336), (4100, 1024)])
+def test_prefill_rows_of_few_columns(fmt, N, K):
+    data = synth.gguf_weight(fmt, N, K, seed=N + K + fmt)
+    bias = ((np.arange(N, dtype=np.float32) % 13) - 6) * np.float32(0.25)
+    layer = ops.QLinear(fmt, to_dev(data), K, N, to_dev(bias, torch.bfloat16), torch.bfloat16)
+    assert layer.resident
+    w = oracle.dequantize_gguf(fmt, data, N, K)
+    wr = oracle.round_through(w, oracle.BF16)
+    for m, slices in ((33, None), (64, 2), (65, None), (200, 3), (300, None)):
+        tune("OXQ_GGUF_GEMM_SLICES", slices)
+        x = np.random.default_rng(K + m).standard_normal((m, K)).astype(np.float32)
+        y = layer.forward(to_dev(x, torch.bfloat16))
+        plan = ops.default_context().last_plan()
+        say(f"gguf slices {synth.GGUF_NAMES[fmt]} N={N} K={K} m={m} {plan['kernel']} x {plan['split_k']}")
+        whole = "_res_int" in plan["kernel"]  # row tiles of the integer kernel: the weights unrounded
+        assert plan["launches"] == (2 if plan["split_k"] > 1 else 1) and (slices is None or plan["split_k"] > 1), plan
+        assert whole or "_res_x2k4" in plan["kernel"] or "_gemm_" in plan["kernel"], plan
+        ref = oracle.matmul_nt_f32(round_x(x, oracle.BF16), w if whole else wr, round_x(bias, oracle.BF16))
+        assert_close(y, ref, f"{synth.GGUF_NAMES[fmt]} m={m}", bf16_out=True)
+    for m in (1, 17, 32):  # the integer kernel on a ragged last strip
+        x = np.random.default_rng(m).standard_normal((m, K)).astype(np.float32)
+        ref = oracle.matmul_nt_f32(round_x(x, oracle.BF16), w, round_x(bias, oracle.BF16))
+        assert_close(layer.forward(to_dev(x, torch.bfloat16)), ref, f"m={m}", bf16_out=True)
+
+
+@pytest.mark.parametrize("fmt", [synth.GGUF_Q4_K, synth.GGUF_Q6_K])
+@pytest.mark.parametrize("slices", [2, None])
+def test_ffn_without_room_for_the_fused_activation(fmt, slices):
+    """A gate|up layer of few columns: the projection runs in K slices on the interleaved copy, its columns put back in
+    the file's order, and the activation by itself - the plain layer's bits.  Unforced: row tiles of the integer kernel,
+    the activation in its epilogue, again the plain layer's bits."""
+    tune("OXQ_GGUF_GEMM_SLICES", slices)
+    K, inter, m = 2048, 512, 40
+    say(f"gguf ffn slices {synth.GGUF_NAMES[fmt]}")
+    gu, dn = synth.gguf_weight(fmt, 2 * inter, K, seed=1), synth.gguf_weight(fmt, K, inter, seed=2)
+    fused = ops.QLinear(fmt, to_dev(gu), K, 2 * inter, None, torch.bfloat16, gate_up_act=ops.ACT_GATED_SILU)
+    plain = ops.QLinear(fmt, to_dev(gu), K, 2 * inter, None, torch.bfloat16)
+    down = ops.QLinear(fmt, to_dev(dn), inter, K, None, torch.bfloat16)
+    x = to_dev(np.random.default_rng(3).standard_normal((m, K)).astype(np.float32) * 0.25, torch.bfloat16)
+    want = down.forward(ops.gated_activation(plain.forward(x), ops.ACT_GATED_SILU))
+    got = ops.FeedForward(ops.GATE_UP_FUSED, fused, None, down, inter).forward(x)
+    np.testing.assert_array_equal(bits_of(got), bits_of(want))
