@@ -495,12 +495,15 @@ int launch_mxfp4_mm(oxq_ctx *ctx, hipStream_t s, const Mxfp4Problem &p) {
 }
 
 bool f8_mm_eligible(const oxq_ctx *ctx, const F8Problem &p) {
-    const int min_m = tune(ctx, OXQ_TUNE_F8_MM_MIN_M, 3);  // measured 4096^2 at m = 8: GEMV 19.9 us, tile matmul 11.5 us
+    // The GEMV is the better one for one and two rows of a small matrix only (512 x 768: 2.4 us); from 2^22 weights on the
+    // tiles that read the tensor as matrix-core operands beat it at one row too (5632^2: 11.3 us, tiles 8.2 us)
+    const int min_m = tune(ctx, OXQ_TUNE_F8_MM_MIN_M, p.K * p.N >= (1ll << 22) && f8_direct_takes(ctx, p) ? 1 : 3);
     return p.M >= min_m && p.K % 32 == 0 && p.block_c % 32 == 0 && ((uintptr_t)p.x & 15) == 0 &&
            ((uintptr_t)p.w & 15) == 0;
 }
 
 int launch_f8_mm(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
+    if (!tune_given(ctx, OXQ_TUNE_F8_MM_MT) && !tune_given(ctx, OXQ_TUNE_F8_MM_KS) && f8_direct_takes(ctx, p)) return launch_f8_direct(ctx, s, p);
     MmArgs a = {};
     a.x = (const uint16_t *)p.x, a.w = p.w, a.y = (uint16_t *)p.y;
     a.M = (int)p.M, a.K = (int)p.K, a.N = (int)p.N;

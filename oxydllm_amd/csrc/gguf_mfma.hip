@@ -954,7 +954,13 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
             chunk(r, std::integral_constant<int, 0>{});
             chunk(r + 1, std::integral_constant<int, 1>{});
         }
-        if (r < NR) chunk(r, std::integral_constant<int, 0>{});
+        if (r < NR) {
+            chunk(r, std::integral_constant<int, 0>{});
+            // no weights are requested past this round, so RING counts loads that are not there: the zeros requested for
+            // the round after it must be in LDS before the sum uses the place
+            pk4g_wait_vmcnt<0>();
+            __syncthreads();
+        }
     }
 
     // the finished tile rows of this wave: all of them (KS = 1), or row tile kq summed over the column group's waves

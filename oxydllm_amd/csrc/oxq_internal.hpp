@@ -17,7 +17,7 @@
 // and can be set per ctx with oxq_ctx_set_tuning; the launchers only ever look at the ctx, so a forward
 // call costs no getenv and two engine threads cannot race on the process environment.
 #define OXQ_TUNE_LIST(X)                                                                                      \
-    X(ACT_VEC) X(F8_MM_KS) X(F8_MM_MIN_M) X(F8_MM_MT) X(FORCE_GENERIC) X(GEMV_CFG) X(GEMV_GPW) X(GEMV_TILE)   \
+    X(ACT_VEC) X(F8_FORM) X(F8_MM_KS) X(F8_MM_MIN_M) X(F8_MM_MT) X(F8_SLICES) X(FORCE_GENERIC) X(GEMV_CFG) X(GEMV_GPW) X(GEMV_TILE)   \
     X(GGR_GRID) X(GGR_WAVES) X(GGUF_BIG_LDS) X(GGUF_GEMM_KS) X(GGUF_GEMM_MIN_M) X(GGUF_GEMM_SLICES) X(GGUF_MFMA)                  \
     X(GGUF_MFMA_MAX_M) X(GGUF_MFMA_NS) X(GGUF_MM_KS) X(GGUF_MM_MIN_M) X(GGUF_MM_MT) X(GGUF_PW) X(GGUF_RPWG)   \
     X(GPTQ_TILE) X(GPTQ_TILE_KS) X(MFMA_MT) X(MFMA_SPLITK) X(MFMA_VARIANT) X(MXFP4_FR) X(MXFP4_GEMM_MIN_PAIRS) \
@@ -269,6 +269,8 @@ int launch_rtn_quantize_awq(oxq_ctx *ctx, hipStream_t s, const void *weight, int
 int launch_cast_f8e4m3_f32(oxq_ctx *ctx, hipStream_t s, const uint8_t *in, float *out, size_t n);
 int launch_f8_block_dequant(oxq_ctx *ctx, hipStream_t s, const F8Problem &p, uint16_t *out);
 int launch_f8_gemv(oxq_ctx *ctx, hipStream_t s, const F8Problem &p);
+bool f8_direct_takes(const oxq_ctx *ctx, const F8Problem &p);  // f8_mm.hip: straight from the tensor to the matrix cores
+int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p);
 bool f8_mm_eligible(const oxq_ctx *ctx, const F8Problem &p);
 int launch_f8_mm(oxq_ctx *ctx, hipStream_t s, const F8Problem &p);
 // MXFP4 prefill (plain m > 16, or grouped with many pairs per expert): same tile matmul
