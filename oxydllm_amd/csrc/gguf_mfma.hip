@@ -910,21 +910,17 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
                 uint32_t b[4];
                 const float sc = f0[f][st];
                 if constexpr (NIB) {
-                    // plain nibbles (pair pp = nibble pp of each 16-bit half): masked in place a byte holds q or 16 q,
-                    // which v_cvt_f32_ubyteN widens; one fma a weight
-                    uint32_t tl, th;
-                    pk4g_nibbles(wr[CUR][f].q[0][st], tl, th);
+                    // plain nibbles (pair pp = nibble pp of each 16-bit half)
                     Pk4gBf16 cv;
-                    cv.s = sc, cv.s16 = sc * 0.0625f, cv.c = C::HAS_MIN ? c2[f][st] : (NEGF + 128.0f) * sc;
-                    b[0] = cv.template pair<0, false>(tl), b[1] = cv.template pair<0, true>(th);
-                    b[2] = cv.template pair<1, false>(tl), b[3] = cv.template pair<1, true>(th);
+                    cv.s = sc, cv.c = C::HAS_MIN ? c2[f][st] : (NEGF + 128.0f) * sc;
+                    cv.rows(wr[CUR][f].q[0][st], b);
                 } else if constexpr (FMT == OXQ_GGUF_Q8_0) {
                     // bytes q + 128, elements 0, 2, 1, 3 of a word's four: pairs in bytes (0, 2) and (1, 3)
                     const uint32_t w0 = wr[CUR][f].q[st >> 1][2 * (st & 1)], w1 = wr[CUR][f].q[st >> 1][2 * (st & 1) + 1];
                     Pk4gBf16 cv;
-                    cv.s = sc, cv.s16 = 0.f, cv.c = -128.0f * sc;
-                    b[0] = cv.template pair<0, false>(w0), b[1] = cv.template pair<1, false>(w0);
-                    b[2] = cv.template pair<0, false>(w1), b[3] = cv.template pair<1, false>(w1);
+                    cv.s = sc, cv.c = -128.0f * sc;
+                    b[0] = cv.template bytes<0>(w0), b[1] = cv.template bytes<1>(w0);
+                    b[2] = cv.template bytes<0>(w1), b[3] = cv.template bytes<1>(w1);
                 } else {
                     // bias + q as bf16 (the integer kernel's operand): f0 (bias + q) + NEG f0 is exact in one fma
                     wr[CUR][f].operand(st, b, nm);

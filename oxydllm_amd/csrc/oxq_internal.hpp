@@ -217,7 +217,9 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p);
 int launch_pk4_dequant(oxq_ctx *ctx, hipStream_t s, const Pk4Weights &w, void *out_kn);
 // groups of 32 or 64 rows (pk4_fine.hip): the ring kernel of launch_pk4_forward and the prefill kernel
 int launch_pk4_fine(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p, int bslice, int mt, bool fold);
-int launch_pk4_gemm_fine(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows, int ks, int NG, int RT);
+int launch_pk4_gemm_fine(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows, int NG, int RT);
+// 64 rows x two groups of 64 columns a workgroup, K split inside it (pk4_mid.hip)
+int launch_pk4_mid(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);
 // 49 - 64 rows on a 4-bit layer in 64-column strips (pk4_tile.hip)
 bool pk4_tile64_takes(const Pk4Problem &p, int ks);
 int launch_pk4_tile64(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p);

@@ -501,7 +501,12 @@ __global__ __launch_bounds__(NW * 64) void pk4n_mfma_kernel(const uint16_t *__re
         load_w(i + RD - 1, wr[NXT], zr[ZN]);
         float4_t tmp[GS ? MT : 1][NS], tmp1[GS ? MT : 1], tmpb[(GS && DUAL) ? MT : 1];
         Pk4N<TT> cst[(GS && !EXACT) ? 1 : NS];
-        if (!GS || EXACT) {
+        constexpr bool WIDEN = !GS && TT::DTYPE == BF16Traits::DTYPE;
+        Pk4gBf16 cb[WIDEN ? NS : 1];
+        if constexpr (WIDEN) {
+#pragma unroll
+            for (int f = 0; f < NS; ++f) cb[f].set(__builtin_bit_cast(float, zr[ZC][f] & 0xFFFF0000u), __builtin_bit_cast(float, zr[ZC][f] << 16));
+        } else if (!GS || EXACT) {
 #pragma unroll
             for (int f = 0; f < NS; ++f) cst[f].prep(zr[ZC][f]);
         }
@@ -521,8 +526,9 @@ __global__ __launch_bounds__(NW * 64) void pk4n_mfma_kernel(const uint16_t *__re
                 const uint32_t w = wr[CUR][f][st];
                 uint32_t b[4];
                 if constexpr (!GS && MT == 4) cst[f].odd_from_even();
+                if constexpr (WIDEN) cb[f].rows(w, b);
 #pragma unroll
-                for (int pp = 0; pp < 4; ++pp) {
+                for (int pp = 0; pp < (WIDEN ? 0 : 4); ++pp) {
                     const uint32_t pr = TT::unpack1(w, pp, nm);
                     if constexpr (EXACT) b[pp] = cst[f].minus_zero(pr, pp);
                     else b[pp] = GS ? pr : cst[f].deq(pr, pp);

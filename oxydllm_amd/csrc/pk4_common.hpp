@@ -66,23 +66,47 @@ __device__ __forceinline__ void pk4g_tile_of(int id, int RT, int NG, int &rt, in
     }
 }
 
-// bf16 has no packed 16-bit arithmetic: a weight goes nibble -> f32 -> fma -> (a pair at a time) bf16.  Masked in
-// place, a byte of the word holds q (low nibbles) or 16 q (high nibbles), which v_cvt_f32_ubyteN widens in one
-// instruction; the high nibbles' fma takes s / 16.  (q - z) s is exact in f32 either way: the same bits as
-// Pk4T<BF16Traits>::deq, with a sixth fewer instructions.
+// bf16 has no packed 16-bit arithmetic: a weight goes to f32, through an fma and (a pair at a time) to bf16.
+// (q - z) s is exact in f32, so the bits are those of Pk4T<BF16Traits>::deq.  These kernels are bound by the issue of
+// vector instructions beside the MFMAs (4.5 clocks each, 2.8 for an fma, against 17 of an MFMA; two waves a SIMD), so
+// what counts is their number: 19 for eight nibbles of a column.
+//
+// A nibble in a byte of its own is an f8 E4M3 code of value q / 512 - subnormal up to 7, then the first binade,
+// whose spacing is the same - and v_cvt_scalef32_pk_f32_fp8 with a scale of 512 widens two neighbouring bytes to
+// q exactly: half the conversions of v_cvt_f32_ubyteN.  q[i] = byte i of v, each below 16.
+__device__ __forceinline__ void pk4g_widen(uint32_t v, float (&q)[4]) {
+    const float2_t lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(v, 512.0f, false);
+    const float2_t hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(v, 512.0f, true);
+    q[0] = lo[0], q[1] = lo[1], q[2] = hi[0], q[3] = hi[1];
+}
+__device__ __forceinline__ uint32_t pk4g_low(uint32_t w) { return w & 0x0F0F0F0Fu; }
+__device__ __forceinline__ uint32_t pk4g_high(uint32_t w) { return (w >> 4) & 0x0F0F0F0Fu; }
 struct Pk4gBf16 {
-    float s, s16, c;  // scale, scale / 16, -z * scale
-    __device__ __forceinline__ void set(float scale, float minus_z) { s = scale, s16 = scale * 0.0625f, c = minus_z * scale; }
-    // the pair in bytes B and B + 2 of v; HIGH: v holds high nibbles
-    template <int B, bool HIGH> __device__ __forceinline__ uint32_t pair(uint32_t v) const {
-        const float lo = (float)((v >> (8 * B)) & 0xFFu), hi = (float)((v >> (8 * B + 16)) & 0xFFu);
-        const float m = HIGH ? s16 : s;
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{__builtin_fmaf(lo, m, c), __builtin_fmaf(hi, m, c)}, bf16x2_t));
+    float s, c;  // scale, -z * scale
+    __device__ __forceinline__ void set(float scale, float minus_z) { s = scale, c = minus_z * scale; }
+    __device__ __forceinline__ uint32_t pair(float lo, float hi) const {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{__builtin_fmaf(lo, s, c), __builtin_fmaf(hi, s, c)}, bf16x2_t));
+    }
+    // 8-bit codes: the pair in bytes B and B + 2 of v
+    template <int B> __device__ __forceinline__ uint32_t bytes(uint32_t v) const {
+        return pair((float)((v >> (8 * B)) & 0xFFu), (float)((v >> (8 * B + 16)) & 0xFFu));
+    }
+    // eight rows of a column whose row pair pp is nibble pp of the word's 16-bit halves
+    __device__ __forceinline__ void rows(uint32_t w, uint32_t (&b)[4]) const {
+        float lo[4], hi[4];
+        pk4g_widen(pk4g_low(w), lo), pk4g_widen(pk4g_high(w), hi);
+        b[0] = pair(lo[0], lo[2]), b[1] = pair(hi[0], hi[2]), b[2] = pair(lo[1], lo[3]), b[3] = pair(hi[1], hi[3]);
     }
 };
-__device__ __forceinline__ void pk4g_nibbles(uint32_t w, uint32_t &lo, uint32_t &hi) {
-    lo = w & 0x0F0F0F0Fu, hi = w & 0xF0F0F0F0u;
-    asm volatile("" : "+v"(lo), "+v"(hi));  // keep the masks here: folded into the byte extracts they cost one each
+// Columns H and H + 2 of the 64-column layout's words (word pp: nibble f of each 16-bit half is column f of row pair pp).
+template <int H> __device__ __forceinline__ void pk4g_columns(const uint32_t (&w)[4], const Pk4gBf16 &c0, const Pk4gBf16 &c2,
+                                                              uint32_t (&b0)[4], uint32_t (&b2)[4]) {
+#pragma unroll
+    for (int pp = 0; pp < 4; ++pp) {
+        float q[4];
+        pk4g_widen(H ? pk4g_high(w[pp]) : pk4g_low(w[pp]), q);
+        b0[pp] = c0.pair(q[0], q[2]), b2[pp] = c2.pair(q[1], q[3]);
+    }
 }
 
 constexpr int PK4N_BW = 272;  // 16-column strips: words of one block, 256 of weights and 16 of pairs

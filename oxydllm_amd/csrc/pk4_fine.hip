@@ -45,23 +45,18 @@ int launch_pk4_fine(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p,
                                 : fine_go<BF16Traits>(ctx, s, grid, p, bslice, mt, fold);
 }
 
-template <typename TT, int MT, int KS>
+template <typename TT, int MT>
 static int fine_gemm(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT) {
     const bool g64 = pk4_sets(p.w.group_shift) == 2;
     if (p.w.bits == 4)
-        return g64 ? pk4_gemm_wide_go<TT, MT, 4, KS, 2>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, MT, 4, KS, 4>(s, grid, p, NG, RT);
-    return g64 ? pk4_gemm_wide_go<TT, MT, 8, KS, 2>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, MT, 8, KS, 4>(s, grid, p, NG, RT);
+        return g64 ? pk4_gemm_wide_go<TT, MT, 4, 2>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, MT, 4, 4>(s, grid, p, NG, RT);
+    return g64 ? pk4_gemm_wide_go<TT, MT, 8, 2>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, MT, 8, 4>(s, grid, p, NG, RT);
 }
 
-template <typename TT>
-static int fine_gemm_form(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows, int ks, int NG, int RT) {
-    if (ks == 4) return fine_gemm<TT, 4, 4>(s, grid, p, NG, RT);
-    return rows == 128 ? fine_gemm<TT, 8, 1>(s, grid, p, NG, RT) : fine_gemm<TT, 4, 1>(s, grid, p, NG, RT);
-}
-
-int launch_pk4_gemm_fine(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows, int ks, int NG, int RT) {
-    return p.w.dtype == OXQ_F16 ? fine_gemm_form<F16Traits>(s, grid, p, rows, ks, NG, RT)
-                                : fine_gemm_form<BF16Traits>(s, grid, p, rows, ks, NG, RT);
+int launch_pk4_gemm_fine(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows, int NG, int RT) {
+    const bool f16 = p.w.dtype == OXQ_F16;
+    if (rows == 128) return f16 ? fine_gemm<F16Traits, 8>(s, grid, p, NG, RT) : fine_gemm<BF16Traits, 8>(s, grid, p, NG, RT);
+    return f16 ? fine_gemm<F16Traits, 4>(s, grid, p, NG, RT) : fine_gemm<BF16Traits, 4>(s, grid, p, NG, RT);
 }
 
 }  // namespace oxq

@@ -28,32 +28,25 @@ namespace oxq {
 // projections): a wave's 64 columns are four neighbouring strips, a strip's block is one 16-byte load a lane
 // whose words are the block's four steps - so the ring holds whole blocks, two of them: the next block is
 // requested into the other half when a block starts.  Lane (ni, kb) holds column 16 f + ni of strip f.
-template <typename TT, int MT, int KS>
+template <typename TT, int MT>
 __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
                                                         const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                         int M, int K, int N, int NG, int RT) {
     typedef MfmaOps<TT> Ops;
-    static_assert(KS == 1 || KS == MT, "wave kq of a column group finishes row tile kq");
-    constexpr int SPW = PK4G_STRIPS / KS;  // 64-column groups a workgroup
-    constexpr int ROWS = 16 * MT, BB = PK4N_BW * 4, XBUF = KS * ROWS * 256, XV = ROWS / 4 / SPW;
+    constexpr int ROWS = 16 * MT, BB = PK4N_BW * 4, XBUF = ROWS * 256, XV = ROWS / 4 / PK4G_STRIPS;
     constexpr bool BF = TT::DTYPE == BF16Traits::DTYPE;
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ni = lane & 15, kb = lane >> 4;
-    const int ws = wave % SPW, kq = wave / SPW;  // as in pk4_gemm_kernel
     int rt, g;
-    if constexpr (KS == 1) {
-        pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
-        if (g >= NG) return;  // the whole workgroup, before any barrier
-    } else {
-        rt = (int)blockIdx.x / NG, g = (int)blockIdx.x % NG;
-    }
-    const int j = g * SPW + ws;  // the wave's 64 columns: strips 4 j .. 4 j + 3
+    pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
+    if (g >= NG) return;  // the whole workgroup, before any barrier
+    const int j = g * PK4G_STRIPS + wave;  // the wave's 64 columns: strips 4 j .. 4 j + 3
     const bool live = j < (N >> 6);
     const int m0 = rt * ROWS;
-    const int NB = K >> 7, NR = (NB + KS - 1) / KS;
+    const int NB = K >> 7;
     const int xrows = min(M - m0, ROWS);
 
     const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);
@@ -65,7 +58,7 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
     int xo[XV];
 #pragma unroll
     for (int q = 0; q < XV; ++q) {
-        const int r = 4 * (ws * XV + q) + (lane >> 4);
+        const int r = 4 * (wave * XV + q) + (lane >> 4);
         xo[q] = r * K * 2 + (((lane & 15) ^ (r & 15)) << 4);
     }
     int a_rd[4];
@@ -75,13 +68,11 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 
     u32x4_t wring[2][4];
     uint32_t zring[4];
-    // round r: the wave's block is KS r + kq, its tile of x at kq ROWS 256 of the round's buffer
-    auto dma_x = [&](int r) {
-        const int i = KS * r + kq;
+    auto dma_x = [&](int i) {
         const __amdgpu_buffer_rsrc_t rs = i < NB ? rs_x : rs_none;
 #pragma unroll
         for (int q = 0; q < XV; ++q)
-            pk4g_load_lds16(rs, pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256) + (ws * XV + q) * 1024, xo[q], i * 256);
+            pk4g_load_lds16(rs, pk4_lds + (i & 1) * XBUF + (wave * XV + q) * 1024, xo[q], i * 256);
     };
     auto load_w = [&](int i, u32x4_t (&w)[4]) {
         const __amdgpu_buffer_rsrc_t rs = i < NB ? rs_w : rs_none;
@@ -96,8 +87,8 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 
     dma_x(0);
     __builtin_amdgcn_sched_barrier(0);  // requests keep this order: the wait counts rely on it
-    load_z(kq);
-    load_w(kq, wring[0]);
+    load_z(0);
+    load_w(0, wring[0]);
     __builtin_amdgcn_sched_barrier(0);
     float4_t acc[MT][4];
 #pragma unroll
@@ -107,15 +98,14 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
     pk4g_wait_vmcnt<8>();
     __syncthreads();
 
-    // one round, the block's weights in ring half CUR; eight ring loads are younger than the round's loads of x
-    auto block = [&](int r, auto cur_c) {
+    // one block, its weights in ring half CUR; eight ring loads are younger than the block's loads of x
+    auto block = [&](int i, auto cur_c) {
         constexpr int CUR = decltype(cur_c)::value;
-        const int i = KS * r + kq;  // past NB (a ragged last round): zeros from both streams
-        dma_x(r + 1);
+        dma_x(i + 1);
         __builtin_amdgcn_sched_barrier(0);
-        load_w(i + KS, wring[CUR ^ 1]);
+        load_w(i + 1, wring[CUR ^ 1]);
         __builtin_amdgcn_sched_barrier(0);  // not sunk to the block's end, where the next block would wait for them
-        const unsigned char *buf = pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256);
+        const unsigned char *buf = pk4_lds + (i & 1) * XBUF;
         Pk4N<TT> cst[4];
         Pk4gBf16 cb[4];
 #pragma unroll
@@ -126,7 +116,7 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
                 cst[f].prep(zring[f]);
             }
         }
-        load_z(i + KS);
+        load_z(i + 1);
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             uint32_t a[MT][4];
@@ -140,10 +130,7 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
                 const uint32_t w = wring[CUR][f][st];
                 uint32_t b[4];
                 if constexpr (BF) {  // row pair pp: nibble pp of each 16-bit half
-                    uint32_t tl, th;
-                    pk4g_nibbles(w, tl, th);
-                    b[0] = cb[f].template pair<0, false>(tl), b[1] = cb[f].template pair<0, true>(th);
-                    b[2] = cb[f].template pair<1, false>(tl), b[3] = cb[f].template pair<1, true>(th);
+                    cb[f].rows(w, b);
                 } else {
 #pragma unroll
                     for (int pp = 0; pp < 4; ++pp) b[pp] = cst[f].deq(TT::unpack1(w, pp, nm), pp);
@@ -153,43 +140,18 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        pk4g_wait_vmcnt<8>();  // this wave's part of the next round of x is in LDS
+        pk4g_wait_vmcnt<8>();  // this wave's part of the next block of x is in LDS
         __syncthreads();
     };
     {
-        int r = 0;
-        for (; r + 1 < NR; r += 2) {
-            block(r, std::integral_constant<int, 0>{});
-            block(r + 1, std::integral_constant<int, 1>{});
+        int i = 0;
+        for (; i + 1 < NB; i += 2) {
+            block(i, std::integral_constant<int, 0>{});
+            block(i + 1, std::integral_constant<int, 1>{});
         }
-        if (r < NR) block(r, std::integral_constant<int, 0>{});
+        if (i < NB) block(i, std::integral_constant<int, 0>{});
     }
 
-    // the finished tile rows of this wave, as in pk4_gemm_kernel
-    float4_t fin[KS == 1 ? MT : 1][4];
-    if constexpr (KS == 1) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) fin[mt][f] = acc[mt][f];
-    } else {
-        float4_t *red = (float4_t *)pk4_lds;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                red[((wave * MT + mt) * 4 + e) * 64 + lane] = float4_t{acc[mt][0][e], acc[mt][1][e], acc[mt][2][e], acc[mt][3][e]};
-        __syncthreads();
-#pragma unroll
-        for (int f = 0; f < 4; ++f) fin[0][f] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < KS; ++k)  // K order: the same sum whatever the timing
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float4_t v = red[(((k * SPW + ws) * MT + kq) * 4 + e) * 64 + lane];
-                fin[0][0][e] += v[0], fin[0][1][e] += v[1], fin[0][2][e] += v[2], fin[0][3][e] += v[3];
-            }
-    }
     if (!live) return;
     // row 16 mt + 4 kb + e, column 64 j + 16 f + ni
     float bv[4] = {0.f, 0.f, 0.f, 0.f};
@@ -197,15 +159,14 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 #pragma unroll
         for (int f = 0; f < 4; ++f) bv[f] = TT::to_f32(bias[64 * j + 16 * f + ni]);
     }
-    constexpr int FT = KS == 1 ? MT : 1;
 #pragma unroll
-    for (int t = 0; t < FT; ++t)
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
+            const int row = m0 + 16 * t + 4 * kb + e;
             if (row >= M) continue;
 #pragma unroll
-            for (int f = 0; f < 4; ++f) y[(size_t)row * N + 64 * j + 16 * f + ni] = TT::from_f32(fin[t][f][e] + bv[f]);
+            for (int f = 0; f < 4; ++f) y[(size_t)row * N + 64 * j + 16 * f + ni] = TT::from_f32(acc[t][f][e] + bv[f]);
         }
 }
 
@@ -232,17 +193,29 @@ struct Pk4GemmCost {
     bool pairs64;
     double part64, a64, b64, slope64, full128, part128, split_lo, split_hi;
 };
-// rows of a workgroup (0: the split-K tiles) and the K split inside it (4: two strips a workgroup)
+// rows of a workgroup (0: the split-K tiles) and the K split inside it (4: pk4_mid_kernel, two strips a workgroup)
 struct Pk4GemmForm {
     int rows, ks;
 };
+// pk4_mid_kernel at up to 64 rows of 64-column strips, against the one-strip workgroups of pk4_mfma_kernel and
+// pk4_tile64_kernel, both one a CU: a round of it costs 1.6 - 1.8 of theirs (4096 x 28672 at 48 / 64 rows: bf16 28.5 / 31.3 ->
+// 25.2 / 26.3 us, f16 at 64 rows 29.3 -> 25.5; 8-bit 4096 x 22016 at 64 rows 39.2 -> 30.4; bf16 at 32 rows 23.0 -> 24.3).
+// f16 only from where its weights are rounded anyway (pk4_folds).
+static bool pk4_mid_decode(double cus, const Pk4Problem &p) {
+    const int64_t from = p.w.dtype == OXQ_F16 ? 49 : 33;
+    if (p.w.strip != 64 || p.M < from || p.M > 64 || pk4_sets(p.w.group_shift) > 1) return false;
+    const double strips = (double)ceil_div(p.w.N, (int64_t)64);
+    return 1.8 * std::ceil(strips / (2 * cus)) < std::ceil(strips / cus);
+}
 static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
-    const int64_t min_m = tune(ctx, OXQ_TUNE_PK4_GEMM_MIN_M, pk4_sets(p.w.group_shift) > 1 ? 49 : 65);
+    const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    const int64_t min_m = tune(ctx, OXQ_TUNE_PK4_GEMM_MIN_M, pk4_sets(p.w.group_shift) > 1 ? 49 : pk4_mid_decode(cus, p) ? 33 : 65);
     if (min_m <= 0 || (p.w.bits != 4 && p.w.bits != 8) || (p.act && p.w.strip == 16) || p.M < min_m) return {0, 1};
     if (p.w.bits == 8 && p.w.strip == 16) return {0, 1};  // (16-column strips are a 4-bit layout)
     const int forced = tune(ctx, OXQ_TUNE_PK4_GEMM_ROWS, 0), forced_ks = tune(ctx, OXQ_TUNE_PK4_GEMM_KS, 0);
     if (forced_ks == 4) return {64, 4};
     if (forced == 64 || forced == 128) return {forced, 1};
+    if (p.M <= 64 && pk4_mid_decode(cus, p) && forced_ks != 1) return {64, 4};
     static const Pk4GemmCost WIDE_F16 = {true, 0.88, 1.20, 0.30, 0.97, 1.50, 1.27, 1.93, 1.50};
     static const Pk4GemmCost WIDE_BF16 = {true, 0.93, 1.29, 0.27, 0.98, 1.44, 1.35, 2.00, 1.53};
     static const Pk4GemmCost NARROW_F16 = {false, 0.86, 0, 0, 0, 1.64, 1.30, 1.60, 1.50};
@@ -253,7 +226,6 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     const Pk4GemmCost &c = p.w.bits == 8      ? (f16 ? WIDE8_F16 : WIDE8_BF16)
                            : p.w.strip == 16 ? (f16 ? NARROW_F16 : NARROW_BF16)
                                              : (f16 ? WIDE_F16 : WIDE_BF16);
-    const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int64_t groups = ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)PK4G_STRIPS);
     const double w64 = (double)(groups * ceil_div(p.M, (int64_t)64)) / cus, w128 = (double)(groups * ceil_div(p.M, (int64_t)128)) / cus;
     auto rounds = [](double w, double full, double part, double part_upto) {
@@ -276,20 +248,20 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
 }
 bool pk4_gemm_takes(const oxq_ctx *ctx, const Pk4Problem &p) { return pk4_gemm_form(ctx, p).rows != 0; }
 
-template <typename TT, int MT, int KS>
+template <typename TT, int MT>
 static int pk4n_gemm_go(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT) {
     static LdsGrant grant;  // one per instantiation
-    const size_t lds = (size_t)2 * KS * 16 * MT * 256;
-    OXQ_HIP_CHECK(grant.ensure((const void *)pk4n_gemm_kernel<TT, MT, KS>, lds));
-    hipLaunchKernelGGL((pk4n_gemm_kernel<TT, MT, KS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
+    const size_t lds = (size_t)2 * 16 * MT * 256;
+    OXQ_HIP_CHECK(grant.ensure((const void *)pk4n_gemm_kernel<TT, MT>, lds));
+    hipLaunchKernelGGL((pk4n_gemm_kernel<TT, MT>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
                        (uint16_t *)p.y, (int)p.M, (int)p.w.K, (int)p.w.N, NG, RT);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
-template <typename TT, int MT, int KS>
+template <typename TT, int MT>
 static int pk4_gemm_go_layout(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT) {
-    if (p.w.strip == 16) return pk4n_gemm_go<TT, MT, KS>(s, grid, p, NG, RT);
-    return p.w.bits == 8 ? pk4_gemm_wide_go<TT, MT, 8, KS, 1>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, MT, 4, KS, 1>(s, grid, p, NG, RT);
+    if (p.w.strip == 16) return pk4n_gemm_go<TT, MT>(s, grid, p, NG, RT);
+    return p.w.bits == 8 ? pk4_gemm_wide_go<TT, MT, 8, 1>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, MT, 4, 1>(s, grid, p, NG, RT);
 }
 
 int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
@@ -302,20 +274,20 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw,
-             form.ks > 1 ? "k4" : "", p.w.strip == 16 ? "_n16" : "", p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
+    snprintf(name, sizeof name, "pk%d_%s_%s_r%dx%d%s%s%s", p.w.bits, form.ks > 1 && p.M <= 64 ? "mid" : "gemm",
+             p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw, form.ks > 1 ? "k4" : "", p.w.strip == 16 ? "_n16" : "",
+             p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if ((uint64_t)rows * (uint64_t)p.w.K * 2 >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: K too large");
     if (((uintptr_t)p.x | (uintptr_t)p.y) & 15) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: x and y must be 16-byte aligned");
     if (p.bias && ((uintptr_t)p.bias & 7)) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: bias must be 8-byte aligned");
-    if (pk4_sets(p.w.group_shift) > 1) return launch_pk4_gemm_fine(s, grid, p, rows, form.ks, (int)NG, (int)RT);
+    if (form.ks == 4) return launch_pk4_mid(s, grid, p, (int)NG);
+    if (pk4_sets(p.w.group_shift) > 1) return launch_pk4_gemm_fine(s, grid, p, rows, (int)NG, (int)RT);
     const bool f16 = p.w.dtype == OXQ_F16;
-    if (form.ks == 4)
-        return f16 ? pk4_gemm_go_layout<F16Traits, 4, 4>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_layout<BF16Traits, 4, 4>(s, grid, p, (int)NG, (int)RT);
     if (rows == 128)
-        return f16 ? pk4_gemm_go_layout<F16Traits, 8, 1>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_layout<BF16Traits, 8, 1>(s, grid, p, (int)NG, (int)RT);
-    return f16 ? pk4_gemm_go_layout<F16Traits, 4, 1>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_layout<BF16Traits, 4, 1>(s, grid, p, (int)NG, (int)RT);
+        return f16 ? pk4_gemm_go_layout<F16Traits, 8>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_layout<BF16Traits, 8>(s, grid, p, (int)NG, (int)RT);
+    return f16 ? pk4_gemm_go_layout<F16Traits, 4>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_layout<BF16Traits, 4>(s, grid, p, (int)NG, (int)RT);
 }
 
 }  // namespace oxq

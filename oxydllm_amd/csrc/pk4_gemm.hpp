@@ -8,44 +8,31 @@ namespace oxq {
 
 constexpr int PK4G_STRIPS = 8;  // strips (= waves) of a workgroup
 
-// KS = 1: eight strips a workgroup, a wave takes every block of its strip.  KS = 4 (the form for 65 to a few hundred
-// rows, where workgroups of eight strips are too few to fill the chip): two strips a workgroup, the four waves of
-// a strip take every fourth block; a round brings four blocks of x into LDS, each loaded by the two waves that use
-// it; at the end the waves' partial tiles meet in LDS (where x was) and wave kq of a strip finishes row tile kq,
-// adding the four partials in K order - the epilogue then runs on the accumulator layout as for KS = 1.
+// Eight strips a workgroup, a wave takes every block of its strip.
 // SETS: as in pk4_mfma_kernel (groups of 128 rows and more, 64, 32).
-template <typename TT, int MT, int BITS, int KS, int SETS = 1>
+template <typename TT, int MT, int BITS, int SETS = 1>
 __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
                                                        const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                        int M, int K, int N, int NG, int RT, int act) {
     typedef MfmaOps<TT> Ops;
-    static_assert(KS == 1 || KS == MT, "wave kq of a strip finishes row tile kq");
-    constexpr int SPW = PK4G_STRIPS / KS;  // strips a workgroup
-    constexpr int ROWS = 16 * MT, BB = pk4_block_words(BITS, SETS) * 4, XBUF = KS * ROWS * 256;
+    constexpr int ROWS = 16 * MT, BB = pk4_block_words(BITS, SETS) * 4, XBUF = ROWS * 256;
     constexpr int WL = BITS / 4;          // 1 KB weight loads a step (8-bit: column pairs 0, 1 and 2, 3)
     constexpr int RING = 4 * WL + SETS;      // ring loads of a block: younger than the block's loads of x
     constexpr bool BF = TT::DTYPE == BF16Traits::DTYPE;
     constexpr int SPS = 4 / SETS;         // steps that share a set of pairs
-    constexpr int XV = ROWS / 4 / SPW;  // loads of x a wave issues per round: 64 lanes x 16 bytes = 4 rows each
+    constexpr int XV = ROWS / 4 / PK4G_STRIPS;  // loads of x a wave issues per block: 64 lanes x 16 bytes = 4 rows each
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ni = lane & 15, kb = lane >> 4;
-    const int ws = wave % SPW, kq = wave / SPW;  // the wave's strip of the workgroup, and its share of K
     int rt, g;
-    if constexpr (KS == 1) {
-        pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
-        if (g >= NG) return;  // the whole workgroup, before any barrier: the ragged last column of squares
-    } else {
-        // a row tile's strip groups are neighbours: the eight XCDs share its rows of x, and with NG a multiple of 8
-        // the row tiles of a strip group meet on one XCD, whose L2 then holds the group's weights
-        rt = (int)blockIdx.x / NG, g = (int)blockIdx.x % NG;
-    }
-    const int j = g * SPW + ws;
+    pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
+    if (g >= NG) return;  // the whole workgroup, before any barrier: the ragged last column of squares
+    const int j = g * PK4G_STRIPS + wave;
     const bool live = j < ((N + 63) >> 6);  // wave-uniform: the last group of a layer may have fewer strips
     const int m0 = rt * ROWS;
-    const int NB = SETS > 1 ? (K + 127) >> 7 : K >> 7, NR = (NB + KS - 1) / KS;  // blocks; rounds of KS blocks
+    const int NB = SETS > 1 ? (K + 127) >> 7 : K >> 7;
     const int xrows = min(M - m0, ROWS);
 
     const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);
@@ -54,13 +41,13 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
     const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x + (size_t)m0 * K, (uint32_t)xrows * (uint32_t)K * 2u);
     const int voff_w = lane * 16;
     const int voff_z = 1024 * WL * 4 + (ni * 4 + kb) * 4;
-    // x: load q of a wave brings rows 4 (XV ws + q) .. + 3 of the wave's block of the round straight into LDS, lane l
+    // x: load q of a wave brings rows 4 (XV wave + q) .. + 3 of a block straight into LDS, lane l
     // the 16 bytes that belong at position l % 16 of row l / 16 - chunk (l % 16) ^ (row % 16) of the row, the
     // swizzle the fragment reads undo.  Rows past M lie beyond the descriptor: LDS receives zeros.
     int xo[XV];
 #pragma unroll
     for (int q = 0; q < XV; ++q) {
-        const int r = 4 * (ws * XV + q) + (lane >> 4);
+        const int r = 4 * (wave * XV + q) + (lane >> 4);
         xo[q] = r * K * 2 + (((lane & 15) ^ (r & 15)) << 4);
     }
     int a_rd[4];  // fragment of step st, row tile mt (+ 4096 mt): row ni
@@ -72,16 +59,14 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
     uint32_t zring[SETS];
     // The compiler orders nothing against these loads: the wait for them (the ring loads of a block are
     // younger) is written out in front of the barrier that publishes the block.
-    // round r: the wave's block is KS r + kq; its tile of x lies at kq ROWS 256 of the round's buffer
-    auto dma_x = [&](int r_) {
-        const int i = KS * r_ + kq;
+    auto dma_x = [&](int i) {
         const __amdgpu_buffer_rsrc_t rs = i < NB ? rs_x : rs_none;
         if constexpr (SETS > 1) {
             if (i == NB - 1 && (K & 127)) {  // K ends inside the block: zeros for the chunks past it, not the next row
 #pragma unroll
                 for (int q = 0; q < XV; ++q) {
-                    const int r = 4 * (ws * XV + q) + (lane >> 4), chunk = (lane & 15) ^ (r & 15);
-                    pk4g_load_lds16(rs, pk4_lds + (r_ & 1) * XBUF + kq * (ROWS * 256) + (ws * XV + q) * 1024,
+                    const int r = 4 * (wave * XV + q) + (lane >> 4), chunk = (lane & 15) ^ (r & 15);
+                    pk4g_load_lds16(rs, pk4_lds + (i & 1) * XBUF + (wave * XV + q) * 1024,
                                     i * 128 + 8 * chunk < K ? xo[q] : 0x7FFFFF00, i * 256);
                 }
                 return;
@@ -89,7 +74,7 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         }
 #pragma unroll
         for (int q = 0; q < XV; ++q)
-            pk4g_load_lds16(rs, pk4_lds + (r_ & 1) * XBUF + kq * (ROWS * 256) + (ws * XV + q) * 1024, xo[q], i * 256);
+            pk4g_load_lds16(rs, pk4_lds + (i & 1) * XBUF + (wave * XV + q) * 1024, xo[q], i * 256);
     };
     auto load_w = [&](int i, int st) {
         const __amdgpu_buffer_rsrc_t rs = i < NB ? rs_w : rs_none;
@@ -111,9 +96,9 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
     dma_x(0);
     __builtin_amdgcn_sched_barrier(0);  // requests keep this order: the wait counts rely on it
 #pragma unroll
-    for (int u = 0; u < SETS; ++u) load_z(kq, u);
+    for (int u = 0; u < SETS; ++u) load_z(0, u);
 #pragma unroll
-    for (int st = 0; st < 4; ++st) load_w(kq, st);
+    for (int st = 0; st < 4; ++st) load_w(0, st);
     __builtin_amdgcn_sched_barrier(0);
     float4_t acc[MT][4];
 #pragma unroll
@@ -123,12 +108,11 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
     pk4g_wait_vmcnt<RING>();
     __syncthreads();
 
-    for (int r = 0; r < NR; ++r) {
-        const int i = KS * r + kq;  // past NB (a ragged last round): zeros from both streams
-        // the other buffer was last read in the previous round, which every wave has left (the barrier below)
-        dma_x(r + 1);
+    for (int i = 0; i < NB; ++i) {
+        // the other buffer was last read in the previous block, which every wave has left (the barrier below)
+        dma_x(i + 1);
         __builtin_amdgcn_sched_barrier(0);
-        const unsigned char *buf = pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256);
+        const unsigned char *buf = pk4_lds + (i & 1) * XBUF;
         uint32_t zv[4], negzb[4], sp[4];
         Pk4gBf16 cb[4];
         auto constants = [&](int set) {  // of a set of pairs; then the next block's are requested
@@ -141,7 +125,7 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
                 Pk4T<TT>::prep(zv[f], negzb[f], sp[f]);
             }
         }
-        load_z(i + KS, set);
+        load_z(i + 1, set);
         };
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
@@ -158,69 +142,62 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
                 const u32x4_t av = *(const u32x4_t *)(buf + mt * 4096 + a_rd[st]);
                 a[mt][0] = av[0], a[mt][1] = av[1], a[mt][2] = av[2], a[mt][3] = av[3];
             }
-            uint32_t tl[4], th[4];
-            if constexpr (BF && BITS == 4) {
-#pragma unroll
-                for (int pp = 0; pp < 4; ++pp) pk4g_nibbles(wp[0][pp], tl[pp], th[pp]);
-            }
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                uint32_t b[4];
-#pragma unroll
-                for (int pp = 0; pp < 4; ++pp) {
-                    if constexpr (BITS == 8) {
-                        // word pp of half f / 2: bytes {row 2 pp, row 2 pp + 1} x {column 2 h, 2 h + 1}: the pair of
-                        // column f in bytes f % 2 and f % 2 + 2
-                        const uint32_t word = wp[f >> 1][pp];
-                        if constexpr (BF) b[pp] = (f & 1) ? cb[f].template pair<1, false>(word) : cb[f].template pair<0, false>(word);
-                        else b[pp] = Pk4T<TT>::deq(TT::unpack_bytes((f & 1) ? (word >> 8) : word), negzb[f], sp[f]);
-                    } else {
-                        // column f of word pp: nibble f of each 16-bit half = the low or high nibble of bytes f / 2 and 2 + f / 2
-                        if constexpr (!BF) b[pp] = Pk4T<TT>::deq(TT::unpack1(wp[0][pp], f, nm), negzb[f], sp[f]);
-                        else if (f == 0) b[pp] = cb[0].template pair<0, false>(tl[pp]);
-                        else if (f == 1) b[pp] = cb[1].template pair<0, true>(th[pp]);
-                        else if (f == 2) b[pp] = cb[2].template pair<1, false>(tl[pp]);
-                        else b[pp] = cb[3].template pair<1, true>(th[pp]);
-                    }
-                }
+            auto column = [&](int f, const uint32_t (&b)[4]) {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) acc[mt][f] = Ops::mfma(a[mt], b, acc[mt][f]);
+            };
+            if constexpr (BF && BITS == 4 && MT == 4) {
+                // 64-row workgroups share a CU in pairs with up to 128 registers, which two columns at a time exceed
+                // (135: 4096 x 14336 at 1536 rows 195 -> 216 us): one column, a conversion a weight
+                uint32_t tl[4], th[4];
+#pragma unroll
+                for (int pp = 0; pp < 4; ++pp) {
+                    tl[pp] = pk4g_low(wp[0][pp]), th[pp] = pk4g_high(wp[0][pp]);
+                    asm volatile("" : "+v"(tl[pp]), "+v"(th[pp]));  // the masks stay here: folded into the byte extracts they cost one each
+                }
+#pragma unroll
+                for (int f = 0; f < 4; ++f) {
+                    uint32_t b[4];
+#pragma unroll
+                    for (int pp = 0; pp < 4; ++pp) {
+                        const uint32_t v = (f & 1) ? th[pp] : tl[pp];
+                        b[pp] = (f >> 1) ? cb[f].template bytes<1>(v) : cb[f].template bytes<0>(v);
+                    }
+                    column(f, b);
+                }
+            } else if constexpr (BF && BITS == 4) {
+                uint32_t b0[4], b2[4];
+                pk4g_columns<0>(wp[0], cb[0], cb[2], b0, b2);
+                column(0, b0), column(2, b2);
+                pk4g_columns<1>(wp[0], cb[1], cb[3], b0, b2);
+                column(1, b0), column(3, b2);
+            } else {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) {
+                    uint32_t b[4];
+#pragma unroll
+                    for (int pp = 0; pp < 4; ++pp) {
+                        if constexpr (BITS == 8) {
+                            // word pp of half f / 2: bytes {row 2 pp, row 2 pp + 1} x {column 2 h, 2 h + 1}: the pair of
+                            // column f in bytes f % 2 and f % 2 + 2
+                            const uint32_t word = wp[f >> 1][pp];
+                            if constexpr (BF) b[pp] = (f & 1) ? cb[f].template bytes<1>(word) : cb[f].template bytes<0>(word);
+                            else b[pp] = Pk4T<TT>::deq(TT::unpack_bytes((f & 1) ? (word >> 8) : word), negzb[f], sp[f]);
+                        } else {
+                            b[pp] = Pk4T<TT>::deq(TT::unpack1(wp[0][pp], f, nm), negzb[f], sp[f]);
+                        }
+                    }
+                    column(f, b);
+                }
             }
-            load_w(i + KS, st);  // into the registers this step has just left
+            load_w(i + 1, st);  // into the registers this step has just left
         }
         __builtin_amdgcn_sched_barrier(0);
-        pk4g_wait_vmcnt<RING>();  // this wave's part of the next round of x is in LDS; its ring loads may still fly
+        pk4g_wait_vmcnt<RING>();  // this wave's part of the next block of x is in LDS; its ring loads may still fly
         __syncthreads();
     }
 
-    // the finished tile rows of this wave: all of them (KS = 1), or row tile kq summed over the strip's waves
-    float4_t fin[KS == 1 ? MT : 1][4];
-    if constexpr (KS == 1) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) fin[mt][f] = acc[mt][f];
-    } else {
-        // slot of wave w: [mt][e][lane] x float4 (f = 0..3), 16 KB; the last round's barrier has freed the buffers
-        float4_t *red = (float4_t *)pk4_lds;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                red[((wave * MT + mt) * 4 + e) * 64 + lane] = float4_t{acc[mt][0][e], acc[mt][1][e], acc[mt][2][e], acc[mt][3][e]};
-        __syncthreads();
-#pragma unroll
-        for (int f = 0; f < 4; ++f) fin[0][f] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < KS; ++k)  // K order: the same sum whatever the timing
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float4_t v = red[(((k * SPW + ws) * MT + kq) * 4 + e) * 64 + lane];
-                fin[0][0][e] += v[0], fin[0][1][e] += v[1], fin[0][2][e] += v[2], fin[0][3][e] += v[3];
-            }
-    }
     if (!live) return;
-    constexpr int FT = KS == 1 ? MT : 1;  // row tiles this wave stores: fin[t] is row tile (KS == 1 ? t : kq)
     if (act) {
         // Fused gate|up layer (pk4_src_col): columns 0..31 of the strip are gate columns 32 j .. 32 j + 31, columns
         // 32..63 the up columns they meet - lane ni < 8 holds four gate columns, lane ni + 8 of the same row of 16
@@ -237,14 +214,14 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
             bv[2] = TT::to_f32((uint16_t)(bw.y & 0xFFFFu)), bv[3] = TT::to_f32((uint16_t)(bw.y >> 16));
         }
 #pragma unroll
-        for (int t = 0; t < FT; ++t)
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
+                const int row = m0 + 16 * t + 4 * kb + e;
                 float mine[4], other[4];
 #pragma unroll
                 for (int f = 0; f < 4; ++f) {
-                    mine[f] = TT::to_f32(TT::from_f32(fin[t][f][e] + bv[f]));
+                    mine[f] = TT::to_f32(TT::from_f32(acc[t][f][e] + bv[f]));
                     other[f] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mine[f]), 0x128, 0xF, 0xF, false));
                 }
                 uint32_t o[2];
@@ -266,23 +243,23 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         bv[2] = TT::to_f32((uint16_t)(bw.y & 0xFFFFu)), bv[3] = TT::to_f32((uint16_t)(bw.y >> 16));
     }
 #pragma unroll
-    for (int t = 0; t < FT; ++t)
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
+            const int row = m0 + 16 * t + 4 * kb + e;
             if (row >= M) continue;
-            const uint32_t o0 = TT::from_f32(fin[t][0][e] + bv[0]), o1 = TT::from_f32(fin[t][1][e] + bv[1]);
-            const uint32_t o2 = TT::from_f32(fin[t][2][e] + bv[2]), o3 = TT::from_f32(fin[t][3][e] + bv[3]);
+            const uint32_t o0 = TT::from_f32(acc[t][0][e] + bv[0]), o1 = TT::from_f32(acc[t][1][e] + bv[1]);
+            const uint32_t o2 = TT::from_f32(acc[t][2][e] + bv[2]), o3 = TT::from_f32(acc[t][3][e] + bv[3]);
             *(uint2 *)(y + (size_t)row * N + 64 * j + 4 * ni) = uint2{o0 | (o1 << 16), o2 | (o3 << 16)};
         }
 }
 
-template <typename TT, int MT, int BITS, int KS, int SETS>
+template <typename TT, int MT, int BITS, int SETS>
 static int pk4_gemm_wide_go(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT) {
     static LdsGrant grant;  // one per instantiation
-    const size_t lds = (size_t)2 * KS * 16 * MT * 256;
-    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_gemm_kernel<TT, MT, BITS, KS, SETS>, lds));
-    hipLaunchKernelGGL((pk4_gemm_kernel<TT, MT, BITS, KS, SETS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
+    const size_t lds = (size_t)2 * 16 * MT * 256;
+    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_gemm_kernel<TT, MT, BITS, SETS>, lds));
+    hipLaunchKernelGGL((pk4_gemm_kernel<TT, MT, BITS, SETS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
                        (uint16_t *)p.y, (int)p.M, (int)p.w.K, (int)p.w.N, NG, RT, p.act);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;

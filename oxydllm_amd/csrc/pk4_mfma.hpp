@@ -218,7 +218,9 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int f = 0; f < 4; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr bool WIDEN = !GS && BITS == 4 && TT::DTYPE == BF16Traits::DTYPE;
     uint32_t negzb[4], sp[4];          // GS = false: the two Pk4T constants per column
+    Pk4gBf16 cb[4];                    // the same of a 4-bit bf16 layer
     const uint32_t ones[4] = {TT::ONES, TT::ONES, TT::ONES, TT::ONES};
     const float4_t zero4 = float4_t{0.f, 0.f, 0.f, 0.f};
 
@@ -255,7 +257,10 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
             uint32_t zv[4];
             zs_words(zring[set], zv);
 #pragma unroll
-            for (int f = 0; f < 4; ++f) Pk4T<TT>::prep(zv[f], negzb[f], sp[f]);
+            for (int f = 0; f < 4; ++f) {
+                if constexpr (WIDEN) cb[f].set(__builtin_bit_cast(float, zv[f] & 0xFFFF0000u), __builtin_bit_cast(float, zv[f] << 16) + 128.0f);
+                else Pk4T<TT>::prep(zv[f], negzb[f], sp[f]);
+            }
             load_z(i + 1, set);
         };
         // the folded form: y += s * (sum - (bias + z) * rowsum), all f32
@@ -312,6 +317,16 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
                 }
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) tmps[mt] = Ops::mfma(a[mt], ones, fresh ? zero4 : tmps[mt]);
+            } else if constexpr (WIDEN) {
+                uint32_t b0[4], b2[4];
+                auto column = [&](int f, const uint32_t (&b)[4]) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) acc[mt][f] = Ops::mfma(a[mt], b, acc[mt][f]);
+                };
+                pk4g_columns<0>(wp[0], cb[0], cb[2], b0, b2);
+                column(0, b0), column(2, b2);
+                pk4g_columns<1>(wp[0], cb[1], cb[3], b0, b2);
+                column(1, b0), column(3, b2);
             } else {
 #pragma unroll
                 for (int f = 0; f < 4; ++f) {

@@ -111,11 +111,25 @@ __global__ __launch_bounds__(512) void pk4_tile64_kernel(const uint16_t *__restr
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int f = 0; f < 4; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr bool BF = TT::DTYPE == BF16Traits::DTYPE;
     uint32_t negzb[4], sp[4];
+    Pk4gBf16 cb[4];
 
     auto multiply = [&](int b, int t, const uint32_t (&a)[MT][4]) {
         const u32x4_t w = wv[b][t];
         const uint32_t wp[4] = {w[0], w[1], w[2], w[3]};
+        if constexpr (BF) {
+            uint32_t b0[4], b2[4];
+            auto column = [&](int f, const uint32_t (&bq)[4]) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) acc[mt][f] = Ops::mfma(a[mt], bq, acc[mt][f]);
+            };
+            pk4g_columns<0>(wp, cb[0], cb[2], b0, b2);
+            column(0, b0), column(2, b2);
+            pk4g_columns<1>(wp, cb[1], cb[3], b0, b2);
+            column(1, b0), column(3, b2);
+            return;
+        }
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
             uint32_t bq[4];
@@ -132,7 +146,10 @@ __global__ __launch_bounds__(512) void pk4_tile64_kernel(const uint16_t *__restr
         const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);
         const uint32_t zq[4] = {pe[0], po[0], pe[1], po[1]};
 #pragma unroll
-        for (int f = 0; f < 4; ++f) Pk4T<TT>::prep(zq[f], negzb[f], sp[f]);
+        for (int f = 0; f < 4; ++f) {
+            if constexpr (BF) cb[f].set(__builtin_bit_cast(float, zq[f] & 0xFFFF0000u), __builtin_bit_cast(float, zq[f] << 16) + 128.0f);
+            else Pk4T<TT>::prep(zq[f], negzb[f], sp[f]);
+        }
     };
 
     // Two fragment sets: the next step's fragments are read while this step multiplies.
