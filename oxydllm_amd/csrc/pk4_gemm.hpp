@@ -148,20 +148,23 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
             };
             if constexpr (BF && BITS == 4 && MT == 4) {
                 // 64-row workgroups share a CU in pairs with up to 128 registers, which two columns at a time exceed
-                // (135: 4096 x 14336 at 1536 rows 195 -> 216 us): one column, a conversion a weight
+                // (135: 4096 x 14336 at 1536 rows 195 -> 216 us): one column, a conversion a weight.  The high nibbles
+                // stay where they are: bytes of 16 q, times s / 16.
                 uint32_t tl[4], th[4];
 #pragma unroll
                 for (int pp = 0; pp < 4; ++pp) {
-                    tl[pp] = pk4g_low(wp[0][pp]), th[pp] = pk4g_high(wp[0][pp]);
+                    tl[pp] = pk4g_low(wp[0][pp]), th[pp] = wp[0][pp] & 0xF0F0F0F0u;
                     asm volatile("" : "+v"(tl[pp]), "+v"(th[pp]));  // the masks stay here: folded into the byte extracts they cost one each
                 }
 #pragma unroll
                 for (int f = 0; f < 4; ++f) {
                     uint32_t b[4];
+                    Pk4gBf16 c = cb[f];
+                    if (f & 1) c.s *= 0.0625f;
 #pragma unroll
                     for (int pp = 0; pp < 4; ++pp) {
                         const uint32_t v = (f & 1) ? th[pp] : tl[pp];
-                        b[pp] = (f >> 1) ? cb[f].template bytes<1>(v) : cb[f].template bytes<0>(v);
+                        b[pp] = (f >> 1) ? c.template bytes<1>(v) : c.template bytes<0>(v);
                     }
                     column(f, b);
                 }

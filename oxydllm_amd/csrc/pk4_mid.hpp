@@ -167,7 +167,9 @@ __global__ __launch_bounds__(512) void pk4_mid_kernel(const uint16_t *__restrict
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) dst[st][mt] = *(const u32x4_t *)(pk4_lds + stage * STAGE + mt * 2048 + a_rd[st]);
     };
-    meet(std::integral_constant<int, 2 * RE + 2 * RO + 2 * MT>{});
+    // The first two stages, counting as younger only the loads of the other two: the compiler may issue the ring loads
+    // above where they are first used, behind this wait (it does so with the second block's), but not those into LDS.
+    meet(std::integral_constant<int, 2 * MT>{});
     read_x(0, a[0]);
     __builtin_amdgcn_sched_barrier(0);
     meet(std::integral_constant<int, 63>{});
