@@ -435,7 +435,9 @@ int oxq_moe_combine(oxq_ctx *ctx, void *stream, const oxq_tensor *expert_out, co
  * the layer (same size as the checkpoint tensors, plus 1.5 bytes per column
  * and group, filled up to whole blocks of 128 rows x 64 columns; strips of 64 output columns, or of 16 for 4-bit layers of at
  * most 8192 columns and 4096 - 14336 rows, such as attention and down projections) and forward never reads the caller's tensors again; it
- * synchronises the null stream once.  Other layers keep descriptors of the
+ * synchronises the null stream once.  GPTQ and 8-bit AWQ layers outside the multiples of 128 / 64 multiply unrounded
+ * weights at every number of rows, as their GEMV on the checkpoint tensors does; all other layers round the dequantized
+ * weight to the activation type at the reference's tile-GEMM sizes.  Other layers keep descriptors of the
  * caller-owned tensors.  OXQ_PREPACK=0 in the environment disables the copy. */
 typedef struct oxq_packed_quant_linear oxq_packed_quant_linear;
 int oxq_packed_quant_linear_new(oxq_ctx *ctx, uint32_t bits, int pack_dim,

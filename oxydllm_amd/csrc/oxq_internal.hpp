@@ -190,6 +190,7 @@ struct Pk4Weights {
     int gemv_rows;          // rows up to which the reference runs its fused GEMV, which never rounds the
                             // dequantized weight (linear.rs:450-480: 16 AWQ, 32 GPTQ); 0 = 16
     int strip;              // columns of a strip of pw: 64 (or 0), or 16 (narrow 4-bit layers, see pk4.hip)
+    bool unrounded = false; // (q - z) * s enters the sums in f32 at every row count (pk4_unrounded)
 };
 
 struct Pk4Problem {
@@ -205,6 +206,7 @@ struct Pk4Problem {
 
 // ---- launchers (defined in the .hip files) ---------------------------------
 bool pk4_eligible(const Wna16Problem &p);
+bool pk4_unrounded(const Wna16Problem &p);
 // resident 4-bit layers at prefill sizes: 64 rows x eight strips a workgroup (pk4_gemm.hip)
 bool pk4_gemm_takes(const oxq_ctx *ctx, const Pk4Problem &p);
 int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p);
@@ -218,6 +220,7 @@ int launch_pk4_dequant(oxq_ctx *ctx, hipStream_t s, const Pk4Weights &w, void *o
 // groups of 32 or 64 rows (pk4_fine.hip): the ring kernel of launch_pk4_forward and the prefill kernel
 int launch_pk4_fine(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p, int bslice, int mt, bool fold);
 int launch_pk4_gemm_fine(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows, int NG, int RT);
+int launch_pk4_gemm_fold(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT);  // unrounded layers (pk4_fold.hip)
 // 64 rows x two groups of 64 columns a workgroup, K split inside it (pk4_mid.hip)
 int launch_pk4_mid(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);
 // 49 - 64 rows on a 4-bit layer in 64-column strips (pk4_tile.hip)

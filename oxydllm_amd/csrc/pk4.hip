@@ -729,6 +729,13 @@ bool pk4_eligible(const Wna16Problem &p) {
     return true;
 }
 
+// Shapes for which the checkpoint layout has no tile kernel: GPTQ and 8-bit AWQ with groups of 32 or 64 rows, K that is no
+// multiple of 128 or N that is none of 64.  There (q - z) * s enters f32 sums unrounded at every row count (one pass of
+// the dot-product kernel per eight rows), and so it does on the copy.
+bool pk4_unrounded(const Wna16Problem &p) {
+    return !(p.bits == 4 && p.pack_dim == OXQ_PACK_OUT) && (p.K % 128 != 0 || p.N % 64 != 0 || p.group_size % 128 != 0);
+}
+
 int launch_pk4_prepack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &src, const Pk4Weights &dst) {
     const int K = (int)src.K, N = (int)src.N;
     const int sets = pk4_sets(src.group_shift);
@@ -898,11 +905,20 @@ static int pk4_go(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p, i
 // (4096 x 14336 f16: 17 rows 10.8 -> 9.9 us, 48 rows 14.3 -> 13.5 us; bf16 GPTQ 17 rows 13.3 -> 10.1 us).
 // At four row tiles the fold costs what the dequant costs and its extra accumulators do not fit.
 static bool pk4_folds(const oxq_ctx *ctx, const Pk4Problem &p, int mt) {
-    if (mt == 1) return true;
+    if (mt == 1 || p.w.unrounded) return true;
     if (mt > 3 || !tune(ctx, OXQ_TUNE_PK4_FOLD, 1)) return false;
     const int gemv_rows = p.w.gemv_rows ? p.w.gemv_rows : 16;
     if (p.w.dtype == OXQ_F16) return true;
     return mt == 2 && p.M <= gemv_rows;
+}
+
+// Row tiles (of 16) a workgroup of pk4_mfma_kernel takes.  Unrounded layers run the folded form only, two at a time; in f16
+// three where they are all (4096 x 11000, 4-bit, 40 rows: 12.2 us, 18.5 as two tiles of 32; but 128 rows 37.3, 31.9 as
+// tiles of 32), except beside two sets of pairs, where three spill (4096 x 11008, groups of 64, 40 rows: 23.8, 21.2 as two).
+static int pk4_row_tiles(const Pk4Problem &p) {
+    if (!p.w.unrounded) return (int)std::min<int64_t>(4, ceil_div(p.M, 16));
+    const bool three = p.w.dtype == OXQ_F16 && p.M <= 48 && pk4_sets(p.w.group_shift) != 2;
+    return (int)std::min<int64_t>(three ? 3 : 2, ceil_div(p.M, 16));
 }
 
 template <typename TT, int BITS>
@@ -1085,7 +1101,7 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (pk4_gemm_takes(ctx, p)) return launch_pk4_gemm(ctx, s, p);  // prefill sizes, either layout
     if (p.w.strip == 16) return launch_pk4n_forward(ctx, s, p);
     const int64_t M = p.M;
-    const int mt = M > 48 ? 4 : (int)ceil_div(M, 16);
+    const int mt = pk4_row_tiles(p);
     const int NB = (int)ceil_div(p.w.K, 128), sets = pk4_sets(p.w.group_shift);
     const int64_t strips = ceil_div(p.w.N, 64);
     // Few column strips and a long K (a down projection: N = 4096 is 64 strips for 256 CUs):
@@ -1163,7 +1179,7 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
         if (rc != OXQ_OK || ks == 1) return rc;
         return launch_splitk_reduce(ctx, s, (const float *)ctx->workspace, p.bias, p.y, M, p.w.N, ks, p.w.dtype);
     }
-    if (tune(ctx, OXQ_TUNE_PK4_T64, 1) && pk4_tile64_takes(p, ks)) {
+    if (tune(ctx, OXQ_TUNE_PK4_T64, 1) && !p.w.unrounded && pk4_tile64_takes(p, ks)) {
         Pk4Problem q = p;
         q.ws = ctx->workspace;
         return launch_pk4_tile64(ctx, s, q);

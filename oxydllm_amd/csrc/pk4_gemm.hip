@@ -207,12 +207,28 @@ static bool pk4_mid_decode(double cus, const Pk4Problem &p) {
     const double strips = (double)ceil_div(p.w.N, (int64_t)64);
     return 1.8 * std::ceil(strips / (2 * cus)) < std::ceil(strips / cus);
 }
+// Unrounded layers: the folded prefill form (one workgroup a CU, whole rounds) against row tiles of 32 of pk4_mfma_kernel, whose
+// time goes with their number.  A round costs as much as `unit` tiles on every CU, fitted to 4096 x 11008, 11008 x 4096,
+// 4096 x 4096, 2048 x 28672 and 4096 x 11000 at 33 - 2048 rows in both types (us, row tiles / prefill form, f16 except the
+// last): GPTQ 4-bit groups of 64 4096 x 11008 at 256 / 512 / 2048 rows 67.9 / 86.3, 128.6 / 88.7, 493 / 265; groups of 32
+// 4096 x 4096 at 1024 / 2048 rows 100 / 116, 195 / 124; AWQ 8-bit groups of 64 11008 x 4096 at 512 / 1024 rows 131 / 235,
+// 267 / 235 (bf16).
+static bool pk4_fold_prefill(double cus, const Pk4Problem &p) {
+    static const double unit4[3] = {6.3, 8.0, 9.0}, unit8[3] = {4.8, 5.7, 6.9};  // groups of 128 rows and more, 64, 32
+    const int sets = pk4_sets(p.w.group_shift), i = sets == 1 ? 0 : sets == 2 ? 1 : 2;
+    // the row tiles address the whole of x with 32 bits and are one grid dimension
+    if ((uint64_t)p.M * (uint64_t)p.w.K * 2 >= (1ull << 31) || ceil_div(p.M, (int64_t)32) > 65535) return true;
+    const int64_t strips = ceil_div(p.w.N, (int64_t)64);
+    const double rounds = std::ceil((double)(ceil_div(strips, (int64_t)PK4G_STRIPS) * ceil_div(p.M, (int64_t)64)) / cus);
+    return rounds * (p.w.bits == 4 ? unit4[i] : unit8[i]) < (double)(strips * ceil_div(p.M, (int64_t)32)) / cus;
+}
 static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int64_t min_m = tune(ctx, OXQ_TUNE_PK4_GEMM_MIN_M, pk4_sets(p.w.group_shift) > 1 ? 49 : pk4_mid_decode(cus, p) ? 33 : 65);
     if (min_m <= 0 || (p.w.bits != 4 && p.w.bits != 8) || (p.act && p.w.strip == 16) || p.M < min_m) return {0, 1};
     if (p.w.bits == 8 && p.w.strip == 16) return {0, 1};  // (16-column strips are a 4-bit layout)
     const int forced = tune(ctx, OXQ_TUNE_PK4_GEMM_ROWS, 0), forced_ks = tune(ctx, OXQ_TUNE_PK4_GEMM_KS, 0);
+    if (p.w.unrounded) return {forced || pk4_fold_prefill(cus, p) ? 64 : 0, 1};
     if (forced_ks == 4) return {64, 4};
     if (forced == 64 || forced == 128) return {forced, 1};
     if (p.M <= 64 && pk4_mid_decode(cus, p) && forced_ks != 1) return {64, 4};
@@ -274,14 +290,15 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_%s_%s_r%dx%d%s%s%s", p.w.bits, form.ks > 1 && p.M <= 64 ? "mid" : "gemm",
-             p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw, form.ks > 1 ? "k4" : "", p.w.strip == 16 ? "_n16" : "",
+    snprintf(name, sizeof name, "pk%d_%s_%s_r%dx%d%s%s%s%s", p.w.bits, form.ks > 1 && p.M <= 64 ? "mid" : "gemm",
+             p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw, form.ks > 1 ? "k4" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
              p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if ((uint64_t)rows * (uint64_t)p.w.K * 2 >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: K too large");
     if (((uintptr_t)p.x | (uintptr_t)p.y) & 15) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: x and y must be 16-byte aligned");
     if (p.bias && ((uintptr_t)p.bias & 7)) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: bias must be 8-byte aligned");
+    if (p.w.unrounded) return launch_pk4_gemm_fold(s, grid, p, (int)NG, (int)RT);
     if (form.ks == 4) return launch_pk4_mid(s, grid, p, (int)NG);
     if (pk4_sets(p.w.group_shift) > 1) return launch_pk4_gemm_fine(s, grid, p, rows, (int)NG, (int)RT);
     const bool f16 = p.w.dtype == OXQ_F16;

@@ -8,9 +8,35 @@ namespace oxq {
 
 constexpr int PK4G_STRIPS = 8;  // strips (= waves) of a workgroup
 
+// The integers bias + q of the folded form as pairs of 16-bit floats, with the smallest bias that a pair comes out of the
+// word with two instructions: what the bias adds to a group's sum is taken out again in f32, and the rounding of that sum
+// grows with it.  pair(): row pair pp of column f from word pp of the column's half; offset(): what the copy's
+// pair word (-(bias_f + z) of Pk4T) lacks to -(BIAS + z).
+template <typename TT, int BITS> struct Pk4Fold {
+    static constexpr bool BF = TT::DTYPE == BF16Traits::DTYPE;
+    static constexpr int AT = BF ? 3 : 6;  // 4 bits: mantissa bit of the nibble's lowest at an exponent of 16
+    static constexpr float BIAS = BITS == 4 ? 16.0f : BF ? 0.0f : 256.0f;
+    __device__ static __forceinline__ uint32_t pair(uint32_t word, int f) {
+        if constexpr (BITS == 4) {
+            const int left = AT - 4 * f;
+            return ((left >= 0 ? word << left : word >> -left) & ((0xFu << AT) * 0x10001u)) | (BF ? 0x41804180u : 0x4C004C00u);
+        } else if constexpr (BF) {
+            return TT::unpack_bytes((f & 1) ? (word >> 8) : word);
+        } else {
+            return (((f & 1) ? word >> 6 : word << 2) & 0x03FC03FCu) | 0x5C005C00u;
+        }
+    }
+    __device__ static __forceinline__ float offset(int f) {
+        return BITS == 4 ? (BF ? 112.0f : (f & 1) ? 48.0f : 1008.0f) : BF ? 0.0f : 768.0f;
+    }
+};
+
 // Eight strips a workgroup, a wave takes every block of its strip.
 // SETS: as in pk4_mfma_kernel (groups of 128 rows and more, 64, 32).
-template <typename TT, int MT, int BITS, int SETS = 1>
+// FOLD (layers with `unrounded`): the folded form of pk4_mfma_kernel - the matrix cores multiply x by the integers, one
+// more MFMA a step against ones yields the row sums of x, and a group's sums enter the accumulators through
+// s * (sum - (bias + z) * rowsum), all f32.
+template <typename TT, int MT, int BITS, int SETS = 1, bool FOLD = false>
 __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
                                                        const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                        int M, int K, int N, int NG, int RT, int act) {
@@ -127,9 +153,22 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         }
         load_z(i + 1, set);
         };
+        float4_t tmp[FOLD ? MT : 1][4], tmps[FOLD ? MT : 1];  // a group's sums of the folded form
+        auto fold = [&](int set) {
+            zs_words(zring[set], zv);
+            load_z(i + 1, set);
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                const float sf = TT::to_f32((uint16_t)(zv[f] >> 16)), nz = TT::to_f32((uint16_t)(zv[f] & 0xFFFFu)) + Pk4Fold<TT, BITS>::offset(f);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[mt][f][e] = fmaf(sf, fmaf(nz, tmps[mt][e], tmp[mt][f][e]), acc[mt][f][e]);
+            }
+        };
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
-            if (st % SPS == 0) constants(st / SPS);
+            if (!FOLD && st % SPS == 0) constants(st / SPS);
             uint32_t wp[WL][4];
 #pragma unroll
             for (int h = 0; h < WL; ++h) {
@@ -146,7 +185,21 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) acc[mt][f] = Ops::mfma(a[mt], b, acc[mt][f]);
             };
-            if constexpr (BF && BITS == 4 && MT == 4) {
+            if constexpr (FOLD) {
+                const bool fresh = st % SPS == 0;  // a group's sums start from zero: no clearing
+                const float4_t zero4 = float4_t{0.f, 0.f, 0.f, 0.f};
+                const uint32_t ones[4] = {TT::ONES, TT::ONES, TT::ONES, TT::ONES};
+#pragma unroll
+                for (int f = 0; f < 4; ++f) {
+                    uint32_t b[4];
+#pragma unroll
+                    for (int pp = 0; pp < 4; ++pp) b[pp] = Pk4Fold<TT, BITS>::pair(wp[(f >> 1) % WL][pp], f);
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) tmp[mt][f] = Ops::mfma(a[mt], b, fresh ? zero4 : tmp[mt][f]);
+                }
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) tmps[mt] = Ops::mfma(a[mt], ones, fresh ? zero4 : tmps[mt]);
+            } else if constexpr (BF && BITS == 4 && MT == 4) {
                 // 64-row workgroups share a CU in pairs with up to 128 registers, which two columns at a time exceed
                 // (135: 4096 x 14336 at 1536 rows 195 -> 216 us): one column, a conversion a weight.  The high nibbles
                 // stay where they are: bytes of 16 q, times s / 16.
@@ -194,6 +247,10 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
                 }
             }
             load_w(i + 1, st);  // into the registers this step has just left
+            if constexpr (FOLD) {
+                if ((st + 1) % SPS == 0) fold(st / SPS);
+                __builtin_amdgcn_sched_barrier(0);  // one step's operands in the registers at a time
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
         pk4g_wait_vmcnt<RING>();  // this wave's part of the next block of x is in LDS; its ring loads may still fly
@@ -257,12 +314,12 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         }
 }
 
-template <typename TT, int MT, int BITS, int SETS>
+template <typename TT, int MT, int BITS, int SETS, bool FOLD = false>
 static int pk4_gemm_wide_go(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT) {
     static LdsGrant grant;  // one per instantiation
     const size_t lds = (size_t)2 * 16 * MT * 256;
-    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_gemm_kernel<TT, MT, BITS, SETS>, lds));
-    hipLaunchKernelGGL((pk4_gemm_kernel<TT, MT, BITS, SETS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
+    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_gemm_kernel<TT, MT, BITS, SETS, FOLD>, lds));
+    hipLaunchKernelGGL((pk4_gemm_kernel<TT, MT, BITS, SETS, FOLD>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
                        (uint16_t *)p.y, (int)p.M, (int)p.w.K, (int)p.w.N, NG, RT, p.act);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;

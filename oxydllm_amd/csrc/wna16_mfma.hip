@@ -703,7 +703,7 @@ static bool transient_repack_fits(const oxq_ctx *ctx, const Wna16Problem &p) {
 }
 static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     Pk4Weights w{(uint32_t *)ctx->workspace, nullptr, p.K, p.N, p.group_shift, p.dtype, p.bits, 0,
-                   p.pack_dim == OXQ_PACK_IN ? 32 : 16, 64};
+                   p.pack_dim == OXQ_PACK_IN ? 32 : 16, 64, pk4_unrounded(p)};
     int rc = launch_pk4_prepack(ctx, s, p, w);
     if (rc != OXQ_OK) return rc;
     Pk4Problem q;

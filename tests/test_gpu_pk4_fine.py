@@ -2,7 +2,8 @@
 inside a strip of 64 columns: dense dequant bit for bit, products against the oracle.
 
 Tolerance as in the other parity tests, 2e-3 relative / 1e-2 absolute on the f32-accumulated product (bf16 outputs
-plus their own half ulp); the reference rounds the weights where the resident layers do (test helper)."""
+plus their own half ulp).  The reference rounds the weights of 4-bit AWQ layers where the resident layers do (test helper);
+those of GPTQ and 8-bit AWQ layers of these shapes are never rounded."""
 import sys
 
 import numpy as np
@@ -35,6 +36,57 @@ def build(kind, bits, K, N, g, dt, tdt, seed, bias=None):
     return layer, args, w
 
 
+def rounds(kind, bits, m, dt):
+    return (kind, bits) == ("awq", 4) and resident_rounds_weights(m, dt, False)
+
+
+def correctly_rounded_share(y, x, w, dt, tdt, bias=None):
+    """Share of outputs that are the 64-bit product rounded once to the output type.  The f32 sums of unrounded weights
+    move one over a rounding boundary in 0.1 - 3 % of the cases (bias of the folded integers against the result's ulp);
+    weights rounded to the type miss it in 40 %."""
+    ref = round_x(x, dt).astype(np.float64) @ w.astype(np.float64).T
+    if bias is not None:
+        ref = ref + round_x(bias, dt)
+    return (y.cpu() == torch.from_numpy(ref).to(tdt)).double().mean().item()
+
+
+@pytest.mark.parametrize("dtn", ["f16", "bf16"])
+@pytest.mark.parametrize("kind,bits", [("awq", 8), ("gptq", 4), ("gptq", 8)])
+@pytest.mark.parametrize("K,N,g", [(1024, 256, 32), (1088, 328, 64), (1024, 328, 128), (672, 1096, 32), (2048, 264, 256)])
+def test_weights_stay_unrounded(kind, bits, K, N, g, dtn):
+    """GPTQ and 8-bit AWQ layers of these shapes and the stateless tile op on their tensors, in every form: one and two
+    row tiles of the ring kernel, the prefill kernel at whole and ragged tiles of 64 rows, an unfilled group of strips."""
+    dt, tdt = (oracle.F16, torch.float16) if dtn == "f16" else (oracle.BF16, torch.bfloat16)
+    rng = np.random.default_rng(K + N + g + bits)
+    layer, args, w = build(kind, bits, K, N, g, dt, tdt, K + bits)
+    assert layer.prepacked
+    for m in (16, 17, 32, 33, 48, 49, 64, 65, 128, 200, 700):
+        x = rng.standard_normal((m, K)).astype(np.float32)
+        y = layer.forward(to_dev(x, tdt))
+        kernel = ops.default_context().last_plan()["kernel"]
+        say(f"unrounded {kind}{bits} {dtn} {K}x{N} g={g} m={m} {kernel}")
+        share = correctly_rounded_share(y, x, w, dt, tdt)
+        assert share > 0.9, f"{kernel}: {share:.3f} of the outputs correctly rounded"
+        if m in (17, 200):
+            y = ops.mpp_quant_matmul(to_dev(x, tdt), *args, bits, ops.PACK_IN if kind == "gptq" else ops.PACK_OUT)
+            share = correctly_rounded_share(y, x, w, dt, tdt)
+            assert share > 0.9, f"stateless, {ops.default_context().last_plan()['kernel']}: {share:.3f}"
+
+
+@pytest.mark.parametrize("kind", ["awq", "gptq"])
+def test_fused_activation_is_that_of_the_plain_layer(kind):
+    """The gate|up epilogue of the folded prefill form and of the ring kernel: the plain layer's bits."""
+    K, N, m_all, tdt = 1088, 1152, (17, 64, 65, 130), torch.bfloat16
+    _, args, _ = build(kind, 8, K, N, 64, oracle.BF16, tdt, 11)
+    pack = ops.PACK_IN if kind == "gptq" else ops.PACK_OUT
+    fused = ops.PackedQuantLinear(8, pack, *args, None, tdt, gate_up_act=ops.ACT_GATED_SILU)
+    plain = ops.PackedQuantLinear(8, pack, *args, None, tdt)
+    for m in m_all:
+        say(f"fused activation {kind}8 m={m}")
+        x = to_dev(np.random.default_rng(m).standard_normal((m, K)).astype(np.float32) * 0.25, tdt)
+        np.testing.assert_array_equal(bits_of(fused.forward(x)), bits_of(ops.gated_activation(plain.forward(x), ops.ACT_GATED_SILU)))
+
+
 @pytest.mark.parametrize("dtn", ["f16", "bf16"])
 @pytest.mark.parametrize("kind,bits", [("awq", 4), ("awq", 8), ("gptq", 4), ("gptq", 8)])
 @pytest.mark.parametrize("K,N,g", [(1024, 256, 32), (1024, 264, 64), (672, 520, 32), (1088, 328, 64), (1024, 328, 128)])
@@ -51,7 +103,7 @@ def test_fine_groups_and_ragged_edges(kind, bits, K, N, g, dtn):
     for m in (1, 4, 5, 9, 16, 17, 33, 49, 64, 65, 130, 700):
         x = rng.standard_normal((m, K)).astype(np.float32)
         xd = to_dev(x, tdt)
-        wr = oracle.round_through(w, dt) if resident_rounds_weights(m, dt, kind == "gptq") else w
+        wr = oracle.round_through(w, dt) if rounds(kind, bits, m, dt) else w
         ref = oracle.matmul_nt_f32(round_x(x, dt), wr, bias)
         y = layer.forward(xd)
         kernel = ops.default_context().last_plan()["kernel"]
@@ -69,7 +121,7 @@ def test_fine_groups_and_ragged_edges(kind, bits, K, N, g, dtn):
 def test_fine_prefill_forms(tune_rows):
     """The eight-strip forms, forced: an unfilled last group of strips, K inside a block, every row-tile remainder class."""
     from tests.helpers import tune
-    for dtn, bits, K, N, g in [("f16", 4, 672, 1096, 32), ("bf16", 8, 1088, 584, 64)]:
+    for dtn, bits, K, N, g in [("f16", 4, 672, 1096, 32), ("bf16", 4, 1088, 584, 64)]:
         dt, tdt = (oracle.F16, torch.float16) if dtn == "f16" else (oracle.BF16, torch.bfloat16)
         layer, _, w = build("awq", bits, K, N, g, dt, tdt, 7)
         tune("OXQ_PK4_GEMM_ROWS", tune_rows)
@@ -90,5 +142,5 @@ def test_stateless_op_on_fine_groups(kind, bits, K, N, g):
         _, args, w = build(kind, bits, K, N, g, dt, tdt, 3)
         x = np.random.default_rng(m).standard_normal((m, K)).astype(np.float32)
         y = ops.mpp_quant_matmul(to_dev(x, tdt), *args, bits, ops.PACK_IN if kind == "gptq" else ops.PACK_OUT)
-        wr = oracle.round_through(w, dt) if resident_rounds_weights(m, dt, kind == "gptq") else w
+        wr = oracle.round_through(w, dt) if rounds(kind, bits, m, dt) else w
         assert_close(y, oracle.matmul_nt_f32(round_x(x, dt), wr), f"{kind}{bits} m{m}")
