@@ -912,13 +912,16 @@ static bool pk4_folds(const oxq_ctx *ctx, const Pk4Problem &p, int mt) {
     return mt == 2 && p.M <= gemv_rows;
 }
 
-// Row tiles (of 16) a workgroup of pk4_mfma_kernel takes.  Unrounded layers run the folded form only, two at a time; in f16
-// three where they are all (4096 x 11000, 4-bit, 40 rows: 12.2 us, 18.5 as two tiles of 32; but 128 rows 37.3, 31.9 as
-// tiles of 32), except beside two sets of pairs, where three spill (4096 x 11008, groups of 64, 40 rows: 23.8, 21.2 as two).
-static int pk4_row_tiles(const Pk4Problem &p) {
-    if (!p.w.unrounded) return (int)std::min<int64_t>(4, ceil_div(p.M, 16));
-    const bool three = p.w.dtype == OXQ_F16 && p.M <= 48 && pk4_sets(p.w.group_shift) != 2;
-    return (int)std::min<int64_t>(three ? 3 : 2, ceil_div(p.M, 16));
+// Row tiles (of 16) a workgroup of pk4_mfma_kernel takes: up to four, of which one to three run folded in f16 (pk4_folds).  Beside
+// two sets of pairs three tiles of folded sums spill: 33 - 48 rows then run as two tiles of 32 (4096 x 11008, groups of 64,
+// f16, 33 / 40 / 48 rows: 23.7 / 23.7 / 24.0 -> 20.9 / 20.9 / 21.3 us; 5120 x 6144 at 40 rows 20.6 -> 12.5).  Unrounded layers run the folded form only, two tiles at a time and
+// three in f16 where they are all (4096 x 11000, 4-bit, 40 rows: 12.2 us, 18.5 as two tiles of 32; but 128 rows 37.3, 31.9 as
+// tiles of 32).
+static int pk4_row_tiles(const oxq_ctx *ctx, const Pk4Problem &p) {
+    const int all = (int)std::min<int64_t>(4, ceil_div(p.M, 16));
+    const bool f16 = p.w.dtype == OXQ_F16, spills = pk4_sets(p.w.group_shift) == 2;
+    if (p.w.unrounded) return std::min(all, f16 && p.M <= 48 && !spills ? 3 : 2);
+    return all == 3 && spills && pk4_folds(ctx, p, 3) ? 2 : all;
 }
 
 template <typename TT, int BITS>
@@ -1101,7 +1104,7 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (pk4_gemm_takes(ctx, p)) return launch_pk4_gemm(ctx, s, p);  // prefill sizes, either layout
     if (p.w.strip == 16) return launch_pk4n_forward(ctx, s, p);
     const int64_t M = p.M;
-    const int mt = pk4_row_tiles(p);
+    const int mt = pk4_row_tiles(ctx, p);
     const int NB = (int)ceil_div(p.w.K, 128), sets = pk4_sets(p.w.group_shift);
     const int64_t strips = ceil_div(p.w.N, 64);
     // Few column strips and a long K (a down projection: N = 4096 is 64 strips for 256 CUs):

@@ -26,7 +26,7 @@ static int fine_by_mt(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &
         return fold ? pk4_mfma_go<TT, BITS, 2, true, WD, 8, false, 0, SETS>(ctx, s, grid, p, bslice)
                     : pk4_mfma_go<TT, BITS, 2, false, WD, 8, false, 0, SETS>(ctx, s, grid, p, bslice);
     case 3:
-        if constexpr (TT::DTYPE == F16Traits::DTYPE)
+        if constexpr (TT::DTYPE == F16Traits::DTYPE && SETS == 4)  // (two sets: pk4_row_tiles)
             if (fold) return pk4_mfma_go<TT, BITS, 3, true, WD, 12, false, 0, SETS>(ctx, s, grid, p, bslice);
         return pk4_mfma_go<TT, BITS, 3, false, WD, 12, false, 0, SETS>(ctx, s, grid, p, bslice);
     default: return pk4_mfma_go<TT, BITS, 4, false, WD, 16, false, 0, SETS>(ctx, s, grid, p, bslice);

@@ -1,0 +1,41 @@
+"""Which kernel a resident packed layer runs, asked of a plan-only ctx: no GPU needed."""
+import ctypes as C
+
+import pytest
+
+from oxydllm_amd import _lib, ops
+from tests.helpers import fake
+
+
+def kernels(pack, bits, K, N, g, dt, rows):
+    lib, plan = _lib.load(), ops.Context(plan_only=True)
+    pf = 32 // bits
+    qw = fake((K, N // pf) if pack == ops.PACK_OUT else (K // pf, N), _lib.I32)
+    h = C.c_void_p()
+    rc = lib.oxq_packed_quant_linear_new(plan.handle, bits, pack, C.byref(qw), C.byref(fake((K // g, N // pf), _lib.I32)),
+                                         C.byref(fake((K // g, N), dt)), None, dt, C.byref(h))
+    assert rc == 0, lib.oxq_last_error().decode()
+    out = []
+    for m in rows:
+        assert lib.oxq_packed_quant_linear_forward(h, None, C.byref(fake((m, K), dt)), C.byref(fake((m, N), dt))) == 0
+        out.append((plan.last_plan()["kernel"], plan.last_plan()["grid"][2]))
+    lib.oxq_packed_quant_linear_free(h)
+    return out
+
+
+def test_no_three_tiles_of_folded_sums_beside_two_sets_of_pairs():
+    """f16, groups of 64, 33 - 48 rows: that form spills; the rows run as two tiles of 32, still folded."""
+    rows = (33, 40, 48)
+    assert kernels(ops.PACK_OUT, 4, 4096, 11008, 64, _lib.F16, rows) == [("pk4_mfma_f16_mt2_gs_g64", 2)] * 3
+    assert kernels(ops.PACK_OUT, 4, 4096, 11008, 32, _lib.F16, rows) == [("pk4_mfma_f16_mt3_gs_g32", 1)] * 3
+    assert kernels(ops.PACK_OUT, 4, 4096, 11008, 64, _lib.BF16, rows) == [("pk4_mfma_bf16_mt3_g64", 1)] * 3
+    assert kernels(ops.PACK_OUT, 4, 4096, 11008, 64, _lib.F16, (32, 49)) == [("pk4_mfma_f16_mt2_gs_g64", 1), ("pk4_mfma_f16_mt4_g64", 1)]
+
+
+@pytest.mark.parametrize("pack,bits,K,N,g", [(ops.PACK_IN, 4, 4096, 11008, 64), (ops.PACK_IN, 8, 4096, 4096, 32),
+                                             (ops.PACK_OUT, 8, 4096, 11000, 128), (ops.PACK_IN, 4, 4128, 4096, 32)])
+@pytest.mark.parametrize("dt", [_lib.F16, _lib.BF16])
+def test_unrounded_layers_run_folded_forms_only(pack, bits, K, N, g, dt):
+    rows = (1, 16, 17, 32, 33, 48, 49, 64, 65, 128, 200, 512, 1024, 2048, 4096, 1 << 20)
+    for m, (kernel, _) in zip(rows, kernels(pack, bits, K, N, g, dt, rows)):
+        assert "_gs" in kernel and "_mt4" not in kernel, (m, kernel)
