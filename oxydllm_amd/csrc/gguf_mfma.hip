@@ -413,22 +413,40 @@ template <int FMT> struct GgmChunk {
 };
 
 // The B operand with the smallest bias that leaves the integers exact, for f32 activations: 16 + q (4-bit formats), 32 + q
-// (5-bit), 64 + q (Q6_K).  The bias and the format's offset come out in the same f32 accumulator, and what is taken out
-// there costs precision in proportion to its size: with 128 + q the sums carry seven times the rounding of the integers'
-// own products.  Bytes (Q8_0) have no bias.  A pair is built as for 128 + q, with the bits moved to the mantissa position
-// that the exponent asks for: as many instructions.
+// (5-bit), 64 + q (Q6_K).  The bias and the format's offset come out in the same f32 accumulator, and the rounding of what
+// is taken out there grows with its size: with 128 + q the sums carry seven times that of the integers' own products.  Bytes
+// (Q8_0) have no bias.  A pair is built as for 128 + q, with the bits moved to the mantissa position that the exponent asks
+// for: as many instructions.
+//
+// Q4_1 and Q5_1, d q + m with q >= 0: no bias at all - nibbles widened as f8 codes, five-bit bytes through f32 - and the row's
+// sum against ones.  Nothing is taken out, so an infinite x gives the infinity that the vector kernels give (in the other
+// formats the offset or the subtracted minimum makes it NaN there and here).  Widened through f32 Q4_1 took up to 1.25 x as
+// long; Q5_1 at 3 - 16 rows is at 1.03 - 1.13 x the biased operand's time.
 template <int FMT> struct GgmSmallBias {
+    static constexpr bool PLAIN = FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q5_1;
+    static constexpr bool FOURS = FMT == OXQ_GGUF_Q4_1;  // pair i of the operand holds elements i and i + 4, else 2 i and 2 i + 1
     static constexpr bool NIB = FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q4_K;
     static constexpr float BIAS = NIB ? 16.f : ggm_fifth_bit<FMT> ? 32.f : FMT == OXQ_GGUF_Q6_K ? 64.f : 0.f;
     // the constant that takes bias and offset out (the minimum's term divides by it)
-    static constexpr float NEG = -(BIAS + (FMT == OXQ_GGUF_Q4_0 ? 8.f : FMT == OXQ_GGUF_Q5_0 ? 16.f : FMT == OXQ_GGUF_Q6_K ? 32.f : FMT == OXQ_GGUF_Q8_0 ? 128.f : 0.f));
+    static constexpr float NEG = PLAIN ? 1.f : -(BIAS + (FMT == OXQ_GGUF_Q4_0 ? 8.f : FMT == OXQ_GGUF_Q5_0 ? 16.f : FMT == OXQ_GGUF_Q6_K ? 32.f : FMT == OXQ_GGUF_Q8_0 ? 128.f : 0.f));
     static constexpr uint32_t NEG_PAIR = (__builtin_bit_cast(uint32_t, NEG) >> 16) | (__builtin_bit_cast(uint32_t, NEG) & 0xFFFF0000u);
     static constexpr int AT = NIB ? 3 : ggm_fifth_bit<FMT> ? 2 : 1;  // mantissa bit of the nibble's lowest
     static constexpr uint32_t EXP = NIB ? 0x41804180u : ggm_fifth_bit<FMT> ? 0x42004200u : 0x42804280u;
     static constexpr uint32_t M0 = (0xFu << AT) * 0x10001u, M1 = (ggm_fifth_bit<FMT> ? 0x40u : 0x60u) * 0x10001u;
     __device__ static __forceinline__ uint32_t move(uint32_t v, int left) { return left >= 0 ? v << left : v >> -left; }
     __device__ static __forceinline__ void operand(const GgmChunk<FMT> &w, int st, uint32_t (&b)[4], const NibbleMasks &nm) {
-        if constexpr (NIB) {
+        if constexpr (FMT == OXQ_GGUF_Q4_1) {  // nibbles as f8 codes (pk4g_widen): elements (0, 4), (1, 5), (2, 6), (3, 7)
+            const uint32_t lo = w.q[0][st] & 0x0F0F0F0Fu, hi = (w.q[0][st] >> 4) & 0x0F0F0F0Fu;
+            b[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false));
+            b[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
+            b[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
+            b[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
+        } else if constexpr (PLAIN) {  // pair pp: nibble pp and bit 4 st + pp of each half; bytes 0, 2 hold pair 0 or 1, bytes 1, 3 pair 2 or 3
+            const uint32_t h = w.qh[0] >> (4 * st);
+            const uint32_t lo = (w.q[0][st] & 0x0F0F0F0Fu) | ((h & 0x00010001u) << 4) | ((h & 0x00040004u) << 10);
+            const uint32_t hi = ((w.q[0][st] >> 4) & 0x0F0F0F0Fu) | ((h & 0x00020002u) << 3) | ((h & 0x00080008u) << 9);
+            b[0] = ggm_bytes02(lo), b[1] = ggm_bytes02(hi), b[2] = ggm_bytes13(lo), b[3] = ggm_bytes13(hi);
+        } else if constexpr (NIB) {
 #pragma unroll
             for (int pp = 0; pp < 4; ++pp) b[pp] = (move(w.q[0][st], AT - 4 * pp) & nm.m0) | EXP;
         } else if constexpr (ggm_fifth_bit<FMT>) {  // the bit of pair pp: bit 4 st + pp -> 6
@@ -527,20 +545,25 @@ __device__ __forceinline__ void ggm_epilogue_f32(const float4_t (&acc)[MT][NS], 
         }
 }
 // Eight f32 as three bf16 pieces whose sum they are, exactly: truncated to 8 significant bits, the rest truncated, the
-// rest of that (at most 8 bits).
-__device__ __forceinline__ void ggm_split3_pair(uint32_t a, uint32_t b, uint32_t (&p)[3]) {
-    const float ra = __builtin_bit_cast(float, a) - __builtin_bit_cast(float, a & 0xFFFF0000u);
-    const float rb = __builtin_bit_cast(float, b) - __builtin_bit_cast(float, b & 0xFFFF0000u);
+// rest of that (at most 8 bits).  INF: an infinity is its first piece alone (formats whose sums can keep one).
+template <bool INF> __device__ __forceinline__ void ggm_split3_pair(uint32_t a, uint32_t b, uint32_t (&p)[3]) {
+    float ra = __builtin_bit_cast(float, a) - __builtin_bit_cast(float, a & 0xFFFF0000u);
+    float rb = __builtin_bit_cast(float, b) - __builtin_bit_cast(float, b & 0xFFFF0000u);
+    if constexpr (INF) {
+        if (__builtin_isinf(__builtin_bit_cast(float, a))) ra = 0.f;
+        if (__builtin_isinf(__builtin_bit_cast(float, b))) rb = 0.f;
+    }
     const uint32_t am = __builtin_bit_cast(uint32_t, ra), bm = __builtin_bit_cast(uint32_t, rb);
     const float sa = ra - __builtin_bit_cast(float, am & 0xFFFF0000u), sb = rb - __builtin_bit_cast(float, bm & 0xFFFF0000u);
     p[0] = pack_hi16(a, b), p[1] = pack_hi16(am, bm);
     p[2] = pack_hi16(__builtin_bit_cast(uint32_t, sa), __builtin_bit_cast(uint32_t, sb));
 }
-__device__ __forceinline__ void ggm_split3(const u32x4_t &v0, const u32x4_t &v1, u32x4_t (&p)[3]) {
+template <bool INF, bool FOURS> __device__ __forceinline__ void ggm_split3(const u32x4_t &v0, const u32x4_t &v1, u32x4_t (&p)[3]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t t[3];
-        ggm_split3_pair(i < 2 ? v0[2 * i] : v1[2 * i - 4], i < 2 ? v0[2 * i + 1] : v1[2 * i - 3], t);
+        if constexpr (FOURS) ggm_split3_pair<INF>(v0[i], v1[i], t);
+        else ggm_split3_pair<INF>(i < 2 ? v0[2 * i] : v1[2 * i - 4], i < 2 ? v0[2 * i + 1] : v1[2 * i - 3], t);
         p[0][i] = t[0], p[1][i] = t[1], p[2][i] = t[2];
     }
 }
@@ -592,7 +615,7 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 #pragma unroll
     for (int q = 0; q < AQ; ++q) {
         const int r = ONE ? 0 : XF32 ? 4 * (q >> 1) + kb : 4 * q + kb;
-        const int at = ONE ? ni * 32 + kb * 8 : XF32 ? r * K * 4 + ni * 32 + (q & 1) * 16 : r * K * 2 + ni * 16;
+        const int at = ONE ? ni * 32 + kb * (GgmSmallBias<FMT>::FOURS ? 4 : 8) : XF32 ? r * K * 4 + ni * 32 + (q & 1) * 16 : r * K * 2 + ni * 16;
         voff_a[q] = r < xrows ? at : OOB;
     }
     // x in LDS: row r of the tile at r * 256, its sixteen 16-byte pieces XOR-swizzled by the row
@@ -622,7 +645,10 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
         const int c = cc0 + i;
 #pragma unroll
         for (int q = 0; q < AQ; ++q) {
-            if constexpr (ONE) {
+            if constexpr (ONE && GgmSmallBias<FMT>::FOURS) {
+                a[0][0] = __builtin_amdgcn_raw_buffer_load_b32(rx, voff_a[0], c * 512, 0);
+                a[0][1] = __builtin_amdgcn_raw_buffer_load_b32(rx, voff_a[0], c * 512 + 16, 0);
+            } else if constexpr (ONE) {
                 const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rx, voff_a[0], c * 512, 0);
                 a[0][0] = v[0], a[0][1] = v[1];
             } else {
@@ -641,6 +667,8 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int f = 0; f < NS; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr bool FOURS = XF32 && GgmSmallBias<FMT>::FOURS;
+    constexpr bool PLAIN = XF32 && GgmSmallBias<FMT>::PLAIN;  // the integers without a bias: their sums start from zero
     constexpr uint32_t NEGP = XF32 ? GgmSmallBias<FMT>::NEG_PAIR : F::NEG;
     const uint32_t neg[4] = {NEGP, NEGP, NEGP, NEGP};
     // the minimum's factor is per 128 (factors()); here the bias term is smaller
@@ -670,14 +698,14 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
         constexpr int CUR = decltype(cur_c)::value;
         if constexpr (ONE) {
             uint32_t part[3];
-            ggm_split3_pair(ar[CUR][0][0], ar[CUR][0][1], part);
+            ggm_split3_pair<PLAIN>(ar[CUR][0][0], ar[CUR][0][1], part);
 #pragma unroll
             for (int p = 0; p < 3; ++p) *(uint32_t *)(slot + p * 1024 + ((ni ^ (4 * p)) << 4) + kb * 4) = part[p];
         } else if constexpr (XF32) {
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 u32x4_t part[3];
-                ggm_split3(ar[CUR][2 * t], ar[CUR][2 * t + 1], part);
+                ggm_split3<PLAIN, FOURS>(ar[CUR][2 * t], ar[CUR][2 * t + 1], part);
 #pragma unroll
                 for (int p = 0; p < 3; ++p) *(u32x4_t *)(slot + (4 * t + p) * 1024 + a_wr[p]) = part[p];
             }
@@ -712,7 +740,7 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
                     for (int s4 = 0; s4 < 4; ++s4) {
                         uint32_t b[4];
                         operand(w, g + s4, b, nm);
-                        const float4_t t = mma(a[s4], b, tn[s4]);
+                        const float4_t t = mma(a[s4], b, PLAIN ? zero4 : tn[s4]);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) acc[0][f][e] = fmaf(f0[g + s4], t[e], acc[0][f][e]);
                     }
@@ -733,7 +761,7 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
                         uint32_t a[4];
                         load_a(st, mt, a);
                         const float4_t tn = mma(a, neg, zero4);
-                        const float4_t t = mma(a, b, tn);
+                        const float4_t t = mma(a, b, PLAIN ? zero4 : tn);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             acc[mt][f][e] = fmaf(f0[st], t[e], acc[mt][f][e]);

@@ -47,6 +47,28 @@ def test_f32_rows_on_the_matrix_core_copy(fmt, N, K):
 
 
 @pytest.mark.parametrize("fmt", FMTS)
+def test_infinite_and_nan_rows_of_f32(fmt):
+    """An infinity, and a NaN whose payload lies in the bits that the first piece drops, give what the vector kernels give and
+    stay in their row."""
+    N, K = 1024, 2048
+    data = to_dev(synth.gguf_weight(fmt, N, K, seed=fmt))
+    plain = ops.Context()
+    tune("OXQ_GGUF_MFMA", 0, plain)
+    layer, former = ops.QLinear(fmt, data, K, N, None, torch.float32), ops.QLinear(fmt, data, K, N, None, torch.float32, ctx=plain)
+    for m in (3, 8, 9):
+        x = to_dev(np.random.default_rng(m).standard_normal((m, K)).astype(np.float32))
+        x[0, 77], x[1, 1500] = float("inf"), -float("inf")
+        x.view(torch.int32)[2, 5] = 0x7F800001
+        say(f"gguf f32 infinities {synth.GGUF_NAMES[fmt]} m={m}")
+        got, want = layer.forward(x), former.forward(x)
+        assert "_f32_mfma" in layer.ctx.last_plan()["kernel"]
+        assert torch.equal(torch.nan_to_num(got[:3], 0.0, 1.0, -1.0), torch.nan_to_num(want[:3], 0.0, 1.0, -1.0))
+        assert bool(got[2].isnan().all()) and bool(got[3:].isfinite().all())
+        if fmt in (synth.GGUF_Q4_1, synth.GGUF_Q5_1):
+            assert got[0].isinf().sum() > N // 2 and got[1].isinf().sum() > N // 2
+
+
+@pytest.mark.parametrize("fmt", FMTS)
 @pytest.mark.parametrize("N,K", [(256, 4096), (1032, 2304), (640, 14336), (4100, 1024)])
 def test_prefill_rows_of_few_columns(fmt, N, K):
     data = synth.gguf_weight(fmt, N, K, seed=N + K + fmt)
