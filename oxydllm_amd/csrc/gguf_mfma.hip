@@ -541,7 +541,7 @@ __device__ __forceinline__ void ggm_epilogue_f32(const float4_t (&acc)[MT][NS], 
             for (int d = 1; d < NW; d *= 2)
 #pragma unroll
                 for (int s = 0; s < NW; s += 2 * d) w[s] += w[s + d];
-            const float v = w[0], v1 = __shfl_down(v, 16), v2 = __shfl_down(v, 32);
+            const float v = w[0] * (lane < 16 ? 1.0f : lane < 32 ? 0x1p-8f : 0x1p-16f), v1 = __shfl_down(v, 16), v2 = __shfl_down(v, 32);
             const int n = 16 * (NS * j + f) + lane;
             if (lane < 16 && n < N) {
                 const float tot = (v2 + v1) + v;
@@ -549,8 +549,9 @@ __device__ __forceinline__ void ggm_epilogue_f32(const float4_t (&acc)[MT][NS], 
             }
         }
 }
-// Eight f32 as three bf16 pieces whose sum they are, exactly: truncated to 8 significant bits, the rest truncated, the
-// rest of that (at most 8 bits).  INF: an infinity is its first piece alone (formats whose sums can keep one).
+// f32 as three bf16 pieces, exactly: truncated to 8 significant bits, 2^8 times the rest truncated, 2^16 times the rest of
+// that (at most 8 bits); the epilogue divides the pieces' sums again.  Unscaled, the second and third piece of values
+// below 1e-34 fall below bf16's normal range, where they lose bits (values around 1e-36: 5e-5 of the result).  INF: an infinity is its first piece alone (formats whose sums can keep one).
 template <bool INF> __device__ __forceinline__ void ggm_split3_pair(uint32_t a, uint32_t b, uint32_t (&p)[3]) {
     float ra = __builtin_bit_cast(float, a) - __builtin_bit_cast(float, a & 0xFFFF0000u);
     float rb = __builtin_bit_cast(float, b) - __builtin_bit_cast(float, b & 0xFFFF0000u);
@@ -558,8 +559,9 @@ template <bool INF> __device__ __forceinline__ void ggm_split3_pair(uint32_t a, 
         if (__builtin_isinf(__builtin_bit_cast(float, a))) ra = 0.f;
         if (__builtin_isinf(__builtin_bit_cast(float, b))) rb = 0.f;
     }
+    ra *= 256.0f, rb *= 256.0f;
     const uint32_t am = __builtin_bit_cast(uint32_t, ra), bm = __builtin_bit_cast(uint32_t, rb);
-    const float sa = ra - __builtin_bit_cast(float, am & 0xFFFF0000u), sb = rb - __builtin_bit_cast(float, bm & 0xFFFF0000u);
+    const float sa = 256.0f * (ra - __builtin_bit_cast(float, am & 0xFFFF0000u)), sb = 256.0f * (rb - __builtin_bit_cast(float, bm & 0xFFFF0000u));
     p[0] = pack_hi16(a, b), p[1] = pack_hi16(am, bm);
     p[2] = pack_hi16(__builtin_bit_cast(uint32_t, sa), __builtin_bit_cast(uint32_t, sb));
 }

@@ -67,6 +67,25 @@ def test_f32_rows_are_no_further_from_64_bits_than_the_vector_kernels(fmt, N, K)
 
 
 @pytest.mark.parametrize("fmt", FMTS)
+def test_small_f32_rows_keep_their_bits(fmt):
+    """Rows whose values lie near 1e-36 (one row: 1e-30 beside them): all three pieces of a value count, up to one row."""
+    N, K = 1032, 2048  # ragged: the matrix cores take every row count
+    layer = ops.QLinear(fmt, to_dev(synth.gguf_weight(fmt, N, K, seed=fmt)), K, N, None, torch.float32)
+    w = layer.dequantize().double()
+    for m in (1, 3, 8):
+        say(f"gguf f32 small values {synth.GGUF_NAMES[fmt]} m={m}")
+        x = to_dev(np.random.default_rng(m).standard_normal((m, K)).astype(np.float32)) * 1e-36
+        if m > 1:
+            x[1] *= 1e6
+        ref = x.double() @ w.T
+        y = layer.forward(x)
+        assert "_f32_mfma" in layer.ctx.last_plan()["kernel"]
+        for r in range(m):
+            err = ((y[r].double() - ref[r]).norm() / ref[r].norm()).item()
+            assert err < 4e-7, f"{synth.GGUF_NAMES[fmt]} m={m} row {r}: {err:.2e}"
+
+
+@pytest.mark.parametrize("fmt", FMTS)
 def test_infinite_and_nan_rows_of_f32(fmt):
     """An infinity, and a NaN whose payload lies in the bits that the first piece drops, give what the vector kernels give and
     stay in their row."""
