@@ -505,7 +505,8 @@ int oxq_qlinear_forward(oxq_qlinear *layer, void *stream, const oxq_tensor *x,
  * layer of those formats with at least 2^20 weights holds both copies (three times the layer's bytes with
  * weight_bytes): from three rows on - fewer on some shapes - the matrix cores multiply each f32 as the sum of three bf16
  * pieces, exact products in f32 sums, at any row count.  The tuning switch OXQ_PREPACK=0 turns the copies off,
- * OXQ_GGUF_MFMA=0 keeps the first layout alone.
+ * OXQ_GGUF_MFMA=0 keeps the first layout alone, OXQ_GGUF_MFMA=2 the matrix-core layout alone (twice the layer's bytes for an
+ * F32 layer too, whose one and two rows then run on it as well).
  * *resident = 1 if the layer holds a copy. */
 int oxq_qlinear_is_resident(const oxq_qlinear *layer, int *resident);
 /* Dense f32 [out_features, in_features] of the layer's weights, read from the copy when there is one:

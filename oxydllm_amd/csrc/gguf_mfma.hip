@@ -1137,6 +1137,9 @@ bool gguf_mfma_eligible(const oxq_ctx *ctx, int quant, int64_t K, int64_t N) {
 bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int act_dtype) {
     return gguf_mfma_eligible(ctx, quant, K, N) && (act_dtype == OXQ_BF16 || (act_dtype == OXQ_F32 && N * K >= (1 << 20)));
 }
+// Whether such a layer does without the rotated copy: bf16, and f32 where OXQ_GGUF_MFMA is 2 (one copy fewer; what one and two
+// rows then take stands below: up to 8 % more on layers of one round of strips).
+bool gguf_mfma_alone(const oxq_ctx *ctx, int act_dtype) { return act_dtype == OXQ_BF16 || tune(ctx, OXQ_TUNE_GGUF_MFMA, 1) == 2; }
 // f32 rows of a layer that has both copies: the vector GEMV's arithmetic grows with the rows and is slow on many short
 // strips; the matrix cores take four rows as one.  us on the rotated / the matrix-core copy, Q4_K, 1 / 2 / 4 / 8 rows:
 // 4096 x 4096 4.2 / 5.0 / 6.5 / 12.7 against 4.5 / 5.2 / 5.5 / 7.8, 14336 x 4096 10.7 / 13.3 / 17.8 / 35.2 against 10.0 / 11.7 /

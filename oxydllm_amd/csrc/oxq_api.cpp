@@ -845,7 +845,7 @@ static bool wcache_forward_gguf(oxq_ctx *ctx, hipStream_t s, const GgufProblem &
     if (!ctx->wcache_limit || ctx->plan_only) return false;
     const bool rotated = gguf_res_eligible(p.quant, p.K, p.N);
     const bool mfma = gguf_mfma_layer(ctx, p.quant, p.K, p.N, p.act_dtype) &&
-                      !(p.act_dtype == OXQ_F32 && rotated && !gguf_f32_on_mfma(ctx, p.M, p.K, p.N));
+                      (gguf_mfma_alone(ctx, p.act_dtype) || !rotated || gguf_f32_on_mfma(ctx, p.M, p.K, p.N));
     if (!mfma && !rotated) return false;
     const bool gemm = mfma && gguf_gemm_takes(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);  // prefill sizes, same copy
     const bool tiles = mfma && gguf_mfma_tiles(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);
@@ -2047,7 +2047,7 @@ static int build_resident_gguf(oxq_qlinear *l) {
     // f32 layer where it is large
     l->mfma = gguf_mfma_layer(ctx, l->quant, l->in_features, l->out_features, l->out_dtype) &&
               !(l->act && (l->out_features % 16 != 0 || l->out_dtype != OXQ_BF16));
-    l->rotated = !(l->mfma && l->out_dtype == OXQ_BF16) && gguf_res_eligible(l->quant, l->in_features, l->out_features);
+    l->rotated = !(l->mfma && gguf_mfma_alone(ctx, l->out_dtype)) && gguf_res_eligible(l->quant, l->in_features, l->out_features);
     if (!l->mfma && !l->rotated) return OXQ_OK;
     if (l->act && !l->mfma) return OXQ_OK;  // the caller reports it
     if (ctx->plan_only) {

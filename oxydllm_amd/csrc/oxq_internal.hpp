@@ -245,6 +245,7 @@ int launch_gguf_res_gemv(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);  //
 // matrix-core copy of a GGUF weight for 16-bit activations and its matmul (gguf_mfma.hip)
 bool gguf_mfma_eligible(const oxq_ctx *ctx, int quant, int64_t K, int64_t N);
 bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int act_dtype);
+bool gguf_mfma_alone(const oxq_ctx *ctx, int act_dtype);
 size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N);
 bool gguf_f32_on_mfma(const oxq_ctx *ctx, int64_t M, int64_t K, int64_t N);
 bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);

@@ -136,7 +136,8 @@ def test_switches_and_rows_beyond_the_kernel(fmt):
 
 
 def test_f32_layers_keep_the_rotated_copy():
-    """f32 activations are the reference's CPU contract (linear.rs:357-372): exact f32 arithmetic on the vector ALU."""
+    """f32 activations are the reference's CPU contract (linear.rs:357-372).  Layers below 2^20 weights run on the vector ALU
+    at every row count, larger ones on the matrix cores with f32 kept whole (test_gpu_gguf_slices_f32.py)."""
     fmt, N, K = synth.GGUF_Q4_K, 64, 512
     data = synth.gguf_weight(fmt, N, K, seed=41)
     layer = ops.QLinear(fmt, to_dev(data), K, N, None, torch.float32)

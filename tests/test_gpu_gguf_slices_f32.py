@@ -66,6 +66,29 @@ def test_f32_rows_are_no_further_from_64_bits_than_the_vector_kernels(fmt, N, K)
         assert err <= 1.04 * was, f"{synth.GGUF_NAMES[fmt]} m={m}: {err:.3e}, vector kernel {was:.3e}"
 
 
+def test_f32_layer_with_one_copy():
+    """OXQ_GGUF_MFMA = 2: the matrix-core copy alone, at every row count, and the memory of one copy less."""
+    fmt, N, K = synth.GGUF_Q8_0, 4096, 4096
+    data = to_dev(synth.gguf_weight(fmt, N, K, seed=9))
+    x = to_dev(np.random.default_rng(9).standard_normal((8, K)).astype(np.float32))
+    ctx, taken, layers = ops.Context(), [], []
+    for value in (2, None):
+        tune("OXQ_GGUF_MFMA", value, ctx)
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        layers.append(ops.QLinear(fmt, data, K, N, None, torch.float32, ctx=ctx))
+        taken.append(before - torch.cuda.mem_get_info()[0])
+    copy = 4096 * (4096 // 32) * 34
+    assert copy <= taken[0] < 1.3 * copy and 2 * copy <= taken[1] < 2.3 * copy, taken
+    for m in (1, 2, 8):
+        say(f"gguf f32 one copy m={m}")
+        y = layers[0].forward(x[:m])
+        assert "_f32_mfma" in ctx.last_plan()["kernel"]
+        want = layers[1].forward(x[:m])
+        assert ("_f32_mfma" in ctx.last_plan()["kernel"]) == (m > 2)
+        assert ((y - want).norm() / want.norm()).item() < 8e-7  # two forms, each within 4e-7 of the 64-bit product
+
+
 @pytest.mark.parametrize("fmt", FMTS)
 def test_small_f32_rows_keep_their_bits(fmt):
     """Rows whose values lie near 1e-36 (one row: 1e-30 beside them): all three pieces of a value count, up to one row."""
