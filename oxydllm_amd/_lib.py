@@ -208,7 +208,8 @@ def load_native():
     except ImportError as e:
         raise ImportError(f"oxydllm_amd/_oxq_torch is missing or does not load ({e}): build it with "
                           "`python -m oxydllm_amd.build`") from e
-    _oxq_torch.bind(lib._handle, OxqError, OxqTensor)
+    import torch
+    _oxq_torch.bind(lib._handle, OxqError, OxqTensor, torch.empty, torch.empty_like)
     return _oxq_torch
 
 

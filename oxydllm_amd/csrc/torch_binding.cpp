@@ -14,9 +14,11 @@
 #include <dlfcn.h>
 
 #include <ATen/ATen.h>
-#include <ATen/hip/EmptyTensor.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Device.h>
+#include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -41,6 +43,8 @@ struct Api {
 Api api;
 PyObject *error_class = nullptr;   // OxqError(status, message)
 PyObject *tensor_struct = nullptr; // the ctypes descriptor class, accepted wherever a tensor is
+PyObject *torch_empty = nullptr;   // torch.empty and torch.empty_like, for the modes that watch Python calls
+PyObject *torch_empty_like = nullptr;
 
 struct Failed {};  // a Python error is set
 
@@ -142,9 +146,39 @@ double real(PyObject *o) {
     return v;
 }
 
+// An owned reference, dropped at the end of the scope.
+struct Ref {
+    PyObject *o;
+    explicit Ref(PyObject *p) : o(p) {
+        if (!o) throw Failed();
+    }
+    Ref(const Ref &) = delete;
+    ~Ref() { Py_DECREF(o); }
+};
+
+at::Tensor unpacked(const Ref &r) { return THPVariable_Unpack(r.o); }
+
+// Outputs are what torch.empty makes: allocated through the dispatcher, so that dispatch modes see them and they are
+// filled under deterministic algorithms (0.25 us more than asking the allocator), and through the Python function itself
+// while a torch function mode is active.
 at::Tensor empty(at::IntArrayRef shape, at::ScalarType dtype, const at::Device &dev) {
-    if (dev.is_cuda()) return at::detail::empty_cuda(shape, dtype, dev, std::nullopt);
+    if (at::impl::torch_function_mode_enabled()) {
+        const Ref size(PyTuple_New((Py_ssize_t)shape.size()));
+        for (size_t i = 0; i < shape.size(); ++i) {
+            PyObject *n = PyLong_FromLongLong(shape[i]);
+            if (!n) throw Failed();
+            PyTuple_SET_ITEM(size.o, (Py_ssize_t)i, n);
+        }
+        const Ref args(PyTuple_Pack(1, size.o)), device(THPDevice_New(dev));
+        const Ref kwargs(Py_BuildValue("{sOsO}", "dtype", (PyObject *)torch::getTHPDtype(dtype), "device", device.o));
+        return unpacked(Ref(PyObject_Call(torch_empty, args.o, kwargs.o)));
+    }
     return at::empty(shape, at::TensorOptions().dtype(dtype).device(dev));
+}
+at::Tensor empty_like(PyObject *x) {
+    const at::Tensor &t = tensor(x);
+    if (at::impl::torch_function_mode_enabled()) return unpacked(Ref(PyObject_CallOneArg(torch_empty_like, x)));
+    return at::empty_like(t);
 }
 
 // The output of a call: the caller's tensor (or descriptor), or a new one.
@@ -203,8 +237,8 @@ at::Tensor empty_rows(const at::Tensor &x, int64_t width) {
 }
 
 // One resident 4096 x 4096 4-bit layer at one row of f16, called back to back without waiting: 12.2 us through
-// Python-built descriptors, 4.6 us here (4.1 with the caller's output tensor; the kernel alone takes 3.6 us, torch's
-// own zero_() 3.8 us a call).  The six outputs and one launch of moe_route_group: 27.8 -> 7.3 us.
+// Python-built descriptors, 4.9 us here (4.1 with the caller's output tensor; the kernel alone takes 3.6 us, torch's
+// own zero_() 3.8 us a call).  The six outputs and one launch of moe_route_group: 27.8 -> 8.5 us.
 PyObject *layer_call(PyObject *self, PyObject *const *args, size_t nargsf, PyObject *kwnames) {
     OXQ_BODY_BEGIN
     Handle *h = (Handle *)self;
@@ -527,7 +561,7 @@ PyObject *activation_mul(PyObject *, PyObject *const *a, Py_ssize_t n) {
     want(n, 5);
     const Handle &h = handle(a[0]);
     const Desc gate(a[1]), up(a[2]);
-    Out out(a[3], [&] { return at::empty_like(tensor(a[1])); });
+    Out out(a[3], [&] { return empty_like(a[1]); });
     const int kind = (int)integer(a[4]);
     void *const s = h.stream();
     call([&] { return api.oxq_activation_mul(ctx_of(h), s, gate, up, kind, out); });
@@ -558,11 +592,11 @@ PyObject *current_device(PyObject *, PyObject *) {
     OXQ_BODY_END
 }
 
-// bind(dlopen handle, error class, descriptor class)
+// bind(dlopen handle, error class, descriptor class, torch.empty, torch.empty_like)
 PyObject *bind(PyObject *, PyObject *args) {
     unsigned long long lib;
-    PyObject *err, *st;
-    if (!PyArg_ParseTuple(args, "KOO", &lib, &err, &st)) return nullptr;
+    PyObject *err, *st, *make, *like;
+    if (!PyArg_ParseTuple(args, "KOOOO", &lib, &err, &st, &make, &like)) return nullptr;
 #define OXQ_RESOLVE(f)                                                                           \
     if (!(api.f = (decltype(&::f))dlsym((void *)(uintptr_t)lib, #f)))                            \
         return PyErr_Format(PyExc_ImportError, "the library does not export %s", #f);
@@ -572,6 +606,10 @@ PyObject *bind(PyObject *, PyObject *args) {
     Py_XSETREF(error_class, err);
     Py_INCREF(st);
     Py_XSETREF(tensor_struct, st);
+    Py_INCREF(make);
+    Py_XSETREF(torch_empty, make);
+    Py_INCREF(like);
+    Py_XSETREF(torch_empty_like, like);
     Py_RETURN_NONE;
 }
 
