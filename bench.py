@@ -177,9 +177,8 @@ def main():
     import torch
     if not torch.cuda.is_available():
         sys.exit("bench.py needs a GPU")
-    from oxydllm_amd import _lib
-    if not os.path.exists(_lib.LIB_PATH):  # load what is built; build only if nothing is
-        from oxydllm_amd import build
+    from oxydllm_amd import build
+    if build.missing():  # load what is built; build only what is not there
         build.build(force=False)
     from oxydllm_amd import ops, synth
 

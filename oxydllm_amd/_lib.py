@@ -202,13 +202,13 @@ def load() -> C.CDLL:
 
 def load_native():
     """The native half of the torch binding (``csrc/torch_binding.cpp``), bound to the library ``load`` opened."""
+    import torch  # its libraries first: the module links against them
     lib = load()
     try:
         from . import _oxq_torch
     except ImportError as e:
         raise ImportError(f"oxydllm_amd/_oxq_torch is missing or does not load ({e}): build it with "
                           "`python -m oxydllm_amd.build`") from e
-    import torch
     _oxq_torch.bind(lib._handle, OxqError, OxqTensor, torch.empty, torch.empty_like)
     return _oxq_torch
 

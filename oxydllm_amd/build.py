@@ -1,5 +1,6 @@
 """Compiles the HIP sources into ``oxydllm_amd/liboxq_hip.so`` for gfx950, and the torch binding's native
-half into ``oxydllm_amd/_oxq_torch.so`` (host code, linked against torch and not against the library).
+half into ``oxydllm_amd/_oxq_torch.<abi>.so`` (host code, linked against torch and not against the library; <abi> is the
+interpreter's tag, so that another one does not load it).
 
 hipcc cross-compiles without a GPU.  Both are built in-tree so they
 travel with the source snapshot; nothing is JIT-compiled at import time.
@@ -30,24 +31,35 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-x", "hip",
 
 
 TORCH_SOURCE = "torch_binding.cpp"
-TORCH_LIB = os.path.join(HERE, "_oxq_torch.so")
+TORCH_LIB = os.path.join(HERE, "_oxq_torch" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
-def _build_torch_binding(force: bool) -> None:
-    src = os.path.join(CSRC, TORCH_SOURCE)
-    newest = max(os.path.getmtime(p) for p in (src, os.path.join(INCLUDE, "oxq.h")))
-    if not force and os.path.exists(TORCH_LIB) and os.path.getmtime(TORCH_LIB) >= newest:
-        return
+def build_torch_binding(out: str = TORCH_LIB, gpu: bool | None = None, opt: str = "-O2") -> None:
+    """``gpu``: whether torch has ROCm support to link against (without it, plan-only contexts work)."""
     import torch
+    gpu = torch.version.hip is not None if gpu is None else gpu
     root = os.path.dirname(torch.__file__)
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    hip = ["-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I/opt/rocm/include"] if gpu else []
+    cmd = ["g++", opt, "-std=c++17", "-fPIC", "-shared", f"-DOXQ_TORCH_HIP={int(gpu)}", *hip,
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
-           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", "-I/opt/rocm/include",
-           f"-I{sysconfig.get_paths()['include']}", src, "-o", TORCH_LIB, f"-L{root}/lib", "-ltorch_python", "-ltorch_hip",
-           "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10", "-ldl"]
+           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
+           os.path.join(CSRC, TORCH_SOURCE), "-o", out, f"-L{root}/lib", "-ltorch_python", *(["-ltorch_hip"] if gpu else []),
+           "-ltorch_cpu", "-ltorch", *(["-lc10_hip"] if gpu else []), "-lc10", "-ldl"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed for {TORCH_SOURCE}:\n{res.stderr}")
+
+
+def _update_torch_binding(force: bool) -> None:
+    newest = max(os.path.getmtime(p) for p in (os.path.join(CSRC, TORCH_SOURCE), os.path.join(INCLUDE, "oxq.h")))
+    if force or not os.path.exists(TORCH_LIB) or os.path.getmtime(TORCH_LIB) < newest:
+        build_torch_binding()
+
+
+def missing() -> list:
+    """The built files that are not there."""
+    from . import _lib
+    return [p for p in (_lib.LIB_PATH, TORCH_LIB) if not os.path.exists(p)]
 
 
 def _deps():
@@ -74,7 +86,7 @@ def _compile(src: str, force: bool) -> str:
 def build(force: bool = False, jobs: int = 6) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        binding = ex.submit(_build_torch_binding, force)
+        binding = ex.submit(_update_torch_binding, force)
         objs = list(ex.map(lambda s: _compile(s, force), SOURCES))
         binding.result()
     newest = max(os.path.getmtime(o) for o in objs)

@@ -8,6 +8,7 @@
 //
 // The module links against torch only.  The library's entry points are looked up in the handle that the ctypes
 // loader opened (`bind`), so both bindings always talk to the same copy of it.
+// OXQ_TORCH_HIP is 0 for a torch without GPU support: there plan-only contexts work, and nothing else could.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -15,8 +16,10 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#if OXQ_TORCH_HIP
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#endif
 #include <torch/csrc/Device.h>
 #include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
@@ -218,6 +221,17 @@ void want(Py_ssize_t got, Py_ssize_t n) {
 // ---------------------------------------------------------------- handles
 enum { KIND_MLP = OXQ_LINEAR_MXFP4 + 1, KIND_PLAIN };  // beyond oxq_linear_kind: a FeedForward; a ctx or an expert set
 
+#if OXQ_TORCH_HIP
+int device() { return c10::hip::current_device(); }
+void *current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+#else
+[[noreturn]] int device() {
+    PyErr_SetString(PyExc_RuntimeError, "this torch has no GPU support: only plan-only contexts work");
+    throw Failed();
+}
+void *current_stream() { device(); }
+#endif
+
 // A C handle: a ctx, an expert set, or a layer, which is called as `layer(x, out)` (a FeedForward: `(x, out, scratch)`).
 struct Handle {
     PyObject_HEAD
@@ -226,7 +240,7 @@ struct Handle {
     int64_t width;  // columns of the output
     int kind;
     bool plan_only;  // validates and plans only: there may be no GPU to ask for a stream
-    void *stream() const { return plan_only ? nullptr : (void *)c10::hip::getCurrentHIPStream().stream(); }
+    void *stream() const { return plan_only ? nullptr : current_stream(); }
 };
 
 // [.., k] -> [.., width]
@@ -588,7 +602,7 @@ PyObject *moe_combine(PyObject *, PyObject *const *a, Py_ssize_t n) {
 // ---------------------------------------------------------------- module
 PyObject *current_device(PyObject *, PyObject *) {
     OXQ_BODY_BEGIN
-    return PyLong_FromLong(c10::hip::current_device());
+    return PyLong_FromLong(device());
     OXQ_BODY_END
 }
 

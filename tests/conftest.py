@@ -15,9 +15,8 @@ def pytest_configure(config):
 def pytest_sessionstart(session):
     """Tests load the libraries that are built; only when there is none do they build
     (hipcc cross-compiles gfx950 without a GPU).  The product itself never builds or falls back."""
-    from oxydllm_amd import _lib
-    if not os.path.exists(_lib.LIB_PATH):
-        from oxydllm_amd import build
+    from oxydllm_amd import build
+    if build.missing():
         build.build(force=False)
 
 
