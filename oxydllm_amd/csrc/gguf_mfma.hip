@@ -1283,9 +1283,7 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     const int nw = (chunks < 16 || chunks >= 64 || mt == 2 || ns == 4 || f32 || !one_round || tune(ctx, OXQ_TUNE_GGR_WAVES, 16) == 8) ? 8 : 16;
     dim3 grid((unsigned)ceil_div(p.N, (int64_t)16 * ns), 1, (unsigned)ceil_div(p.M, (int64_t)tile * mt));
     char name[64];
-    if (f32) snprintf(name, sizeof name, "gguf_%s_res_gemv_f32_mfma_mt%d%s", ggm_name(p.quant), mt, ns == 4 ? "_n64" : "");
-    else if (p.M > 32 && !p.act) snprintf(name, sizeof name, "gguf_%s_mul_mm_bf16_mt%d_res_int%s", ggm_name(p.quant), mt, ns == 4 ? "_n64" : "");
-    else snprintf(name, sizeof name, "gguf_%s_mfma_bf16_mt%d%s%s", ggm_name(p.quant), mt, ns == 4 ? "_n64" : "", p.act ? "_act" : "");
+    snprintf(name, sizeof name, "gguf_%s_mfma_%s_mt%d%s%s", ggm_name(p.quant), f32 ? "f32" : "bf16", mt, ns == 4 ? "_n64" : "", p.act ? "_act" : "");
     set_plan(ctx, name, grid, dim3(nw * 64), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if (!f32 && p.act_dtype != OXQ_BF16) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: activations must be BF16 or F32");
@@ -1424,9 +1422,7 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)4) * 4) : (int)chunks;
     dim3 grid((unsigned)wgs, (unsigned)form.slices);
     char name[64];
-    if (form.slices > 1 && p.M <= 128)  // the rows of the file layout's tile matmul
-        snprintf(name, sizeof name, "gguf_%s_mul_mm_bf16_mt4_res_x%dk4s%d", ggm_name(p.quant), spw, form.slices);
-    else if (form.slices > 1)
+    if (form.slices > 1)
         snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%dk4_s%d", ggm_name(p.quant), rows, spw, form.slices);
     else
         snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%d%s%s", ggm_name(p.quant), rows, spw, ks > 1 ? "k4" : "",

@@ -103,8 +103,8 @@ def test_rows_do_not_depend_on_the_batch(fmt):
 
 @pytest.mark.parametrize("fmt", FMTS)
 def test_switches_and_rows_beyond_the_kernel(fmt):
-    """More than 32 rows go to the tile matmul on the file layout; OXQ_GGUF_MFMA_MAX_M moves that bound;
-    OXQ_GGUF_MFMA = 0 builds the rotated copy of the vector GEMV instead (1 - 4 rows)."""
+    """More than 32 rows of a layer below 2^20 weights go to the tile matmul on the file layout; OXQ_GGUF_MFMA_MAX_M moves
+    that bound; OXQ_GGUF_MFMA = 0 builds the rotated copy of the vector GEMV instead (1 - 4 rows)."""
     from tests.test_gpu_gguf_mxfp4 import _check_mul_mm
     N, K = 96, 512
     data, layer = _layer(fmt, N, K, seed=31 + fmt)

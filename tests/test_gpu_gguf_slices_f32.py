@@ -40,7 +40,7 @@ def test_f32_rows_on_the_matrix_core_copy(fmt, N, K):
         x = np.random.default_rng(K + m).standard_normal((m, K)).astype(np.float32)
         y = layer.forward(to_dev(x))
         kernel = ops.default_context().last_plan()["kernel"]
-        assert ("_res_gemv_f32_mfma" if m >= 3 or N % 16 else "_res_gemv_f32") in kernel, kernel
+        assert ("_mfma_f32" if m >= 3 or N % 16 else "_f32") in kernel, kernel
         ref = x.astype(np.float64) @ w.astype(np.float64).T + bias
         err = np.linalg.norm(y.cpu().numpy() - ref) / np.linalg.norm(ref)
         assert err < 4e-7, f"{synth.GGUF_NAMES[fmt]} m={m}: {err:.2e}"
@@ -62,7 +62,7 @@ def test_f32_rows_are_no_further_from_64_bits_than_the_vector_kernels(fmt, N, K)
         x = to_dev(np.random.default_rng(K + m).standard_normal((m, K)).astype(np.float32))
         ref = x.double() @ w.T
         err, was = [((y.double() - ref).norm() / ref.norm()).item() for y in (layer.forward(x), former.forward(x))]
-        assert "_f32_mfma" in layer.ctx.last_plan()["kernel"] and "mfma" not in plain.last_plan()["kernel"]
+        assert "_mfma_f32" in layer.ctx.last_plan()["kernel"] and "mfma" not in plain.last_plan()["kernel"]
         assert err <= 1.04 * was, f"{synth.GGUF_NAMES[fmt]} m={m}: {err:.3e}, vector kernel {was:.3e}"
 
 
@@ -83,9 +83,9 @@ def test_f32_layer_with_one_copy():
     for m in (1, 2, 8):
         say(f"gguf f32 one copy m={m}")
         y = layers[0].forward(x[:m])
-        assert "_f32_mfma" in ctx.last_plan()["kernel"]
+        assert "_mfma_f32" in ctx.last_plan()["kernel"]
         want = layers[1].forward(x[:m])
-        assert ("_f32_mfma" in ctx.last_plan()["kernel"]) == (m > 2)
+        assert ("_mfma_f32" in ctx.last_plan()["kernel"]) == (m > 2)
         assert ((y - want).norm() / want.norm()).item() < 8e-7  # two forms, each within 4e-7 of the 64-bit product
 
 
@@ -102,7 +102,7 @@ def test_small_f32_rows_keep_their_bits(fmt):
             x[1] *= 1e6
         ref = x.double() @ w.T
         y = layer.forward(x)
-        assert "_f32_mfma" in layer.ctx.last_plan()["kernel"]
+        assert "_mfma_f32" in layer.ctx.last_plan()["kernel"]
         for r in range(m):
             err = ((y[r].double() - ref[r]).norm() / ref[r].norm()).item()
             assert err < 4e-7, f"{synth.GGUF_NAMES[fmt]} m={m} row {r}: {err:.2e}"
@@ -123,7 +123,7 @@ def test_infinite_and_nan_rows_of_f32(fmt):
         x.view(torch.int32)[2, 5] = 0x7F800001
         say(f"gguf f32 infinities {synth.GGUF_NAMES[fmt]} m={m}")
         got, want = layer.forward(x), former.forward(x)
-        assert "_f32_mfma" in layer.ctx.last_plan()["kernel"]
+        assert "_mfma_f32" in layer.ctx.last_plan()["kernel"]
         assert torch.equal(torch.nan_to_num(got[:3], 0.0, 1.0, -1.0), torch.nan_to_num(want[:3], 0.0, 1.0, -1.0))
         assert bool(got[2].isnan().all()) and bool(got[3:].isfinite().all())
         if fmt in (synth.GGUF_Q4_1, synth.GGUF_Q5_1):
@@ -145,9 +145,9 @@ def test_prefill_rows_of_few_columns(fmt, N, K):
         y = layer.forward(to_dev(x, torch.bfloat16))
         plan = ops.default_context().last_plan()
         say(f"gguf slices {synth.GGUF_NAMES[fmt]} N={N} K={K} m={m} {plan['kernel']} x {plan['split_k']}")
-        whole = "_res_int" in plan["kernel"]  # row tiles of the integer kernel: the weights unrounded
+        whole = "_mfma_bf16_mt2" in plan["kernel"]  # row tiles of the integer kernel: the weights unrounded
         assert plan["launches"] == (2 if plan["split_k"] > 1 else 1) and (slices is None or plan["split_k"] > 1), plan
-        assert whole or "_res_x2k4" in plan["kernel"] or "_gemm_" in plan["kernel"], plan
+        assert whole or "_gemm_bf16_r64x" in plan["kernel"], plan
         ref = oracle.matmul_nt_f32(round_x(x, oracle.BF16), w if whole else wr, round_x(bias, oracle.BF16))
         assert_close(y, ref, f"{synth.GGUF_NAMES[fmt]} m={m}", bf16_out=True)
     for m in (1, 17, 32):  # the integer kernel on a ragged last strip

@@ -47,11 +47,11 @@ def test_wide_layers_at_33_to_64_rows(K, bits, dtn):
         print(f"[case] mid {bits}-bit {dtn} K={K} m={m}", flush=True)
         y = layer.forward(xd[:m])
         plan = ops.default_context().last_plan()
-        assert plan["kernel"] == f"pk{bits}_mid_{dtn}_r64x2k4" and plan["launches"] == 1 and plan["grid"][0] == 129, plan
+        assert plan["kernel"] == f"pk{bits}_gemm_{dtn}_r64x2k4" and plan["launches"] == 1 and plan["grid"][0] == 129, plan
         assert_close(y, tile[:m], f"mid m{m}")
         np.testing.assert_array_equal(bits_of(y), first[:m])  # a row's bits do not depend on m
     layer.forward(xd[:32 if dtn == "bf16" else 48])  # f16 weights stay unrounded up to 48 rows
-    assert "_mid_" not in ops.default_context().last_plan()["kernel"]
+    assert "_gemm_" not in ops.default_context().last_plan()["kernel"]
 
 
 @pytest.mark.parametrize("kind", ["awq", "gptq"])
