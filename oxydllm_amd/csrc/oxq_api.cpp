@@ -1991,7 +1991,10 @@ static int prepack_layer(oxq_packed_quant_linear *l) {
     if (check_wna16(ctx, "PackedQuantLinear", KIND_DEQUANT, nullptr, &l->qweight, &l->qzeros, &l->scales,
                     l->bits, l->pack_dim, &shape_only, &src) != OXQ_OK)
         return OXQ_OK;
-    if (!pk4_eligible(src) || (l->act && src.N % 64 != 0) || (l->has_bias && ((uintptr_t)l->bias.data & 7))) return OXQ_OK;  // a strip pairs 32 gate with 32 up columns
+    if (!pk4_eligible(src) || (l->act && src.N % 64 != 0)) return OXQ_OK;  // a strip pairs 32 gate with 32 up columns
+    // The prefill kernels read four columns' bias at once.  A plain layer has the checkpoint layout's kernels instead; a fused
+    // gate|up layer only the copy: its rows then all run on the tiles whose epilogue reads column by column.
+    if (!l->act && l->has_bias && ((uintptr_t)l->bias.data & 7)) return OXQ_OK;
     l->pk.K = src.K;
     l->pk.N = src.N;
     l->pk.group_shift = src.group_shift;

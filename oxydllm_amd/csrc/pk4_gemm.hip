@@ -226,6 +226,7 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int64_t min_m = tune(ctx, OXQ_TUNE_PK4_GEMM_MIN_M, pk4_sets(p.w.group_shift) > 1 ? 49 : pk4_mid_decode(cus, p) ? 33 : 65);
     if (min_m <= 0 || (p.w.bits != 4 && p.w.bits != 8) || (p.act && p.w.strip == 16) || p.M < min_m) return {0, 1};
+    if ((uintptr_t)p.bias & 7) return {0, 1};  // (fused gate|up layers only: oxq_api.cpp, prepack_layer)
     if (p.w.bits == 8 && p.w.strip == 16) return {0, 1};  // (16-column strips are a 4-bit layout)
     const int forced = tune(ctx, OXQ_TUNE_PK4_GEMM_ROWS, 0), forced_ks = tune(ctx, OXQ_TUNE_PK4_GEMM_KS, 0);
     if (p.w.unrounded) return {forced || pk4_fold_prefill(cus, p) ? 64 : 0, 1};

@@ -618,3 +618,24 @@ def test_fused_gate_up_benchmark_shape_and_refusals():
     with pytest.raises(ops.OxqError) as e:
         ops.PackedQuantLinear(*args, gate_up_act=ops.ACT_GPT_OSS_SWIGLU)
     assert e.value.status == -1
+
+
+@pytest.mark.parametrize("m", [1, 33, 64, 100])
+def test_fused_gate_up_with_a_bias_at_an_odd_address(m):
+    K, N, dt, tdt = 512, 1024, oracle.BF16, torch.bfloat16
+    qw, qz, sc = synth.awq_checkpoint(K, N, 128, 4, seed=6)
+    bias = (np.arange(N, dtype=np.float32) % 9 - 4) * np.float32(0.25)
+    odd = torch.empty(N + 1, dtype=tdt, device="cuda")
+    odd[1:] = to_dev(bias, tdt)
+    args = (4, ops.PACK_OUT, to_dev(qw), to_dev(qz), to_dev(sc, tdt))
+    fused = ops.PackedQuantLinear(*args, odd[1:], tdt, gate_up_act=ops.ACT_GATED_SILU)
+    say(f"fused, bias at an odd element, m={m}")
+    x = np.random.default_rng(m).standard_normal((m, K)).astype(np.float32) * np.float32(0.25)
+    y = fused.forward(to_dev(x, tdt))
+    w = oracle.dequantize_awq(qw, qz, oracle.round_through(sc, dt))
+    gu = oracle.round_through(oracle.matmul_nt_f32(round_x(x, dt), oracle.round_through(w, dt) if m > 16 else w, bias), dt)
+    g, u = gu[:, :N // 2].astype(np.float64), gu[:, N // 2:].astype(np.float64)
+    # a factor may round to the neighbouring bf16 value (2^-8 of it), as may the product: three roundings
+    ref = g / (1 + np.exp(-g)) * u
+    err = np.abs(as_f32(y) - ref)
+    assert np.all(err <= 1e-2 + 3 * 2.0 ** -8 * (np.abs(ref) + np.abs(u))), err.max()

@@ -23,6 +23,24 @@ def kernels(pack, bits, K, N, g, dt, rows):
     return out
 
 
+def test_fused_layer_with_a_bias_at_any_address():
+    """A bias that is no multiple of eight bytes: the fused layer is built as before, and every row count runs on the tiles
+    that read it column by column."""
+    lib, plan = _lib.load(), ops.Context(plan_only=True)
+    K, N, dt = 4096, 28672, _lib.BF16
+    bias = fake((N,), dt)
+    bias.data = 0x1002
+    h = C.c_void_p()
+    rc = lib.oxq_packed_quant_linear_new_gate_up(plan.handle, 4, ops.PACK_OUT, C.byref(fake((K, N // 8), _lib.I32)),
+                                                 C.byref(fake((K // 128, N // 8), _lib.I32)), C.byref(fake((K // 128, N), dt)),
+                                                 C.byref(bias), ops.ACT_GATED_SILU, dt, C.byref(h))
+    assert rc == 0, lib.oxq_last_error().decode()
+    for m in (1, 33, 64, 65, 1000):
+        assert lib.oxq_packed_quant_linear_forward(h, None, C.byref(fake((m, K), dt)), C.byref(fake((m, N // 2), dt))) == 0
+        assert plan.last_plan()["kernel"].startswith("pk4_mfma_") and plan.last_plan()["launches"] == 1
+    lib.oxq_packed_quant_linear_free(h)
+
+
 def test_no_three_tiles_of_folded_sums_beside_two_sets_of_pairs():
     """f16, groups of 64, 33 - 48 rows: that form spills; the rows run as two tiles of 32, still folded."""
     rows = (33, 40, 48)
