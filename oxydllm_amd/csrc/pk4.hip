@@ -283,11 +283,8 @@ __global__ __launch_bounds__(NW * 64) void pk4_front_kernel(const uint16_t *__re
                 tmps = Ops::mfma(a, ones, fresh ? zero4 : tmps);
             }
             // the pairs of the four columns: the four lane groups fetched one word each
-            const auto p16 = __builtin_amdgcn_permlane16_swap(zv[b % WIN], zv[b % WIN], false, false);
-            const uint32_t even = p16[0], odd = p16[1];
-            const auto pe = __builtin_amdgcn_permlane32_swap(even, even, false, false);
-            const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);
-            const uint32_t zq[4] = {pe[0], po[0], pe[1], po[1]};
+            uint32_t zq[4];
+            pk4_pair_words(zv[b % WIN], zq);
 #pragma unroll
             for (int f = 0; f < 4; ++f) {
                 const float sf = TT::to_f32((uint16_t)(zq[f] >> 16));

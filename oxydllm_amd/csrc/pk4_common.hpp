@@ -109,6 +109,17 @@ template <int H> __device__ __forceinline__ void pk4g_columns(const uint32_t (&w
     }
 }
 
+// The zero/scale pairs of a lane's four columns in the 64-column layout: lane group f has fetched word f of the quad, and the
+// lane-swap instructions exchange 16-lane rows between two registers (odd rows of one with even rows of the other, then
+// the upper half of one with the lower half of the other).
+__device__ __forceinline__ void pk4_pair_words(uint32_t z, uint32_t (&zv)[4]) {
+    const auto p16 = __builtin_amdgcn_permlane16_swap(z, z, false, false);  // {r0 r0 r2 r2}, {r1 r1 r3 r3}
+    const uint32_t even = p16[0], odd = p16[1];
+    const auto pe = __builtin_amdgcn_permlane32_swap(even, even, false, false);  // {r0 x4}, {r2 x4}
+    const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);    // {r1 x4}, {r3 x4}
+    zv[0] = pe[0], zv[2] = pe[1], zv[1] = po[0], zv[3] = po[1];
+}
+
 constexpr int PK4N_BW = 272;  // 16-column strips: words of one block, 256 of weights and 16 of pairs
 
 // The constants of one column and block from its pair word {-z, s}; deq() = T((q - z) * s) of a row pair.

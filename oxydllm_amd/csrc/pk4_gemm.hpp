@@ -111,13 +111,6 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         const __amdgpu_buffer_rsrc_t rs = i < NB ? rs_w : rs_none;
         zring[set] = __builtin_amdgcn_raw_buffer_load_b32(rs, voff_z, i * BB + set * 256, 0);
     };
-    auto zs_words = [&](uint32_t z, uint32_t (&zv)[4]) {
-        const auto p16 = __builtin_amdgcn_permlane16_swap(z, z, false, false);
-        const uint32_t even = p16[0], odd = p16[1];
-        const auto pe = __builtin_amdgcn_permlane32_swap(even, even, false, false);
-        const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);
-        zv[0] = pe[0], zv[2] = pe[1], zv[1] = po[0], zv[3] = po[1];
-    };
 
     dma_x(0);
     __builtin_amdgcn_sched_barrier(0);  // requests keep this order: the wait counts rely on it
@@ -142,7 +135,7 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         uint32_t zv[4], negzb[4], sp[4];
         Pk4gBf16 cb[4];
         auto constants = [&](int set) {  // of a set of pairs; then the next block's are requested
-        zs_words(zring[set], zv);
+        pk4_pair_words(zring[set], zv);
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
             if constexpr (BF) {  // the pair word holds {-(bias + z), s}, bias = 128 for nibbles and 0 for bytes
@@ -155,7 +148,7 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         };
         float4_t tmp[FOLD ? MT : 1][4], tmps[FOLD ? MT : 1];  // a group's sums of the folded form
         auto fold = [&](int set) {
-            zs_words(zring[set], zv);
+            pk4_pair_words(zring[set], zv);
             load_z(i + 1, set);
 #pragma unroll
             for (int f = 0; f < 4; ++f) {

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
     const int voff_w = lane * 16;
     // The block's zero/scale pairs: lane (ni, kb) fetches word kb of column quad ni (one 4-byte load a lane,
     // 256 contiguous bytes a wave: a quarter of what a 16-byte load costs the address unit, which is the
-    // busiest unit from 32 rows on) and the four lane groups then exchange their words (zs_words).
+    // busiest unit from 32 rows on) and the four lane groups then exchange their words (pk4_pair_words).
     const int voff_z = 1024 * WL * 4 + (ni * 4 + kb) * 4;
     // activation load q of a block: row 4q + lane/16, 16-byte chunk lane%16 of the row's 256 bytes; rows
     // past M get an offset beyond any buffer, for which the buffer unit returns zeros without touching
@@ -182,16 +182,6 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
         const __amdgpu_buffer_rsrc_t rs = i < nloc ? rs_w : rs_none;
         zring[set] = __builtin_amdgcn_raw_buffer_load_b32(rs, voff_z, blk_of(i) * BB + set * 256, WNT);
     };
-    // zv[f] = the word that lane group f fetched, in every lane group: the lane-swap instructions
-    // exchange 16-lane rows between two registers (odd rows of one with even rows of the other, then
-    // the upper half of one with the lower half of the other).
-    auto zs_words = [&](uint32_t z, uint32_t (&zv)[4]) {
-        const auto p16 = __builtin_amdgcn_permlane16_swap(z, z, false, false);  // {r0 r0 r2 r2}, {r1 r1 r3 r3}
-        const uint32_t even = p16[0], odd = p16[1];
-        const auto pe = __builtin_amdgcn_permlane32_swap(even, even, false, false);  // {r0 x4}, {r2 x4}
-        const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);    // {r1 x4}, {r3 x4}
-        zv[0] = pe[0], zv[2] = pe[1], zv[1] = po[0], zv[3] = po[1];
-    };
     auto store_a = [&](const u32x4_t (&a)[AQ]) {
 #pragma unroll
         for (int q = 0; q < AQ; ++q) *(u32x4_t *)(slot + q * 1024 + a_wr[q & 3]) = a[q];
@@ -255,7 +245,7 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
         // the tile form's constants of a set, and the request for the next block's
         auto constants = [&](int set) {
             uint32_t zv[4];
-            zs_words(zring[set], zv);
+            pk4_pair_words(zring[set], zv);
 #pragma unroll
             for (int f = 0; f < 4; ++f) {
                 if constexpr (WIDEN) cb[f].set(__builtin_bit_cast(float, zv[f] & 0xFFFF0000u), __builtin_bit_cast(float, zv[f] << 16) + 128.0f);
@@ -266,7 +256,7 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
         // the folded form: y += s * (sum - (bias + z) * rowsum), all f32
         auto fold = [&](int set) {
             uint32_t zv[4];
-            zs_words(zring[set], zv);
+            pk4_pair_words(zring[set], zv);
             load_z(i + 1, set);
 #pragma unroll
             for (int f = 0; f < 4; ++f) {

@@ -212,12 +212,9 @@ __global__ __launch_bounds__(512) void pk4_mid_kernel(const uint16_t *__restrict
             if constexpr (!NARROW) {
                 if (n == 0) {
                     if (st % SPS == 0) {
-                        const uint32_t z = zring[PAR][st / SPS];
-                        const auto p16 = __builtin_amdgcn_permlane16_swap(z, z, false, false);
-                        const uint32_t even = p16[0], odd = p16[1];
-                        const auto pe = __builtin_amdgcn_permlane32_swap(even, even, false, false);
-                        const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);
-                        constant(0, pe[0]), constant(2, pe[1]), constant(1, po[0]), constant(3, po[1]);
+                        uint32_t zv[4];
+                        pk4_pair_words(zring[PAR][st / SPS], zv);
+                        constant(0, zv[0]), constant(2, zv[2]), constant(1, zv[1]), constant(3, zv[3]);
                         load_z(i2, PAR, st / SPS);
                     }
 #pragma unroll

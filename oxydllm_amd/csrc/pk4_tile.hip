@@ -140,11 +140,8 @@ __global__ __launch_bounds__(512) void pk4_tile64_kernel(const uint16_t *__restr
         }
     };
     auto pairs = [&](int b) {
-        const auto p16 = __builtin_amdgcn_permlane16_swap(zv[b], zv[b], false, false);
-        const uint32_t even = p16[0], odd = p16[1];
-        const auto pe = __builtin_amdgcn_permlane32_swap(even, even, false, false);
-        const auto po = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);
-        const uint32_t zq[4] = {pe[0], po[0], pe[1], po[1]};
+        uint32_t zq[4];
+        pk4_pair_words(zv[b], zq);
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
             if constexpr (BF) cb[f].set(__builtin_bit_cast(float, zq[f] & 0xFFFF0000u), __builtin_bit_cast(float, zq[f] << 16) + 128.0f);
