@@ -3,14 +3,14 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--all]
 
-Workload (BASELINE.json configs[1]): AWQ W4A16, K=4096, N=14336, g=128, f16
+Workload: AWQ W4A16, K=4096, N=14336, g=128, f16
 activations/scales, at M = 1 (GEMV), 16 and 64 (MFMA tile GEMM).  A "step" is
 one call of the hot path at M=1 on synthetic inputs already resident in HBM;
 consecutive steps rotate over enough weight copies (> 256 MB) that no step finds
 its weights in L2 or the memory-side cache.  The K timed steps are replayed from
 one HIP graph so that host launch overhead is not what is measured.
 
-Prints ONE JSON line: `value` is the M=1 throughput in GB/s of algorithmic
+Prints ONE JSON line of at most 4 KB: `value` is the M=1 throughput in GB/s of algorithmic
 bytes (packed weights + zeros + scales + x + y per call); the M=16 / M=64
 results, in GB/s and TFLOP/s, ride along in `cases`.  `roofline` describes the
 dominant kernel (the M=1 GEMV, HBM-bound); `cpu_baseline` times the CPU oracle's
@@ -19,8 +19,9 @@ x.W^T per call, linear.rs:40-79, 597-600) on this machine's cores.
 `roofline.bare_read_us` / `bare_read_nt_us` / `bare_read_best_us` are plain reads of the same
 packed weights with no arithmetic (in passes, plain / nontemporal; everything requested first),
 `roofline.empty_launch_us` an empty kernel of the same launch shape.
-`other_configs` holds one compact row per case of BASELINE configs 0, 2, 3 and 4,
-each with its own roofline fraction and a CPU baseline per configuration.
+Everything measured - the down projection, the stateless ops, and `other_configs`, one row per case of
+the square AWQ layer, the GPTQ, GGUF and MXFP4 layers, each with its own roofline fraction and a CPU
+baseline per configuration - goes to stderr as `[bench] details: {...}`.
 """
 from __future__ import annotations
 
@@ -180,7 +181,7 @@ def main():
                     help="skip the same-weights-every-call (cache-resident) timings, so that a profiler "
                          "run sees only the launches `value` is computed from plus the warm-up")
     ap.add_argument("--no-others", action="store_true",
-                    help="skip the compact rows for BASELINE configs 0, 2, 3 and 4 (`other_configs`)")
+                    help="skip the rows of the other layers (`other_configs`: square AWQ, GPTQ, GGUF, MXFP4)")
     ap.add_argument("--no-bare-read", action="store_true",
                     help="skip the plain-read calibration (`roofline.bare_read_us`)")
     ap.add_argument("--all", action="store_true",
@@ -303,7 +304,7 @@ def main():
         ctx.set_weight_cache(0)
         ctx.forget_weights(None)
 
-    # The same weight shape the other way round (the MLP's down projection
+    # The same weight shape the other way round (the MLP's down projection of the workload
     # names both orientations): 64 column strips, so K is also cut into slices.
     down_cases = []
     if not args.skip_ops:

@@ -181,6 +181,11 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 //     (w = workgroups / CUs); those of the 16-column layout (144..145 registers) run in whole rounds;
 //   - the split-K tiles cost `split_lo` (below one round) or `split_hi` times w at any M: small workgroups, no
 //     ragged round, but the rate they have at 64 rows.
+// The bf16 conversion and the two-strip form are newer than these fits, and groups of 32 and 64 rows are in none.  With every
+// form forced at 14 row counts from 65 to 4096 (4- and 8-bit layers of 3584 x 18944, 4096 x 6144, 4096 x 11008, 4096 x 14336,
+// 5120 x 6144) the choice is within 8 % of the fastest, except where a launch holds one to one and a half rounds: 8-bit
+// 4096 x 6144 at 150 rows split-K 32 us, two strips 23; groups of 64, 4096 x 11008 at 150 rows 46 and 40; groups of 32,
+// 5120 x 6144 at 150 / 777 / 900 / 1200 rows f16 33 / 96 / 96 / 143 as chosen, 26 / 81 / 84 / 108 with two strips.
 // OXQ_PK4_GEMM_ROWS = 64 | 128 takes the choice (tests, sweeps); OXQ_PK4_GEMM_MIN_M = 0 switches the kernels off.
 // a round of the two-strip form (one workgroup a CU) against a full round of 64-row workgroups of eight strips:
 // 19 - 24 us against 65 - 78 at K = 4096 over both widths and types

@@ -13,8 +13,9 @@
 // stands between the MFMAs of the column before, and loads and LDS reads are dealt over the columns - all eight waves
 // issuing theirs right behind a barrier kept the address and LDS units busy for a third of the half block while the
 // matrix cores waited.  Against one block of x a round behind one barrier, everything read where it is used (us, 64-row
-// tiles): 14336 x 4096 at 384 rows f16 63.7 -> 60.0, bf16 72.9 -> 68.6 (66 with pk4g_widen); 4096 x 14336 at 128 rows 23.9 ->
-// 22.3, 26.2 -> 24.4 (23.6).  Deeper requests alone (two blocks of weights, three stages of x) changed nothing, nor did
+// tiles, bf16 with pk4g_widen, called back to back; graph replays are 1 - 2 us shorter): 14336 x 4096 at 384 rows f16 60.6 ->
+// 59.6, bf16 71.4 -> 65.0; 4096 x 14336 at 128 rows 22.4 -> 21.6, 24.1 -> 22.4; 8-bit f16 4096 x 14336 at 128 / 256 rows 26.3 /
+// 45.6 -> 27.0 / 47.0.  Deeper requests alone (two blocks of weights, three stages of x) changed nothing, nor did
 // K slices over workgroups on narrow layers (8192 x 8192 at 128 rows 28.6 -> 30.8, 14336 x 4096 at 64 rows 20.1 -> 23.4).
 #pragma once
 

@@ -7,7 +7,7 @@ from oxydllm_amd import _lib
 
 TORCH_DT = {oracle.F16: torch.float16, oracle.BF16: torch.bfloat16, oracle.F32: torch.float32}
 
-# 2e-3 relative / 1e-2 absolute of the f32-accumulated reference
+# tolerance of the parity tests: 2e-3 relative / 1e-2 absolute of the f32-accumulated reference
 RTOL, ATOL = 2e-3, 1e-2
 
 
