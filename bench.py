@@ -304,8 +304,8 @@ def main():
         ctx.set_weight_cache(0)
         ctx.forget_weights(None)
 
-    # The same weight shape the other way round (the MLP's down projection of the workload
-    # names both orientations): 64 column strips, so K is also cut into slices.
+    # The same weight shape the other way round (the MLP's down projection):
+    # 64 column strips, so K is also cut into slices.
     down_cases = []
     if not args.skip_ops:
         kd, nd = N, K

@@ -144,3 +144,17 @@ def test_stateless_op_on_fine_groups(kind, bits, K, N, g):
         y = ops.mpp_quant_matmul(to_dev(x, tdt), *args, bits, ops.PACK_IN if kind == "gptq" else ops.PACK_OUT)
         wr = oracle.round_through(w, dt) if rounds(kind, bits, m, dt) else w
         assert_close(y, oracle.matmul_nt_f32(round_x(x, dt), wr), f"{kind}{bits} m{m}")
+
+
+def test_rows_beyond_32_bit_offsets():
+    """x of more than 2 GiB on an unrounded layer: only the prefill form addresses it, whatever the cost rule says."""
+    K, N, g, tdt = 4096, 136, 64, torch.float16
+    m = (1 << 31) // (2 * K) + 65
+    layer, _, w = build("gptq", 4, K, N, g, oracle.F16, tdt, 5)
+    say(f"unrounded, {m} rows")
+    x = torch.randn((1024, K), device="cuda").to(tdt).repeat((m + 1023) // 1024, 1)[:m]
+    y = layer.forward(x)
+    assert "_gemm_f16_r64x8_gs" in ops.default_context().last_plan()["kernel"]
+    assert torch.equal(y[1024:2048], y[:1024]) and torch.equal(y[m - 65:], y[(m - 65) % 1024:][:65])
+    ref = x[:64].cpu().numpy().astype(np.float64) @ w.astype(np.float64).T
+    assert (y[:64].cpu() == torch.from_numpy(ref).to(tdt)).double().mean().item() > 0.9
