@@ -1264,10 +1264,24 @@ bool gguf_mfma_takes(const oxq_ctx *ctx, int64_t M, int64_t, int act_dtype) {
 // p.w is the matrix-core copy; p.act: 0, or 1 + the gated activation of a fused gate|up layer, whose y is [M, N / 2].
 // More rows than gguf_mfma_takes allows run as row tiles of the grid (every tile reads the weights again: the
 // callers send such calls elsewhere where they can).
-
 int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     const bool f32 = p.act_dtype == OXQ_F32;
     const int tile = f32 ? 4 : 16;  // rows of x a matrix-core tile takes
+    if (p.M > 65535 * 2 * tile) {  // more row tiles than a grid dimension has: that many at a time
+        const int64_t most = 65535 * 2 * tile, elem = f32 ? 4 : 2;
+        uint32_t launches = 0;
+        for (int64_t m0 = 0; m0 < p.M; m0 += most) {
+            GgufProblem q = p;
+            q.M = std::min(most, p.M - m0);
+            q.x = (const uint8_t *)p.x + m0 * p.K * elem;
+            q.y = (uint8_t *)p.y + m0 * (p.act ? p.N / 2 : p.N) * elem;
+            const int rc = launch_gguf_mfma(ctx, s, q);
+            if (rc != OXQ_OK) return rc;
+            ++launches;
+        }
+        ctx->plan.launches = launches;
+        return OXQ_OK;
+    }
     const int ns = ggm_strips(ctx, p.N);
     const int mt = p.M > tile ? 2 : 1;
     const int rows = (int)std::min<int64_t>(p.M, tile * mt);
@@ -1290,7 +1304,6 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     if (f32 && p.act) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: a fused activation needs BF16");
     if ((uintptr_t)p.x & 15) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: x must be 16-byte aligned");
     if ((uint64_t)16 * mt * (uint64_t)p.K * 2 >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: K too large");
-    if (grid.z > 65535) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: m = %lld exceeds the grid", (long long)p.M);
     if (gguf_res_bytes(p.quant, p.K, 16) * (uint64_t)ns >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: K too large");
     const int cslice = (int)(p.K / 128);
 #define OXQ_GGM(F) \

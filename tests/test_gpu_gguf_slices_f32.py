@@ -66,6 +66,22 @@ def test_f32_rows_are_no_further_from_64_bits_than_the_vector_kernels(fmt, N, K)
         assert err <= 1.04 * was, f"{synth.GGUF_NAMES[fmt]} m={m}: {err:.3e}, vector kernel {was:.3e}"
 
 
+def test_f32_rows_beyond_one_grid():
+    """More rows than 65535 row tiles of eight: two launches."""
+    fmt, N, K, m = synth.GGUF_Q4_0, 1040, 1024, 65535 * 8 + 9
+    layer = ops.QLinear(fmt, to_dev(synth.gguf_weight(fmt, N, K, seed=3)), K, N, None, torch.float32)
+    say(f"gguf f32 {m} rows")
+    x = torch.randn((4096, K), device="cuda").repeat((m + 4095) // 4096, 1)[:m]
+    y = layer.forward(x)
+    plan = layer.ctx.last_plan()
+    assert "_mfma_f32" in plan["kernel"] and plan["launches"] == 2
+    assert torch.equal(y[65536:131072], y[:65536])  # 65536 = 16 x 4096 rows on, the same rows of x in tiles of their own
+    tail = torch.arange(m - 9 - 16, m, device="cuda")
+    assert torch.equal(y[tail], y[tail % 4096])
+    ref = x[:64].double() @ layer.dequantize().double().T
+    assert ((y[:64].double() - ref).norm() / ref.norm()).item() < 4e-7
+
+
 def test_f32_layer_with_one_copy():
     """OXQ_GGUF_MFMA = 2: the matrix-core copy alone, at every row count, and the memory of one copy less."""
     fmt, N, K = synth.GGUF_Q8_0, 4096, 4096
