@@ -921,11 +921,36 @@ static int pk4_row_tiles(const oxq_ctx *ctx, const Pk4Problem &p) {
     return all == 3 && spills && pk4_folds(ctx, p, 3) ? 2 : all;
 }
 
+static const char *pk4_by_name(int mt, int rows_mt) {  // in a plan's name: row tiles a workgroup takes, if not all
+    return mt == rows_mt ? "" : mt == 1 ? "_by1" : mt == 2 ? "_by2" : "_by3";
+}
+
+// Row tiles a workgroup takes of the `mt` that the rows come to, where the workgroups of `mt` would leave compute units idle: as
+// few as still fit one round.  A wave's chain of blocks gets shorter (fewer MFMAs, fewer rows of x) and nothing is paid for
+// it but the weights' second way out of L2.  Same form and same K split within a workgroup: the results do not change, unless
+// K slices are given up.  `ks` slices stay, or (0 returned in it) are given up where they fill the chip by themselves and K is
+// short enough that a workgroup does the whole of it in less than the slices' second launch takes; bf16 rows that convert
+// the weights for one or two row tiles lose by it.  Nor do 8-bit layers gain from two tiles of eight (2816 x 2944 f16 at 128 rows
+// 12.2 -> 12.7).
+// us, a workgroup with all the rows / as chosen here (4-bit, unless said): 2304 x 3328 bf16 at 20 / 48 / 64 / 128 rows 7.5 / 9.4 /
+// 10.7 / 10.8 -> 6.8 / 6.9 / 6.9 / 8.1; 3840 x 3840 f16 at 20 / 64 rows 10.1 / 13.6 -> 7.9 / 8.7, bf16 at 128 rows 15.4 -> 11.8;
+// 1792 x 2112 f16, groups of 64, at 65 / 200 rows 11.1 / 11.5 -> 6.2 / 8.5; 8-bit 2816 x 2944 f16 at 64 rows 11.9 -> 10.0.
+// Slices given up: 4096 x 4096 f16 at 20 / 64 rows 7.4 / 11.4 -> 7.2 / 8.4, bf16 at 64 rows 11.9 -> 9.6 (at 20 rows 7.9 -> 9.5),
+// 4096 x 6144 f16 at 32 / 64 rows 9.9 / 13.7 -> 7.7 / 10.4; but 5632 x 2304 bf16 at 32 / 64 rows 8.2 / 11.3 -> 9.0 / 11.9.
+static int pk4_spread(const oxq_ctx *ctx, const Pk4Problem &p, int64_t strips, int mt, int *ks) {
+    if (p.M <= 16) return mt;
+    const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    auto fits = [&](int n, int slices) { return strips * ceil_div(p.M, (int64_t)16 * n) * slices <= cus; };
+    if (*ks > 1 && !fits(1, *ks) && p.w.K <= 4096 && (p.w.dtype == OXQ_F16 || p.M > 32) && fits(mt, 1)) *ks = 0;
+    int n = mt;
+    while (n > 1 && fits(n - 1, std::max(*ks, 1))) --n;
+    return p.w.bits == 8 && p.M > 64 && n > 1 ? mt : n;
+}
+
 template <typename TT, int BITS>
-static int pk4_by_mt(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p, int bslice, int mt, int front) {
-    const bool fold = pk4_folds(ctx, p, mt);
+static int pk4_by_mt(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &p, int bslice, int mt, bool fold, int front) {
     switch (mt) {
-    case 1: return pk4_go<TT, BITS, 1, true>(ctx, s, grid, p, bslice, front);
+    case 1: return fold ? pk4_go<TT, BITS, 1, true>(ctx, s, grid, p, bslice, front) : pk4_go4<TT, BITS, 1, false, 4>(ctx, s, grid, p, bslice, 0);
     case 2: return fold ? pk4_go<TT, BITS, 2, true>(ctx, s, grid, p, bslice, 0) : pk4_go<TT, BITS, 2, false>(ctx, s, grid, p, bslice, 0);
     case 3: return fold ? pk4_go<TT, BITS, 3, true>(ctx, s, grid, p, bslice, 0) : pk4_go<TT, BITS, 3, false>(ctx, s, grid, p, bslice, 0);
     default: return pk4_go<TT, BITS, 4, false>(ctx, s, grid, p, bslice, 0);
@@ -1021,6 +1046,7 @@ static int pk4n_by_shape(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Proble
     }
     switch (mt) {
     case 1: {
+        if (!fold) return pk4n_go4<TT, 1, false, 4, 4>(ctx, s, grid, p, bslice);
         const int xq = tune(ctx, OXQ_TUNE_PK4_XQ, 1) ? (int)ceil_div(p.M, 4) : 4;
         if (xq == 1) return pk4n_go4<TT, 1, true, 4, 1>(ctx, s, grid, p, bslice);
         if (xq == 2) return pk4n_go4<TT, 1, true, 4, 2>(ctx, s, grid, p, bslice);
@@ -1035,7 +1061,7 @@ static int pk4n_by_shape(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Proble
 // forward on a layer stored in 16-column strips
 static int launch_pk4n_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const int64_t M = p.M, N = p.w.N;
-    const int mt = M > 48 ? 4 : (int)ceil_div(M, 16);
+    const int rows_mt = M > 48 ? 4 : (int)ceil_div(M, 16);  // row tiles that the rows come to, up to four: they settle the form
     const int NB = (int)(p.w.K / 128);
     // One workgroup per strip when that gives the chip enough workgroups and x is small: every strip
     // re-reads x (four rows against a strip's 16 columns are what 16 rows are against 64).  Measured, f16,
@@ -1047,21 +1073,23 @@ static int launch_pk4n_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p)
     // against 10.3 / 10.7) and not on half a round (8192 x 2048 at 16 rows 7.52 against 6.63).
     const int ns1_rows = tune(ctx, OXQ_TUNE_PK4N_NS1_ROWS, ((N / 16 <= 256 && NB <= 32) || ((N / 16) % 256 == 0 && NB <= 64)) ? 16 : 8);
     const int ns = (M <= ns1_rows && M <= 16 && N / 16 >= 128) ? 1 : 4;
-    const int64_t tiles = (N / (16 * ns)) * ceil_div(M, 16 * mt);
+    const int64_t tiles = (N / (16 * ns)) * ceil_div(M, 16 * rows_mt);
     int ks = 1;
     if (tiles <= 96 && NB >= 32) ks = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tiles, NB / 8));
     else if (ns == 4 && tiles <= 128 && NB >= 64) ks = 2;  // as in the wide form; 128 single strips are faster whole
                                                            // (8192 x 2048 at one row: 5.20 against 5.65 us)
-    ks = tune(ctx, OXQ_TUNE_PK4_KS, ks);
-    ks = std::max(1, std::min(ks, NB));
     if (p.no_split) ks = 1;
+    const bool spread = tune(ctx, OXQ_TUNE_PK4_KS, 0) == 0;
+    const int mt = spread ? pk4_spread(ctx, p, N / (16 * ns), rows_mt, &ks) : rows_mt;
+    if (!spread) ks = p.no_split ? 1 : tune(ctx, OXQ_TUNE_PK4_KS, 0);
+    ks = std::max(1, std::min(ks, NB));
     while (ks > 1 && (size_t)ks * M * N * 4 > ctx->workspace_bytes) --ks;
     const int bslice = (int)ceil_div(NB, ks);
     ks = (int)ceil_div(NB, bslice);
     if (ceil_div(M, 16 * mt) > 65535)
         return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid limit (65535 row tiles)", (long long)M);
     if (p.act) return fail(OXQ_ERR_ARG, "repacked matmul: a fused activation on a layer in 16-column strips");
-    const bool fold = mt <= 2 && pk4_folds(ctx, p, mt);  // three row tiles of folded sums do not fit beside the two-block ring
+    const bool fold = rows_mt <= 2 && pk4_folds(ctx, p, rows_mt);  // three row tiles of folded sums do not fit beside the two-block ring
     dim3 grid((unsigned)(N / (16 * ns)), (unsigned)ks, (unsigned)ceil_div(M, 16 * mt));
     // One or two rows of a single strip on a long K: 16 waves, so that a wave's chain of blocks is half as
     // long (f16, one / two rows, 8 -> 16 waves: 14336 x 4096 7.44 / 7.55 -> 7.00 / 7.37 us, 8192 x 2048 at one
@@ -1078,8 +1106,8 @@ static int launch_pk4n_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p)
                         (M <= 8 || (M <= 16 && ceil_div(bslice, 16) <= 4));
     const bool w16 = nfront || (ns == 1 && M <= 2 && tune(ctx, OXQ_TUNE_PK4N_W16, NB >= 64));
     char name[64];
-    snprintf(name, sizeof name, "pk4_mfma_%s_mt%d%s_n16x%d", p.w.dtype == OXQ_F16 ? "f16" : "bf16", mt,
-             (fold || ns == 1) ? "_gs" : "", ns);
+    snprintf(name, sizeof name, "pk4_mfma_%s_mt%d%s_n16x%d%s", p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows_mt,
+             (fold || ns == 1) ? "_gs" : "", ns, pk4_by_name(mt, rows_mt));
     set_plan(ctx, name, grid, dim3(w16 ? 1024 : 512), ks, 1, ks > 1 ? (size_t)ks * M * N * 4 : 0);
     if (ctx->plan_only) {
         if (ks > 1) add_launch(ctx);
@@ -1101,7 +1129,7 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (pk4_gemm_takes(ctx, p)) return launch_pk4_gemm(ctx, s, p);  // prefill sizes, either layout
     if (p.w.strip == 16) return launch_pk4n_forward(ctx, s, p);
     const int64_t M = p.M;
-    const int mt = pk4_row_tiles(ctx, p);
+    const int rows_mt = pk4_row_tiles(ctx, p);  // settles the form
     const int NB = (int)ceil_div(p.w.K, 128), sets = pk4_sets(p.w.group_shift);
     const int64_t strips = ceil_div(p.w.N, 64);
     // Few column strips and a long K (a down projection: N = 4096 is 64 strips for 256 CUs):
@@ -1109,7 +1137,7 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     // runs; the slices' f32 partial tiles are added in slice order by a second launch.  Measured
     // (f16, M = 1 / 16): 14336 x 4096 16.9 / 19.1 us unsplit, 9.0 / 10.0 us in 4 slices, 9.5 - 10.2 /
     // 11.4 - 12.1 us in 3, 6 or 8; a 4096 x 4096 layer 6.4 / 7.4 us unsplit, 5.7 / 6.6 us in 4 slices.
-    const int64_t tiles = strips * ceil_div(M, 16 * mt);
+    const int64_t tiles = strips * ceil_div(M, 16 * rows_mt);
     int ks = 1;
     if (tiles <= 96 && NB >= 32) ks = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tiles, NB / 8));
     // Half a round of workgroups and a long K: two slices.  Measured (f16, 1 / 16 / 64 rows): 8192 x 8192
@@ -1117,10 +1145,12 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     // against 23.3 / 25.9 / 49.4 us (four slices: 23.4 / 26.8 / 54.2).  At K = 4096 or 5120 the second
     // launch costs more than the slices save (4096 x 8192: 6.7 / 7.8 / 13.5 against 7.0 / 8.0 / 14.9 us).
     else if (tiles <= 128 && NB >= 64) ks = 2;
-    ks = tune(ctx, OXQ_TUNE_PK4_KS, ks);
+    const bool whole = p.act || p.no_split;  // the activation needs the whole sum: gate|up layers are wide, one slice fills the chip
+    if (whole) ks = 1;
+    const bool spread = tune(ctx, OXQ_TUNE_PK4_KS, 0) == 0;
+    const int mt = spread ? pk4_spread(ctx, p, strips, rows_mt, &ks) : rows_mt;
+    if (!spread) ks = whole ? 1 : tune(ctx, OXQ_TUNE_PK4_KS, 0);
     ks = std::max(1, std::min(ks, NB));
-    if (p.act) ks = 1;  // the activation needs the whole sum: gate|up layers are wide, one slice fills the chip
-    if (p.no_split) ks = 1;
     while (ks > 1 && (size_t)ks * M * p.w.N * 4 > ctx->workspace_bytes) --ks;
     const int bslice = (int)ceil_div(NB, ks);
     ks = (int)ceil_div(NB, bslice);  // no empty slice
@@ -1154,15 +1184,16 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const int front_mode = tune(ctx, OXQ_TUNE_PK4_FRONT, 1);  // 0: the ring kernel, 2: never 16 waves
     const int share8 = (bslice + 7) / 8;
     int front = 0;
-    if (mt == 1 && front_mode != 0 && sets == 1) {
+    if (M <= 16 && front_mode != 0 && sets == 1) {
         if (p.w.bits == 4)
             front = (front_mode != 2 && bslice == 32 && front_xq <= 2) ? 1 : share8 <= 8 ? 2 : 0;
         else
             front = (front_mode != 2 && bslice == 32 && ks == 1) ? 1 : (bslice % 8 == 0 && share8 <= 8 && share8 != 7) ? 2 : 0;
     }
-    snprintf(name, sizeof name, "pk%d_mfma_%s_mt%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", mt,
-             pk4_folds(ctx, p, mt) ? "_gs" : "", sets == 2 ? "_g64" : sets == 4 ? "_g32" : "", front == 1 ? "_front" : front == 2 ? "_line" : "",
-             p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
+    const bool fold = pk4_folds(ctx, p, rows_mt);
+    snprintf(name, sizeof name, "pk%d_mfma_%s_mt%d%s%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows_mt,
+             fold ? "_gs" : "", sets == 2 ? "_g64" : sets == 4 ? "_g32" : "", front == 1 ? "_front" : front == 2 ? "_line" : "",
+             pk4_by_name(mt, rows_mt), p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(front == 1 ? 1024 : 512), ks, 1, ks > 1 ? (size_t)ks * M * p.w.N * 4 : 0);
     if (ctx->plan_only) {
         if (ks > 1) add_launch(ctx);
@@ -1175,21 +1206,21 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const bool f16 = p.w.dtype == OXQ_F16;
     int rc;
     if (sets > 1) {
-        rc = launch_pk4_fine(ctx, s, grid, p, bslice, mt, pk4_folds(ctx, p, mt));
+        rc = launch_pk4_fine(ctx, s, grid, p, bslice, mt, fold);
         if (rc != OXQ_OK || ks == 1) return rc;
         return launch_splitk_reduce(ctx, s, (const float *)ctx->workspace, p.bias, p.y, M, p.w.N, ks, p.w.dtype);
     }
-    if (tune(ctx, OXQ_TUNE_PK4_T64, 1) && !p.w.unrounded && pk4_tile64_takes(p, ks)) {
+    if (mt == 4 && tune(ctx, OXQ_TUNE_PK4_T64, 1) && !p.w.unrounded && pk4_tile64_takes(p, ks)) {
         Pk4Problem q = p;
         q.ws = ctx->workspace;
         return launch_pk4_tile64(ctx, s, q);
     }
     if (p.w.bits == 4)
-        rc = f16 ? pk4_by_mt<F16Traits, 4>(ctx, s, grid, p, bslice, mt, front)
-                 : pk4_by_mt<BF16Traits, 4>(ctx, s, grid, p, bslice, mt, front);
+        rc = f16 ? pk4_by_mt<F16Traits, 4>(ctx, s, grid, p, bslice, mt, fold, front)
+                 : pk4_by_mt<BF16Traits, 4>(ctx, s, grid, p, bslice, mt, fold, front);
     else
-        rc = f16 ? pk4_by_mt<F16Traits, 8>(ctx, s, grid, p, bslice, mt, front)
-                 : pk4_by_mt<BF16Traits, 8>(ctx, s, grid, p, bslice, mt, front);
+        rc = f16 ? pk4_by_mt<F16Traits, 8>(ctx, s, grid, p, bslice, mt, fold, front)
+                 : pk4_by_mt<BF16Traits, 8>(ctx, s, grid, p, bslice, mt, fold, front);
     if (rc != OXQ_OK || ks == 1) return rc;
     return launch_splitk_reduce(ctx, s, (const float *)ctx->workspace, p.bias, p.y, M, p.w.N, ks, p.w.dtype);
 }

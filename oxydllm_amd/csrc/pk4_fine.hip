@@ -19,6 +19,7 @@ static int fine_by_mt(oxq_ctx *ctx, hipStream_t s, dim3 grid, const Pk4Problem &
     constexpr int WD = 4;
     switch (mt) {
     case 1:
+        if (!fold) return pk4_mfma_go<TT, BITS, 1, false, WD, 4, false, 0, SETS>(ctx, s, grid, p, bslice);
         if (p.M <= 4) return pk4_mfma_go<TT, BITS, 1, true, WD, 1, false, 0, SETS>(ctx, s, grid, p, bslice);
         if (p.M <= 8) return pk4_mfma_go<TT, BITS, 1, true, WD, 2, false, 0, SETS>(ctx, s, grid, p, bslice);
         return pk4_mfma_go<TT, BITS, 1, true, WD, 4, false, 0, SETS>(ctx, s, grid, p, bslice);

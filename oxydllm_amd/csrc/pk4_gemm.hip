@@ -256,8 +256,9 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     };
     const double c64 = !c.pairs64 || w64 <= 1.0 ? rounds(w64, 1.0, c.part64, 0.75) : w64 <= 2.0 ? c.a64 + c.b64 * w64 : c.slope64 * w64;
     const double c128 = rounds(w128, c.full128, c.part128, 0.7);
-    // the split-K tiles of the 16-column layout are one workgroup a row tile and 64 columns, in whole rounds too
-    const double c_split = (w64 < 1.0 ? c.split_lo : c.split_hi) * (p.w.strip == 16 ? std::ceil(8.0 * w64 - 1e-9) / 8.0 : w64);
+    // the split-K tiles are one workgroup a row tile and 64 columns, in whole rounds too (64-column strips: up to two of them,
+    // beyond that fitted without; 1664 x 4224 f16 at 200 rows, 264 tiles, 15.4 us, 12.1 at 300 rows in the two-strip form)
+    const double c_split = (w64 < 1.0 ? c.split_lo : c.split_hi) * (p.w.strip == 16 || w64 <= 0.25 ? std::ceil(8.0 * w64 - 1e-9) / 8.0 : w64);
     // two strips a workgroup (128 KB of LDS: one a CU), whole rounds of `PK4_MID_ROUND` each
     const double w_mid = (double)(ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)2) * ceil_div(p.M, (int64_t)64)) / cus;
     const double c_mid = forced_ks == 1        ? 1e30
