@@ -1,0 +1,72 @@
+"""AWQ checkpoint layout, few rows on the matrix cores (awq_slab_kernel): against the oracle's unrounded weights."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from oxydllm_amd import ops, synth
+from tests.helpers import TORCH_DT, assert_close, bits_of, round_x, to_dev, tune
+
+pytestmark = pytest.mark.gpu
+DT = {"f16": oracle.F16, "bf16": oracle.BF16}
+
+
+def call(x, d, bits, m):
+    if m > 8:
+        return ops.mpp_quant_matmul(x, *d, bits, ops.PACK_OUT)
+    return ops.w4a16_matmul(x, *d) if bits == 4 else ops.w8a16_matmul(x, *d)
+
+
+@pytest.mark.parametrize("bits,K,N,g,ms", [
+    (4, 1152, 3080, 128, (2, 3, 8)),      # 64-row runs; the last workgroup 8 columns wide
+    (4, 1120, 1032, 32, (1, 4, 5, 8)),    # K ends inside a run; groups inside a run
+    (4, 1216, 264, 64, (2, 7)),
+    (4, 4096, 6144, 128, (2, 8)),         # 128-row runs
+    (4, 5120, 13824, 64, (2,)),           # two runs a wave
+    (4, 4064, 8200, 32, (1, 6)),          # 128-row runs of four groups, K inside one
+    (8, 576, 1032, 64, (2, 5, 8)),
+    (8, 1120, 1000, 32, (1, 3, 8, 9, 16)),
+    (8, 8192, 14336, 128, (2, 16)),       # several runs a wave
+])
+@pytest.mark.parametrize("dtn", ["f16", "bf16"])
+def test_against_the_oracle(bits, K, N, g, ms, dtn):
+    dt = DT[dtn]
+    qw, qz, sc = synth.awq_checkpoint(K, N, g, bits, seed=K + N)
+    d = (to_dev(qw), to_dev(qz), to_dev(sc, TORCH_DT[dt]))
+    s = oracle.round_through(sc, dt)
+    w = oracle.dequantize_awq(qw, qz, s) if bits == 4 else oracle.dequantize_awq8(qw, qz, s)
+    rng = np.random.default_rng(K)
+    for m in ms:
+        print(f"[case] awq slab {bits} {dtn} K={K} N={N} g={g} m={m}", flush=True)
+        x = rng.standard_normal((m, K)).astype(np.float32)
+        xd = to_dev(x, TORCH_DT[dt])
+        y = call(xd, d, bits, m)
+        assert "_slab" in ops.default_context().last_plan()["kernel"], ops.default_context().last_plan()
+        assert_close(y, oracle.matmul_nt_f32(round_x(x, dt), w), f"awq slab {bits} {dtn} m{m}")
+        assert np.array_equal(bits_of(call(xd, d, bits, m)), bits_of(y))
+
+
+def test_an_infinite_f16_row_keeps_its_signs():
+    """Where the weight is not zero, infinity times it; the other rows as without it.  The rows-of-16 kernel that such calls ran
+    on gives the same."""
+    K, N = 1024, 1024
+    qw, qz, sc = synth.awq_checkpoint(K, N, 128, 4, seed=9)
+    d = (to_dev(qw), to_dev(qz), to_dev(sc, torch.float16))
+    x = np.random.default_rng(1).standard_normal((4, K)).astype(np.float32)
+    clean = to_dev(x, torch.float16)
+    x[1, 37], x[2, 900], x[3, 5], x[3, 6] = np.inf, -np.inf, np.nan, np.inf
+    xd = to_dev(x, torch.float16)
+    tune("OXQ_GEMV_TILE", None)
+    big = [torch.cat([t, t], 1).contiguous() for t in d]   # 2048 columns: enough workgroups for the kernel
+    big = [torch.cat([t] * 4, 1).contiguous() for t in big]
+    y = ops.w4a16_matmul(xd, *big)
+    assert "_slab" in ops.default_context().last_plan()["kernel"]
+    tune("OXQ_GEMV_TILE", 0)
+    old = ops.mpp_quant_matmul(torch.cat([xd] * 3), *big, 4, ops.PACK_OUT)[:4]
+    assert "awq4_mfma" in ops.default_context().last_plan()["kernel"]
+    tune("OXQ_GEMV_TILE", None)
+    for r in (1, 2, 3):
+        a, b = y[r].float(), old[r].float()
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+    assert bool(torch.isposinf(y[1]).any()) and bool(torch.isneginf(y[1]).any())
+    assert torch.equal(y[0], ops.w4a16_matmul(clean, *big)[0]) or bool(((y[0] - ops.w4a16_matmul(clean, *big)[0]).abs() <= 2e-3 * y[0].abs() + 1e-2).all())
