@@ -205,9 +205,9 @@ struct Pk4Problem {
 };
 
 // ---- launchers (defined in the .hip files) ---------------------------------
-// AWQ checkpoint layout, few rows on the matrix cores (awq_slab.hip)
-bool awq_slab_takes(const oxq_ctx *ctx, const Wna16Problem &p);
-int launch_awq_slab(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p);
+// checkpoint layouts, few rows on the matrix cores (wna16_slab.hip)
+bool wna16_slab_takes(const oxq_ctx *ctx, const Wna16Problem &p);
+int launch_wna16_slab(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p);
 bool pk4_eligible(const Wna16Problem &p);
 bool pk4_unrounded(const Wna16Problem &p);
 // resident 4-bit layers at prefill sizes: 64 rows x eight strips a workgroup (pk4_gemm.hip)

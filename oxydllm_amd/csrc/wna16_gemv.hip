@@ -920,7 +920,7 @@ static int launch_gptq_fast(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) 
 
 int launch_wna16_gemv(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     const bool f16 = p.dtype == OXQ_F16;
-    if (awq_slab_takes(ctx, p)) return launch_awq_slab(ctx, s, p);
+    if (wna16_slab_takes(ctx, p)) return launch_wna16_slab(ctx, s, p);
     // 2..8 rows of f16 on 4-bit AWQ: the matrix-core tile kernel reads the weights once for all
     // rows (13 - 14 us against 17 - 33 us for the dot2 kernel at 4096 x 14336).  Its B operand is
     // the dequantized weight rounded to f16, 2^-12 relative: far inside the tolerance; bf16, whose

@@ -735,19 +735,21 @@ int launch_wna16_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
                                   : launch_awq4_mfma<BF16Traits>(ctx, s, p);
     if (gptq_tile_ok(p) && tune(ctx, OXQ_TUNE_GPTQ_TILE, 1) && !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0))
         return launch_gptq_tile(ctx, s, p);
-    // 8-bit AWQ up to 16 rows: the kernel of the decode ops (4096 x 14336 / 4096 x 4096 at 16 rows 67.5 / 24.5 -> 22.3 / 12.5 us)
-    if (p.bits == 8 && awq_slab_takes(ctx, p)) return launch_awq_slab(ctx, s, p);
+    // up to 16 rows: the kernel of the decode ops (AWQ 8-bit 4096 x 14336 / 4096 x 4096 at 16 rows 67.5 / 24.5 -> 22.3 / 12.5 us)
+    if (wna16_slab_takes(ctx, p)) return launch_wna16_slab(ctx, s, p);
     // Layouts without a tile kernel of their own on the checkpoint layout (8-bit AWQ, unaligned GPTQ): when the
     // tile-major copy fits the ctx workspace, build it there and run the resident-layer kernel on it: one launch
     // more instead of one GEMV pass over the weights per 8 rows (35 - 45 us each): ahead from m = 9.
     if (transient_repack_fits(ctx, p)) return launch_transient_repack(ctx, s, p);
     // Otherwise (unaligned shapes, copies larger than the workspace): the GEMV kernel over chunks of 8
-    // rows, as the reference does below its tile-GEMM threshold (linear.rs:457-480).
+    // rows, as the reference does below its tile-GEMM threshold (linear.rs:457-480); of 16 where the matrix cores take them.
     uint32_t launches = 0;
     const size_t eb = 2;
-    for (int64_t m0 = 0; m0 < p.M; m0 += 8) {
-        Wna16Problem c = p;
-        c.M = (p.M - m0) < 8 ? (p.M - m0) : 8;
+    Wna16Problem c = p;
+    c.M = std::min<int64_t>(p.M, 16);
+    const int64_t step = wna16_slab_takes(ctx, c) ? 16 : 8;
+    for (int64_t m0 = 0; m0 < p.M; m0 += step) {
+        c.M = std::min(p.M - m0, step);
         c.x = (const uint8_t *)p.x + (size_t)m0 * p.K * eb;
         c.y = (uint8_t *)p.y + (size_t)m0 * p.N * eb;
         int rc = launch_wna16_gemv(ctx, s, c);

@@ -1,4 +1,4 @@
-"""AWQ checkpoint layout, few rows on the matrix cores (awq_slab_kernel): against the oracle's unrounded weights."""
+"""The checkpoint layouts at few rows on the matrix cores (wna16_slab_kernel): against the oracle's unrounded weights."""
 import numpy as np
 import pytest
 import torch
@@ -22,14 +22,14 @@ def call(x, d, bits, m):
     (4, 1120, 1032, 32, (1, 4, 5, 8)),    # K ends inside a run; groups inside a run
     (4, 1216, 264, 64, (2, 7)),
     (4, 4096, 6144, 128, (2, 8)),         # 128-row runs
-    (4, 5120, 13824, 64, (2,)),           # two runs a wave
-    (4, 4064, 8200, 32, (1, 6)),          # 128-row runs of four groups, K inside one
+    (4, 5120, 13824, 128, (2,)),          # two runs a wave
+    (4, 4064, 8200, 32, (1, 6)),          # K ends inside a run
     (8, 576, 1032, 64, (2, 5, 8)),
     (8, 1120, 1000, 32, (1, 3, 8, 9, 16)),
     (8, 8192, 14336, 128, (2, 16)),       # several runs a wave
 ])
 @pytest.mark.parametrize("dtn", ["f16", "bf16"])
-def test_against_the_oracle(bits, K, N, g, ms, dtn):
+def test_awq_against_the_oracle(bits, K, N, g, ms, dtn):
     dt = DT[dtn]
     qw, qz, sc = synth.awq_checkpoint(K, N, g, bits, seed=K + N)
     d = (to_dev(qw), to_dev(qz), to_dev(sc, TORCH_DT[dt]))
@@ -44,6 +44,62 @@ def test_against_the_oracle(bits, K, N, g, ms, dtn):
         assert "_slab" in ops.default_context().last_plan()["kernel"], ops.default_context().last_plan()
         assert_close(y, oracle.matmul_nt_f32(round_x(x, dt), w), f"awq slab {bits} {dtn} m{m}")
         assert np.array_equal(bits_of(call(xd, d, bits, m)), bits_of(y))
+
+
+@pytest.mark.parametrize("bits,K,N,g,ms", [
+    (4, 1120, 1032, 32, (3, 8, 9, 16)),   # K ends inside a run; the last workgroup 8 columns wide
+    (4, 4096, 4096, 64, (1, 2, 7, 16)),
+    (4, 5120, 13832, 128, (2, 16)),       # 128-row runs, two a wave
+    (8, 1216, 1000, 64, (3, 8, 16)),
+    (8, 1120, 1032, 32, (5, 12)),
+    (8, 4096, 4104, 128, (2, 9, 40)),     # 40 rows: the copy in the workspace
+])
+@pytest.mark.parametrize("dtn", ["f16", "bf16"])
+def test_gptq_against_the_oracle(bits, K, N, g, ms, dtn):
+    dt = DT[dtn]
+    qw, qz, sc = synth.gptq_checkpoint(K, N, g, bits, seed=K + N)
+    d = (to_dev(qw), to_dev(qz), to_dev(sc, TORCH_DT[dt]))
+    w = oracle.dequantize_gptq(qw, qz, oracle.round_through(sc, dt), bits)
+    rng = np.random.default_rng(K)
+    for m in ms:
+        print(f"[case] gptq slab {bits} {dtn} K={K} N={N} g={g} m={m}", flush=True)
+        x = rng.standard_normal((m, K)).astype(np.float32)
+        xd = to_dev(x, TORCH_DT[dt])
+        y = ops.gptq_matmul(xd, *d, bits) if m <= 8 else ops.mpp_quant_matmul(xd, *d, bits, ops.PACK_IN)
+        assert ("_slab" in ops.default_context().last_plan()["kernel"]) == (m <= 16), ops.default_context().last_plan()
+        ref = oracle.matmul_nt_f32(round_x(x, dt), w)
+        assert_close(y, ref, f"gptq slab {bits} {dtn} m{m}")
+        if m > 16:  # passes of 16 rows
+            tune("OXQ_TRANSIENT_REPACK", 0)
+            y = ops.mpp_quant_matmul(xd, *d, bits, ops.PACK_IN)
+            assert "_slab" in ops.default_context().last_plan()["kernel"]
+            assert_close(y, ref, f"gptq slab passes {bits} {dtn} m{m}")
+            tune("OXQ_TRANSIENT_REPACK", None)
+
+
+@pytest.mark.parametrize("dtn", ["f16", "bf16"])
+@pytest.mark.parametrize("method,bits", [("gptq", 4), ("gptq", 8), ("awq", 4), ("awq", 8)])
+def test_infinite_rows_give_what_the_generic_kernel_gives(method, bits, dtn):
+    K, N, g, dt = 4096, 2048, 32, DT[dtn]
+    qw, qz, sc = (synth.gptq_checkpoint if method == "gptq" else synth.awq_checkpoint)(K, N, g, bits, seed=3)
+    d = (to_dev(qw), to_dev(qz), to_dev(sc, TORCH_DT[dt]))
+    x = np.random.default_rng(1).standard_normal((4, K)).astype(np.float32)
+    x[1, 37], x[2, 900], x[3, 5], x[3, 6] = np.inf, -np.inf, np.nan, np.inf
+    xd = to_dev(x, TORCH_DT[dt])
+
+    def op():
+        if method == "gptq":
+            return ops.gptq_matmul(xd, *d, bits)
+        return ops.w4a16_matmul(xd, *d) if bits == 4 else ops.w8a16_matmul(xd, *d)
+    y = op()
+    assert "_slab" in ops.default_context().last_plan()["kernel"]
+    tune("OXQ_FORCE_GENERIC", 1)
+    old = op()
+    assert "generic" in ops.default_context().last_plan()["kernel"]
+    tune("OXQ_FORCE_GENERIC", None)
+    for r in (1, 2, 3):
+        assert torch.equal(torch.isnan(y[r]), torch.isnan(old[r])) and torch.equal(torch.nan_to_num(y[r]), torch.nan_to_num(old[r]))
+    assert bool(torch.isposinf(y[1]).any()) and bool(torch.isneginf(y[1]).any())
 
 
 def test_an_infinite_f16_row_keeps_its_signs():
