@@ -16,7 +16,8 @@
 //                 its four, stored as q + 128) + [16 columns][4 units] f16 d                             2176 B
 //   Q4_1  as Q4_0, the unit headers are {d, m} pairs                                                     1280 B
 //   Q5_0  as Q4_0 + [64 lanes][4 B] of fifth bits: the bit of element 2 pp (2 pp + 1) of unit t in bit
-//         4 t + pp (16 + 4 t + pp), so that one shift puts a pair's bits at positions 4 and 20           1408 B
+//         ggm_bit_at(t, pp) of the low (high) half: one shift puts a pair's bits at positions 4 and 20, or those of
+//         pairs 0 and 2 (1 and 3) at bit 4 of the four bytes that hold their nibbles                        1408 B
 //   Q5_1  as Q5_0 with {d, m} pairs                                                                      1536 B
 //   Q5_K  as Q4_K with the plane of fifth bits in every chunk                                            2816 B
 //   Q4_K  block = 2 chunks of [64 lanes][16 B] nibbles as Q4_0 + [16 columns] the super-block's first 16
@@ -25,7 +26,7 @@
 //                 int8 scales } + [16 columns] f16 d.  A scale covers 16 elements, so a step is a sub-block of 16
 //                 and v_mfma_f32_16x16x16_bf16: step s of the chunk takes elements 16 s + 4 kb .. + 3; their
 //                 nibbles sit in word s / 2 as Q4_0's pairs 2 (s % 2) and 2 (s % 2) + 1, their bit pairs in
-//                 word s / 4 of the second plane, field 2 (s % 4) + pair of each 16-bit half              3360 B
+//                 word s / 4 of the second plane, bit ggm_pair_at(2 (s % 4) + pair) of each 16-bit half   3360 B
 //
 // Exactly the file's bytes per weight.  The integers stay integers: the MFMA accumulates x * (bias + q) in f32
 // (products of 8-bit significands are exact), a second MFMA against the constant -(bias + offset) takes the
@@ -54,6 +55,11 @@ template <> struct GgmFmt<OXQ_GGUF_Q6_K> { static constexpr int WQ = 1, CH = 2, 
 // formats with a fifth bit; with a minimum beside the scale
 template <int FMT> constexpr bool ggm_fifth_bit = FMT == OXQ_GGUF_Q5_0 || FMT == OXQ_GGUF_Q5_1 || FMT == OXQ_GGUF_Q5_K;
 template <int FMT> constexpr bool ggm_has_min = FMT == OXQ_GGUF_Q4_K || FMT == OXQ_GGUF_Q5_K || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q5_1;
+
+// Place in its 16-bit half of the fifth bit of pair pp of unit t, and of the bit pair of field f (Q6_K): pairs 0, 1 of a unit in the
+// low byte, 2, 3 in the high one.
+__device__ constexpr int ggm_bit_at(int t, int pp) { return 2 * t + (pp & 1) + 8 * (pp >> 1); }
+__device__ constexpr int ggm_pair_at(int f) { return 2 * (2 * (f >> 2) + (f & 1)) + 8 * ((f >> 1) & 1); }
 
 template <int FMT> struct GgmLayout {
     typedef GgmFmt<FMT> F;
@@ -151,7 +157,7 @@ __global__ __launch_bounds__(256) void ggm_repack_kernel(const uint8_t *__restri
                 const int e = 8 * kb + i;
                 const uint32_t nib = e < 16 ? (p[QS + e] & 0xFu) : (p[QS + e - 16] >> 4);
                 v |= nib << (4 * (i >> 1) + 16 * (i & 1));
-                hb |= ((qh >> e) & 1u) << (4 * t + (i >> 1) + 16 * (i & 1));
+                hb |= ((qh >> e) & 1u) << (ggm_bit_at(t, i >> 1) + 16 * (i & 1));
             }
             q[t] = v;
             if (t == kb) {
@@ -176,7 +182,7 @@ __global__ __launch_bounds__(256) void ggm_repack_kernel(const uint8_t *__restri
             for (int i = 0; i < 8; ++i) {
                 const uint32_t byte = qs[(sb >> 1) * 32 + 8 * kb + i];
                 v |= ((sb & 1) ? (byte >> 4) : (byte & 0xFu)) << (4 * (i >> 1) + 16 * (i & 1));
-                if constexpr (FIFTH) hb |= (((uint32_t)p[16 + 8 * kb + i] >> sb) & 1u) << (4 * t + (i >> 1) + 16 * (i & 1));
+                if constexpr (FIFTH) hb |= (((uint32_t)p[16 + 8 * kb + i] >> sb) & 1u) << (ggm_bit_at(t, i >> 1) + 16 * (i & 1));
             }
             q[t] = v;
         }
@@ -200,7 +206,7 @@ __global__ __launch_bounds__(256) void ggm_repack_kernel(const uint8_t *__restri
                 const uint32_t hi = (p[128 + 32 * h + l] >> (2 * qq)) & 3u;
                 const int pair = i >> 1, half = i & 1;
                 lw[s2 >> 1] |= lo << (4 * (2 * (s2 & 1) + pair) + 16 * half);
-                hw[s2 >> 2] |= hi << (2 * (2 * (s2 & 3) + pair) + 16 * half);
+                hw[s2 >> 2] |= hi << (ggm_pair_at(2 * (s2 & 3) + pair) + 16 * half);
             }
         *(u32x4_t *)(chunk + lane * 16) = u32x4_t{lw[0], lw[1], lw[2], lw[3]};
         *(uint2 *)(chunk + L::H_OFF + lane * 8) = uint2{hw[0], hw[1]};
@@ -261,7 +267,7 @@ __global__ __launch_bounds__(256) void ggm_dequant_kernel(const uint8_t *__restr
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const uint32_t v = ((q[t] >> (4 * (i >> 1) + 16 * (i & 1))) & 0xFu) |
-                                   (((hb >> (4 * t + (i >> 1) + 16 * (i & 1))) & 1u) << 4);
+                                   (((hb >> (ggm_bit_at(t, i >> 1) + 16 * (i & 1))) & 1u) << 4);
                 o[32 * t + i] = MIN ? (float)v * d + m : (float)((int)v - 16) * d;
             }
         }
@@ -279,7 +285,7 @@ __global__ __launch_bounds__(256) void ggm_dequant_kernel(const uint8_t *__restr
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 o[32 * t + i] = d1 * (float)(((q[t] >> (4 * (i >> 1) + 16 * (i & 1))) & 0xFu) |
-                                             (((hb >> (4 * t + (i >> 1) + 16 * (i & 1))) & 1u) << 4)) - m1;
+                                             (((hb >> (ggm_bit_at(t, i >> 1) + 16 * (i & 1))) & 1u) << 4)) - m1;
         }
     } else if constexpr (FMT == OXQ_GGUF_Q6_K) {
         const u32x4_t lw = *(const u32x4_t *)(chunk + lane * 16);
@@ -293,7 +299,7 @@ __global__ __launch_bounds__(256) void ggm_dequant_kernel(const uint8_t *__restr
             for (int i = 0; i < 4; ++i) {
                 const int pair = i >> 1, half = i & 1;
                 const uint32_t lo = (lw[s2 >> 1] >> (4 * (2 * (s2 & 1) + pair) + 16 * half)) & 0xFu;
-                const uint32_t hi = ((s2 < 4 ? hw.x : hw.y) >> (2 * (2 * (s2 & 3) + pair) + 16 * half)) & 3u;
+                const uint32_t hi = ((s2 < 4 ? hw.x : hw.y) >> (ggm_pair_at(2 * (s2 & 3) + pair) + 16 * half)) & 3u;
                 o6[16 * s2 + i] = ds * (float)((int)(lo | (hi << 4)) - 32);
             }
         }
@@ -384,6 +390,14 @@ template <int FMT> struct GgmChunk {
             for (int st = 0; st < 4; ++st) f0[st] = ggm_f16((st & 1) ? (uh[st >> 1] >> 16) : (uh[st >> 1] & 0xFFFFu)), f1[st] = 0.f;
         }
     }
+    // The five- and six-bit integers of 32 elements, a byte each: bytes 0, 2 of lo, hi pairs 0, 1; bytes 1, 3 pairs 2, 3
+    __device__ __forceinline__ void bytes(int st, uint32_t &lo, uint32_t &hi) const {
+        const int at = FMT == OXQ_GGUF_Q6_K ? ggm_pair_at(4 * (st & 1)) : ggm_bit_at(st, 0), next = FMT == OXQ_GGUF_Q6_K ? 2 : 1;
+        constexpr uint32_t MASK = FMT == OXQ_GGUF_Q6_K ? 0x30303030u : 0x10101010u;
+        const uint32_t w = q[0][st], h = FMT == OXQ_GGUF_Q6_K ? qh[st >> 1] : qh[0];
+        auto moved = [&](int a) { return a < 4 ? h << (4 - a) : h >> (a - 4); };
+        lo = (moved(at) & MASK) | (w & 0x0F0F0F0Fu), hi = (moved(at + next) & MASK) | ((w >> 4) & 0x0F0F0F0Fu);
+    }
     // B operand of step st: bias + q as bf16 pairs (four for a step of 32 elements, two for one of 16)
     __device__ __forceinline__ void operand(int st, uint32_t (&b)[4], const NibbleMasks &nm) const {
         if constexpr (FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_K || FMT == OXQ_GGUF_Q4_1) {
@@ -392,7 +406,7 @@ template <int FMT> struct GgmChunk {
         } else if constexpr (ggm_fifth_bit<FMT>) {  // nibble | fifth bit << 4; m1: the bits' mask, in a register
 #pragma unroll
             for (int pp = 0; pp < 4; ++pp) {
-                const int sft = 4 * st + pp - 4;
+                const int sft = ggm_bit_at(st, pp) - 4;
                 const uint32_t hs = sft < 0 ? (qh[0] << -sft) : (qh[0] >> sft);
                 b[pp] = (hs & nm.m1) | BF16Traits::unpack1(q[0][st], pp, nm);
             }
@@ -403,8 +417,8 @@ template <int FMT> struct GgmChunk {
             const uint32_t lw = q[0][st >> 1], hw = qh[st >> 2];
 #pragma unroll
             for (int pr = 0; pr < 2; ++pr) {
-                const int f = 2 * (st & 3) + pr;
-                const uint32_t hs = f < 2 ? (hw << (4 - 2 * f)) : (hw >> (2 * f - 4));
+                const int at = ggm_pair_at(2 * (st & 3) + pr);
+                const uint32_t hs = at < 4 ? (hw << (4 - at)) : (hw >> (at - 4));
                 b[pr] = (hs & nm.m1) | BF16Traits::unpack1(lw, 2 * (st & 1) + pr, nm);  // m1: the bit pairs' mask, in a register
             }
             b[2] = b[3] = 0u;
@@ -442,22 +456,21 @@ template <int FMT> struct GgmSmallBias {
             b[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
             b[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
             b[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
-        } else if constexpr (PLAIN) {  // pair pp: nibble pp and bit 4 st + pp of each half; bytes 0, 2 hold pair 0 or 1, bytes 1, 3 pair 2 or 3
-            const uint32_t h = w.qh[0] >> (4 * st);
-            const uint32_t lo = (w.q[0][st] & 0x0F0F0F0Fu) | ((h & 0x00010001u) << 4) | ((h & 0x00040004u) << 10);
-            const uint32_t hi = ((w.q[0][st] >> 4) & 0x0F0F0F0Fu) | ((h & 0x00020002u) << 3) | ((h & 0x00080008u) << 9);
+        } else if constexpr (PLAIN) {  // bytes 0, 2 hold pair 0 or 1, bytes 1, 3 pair 2 or 3
+            uint32_t lo, hi;
+            w.bytes(st, lo, hi);
             b[0] = ggm_bytes02(lo), b[1] = ggm_bytes02(hi), b[2] = ggm_bytes13(lo), b[3] = ggm_bytes13(hi);
         } else if constexpr (NIB) {
 #pragma unroll
             for (int pp = 0; pp < 4; ++pp) b[pp] = (move(w.q[0][st], AT - 4 * pp) & nm.m0) | EXP;
-        } else if constexpr (ggm_fifth_bit<FMT>) {  // the bit of pair pp: bit 4 st + pp -> 6
+        } else if constexpr (ggm_fifth_bit<FMT>) {  // the bit of pair pp -> 6
 #pragma unroll
             for (int pp = 0; pp < 4; ++pp)
-                b[pp] = (move(w.qh[0], 6 - 4 * st - pp) & nm.m1) | ((move(w.q[0][st], AT - 4 * pp) & nm.m0) | EXP);
-        } else if constexpr (FMT == OXQ_GGUF_Q6_K) {  // the bit pair of field f: bits 2 f, 2 f + 1 -> 5, 6
+                b[pp] = (move(w.qh[0], 6 - ggm_bit_at(st, pp)) & nm.m1) | ((move(w.q[0][st], AT - 4 * pp) & nm.m0) | EXP);
+        } else if constexpr (FMT == OXQ_GGUF_Q6_K) {  // the bit pair of field f -> 5, 6
 #pragma unroll
             for (int pr = 0; pr < 2; ++pr)
-                b[pr] = (move(w.qh[st >> 2], 5 - 2 * (2 * (st & 3) + pr)) & nm.m1) |
+                b[pr] = (move(w.qh[st >> 2], 5 - ggm_pair_at(2 * (st & 3) + pr)) & nm.m1) |
                         ((move(w.q[0][st >> 1], AT - 4 * (2 * (st & 1) + pr)) & nm.m0) | EXP);
             b[2] = b[3] = 0u;
         } else {
@@ -835,6 +848,11 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 // with such workgroups: gridDim.y slices of `cslice` chunks each then write their f32 tiles to `part` and a second
 // launch adds them in slice order.  half: a fused gate|up layer without its activation - columns go back to the
 // file's order (ggm_src_row).
+// What bounds it: the conversion's vector instructions beside the MFMAs.  The five- and six-bit formats join nibble and plane bits
+// four weights at a time into bytes (GgmChunk::bytes), 3.4 instructions a weight; pair by pair as the integer kernel's operand
+// they took 4.3, and 5.3 with a minimum added behind the fma.  Q6_K multiplies its two scales of a 32-element step into one
+// MFMA's operand (of 16 elements each before).  bf16, us, before -> here: Q6_K / Q5_K / Q5_1 / Q5_0 4096 x 4096 at 2048 rows 127 / 130 /
+// 123 / 108 -> 113 / 105 / 96 / 95, 14336 x 4096 at 33 rows 25.8 / 25.4 / 24.6 / 22.8 -> 22.6 / 21.1 / 20.1 / 20.0.
 template <int FMT, int MT, int KS>
 __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw,
                                                        const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
@@ -845,10 +863,10 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
     typedef GgmFmt<FMT> F;
     typedef GgmLayout<FMT> L;
     typedef GgmChunk<FMT> C;
-    static_assert(KS == 1 || KS == MT, "wave kq of a column group finishes row tile kq");
+    static_assert(KS == 1 || KS >= MT, "wave kq of a column group finishes row tile kq");
     constexpr int SPW = 8 / KS;  // waves of 64 columns a workgroup
     constexpr int ROWS = 16 * MT, XBUF = KS * ROWS * 256, XV = ROWS / 4 / SPW, NSTEP = C::NSTEP;
-    constexpr bool K16 = NSTEP == 8;
+    constexpr bool K16 = NSTEP == 8;  // scales of 16 elements: an MFMA takes two of them, four elements a lane each
     constexpr int RING = 4 * C::LOADS;  // vector loads of a chunk's weights: younger than the chunk's loads of x
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
 
@@ -890,8 +908,6 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
 #pragma unroll
     for (int st = 0; st < NSTEP; ++st)
         a_rd[st] = K16 ? ni * 256 + (((2 * st + (kb >> 1)) ^ ni) << 4) + (kb & 1) * 8 : ni * 256 + (((4 * st + kb) ^ ni) << 4);
-    const NibbleMasks nm = FMT == OXQ_GGUF_Q6_K ? NibbleMasks{vgpr_const(0x000F000Fu), vgpr_const(0x00300030u)}
-                           : ggm_fifth_bit<FMT> ? NibbleMasks{vgpr_const(0x000F000Fu), vgpr_const(0x00100010u)} : nibble_masks();
     constexpr float NEGF = __builtin_bit_cast(float, (F::NEG & 0xFFFFu) << 16);
     constexpr bool NIB = FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q4_K;
 
@@ -942,13 +958,13 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
             }
         }
 #pragma unroll
-        for (int st = 0; st < NSTEP; ++st) {
+        for (int st = 0; st < 4; ++st) {
             uint32_t a[MT][4];
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 if constexpr (K16) {
-                    const uint2 av = *(const uint2 *)(buf + mt * 4096 + a_rd[st]);
-                    a[mt][0] = av.x, a[mt][1] = av.y, a[mt][2] = 0u, a[mt][3] = 0u;
+                    const uint2 a0 = *(const uint2 *)(buf + mt * 4096 + a_rd[2 * st]), a1 = *(const uint2 *)(buf + mt * 4096 + a_rd[2 * st + 1]);
+                    a[mt][0] = a0.x, a[mt][1] = a0.y, a[mt][2] = a1.x, a[mt][3] = a1.y;
                 } else {
                     const u32x4_t av = *(const u32x4_t *)(buf + mt * 4096 + a_rd[st]);
                     a[mt][0] = av[0], a[mt][1] = av[1], a[mt][2] = av[2], a[mt][3] = av[3];
@@ -958,7 +974,13 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
             for (int f = 0; f < 4; ++f) {
                 uint32_t b[4];
                 const float sc = f0[f][st];
-                if constexpr (NIB) {
+                if constexpr (K16) {
+                    uint32_t lo, hi;
+                    wr[CUR][f].bytes(st, lo, hi);
+                    Pk4gBf16 c0, c1;
+                    c0.set(f0[f][2 * st], -32.0f), c1.set(f0[f][2 * st + 1], -32.0f);
+                    b[0] = c0.template bytes<0>(lo), b[1] = c0.template bytes<0>(hi), b[2] = c1.template bytes<1>(lo), b[3] = c1.template bytes<1>(hi);
+                } else if constexpr (NIB) {
                     // plain nibbles (pair pp = nibble pp of each 16-bit half)
                     Pk4gBf16 cv;
                     cv.s = sc, cv.c = C::HAS_MIN ? c2[f][st] : (NEGF + 128.0f) * sc;
@@ -970,23 +992,15 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
                     cv.s = sc, cv.c = -128.0f * sc;
                     b[0] = cv.template bytes<0>(w0), b[1] = cv.template bytes<1>(w0);
                     b[2] = cv.template bytes<0>(w1), b[3] = cv.template bytes<1>(w1);
-                } else {
-                    // bias + q as bf16 (the integer kernel's operand): f0 (bias + q) + NEG f0 is exact in one fma
-                    wr[CUR][f].operand(st, b, nm);
-                    const float c = NEGF * sc;
-#pragma unroll
-                    for (int pp = 0; pp < (K16 ? 2 : 4); ++pp) {
-                        float lo = __builtin_fmaf(__builtin_bit_cast(float, b[pp] << 16), sc, c);
-                        float hi = __builtin_fmaf(__builtin_bit_cast(float, b[pp] & 0xFFFF0000u), sc, c);
-                        if constexpr (C::HAS_MIN) lo += c2[f][st], hi += c2[f][st];
-                        b[pp] = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{lo, hi}, bf16x2_t));
-                    }
+                } else {  // five bits
+                    uint32_t lo, hi;
+                    wr[CUR][f].bytes(st, lo, hi);
+                    Pk4gBf16 cv;
+                    cv.s = sc, cv.c = C::HAS_MIN ? c2[f][st] : (NEGF + 128.0f) * sc;
+                    b[0] = cv.template bytes<0>(lo), b[1] = cv.template bytes<0>(hi), b[2] = cv.template bytes<1>(lo), b[3] = cv.template bytes<1>(hi);
                 }
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    if constexpr (K16) acc[mt][f] = ggm_mfma16(a[mt][0], a[mt][1], b[0], b[1], acc[mt][f]);
-                    else acc[mt][f] = Ops::mfma(a[mt], b, acc[mt][f]);
-                }
+                for (int mt = 0; mt < MT; ++mt) acc[mt][f] = Ops::mfma(a[mt], b, acc[mt][f]);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1031,11 +1045,11 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         for (int k = 0; k < KS; ++k)  // K order: the same sum whatever the timing
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float4_t v = red[(((k * SPW + ws) * MT + kq) * 4 + e) * 64 + lane];
+                const float4_t v = red[(((k * SPW + ws) * MT + min(kq, MT - 1)) * 4 + e) * 64 + lane];
                 fin[0][0][e] += v[0], fin[0][1][e] += v[1], fin[0][2][e] += v[2], fin[0][3][e] += v[3];
             }
     }
-    if (!live) return;
+    if (!live || (KS > MT && kq >= MT)) return;
     if (act) {
         // Fused gate|up layer (ggm_src_row): strip 4 j + f holds gate columns 8 (4 j + f) .. + 7 in lanes ni < 8 and
         // the up columns they meet in lanes ni + 8.  The two lanes of a pair exchange their four values (row_ror:8)
@@ -1327,7 +1341,8 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
 // `slices` workgroups); ks = -1: the integer kernel in row tiles of 32; 0: the tile matmul on the file layout (gguf_mm).
 //
 // From 2^20 weights the cheapest of these by estimate, in us (fitted on one box to 4096 x 4096, 14336 x 4096, 5120 x
-// 1408, 3072 x 7424, 2048 x 1024, 4096 x 14336 and 4096 x 28672 at 33 - 512 rows in Q4_K, Q6_K and Q8_0):
+// 1408, 3072 x 7424, 2048 x 1024, 4096 x 14336 and 4096 x 28672 at 33 - 512 rows in Q4_K, Q6_K and Q8_0; the five- and six-bit
+// formats' rounds again at 512 and 2048 rows of 4096 x 4096 when their conversion changed):
 //   integer row tiles   2.6 + chunks a wave x `chunk` x rounds of 256 workgroups (four strips each: 2.5 x).  Ahead where the
 //                       tiles fit one round: 2048 x 1024 at 128 rows 9.7 -> 5.3 us, 5120 x 1408 at 64 rows 12.0 -> 10.5
 //   two waves           rounds of workgroups x (4.5 + K rounds of four chunks x `round`), and with K slices a second launch of
@@ -1348,8 +1363,8 @@ static GgmCost ggm_cost(int quant) {
     switch (quant) {
     case OXQ_GGUF_Q4_0: case OXQ_GGUF_Q4_1: case OXQ_GGUF_Q4_K: return {1.45, 2.9, 2.6};
     case OXQ_GGUF_Q8_0: return {1.6, 2.9, 2.9};
-    case OXQ_GGUF_Q6_K: return {1.75, 4.0, 3.75};
-    default: return {1.6, 4.1, 4.0};  // Q5_0, Q5_1, Q5_K
+    case OXQ_GGUF_Q6_K: return {1.75, 3.6, 3.4};
+    default: return {1.6, 3.3, 3.0};  // Q5_0, Q5_1, Q5_K
     }
 }
 static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
@@ -1404,10 +1419,9 @@ bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_
     return gguf_gemm_form(ctx, quant, M, K, N, act_dtype).ks < 0;
 }
 
-template <int FMT, int KS>
+template <int FMT, int MT, int KS>
 static int ggm_gemm_go(hipStream_t s, dim3 grid, const GgufProblem &p, float *part, int NG, int RT, int cslice) {
     static LdsGrant grant;  // one per instantiation
-    constexpr int MT = 4;
     const size_t lds = (size_t)2 * KS * 16 * MT * 256;
     OXQ_HIP_CHECK(grant.ensure((const void *)ggm_gemm_kernel<FMT, MT, KS>, lds));
     hipLaunchKernelGGL((ggm_gemm_kernel<FMT, MT, KS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w, (const uint16_t *)p.bias,
@@ -1417,7 +1431,10 @@ static int ggm_gemm_go(hipStream_t s, dim3 grid, const GgufProblem &p, float *pa
 }
 template <int FMT>
 static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, float *part, int NG, int RT, int ks, int cslice) {
-    return ks == 4 ? ggm_gemm_go<FMT, 4>(s, grid, p, part, NG, RT, cslice) : ggm_gemm_go<FMT, 1>(s, grid, p, part, NG, RT, cslice);
+    if (ks == 1) return ggm_gemm_go<FMT, 4, 1>(s, grid, p, part, NG, RT, cslice);
+    // up to 48 rows: the 64-row tile without its fourth row tile of MFMAs, and of x (14336 x 4096 at 48 rows, us: Q4_K 21.4 ->
+    // 20.3, Q6_K 25.9 -> 24.5, Q8_0 23.3 -> 22.2)
+    return p.M <= 48 ? ggm_gemm_go<FMT, 3, 4>(s, grid, p, part, NG, RT, cslice) : ggm_gemm_go<FMT, 4, 4>(s, grid, p, part, NG, RT, cslice);
 }
 
 // p.w is the matrix-core copy; p.act as for launch_gguf_mfma; p.gate_half: the copy of a fused gate|up layer whose
