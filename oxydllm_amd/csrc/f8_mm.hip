@@ -437,6 +437,12 @@ static bool f8_shape_ok(const F8Problem &p) {
 //   tiles of 32 rows x 16 columns        2.0 + rounds of 256 workgroups x (0.9 + 1.25 x chunks a wave)
 //   tiles of 32 rows x 64 columns        1.4 + rounds x (2.5 + 2.05 x chunks a wave)
 //   tiles of 48 rows x 64 columns        1.4 + rounds x (4.4 + 2.15 x chunks a wave)
+//   tiles of 32 rows x 32 columns        1.4 + rounds x (1.15 + 1.8 x chunks a wave)
+//   tiles of 48 rows x 32 columns        1.4 + rounds x (1.7 + 2.0 x chunks a wave)
+// A workgroup's LDS slots leave room for one a CU, so the tile that just fits one round of CUs is ahead; the two of 32
+// columns stand between the strips and the 64-column groups (fitted over 512..7168 x 768..7168 at 20..320 rows, 1.15 x the fit:
+// ahead at 163 of 480 points, by 1.28 x there, and behind at none).  Us, without them -> with: 3968 x 3456 at 33, 64, 96 rows
+// 13.1 -> 9.8, 13.3 -> 10.1, 15.1 -> 11.4; 5632 x 5632 at 33 rows 15.7 -> 12.1; 1408 x 2048 at 96 rows 6.7 -> 4.9.
 //   64 rows x 128 columns, K over waves  rounds x (7.5 + 2.6 x rounds of four chunks); K slices add a second launch and
 //                                        the partials' traffic
 //   64 rows x 512 columns                rounds x (7 + 2.3 x chunks)
@@ -461,6 +467,9 @@ static F8Form f8_form(const oxq_ctx *ctx, const F8Problem &p) {
     if (p.M <= 16) return best;  // a single row tile is bound by the weights' latency: the most workgroups
     offer(2, 1.4 + std::ceil((double)groups * tiles / cus) * (2.5 + 2.05 * per_wave), {0, 4, 1});
     offer(3, 1.4 + std::ceil((double)groups * (double)ceil_div(p.M, (int64_t)48) / cus) * (4.4 + 2.15 * per_wave), {0, 4, 1, 3});
+    const double pairs = (double)ceil_div(strips, (int64_t)2);
+    offer(5, 1.4 + std::ceil(pairs * tiles / cus) * (1.15 + 1.8 * per_wave), {0, 2, 1, 2});
+    offer(6, 1.4 + std::ceil(pairs * (double)ceil_div(p.M, (int64_t)48) / cus) * (1.7 + 2.0 * per_wave), {0, 2, 1, 3});
     if (p.M <= 32) return best;
     const int64_t rt = ceil_div(p.M, (int64_t)64), wgs = ceil_div(groups, (int64_t)2) * rt;
     const int64_t most = p.N % 4 == 0 ? std::min<int64_t>(ceil_div(chunks, (int64_t)4), 32) : 1;
@@ -513,9 +522,10 @@ int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
         const int mt = form.mt ? form.mt : p.M > 16 ? 2 : 1;
         dim3 grid((unsigned)ceil_div(p.N, (int64_t)16 * form.ns), 1, (unsigned)ceil_div(p.M, (int64_t)16 * mt));
         if (grid.z > 65535) return fail(OXQ_ERR_UNSUPPORTED, "f8 matmul: m = %lld exceeds the grid", (long long)p.M);
-        snprintf(name, sizeof name, "f8_mul_mm_bf16_mt%d%s", mt, form.ns == 4 ? "_n64" : "");
+        snprintf(name, sizeof name, "f8_mul_mm_bf16_mt%d%s", mt, form.ns == 4 ? "_n64" : form.ns == 2 ? "_n32" : "");
         set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
         if (ctx->plan_only) return OXQ_OK;
+        if (form.ns == 2) return mt == 3 ? f8_tile_go<3, 2, 12>(s, grid, p) : f8_tile_go<2, 2, 8>(s, grid, p);
         if (mt == 3) return f8_tile_go<3, 4, 12>(s, grid, p);
         return form.ns == 4 ? f8_tile_rows<4>(s, grid, p) : f8_tile_rows<1>(s, grid, p);
     }

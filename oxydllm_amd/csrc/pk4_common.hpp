@@ -366,7 +366,9 @@ __device__ __forceinline__ void pk4n_epilogue(const float4_t (&acc)[MT][NS], con
         for (int e = 0; e < 4; ++e) {
             float *dst = (float *)(pk4_lds + (size_t)wave * MT * 4096) + ((mt * 4 + e) * 64 + lane) * NS;
             if constexpr (NS == 4) *(float4_t *)dst = float4_t{acc[mt][0][e], acc[mt][1][e], acc[mt][2][e], acc[mt][3][e]};
-            else dst[0] = acc[mt][0][e];
+            else
+#pragma unroll
+                for (int f = 0; f < NS; ++f) dst[f] = acc[mt][f][e];
         }
     __syncthreads();
     for (int t = threadIdx.x; t < ROWS * 16; t += NT) {
@@ -383,7 +385,8 @@ __device__ __forceinline__ void pk4n_epilogue(const float4_t (&acc)[MT][NS], con
                 const float4_t q = *(const float4_t *)src;
                 v[0] += q[0], v[1] += q[1], v[2] += q[2], v[3] += q[3];
             } else {
-                v[0] += src[0];
+#pragma unroll
+                for (int f = 0; f < NS; ++f) v[f] += src[f];
             }
         }
 #pragma unroll
