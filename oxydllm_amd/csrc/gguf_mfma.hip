@@ -27,8 +27,13 @@
 //                 and v_mfma_f32_16x16x16_bf16: step s of the chunk takes elements 16 s + 4 kb .. + 3; their
 //                 nibbles sit in word s / 2 as Q4_0's pairs 2 (s % 2) and 2 (s % 2) + 1, their bit pairs in
 //                 word s / 4 of the second plane, bit ggm_pair_at(2 (s % 4) + pair) of each 16-bit half   3360 B
+//   Q2_K  block = 2 chunks of { [64 lanes][8 B] bit pairs, [16 columns][8] scale bytes } + [16 columns] {d, dmin}.  Steps as
+//                 Q6_K's; pair p of steps 2 t and 2 t + 1 is field 2 (t % 2) + p of the bytes of word t / 2: bytes 0, 1 the
+//                 step of 16 before, 2, 3 the one behind                                                  1344 B
+//   Q3_K  block = 2 chunks of { [64 lanes][8 B] bit pairs as Q2_K, [64 lanes][4 B] third bits (bit 2 t + p of the same byte),
+//                 [16 columns][8] int8 scales } + [16 columns] f16 d (the file packs its six-bit scales)     1824 B
 //
-// Exactly the file's bytes per weight.  The integers stay integers: the MFMA accumulates x * (bias + q) in f32
+// Exactly the file's bytes per weight (Q3_K: 114 for 110).  The integers stay integers: the MFMA accumulates x * (bias + q) in f32
 // (products of 8-bit significands are exact), a second MFMA against the constant -(bias + offset) takes the
 // bias and the format's offset out in the same accumulator, and the unit's scale multiplies the sum once per
 // output, in f32, as the reference's GEMV does (d * sum of q * x, quant_kernels.metal:1097-1221).
@@ -51,10 +56,15 @@ template <> struct GgmFmt<OXQ_GGUF_Q5_1> { static constexpr int WQ = 1, CH = 1, 
 template <> struct GgmFmt<OXQ_GGUF_Q5_K> { static constexpr int WQ = 1, CH = 2, UH = 0, BH = 16; static constexpr uint32_t NEG = 0xC300C300u; };  // -128
 template <> struct GgmFmt<OXQ_GGUF_Q4_K> { static constexpr int WQ = 1, CH = 2, UH = 0, BH = 16; static constexpr uint32_t NEG = 0xC300C300u; };  // -128
 template <> struct GgmFmt<OXQ_GGUF_Q6_K> { static constexpr int WQ = 1, CH = 2, UH = 8, BH = 2; static constexpr uint32_t NEG = 0xC320C320u; };  // -160
+template <> struct GgmFmt<OXQ_GGUF_Q2_K> { static constexpr int WQ = 0, CH = 2, UH = 8, BH = 4; static constexpr uint32_t NEG = 0x3F803F80u; };  // 1: no bias
+template <> struct GgmFmt<OXQ_GGUF_Q3_K> { static constexpr int WQ = 0, CH = 2, UH = 8, BH = 2; static constexpr uint32_t NEG = 0x3F803F80u; };
 
-// formats with a fifth bit; with a minimum beside the scale
+// formats of two and three bits: 16-element scales as Q6_K, no plane of nibbles
+template <int FMT> constexpr bool ggm_narrow = FMT == OXQ_GGUF_Q2_K || FMT == OXQ_GGUF_Q3_K;
+template <int FMT> constexpr bool ggm_k16 = FMT == OXQ_GGUF_Q6_K || ggm_narrow<FMT>;  // a scale covers 16 elements
+// formats with a fifth bit; with a term that multiplies the sum of x: a minimum beside the scale, or Q3_K's offset
 template <int FMT> constexpr bool ggm_fifth_bit = FMT == OXQ_GGUF_Q5_0 || FMT == OXQ_GGUF_Q5_1 || FMT == OXQ_GGUF_Q5_K;
-template <int FMT> constexpr bool ggm_has_min = FMT == OXQ_GGUF_Q4_K || FMT == OXQ_GGUF_Q5_K || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q5_1;
+template <int FMT> constexpr bool ggm_has_min = FMT == OXQ_GGUF_Q4_K || FMT == OXQ_GGUF_Q5_K || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q5_1 || ggm_narrow<FMT>;
 
 // Place in its 16-bit half of the fifth bit of pair pp of unit t, and of the bit pair of field f (Q6_K): pairs 0, 1 of a unit in the
 // low byte, 2, 3 in the high one.
@@ -64,11 +74,11 @@ __device__ constexpr int ggm_pair_at(int f) { return 2 * (2 * (f >> 2) + (f & 1)
 template <int FMT> struct GgmLayout {
     typedef GgmFmt<FMT> F;
     static constexpr int H_OFF = F::WQ * 1024;                                  // Q6_K: the plane of bit pairs; fifth bits
-    static constexpr int UH_OFF = F::WQ * 1024 + (FMT == OXQ_GGUF_Q6_K ? 512 : ggm_fifth_bit<FMT> ? 256 : 0);
+    static constexpr int UH_OFF = F::WQ * 1024 + (ggm_k16<FMT> ? 512 : 0) + (ggm_fifth_bit<FMT> || FMT == OXQ_GGUF_Q3_K ? 256 : 0);
     static constexpr int CHB = UH_OFF + 16 * F::UH;
     static constexpr int BH_OFF = F::CH * CHB;
     static constexpr int BLKB = F::CH * CHB + 16 * F::BH;
-    static_assert(BLKB == 16 * (128 * F::CH / GgufFmt<FMT>::BE) * GgufFmt<FMT>::BB, "the copy has the file's size");
+    static_assert(BLKB == 16 * (128 * F::CH / GgufFmt<FMT>::BE) * (GgufFmt<FMT>::BB + (FMT == OXQ_GGUF_Q3_K ? 4 : 0)), "the copy has the file's size");
 };
 
 // ---------------------------------------------------------------------------
@@ -97,7 +107,8 @@ __global__ __launch_bounds__(256) void ggm_repack_kernel(const uint8_t *__restri
         uint8_t *zb = pw + ((size_t)strip * (nch / F::CH) + c / F::CH) * L::BLKB, *zc = zb + (c % F::CH) * L::CHB;
 #pragma unroll
         for (int pl = 0; pl < F::WQ; ++pl) *(u32x4_t *)(zc + pl * 1024 + lane * 16) = u32x4_t{0u, 0u, 0u, 0u};
-        if constexpr (FMT == OXQ_GGUF_Q6_K) *(uint2 *)(zc + L::H_OFF + lane * 8) = uint2{0u, 0u};
+        if constexpr (ggm_k16<FMT>) *(uint2 *)(zc + L::H_OFF + lane * 8) = uint2{0u, 0u};
+        if constexpr (FMT == OXQ_GGUF_Q3_K) *(uint32_t *)(zc + 512 + lane * 4) = 0u;
         if constexpr (ggm_fifth_bit<FMT>) *(uint32_t *)(zc + L::H_OFF + lane * 4) = 0u;
         for (int b = kb; b < F::UH; b += 4) zc[L::UH_OFF + ni * F::UH + b] = 0;
         if (c % F::CH == 0)
@@ -212,6 +223,33 @@ __global__ __launch_bounds__(256) void ggm_repack_kernel(const uint8_t *__restri
         *(uint2 *)(chunk + L::H_OFF + lane * 8) = uint2{hw[0], hw[1]};
         if (kb < 2) *(uint32_t *)(chunk + L::UH_OFF + ni * 8 + kb * 4) = ld32a2(p + 192 + 8 * h + 4 * kb);
         if (h == 0 && kb == 0) *(uint16_t *)(blk + L::BH_OFF + ni * 2) = ld16(p + 208);
+    } else if constexpr (ggm_narrow<FMT>) {
+        // quant_kernels.metal:2556-2680: element j of the super-block, h = j / 128, q = (j % 128) / 32, l = j % 32: bit pair
+        // 2 q of qs[32 h + l]; Q3_K's third bit is bit 4 h + q of hmask[l]
+        constexpr bool THREE = FMT == OXQ_GGUF_Q3_K;
+        const uint8_t *p = row + (size_t)(c >> 1) * GgufFmt<FMT>::BB;
+        const int h = c & 1;
+        const uint8_t *qs = p + (THREE ? 32 : 16) + 32 * h;
+        uint32_t w2[2] = {0u, 0u}, w3 = 0u;
+#pragma unroll
+        for (int s2 = 0; s2 < 8; ++s2)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int jj = 16 * s2 + 4 * kb + i, qq = jj >> 5, l = jj & 31;
+                const int t = s2 >> 1, pr = i >> 1, byte = 2 * (s2 & 1) + (i & 1);
+                w2[t >> 1] |= (((uint32_t)qs[l] >> (2 * qq)) & 3u) << (8 * byte + 4 * (t & 1) + 2 * pr);
+                if constexpr (THREE) w3 |= (((uint32_t)p[l] >> (4 * h + qq)) & 1u) << (8 * byte + 2 * t + pr);
+            }
+        *(uint2 *)(chunk + lane * 8) = uint2{w2[0], w2[1]};
+        if constexpr (THREE) *(uint32_t *)(chunk + 512 + lane * 4) = w3;
+        // two scales of the chunk's eight a lane group
+#pragma unroll
+        for (int b = 2 * kb; b < 2 * kb + 2; ++b)
+            chunk[L::UH_OFF + ni * 8 + b] = THREE ? (uint8_t)(int8_t)q3k_scale(p + 96, 8 * h + b) : p[8 * h + b];
+        if (h == 0 && kb == 0) {
+            if constexpr (THREE) *(uint16_t *)(blk + L::BH_OFF + ni * 2) = ld16(p + 108);
+            else *(uint32_t *)(blk + L::BH_OFF + ni * 4) = ld16(p + 80) | (ld16(p + 82) << 16);
+        }
     }
 }
 
@@ -327,12 +365,12 @@ __device__ __forceinline__ float ggm_f16(uint32_t bits) { return (float)__builti
 template <int FMT> struct GgmChunk {
     typedef GgmFmt<FMT> F;
     typedef GgmLayout<FMT> L;
-    static constexpr int NSTEP = FMT == OXQ_GGUF_Q6_K ? 8 : 4;
+    static constexpr int NSTEP = ggm_k16<FMT> ? 8 : 4;
     static constexpr bool HAS_MIN = ggm_has_min<FMT>;
     // vector loads of one request()
-    static constexpr int LOADS = (F::UH ? 1 : 0) + (F::BH ? 1 : 0) + F::WQ + ((FMT == OXQ_GGUF_Q6_K || ggm_fifth_bit<FMT>) ? 1 : 0);
-    u32x4_t q[F::WQ];
-    uint32_t qh[FMT == OXQ_GGUF_Q6_K ? 2 : 1];
+    static constexpr int LOADS = (F::UH ? 1 : 0) + (F::BH ? 1 : 0) + F::WQ + ((ggm_k16<FMT> || ggm_fifth_bit<FMT>) ? 1 : 0) + (FMT == OXQ_GGUF_Q3_K ? 1 : 0);
+    u32x4_t q[F::WQ ? F::WQ : 1];
+    uint32_t qh[FMT == OXQ_GGUF_Q3_K ? 3 : ggm_k16<FMT> ? 2 : 1];  // Q2_K, Q3_K: two words of bit pairs, one of third bits
     uint32_t uh[F::UH == 16 ? 4 : F::UH ? 2 : 1];   // unit headers of the column: four f16 d or {d, m} pairs, eight int8 scales (Q6_K)
     uint32_t bh[F::BH == 16 ? 4 : 1];  // block header of the column
 
@@ -353,12 +391,15 @@ template <int FMT> struct GgmChunk {
             bh[0] = v[0], bh[1] = v[1], bh[2] = v[2], bh[3] = v[3];
         } else if constexpr (F::BH == 2) {
             bh[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (ni >> 1) * 4, blk + L::BH_OFF, 0);
+        } else if constexpr (F::BH == 4) {
+            bh[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, ni * 4, blk + L::BH_OFF, 0);
         }
 #pragma unroll
         for (int pl = 0; pl < F::WQ; ++pl) q[pl] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, soff + pl * 1024, 2);
-        if constexpr (FMT == OXQ_GGUF_Q6_K) {
+        if constexpr (ggm_k16<FMT>) {
             const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rs, lane * 8, soff + L::H_OFF, 2);
             qh[0] = v[0], qh[1] = v[1];
+            if constexpr (FMT == OXQ_GGUF_Q3_K) qh[2] = __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4, soff + 512, 2);
         } else if constexpr (ggm_fifth_bit<FMT>) {
             qh[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4, soff + L::H_OFF, 2);
         }
@@ -382,6 +423,17 @@ template <int FMT> struct GgmChunk {
             const float d = ggm_f16((ni & 1) ? (bh[0] >> 16) : (bh[0] & 0xFFFFu));
 #pragma unroll
             for (int st = 0; st < 8; ++st) f0[st] = d * (float)(int)(int8_t)((uh[st >> 2] >> (8 * (st & 3))) & 0xFFu), f1[st] = 0.f;
+        } else if constexpr (FMT == OXQ_GGUF_Q3_K) {  // w = f0 (q + 4) - 4 f0
+            const float d = ggm_f16((ni & 1) ? (bh[0] >> 16) : (bh[0] & 0xFFFFu));
+#pragma unroll
+            for (int st = 0; st < 8; ++st) f0[st] = d * (float)(int)(int8_t)((uh[st >> 2] >> (8 * (st & 3))) & 0xFFu), f1[st] = f0[st] * 0.03125f;
+        } else if constexpr (FMT == OXQ_GGUF_Q2_K) {
+            const float d = ggm_f16(bh[0] & 0xFFFFu), dm = ggm_f16(bh[0] >> 16) * 0.0078125f;  // dmin / 128
+#pragma unroll
+            for (int st = 0; st < 8; ++st) {
+                f0[st] = d * (float)((uh[st >> 2] >> (8 * (st & 3))) & 0xFu);
+                f1[st] = dm * (float)((uh[st >> 2] >> (8 * (st & 3) + 4)) & 0xFu);
+            }
         } else if constexpr (F::UH == 16) {  // w = d q + m: the minimum times sum(x) = -m / 128 times the bias term
 #pragma unroll
             for (int st = 0; st < 4; ++st) f0[st] = ggm_f16(uh[st] & 0xFFFFu), f1[st] = ggm_f16(uh[st] >> 16) * -0.0078125f;
@@ -398,6 +450,15 @@ template <int FMT> struct GgmChunk {
         auto moved = [&](int a) { return a < 4 ? h << (4 - a) : h >> (a - 4); };
         lo = (moved(at) & MASK) | (w & 0x0F0F0F0Fu), hi = (moved(at + next) & MASK) | ((w >> 4) & 0x0F0F0F0Fu);
     }
+    // Q2_K, Q3_K: the unsigned integers of 32 elements, a byte each: lo pair 0, hi pair 1; bytes 0, 1 of step 2 st, 2, 3 of 2 st + 1
+    __device__ __forceinline__ void bytes2(int st, uint32_t &lo, uint32_t &hi) const {
+        const uint32_t w = qh[st >> 1] >> (4 * (st & 1));
+        lo = w & 0x03030303u, hi = (w >> 2) & 0x03030303u;
+        if constexpr (FMT == OXQ_GGUF_Q3_K) {
+            auto third = [&](int at) { return (at < 2 ? qh[2] << (2 - at) : qh[2] >> (at - 2)) & 0x04040404u; };
+            lo |= third(2 * st), hi |= third(2 * st + 1);
+        }
+    }
     // B operand of step st: bias + q as bf16 pairs (four for a step of 32 elements, two for one of 16)
     __device__ __forceinline__ void operand(int st, uint32_t (&b)[4], const NibbleMasks &nm) const {
         if constexpr (FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_K || FMT == OXQ_GGUF_Q4_1) {
@@ -413,6 +474,14 @@ template <int FMT> struct GgmChunk {
         } else if constexpr (FMT == OXQ_GGUF_Q8_0) {
             const uint32_t w0 = q[st >> 1][2 * (st & 1)], w1 = q[st >> 1][2 * (st & 1) + 1];
             b[0] = ggm_bytes02(w0), b[1] = ggm_bytes13(w0), b[2] = ggm_bytes02(w1), b[3] = ggm_bytes13(w1);
+        } else if constexpr (ggm_narrow<FMT>) {  // 0 .. 7 as f8 codes (512ths): no bias
+            uint32_t lo, hi;
+            bytes2(st >> 1, lo, hi);
+            b[0] = __builtin_bit_cast(uint32_t, (st & 1) ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true)
+                                                         : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false));
+            b[1] = __builtin_bit_cast(uint32_t, (st & 1) ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true)
+                                                         : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
+            b[2] = b[3] = 0u;
         } else {  // Q6_K: nibble | bit pair << 4, 128 + (0 .. 63) is exact in bf16
             const uint32_t lw = q[0][st >> 1], hw = qh[st >> 2];
 #pragma unroll
@@ -438,7 +507,7 @@ template <int FMT> struct GgmChunk {
 // formats the offset or the subtracted minimum makes it NaN there and here).  Widened through f32 Q4_1 took up to 1.25 x as
 // long; Q5_1 at 3 - 16 rows is at 1.03 - 1.13 x the biased operand's time.
 template <int FMT> struct GgmSmallBias {
-    static constexpr bool PLAIN = FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q5_1;
+    static constexpr bool PLAIN = FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q5_1 || ggm_narrow<FMT>;
     static constexpr bool FOURS = FMT == OXQ_GGUF_Q4_1;  // pair i of the operand holds elements i and i + 4, else 2 i and 2 i + 1
     static constexpr bool NIB = FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q4_K;
     static constexpr float BIAS = NIB ? 16.f : ggm_fifth_bit<FMT> ? 32.f : FMT == OXQ_GGUF_Q6_K ? 64.f : 0.f;
@@ -456,7 +525,7 @@ template <int FMT> struct GgmSmallBias {
             b[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
             b[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
             b[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
-        } else if constexpr (PLAIN) {  // bytes 0, 2 hold pair 0 or 1, bytes 1, 3 pair 2 or 3
+        } else if constexpr (PLAIN && !ggm_narrow<FMT>) {  // bytes 0, 2 hold pair 0 or 1, bytes 1, 3 pair 2 or 3
             uint32_t lo, hi;
             w.bytes(st, lo, hi);
             b[0] = ggm_bytes02(lo), b[1] = ggm_bytes02(hi), b[2] = ggm_bytes13(lo), b[3] = ggm_bytes13(hi);
@@ -691,11 +760,11 @@ __global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict
 #pragma unroll
         for (int f = 0; f < NS; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
     constexpr bool FOURS = XF32 && GgmSmallBias<FMT>::FOURS;
-    constexpr bool PLAIN = XF32 && GgmSmallBias<FMT>::PLAIN;  // the integers without a bias: their sums start from zero
+    constexpr bool PLAIN = (XF32 || ggm_narrow<FMT>) && GgmSmallBias<FMT>::PLAIN;  // the integers without a bias: their sums start from zero
     constexpr uint32_t NEGP = XF32 ? GgmSmallBias<FMT>::NEG_PAIR : F::NEG;
     const uint32_t neg[4] = {NEGP, NEGP, NEGP, NEGP};
     // the minimum's factor is per 128 (factors()); here the bias term is smaller
-    constexpr float MINF = XF32 && C::HAS_MIN ? 128.0f / -GgmSmallBias<FMT>::NEG : 1.0f;
+    constexpr float MINF = (XF32 || ggm_narrow<FMT>) && C::HAS_MIN ? 128.0f / -GgmSmallBias<FMT>::NEG : 1.0f;
     auto operand = [&](const C &w, int st, uint32_t (&b)[4], const NibbleMasks &k) {
         if constexpr (XF32) GgmSmallBias<FMT>::operand(w, st, b, k);
         else w.operand(st, b, k);
@@ -974,7 +1043,14 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
             for (int f = 0; f < 4; ++f) {
                 uint32_t b[4];
                 const float sc = f0[f][st];
-                if constexpr (K16) {
+                if constexpr (ggm_narrow<FMT>) {
+                    uint32_t lo, hi;
+                    wr[CUR][f].bytes2(st, lo, hi);
+                    float ql[4], qu[4];
+                    pk4g_widen(lo, ql), pk4g_widen(hi, qu);
+                    const Pk4gBf16 c0 = {f0[f][2 * st], c2[f][2 * st]}, c1 = {f0[f][2 * st + 1], c2[f][2 * st + 1]};
+                    b[0] = c0.pair(ql[0], ql[1]), b[1] = c0.pair(qu[0], qu[1]), b[2] = c1.pair(ql[2], ql[3]), b[3] = c1.pair(qu[2], qu[3]);
+                } else if constexpr (K16) {
                     uint32_t lo, hi;
                     wr[CUR][f].bytes(st, lo, hi);
                     Pk4gBf16 c0, c1;
@@ -1126,6 +1202,7 @@ static bool ggm_format(int quant) {
     return quant == OXQ_GGUF_Q4_0 || quant == OXQ_GGUF_Q8_0 || quant == OXQ_GGUF_Q4_K || quant == OXQ_GGUF_Q6_K ||
            quant == OXQ_GGUF_Q4_1 || quant == OXQ_GGUF_Q5_0 || quant == OXQ_GGUF_Q5_1 || quant == OXQ_GGUF_Q5_K;
 }
+static bool ggm_narrow_format(int quant) { return quant == OXQ_GGUF_Q2_K || quant == OXQ_GGUF_Q3_K; }
 static const char *ggm_name(int q) {
     switch (q) {
     case OXQ_GGUF_Q4_0: return "q4_0";
@@ -1135,6 +1212,8 @@ static const char *ggm_name(int q) {
     case OXQ_GGUF_Q5_0: return "q5_0";
     case OXQ_GGUF_Q5_1: return "q5_1";
     case OXQ_GGUF_Q5_K: return "q5k";
+    case OXQ_GGUF_Q2_K: return "q2k";
+    case OXQ_GGUF_Q3_K: return "q3k";
     default: return "q6k";
     }
 }
@@ -1148,12 +1227,18 @@ bool gguf_mfma_eligible(const oxq_ctx *ctx, int quant, int64_t K, int64_t N) {
 }
 // Whether a layer of these activations holds the matrix-core copy.  bf16: always where it exists.  f32: from 2^20
 // weights, beside the rotated copy of the vector GEMV; on smaller layers that one takes a launch's time.
+// Q2_K and Q3_K layers hold it beside the rotated copy, which stays ahead at one row and on smaller layers.
 bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int act_dtype) {
+    if (ggm_narrow_format(quant))
+        return tune(ctx, OXQ_TUNE_GGUF_MFMA, 1) != 0 && N * K >= (1 << 20) && gguf_res_eligible(quant, K, N) &&
+               (act_dtype == OXQ_BF16 || act_dtype == OXQ_F32);
     return gguf_mfma_eligible(ctx, quant, K, N) && (act_dtype == OXQ_BF16 || (act_dtype == OXQ_F32 && N * K >= (1 << 20)));
 }
 // Whether such a layer does without the rotated copy: bf16, and f32 where OXQ_GGUF_MFMA is 2 (one copy fewer; what one and two
 // rows then take stands below: up to 8 % more on layers of one round of strips).
-bool gguf_mfma_alone(const oxq_ctx *ctx, int act_dtype) { return act_dtype == OXQ_BF16 || tune(ctx, OXQ_TUNE_GGUF_MFMA, 1) == 2; }
+bool gguf_mfma_alone(const oxq_ctx *ctx, int quant, int act_dtype) {
+    return !ggm_narrow_format(quant) && (act_dtype == OXQ_BF16 || tune(ctx, OXQ_TUNE_GGUF_MFMA, 1) == 2);
+}
 // f32 rows of a layer that has both copies: the vector GEMV's arithmetic grows with the rows and is slow on many short
 // strips; the matrix cores take four rows as one.  us on the rotated / the matrix-core copy, Q4_K, 1 / 2 / 4 / 8 rows:
 // 4096 x 4096 4.2 / 5.0 / 6.5 / 12.7 against 4.5 / 5.2 / 5.5 / 7.8, 14336 x 4096 10.7 / 13.3 / 17.8 / 35.2 against 10.0 / 11.7 /
@@ -1162,7 +1247,18 @@ bool gguf_f32_on_mfma(const oxq_ctx *ctx, int64_t M, int64_t K, int64_t N) {
     const bool many = ceil_div(N, (int64_t)16) > (ctx->num_cus > 0 ? ctx->num_cus : 256);
     return M >= 3 || (M == 2 ? many || K >= 8192 : many && K <= 2048);
 }
-size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N) { return gguf_res_bytes(quant, K, (N + 15) & ~(int64_t)15); }
+// Rows of a layer that holds both copies: whether they run on the matrix-core one.  Q2_K and Q3_K, us on the rotated / the
+// matrix-core copy: 4096 x 4096 bf16 3 rows 6.7 / 5.2, 2 rows 5.0 / 5.2 (Q3_K 5.6 / 5.4), 1024 x 5056 2 rows 7.2 / 3.8, 14336 x 4096
+// 13.4 / 11.8; f32 3 rows 6.5 / 6.5, 18.2 / 15.9 at 14336 x 4096, 8 rows 12.8 / 9.6, 36 / 26, but 2 rows 12.6 / 15.9.
+bool gguf_rows_on_mfma(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
+    const bool many = ceil_div(N, (int64_t)16) > (ctx->num_cus > 0 ? ctx->num_cus : 256);
+    if (ggm_narrow_format(quant)) return act_dtype == OXQ_BF16 ? M >= 3 || (M == 2 && (many || quant == OXQ_GGUF_Q3_K)) : M >= 3 && M <= 8;
+    return act_dtype == OXQ_BF16 || gguf_f32_on_mfma(ctx, M, K, N);
+}
+size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N) {
+    if (quant == OXQ_GGUF_Q3_K) return (size_t)N * (size_t)(K / 256) * 114;  // its scales are a byte each
+    return gguf_res_bytes(quant, K, (N + 15) & ~(int64_t)15);
+}
 
 int launch_gguf_mfma_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_t *w, void *pw, int64_t K, int64_t N,
                             int64_t gate_half) {
@@ -1181,6 +1277,8 @@ int launch_gguf_mfma_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_
     case OXQ_GGUF_Q5_0: hipLaunchKernelGGL((ggm_repack_kernel<OXQ_GGUF_Q5_0>), grid, block, 0, s, w, (uint8_t *)pw, (int)K, (int)N, (int)gate_half); break;
     case OXQ_GGUF_Q5_1: hipLaunchKernelGGL((ggm_repack_kernel<OXQ_GGUF_Q5_1>), grid, block, 0, s, w, (uint8_t *)pw, (int)K, (int)N, (int)gate_half); break;
     case OXQ_GGUF_Q5_K: hipLaunchKernelGGL((ggm_repack_kernel<OXQ_GGUF_Q5_K>), grid, block, 0, s, w, (uint8_t *)pw, (int)K, (int)N, (int)gate_half); break;
+    case OXQ_GGUF_Q2_K: hipLaunchKernelGGL((ggm_repack_kernel<OXQ_GGUF_Q2_K>), grid, block, 0, s, w, (uint8_t *)pw, (int)K, (int)N, (int)gate_half); break;
+    case OXQ_GGUF_Q3_K: hipLaunchKernelGGL((ggm_repack_kernel<OXQ_GGUF_Q3_K>), grid, block, 0, s, w, (uint8_t *)pw, (int)K, (int)N, (int)gate_half); break;
     default: return fail(OXQ_ERR_UNSUPPORTED, "gguf repack: format %d has no matrix-core layout", quant);
     }
     OXQ_HIP_CHECK(hipGetLastError());
@@ -1232,16 +1330,26 @@ static int ggm_f32_go(hipStream_t s, dim3 grid, const GgufProblem &p, int cslice
 }
 template <int FMT>
 static int ggm_f32_by_shape(hipStream_t s, dim3 grid, const GgufProblem &p, int cslice, int mt, int ns) {
+    if constexpr (ggm_narrow<FMT>) {
+        if (ns == 4) return mt == 2 ? ggm_f32_go<FMT, 2, 4, 8, 4>(s, grid, p, cslice) : ggm_f32_go<FMT, 1, 2, 8, 4>(s, grid, p, cslice);
+        return mt == 2 ? ggm_f32_go<FMT, 2, 4, 8, 1>(s, grid, p, cslice) : ggm_f32_go<FMT, 1, 2, 8, 1>(s, grid, p, cslice);
+    } else {
     if (ns == 4) {
         if (p.M == 1) return ggm_f32_go<FMT, 1, 1, 8, 4>(s, grid, p, cslice);
         return mt == 2 ? ggm_f32_go<FMT, 2, 4, 8, 4>(s, grid, p, cslice) : ggm_f32_go<FMT, 1, 2, 8, 4>(s, grid, p, cslice);
     }
     if (mt == 2) return ggm_f32_go<FMT, 2, 4, 8, 1>(s, grid, p, cslice);
     return p.M == 1 ? ggm_f32_go<FMT, 1, 1, 8, 1>(s, grid, p, cslice) : ggm_f32_go<FMT, 1, 2, 8, 1>(s, grid, p, cslice);
+    }
 }
 
 template <int FMT>
 static int ggm_by_shape(hipStream_t s, dim3 grid, const GgufProblem &p, float *ws, int cslice, int mt, int xq, int nw, int ns) {
+    if constexpr (ggm_narrow<FMT>) {  // 2 - 8 rows (gguf_mfma_takes)
+        if (ns == 4) return xq == 1 ? ggm_go<FMT, 1, 1, 8, 4>(s, grid, p, ws, cslice) : ggm_go<FMT, 1, 2, 8, 4>(s, grid, p, ws, cslice);
+        if (nw == 8) return xq == 1 ? ggm_go<FMT, 1, 1, 8, 1>(s, grid, p, ws, cslice) : ggm_go<FMT, 1, 2, 8, 1>(s, grid, p, ws, cslice);
+        return xq == 1 ? ggm_go<FMT, 1, 1, 16, 1>(s, grid, p, ws, cslice) : ggm_go<FMT, 1, 2, 16, 1>(s, grid, p, ws, cslice);
+    } else {
     if (ns == 4) {  // 8 waves: four strips' quants in flight take the registers of two waves of a 16-wave workgroup
         if (mt == 2) return ggm_go<FMT, 2, 8, 8, 4>(s, grid, p, ws, cslice);
         if (xq == 1) return ggm_go<FMT, 1, 1, 8, 4>(s, grid, p, ws, cslice);
@@ -1257,6 +1365,7 @@ static int ggm_by_shape(hipStream_t s, dim3 grid, const GgufProblem &p, float *w
     if (xq == 1) return ggm_go<FMT, 1, 1, 16, 1>(s, grid, p, ws, cslice);
     if (xq == 2) return ggm_go<FMT, 1, 2, 16, 1>(s, grid, p, ws, cslice);
     return ggm_go<FMT, 1, 4, 16, 1>(s, grid, p, ws, cslice);
+    }
 }
 
 // A wide layer (768 strips or more) gives a workgroup four neighbouring strips: every strip of a workgroup re-reads
@@ -1270,7 +1379,10 @@ static int ggm_strips(const oxq_ctx *ctx, int64_t N) {
 }
 
 // rows of x a launch of the matrix-core kernel takes (more go to the tile matmul on the file layout)
-bool gguf_mfma_takes(const oxq_ctx *ctx, int64_t M, int64_t, int act_dtype) {
+bool gguf_mfma_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t, int act_dtype) {
+    // the decode range, whose weights stay unrounded; more rows go to the prefill kernel, whose rounded weights the tile
+    // matmul on the file layout has
+    if (ggm_narrow_format(quant)) return M >= 1 && M <= 8;
     if (act_dtype == OXQ_F32) return M >= 1;  // row tiles of eight: there is no other kernel for more f32 rows
     return act_dtype == OXQ_BF16 && M >= 1 && M <= tune(ctx, OXQ_TUNE_GGUF_MFMA_MAX_M, 32);
 }
@@ -1315,6 +1427,8 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     set_plan(ctx, name, grid, dim3(nw * 64), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if (!f32 && p.act_dtype != OXQ_BF16) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: activations must be BF16 or F32");
+    if (ggm_narrow_format(p.quant) && (p.act || !gguf_mfma_takes(ctx, p.quant, p.M, p.N, p.act_dtype)))
+        return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: %s takes up to 8 rows", ggm_name(p.quant));
     if (f32 && p.act) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: a fused activation needs BF16");
     if ((uintptr_t)p.x & 15) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: x must be 16-byte aligned");
     if ((uint64_t)16 * mt * (uint64_t)p.K * 2 >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: K too large");
@@ -1331,6 +1445,8 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
         OXQ_GGM(OXQ_GGUF_Q5_0);
         OXQ_GGM(OXQ_GGUF_Q5_1);
         OXQ_GGM(OXQ_GGUF_Q5_K);
+        OXQ_GGM(OXQ_GGUF_Q2_K);
+        OXQ_GGM(OXQ_GGUF_Q3_K);
     default: return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: format %d", p.quant);
     }
 #undef OXQ_GGM
@@ -1349,8 +1465,13 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
 //                       3.5 us + the partials' bytes at 4.2 TB/s.  14336 x 4096 Q4_K at 33 / 128 / 256 rows 31.8 / 57.8 / 86 ->
 //                       20.9 / 30.7 / 53 us (7, 4 and 2 slices), 4096 x 14336 at 64 rows 28.5 -> 23.5 (2 slices)
 //   eight waves         rounds of workgroups (a last one on at most three quarters of the CUs 0.95) x chunks x `wide` + 5
-// The file layout's matmul is not ahead of all of these there.  Smaller layers compare it with the unsliced forms only, in
-// rounds of 256 workgroups of 64 rows x 512 columns: 0.17 + 1.45 w (1.3 w for the five- and six-bit formats).
+// The file layout's matmul is not ahead of all of these there.  It is for some calls of Q2_K and Q3_K, whose 9 - 32 rows come
+// here too: where it has 400 tiles of 64 x 64 and more it runs at 400 T/s (Q3_K 15 % less) behind 6 us; with fewer it is ahead
+// where K or the layer is short (Q2_K, us, file layout / here: 1024 x 5056 at 16 rows 6.9 / 8.8, 4096 x 1024 6.9 / 8.1, 2816 x
+// 6528 10.7 / 11.1; elsewhere 4096 x 4096 at 16, 48, 101, 512 rows 10.0 / 9.2, 15.5 / 13.0, 24 / 17.6, 46 / 32,
+// 14336 x 4096 23 / 16, 38 / 22, 68 / 33, 149 / 99, 9984 x 21056 at 16 rows 61 / 42, Q3_K 79 / 42).
+// Smaller layers compare it with the unsliced forms only, in rounds of 256 workgroups of 64 rows x 512 columns: 0.17 + 1.45 w
+// (1.3 w for the five- and six-bit formats).
 // OXQ_GGUF_GEMM_MIN_M: unset = by cost, 0 = never, n = the eight-wave form from n rows on whatever the cost;
 // OXQ_GGUF_GEMM_KS = 4 | 1: always | never the two-wave form; OXQ_GGUF_GEMM_SLICES = n: that many slices of it.
 struct GgmGemmForm {
@@ -1364,12 +1485,14 @@ static GgmCost ggm_cost(int quant) {
     case OXQ_GGUF_Q4_0: case OXQ_GGUF_Q4_1: case OXQ_GGUF_Q4_K: return {1.45, 2.9, 2.6};
     case OXQ_GGUF_Q8_0: return {1.6, 2.9, 2.9};
     case OXQ_GGUF_Q6_K: return {1.75, 3.6, 3.4};
+    case OXQ_GGUF_Q2_K: case OXQ_GGUF_Q3_K: return {0.0, 3.5, 3.2};  // `round`: of 64 rows, below of fewer
     default: return {1.6, 3.3, 3.0};  // Q5_0, Q5_1, Q5_K
     }
 }
 static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
     const int64_t v = tune(ctx, OXQ_TUNE_GGUF_GEMM_MIN_M, -1);
-    if (v == 0 || act_dtype != OXQ_BF16 || !ggm_format(quant) || M <= 32) return {0, 1};
+    const bool narrow = ggm_narrow_format(quant);
+    if (v == 0 || act_dtype != OXQ_BF16 || !(narrow ? M > 8 : ggm_format(quant) && M > 32)) return {0, 1};
     const int ks = tune(ctx, OXQ_TUNE_GGUF_GEMM_KS, 0);
     if (ks == 4) return {N % 64 == 0 ? 4 : 0, 1};
     if (v > 0) return {N % 64 == 0 && M >= v ? 1 : 0, 1};
@@ -1377,7 +1500,7 @@ static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int6
     const int64_t row_tiles = ceil_div(M, (int64_t)64), groups = ceil_div(N, (int64_t)64), chunks = K / 128;
     const double w64 = (double)(ceil_div(groups, (int64_t)8) * row_tiles) / cus;
     const double whole = std::floor(w64), rest = w64 - whole;
-    const double r64 = whole + (rest <= 0.0 ? 0.0 : rest <= 0.75 ? 0.95 : 1.0);
+    double r64 = whole + (rest <= 0.0 ? 0.0 : rest <= 0.75 ? 0.95 : 1.0);
     const int64_t mid_wgs = ceil_div(groups, (int64_t)2) * row_tiles;
     if (N * K < (1 << 20)) {
         if (N % 64 != 0) return {0, 1};
@@ -1388,7 +1511,9 @@ static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int6
         if (c_file <= std::min(r64, c_mid)) return {0, 1};
         return {c_mid < r64 ? 4 : 1, 1};
     }
-    const GgmCost c = ggm_cost(quant);
+    GgmCost c = ggm_cost(quant);
+    if (narrow) r64 = std::ceil((double)((row_tiles / 8) * ceil_div(groups, (int64_t)64) * 64 + (row_tiles % 8) * ceil_div(groups, (int64_t)8)) / cus);
+    if (narrow && M <= 48) c.round = M <= 16 ? 2.2 : M <= 32 ? 2.7 : 3.1;
     GgmGemmForm best = {1, 1};
     double least = r64 * ((double)chunks * c.wide + 5.0);
     if (ks != 1) {
@@ -1402,6 +1527,16 @@ static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int6
             if (S > 1) t += 3.5 + ((double)S * 8.0 + 2.0) * (double)M * (double)N / 4.2e6;
             if (t < least || given > 0) least = given > 0 ? 0.0 : t, best = {4, (int)S};
         }
+    }
+    if (narrow) {
+        if (v > 0 || ks || tune(ctx, OXQ_TUNE_GGUF_GEMM_SLICES, 0) > 0) return best;
+        const int64_t size = N * K;
+        const double file = 6.0 + (double)(row_tiles * 64) * (double)size / 2e8 * (quant == OXQ_GGUF_Q3_K ? 1.15 : 1.0) * (M <= 16 ? 0.55 : M <= 32 ? 0.67 : 1.0);
+        bool ahead;
+        if (row_tiles * groups >= 400) ahead = 1.15 * least < file;
+        else if (M > 64) ahead = size >= (M > 128 ? 1 << 22 : 1 << 23);
+        else ahead = K >= 3072 && (size >= 1 << 24 || (size >= 1 << 23 && (K >= 7168 || M > 32)));
+        return ahead ? best : GgmGemmForm{0, 1};
     }
     const int ns = ggm_strips(ctx, N);
     const double int_wgs = (double)(ceil_div(N, (int64_t)16 * ns) * ceil_div(M, (int64_t)32));
@@ -1434,6 +1569,10 @@ static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, floa
     if (ks == 1) return ggm_gemm_go<FMT, 4, 1>(s, grid, p, part, NG, RT, cslice);
     // up to 48 rows: the 64-row tile without its fourth row tile of MFMAs, and of x (14336 x 4096 at 48 rows, us: Q4_K 21.4 ->
     // 20.3, Q6_K 25.9 -> 24.5, Q8_0 23.3 -> 22.2)
+    if constexpr (ggm_narrow<FMT>) {
+        if (p.M <= 16) return ggm_gemm_go<FMT, 1, 4>(s, grid, p, part, NG, RT, cslice);
+        if (p.M <= 32) return ggm_gemm_go<FMT, 2, 4>(s, grid, p, part, NG, RT, cslice);
+    }
     return p.M <= 48 ? ggm_gemm_go<FMT, 3, 4>(s, grid, p, part, NG, RT, cslice) : ggm_gemm_go<FMT, 4, 4>(s, grid, p, part, NG, RT, cslice);
 }
 
@@ -1478,6 +1617,8 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
         OXQ_GGM(OXQ_GGUF_Q5_0);
         OXQ_GGM(OXQ_GGUF_Q5_1);
         OXQ_GGM(OXQ_GGUF_Q5_K);
+        OXQ_GGM(OXQ_GGUF_Q2_K);
+        OXQ_GGM(OXQ_GGUF_Q3_K);
     default: return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: format %d has no matrix-core layout", p.quant);
     }
 #undef OXQ_GGM

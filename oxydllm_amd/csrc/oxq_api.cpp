@@ -844,12 +844,12 @@ static bool wcache_forward(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p, i
 static bool wcache_forward_gguf(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, int *rc) {
     if (!ctx->wcache_limit || ctx->plan_only) return false;
     const bool rotated = gguf_res_eligible(p.quant, p.K, p.N);
-    const bool mfma = gguf_mfma_layer(ctx, p.quant, p.K, p.N, p.act_dtype) &&
-                      (gguf_mfma_alone(ctx, p.act_dtype) || !rotated || gguf_f32_on_mfma(ctx, p.M, p.K, p.N));
+    const bool mfma = p.quant != OXQ_GGUF_Q2_K && p.quant != OXQ_GGUF_Q3_K && gguf_mfma_layer(ctx, p.quant, p.K, p.N, p.act_dtype) &&
+                      (gguf_mfma_alone(ctx, p.quant, p.act_dtype) || !rotated || gguf_f32_on_mfma(ctx, p.M, p.K, p.N));
     if (!mfma && !rotated) return false;
     const bool gemm = mfma && gguf_gemm_takes(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);  // prefill sizes, same copy
     const bool tiles = mfma && gguf_mfma_tiles(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);
-    if (!gemm && !tiles && !(mfma ? gguf_mfma_takes(ctx, p.M, p.N, p.act_dtype) : gguf_res_takes(p.K, p.M, p.act_dtype))) return false;
+    if (!gemm && !tiles && !(mfma ? gguf_mfma_takes(ctx, p.quant, p.M, p.N, p.act_dtype) : gguf_res_takes(p.K, p.M, p.act_dtype))) return false;
     const int kind = mfma ? -2 : -1;
     if (((uintptr_t)p.x & 15) || ((uintptr_t)p.w & 1)) return false;
     if (!ctx->wcache) {
@@ -2049,8 +2049,8 @@ static int build_resident_gguf(oxq_qlinear *l) {
     // a bf16 layer (the reference's GPU path: bf16 x and y) of a format that has it takes the matrix-core layout, an
     // f32 layer where it is large
     l->mfma = gguf_mfma_layer(ctx, l->quant, l->in_features, l->out_features, l->out_dtype) &&
-              !(l->act && (l->out_features % 16 != 0 || l->out_dtype != OXQ_BF16));
-    l->rotated = !(l->mfma && gguf_mfma_alone(ctx, l->out_dtype)) && gguf_res_eligible(l->quant, l->in_features, l->out_features);
+              !(l->act && (l->out_features % 16 != 0 || l->out_dtype != OXQ_BF16 || !gguf_mfma_alone(ctx, l->quant, l->out_dtype)));
+    l->rotated = !(l->mfma && gguf_mfma_alone(ctx, l->quant, l->out_dtype)) && gguf_res_eligible(l->quant, l->in_features, l->out_features);
     if (!l->mfma && !l->rotated) return OXQ_OK;
     if (l->act && !l->mfma) return OXQ_OK;  // the caller reports it
     if (ctx->plan_only) {
@@ -2063,6 +2063,11 @@ static int build_resident_gguf(oxq_qlinear *l) {
     int rc = OXQ_OK;
     const size_t rot_bytes = l->rotated ? (gguf_res_bytes(l->quant, l->in_features, l->out_features) + 255) & ~(size_t)255 : 0;
     hipError_t e = hipMalloc(&l->res, rot_bytes + (l->mfma ? gguf_mfma_bytes(l->quant, l->in_features, l->out_features) : 0));
+    if (e != hipSuccess && l->rotated && l->mfma) {  // no room for both: the rotated copy serves every row it did alone
+        (void)hipGetLastError();
+        l->mfma = false;
+        e = hipMalloc(&l->res, rot_bytes);
+    }
     if (e != hipSuccess) {
         l->res = nullptr;
         rc = fail(OXQ_ERR_RUNTIME, "QLinear: repack allocation failed: %s", hipGetErrorString(e));
@@ -2378,15 +2383,15 @@ int oxq_qlinear_forward(oxq_qlinear *l, void *stream, const oxq_tensor *x, const
                        &l->weight_bytes, l->in_features, l->out_features, l->quant, &o2, &p));
     p.bias = l->has_bias ? l->bias.data : nullptr;
     if (l->resident && ((uintptr_t)p.x & 15) == 0) {
-        const bool f32_rotated = p.act_dtype == OXQ_F32 && l->rotated && gguf_res_takes(p.K, p.M, p.act_dtype) &&
-                                 !(l->mfma && gguf_f32_on_mfma(l->ctx, p.M, p.K, p.N));
-        if (l->mfma && !f32_rotated) {
+        const bool on_rotated = l->rotated && gguf_res_takes(p.K, p.M, p.act_dtype) &&
+                                !(l->mfma && gguf_rows_on_mfma(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype));
+        if (l->mfma && !on_rotated) {
             GgufProblem q = p;
             q.w = (const uint8_t *)l->mm;
-            if (gguf_mfma_takes(l->ctx, p.M, p.N, p.act_dtype) || gguf_mfma_tiles(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype))
+            if (gguf_mfma_takes(l->ctx, l->quant, p.M, p.N, p.act_dtype) || gguf_mfma_tiles(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype))
                 return launch_gguf_mfma(l->ctx, (hipStream_t)stream, q);
             if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype)) return launch_gguf_gemm(l->ctx, (hipStream_t)stream, q);
-        } else if (l->rotated && gguf_res_takes(p.K, p.M, p.act_dtype)) {
+        } else if (on_rotated) {
             p.w = (const uint8_t *)l->rot;
             return launch_gguf_res_gemv(l->ctx, (hipStream_t)stream, p);
         }

@@ -248,11 +248,12 @@ int launch_gguf_res_gemv(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);  //
 // matrix-core copy of a GGUF weight for 16-bit activations and its matmul (gguf_mfma.hip)
 bool gguf_mfma_eligible(const oxq_ctx *ctx, int quant, int64_t K, int64_t N);
 bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int act_dtype);
-bool gguf_mfma_alone(const oxq_ctx *ctx, int act_dtype);
+bool gguf_mfma_alone(const oxq_ctx *ctx, int quant, int act_dtype);
 size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N);
 bool gguf_f32_on_mfma(const oxq_ctx *ctx, int64_t M, int64_t K, int64_t N);
+bool gguf_rows_on_mfma(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);
 bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);
-bool gguf_mfma_takes(const oxq_ctx *ctx, int64_t M, int64_t N, int act_dtype);
+bool gguf_mfma_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t N, int act_dtype);
 int launch_gguf_mfma_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_t *w, void *pw, int64_t K, int64_t N,
                             int64_t gate_half = 0);
 int launch_gguf_mfma_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void *pw, int64_t K, int64_t N, float *out_nk,
