@@ -179,6 +179,11 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 //   - 64-row workgroups of the 64-column layout (121..125 registers) share a CU in pairs: up to one a CU the launch
 //     costs 1 (`part64` up to three quarters of the CUs), up to two a CU a64 + b64 w, beyond that slope64 w
 //     (w = workgroups / CUs); those of the 16-column layout (144..145 registers) run in whole rounds;
+//   - the last rows behind whole tiles of 128, if at most 32, can be tiles of 32 of the same launch (64-column strips, groups of 128
+//     and more), on the CUs that the whole tiles leave idle: a padded tile of 128 costs four times its rows' arithmetic and
+//     often one more round.  Us, 64- or 128-row tiles alone -> with them: 4-bit bf16 3584 x 18944 at 777 rows 127 -> 103,
+//     gate|up 4096 x 28672 at 520 rows 155 -> 122, 4096 x 11008 at 641, 1300, 4100 rows 121 -> 99, 192 -> 156, 397 -> 362; 8-bit f16
+//     4096 x 14336 at 1160 rows 204 -> 170;
 //   - the split-K tiles cost `split_lo` (below one round) or `split_hi` times w at any M: small workgroups, no
 //     ragged round, but the rate they have at 64 rows.
 // The bf16 conversion and the two-strip form are newer than these fits, and groups of 32 and 64 rows are in none.  With every
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 // 5120 x 6144) the choice is within 8 % of the fastest, except where a launch holds one to one and a half rounds: 8-bit
 // 4096 x 6144 at 150 rows split-K 32 us, two strips 23; groups of 64, 4096 x 11008 at 150 rows 46 and 40; groups of 32,
 // 5120 x 6144 at 150 / 777 / 900 / 1200 rows f16 33 / 96 / 96 / 143 as chosen, 26 / 81 / 84 / 108 with two strips.
-// OXQ_PK4_GEMM_ROWS = 64 | 128 takes the choice (tests, sweeps); OXQ_PK4_GEMM_MIN_M = 0 switches the kernels off.
+// OXQ_PK4_GEMM_ROWS = 64 | 128 | 32 (128 and the last tile of 32) takes the choice (tests, sweeps); OXQ_PK4_GEMM_MIN_M = 0 switches the kernels off.
 // a round of the two-strip form (one workgroup a CU) against a full round of 64-row workgroups of eight strips:
 // 19 - 24 us against 65 - 78 at K = 4096 over both widths and types
 constexpr double PK4_MID_ROUND = 0.31;
@@ -201,6 +206,7 @@ struct Pk4GemmCost {
 // rows of a workgroup (0: the split-K tiles) and the K split inside it (4: pk4_mid_kernel, two strips a workgroup)
 struct Pk4GemmForm {
     int rows, ks;
+    bool light = false;  // 128 rows, and those behind the whole tiles in tiles of 32
 };
 // pk4_mid_kernel at up to 64 rows of 64-column strips, against the one-strip workgroups of pk4_mfma_kernel and
 // pk4_tile64_kernel, both one a CU: a round of it costs 1.6 - 1.8 of theirs (4096 x 28672 at 48 / 64 rows: bf16 28.5 / 31.3 ->
@@ -236,6 +242,9 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     const int forced = tune(ctx, OXQ_TUNE_PK4_GEMM_ROWS, 0), forced_ks = tune(ctx, OXQ_TUNE_PK4_GEMM_KS, 0);
     if (p.w.unrounded) return {forced || pk4_fold_prefill(cus, p) ? 64 : 0, 1};
     if (forced_ks == 4) return {64, 4};
+    const int64_t rest = p.M % 128;
+    const bool can_light = p.M > 128 && rest >= 1 && rest <= 32 && p.w.strip != 16 && pk4_sets(p.w.group_shift) == 1;
+    if (forced == 32 && can_light) return {128, 1, true};
     if (forced == 64 || forced == 128) return {forced, 1};
     if (p.M <= 64 && pk4_mid_decode(cus, p) && forced_ks != 1) return {64, 4};
     static const Pk4GemmCost WIDE_F16 = {true, 0.88, 1.20, 0.30, 0.97, 1.50, 1.27, 1.93, 1.50};
@@ -256,6 +265,17 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     };
     const double c64 = !c.pairs64 || w64 <= 1.0 ? rounds(w64, 1.0, c.part64, 0.75) : w64 <= 2.0 ? c.a64 + c.b64 * w64 : c.slope64 * w64;
     const double c128 = rounds(w128, c.full128, c.part128, 0.7);
+    // 128-row workgroups whose last rows (at most 32 behind the whole tiles) are tiles of 32: they start on the CUs that the whole
+    // tiles leave idle and take 0.59 of a round.  Near one 64-row workgroup a CU its squares (pk4g_tile_of) leave some CU two.
+    double c_light = 1e30, c64_light = c64;
+    if (can_light) {
+        const int64_t whole = groups * (p.M / 128), ncu = (int64_t)cus, h = whole % ncu;
+        const double after = h == 0 ? 0.59 * std::ceil((double)groups / cus) * c.full128
+                                    : std::max((double)(h + groups) / cus <= 0.7 ? c.part128 : c.full128,
+                                               std::min(1.59, 0.59 * std::ceil((double)groups / (double)(ncu - h))) * c.full128);
+        c_light = (double)(whole / ncu) * c.full128 + after;
+        if (c.pairs64 && w64 > 0.9 && w64 <= 1.0 && groups % 8) c64_light = c.a64 + c.b64 * w64;
+    }
     // the split-K tiles are one workgroup a row tile and 64 columns, in whole rounds too (64-column strips: up to two of them,
     // beyond that fitted without; 1664 x 4224 f16 at 200 rows, 264 tiles, 15.4 us, 12.1 at 300 rows in the two-strip form)
     const double c_split = (w64 < 1.0 ? c.split_lo : c.split_hi) * (p.w.strip == 16 || w64 <= 0.25 ? std::ceil(8.0 * w64 - 1e-9) / 8.0 : w64);
@@ -265,8 +285,10 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
                          : p.w.strip == 16 ? rounds(w_mid, PK4N_MID_ROUND, PK4N_MID_PART, 0.5)
                                            : std::ceil(w_mid) * PK4_MID_ROUND;
     // (the split-K tiles address the whole of x with 32 bits)
-    if (c_split <= c64 && c_split <= c128 && c_split <= c_mid && (uint64_t)p.M * (uint64_t)p.w.K * 2 < (1ull << 31)) return {0, 1};
-    if (c_mid < c64 && c_mid < c128) return {64, 4};
+    if (c_split <= c64 && c_split <= c128 && c_split <= c_light && c_split <= c_mid && (uint64_t)p.M * (uint64_t)p.w.K * 2 < (1ull << 31)) return {0, 1};
+    if (c_mid < c64 && c_mid < c128 && c_mid < c_light) return {64, 4};
+    // (in f16 the 64-row workgroups are ahead at equal estimates: 2048 x 22016 at 1040 rows 98 us against 102)
+    if (c_light <= (f16 ? 0.99 : 1.02) * c64_light && c_light <= 1.02 * c128) return {128, 1, true};
     return {c128 < c64 ? 128 : 64, 1};
 }
 bool pk4_gemm_takes(const oxq_ctx *ctx, const Pk4Problem &p) { return pk4_gemm_form(ctx, p).rows != 0; }
@@ -286,19 +308,23 @@ static int pk4_gemm_go_layout(hipStream_t s, dim3 grid, const Pk4Problem &p, int
     if (p.w.strip == 16) return pk4n_gemm_go<TT, MT>(s, grid, p, NG, RT);
     return p.w.bits == 8 ? pk4_gemm_wide_go<TT, MT, 8, 1>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, MT, 4, 1>(s, grid, p, NG, RT);
 }
+template <typename TT>
+static int pk4_gemm_go_light(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT) {
+    return p.w.bits == 8 ? pk4_gemm_wide_go<TT, 8, 8, 1, false, 2>(s, grid, p, NG, RT) : pk4_gemm_wide_go<TT, 8, 4, 1, false, 2>(s, grid, p, NG, RT);
+}
 
 int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const Pk4GemmForm form = pk4_gemm_form(ctx, p);
     const int rows = form.rows, spw = PK4G_STRIPS / form.ks;
-    const int64_t NG = ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows);
+    const int64_t NG = ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)spw), RT = form.light ? p.M / rows : ceil_div(p.M, (int64_t)rows);
     // eight strips a workgroup: whole bands of 8 row tiles in squares of 64 workgroups, then the last RT % 8 row
     // tiles x NG groups; two strips: row tile by row tile
-    const int64_t wgs = form.ks == 1 ? (RT / 8) * ceil_div(NG, (int64_t)8) * 64 + (RT % 8) * NG : RT * NG;
+    const int64_t wgs = form.ks == 1 ? (RT / 8) * ceil_div(NG, (int64_t)8) * 64 + (RT % 8) * NG + (form.light ? NG : 0) : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];
     snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw,
-             form.ks > 1 ? "k4" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
+             form.ks > 1 ? "k4" : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
              p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
@@ -309,6 +335,7 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (form.ks == 4) return launch_pk4_mid(s, grid, p, (int)NG);
     if (pk4_sets(p.w.group_shift) > 1) return launch_pk4_gemm_fine(s, grid, p, rows, (int)NG, (int)RT);
     const bool f16 = p.w.dtype == OXQ_F16;
+    if (form.light) return f16 ? pk4_gemm_go_light<F16Traits>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_light<BF16Traits>(s, grid, p, (int)NG, (int)RT);
     if (rows == 128)
         return f16 ? pk4_gemm_go_layout<F16Traits, 8>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_layout<BF16Traits, 8>(s, grid, p, (int)NG, (int)RT);
     return f16 ? pk4_gemm_go_layout<F16Traits, 4>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_layout<BF16Traits, 4>(s, grid, p, (int)NG, (int)RT);

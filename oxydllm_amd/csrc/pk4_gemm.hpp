@@ -36,10 +36,11 @@ template <typename TT, int BITS> struct Pk4Fold {
 // FOLD (layers with `unrounded`): the folded form of pk4_mfma_kernel - the matrix cores multiply x by the integers, one
 // more MFMA a step against ones yields the row sums of x, and a group's sums enter the accumulators through
 // s * (sum - (bias + z) * rowsum), all f32.
-template <typename TT, int MT, int BITS, int SETS = 1, bool FOLD = false>
-__global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
-                                                       const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
-                                                       int M, int K, int N, int NG, int RT, int act) {
+// Rows from m0 on, strip group g.
+template <typename TT, int MT, int BITS, int SETS, bool FOLD>
+__device__ __forceinline__ void pk4_gemm_tile(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
+                                              const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int M, int K, int N,
+                                              int m0, int g, int act) {
     typedef MfmaOps<TT> Ops;
     constexpr int ROWS = 16 * MT, BB = pk4_block_words(BITS, SETS) * 4, XBUF = ROWS * 256;
     constexpr int WL = BITS / 4;          // 1 KB weight loads a step (8-bit: column pairs 0, 1 and 2, 3)
@@ -52,12 +53,8 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ni = lane & 15, kb = lane >> 4;
-    int rt, g;
-    pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
-    if (g >= NG) return;  // the whole workgroup, before any barrier: the ragged last column of squares
     const int j = g * PK4G_STRIPS + wave;
     const bool live = j < ((N + 63) >> 6);  // wave-uniform: the last group of a layer may have fewer strips
-    const int m0 = rt * ROWS;
     const int NB = SETS > 1 ? (K + 127) >> 7 : K >> 7;
     const int xrows = min(M - m0, ROWS);
 
@@ -307,12 +304,30 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         }
 }
 
-template <typename TT, int MT, int BITS, int SETS, bool FOLD = false>
+// LIGHT: the rows behind the RT whole tiles, at most 16 LIGHT, are a tile of their own size in the last NG workgroups.
+template <typename TT, int MT, int BITS, int SETS = 1, bool FOLD = false, int LIGHT = 0>
+__global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
+                                                       const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
+                                                       int M, int K, int N, int NG, int RT, int act) {
+    int rt, g;
+    if constexpr (LIGHT > 0) {
+        const int whole = (int)gridDim.x - NG;
+        if ((int)blockIdx.x >= whole) {
+            pk4_gemm_tile<TT, LIGHT, BITS, SETS, FOLD>(x, pw, bias, y, M, K, N, RT * 16 * MT, (int)blockIdx.x - whole, act);
+            return;
+        }
+    }
+    pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
+    if (g >= NG) return;  // the whole workgroup, before any barrier: the ragged last column of squares
+    pk4_gemm_tile<TT, MT, BITS, SETS, FOLD>(x, pw, bias, y, M, K, N, rt * 16 * MT, g, act);
+}
+
+template <typename TT, int MT, int BITS, int SETS, bool FOLD = false, int LIGHT = 0>
 static int pk4_gemm_wide_go(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT) {
     static LdsGrant grant;  // one per instantiation
     const size_t lds = (size_t)2 * 16 * MT * 256;
-    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_gemm_kernel<TT, MT, BITS, SETS, FOLD>, lds));
-    hipLaunchKernelGGL((pk4_gemm_kernel<TT, MT, BITS, SETS, FOLD>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
+    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_gemm_kernel<TT, MT, BITS, SETS, FOLD, LIGHT>, lds));
+    hipLaunchKernelGGL((pk4_gemm_kernel<TT, MT, BITS, SETS, FOLD, LIGHT>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw, (const uint16_t *)p.bias,
                        (uint16_t *)p.y, (int)p.M, (int)p.w.K, (int)p.w.N, NG, RT, p.act);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
