@@ -53,14 +53,21 @@ template <int N> __device__ __forceinline__ void pk4g_wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Workgroup -> (row tile, strip group).  Bands of 8 row tiles are cut into squares of 8 row tiles x 8 strip groups,
-// 64 neighbouring workgroups each (neighbour i runs on XCD i % 8: a row tile stays on one XCD); the last RT % 8
-// row tiles are numbered row tile first, so that no XCD is handed only idle workgroups.
+// Workgroup -> (row tile, strip group), RT x NG of them.  Bands of 8 row tiles are cut into squares of 8 row tiles x 8 strip
+// groups (the last column of them as wide as the groups left), neighbouring workgroups each (neighbour i runs on XCD
+// i % 8: a row tile stays on one XCD); the last RT % 8 row tiles are numbered row tile first.
+// No number is left without a tile: with whole squares, workgroups that left at once still took their turn in the round over
+// an XCD's shader engines, so that some CUs got two tiles and others none.  Us, whole squares -> here: 8-bit f16 5376 x 2368
+// at 2127 rows (5 groups x 34 tiles of 64) 163 -> 86, 4-bit bf16 groups of 64 1280 x 2752 at 2655 rows 59 -> 33; Q5_K 7680 x 6272
+// at 1042 rows 361 -> 188, Q4_K 1280 x 19008 at 1278 rows 130 -> 102.
 __device__ __forceinline__ void pk4g_tile_of(int id, int RT, int NG, int &rt, int &g) {
-    const int full = (RT >> 3) * ((NG + 7) >> 3) * 64, tail = RT & 7;
-    if (id < full) {
-        const int sq = id >> 6, within = id & 63, bands = RT >> 3;
+    const int bands = RT >> 3, whole = bands * (NG >> 3) * 64, full = bands * NG * 8, tail = RT & 7;
+    if (id < whole) {
+        const int sq = id >> 6, within = id & 63;
         rt = (sq % bands) * 8 + (within & 7), g = (sq / bands) * 8 + (within >> 3);
+    } else if (id < full) {
+        const int size = (NG & 7) * 8, within = (id - whole) % size;
+        rt = (id - whole) / size * 8 + (within & 7), g = (NG & ~7) + (within >> 3);
     } else {
         rt = (RT & ~7) + (id - full) % tail, g = (id - full) / tail;
     }

@@ -42,7 +42,6 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
     const int ni = lane & 15, kb = lane >> 4;
     int rt, g;
     pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
-    if (g >= NG) return;  // the whole workgroup, before any barrier
     const int j = g * PK4G_STRIPS + wave;  // the wave's 64 columns: strips 4 j .. 4 j + 3
     const bool live = j < (N >> 6);
     const int m0 = rt * ROWS;
@@ -317,9 +316,8 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const Pk4GemmForm form = pk4_gemm_form(ctx, p);
     const int rows = form.rows, spw = PK4G_STRIPS / form.ks;
     const int64_t NG = ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)spw), RT = form.light ? p.M / rows : ceil_div(p.M, (int64_t)rows);
-    // eight strips a workgroup: whole bands of 8 row tiles in squares of 64 workgroups, then the last RT % 8 row
-    // tiles x NG groups; two strips: row tile by row tile
-    const int64_t wgs = form.ks == 1 ? (RT / 8) * ceil_div(NG, (int64_t)8) * 64 + (RT % 8) * NG + (form.light ? NG : 0) : RT * NG;
+    // eight strips a workgroup: in the order of pk4g_tile_of; two strips: row tile by row tile
+    const int64_t wgs = RT * NG + (form.light ? NG : 0);
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];

@@ -318,7 +318,6 @@ __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restric
         }
     }
     pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
-    if (g >= NG) return;  // the whole workgroup, before any barrier: the ragged last column of squares
     pk4_gemm_tile<TT, MT, BITS, SETS, FOLD>(x, pw, bias, y, M, K, N, rt * 16 * MT, g, act);
 }
 
