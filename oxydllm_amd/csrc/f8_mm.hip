@@ -214,6 +214,7 @@ __global__ __launch_bounds__(512) void f8_gemm_kernel(const uint16_t *__restrict
     const int ws = wave % SPW, kq = wave / SPW;  // the wave's column group of the workgroup, and its share of K
     int rt, g;
     if constexpr (KS == 1) {
+        if ((int)blockIdx.x >= RT * NG) return;  // the whole workgroup, before any barrier
         pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
     } else {
         rt = (int)blockIdx.x / NG, g = (int)blockIdx.x % NG;
@@ -530,7 +531,7 @@ int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
     }
     const int ks = form.kind, spw = 8 / ks;
     const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)64), (int64_t)spw), RT = ceil_div(p.M, (int64_t)64), chunks = p.K / 128;
-    const int64_t wgs = RT * NG;
+    const int64_t wgs = ks == 1 ? pk4g_workgroups(RT, NG) : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "f8 matmul: m = %lld exceeds the grid", (long long)p.M);
     const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)4) * 4) : (int)chunks;
     dim3 grid((unsigned)wgs, (unsigned)form.slices);

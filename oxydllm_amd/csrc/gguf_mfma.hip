@@ -945,6 +945,7 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
     const int ws = wave % SPW, kq = wave / SPW;  // the wave's column group of the workgroup, and its share of K
     int rt, g;
     if constexpr (KS == 1) {
+        if ((int)blockIdx.x >= RT * NG) return;  // the whole workgroup, before any barrier
         pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
     } else {
         rt = (int)blockIdx.x / NG, g = (int)blockIdx.x % NG;
@@ -1584,7 +1585,7 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     if (p.act) form.slices = 1;
     const int ks = form.ks, spw = 8 / ks;
     const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)64), (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows);
-    const int64_t wgs = RT * NG;
+    const int64_t wgs = ks == 1 ? pk4g_workgroups(RT, NG) : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: m = %lld exceeds the grid", (long long)p.M);
     const int64_t chunks = p.K / 128;
     const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)4) * 4) : (int)chunks;

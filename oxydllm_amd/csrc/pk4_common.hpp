@@ -56,8 +56,9 @@ template <int N> __device__ __forceinline__ void pk4g_wait_vmcnt() {
 // Workgroup -> (row tile, strip group), RT x NG of them.  Bands of 8 row tiles are cut into squares of 8 row tiles x 8 strip
 // groups (the last column of them as wide as the groups left), neighbouring workgroups each (neighbour i runs on XCD
 // i % 8: a row tile stays on one XCD); the last RT % 8 row tiles are numbered row tile first.
-// No number is left without a tile: with whole squares, workgroups that left at once still took their turn in the round over
-// an XCD's shader engines, so that some CUs got two tiles and others none.  Us, whole squares -> here: 8-bit f16 5376 x 2368
+// The numbers of tiles have no gaps; a launch, whose size plans report as whole squares, holds its idle workgroups behind the
+// last tile.  Between the tiles they took their turn in the round over an XCD's shader engines, so that some CUs got two tiles
+// and others none.  Us, between -> behind: 8-bit f16 5376 x 2368
 // at 2127 rows (5 groups x 34 tiles of 64) 163 -> 86, 4-bit bf16 groups of 64 1280 x 2752 at 2655 rows 59 -> 33; Q5_K 7680 x 6272
 // at 1042 rows 361 -> 188, Q4_K 1280 x 19008 at 1278 rows 130 -> 102.
 __device__ __forceinline__ void pk4g_tile_of(int id, int RT, int NG, int &rt, int &g) {
@@ -72,6 +73,8 @@ __device__ __forceinline__ void pk4g_tile_of(int id, int RT, int NG, int &rt, in
         rt = (RT & ~7) + (id - full) % tail, g = (id - full) / tail;
     }
 }
+
+inline int64_t pk4g_workgroups(int64_t RT, int64_t NG) { return (RT / 8) * ((NG + 7) / 8) * 64 + (RT % 8) * NG; }
 
 // bf16 has no packed 16-bit arithmetic: a weight goes to f32, through an fma and (a pair at a time) to bf16.
 // (q - z) s is exact in f32, so the bits are those of Pk4T<BF16Traits>::deq.  These kernels are bound by the issue of

@@ -41,6 +41,7 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ni = lane & 15, kb = lane >> 4;
     int rt, g;
+    if ((int)blockIdx.x >= RT * NG) return;  // the whole workgroup, before any barrier
     pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
     const int j = g * PK4G_STRIPS + wave;  // the wave's 64 columns: strips 4 j .. 4 j + 3
     const bool live = j < (N >> 6);
@@ -317,7 +318,7 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const int rows = form.rows, spw = PK4G_STRIPS / form.ks;
     const int64_t NG = ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)spw), RT = form.light ? p.M / rows : ceil_div(p.M, (int64_t)rows);
     // eight strips a workgroup: in the order of pk4g_tile_of; two strips: row tile by row tile
-    const int64_t wgs = RT * NG + (form.light ? NG : 0);
+    const int64_t wgs = form.ks == 1 ? pk4g_workgroups(RT, NG) + (form.light ? NG : 0) : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];

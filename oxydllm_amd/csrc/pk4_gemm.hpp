@@ -304,19 +304,21 @@ __device__ __forceinline__ void pk4_gemm_tile(const uint16_t *__restrict__ x, co
         }
 }
 
-// LIGHT: the rows behind the RT whole tiles, at most 16 LIGHT, are a tile of their own size in the last NG workgroups.
+// LIGHT: the rows behind the RT whole tiles, at most 16 LIGHT, are a tile of their own size in the NG workgroups after them.
 template <typename TT, int MT, int BITS, int SETS = 1, bool FOLD = false, int LIGHT = 0>
 __global__ __launch_bounds__(512) void pk4_gemm_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
                                                        const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                        int M, int K, int N, int NG, int RT, int act) {
     int rt, g;
     if constexpr (LIGHT > 0) {
-        const int whole = (int)gridDim.x - NG;
+        const int whole = RT * NG;
+        if ((int)blockIdx.x >= whole + NG) return;
         if ((int)blockIdx.x >= whole) {
             pk4_gemm_tile<TT, LIGHT, BITS, SETS, FOLD>(x, pw, bias, y, M, K, N, RT * 16 * MT, (int)blockIdx.x - whole, act);
             return;
         }
     }
+    if ((int)blockIdx.x >= RT * NG) return;  // the whole workgroup, before any barrier
     pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
     pk4_gemm_tile<TT, MT, BITS, SETS, FOLD>(x, pw, bias, y, M, K, N, rt * 16 * MT, g, act);
 }
