@@ -1512,7 +1512,9 @@ static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int6
         return {c_mid < r64 ? 4 : 1, 1};
     }
     GgmCost c = ggm_cost(quant);
-    if (narrow) r64 = std::ceil((double)((row_tiles / 8) * ceil_div(groups, (int64_t)64) * 64 + (row_tiles % 8) * ceil_div(groups, (int64_t)8)) / cus);
+    // whole rounds of the workgroups that have a tile (us, idle ones counted / not: Q3_K 2816 x 2304 at 2871 rows, file layout, 113 / 76, Q2_K
+    // 4352 x 12544 at 576 140 / 110, Q3_K 3840 x 8576 at 1718, two strips, 251 / 198)
+    if (narrow) r64 = std::ceil(w64);
     if (narrow && M <= 48) c.round = M <= 16 ? 2.2 : M <= 32 ? 2.7 : 3.1;
     GgmGemmForm best = {1, 1};
     double least = r64 * ((double)chunks * c.wide + 5.0);

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 //   - the last rows behind whole tiles of 128, if at most 32, can be tiles of 32 of the same launch (64-column strips, groups of 128
 //     and more), on the CUs that the whole tiles leave idle: a padded tile of 128 costs four times its rows' arithmetic and
 //     often one more round.  Us, 64- or 128-row tiles alone -> with them: 4-bit bf16 3584 x 18944 at 777 rows 127 -> 103,
-//     gate|up 4096 x 28672 at 520 rows 155 -> 122, 4096 x 11008 at 641, 1300, 4100 rows 121 -> 99, 192 -> 156, 397 -> 362; 8-bit f16
+//     gate|up 4096 x 28672 at 520 rows 155 -> 122, 4096 x 11008 at 1300, 4100 rows 192 -> 156, 397 -> 362; 8-bit f16
 //     4096 x 14336 at 1160 rows 204 -> 170;
 //   - the split-K tiles cost `split_lo` (below one round) or `split_hi` times w at any M: small workgroups, no
 //     ragged round, but the rate they have at 64 rows.
@@ -266,15 +266,16 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     const double c64 = !c.pairs64 || w64 <= 1.0 ? rounds(w64, 1.0, c.part64, 0.75) : w64 <= 2.0 ? c.a64 + c.b64 * w64 : c.slope64 * w64;
     const double c128 = rounds(w128, c.full128, c.part128, 0.7);
     // 128-row workgroups whose last rows (at most 32 behind the whole tiles) are tiles of 32: they start on the CUs that the whole
-    // tiles leave idle and take 0.59 of a round.  Near one 64-row workgroup a CU its squares (pk4g_tile_of) leave some CU two.
-    double c_light = 1e30, c64_light = c64;
+    // tiles leave idle and take 0.59 of a round.  (At 0.9 - 1 64-row workgroups a CU those are ahead, now that each gets one: us, last rows in
+    // tiles of 32 / 64-row workgroups, f16 7552 x 10368 at 651 rows 151 / 112, 1152 x 4672 at 1557 31.5 / 23.3, bf16 4736 x 11712 at 662
+    // 111 / 88, 8064 x 18176 at 406 181 / 148.)
+    double c_light = 1e30;
     if (can_light) {
         const int64_t whole = groups * (p.M / 128), ncu = (int64_t)cus, h = whole % ncu;
         const double after = h == 0 ? 0.59 * std::ceil((double)groups / cus) * c.full128
                                     : std::max((double)(h + groups) / cus <= 0.7 ? c.part128 : c.full128,
                                                std::min(1.59, 0.59 * std::ceil((double)groups / (double)(ncu - h))) * c.full128);
         c_light = (double)(whole / ncu) * c.full128 + after;
-        if (c.pairs64 && w64 > 0.9 && w64 <= 1.0 && groups % 8) c64_light = c.a64 + c.b64 * w64;
     }
     // the split-K tiles are one workgroup a row tile and 64 columns, in whole rounds too (64-column strips: up to two of them,
     // beyond that fitted without; 1664 x 4224 f16 at 200 rows, 264 tiles, 15.4 us, 12.1 at 300 rows in the two-strip form)
@@ -288,7 +289,7 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     if (c_split <= c64 && c_split <= c128 && c_split <= c_light && c_split <= c_mid && (uint64_t)p.M * (uint64_t)p.w.K * 2 < (1ull << 31)) return {0, 1};
     if (c_mid < c64 && c_mid < c128 && c_mid < c_light) return {64, 4};
     // (in f16 the 64-row workgroups are ahead at equal estimates: 2048 x 22016 at 1040 rows 98 us against 102)
-    if (c_light <= (f16 ? 0.99 : 1.02) * c64_light && c_light <= 1.02 * c128) return {128, 1, true};
+    if (c_light <= (f16 ? 0.99 : 1.02) * c64 && c_light <= 1.02 * c128) return {128, 1, true};
     return {c128 < c64 ? 128 : 64, 1};
 }
 bool pk4_gemm_takes(const oxq_ctx *ctx, const Pk4Problem &p) { return pk4_gemm_form(ctx, p).rows != 0; }

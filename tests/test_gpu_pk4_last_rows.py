@@ -15,7 +15,7 @@ def test_last_rows_take_idle_compute_units():
     """Where the whole tiles leave compute units idle or a padded one would start a round; not where 64-row tiles are ahead."""
     names = lambda k, n, rows: [kern for kern, _ in kernels(ops.PACK_IN, 4, k, n, 128, _lib.BF16, rows)]
     assert names(3584, 18944, (768, 777, 800, 801, 1040)) == ["pk4_gemm_bf16_r128x8"] + ["pk4_gemm_bf16_r128x8r32"] * 2 + ["pk4_gemm_bf16_r64x8"] * 2
-    assert names(4096, 11008, (641, 1300)) == ["pk4_gemm_bf16_r128x8r32"] * 2 and names(2048, 8192, (905,)) == ["pk4_gemm_bf16_r64x8"]
+    assert names(4096, 11008, (641, 1300)) == ["pk4_gemm_bf16_r64x8", "pk4_gemm_bf16_r128x8r32"] and names(2048, 8192, (905,)) == ["pk4_gemm_bf16_r64x8"]
 
 
 # the last group: seven strips of eight, two of eight; K of two and five blocks; whole bands of eight row tiles and a last one
