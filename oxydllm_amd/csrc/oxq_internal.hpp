@@ -205,6 +205,7 @@ struct Pk4Problem {
 };
 
 // ---- launchers (defined in the .hip files) ---------------------------------
+bool awq_fast_ok(const Wna16Problem &p);  // whether the AWQ dot-product kernel takes these tensors (wna16_gemv.hip)
 // checkpoint layouts, few rows on the matrix cores (wna16_slab.hip)
 bool wna16_slab_takes(const oxq_ctx *ctx, const Wna16Problem &p);
 int launch_wna16_slab(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p);

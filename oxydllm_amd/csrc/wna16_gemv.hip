@@ -801,7 +801,7 @@ static int launch_awq_fast(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
                : launch_awq_fast_t<TT, BITS, 8, 1, 4, 1, 2, 4>(ctx, s, p, gpw_for(256 * CPW / 8, 1));
 }
 
-static bool awq_fast_ok(const Wna16Problem &p) {
+bool awq_fast_ok(const Wna16Problem &p) {
     if ((p.bits != 4 && p.bits != 8) || p.pack_dim != OXQ_PACK_OUT) return false;
     if (p.N % 32 != 0 || p.K % 2 != 0) return false;
     if (p.group_size < 64) return false;  // 2 * WPG * RPW * PS rows per chunk

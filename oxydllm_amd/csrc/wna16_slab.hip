@@ -347,9 +347,10 @@ static int slab_go(hipStream_t s, dim3 grid, const Wna16Problem &p, float *ws, i
 }
 template <typename TT, bool GPTQ>
 static int slab_by_shape(hipStream_t s, dim3 grid, const Wna16Problem &p, float *ws, int blocks, int run) {
-    // bf16 AWQ as its dot-product kernel: NaN for infinite x (the second path's registers cost 4 rows of 4096 x 14336 12.7 -> 13.3 us)
+    // bf16 AWQ tensors that the dot-product kernel takes, as there: NaN for infinite x (the second path's registers cost 4 rows of
+    // 4096 x 14336 12.7 -> 13.3 us).  Others (their address counts too) keep the signs that the generic kernel gives.
     if constexpr (TT::DTYPE != F16Traits::DTYPE && !GPTQ) {
-        if (p.group_size >= 64 && p.N % 32 == 0)
+        if (awq_fast_ok(p))
             return p.bits == 8 ? slab_go<TT, 8, GPTQ, 2, 1, false>(s, grid, p, ws, blocks)
                    : run == 64 ? slab_go<TT, 4, GPTQ, 2, 1, false>(s, grid, p, ws, blocks)
                                : slab_go<TT, 4, GPTQ, 4, 1, false>(s, grid, p, ws, blocks);

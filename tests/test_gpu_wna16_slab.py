@@ -126,3 +126,39 @@ def test_an_infinite_f16_row_keeps_its_signs():
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
     assert bool(torch.isposinf(y[1]).any()) and bool(torch.isneginf(y[1]).any())
     assert torch.equal(y[0], ops.w4a16_matmul(clean, *big)[0]) or bool(((y[0] - ops.w4a16_matmul(clean, *big)[0]).abs() <= 2e-3 * y[0].abs() + 1e-2).all())
+
+
+def at_address(t, off):
+    """The same words ``off`` elements behind a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 16, device="cuda", dtype=t.dtype)
+    v = buf[off:off + t.numel()].view(t.shape)
+    v.copy_(t)
+    assert v.data_ptr() % 16 == off * t.element_size()
+    return v
+
+
+@pytest.mark.parametrize("bits,g", [(4, 64), (4, 128), (8, 128)])
+@pytest.mark.parametrize("which", ["qweight", "qzeros", "neither"])
+def test_infinite_bf16_rows_where_the_dot_product_kernel_does_not_take_the_address(bits, g, which):
+    """AWQ tensors off a 16-byte boundary ran the generic kernel, which keeps the sign of an infinity; on one, the
+    dot-product kernel, where such a row is NaN."""
+    K, N = 1024, 2048
+    print(f"[case] awq slab {bits} g={g} {which} off a boundary", flush=True)
+    qw, qz, sc = synth.awq_checkpoint(K, N, g, bits, seed=5)
+    d = [to_dev(qw), to_dev(qz), to_dev(sc, torch.bfloat16)]
+    if which != "neither":
+        i = ["qweight", "qzeros"].index(which)
+        d[i] = at_address(d[i], 1)
+    x = np.random.default_rng(1).standard_normal((4, K)).astype(np.float32)
+    x[1, 37], x[2, 900], x[3, 5], x[3, 6] = np.inf, -np.inf, np.nan, np.inf
+    xd = to_dev(x, torch.bfloat16)
+    op = ops.w4a16_matmul if bits == 4 else ops.w8a16_matmul
+    y = op(xd, *d)
+    assert "_slab" in ops.default_context().last_plan()["kernel"]
+    tune("OXQ_GEMV_TILE", 0)
+    old = op(xd, *d)
+    assert ("generic" in ops.default_context().last_plan()["kernel"]) == (which != "neither")
+    tune("OXQ_GEMV_TILE", None)
+    for r in (1, 2, 3):
+        assert torch.equal(torch.isnan(y[r]), torch.isnan(old[r])) and torch.equal(torch.nan_to_num(y[r]), torch.nan_to_num(old[r]))
+    assert bool(torch.isposinf(y[1]).any()) == (which != "neither")
