@@ -10,8 +10,8 @@
 // order by a second launch.
 //
 // The weight is never rounded: bias and zero point come out through the row sums of x, the scale multiplies the group's
-// f32 sum.  (Where a row is not finite, the zero point leaves the integers instead: such
-// sums have a sign.)
+// f32 sum.  (Where a row is not finite, or so large that the biased products could overflow, the zero point leaves the
+// integers instead: such sums have a sign.)
 //
 // What bounds it: the read of the weights plus a launch (the sum).  Every load of a wave's rows is requested before
 // the first is waited for - 16 KB a wave, two workgroups a compute unit.
@@ -65,7 +65,7 @@ template <int BITS> __device__ __forceinline__ u32x4_t slab_gptq_x(u32x4_t d) {
 }
 
 // STEPS: MFMA steps (32 rows of K) of a run, which a wave holds at once.  SETS: groups in it (1: a group is a run or more).
-// SIGNS: infinite x give signed sums.  `blocks`: runs a wave takes.
+// SIGNS: infinite x give signed sums, and very large ones those of the weights themselves.  `blocks`: runs a wave takes.
 template <typename TT, int BITS, bool GPTQ, int STEPS, int SETS, bool SIGNS>
 __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ qw,
                                                                       const uint32_t *__restrict__ qz, const uint16_t *__restrict__ sc,
@@ -180,6 +180,7 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
 #pragma unroll
         for (int set = 0; set < SETS; ++set) {
             float4_t rs = float4_t{0.f, 0.f, 0.f, 0.f};  // row sums of x, in the layout of the products
+            float4_t sq = float4_t{0.f, 0.f, 0.f, 0.f};  // x times itself transposed: a row's squares on the diagonal
             {
                 constexpr uint32_t ONE = F16 ? 0x3C003C00u : 0x3F803F80u;
                 const uint32_t ones[4] = {ONE, ONE, ONE, ONE};
@@ -187,12 +188,15 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
                 for (int st = set * ST; st < set * ST + ST; ++st) {
                     const uint32_t a[4] = {xa[st][0], xa[st][1], xa[st][2], xa[st][3]};
                     rs = Ops::mfma(a, ones, rs);
+                    if constexpr (SIGNS) sq = Ops::mfma(a, a, sq);
                 }
             }
-            // EXACT: the zero point leaves the integers instead of the sums, so that an infinite x gives what it gives where
-            // every weight is multiplied by itself
+            // EXACT: the zero point leaves the integers instead of the sums, so that an infinite or very large x gives what it
+            // gives where every weight is multiplied by itself.  In bf16 a group's sum of up to 2^15 |x| is kept down by as much
+            // until the scale multiplies it.
             auto columns = [&](auto exact) {
                 constexpr bool EXACT = decltype(exact)::value;
+                constexpr float DOWN = 0x1p-15f;
 #pragma unroll
                 for (int c = 0; c < 16; ++c) {  // AWQ: slot s of word i; GPTQ: the lane's columns in order
                     const int i = c / CPW, s = c % CPW, HALF = CPW / 2;  // HALF: slots in a 16-bit half
@@ -220,7 +224,7 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
                                     const half2_t off2 = {(_Float16)off, (_Float16)off};
                                     bq[j] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, bq[j]) + off2);
                                 } else {
-                                    const float lo = __builtin_bit_cast(float, bq[j] << 16) + off, hi = __builtin_bit_cast(float, bq[j] & 0xFFFF0000u) + off;
+                                    const float lo = (__builtin_bit_cast(float, bq[j] << 16) + off) * DOWN, hi = (__builtin_bit_cast(float, bq[j] & 0xFFFF0000u) + off) * DOWN;
                                     bq[j] = perm_b32(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
                                 }
                             }
@@ -228,7 +232,7 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
                         p = Ops::mfma(a, bq, p);
                     }
                     const uint32_t sw = sv[set][col >> 1];
-                    const float scale = TT::to_f32((uint16_t)(col & 1 ? sw >> 16 : sw));
+                    const float scale = TT::to_f32((uint16_t)(col & 1 ? sw >> 16 : sw)) * (EXACT && !F16 ? 1.0f / DOWN : 1.0f);
                     if constexpr (!EXACT) {
 #pragma unroll
                         for (int q = 0; q < 4; ++q) p[q] = __builtin_fmaf(off, rs[q], p[q]);
@@ -237,8 +241,10 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
                     for (int q = 0; q < 4; ++q) acc[col][q] = __builtin_fmaf(scale, p[q], acc[col][q]);
                 }
             };
-            const float sum = (rs[0] + rs[1]) + (rs[2] + rs[3]);  // finite where all four are (four sums of 128 16-bit floats)
             if constexpr (SIGNS) {
+                // Finite squares: no |x| beyond 2^64, so neither the biased products (at most 2^11 |x|) nor their sums overflow.
+                // (The sum of four finite ones may overflow: the exact columns then, for nothing but time.)
+                const float sum = (sq[0] + sq[1]) + (sq[2] + sq[3]);
                 if (__builtin_expect(__any(!(fabsf(sum) <= 3.4e38f)), 0)) columns(std::true_type{});
                 else columns(std::false_type{});
             } else {

@@ -162,3 +162,31 @@ def test_infinite_bf16_rows_where_the_dot_product_kernel_does_not_take_the_addre
     for r in (1, 2, 3):
         assert torch.equal(torch.isnan(y[r]), torch.isnan(old[r])) and torch.equal(torch.nan_to_num(y[r]), torch.nan_to_num(old[r]))
     assert bool(torch.isposinf(y[1]).any()) == (which != "neither")
+
+
+@pytest.mark.parametrize("method,bits,g", [("gptq", 4, 32), ("gptq", 4, 64), ("gptq", 8, 64), ("awq", 4, 32), ("awq", 8, 32)])
+def test_large_finite_bf16_rows_do_not_overflow(method, bits, g):
+    """Rows whose products with bias + q overflow f32 while those with q - z do not.  A result is one bf16 rounding and the
+    f32 sums off (2^-8 and 2^-20 of the sum of the terms' magnitudes)."""
+    K, N = 1024, 4096
+    print(f"[case] slab large finite rows {method} {bits} g={g}", flush=True)
+    make = synth.gptq_checkpoint if method == "gptq" else synth.awq_checkpoint
+    qw, qz, sc = make(K, N, g, bits, seed=7)
+    s = oracle.round_through(sc, oracle.BF16)
+    w = oracle.dequantize_gptq(qw, qz, s, bits) if method == "gptq" else (oracle.dequantize_awq if bits == 4 else oracle.dequantize_awq8)(qw, qz, s)
+    x = np.random.default_rng(2).standard_normal((4, K)).astype(np.float32)
+    x[1] = np.abs(x[1]) * (1e36 if bits == 4 else 1.2e35)   # 32 products with 128 + q, with q of 8 bits: beyond 3.4e38
+    x[2, 5], x[3, 5], x[3, 6] = 3e38 if bits == 4 else 2e37, 3e36, -3e36   # one weight without its scale
+    xr = round_x(x, oracle.BF16)
+    d = (to_dev(qw), to_dev(qz), to_dev(sc, torch.bfloat16))
+    xd = to_dev(x, torch.bfloat16)
+    if method == "gptq":
+        y = ops.gptq_matmul(xd, *d, bits)
+    else:
+        y = (ops.w4a16_matmul if bits == 4 else ops.w8a16_matmul)(xd, *d)
+    assert "_slab" in ops.default_context().last_plan()["kernel"]
+    y = y.double().cpu().numpy()
+    x64, w64 = xr.astype(np.float64), w.reshape(N, K).astype(np.float64)
+    ref, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64.T)
+    assert np.isfinite(y).all()
+    assert (np.abs(y - ref) <= 2.0 ** -8 * np.abs(ref) + 2.0 ** -20 * mag).all()
