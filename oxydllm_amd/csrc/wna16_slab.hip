@@ -25,9 +25,14 @@ namespace oxq {
 
 constexpr int SLAB_COLS = 256, SLAB_WAVES = 4;
 
-// B operands hold bias + q: the bias
-template <typename TT, int BITS, bool GPTQ> __device__ __forceinline__ constexpr float slab_bias(int s) {
-    return TT::DTYPE == F16Traits::DTYPE ? (BITS == 4 && !GPTQ && (s & 1) ? 64.f : 1024.f) : (BITS == 4 ? 128.f : 0.f);
+// B operands hold bias + q: the bias.  In f16 the bias takes bits of the sums: 1024 beside four-bit codes left errors of small
+// outputs three times those of weights multiplied one by one (1e-6 against 3e-7 of the sum of the terms' magnitudes at K =
+// 4096), 64 leaves none to be seen.  GPTQ has it for nothing.  For AWQ it is two shifts more (4096 x 14336, groups of 32, 13.3 ->
+// 13.6 us), and LOW asks for it: calls that otherwise run the generic kernel, not those whose weights the tile kernel rounds or that
+// the dot products bias as here.
+template <typename TT, int BITS, bool GPTQ, bool LOW> __device__ __forceinline__ constexpr float slab_bias(int s) {
+    if (TT::DTYPE != F16Traits::DTYPE) return BITS == 4 ? 128.f : 0.f;
+    return BITS == 4 && (GPTQ || LOW || (s & 1)) ? 64.f : 1024.f;
 }
 // bytes 0 and 2 of t, or 1 and 3
 template <typename TT> __device__ __forceinline__ uint32_t slab_bytes(uint32_t t, bool high) {
@@ -36,12 +41,14 @@ template <typename TT> __device__ __forceinline__ uint32_t slab_bytes(uint32_t t
     return perm_b32(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);  // 8 bits: exact
 }
 // AWQ: slot `s` of a 16-bit half of the four row pairs t
-template <typename TT, int BITS>
+template <typename TT, int BITS, bool LOW>
 __device__ __forceinline__ void slab_awq_operand(const uint32_t (&t)[4], int s, const NibbleMasks &nm, uint32_t (&b)[4]) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         if constexpr (BITS == 8) {
             b[p] = slab_bytes<TT>(t[p], s & 1);
+        } else if constexpr (TT::DTYPE == F16Traits::DTYPE && LOW) {
+            b[p] = ((s ? t[p] >> (4 * s - 4) : t[p] << 4) & nm.m1) | 0x54005400u;
         } else if constexpr (TT::DTYPE == F16Traits::DTYPE) {
             const uint32_t u = s < 2 ? t[p] : t[p] >> 8;
             b[p] = s & 1 ? (u & nm.m1) | 0x54005400u : (u & nm.m0) | 0x64006400u;
@@ -56,7 +63,10 @@ template <typename TT, int BITS> __device__ __forceinline__ void slab_gptq_opera
         b[0] = slab_bytes<TT>(w0, false), b[1] = slab_bytes<TT>(w0, true), b[2] = slab_bytes<TT>(w1, false), b[3] = slab_bytes<TT>(w1, true);
     } else {
 #pragma unroll
-        for (int n = 0; n < 4; ++n) b[n] = ((w0 >> (4 * n)) & nm.m0) | (TT::DTYPE == F16Traits::DTYPE ? 0x64006400u : 0x43004300u);
+        for (int n = 0; n < 4; ++n) {
+            if constexpr (TT::DTYPE == F16Traits::DTYPE) b[n] = ((n ? w0 >> (4 * n - 4) : w0 << 4) & nm.m1) | 0x54005400u;
+            else b[n] = ((w0 >> (4 * n)) & nm.m0) | 0x43004300u;
+        }
     }
 }
 template <int BITS> __device__ __forceinline__ u32x4_t slab_gptq_x(u32x4_t d) {
@@ -66,7 +76,7 @@ template <int BITS> __device__ __forceinline__ u32x4_t slab_gptq_x(u32x4_t d) {
 
 // STEPS: MFMA steps (32 rows of K) of a run, which a wave holds at once.  SETS: groups in it (1: a group is a run or more).
 // SIGNS: infinite x give signed sums, and very large ones those of the weights themselves.  `blocks`: runs a wave takes.
-template <typename TT, int BITS, bool GPTQ, int STEPS, int SETS, bool SIGNS>
+template <typename TT, int BITS, bool GPTQ, int STEPS, int SETS, bool SIGNS, bool LOW>
 __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ qw,
                                                                       const uint32_t *__restrict__ qz, const uint16_t *__restrict__ sc,
                                                                       const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
@@ -203,7 +213,7 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
                     const int col = GPTQ ? c : i * CPW + (BITS == 4 ? awq_slot_col(s) : s);
                     const uint32_t zero = GPTQ ? ((zw[set][c >> 2] >> (BITS * ((c0 + (c & 3)) % CPW))) & ((1u << BITS) - 1u)) + 1u
                                                : (zw[set][i] >> (BITS * s)) & ((1u << BITS) - 1u);
-                    const float off = -(slab_bias<TT, BITS, GPTQ>(s % HALF) + (float)zero);
+                    const float off = -(slab_bias<TT, BITS, GPTQ, LOW>(s % HALF) + (float)zero);
                     float4_t p = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int st = set * ST; st < set * ST + ST; ++st) {
@@ -215,7 +225,7 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
                             uint32_t t[4];
 #pragma unroll
                             for (int j = 0; j < 4; ++j) t[j] = w[st][((s / HALF) * 4 + j) * W + i];
-                            slab_awq_operand<TT, BITS>(t, s % HALF, nm, bq);
+                            slab_awq_operand<TT, BITS, LOW>(t, s % HALF, nm, bq);
                         }
                         if constexpr (EXACT) {  // integers of at most 9 bits, 256 the only one of 9: exact in either type
 #pragma unroll
@@ -342,10 +352,10 @@ bool wna16_slab_takes(const oxq_ctx *ctx, const Wna16Problem &p) {
     return p.bits == 8 || p.dtype != OXQ_F16 || p.group_size < 128 || 2 * slab_tiles(p) >= 64;
 }
 
-template <typename TT, int BITS, bool GPTQ, int STEPS, int SETS, bool SIGNS = true>
+template <typename TT, int BITS, bool GPTQ, int STEPS, int SETS, bool SIGNS = true, bool LOW = false>
 static int slab_go(hipStream_t s, dim3 grid, const Wna16Problem &p, float *ws, int blocks) {
     const size_t lds = (size_t)SLAB_WAVES * 16 * 16 * ((p.M + 3) / 4) * 16;
-    hipLaunchKernelGGL((wna16_slab_kernel<TT, BITS, GPTQ, STEPS, SETS, SIGNS>), grid, dim3(SLAB_WAVES * 64), lds, s, (const uint16_t *)p.x, p.qweight,
+    hipLaunchKernelGGL((wna16_slab_kernel<TT, BITS, GPTQ, STEPS, SETS, SIGNS, LOW>), grid, dim3(SLAB_WAVES * 64), lds, s, (const uint16_t *)p.x, p.qweight,
                        p.qzeros, (const uint16_t *)p.scales, (const uint16_t *)p.bias, (uint16_t *)p.y, ws, (int)p.M, (int)p.K,
                        (int)p.N, p.group_shift, blocks);
     OXQ_HIP_CHECK(hipGetLastError());
@@ -362,6 +372,12 @@ static int slab_by_shape(hipStream_t s, dim3 grid, const Wna16Problem &p, float 
                                : slab_go<TT, 4, GPTQ, 4, 1, false>(s, grid, p, ws, blocks);
     }
     const bool g32 = p.group_size < 64;
+    if constexpr (TT::DTYPE == F16Traits::DTYPE && !GPTQ) {
+        if (p.bits == 4 && p.M == 1 && !awq_fast_ok(p))  // more rows: the tile kernel's
+            return g32        ? slab_go<TT, 4, GPTQ, 2, 2, true, true>(s, grid, p, ws, blocks)
+                   : run == 64 ? slab_go<TT, 4, GPTQ, 2, 1, true, true>(s, grid, p, ws, blocks)
+                               : slab_go<TT, 4, GPTQ, 4, 1, true, true>(s, grid, p, ws, blocks);
+    }
     if (p.bits == 8) return g32 ? slab_go<TT, 8, GPTQ, 2, 2>(s, grid, p, ws, blocks) : slab_go<TT, 8, GPTQ, 2, 1>(s, grid, p, ws, blocks);
     if (run == 128) return slab_go<TT, 4, GPTQ, 4, 1>(s, grid, p, ws, blocks);
     return g32 ? slab_go<TT, 4, GPTQ, 2, 2>(s, grid, p, ws, blocks) : slab_go<TT, 4, GPTQ, 2, 1>(s, grid, p, ws, blocks);

@@ -190,3 +190,26 @@ def test_large_finite_bf16_rows_do_not_overflow(method, bits, g):
     ref, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64.T)
     assert np.isfinite(y).all()
     assert (np.abs(y - ref) <= 2.0 ** -8 * np.abs(ref) + 2.0 ** -20 * mag).all()
+
+
+@pytest.mark.parametrize("method,bits,K,N,g,m", [("gptq", 4, 4096, 4096, 32, 4), ("gptq", 4, 4096, 4096, 64, 4),
+                                                 ("gptq", 8, 4096, 4096, 32, 4), ("awq", 4, 4096, 8192, 32, 1), ("awq", 4, 4096, 4104, 64, 1),
+                                                 ("awq", 8, 4096, 4096, 32, 4)])
+def test_f16_sums_are_as_exact_as_with_every_weight_by_itself(method, bits, K, N, g, m):
+    """Beyond the result's own rounding, errors of small outputs stay within the generic kernel's f32 sums: K products whose
+    partial sums lie near sqrt(K) of them, 2^-22 of the sum of the terms' magnitudes in all (a bias of 1024: up to 2^-20.5)."""
+    print(f"[case] slab f16 sums {method} {bits} K={K} g={g} m={m}", flush=True)
+    make = synth.gptq_checkpoint if method == "gptq" else synth.awq_checkpoint
+    qw, qz, sc = make(K, N, g, bits, seed=11)
+    s = oracle.round_through(sc, oracle.F16)
+    w = oracle.dequantize_gptq(qw, qz, s, bits) if method == "gptq" else (oracle.dequantize_awq if bits == 4 else oracle.dequantize_awq8)(qw, qz, s)
+    d = (to_dev(qw), to_dev(qz), to_dev(sc, torch.float16))
+    for mean in (0.0, 8.0):
+        x = (np.random.default_rng(5).standard_normal((m, K)) + mean).astype(np.float32)
+        xd = to_dev(x, torch.float16)
+        y = (ops.gptq_matmul(xd, *d, bits) if method == "gptq" else (ops.w4a16_matmul if bits == 4 else ops.w8a16_matmul)(xd, *d))
+        assert "_slab" in ops.default_context().last_plan()["kernel"]
+        x64, w64 = round_x(x, oracle.F16).astype(np.float64), w.reshape(N, K).astype(np.float64)
+        ref, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64.T)
+        over = np.abs(y.double().cpu().numpy() - ref) - 2.0 ** -11 * np.abs(ref)
+        assert (over <= 2.0 ** -22 * mag).all(), (over / mag).max()
