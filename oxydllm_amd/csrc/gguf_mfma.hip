@@ -657,6 +657,12 @@ template <bool INF, bool FOURS> __device__ __forceinline__ void ggm_split3(const
     }
 }
 
+// Waves a SIMD that an instantiation's registers have to leave room for.  Two workgroups of eight waves a compute unit are what
+// hides the waits of one to four rows on layers of more than one round of strips; Q6_K came out two registers over that (a row,
+// us, without / with room: 1024 x 9216 6.5 / 5.5, 4096 x 8704 12.3 / 10.8, 5632 x 7168 10.7 / 10.0).
+template <int FMT, int MT, int XQ, int NW, int NS, bool XF32>
+constexpr int ggm_waves = FMT == OXQ_GGUF_Q6_K && MT == 1 && XQ == 1 && NW == 8 && NS == 1 && !XF32 ? 4 : 1;
+
 // XF32: f32 activations and results.  An f32 value is the sum of three bf16 pieces, so four rows of x are twelve rows of
 // a matrix-core tile (piece p of row m in tile row 4 p + m) and the products stay exact; MT tiles take 4 MT rows of x,
 // XQ = 2 MT loads bring them.  The vector-ALU kernel on the rotated copy does the same work once per row.  XQ = 1: a single
@@ -665,9 +671,9 @@ template <bool INF, bool FOURS> __device__ __forceinline__ void ggm_split3(const
 // one by one, 4 - 16 roundings a chunk at the size of the whole sum, the formats with a minimum were 1.4 - 1.8 x as far from
 // 64 bits as the vector kernels at K = 14336 (Q4_K at 8 rows 1.7e-7 against 1.25e-7; now 1.0e-7, at up to 2.5 % of the time).
 template <int FMT, int MT, int XQ, int NW, int NS, bool XF32 = false>
-__global__ __launch_bounds__(NW * 64) void ggm_kernel(const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw,
-                                                      const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
-                                                      float *__restrict__ ws, int M, int K, int N, int cslice, int act) {
+__global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) void ggm_kernel(
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
+    float *__restrict__ ws, int M, int K, int N, int cslice, int act) {
     constexpr bool ONE = XF32 && XQ == 1;
     static_assert(!XF32 || XQ == 2 * MT || (ONE && MT == 1), "two loads a lane bring four rows' chunk of f32");
     constexpr int TROWS = XF32 ? 4 * MT : 16 * MT;  // rows of x a tile takes

@@ -75,3 +75,10 @@ def loads_under_way_at_barriers(code):
                 todo.append((index[target], flight))
             i += 1
     return at_barrier
+
+
+def registers(code_object):
+    """mangled name -> vector registers (both kinds) of each kernel."""
+    notes = subprocess.run([LLVM + "llvm-readelf", "--notes", str(code_object)], check=True, capture_output=True, text=True).stdout
+    found = re.findall(r"\.name: +(\S+)\n(?:(?!\.name:).)*?\.vgpr_count: +(\d+)", notes, re.S)
+    return {n: int(r) for n, r in found}
