@@ -279,7 +279,9 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     }
     // the split-K tiles are one workgroup a row tile and 64 columns, in whole rounds too (64-column strips: up to two of them,
     // beyond that fitted without; 1664 x 4224 f16 at 200 rows, 264 tiles, 15.4 us, 12.1 at 300 rows in the two-strip form)
-    const double c_split = (w64 < 1.0 ? c.split_lo : c.split_hi) * (p.w.strip == 16 || w64 <= 0.25 ? std::ceil(8.0 * w64 - 1e-9) / 8.0 : w64);
+    const double tiles = (double)(ceil_div(p.w.N, (int64_t)64) * ceil_div(p.M, (int64_t)64)) / cus;
+    const double c_split = (w64 < 1.0 ? c.split_lo : c.split_hi) *
+                           (p.w.strip == 16 ? std::ceil(8.0 * w64 - 1e-9) / 8.0 : tiles <= 2.0 ? std::ceil(tiles) / 8.0 : w64);
     // two strips a workgroup (128 KB of LDS: one a CU), whole rounds of `PK4_MID_ROUND` each
     const double w_mid = (double)(ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)2) * ceil_div(p.M, (int64_t)64)) / cus;
     const double c_mid = forced_ks == 1        ? 1e30

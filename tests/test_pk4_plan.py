@@ -57,3 +57,14 @@ def test_unrounded_layers_run_folded_forms_only(pack, bits, K, N, g, dt):
     rows = (1, 16, 17, 32, 33, 48, 49, 64, 65, 128, 200, 512, 1024, 2048, 4096, 1 << 20)
     for m, (kernel, _) in zip(rows, kernels(pack, bits, K, N, g, dt, rows)):
         assert "_gs" in kernel and "_mt4" not in kernel, (m, kernel)
+
+
+def test_narrow_layers_keep_the_tiles_that_fit_one_round():
+    """64-column strips x row tiles of 64 up to the compute units run as one round of split-K tiles, also where the strips are no
+    multiple of eight: 14 x 18, 12 x 17, 9 x 19 (8-bit: 10 x 20, 19 x 13).  One more round goes to the two-strip form."""
+    for bits, k, n, m, dt in [(4, 1408, 896, 1099, _lib.BF16), (4, 1664, 768, 1053, _lib.F16), (8, 1024, 576, 1170, _lib.BF16),
+                              (8, 5120, 640, 1257, _lib.F16), (4, 3840, 1216, 817, _lib.BF16)]:
+        (kernel, _), = kernels(ops.PACK_OUT, bits, k, n, 128, dt, (m,))
+        assert "_mfma_" in kernel, (k, n, m, kernel)
+    (kernel, _), = kernels(ops.PACK_OUT, 4, 1408, 896, 128, _lib.BF16, (1153,))  # 14 x 19
+    assert "_gemm_" in kernel, kernel
