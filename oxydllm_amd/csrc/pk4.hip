@@ -58,6 +58,8 @@
 #include "pk4_mfma.hpp"
 
 #include <algorithm>
+#include <numeric>
+#include <numeric>
 #include <type_traits>
 #include <cstdlib>
 
@@ -925,26 +927,84 @@ static const char *pk4_by_name(int mt, int rows_mt) {  // in a plan's name: row 
     return mt == rows_mt ? "" : mt == 1 ? "_by1" : mt == 2 ? "_by2" : "_by3";
 }
 
+// us of `n` row tiles a workgroup in `ks` slices of K, launches of one round: a fixed part by the row tiles, the chain of blocks by type,
+// bits and form, the weights through the L2s (a strip's workgroups stand on 8 / gcd(strips x slices, 8) XCDs), x, and the second
+// launch of K slices with their partials.  Fitted to 26000 launches of 6000 calls (17 - 900 rows, K 1024 - 14336, N 512 - 16384, all
+// groups), to 7 % rms.
+static double pk4_spread_cost(const Pk4Problem &p, int64_t strips, int n, int ks, bool fold) {
+    static const double START[4] = {3.3, 3.7, 4.7, 5.7};
+    static const double CHAIN[2][2][2][4] = {{{{1.2, 1.7, 1.75, 1.75}, {1.0, 1.3, 1.65, 1.65}}, {{1.55, 2.05, 2.15, 2.1}, {1.5, 1.85, 2.15, 2.15}}},
+                                             {{{1.55, 2.0, 1.95, 2.05}, {1.05, 1.3, 1.3, 1.3}}, {{1.8, 2.65, 2.5, 2.55}, {1.7, 2.0, 2.0, 2.0}}}};
+    const int sets = pk4_sets(p.w.group_shift);
+    const bool f16 = p.w.dtype == OXQ_F16;
+    const double k = (double)p.w.K, weights = (double)p.w.N * k * p.w.bits / 8e6, x = (double)strips * (double)p.M * k * 2e-6;
+    const double fine = sets == 1 ? 1.0 : sets == 2 ? (fold ? 1.2 : 1.1) : fold ? 1.5 : 1.2;
+    const int64_t xcds = 8 / std::gcd(strips * ks, (int64_t)8);
+    return START[n - 1] + (n == 4 && sets > 1 && f16 ? 1.2 : 0.0) + CHAIN[f16 ? 0 : 1][p.w.bits == 8][fold][n - 1] * fine * k / 1024.0 / ks +
+           0.037 * weights * (double)std::min(ceil_div(p.M, (int64_t)16 * n), xcds) + 0.02 * x +
+           (ks > 1 ? 1.9 + 0.45 * (double)p.M * (double)p.w.N * ks * 4e-6 : 0.0);
+}
+
 // Row tiles a workgroup takes of the `mt` that the rows come to, where the workgroups of `mt` would leave compute units idle: as
 // few as still fit one round.  A wave's chain of blocks gets shorter (fewer MFMAs, fewer rows of x) and nothing is paid for
 // it but the weights' second way out of L2.  Same form and same K split within a workgroup: the results do not change, unless
-// K slices are given up.  `ks` slices stay, or (0 returned in it) are given up where they fill the chip by themselves and K is
-// short enough that a workgroup does the whole of it in less than the slices' second launch takes; bf16 rows that convert
-// the weights for one or two row tiles lose by it.  Nor do 8-bit layers gain from two tiles of eight (2816 x 2944 f16 at 128 rows
-// 12.2 -> 12.7).
+// K slices are given up.
+// One row tile of more is ahead, but for 8-bit f16 layers of nearly a round of strips (4096 x 7424 at 18 rows 11.4 -> 13.3).  Two or three
+// are where a slice of K is short: the 64-row tile has the shorter step, and more workgroups read the weights more often.  A
+// strip's workgroups are `strips` x slices apart: where that is odd each of them has another XCD's L2 to fill, where it is a
+// multiple of eight none has (us, K slices kept, row tiles a workgroup of all -> 2 or 3, 64-column strips, f16: 23 strips, K = 13568 at 340 / 383
+// rows 34.0 -> 39.2, 33.9 -> 40.4; 31 strips, K = 8704 at 343 26.4 -> 29.1; 28 strips, K = 9216 at 393 28.0 -> 26.5; 11 strips, K = 3328
+// at 447 / 758 12.8 -> 12.0, 15.1 -> 15.6; 16-column strips, K = 10880 at 192 30.3 -> 33.3).  Over all of the calls above: beyond
+// the lines below 1.00 - 1.15 x the time, before them 0.75 - 0.96 x.  Nor do 8-bit layers gain from two tiles of eight (2816 x
+// 2944 f16 at 128 rows 12.2 -> 12.7).
+// Slices of K are given up (0 returned in `ks`) up to K = 4096, where the whole of it takes a workgroup less than the slices and their
+// second launch by the estimate above: f16 28 strips, 67 rows 9.6 -> 8.1, 41 strips, groups of 64, 127 rows 14.6 -> 11.7, bf16 44
+// strips, 74 rows 12.2 -> 10.0, 8-bit f16 48 strips, 66 rows 13.3 -> 9.2; but 8-bit with groups of 32 at up to 32 rows x 1.3 - 1.45.
 // us, a workgroup with all the rows / as chosen here (4-bit, unless said): 2304 x 3328 bf16 at 20 / 48 / 64 / 128 rows 7.5 / 9.4 /
 // 10.7 / 10.8 -> 6.8 / 6.9 / 6.9 / 8.1; 3840 x 3840 f16 at 20 / 64 rows 10.1 / 13.6 -> 7.9 / 8.7, bf16 at 128 rows 15.4 -> 11.8;
 // 1792 x 2112 f16, groups of 64, at 65 / 200 rows 11.1 / 11.5 -> 6.2 / 8.5; 8-bit 2816 x 2944 f16 at 64 rows 11.9 -> 10.0.
-// Slices given up: 4096 x 4096 f16 at 20 / 64 rows 7.4 / 11.4 -> 7.2 / 8.4, bf16 at 64 rows 11.9 -> 9.6 (at 20 rows 7.9 -> 9.5),
-// 4096 x 6144 f16 at 32 / 64 rows 9.9 / 13.7 -> 7.7 / 10.4; but 5632 x 2304 bf16 at 32 / 64 rows 8.2 / 11.3 -> 9.0 / 11.9.
-static int pk4_spread(const oxq_ctx *ctx, const Pk4Problem &p, int64_t strips, int mt, int *ks) {
+static int pk4_spread(const oxq_ctx *ctx, const Pk4Problem &p, int64_t strips, int mt, bool fold, int *ks) {
     if (p.M <= 16) return mt;
     const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-    auto fits = [&](int n, int slices) { return strips * ceil_div(p.M, (int64_t)16 * n) * slices <= cus; };
-    if (*ks > 1 && !fits(1, *ks) && p.w.K <= 4096 && (p.w.dtype == OXQ_F16 || p.M > 32) && fits(mt, 1)) *ks = 0;
-    int n = mt;
-    while (n > 1 && fits(n - 1, std::max(*ks, 1))) --n;
-    return p.w.bits == 8 && p.M > 64 && n > 1 ? mt : n;
+    const bool f16 = p.w.dtype == OXQ_F16, b8 = p.w.bits == 8, wide = p.w.strip != 16 && pk4_sets(p.w.group_shift) == 1;
+    auto groups = [&](int n) { return ceil_div(p.M, (int64_t)16 * n); };  // workgroups a strip and slice
+    auto fits = [&](int n, int slices) { return strips * groups(n) * slices <= cus; };
+    auto tiles = [&](int slices) {
+        int n = mt;
+        while (n > 1 && fits(n - 1, slices)) --n;
+        if (n == mt) return n;
+        const int64_t rows = ceil_div(p.w.K, (int64_t)slices);  // of a slice
+        const bool odd = (strips * slices) % 2 != 0 && groups(n) > groups(mt);
+        if (n == 1) return b8 && f16 && wide && mt == 2 && rows >= 4096 && (strips * slices > 96 || (odd && p.M > 64)) ? mt : n;
+        if (b8 && p.M > 64) return mt;
+        if ((strips * slices) % 8 == 0) return n;  // a strip's workgroups share an XCD
+        int64_t most = INT64_MAX;
+        if (p.w.strip == 16) {
+            if (n == 3) most = f16 ? 6144 : odd ? 8192 : INT64_MAX;
+        } else if (!wide) {  // groups of 64: no line found
+            if (pk4_sets(p.w.group_shift) == 4 && n == 3 && f16) most = odd ? 4096 : 8192;
+            else if (pk4_sets(p.w.group_shift) == 4 && mt == 3 && !fold && odd) most = 4096;
+        } else if (b8) {
+            most = odd ? 3072 : 4096;
+        } else if (mt == 3) {
+            if (!fold && odd) most = 3072;
+        } else if (f16) {
+            most = odd ? (n == 2 ? 3840 : 3072) : n == 2 ? 8192 : 6144;
+        } else if (odd) {
+            most = 5120;
+        }
+        return rows > most ? mt : n;
+    };
+    const int n = tiles(*ks);
+    if (*ks > 1 && p.w.K <= 4096 && fits(mt, 1) && !(b8 && strips % 2 != 0)) {
+        const int n1 = tiles(1);
+        if (!(b8 && p.M > 64 && n1 != 1 && n1 != mt) &&
+            pk4_spread_cost(p, strips, n1, 1, fold) < pk4_spread_cost(p, strips, n, *ks, fold)) {
+            *ks = 0;
+            return n1;
+        }
+    }
+    return n;
 }
 
 template <typename TT, int BITS>
@@ -1078,18 +1138,17 @@ static int launch_pk4n_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p)
     if (tiles <= 96 && NB >= 32) ks = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tiles, NB / 8));
     else if (ns == 4 && tiles <= 128 && NB >= 64) ks = 2;  // as in the wide form; 128 single strips are faster whole
                                                            // (8192 x 2048 at one row: 5.20 against 5.65 us)
-    if (p.no_split) ks = 1;
     const bool spread = tune(ctx, OXQ_TUNE_PK4_KS, 0) == 0;
-    const int mt = spread ? pk4_spread(ctx, p, N / (16 * ns), rows_mt, &ks) : rows_mt;
-    if (!spread) ks = p.no_split ? 1 : tune(ctx, OXQ_TUNE_PK4_KS, 0);
-    ks = std::max(1, std::min(ks, NB));
+    ks = p.no_split ? 1 : std::max(1, std::min(spread ? ks : tune(ctx, OXQ_TUNE_PK4_KS, 0), NB));
     while (ks > 1 && (size_t)ks * M * N * 4 > ctx->workspace_bytes) --ks;
+    const bool fold = rows_mt <= 2 && pk4_folds(ctx, p, rows_mt);  // three row tiles of folded sums do not fit beside the two-block ring
+    const int mt = spread ? pk4_spread(ctx, p, N / (16 * ns), rows_mt, fold, &ks) : rows_mt;
+    ks = std::max(1, ks);
     const int bslice = (int)ceil_div(NB, ks);
     ks = (int)ceil_div(NB, bslice);
     if (ceil_div(M, 16 * mt) > 65535)
         return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid limit (65535 row tiles)", (long long)M);
     if (p.act) return fail(OXQ_ERR_ARG, "repacked matmul: a fused activation on a layer in 16-column strips");
-    const bool fold = rows_mt <= 2 && pk4_folds(ctx, p, rows_mt);  // three row tiles of folded sums do not fit beside the two-block ring
     dim3 grid((unsigned)(N / (16 * ns)), (unsigned)ks, (unsigned)ceil_div(M, 16 * mt));
     // One or two rows of a single strip on a long K: 16 waves, so that a wave's chain of blocks is half as
     // long (f16, one / two rows, 8 -> 16 waves: 14336 x 4096 7.44 / 7.55 -> 7.00 / 7.37 us, 8192 x 2048 at one
@@ -1146,12 +1205,12 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     // launch costs more than the slices save (4096 x 8192: 6.7 / 7.8 / 13.5 against 7.0 / 8.0 / 14.9 us).
     else if (tiles <= 128 && NB >= 64) ks = 2;
     const bool whole = p.act || p.no_split;  // the activation needs the whole sum: gate|up layers are wide, one slice fills the chip
-    if (whole) ks = 1;
     const bool spread = tune(ctx, OXQ_TUNE_PK4_KS, 0) == 0;
-    const int mt = spread ? pk4_spread(ctx, p, strips, rows_mt, &ks) : rows_mt;
-    if (!spread) ks = whole ? 1 : tune(ctx, OXQ_TUNE_PK4_KS, 0);
-    ks = std::max(1, std::min(ks, NB));
+    ks = whole ? 1 : std::max(1, std::min(spread ? ks : tune(ctx, OXQ_TUNE_PK4_KS, 0), NB));
     while (ks > 1 && (size_t)ks * M * p.w.N * 4 > ctx->workspace_bytes) --ks;
+    const bool fold = pk4_folds(ctx, p, rows_mt);
+    const int mt = spread ? pk4_spread(ctx, p, strips, rows_mt, fold, &ks) : rows_mt;
+    ks = std::max(1, ks);
     const int bslice = (int)ceil_div(NB, ks);
     ks = (int)ceil_div(NB, bslice);  // no empty slice
     if (ceil_div(M, 16 * mt) > 65535)
@@ -1190,7 +1249,6 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
         else
             front = (front_mode != 2 && bslice == 32 && ks == 1) ? 1 : (bslice % 8 == 0 && share8 <= 8 && share8 != 7) ? 2 : 0;
     }
-    const bool fold = pk4_folds(ctx, p, rows_mt);
     snprintf(name, sizeof name, "pk%d_mfma_%s_mt%d%s%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows_mt,
              fold ? "_gs" : "", sets == 2 ? "_g64" : sets == 4 ? "_g32" : "", front == 1 ? "_front" : front == 2 ? "_line" : "",
              pk4_by_name(mt, rows_mt), p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");

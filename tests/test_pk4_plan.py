@@ -68,3 +68,37 @@ def test_narrow_layers_keep_the_tiles_that_fit_one_round():
         assert "_mfma_" in kernel, (k, n, m, kernel)
     (kernel, _), = kernels(ops.PACK_OUT, 4, 1408, 896, 128, _lib.BF16, (1153,))  # 14 x 19
     assert "_gemm_" in kernel, kernel
+
+
+def k_slices(pack, bits, K, N, g, dt, m):
+    lib, plan = _lib.load(), ops.Context(plan_only=True)
+    pf = 32 // bits
+    h = C.c_void_p()
+    assert lib.oxq_packed_quant_linear_new(plan.handle, bits, pack, C.byref(fake((K, N // pf) if pack == ops.PACK_OUT else (K // pf, N), _lib.I32)),
+                                           C.byref(fake((K // g, N // pf), _lib.I32)), C.byref(fake((K // g, N), dt)), None, dt, C.byref(h)) == 0
+    assert lib.oxq_packed_quant_linear_forward(h, None, C.byref(fake((m, K), dt)), C.byref(fake((m, N), dt))) == 0
+    lib.oxq_packed_quant_linear_free(h)
+    return plan.last_plan()["kernel"], plan.last_plan()["split_k"]
+
+
+def test_k_slices_stay_where_a_whole_k_a_workgroup_takes_longer():
+    """K = 4096, row tiles of few strips: up to 1.45 x the time in 8-bit layers and groups of 32 without their slices."""
+    for bits, n, g, m, dt in [(8, 3072, 32, 30, _lib.F16), (8, 1536, 64, 30, _lib.F16), (8, 768, 128, 30, _lib.BF16), (4, 1152, 32, 60, _lib.BF16),
+                              (8, 704, 128, 164, _lib.BF16), (4, 4096, 128, 20, _lib.BF16)]:
+        kernel, ks = k_slices(ops.PACK_OUT, bits, 4096, n, g, dt, m)
+        assert ks >= 2, (bits, n, g, m, kernel)
+    for bits, n, g, m, dt in [(4, 1792, 128, 67, _lib.F16), (4, 2816, 64, 74, _lib.BF16), (8, 3072, 128, 66, _lib.F16), (4, 4096, 128, 64, _lib.F16)]:
+        kernel, ks = k_slices(ops.PACK_OUT, bits, 4096, n, g, dt, m)
+        assert ks == 1 and "_by" in kernel, (bits, n, g, m, kernel)
+
+
+def test_row_tiles_stay_together_on_long_chains():
+    """Two or three row tiles a workgroup in the place of four: not where a workgroup's K is long and a strip's workgroups stand on
+    all XCDs."""
+    for k, n, m, dt in [(13568, 1472, 383, _lib.F16), (8704, 1984, 343, _lib.F16), (8064, 832, 564, _lib.F16), (10880, 3712, 192, _lib.F16),
+                        (12544, 2624, 256, _lib.BF16), (7680, 2824, 197, _lib.F16), (4096, 5512, 42, _lib.BF16)]:
+        (kernel, _), = kernels(ops.PACK_OUT, 4, k, n, 128, dt, (m,))
+        assert "_by" not in kernel, (k, n, m, kernel)
+    for k, n, m, dt in [(9216, 2048, 340, _lib.F16), (1664, 960, 615, _lib.F16), (3200, 1024, 677, _lib.F16), (9600, 2768, 185, _lib.BF16), (2304, 3328, 128, _lib.BF16)]:
+        (kernel, _), = kernels(ops.PACK_OUT, 4, k, n, 128, dt, (m,))
+        assert "_by" in kernel, (k, n, m, kernel)
