@@ -506,12 +506,23 @@ int oxq_ctx_reset_tuning(oxq_ctx *ctx, const char *name) {
     return OXQ_OK;
 }
 
+static void ctx_delete(oxq_ctx *ctx) {
+    if (ctx->second_copies) ctx->second_copies->give_back(0);
+    delete ctx;
+}
+
 int oxq_ctx_create(int device, oxq_ctx **out) {
     if (!out) return fail(OXQ_ERR_ARG, "oxq_ctx_create: out is NULL");
     *out = nullptr;
     oxq_ctx *ctx = new (std::nothrow) oxq_ctx();
     if (!ctx) return fail(OXQ_ERR_RUNTIME, "oxq_ctx_create: out of host memory");
     memset(ctx, 0, sizeof *ctx);
+    ctx->second_copies = new (std::nothrow) oxq_copy_bytes();
+    if (!ctx->second_copies) {
+        ctx_delete(ctx);
+        return fail(OXQ_ERR_RUNTIME, "oxq_ctx_create: out of host memory");
+    }
+    ctx->device_bytes = (size_t)288 << 30;
     ctx->device = device;
     ctx->plan_only = device == OXQ_DEVICE_PLAN_ONLY;
     ctx->num_cus = 256;
@@ -532,7 +543,7 @@ int oxq_ctx_create(int device, oxq_ctx **out) {
     int count = 0;
     hipError_t e = hipGetDeviceCount(&count);
     if (e != hipSuccess || device < 0 || device >= count) {
-        delete ctx;
+        ctx_delete(ctx);
         return fail(OXQ_ERR_DEVICE, "oxq_ctx_create: no HIP device %d (%d visible%s%s)", device,
                     count, e != hipSuccess ? ": " : "", e != hipSuccess ? hipGetErrorString(e) : "");
     }
@@ -545,6 +556,8 @@ int oxq_ctx_create(int device, oxq_ctx **out) {
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
             cus > 0)
             ctx->num_cus = cus;
+        size_t mem = 0;
+        if (hipDeviceTotalMem(&mem, device) == hipSuccess && mem > 0) ctx->device_bytes = mem;
         if ((e = hipMalloc(&ctx->workspace, ctx->workspace_bytes)) != hipSuccess) break;
         if ((e = hipMalloc((void **)&ctx->counters, ctx->n_counters * sizeof(unsigned))) != hipSuccess)
             break;
@@ -558,14 +571,14 @@ int oxq_ctx_create(int device, oxq_ctx **out) {
     if (e == hipSuccess && rc != OXQ_OK) {  // scratch_lookup has set the message
         (void)hipFree(ctx->workspace);
         (void)hipFree(ctx->counters);
-        delete ctx;
+        ctx_delete(ctx);
         return rc;
     }
     if (e != hipSuccess) {
         rc = fail(OXQ_ERR_RUNTIME, "oxq_ctx_create: %s", hipGetErrorString(e));
         if (ctx->workspace) (void)hipFree(ctx->workspace);
         if (ctx->counters) (void)hipFree(ctx->counters);
-        delete ctx;
+        ctx_delete(ctx);
         return rc;
     }
     *out = ctx;
@@ -581,7 +594,7 @@ int oxq_ctx_destroy(oxq_ctx *ctx) {
         if (ctx->workspace) (void)hipFree(ctx->workspace);
         if (ctx->counters) (void)hipFree(ctx->counters);
     }
-    delete ctx;
+    ctx_delete(ctx);
     return OXQ_OK;
 }
 
@@ -2038,8 +2051,27 @@ struct oxq_qlinear {
     void *rot = nullptr;    // the rotated copy of the vector GEMV, or null
     void *mm = nullptr;     // the copy in the matrix-core layout, or null (large f32 layers hold both)
     bool rotated = false, mfma = false;
+    oxq_copy_bytes *second = nullptr;  // where the bytes of a second copy are counted, or null
+    size_t second_bytes = 0;
     int act = 0;            // 0, or 1 + oxq_gated_act of a fused gate|up layer (matrix-core copy only)
 };
+
+// Q2_K and Q3_K hold a second copy for speed alone, and are chosen to save memory: all of a ctx's layers may hold a 32nd of the
+// device's memory in such copies (9 GB: 29 billion weights of Q2_K, 21 of Q3_K), in the order they are built, so that
+// a model that fits with one copy a layer does not run out for the second ones.  The others run as with OXQ_GGUF_MFMA=0.
+// OXQ_GGUF_BOTH_MB: that many MB instead.
+static bool take_second_copy(oxq_qlinear *l) {
+    oxq_ctx *ctx = l->ctx;
+    const int mb = tune(ctx, OXQ_TUNE_GGUF_BOTH_MB, -1);
+    const size_t bytes = gguf_mfma_bytes(l->quant, l->in_features, l->out_features);
+    if (!ctx->second_copies->take(bytes, mb >= 0 ? (size_t)mb << 20 : ctx->device_bytes / 32)) return false;
+    l->second = ctx->second_copies, l->second_bytes = bytes;
+    return true;
+}
+static void give_back_second_copy(oxq_qlinear *l) {
+    if (l->second) l->second->give_back(l->second_bytes);
+    l->second = nullptr;
+}
 
 // linear.rs:225-240: the fast path copies the block bytes at build; here the copy is strip-major
 static int build_resident_gguf(oxq_qlinear *l) {
@@ -2051,6 +2083,7 @@ static int build_resident_gguf(oxq_qlinear *l) {
     l->mfma = gguf_mfma_layer(ctx, l->quant, l->in_features, l->out_features, l->out_dtype) &&
               !(l->act && (l->out_features % 16 != 0 || l->out_dtype != OXQ_BF16 || !gguf_mfma_alone(ctx, l->quant, l->out_dtype)));
     l->rotated = !(l->mfma && gguf_mfma_alone(ctx, l->quant, l->out_dtype)) && gguf_res_eligible(l->quant, l->in_features, l->out_features);
+    if (l->mfma && l->rotated && (l->quant == OXQ_GGUF_Q2_K || l->quant == OXQ_GGUF_Q3_K)) l->mfma = take_second_copy(l);
     if (!l->mfma && !l->rotated) return OXQ_OK;
     if (l->act && !l->mfma) return OXQ_OK;  // the caller reports it
     if (ctx->plan_only) {
@@ -2066,6 +2099,7 @@ static int build_resident_gguf(oxq_qlinear *l) {
     if (e != hipSuccess && l->rotated && l->mfma) {  // no room for both: the rotated copy serves every row it did alone
         (void)hipGetLastError();
         l->mfma = false;
+        give_back_second_copy(l);
         e = hipMalloc(&l->res, rot_bytes);
     }
     if (e != hipSuccess) {
@@ -2453,6 +2487,7 @@ int oxq_qlinear_dequantize(oxq_qlinear *l, void *stream, const oxq_tensor *out) 
 void oxq_qlinear_free(oxq_qlinear *l) {
     if (!l) return;
     if (l->res) (void)hipFree(l->res);  // by address: the layer may outlive its ctx
+    give_back_second_copy(l);
     delete l;
 }
 

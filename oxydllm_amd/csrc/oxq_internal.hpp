@@ -18,7 +18,7 @@
 // call costs no getenv and two engine threads cannot race on the process environment.
 #define OXQ_TUNE_LIST(X)                                                                                      \
     X(ACT_VEC) X(F8_FORM) X(F8_MM_KS) X(F8_MM_MIN_M) X(F8_MM_MT) X(F8_SLICES) X(FORCE_GENERIC) X(GEMV_CFG) X(GEMV_GPW) X(GEMV_TILE)   \
-    X(GGR_GRID) X(GGR_WAVES) X(GGUF_BIG_LDS) X(GGUF_GEMM_KS) X(GGUF_GEMM_MIN_M) X(GGUF_GEMM_SLICES) X(GGUF_MFMA)                  \
+    X(GGR_GRID) X(GGR_WAVES) X(GGUF_BIG_LDS) X(GGUF_GEMM_KS) X(GGUF_GEMM_MIN_M) X(GGUF_GEMM_SLICES) X(GGUF_MFMA) X(GGUF_BOTH_MB)   \
     X(GGUF_MFMA_MAX_M) X(GGUF_MFMA_NS) X(GGUF_MM_KS) X(GGUF_MM_MIN_M) X(GGUF_MM_MT) X(GGUF_PW) X(GGUF_RPWG)   \
     X(GPTQ_TILE) X(GPTQ_TILE_KS) X(MFMA_MT) X(MFMA_SPLITK) X(MFMA_VARIANT) X(MXFP4_FR) X(MXFP4_GEMM_MIN_PAIRS) \
     X(MXFP4_GEMM_ROWS) X(MXFP4_MM)      \
@@ -33,6 +33,23 @@ enum oxq_tune_key {
 };
 constexpr int OXQ_TUNE_UNSET = -2147483647 - 1;
 
+// Bytes of second copies that the GGUF layers of a ctx hold (build_resident_gguf).  The ctx and each such layer have a share in the
+// count: a layer may outlive its ctx.
+struct oxq_copy_bytes {
+    std::atomic<size_t> held{0};
+    std::atomic<int> shares{1};
+    bool take(size_t bytes, size_t most) {
+        size_t now = held.load();
+        while (now <= most && bytes <= most - now)
+            if (held.compare_exchange_weak(now, now + bytes)) return ++shares, true;
+        return false;
+    }
+    void give_back(size_t bytes) {
+        held -= bytes;
+        if (--shares == 0) delete this;
+    }
+};
+
 struct oxq_ctx {
     int device;             // HIP ordinal, or OXQ_DEVICE_PLAN_ONLY
     bool plan_only;
@@ -45,6 +62,8 @@ struct oxq_ctx {
     oxq_plan plan;
     struct oxq_weight_cache *wcache;  // tile-major copies the stateless ops made (opt-in), or null
     size_t wcache_limit;              // bytes the cache may hold; 0 = off
+    oxq_copy_bytes *second_copies;    // of Q2_K / Q3_K layers
+    size_t device_bytes;              // the device's memory
     int tuning[OXQ_TUNE_COUNT];       // tuning switches (OXQ_TUNE_UNSET = the launcher's own default)
 };
 
