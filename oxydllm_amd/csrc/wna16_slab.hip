@@ -25,18 +25,20 @@ namespace oxq {
 
 constexpr int SLAB_COLS = 256, SLAB_WAVES = 4;
 
-// B operands hold bias + q: the bias.  In f16 the bias takes bits of the sums: 1024 beside four-bit codes left errors of small
+// B operands hold bias + q: the bias.  It takes bits of the sums: 1024 beside four-bit codes in f16 left errors of small
 // outputs three times those of weights multiplied one by one (1e-6 against 3e-7 of the sum of the terms' magnitudes at K =
-// 4096), 64 leaves none to be seen.  GPTQ has it for nothing.  For AWQ it is two shifts more (4096 x 14336, groups of 32, 13.3 ->
-// 13.6 us), and LOW asks for it: calls that otherwise run the generic kernel, not those whose weights the tile kernel rounds or that
-// the dot products bias as here.
+// 4096), 64 leaves none to be seen; 128 in bf16 four to five times as many results that are not the nearest bf16 (9e-4 of them
+// against 2e-4 at 4096 x 14336, 4 rows), 16 fewer (1e-4).  They cost a shift more a word (up to 2 %).  Without
+// LOW two forms keep 1024 and 128, no further off than the kernels that took those calls before: f16 AWQ of more than one row (two
+// shifts, 4096 x 14336, groups of 32, 13.3 -> 13.6 us), whose weights the tile kernel rounds, and bf16 GPTQ in runs of 128 (5120 x
+// 13832, 2 rows, 16.4 -> 17.6 us), where the dot products left 6e-4.
 template <typename TT, int BITS, bool GPTQ, bool LOW> __device__ __forceinline__ constexpr float slab_bias(int s) {
-    if (TT::DTYPE != F16Traits::DTYPE) return BITS == 4 ? 128.f : 0.f;
-    return BITS == 4 && (GPTQ || LOW || (s & 1)) ? 64.f : 1024.f;
+    if (TT::DTYPE != F16Traits::DTYPE) return BITS == 8 ? 0.f : GPTQ && !LOW ? 128.f : 16.f;
+    return BITS == 8 ? 256.f : GPTQ || LOW || (s & 1) ? 64.f : 1024.f;
 }
 // bytes 0 and 2 of t, or 1 and 3
 template <typename TT> __device__ __forceinline__ uint32_t slab_bytes(uint32_t t, bool high) {
-    if constexpr (TT::DTYPE == F16Traits::DTYPE) return ((high ? t >> 8 : t) & 0x00FF00FFu) | 0x64006400u;
+    if constexpr (TT::DTYPE == F16Traits::DTYPE) return ((high ? t >> 6 : t << 2) & 0x03FC03FCu) | 0x5C005C00u;
     const float lo = high ? (float)((t >> 8) & 0xFFu) : (float)(t & 0xFFu), hi = high ? (float)(t >> 24) : (float)((t >> 16) & 0xFFu);
     return perm_b32(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);  // 8 bits: exact
 }
@@ -53,18 +55,19 @@ __device__ __forceinline__ void slab_awq_operand(const uint32_t (&t)[4], int s, 
             const uint32_t u = s < 2 ? t[p] : t[p] >> 8;
             b[p] = s & 1 ? (u & nm.m1) | 0x54005400u : (u & nm.m0) | 0x64006400u;
         } else {
-            b[p] = ((t[p] >> (4 * s)) & nm.m0) | 0x43004300u;
+            b[p] = ((s ? t[p] >> (4 * s - 3) : t[p] << 3) & nm.m0) | 0x41804180u;
         }
     }
 }
 // GPTQ: eight rows of one column, in the order that slab_gptq_x gives x
-template <typename TT, int BITS> __device__ __forceinline__ void slab_gptq_operand(uint32_t w0, uint32_t w1, const NibbleMasks &nm, uint32_t (&b)[4]) {
+template <typename TT, int BITS, bool LOW> __device__ __forceinline__ void slab_gptq_operand(uint32_t w0, uint32_t w1, const NibbleMasks &nm, uint32_t (&b)[4]) {
     if constexpr (BITS == 8) {
         b[0] = slab_bytes<TT>(w0, false), b[1] = slab_bytes<TT>(w0, true), b[2] = slab_bytes<TT>(w1, false), b[3] = slab_bytes<TT>(w1, true);
     } else {
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             if constexpr (TT::DTYPE == F16Traits::DTYPE) b[n] = ((n ? w0 >> (4 * n - 4) : w0 << 4) & nm.m1) | 0x54005400u;
+            else if constexpr (LOW) b[n] = ((n ? w0 >> (4 * n - 3) : w0 << 3) & nm.m0) | 0x41804180u;
             else b[n] = ((w0 >> (4 * n)) & nm.m0) | 0x43004300u;
         }
     }
@@ -108,7 +111,7 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
     auto vo_z = [&](int j) { return exists(j) ? (c0 + (GPTQ ? 64 * j : 0)) / CPW * 4 : OOB; };
     auto vo_s = [&](int j) { return exists(j) ? (c0 + (GPTQ ? 64 * j : 0)) * 2 : OOB; };
     const int vo_x = ni < M ? (ni * K + 8 * kb) * 2 : OOB;
-    const NibbleMasks nm = nibble_masks();
+    const NibbleMasks nm = F16 || (GPTQ && !LOW) ? nibble_masks() : NibbleMasks{vgpr_const(0x00780078u), 0u};
 
     float4_t acc[16];
 #pragma unroll
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(SLAB_WAVES * 64, 2) void wna16_slab_kernel(const ui
                         const uint32_t a[4] = {xa[st][0], xa[st][1], xa[st][2], xa[st][3]};
                         uint32_t bq[4];
                         if constexpr (GPTQ) {
-                            slab_gptq_operand<TT, BITS>(w[st][c * WR], w[st][c * WR + WR - 1], nm, bq);
+                            slab_gptq_operand<TT, BITS, LOW>(w[st][c * WR], w[st][c * WR + WR - 1], nm, bq);
                         } else {
                             uint32_t t[4];
 #pragma unroll
@@ -373,14 +376,14 @@ static int slab_by_shape(hipStream_t s, dim3 grid, const Wna16Problem &p, float 
     }
     const bool g32 = p.group_size < 64;
     if constexpr (TT::DTYPE == F16Traits::DTYPE && !GPTQ) {
-        if (p.bits == 4 && p.M == 1 && !awq_fast_ok(p))  // more rows: the tile kernel's
+        if (p.bits == 4 && p.M == 1)  // more rows: the tile kernel's
             return g32        ? slab_go<TT, 4, GPTQ, 2, 2, true, true>(s, grid, p, ws, blocks)
                    : run == 64 ? slab_go<TT, 4, GPTQ, 2, 1, true, true>(s, grid, p, ws, blocks)
                                : slab_go<TT, 4, GPTQ, 4, 1, true, true>(s, grid, p, ws, blocks);
     }
     if (p.bits == 8) return g32 ? slab_go<TT, 8, GPTQ, 2, 2>(s, grid, p, ws, blocks) : slab_go<TT, 8, GPTQ, 2, 1>(s, grid, p, ws, blocks);
     if (run == 128) return slab_go<TT, 4, GPTQ, 4, 1>(s, grid, p, ws, blocks);
-    return g32 ? slab_go<TT, 4, GPTQ, 2, 2>(s, grid, p, ws, blocks) : slab_go<TT, 4, GPTQ, 2, 1>(s, grid, p, ws, blocks);
+    return g32 ? slab_go<TT, 4, GPTQ, 2, 2, true, GPTQ>(s, grid, p, ws, blocks) : slab_go<TT, 4, GPTQ, 2, 1, true, GPTQ>(s, grid, p, ws, blocks);
 }
 
 int launch_wna16_slab(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {

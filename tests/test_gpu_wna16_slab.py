@@ -213,3 +213,28 @@ def test_f16_sums_are_as_exact_as_with_every_weight_by_itself(method, bits, K, N
         ref, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64.T)
         over = np.abs(y.double().cpu().numpy() - ref) - 2.0 ** -11 * np.abs(ref)
         assert (over <= 2.0 ** -22 * mag).all(), (over / mag).max()
+
+
+# A f32 error of e moves the rounding of a share 2 e / ulp of the results.  Beside a bias of at most the codes' own range (16 in
+# bf16, 64 / 256 in f16) a result's sums are off by a few 2^-24 of it: 2^-13 to 2^-12 of the results in bf16, eight times that
+# share in f16; beside 128, or 1024, four times as many and more.
+@pytest.mark.parametrize("dtn,method,bits,K,N,g,m,most", [
+    ("bf16", "awq", 4, 4096, 14336, 128, 4, 4e-4), ("bf16", "awq", 4, 4096, 4096, 32, 8, 4e-4), ("bf16", "gptq", 4, 4096, 4096, 64, 16, 4e-4),
+    ("f16", "awq", 8, 4096, 4096, 32, 4, 3e-3), ("f16", "gptq", 8, 4096, 4096, 64, 8, 3e-3), ("f16", "awq", 4, 4096, 4096, 128, 1, 8e-3)])
+def test_nearly_all_results_are_the_nearest(dtn, method, bits, K, N, g, m, most):
+    print(f"[case] slab nearest {dtn} {method} {bits} K={K} N={N} g={g} m={m}", flush=True)
+    dt = DT[dtn]
+    qw, qz, sc = (synth.gptq_checkpoint if method == "gptq" else synth.awq_checkpoint)(K, N, g, bits, seed=11)
+    s = oracle.round_through(sc, dt)
+    w = oracle.dequantize_gptq(qw, qz, s, bits) if method == "gptq" else (oracle.dequantize_awq if bits == 4 else oracle.dequantize_awq8)(qw, qz, s)
+    d = (to_dev(qw), to_dev(qz), to_dev(sc, TORCH_DT[dt]))
+    w64 = torch.from_numpy(w.reshape(N, K)).cuda().double()
+    for mean in (0.0, 4.0):
+        xd = to_dev((np.random.default_rng(5).standard_normal((m, K)) + mean).astype(np.float32), TORCH_DT[dt])
+        if m > 8:
+            y = ops.mpp_quant_matmul(xd, *d, bits, ops.PACK_IN if method == "gptq" else ops.PACK_OUT)
+        else:
+            y = ops.gptq_matmul(xd, *d, bits) if method == "gptq" else (ops.w4a16_matmul if bits == 4 else ops.w8a16_matmul)(xd, *d)
+        assert "_slab" in ops.default_context().last_plan()["kernel"], ops.default_context().last_plan()
+        off = (y != (xd.double() @ w64.T.contiguous()).to(y.dtype)).double().mean().item()
+        assert off <= most, (mean, off)
