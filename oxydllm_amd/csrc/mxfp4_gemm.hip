@@ -3,12 +3,12 @@
 //
 // The copy (mxfp4_repack_kernel) stores a tile of 16 weight rows as chunks of 1 KB - 128 elements of K, lane
 // (ni, kb) the 16 bytes of block 4 c + kb of row ni, whose four words are the chunk's four MFMA steps - which is
-// the shape of a block of the 16-column AWQ layout.  So a workgroup takes 64 rows of one expert's pairs and, a wave,
+// the shape of a block of the 16-column AWQ layout.  So a workgroup takes 16 rows of one expert's pairs and, a wave,
 // four neighbouring tiles (64 weight rows = 64 columns of y): the pairs' rows of x come from global memory straight
 // into LDS (gathered through the token list, a chunk of K at a time, two buffers, one barrier a chunk), every wave
 // streams its tiles through a ring of two chunks, turns a word into an MFMA B fragment with four
 // v_cvt_scalef32_pk_bf16_fp4 (the values are exact in bf16, so this is the tile matmul's B) and keeps the whole K in
-// its accumulators: mxfp4_gemm_kernel, row tiles of 16, for few pairs an expert.  With more, mxfp4_wide_kernel below.
+// its accumulators: mxfp4_gemm_kernel, for few pairs an expert.  With more, mxfp4_wide_kernel below.
 // (The K split inside the workgroup that serves AWQ layers at mid sizes was slower than either at every pair count: with
 // 32 experts there are always enough workgroups.)
 #include "oxq_device.hpp"
@@ -22,15 +22,13 @@ namespace oxq {
 
 constexpr int MXG_WAVES = 8;
 
-template <int MT>
 __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw,
                                                          const unsigned char *__restrict__ ps, const uint16_t *__restrict__ bias,
                                                          uint16_t *__restrict__ y, const int32_t *__restrict__ offsets,
                                                          const int32_t *__restrict__ token_ids, int K, int N, int NC, int NG,
                                                          int E, uint32_t x_bytes, int swiglu, float limit) {
     typedef MfmaOps<BF16Traits> Ops;
-    constexpr int ROWS = 16 * MT, XBUF = ROWS * 256;
-    constexpr int XV = ROWS >= 32 ? ROWS / 32 : 1;  // loads of x a wave issues per chunk: 4 rows each (16 rows: waves 0..3 only)
+    constexpr int ROWS = 16, XBUF = ROWS * 256;
     constexpr int OOB = 0x7FFFFF00;
     extern __shared__ __attribute__((aligned(16))) unsigned char mxg_lds[];
 
@@ -56,37 +54,28 @@ __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restr
     const __amdgpu_buffer_rsrc_t rs_s = make_rsrc(ps + et * NG * 256, live ? (uint32_t)live_tiles * (uint32_t)NG * 256u : 0u);
     const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x, x_bytes);
     const int voff_w = lane * 16, voff_s = lane * 4;
-    // x: load q of a wave brings rows 4 (XV wave + q) .. + 3 of a chunk straight into LDS, lane l the 16 bytes that
-    // belong at position l % 16 of row l / 16.  Piece p = 4 kb + st of a row's 128 elements (what lane group kb reads
-    // in step st) is kept at position (4 st + kb) ^ (row % 16): the four lane groups of a fragment read then start in
+    // x: waves 0 .. 3 bring rows 4 wave .. + 3 of a chunk straight into LDS, lane l the 16 bytes that belong at position
+    // l % 16 of row l / 16.  Piece p = 4 kb + st of a row's 128 elements (what lane group kb reads in step st) is kept at position (4 st + kb) ^ (row % 16): the four lane groups of a fragment read then start in
     // different banks (at position p ^ row, groups 0 and 2 would meet 128 bytes apart: four conflict cycles a read).
     // Rows past the expert's pairs, and the elements past K in the last chunk, get an offset beyond the descriptor:
     // LDS receives zeros.
-    int xo[XV], xc[XV];
-#pragma unroll
-    for (int q = 0; q < XV; ++q) {
-        const int r = 4 * (wave * XV + q) + (lane >> 4);
-        const int m = m0 + r;
-        const int pos = (lane & 15) ^ (r & 15);
-        xc[q] = ((pos & 3) << 2) | (pos >> 2);  // the piece kept at this position
-        int src = 0;
-        if (m < m_end) src = token_ids ? token_ids[m] : m;
-        xo[q] = m < m_end ? src * K * 2 + (xc[q] << 4) : OOB;
-    }
-    // fragment of step st, row tile mt (+ 4096 mt): row ni, elements 32 kb + 8 st .. + 7 of the chunk = piece 4 kb + st
+    const int r = 4 * wave + (lane >> 4), m = m0 + r, pos = (lane & 15) ^ (r & 15);
+    const int xc = ((pos & 3) << 2) | (pos >> 2);  // the piece kept at this position
+    int src = 0;
+    if (m < m_end) src = token_ids ? token_ids[m] : m;
+    const int xo = m < m_end ? src * K * 2 + (xc << 4) : OOB;
+    // fragment of step st: row ni, elements 32 kb + 8 st .. + 7 of the chunk = piece 4 kb + st
     int a_rd[4];
 #pragma unroll
     for (int st = 0; st < 4; ++st) a_rd[st] = ni * 256 + (((4 * st + kb) ^ ni) << 4);
 
     u32x4_t wring[2][4];
     uint32_t sring[4];
-    const bool loads_x = 4 * wave * XV < ROWS;  // wave-uniform
+    const bool loads_x = 4 * wave < ROWS;  // wave-uniform
     auto dma_x = [&](int c) {
         const int lim = (K - c * 128) >> 3;  // 16-byte pieces of the row left in this chunk (<= 0 past the row)
         if (!loads_x) return;
-#pragma unroll
-        for (int q = 0; q < XV; ++q)
-            pk4g_load_lds16(rs_x, mxg_lds + (c & 1) * XBUF + (wave * XV + q) * 1024, xc[q] < lim ? xo[q] : OOB, c * 256);
+        pk4g_load_lds16(rs_x, mxg_lds + (c & 1) * XBUF + wave * 1024, xc < lim ? xo : OOB, c * 256);
     };
     // blocks past the row, and tiles past the layer's last, lie beyond the tile but not beyond what the range check
     // looks at (the lane's offset, not the scalar one): the lane carries an offset that is
@@ -106,11 +95,9 @@ __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restr
     load_s(0);
     load_w(0, wring[0]);
     __builtin_amdgcn_sched_barrier(0);
-    float4_t acc[MT][4];
+    float4_t acc[4];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int f = 0; f < 4; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int f = 0; f < 4; ++f) acc[f] = float4_t{0.f, 0.f, 0.f, 0.f};
     pk4g_wait_vmcnt<8>();
     __syncthreads();
 
@@ -128,28 +115,17 @@ __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restr
         load_s(c + 1);
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
-            // four row tiles at a time: at 128 rows the fragments of all eight beside the accumulators do not fit the
-            // registers, and a B fragment is four conversions to make again
-            constexpr int MH = MT < 4 ? MT : 4;
+            const u32x4_t av = *(const u32x4_t *)(buf + a_rd[st]);
+            const uint32_t a[4] = {av[0], av[1], av[2], av[3]};
 #pragma unroll
-            for (int h = 0; h < MT; h += MH) {
-                uint32_t a[MH][4];
-#pragma unroll
-                for (int mt = 0; mt < MH; ++mt) {
-                    const u32x4_t av = *(const u32x4_t *)(buf + (h + mt) * 4096 + a_rd[st]);
-                    a[mt][0] = av[0], a[mt][1] = av[1], a[mt][2] = av[2], a[mt][3] = av[3];
-                }
-#pragma unroll
-                for (int f = 0; f < 4; ++f) {
-                    const uint32_t w = wring[CUR][f][st];
-                    uint32_t b[4];
-                    b[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 0));
-                    b[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 1));
-                    b[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 2));
-                    b[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 3));
-#pragma unroll
-                    for (int mt = 0; mt < MH; ++mt) acc[h + mt][f] = Ops::mfma(a[mt], b, acc[h + mt][f]);
-                }
+            for (int f = 0; f < 4; ++f) {
+                const uint32_t w = wring[CUR][f][st];
+                uint32_t b[4];
+                b[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 0));
+                b[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 1));
+                b[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 2));
+                b[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale[f], 3));
+                acc[f] = Ops::mfma(a, b, acc[f]);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -166,7 +142,7 @@ __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restr
     }
 
     if (!live) return;
-    // lane (ni, kb), value i of acc[t][f]: pair m0 + 16 t + 4 kb + i, weight row 64 j + 16 f + ni
+    // lane (ni, kb), value i of acc[f]: pair m0 + 4 kb + i, weight row 64 j + 16 f + ni
     float bv[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int f = 0; f < 4; ++f)
@@ -175,31 +151,29 @@ __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restr
     // [1, 0, 3, 2]) and share the work - the even lane finishes pairs i = 0 and 2 of the four, the odd lane 1 and 3.
     const bool odd = ni & 1;
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int f = 0; f < 4; ++f) {
+        const int n = 64 * j + 16 * f + (ni & ~1);  // the lane pair's two weight rows: n, n + 1
+        float mine[4], other[4];
 #pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            const int n = 64 * j + 16 * f + (ni & ~1);  // the lane pair's two weight rows: n, n + 1
-            float mine[4], other[4];
+        for (int i = 0; i < 4; ++i) {
+            // rounded to bf16 as the projection's own output is (for the SwiGLU: what it would read)
+            mine[i] = BF16Traits::to_f32(BF16Traits::from_f32(acc[f][i] + bv[f]));
+            other[i] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mine[i]), 0xB1, 0xF, 0xF, false));
+        }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // rounded to bf16 as the projection's own output is (for the SwiGLU: what it would read)
-                mine[i] = BF16Traits::to_f32(BF16Traits::from_f32(acc[t][f][i] + bv[f]));
-                other[i] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mine[i]), 0xB1, 0xF, 0xF, false));
-            }
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int i = 2 * h + (odd ? 1 : 0);
-                const int m = m0 + 16 * t + 4 * kb + i;
-                const float lo = odd ? other[2 * h + 1] : mine[2 * h], hi = odd ? mine[2 * h + 1] : other[2 * h];  // rows n, n + 1
-                if (m >= m_end || f >= live_tiles) continue;
-                if (swiglu) {
-                    // rows 2 c / 2 c + 1 are the gate / up of output c (moe.rs:152-173)
-                    y[(size_t)m * (N >> 1) + (n >> 1)] = BF16Traits::from_f32(gpt_oss_swiglu_f32(lo, hi, limit));
-                } else {
-                    *(uint32_t *)(y + (size_t)m * N + n) = (uint32_t)BF16Traits::from_f32(lo) | ((uint32_t)BF16Traits::from_f32(hi) << 16);
-                }
+        for (int h = 0; h < 2; ++h) {
+            const int i = 2 * h + (odd ? 1 : 0);
+            const int m = m0 + 4 * kb + i;
+            const float lo = odd ? other[2 * h + 1] : mine[2 * h], hi = odd ? mine[2 * h + 1] : other[2 * h];  // rows n, n + 1
+            if (m >= m_end || f >= live_tiles) continue;
+            if (swiglu) {
+                // rows 2 c / 2 c + 1 are the gate / up of output c (moe.rs:152-173)
+                y[(size_t)m * (N >> 1) + (n >> 1)] = BF16Traits::from_f32(gpt_oss_swiglu_f32(lo, hi, limit));
+            } else {
+                *(uint32_t *)(y + (size_t)m * N + n) = (uint32_t)BF16Traits::from_f32(lo) | ((uint32_t)BF16Traits::from_f32(hi) << 16);
             }
         }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -445,7 +419,9 @@ __global__ __launch_bounds__(512, 4) void mxfp4_wide_kernel(const uint16_t *__re
 
 // Takes the grouped problem from three pairs an expert on average (below, the decode kernel's passes of four tokens
 // read the weights once): 0 = not taken, else the rows of a tile that the grid is sized for, which follow the average (the
-// pairs of an expert are only known on the device; workgroups past the last tile leave at once).
+// pairs of an expert are only known on the device; workgroups past the last tile leave at once).  They stand in the
+// plan's name; mxfp4_wide_kernel's tiles have up to 128 rows whatever the grid.  OXQ_MXFP4_GEMM_ROWS gives them: 32, 64 and 128
+// leave the wide kernel alone, 16 lets the rule of launch_mxfp4_res_gemm choose.
 int mxfp4_gemm_form(const oxq_ctx *ctx, int64_t n_pairs, int64_t E, int64_t K, int64_t N) {
     const int64_t min_pairs = tune(ctx, OXQ_TUNE_MXFP4_GEMM_MIN_PAIRS, 3);
     if (min_pairs <= 0 || E <= 0 || n_pairs < min_pairs * E || N % 16 != 0 || K % 32 != 0) return 0;
@@ -470,8 +446,8 @@ static int mxfp4_wide_go(hipStream_t s, dim3 grid, const Mxfp4Problem &p, int NG
 static int mxfp4_gemm_go(hipStream_t s, dim3 grid, const Mxfp4Problem &p, int NC, int NG, uint32_t x_bytes) {
     static LdsGrant grant;
     const size_t lds = (size_t)2 * 16 * 256;
-    OXQ_HIP_CHECK(grant.ensure((const void *)mxfp4_gemm_kernel<1>, lds));
-    hipLaunchKernelGGL((mxfp4_gemm_kernel<1>), grid, dim3(512), lds, s, (const uint16_t *)p.x, (const unsigned char *)p.blocks,
+    OXQ_HIP_CHECK(grant.ensure((const void *)mxfp4_gemm_kernel, lds));
+    hipLaunchKernelGGL(mxfp4_gemm_kernel, grid, dim3(512), lds, s, (const uint16_t *)p.x, (const unsigned char *)p.blocks,
                        (const unsigned char *)p.scales, (const uint16_t *)p.bias, (uint16_t *)p.y, p.expert_offsets, p.token_ids,
                        (int)p.K, (int)p.N, NC, NG, (int)p.n_experts, x_bytes, p.swiglu, p.swiglu_limit);
     OXQ_HIP_CHECK(hipGetLastError());
@@ -487,10 +463,11 @@ int launch_mxfp4_res_gemm(oxq_ctx *ctx, hipStream_t s, const Mxfp4Problem &p) {
     const int64_t ytiles = p.n_pairs / rows + p.n_experts;
     if (ytiles > 65535) return fail(OXQ_ERR_UNSUPPORTED, "mxfp4 experts prefill: %lld row tiles exceed the grid limit of 65535", (long long)ytiles);
     // The 16-row tiles have workgroups of 512 columns that start with less to do: at up to a dozen pairs an expert they are
-    // the faster ones where K is long and the wide kernel's workgroups of 256 columns do not fill the chip's 512 places (32
+    // the faster ones where K is long and the wide kernel's workgroups of 256 columns do not fill two places a compute unit (32
     // experts x 2880 x 2880 at 24 / 48 / 96 tokens 32.2 / 34.1 / 34.6 against 34.6 / 36.4 / 36.7 us; 5760 x 2880, which fills
     // them, 60.5 / 63.6 / 63.6 against 57.6 / 60.6 / 61.6; 64 experts x 1024 x 1024 at 64 tokens 16.8 against 9.4).
-    const bool narrow = rows == 16 && p.K >= 2048 && ceil_div(p.N, 32 * MXG_WAVES) * p.n_experts < 512;
+    const int64_t places = 2 * (ctx->num_cus > 0 ? ctx->num_cus : 256);
+    const bool narrow = rows == 16 && p.K >= 2048 && ceil_div(p.N, 32 * MXG_WAVES) * p.n_experts < places;
     dim3 grid((unsigned)ceil_div(p.N / 16, (int64_t)4 * MXG_WAVES), (unsigned)ytiles, narrow ? 1 : 2);
     char name[64];
     snprintf(name, sizeof name, "mxfp4_experts_gemm_bf16_r%dx8%s", rows, p.swiglu ? "_swiglu" : "");

@@ -59,7 +59,6 @@
 
 #include <algorithm>
 #include <numeric>
-#include <numeric>
 #include <type_traits>
 #include <cstdlib>
 
