@@ -22,11 +22,12 @@ namespace oxq {
 
 constexpr int MXG_WAVES = 8;
 
-__global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw,
-                                                         const unsigned char *__restrict__ ps, const uint16_t *__restrict__ bias,
-                                                         uint16_t *__restrict__ y, const int32_t *__restrict__ offsets,
-                                                         const int32_t *__restrict__ token_ids, int K, int N, int NC, int NG,
-                                                         int E, uint32_t x_bytes, int swiglu, float limit) {
+template <int NW>
+__global__ __launch_bounds__(NW * 64) void mxfp4_gemm_kernel(const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw,
+                                                             const unsigned char *__restrict__ ps, const uint16_t *__restrict__ bias,
+                                                             uint16_t *__restrict__ y, const int32_t *__restrict__ offsets,
+                                                             const int32_t *__restrict__ token_ids, int K, int N, int NC, int NG,
+                                                             int E, uint32_t x_bytes, int swiglu, float limit) {
     typedef MfmaOps<BF16Traits> Ops;
     constexpr int ROWS = 16, XBUF = ROWS * 256;
     constexpr int OOB = 0x7FFFFF00;
@@ -44,7 +45,7 @@ __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restr
     }
     if (e == E) return;  // the whole workgroup, before any barrier
     const int m0 = offsets[e] + rem * ROWS, m_end = offsets[e + 1];
-    const int j = (int)blockIdx.x * MXG_WAVES + wave;  // the wave's 64 columns: tiles 4 j .. 4 j + 3
+    const int j = (int)blockIdx.x * NW + wave;  // the wave's 64 columns: tiles 4 j .. 4 j + 3
     const int ntiles = N >> 4, nb = K >> 5;
     const int live_tiles = min(4, ntiles - 4 * j);  // wave-uniform; <= 0: a wave past the last tile
     const bool live = live_tiles > 0;
@@ -55,8 +56,9 @@ __global__ __launch_bounds__(512) void mxfp4_gemm_kernel(const uint16_t *__restr
     const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x, x_bytes);
     const int voff_w = lane * 16, voff_s = lane * 4;
     // x: waves 0 .. 3 bring rows 4 wave .. + 3 of a chunk straight into LDS, lane l the 16 bytes that belong at position
-    // l % 16 of row l / 16.  Piece p = 4 kb + st of a row's 128 elements (what lane group kb reads in step st) is kept at position (4 st + kb) ^ (row % 16): the four lane groups of a fragment read then start in
-    // different banks (at position p ^ row, groups 0 and 2 would meet 128 bytes apart: four conflict cycles a read).
+    // l % 16 of row l / 16.  Piece p = 4 kb + st of a row's 128 elements (what lane group kb reads in step st) is kept at
+    // position (4 st + kb) ^ (row % 16): the four lane groups of a fragment read then start in different banks (at position
+    // p ^ row, groups 0 and 2 would meet 128 bytes apart: four conflict cycles a read).
     // Rows past the expert's pairs, and the elements past K in the last chunk, get an offset beyond the descriptor:
     // LDS receives zeros.
     const int r = 4 * wave + (lane >> 4), m = m0 + r, pos = (lane & 15) ^ (r & 15);
@@ -446,8 +448,8 @@ static int mxfp4_wide_go(hipStream_t s, dim3 grid, const Mxfp4Problem &p, int NG
 static int mxfp4_gemm_go(hipStream_t s, dim3 grid, const Mxfp4Problem &p, int NC, int NG, uint32_t x_bytes) {
     static LdsGrant grant;
     const size_t lds = (size_t)2 * 16 * 256;
-    OXQ_HIP_CHECK(grant.ensure((const void *)mxfp4_gemm_kernel, lds));
-    hipLaunchKernelGGL(mxfp4_gemm_kernel, grid, dim3(512), lds, s, (const uint16_t *)p.x, (const unsigned char *)p.blocks,
+    OXQ_HIP_CHECK(grant.ensure((const void *)mxfp4_gemm_kernel<MXG_WAVES>, lds));
+    hipLaunchKernelGGL((mxfp4_gemm_kernel<MXG_WAVES>), grid, dim3(MXG_WAVES * 64), lds, s, (const uint16_t *)p.x, (const unsigned char *)p.blocks,
                        (const unsigned char *)p.scales, (const uint16_t *)p.bias, (uint16_t *)p.y, p.expert_offsets, p.token_ids,
                        (int)p.K, (int)p.N, NC, NG, (int)p.n_experts, x_bytes, p.swiglu, p.swiglu_limit);
     OXQ_HIP_CHECK(hipGetLastError());
