@@ -1,6 +1,9 @@
 """Q2_K and Q3_K layers that hold two copies: how many bytes of second ones a ctx's layers may hold (on a plan-only ctx; on a GPU, what
 a layer without one computes)."""
 import ctypes as C
+import shutil
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -13,14 +16,19 @@ MB = {synth.GGUF_Q2_K: 5.25, synth.GGUF_Q3_K: 7.125}  # of the matrix-core copy
 
 
 class Layer:
-    def __init__(self, ctx, fmt, dt=_lib.BF16, n=N):
-        self.lib, self.ctx, self.dt, self.n, self.h = _lib.load(), ctx, dt, n, C.c_void_p()
+    def __init__(self, ctx, fmt, dt=_lib.BF16, n=N, at=0):
+        self.lib, self.ctx, self.dt, self.n, self.at, self.h = _lib.load(), ctx, dt, n, at, C.c_void_p()
         elems, size = synth.GGUF_BLOCK_LAYOUT[fmt]
-        rc = self.lib.oxq_qlinear_new(ctx.handle, fmt, C.byref(fake((n * (K // elems) * size,), _lib.U8)), K, n, None, dt, C.byref(self.h))
+        rc = self.lib.oxq_qlinear_new(ctx.handle, fmt, C.byref(self.tensor((n * (K // elems) * size,), _lib.U8)), K, n, None, dt, C.byref(self.h))
         assert rc == 0, self.lib.oxq_last_error().decode()
 
+    def tensor(self, shape, dt):
+        t = fake(shape, dt)
+        t.data = self.at
+        return t
+
     def kernel(self, m):
-        assert self.lib.oxq_qlinear_forward(self.h, None, C.byref(fake((m, K), self.dt)), C.byref(fake((m, self.n), self.dt))) == 0
+        assert self.lib.oxq_qlinear_forward(self.h, None, C.byref(self.tensor((m, K), self.dt)), C.byref(self.tensor((m, self.n), self.dt))) == 0
         return self.ctx.last_plan()["kernel"]
 
     def both(self):
@@ -73,6 +81,62 @@ def test_the_default_is_a_32nd_of_the_device_and_layers_outlive_their_ctx():
     ctx.close()
     for x in layers:
         x.free()
+
+
+# The calls of the HIP runtime that building and calling a layer makes, on a device that is not there: allocations above `most` bytes
+# fail, launches do nothing.
+NO_DEVICE = r"""
+#include <cstddef>
+#include <cstdlib>
+extern "C" {
+size_t most = ~(size_t)0;
+int failed = 0;
+int hipGetDeviceCount(int *n) { return *n = 1, 0; }
+int hipGetDevice(int *d) { return *d = 0, 0; }
+int hipSetDevice(int) { return 0; }
+int hipDeviceGetAttribute(int *v, int, int) { return *v = 256, 0; }
+int hipDeviceTotalMem(size_t *b, int) { return *b = (size_t)288 << 30, 0; }
+int hipMalloc(void **p, size_t b) { return b > most ? (++failed, 2) : (*p = malloc(b), 0); }
+int hipFree(void *p) { return free(p), 0; }
+int hipMemset(void *, int, size_t) { return 0; }
+int hipDeviceSynchronize() { return 0; }
+int hipStreamSynchronize(void *) { return 0; }
+int hipGetSymbolAddress(void **p, const void *) { static char array[256]; return *p = array, 0; }
+int hipFuncSetAttribute(const void *, int, int) { return 0; }
+int hipLaunchKernel(const void *, ...) { return 0; }
+int hipGetLastError() { return 0; }
+}
+"""
+
+
+def out_of_memory(rt, fmt, dt):
+    """Run by a process of its own (below), where the symbols of NO_DEVICE (rt) stand before the runtime's."""
+    most, failed = C.c_size_t.in_dll(rt, "most"), C.c_int.in_dll(rt, "failed")
+    ctx = ops.Context(device=0)
+    ctx.set_tuning("OXQ_GGUF_BOTH_MB", int(MB[fmt] + 1))  # room for one
+    most.value = int(MB[fmt] * 1.5) << 20
+    a = Layer(ctx, fmt, dt, at=4096)
+    assert failed.value == 1 and "_res_gemv_" in a.kernel(4), (failed.value, a.kernel(4))
+    most.value = ~0 & (2**64 - 1)
+    b = Layer(ctx, fmt, dt, at=4096)
+    c = Layer(ctx, fmt, dt, at=4096)
+    assert failed.value == 1 and b.both() and not c.both()
+    for x in (a, b, c):
+        x.free()
+    print("given back")
+
+
+@pytest.mark.parametrize("fmt", list(MB))
+@pytest.mark.parametrize("dt", [_lib.BF16, _lib.F32])
+def test_a_second_copy_that_cannot_be_allocated_is_left_out_and_not_counted(fmt, dt, tmp_path):
+    if not shutil.which("g++"):
+        pytest.skip("no g++")
+    lib = tmp_path / "no_device.so"
+    subprocess.run(["g++", "-shared", "-fPIC", "-x", "c++", "-", "-o", str(lib)], input=NO_DEVICE, text=True, check=True)
+    code = (f"import ctypes as C; rt = C.CDLL({str(lib)!r}, mode=C.RTLD_GLOBAL)\n"  # before torch, which brings the runtime
+            f"from tests.test_gguf_second_copies import out_of_memory as t; t(rt, {fmt}, {dt})")
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and "given back" in run.stdout, run.stdout + run.stderr
 
 
 @pytest.mark.gpu
