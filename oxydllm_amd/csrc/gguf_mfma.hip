@@ -1471,11 +1471,16 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
 //                       3.5 us + the partials' bytes at 4.2 TB/s.  14336 x 4096 Q4_K at 33 / 128 / 256 rows 31.8 / 57.8 / 86 ->
 //                       20.9 / 30.7 / 53 us (7, 4 and 2 slices), 4096 x 14336 at 64 rows 28.5 -> 23.5 (2 slices)
 //   eight waves         rounds of workgroups (a last one on at most three quarters of the CUs 0.95) x chunks x `wide` + 5
+// (The rounds of eight waves are older than the numbering of tiles without gaps.  With column groups that are no multiple of eight, 36 layers of six
+// formats, 180 calls of 256 - 4000 rows: within 3 % of the faster form at 167, within 8 % at 179.)
 // The file layout's matmul is not ahead of all of these there.  It is for some calls of Q2_K and Q3_K, whose 9 - 32 rows come
 // here too: where it has 400 tiles of 64 x 64 and more it runs at 400 T/s (Q3_K 15 % less) behind 6 us; with fewer it is ahead
 // where K or the layer is short (Q2_K, us, file layout / here: 1024 x 5056 at 16 rows 6.9 / 8.8, 4096 x 1024 6.9 / 8.1, 2816 x
 // 6528 10.7 / 11.1; elsewhere 4096 x 4096 at 16, 48, 101, 512 rows 10.0 / 9.2, 15.5 / 13.0, 24 / 17.6, 46 / 32,
-// 14336 x 4096 23 / 16, 38 / 22, 68 / 33, 149 / 99, 9984 x 21056 at 16 rows 61 / 42, Q3_K 79 / 42).
+// 14336 x 4096 23 / 16, 38 / 22, 68 / 33, 149 / 99, 9984 x 21056 at 16 rows 61 / 42, Q3_K 79 / 42).  On 71 other layers (K 1024 -
+// 14336, N 512 - 19200, 9 - 2000 rows, 497 calls, every form forced): 0.79 x the file layout's time, none of the 342 calls that come here
+// behind it by 3 %, 454 within 3 % of the fastest form; 12 stay on the file layout by 15 - 42 % of their time (Q3_K 4352 x 896 at 1200
+// rows 54.8, here 38.6; 7168 x 4608 at 500 136.7, here 103.9).
 // Smaller layers compare it with the unsliced forms only, in rounds of 256 workgroups of 64 rows x 512 columns: 0.17 + 1.45 w
 // (1.3 w for the five- and six-bit formats).
 // OXQ_GGUF_GEMM_MIN_M: unset = by cost, 0 = never, n = the eight-wave form from n rows on whatever the cost;

@@ -191,6 +191,9 @@ __global__ __launch_bounds__(512) void pk4n_gemm_kernel(const uint16_t *__restri
 // 5120 x 6144) the choice is within 8 % of the fastest, except where a launch holds one to one and a half rounds: 8-bit
 // 4096 x 6144 at 150 rows split-K 32 us, two strips 23; groups of 64, 4096 x 11008 at 150 rows 46 and 40; groups of 32,
 // 5120 x 6144 at 150 / 777 / 900 / 1200 rows f16 33 / 96 / 96 / 143 as chosen, 26 / 81 / 84 / 108 with two strips.
+// The fits are older than the numbering without gaps too.  Where the strip groups are no multiple of eight (32 layers of 64-column
+// strips with 1 - 21 groups, K 1280 - 10240, both types and widths, 160 calls of 256 - 4000 rows, every form forced) the choice is
+// within 3 % of the fastest at 129, within 8 % at 152, 15 % at all.
 // OXQ_PK4_GEMM_ROWS = 64 | 128 | 32 (128 and the last tile of 32) takes the choice (tests, sweeps); OXQ_PK4_GEMM_MIN_M = 0 switches the kernels off.
 // a round of the two-strip form (one workgroup a CU) against a full round of 64-row workgroups of eight strips:
 // 19 - 24 us against 65 - 78 at K = 4096 over both widths and types
