@@ -657,6 +657,48 @@ template <bool INF, bool FOURS> __device__ __forceinline__ void ggm_split3(const
     }
 }
 
+// Q2_K, Q3_K: row x times column n weight by weight, in f32.  5 - 8 bf16 rows ran on the tile matmul with unrounded weights,
+// where an infinity times a weight keeps its sign and a row of 1e37 has finite sums; with the integers in front of the scale, and the
+// minimum or offset behind them, both are NaN.  A sum that is not finite is made again so (up to 4 rows ran on the vector kernel,
+// which splits the weight in the same way), 2^24 smaller, so that it overflows only where the result does.  x: the row, 16-byte aligned.
+template <int FMT>
+__device__ __forceinline__ float ggm_narrow_dot(const uint8_t *__restrict__ pw, const uint16_t *__restrict__ x, int n, int K) {
+    typedef GgmFmt<FMT> F;
+    typedef GgmLayout<FMT> L;
+    constexpr bool THREE = FMT == OXQ_GGUF_Q3_K;
+    const int ni = n & 15;
+    const uint8_t *blk = pw + (size_t)(n >> 4) * (K >> 8) * L::BLKB;
+    float sum = 0.f;
+#pragma unroll 1
+    for (int b = 0; b < K >> 8; ++b, blk += L::BLKB) {
+        const float d = ggm_f16(*(const uint16_t *)(blk + L::BH_OFF + ni * F::BH));
+        const float dm = THREE ? 0.f : ggm_f16(*(const uint16_t *)(blk + L::BH_OFF + ni * F::BH + F::BH - 2));
+#pragma unroll 1
+        for (int s = 0; s < 16; ++s) {  // sixteen elements: step s % 8 of chunk s / 8
+            const uint8_t *chunk = blk + (s >> 3) * L::CHB;
+            const int s2 = s & 7, t = s2 >> 1;
+            const uint32_t sc = chunk[L::UH_OFF + ni * 8 + s2];
+            const float f = d * (THREE ? (float)(int)(int8_t)sc : (float)(sc & 0xFu)), g = dm * (float)(sc >> 4);
+            const u32x4_t xv[2] = {*(const u32x4_t *)(x + b * 256 + s * 16), *(const u32x4_t *)(x + b * 256 + s * 16 + 8)};
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb) {
+                const int lane = 16 * kb + ni, at = 16 * (s2 & 1);
+                const uint32_t w = *(const uint32_t *)(chunk + lane * 8 + 4 * (t >> 1)) >> (at + 4 * (t & 1));
+                const uint32_t w3 = THREE ? *(const uint32_t *)(chunk + 512 + lane * 4) >> (at + 2 * t) : 0u;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int bit = 8 * (i & 1) + (i >> 1);  // byte of the word, pair of the byte
+                    const int q = (int)((w >> (bit + (i >> 1))) & 3u) | (THREE ? (int)((w3 >> bit) & 1u) << 2 : 0);
+                    const float v = THREE ? f * (float)(q - 4) : f * (float)q - g;
+                    const uint32_t pair = xv[kb >> 1][2 * (kb & 1) + (i >> 1)];
+                    sum = __builtin_fmaf(v, __builtin_bit_cast(float, i & 1 ? pair & 0xFFFF0000u : pair << 16) * 0x1p-24f, sum);
+                }
+            }
+        }
+    }
+    return sum * 0x1p24f;
+}
+
 // Waves a SIMD that an instantiation's registers have to leave room for.  Two workgroups of eight waves a compute unit are what
 // hides the waits of one to four rows on layers of more than one round of strips; Q6_K came out two registers over that (a row,
 // us, without / with room: 1024 x 9216 6.5 / 5.5, 4096 x 8704 12.3 / 10.8, 5632 x 7168 10.7 / 10.0).
@@ -904,6 +946,10 @@ __global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) vo
     }
     if constexpr (XF32) ggm_epilogue_f32<MT, NS, NW>(acc, (const float *)bias, (float *)y, M, N, j, m0, wave, lane);
     else if (act) ggm_epilogue_act<MT, NS, NW>(acc, bias, y, M, N, j, m0, act, wave, lane);
+    else if constexpr (ggm_narrow<FMT> && XQ > 1)
+        pk4n_epilogue<TT, MT, NS, NW, true>(acc, bias, y, ws, M, N, j, m0, wave, lane, [&](float v, int m, int n) {
+            return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) == 0x7F800000u ? ggm_narrow_dot<FMT>(pw, x + (size_t)m * K, n, K) : v;
+        });
     else pk4n_epilogue<TT, MT, NS, NW, true>(acc, bias, y, ws, M, N, j, m0, wave, lane);
 }
 

@@ -363,10 +363,14 @@ __device__ __forceinline__ void pk4_epilogue_lanes(const float4_t (&acc)[MT][4],
 // in LDS as in the wide form; a thread then owns (row, column ni of every strip of the workgroup) and adds the
 // waves in order.
 // RAGGED: columns may end inside the last strip (the narrow form's never do).
-template <typename TT, int MT, int NS, int NW, bool RAGGED = false>
+// AGAIN: what becomes of the sum of (row, column) before the bias.
+struct Pk4nAsItIs {
+    __device__ __forceinline__ float operator()(float v, int, int) const { return v; }
+};
+template <typename TT, int MT, int NS, int NW, bool RAGGED = false, typename AGAIN = Pk4nAsItIs>
 __device__ __forceinline__ void pk4n_epilogue(const float4_t (&acc)[MT][NS], const uint16_t *__restrict__ bias,
                                               uint16_t *__restrict__ y, float *__restrict__ ws, int M, int N, int j,
-                                              int m0, int wave, int lane) {
+                                              int m0, int wave, int lane, const AGAIN &again = AGAIN{}) {
     constexpr int NT = NW * 64, ROWS = 16 * MT;
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
     // every wave into its own activation slot (other waves may still be reading theirs): [MT][4 e][64 lanes][NS]
@@ -406,7 +410,7 @@ __device__ __forceinline__ void pk4n_epilogue(const float4_t (&acc)[MT][NS], con
             if (gridDim.y > 1) {  // this K slice's f32 partial; a second kernel adds the slices in order
                 ws[((size_t)blockIdx.y * M + (m0 + ml)) * N + n] = v[f];
             } else {
-                float o = v[f];
+                float o = again(v[f], m0 + ml, n);
                 if (bias) o += TT::to_f32(bias[n]);
                 y[(size_t)(m0 + ml) * N + n] = TT::from_f32(o);
             }

@@ -70,3 +70,38 @@ def test_infinities_follow_the_kernels_of_fewer_and_more_rows(fmt):
         a, b = new.forward(x[:m].cuda()).float().cpu().numpy(), old.forward(x[:m].cuda()).float().cpu().numpy()
         for f in (np.isnan, np.isposinf, np.isneginf):
             np.testing.assert_array_equal(f(a), f(b), err_msg=f"m={m}")
+
+
+@pytest.mark.parametrize("fmt", list(TAG))
+@pytest.mark.parametrize("N,K,m", [(1040, 1024, 5), (2624, 3328, 8), (12352, 256, 7), (528, 2304, 8)])  # 8 and 16 waves; four strips a workgroup
+def test_infinite_and_large_rows_from_five_on(fmt, N, K, m):
+    """5 - 8 rows ran on the tile matmul with unrounded weights before: an infinity times a weight keeps its sign, and large rows have
+    finite sums where the result is one, though those with the integers alone are not."""
+    data = synth.gguf_weight(fmt, N, K, seed=fmt + K)
+    w = oracle.dequantize_gguf(fmt, data, N, K)
+    bias = np.random.default_rng(N).standard_normal(N).astype(np.float32)
+    layer = ops.QLinear(fmt, to_dev(data), K, N, to_dev(bias, torch.bfloat16), torch.bfloat16)
+    x = np.random.default_rng(K + m).standard_normal((m, K)).astype(np.float32)
+    plain = layer.forward(to_dev(x, torch.bfloat16))
+    x[0, 5], x[1, K - 1], x[2, 9] = np.inf, -np.inf, np.nan
+    x[3] *= 3e39 / float((np.abs(x[3]) @ np.abs(w).T).max())
+    x[m - 1] = 0.0
+    x[m - 1, 17] = 3e38 / max(1.0, float(np.abs(w[:, 17]).max()))
+    print(f"[case] gguf {TAG[fmt]} infinite and large rows N={N} K={K} m={m}", flush=True)
+    y = layer.forward(to_dev(x, torch.bfloat16))
+    assert ops.default_context().last_plan()["kernel"].startswith(f"gguf_{TAG[fmt]}_mfma_bf16")
+    got = y.float().cpu().numpy()
+    for r, k, sign in ((0, 5, 1.0), (1, K - 1, -1.0)):
+        np.testing.assert_array_equal(got[r], np.where(w[:, k] == 0, np.nan, sign * np.sign(w[:, k]) * np.inf).astype(np.float32))
+    assert np.isnan(got[2]).all()
+    x64 = round_x(x, oracle.BF16).astype(np.float64)
+    for r in (3, m - 1):
+        ref, mag = x64[r] @ w.T.astype(np.float64), np.abs(x64[r]) @ np.abs(w.T.astype(np.float64))
+        fits = np.abs(ref) < 3.3e38
+        assert fits.any() and np.isfinite(got[r][fits]).all()
+        # one bf16 rounding, f32 sums, the bias
+        assert (np.abs(got[r] - ref)[fits] <= (2.0 ** -8 * np.abs(ref) + 2.0 ** -18 * mag + 8)[fits]).all()
+        big = np.abs(ref) > 3.5e38
+        np.testing.assert_array_equal(got[r][big], (np.sign(ref) * np.inf)[big].astype(np.float32))
+    for r in range(4, m - 1):
+        assert torch.equal(y[r], plain[r])
