@@ -459,6 +459,34 @@ template <int FMT> struct GgmChunk {
             lo |= third(2 * st), hi |= third(2 * st + 1);
         }
     }
+    // Formats with scales of 16 elements, the way rows of x lie: elements 8 kb .. + 7 of unit st, four bytes each in v0 and v1, all of
+    // sub-block 2 st + kb / 2.  The copy gives lane group kb elements 4 kb .. + 3 of both sub-blocks; two exchanges of
+    // lane groups turn one into the other.
+    __device__ __forceinline__ void in_order(int st, uint32_t &v0, uint32_t &v1) const {
+        uint32_t lo, hi, even, odd;  // of sub-block 2 st, 2 st + 1
+        if constexpr (ggm_narrow<FMT>) {
+            bytes2(st, lo, hi);
+            even = pack_lo16(lo, hi), odd = pack_hi16(lo, hi);
+        } else {
+            bytes(st, lo, hi);
+            even = perm_b32(hi, lo, 0x06040200u), odd = perm_b32(hi, lo, 0x07050301u);
+        }
+        const auto halves = __builtin_amdgcn_permlane32_swap(even, odd, false, false);           // {e0 e1 o0 o1}, {e2 e3 o2 o3}
+        const auto rows = __builtin_amdgcn_permlane16_swap(halves[0], halves[1], false, false);  // {e0 e2 o0 o2}, {e1 e3 o1 o3}
+        v0 = rows[0], v1 = rows[1];
+    }
+    // w = f0 q + c of the lane's elements of unit st in that order (q: the unsigned integer)
+    __device__ __forceinline__ void factors_in_order(int ni, int kb, float (&f0)[4], float (&c)[4]) const {
+        const int sh = 8 * (kb >> 1);
+        const uint32_t u[2] = {uh[0] >> sh, uh[1] >> sh};
+        const float d = ggm_f16(FMT == OXQ_GGUF_Q2_K || !(ni & 1) ? bh[0] & 0xFFFFu : bh[0] >> 16), dm = ggm_f16(bh[0] >> 16);
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            const uint32_t b = u[st >> 1] >> (16 * (st & 1));
+            if constexpr (FMT == OXQ_GGUF_Q2_K) f0[st] = d * (float)(b & 0xFu), c[st] = -dm * (float)((b >> 4) & 0xFu);
+            else f0[st] = d * (float)(int)(int8_t)(b & 0xFFu), c[st] = f0[st] * (FMT == OXQ_GGUF_Q3_K ? -4.0f : -32.0f);
+        }
+    }
     // B operand of step st: bias + q as bf16 pairs (four for a step of 32 elements, two for one of 16)
     __device__ __forceinline__ void operand(int st, uint32_t (&b)[4], const NibbleMasks &nm) const {
         if constexpr (FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_K || FMT == OXQ_GGUF_Q4_1) {
@@ -969,12 +997,24 @@ __global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) vo
 // with such workgroups: gridDim.y slices of `cslice` chunks each then write their f32 tiles to `part` and a second
 // launch adds them in slice order.  half: a fused gate|up layer without its activation - columns go back to the
 // file's order (ggm_src_row).
+// NS = 2, MT = 8: 128 rows, a wave has two strips.  What bounds the form above is the conversion's vector instructions, 5 - 7 an
+// MFMA at four row tiles a weight; here a weight serves eight, at the price of LDS, whose fragment then feeds two MFMAs instead of
+// four.  (Four strips do not fit: 128 accumulators beside two ring halves.)  KS = 1: 256 columns, 143 - 161 registers; KS = 2: 128
+// columns, the two waves of a column group take every other chunk and finish four row tiles each - for launches that 256 columns
+// leave CUs idle in.  us, best of the forms of 64 rows -> 128: Q4_K 4096 x 4096 at 520 / 1024 / 2048 rows 55 / 56 / 91 -> 39 / 42 / 71,
+// 4096 x 14336 at 256 / 1024 / 2048 56 / 179 / 345 -> 41 / 136 / 262, 14336 x 4096 at 777 164 -> 122; Q8_0 4096 x 14336 at 2048
+// 344 -> 275; Q6_K 435 -> 312; Q3_K 405 -> 281.
 // What bounds it: the conversion's vector instructions beside the MFMAs.  The five- and six-bit formats join nibble and plane bits
 // four weights at a time into bytes (GgmChunk::bytes), 3.4 instructions a weight; pair by pair as the integer kernel's operand
-// they took 4.3, and 5.3 with a minimum added behind the fma.  Q6_K multiplies its two scales of a 32-element step into one
-// MFMA's operand (of 16 elements each before).  bf16, us, before -> here: Q6_K / Q5_K / Q5_1 / Q5_0 4096 x 4096 at 2048 rows 127 / 130 /
-// 123 / 108 -> 113 / 105 / 96 / 95, 14336 x 4096 at 33 rows 25.8 / 25.4 / 24.6 / 22.8 -> 22.6 / 21.1 / 20.1 / 20.0.
-template <int FMT, int MT, int KS>
+// they took 4.3, and 5.3 with a minimum added behind the fma (Q6_K / Q5_K / Q5_1 / Q5_0 4096 x 4096 at 2048 rows 127 / 130 /
+// 123 / 108 -> 113 / 105 / 96 / 95 us in the 64-row form).  Q6_K multiplies its two scales of a 32-element step into one MFMA's
+// operand (of 16 elements each before).
+// Formats with scales of 16 elements: at 128 rows the integers go into the order of the rows of x (GgmChunk::in_order): one scale a
+// lane and step, half of the factors, and whole 16-byte reads of x instead of two of 8 bytes that met in the banks (3 - 7 cycles a
+// read): Q6_K 4096 x 14336 at 2048 rows 395 -> 312 us.  At 64 rows, where a fragment serves four strips, the exchanges
+// cost what the reads save (439 / 435), and more at 48 (14336 x 4096 at 33 22.1 / 22.5): those keep elements 4 kb .. + 3 of both halves.
+// NS: strips of a wave.
+template <int FMT, int MT, int KS, int NS = 4>
 __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw,
                                                        const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                        float *__restrict__ part, int M, int K, int N, int NG, int RT, int act,
@@ -984,11 +1024,13 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
     typedef GgmFmt<FMT> F;
     typedef GgmLayout<FMT> L;
     typedef GgmChunk<FMT> C;
-    static_assert(KS == 1 || KS >= MT, "wave kq of a column group finishes row tile kq");
-    constexpr int SPW = 8 / KS;  // waves of 64 columns a workgroup
-    constexpr int ROWS = 16 * MT, XBUF = KS * ROWS * 256, XV = ROWS / 4 / SPW, NSTEP = C::NSTEP;
-    constexpr bool K16 = NSTEP == 8;  // scales of 16 elements: an MFMA takes two of them, four elements a lane each
-    constexpr int RING = 4 * C::LOADS;  // vector loads of a chunk's weights: younger than the chunk's loads of x
+    static_assert(KS == 1 || KS >= MT || MT % KS == 0, "the waves of a column group finish as many row tiles each");
+    constexpr int SPW = 8 / KS;  // waves of 16 NS columns a workgroup
+    constexpr int ROWS = 16 * MT, XBUF = KS * ROWS * 256, XV = ROWS / 4 / SPW;
+    constexpr bool K16 = ggm_k16<FMT> && NS == 4;    // scales of 16 elements: an MFMA takes two of them, four elements a lane each
+    constexpr bool ORDER = ggm_k16<FMT> && NS != 4;  // in the order of the rows of x: a lane's eight are within one
+    constexpr int NSTEP = K16 ? C::NSTEP : 4;
+    constexpr int RING = NS * C::LOADS;  // vector loads of a chunk's weights: younger than the chunk's loads of x
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
 
     const int lane = threadIdx.x & 63;
@@ -1002,9 +1044,9 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
     } else {
         rt = (int)blockIdx.x / NG, g = (int)blockIdx.x % NG;
     }
-    const int j = g * SPW + ws;  // the wave's 64 columns: strips 4 j .. 4 j + 3
+    const int j = g * SPW + ws;  // the wave's columns: strips NS j .. NS j + NS - 1
     const int strips = (N + 15) >> 4;
-    const bool live = 4 * j < strips;
+    const bool live = NS * j < strips;
     const int m0 = rt * ROWS;
     const int NC = K >> 7;
     const int cbeg = (int)blockIdx.y * cslice, cend = min(NC, cbeg + cslice);  // the slice's chunks
@@ -1013,7 +1055,7 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
 
     const uint32_t strip_bytes = (uint32_t)(NC / F::CH) * (uint32_t)L::BLKB;
     const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);
-    const __amdgpu_buffer_rsrc_t rs_wl = make_rsrc(pw + (size_t)(live ? 4 * j : 0) * strip_bytes, (uint32_t)min(4, live ? strips - 4 * j : 4) * strip_bytes);
+    const __amdgpu_buffer_rsrc_t rs_wl = make_rsrc(pw + (size_t)(live ? NS * j : 0) * strip_bytes, (uint32_t)min(NS, live ? strips - NS * j : NS) * strip_bytes);
     const __amdgpu_buffer_rsrc_t rs_w = live ? rs_wl : rs_none;
     const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x + (size_t)m0 * K, (uint32_t)xrows * (uint32_t)K * 2u);
     // x: load q of a wave brings rows 4 (XV wave + q) .. + 3 of the chunk, lane l the 16 bytes that belong at
@@ -1032,7 +1074,7 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
     constexpr float NEGF = __builtin_bit_cast(float, (F::NEG & 0xFFFFu) << 16);
     constexpr bool NIB = FMT == OXQ_GGUF_Q4_0 || FMT == OXQ_GGUF_Q4_1 || FMT == OXQ_GGUF_Q4_K;
 
-    C wr[2][4];
+    C wr[2][NS];
     auto dma_x = [&](int r) {  // round r: the wave's chunk is KS r + kq, its tile of x at kq ROWS 256 of the round's buffer
         const int i = cbeg + KS * r + kq;
         const __amdgpu_buffer_rsrc_t rs = i < cend ? rs_x : rs_none;
@@ -1040,21 +1082,21 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         for (int q = 0; q < XV; ++q)
             pk4g_load_lds16(rs, pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256) + (ws * XV + q) * 1024, xo[q], i * 256);
     };
-    auto request = [&](int i, C (&w)[4]) {
+    auto request = [&](int i, C (&w)[NS]) {
         const __amdgpu_buffer_rsrc_t rs = i < cend ? rs_w : rs_none;
 #pragma unroll
-        for (int f = 0; f < 4; ++f) w[f].request(rs, lane, ni, i, (int)(f * strip_bytes));
+        for (int f = 0; f < NS; ++f) w[f].request(rs, lane, ni, i, (int)(f * strip_bytes));
     };
 
     dma_x(0);
     __builtin_amdgcn_sched_barrier(0);  // requests keep this order: the wait counts rely on it
     request(cbeg + kq, wr[0]);
     __builtin_amdgcn_sched_barrier(0);
-    float4_t acc[MT][4];
+    float4_t acc[MT][NS];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int f = 0; f < 4; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int f = 0; f < NS; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
     pk4g_wait_vmcnt<RING>();
     __syncthreads();
 
@@ -1068,14 +1110,18 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         const unsigned char *buf = pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256);
         // w = f0 q' + c2 with q' = q minus the format's offset and c2 = -(minimum): exact products, one rounding -
         // the bits of the dense dequant (ggm_dequant_kernel), so the tile the matrix cores see is the reference's
-        float f0[4][NSTEP], c2[4][C::HAS_MIN ? NSTEP : 1];
+        float f0[NS][NSTEP], c2[NS][C::HAS_MIN || ORDER ? NSTEP : 1];
 #pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            float f1[NSTEP];
-            wr[CUR][f].factors(i & 1, ni, f0[f], f1);
-            if constexpr (C::HAS_MIN) {
+        for (int f = 0; f < NS; ++f) {
+            if constexpr (ORDER) {
+                wr[CUR][f].factors_in_order(ni, kb, f0[f], c2[f]);
+            } else {
+                float f1[NSTEP];
+                wr[CUR][f].factors(i & 1, ni, f0[f], f1);
+                if constexpr (C::HAS_MIN) {
 #pragma unroll
-                for (int st = 0; st < NSTEP; ++st) c2[f][st] = -128.0f * f1[st];
+                    for (int st = 0; st < NSTEP; ++st) c2[f][st] = -128.0f * f1[st];
+                }
             }
         }
 #pragma unroll
@@ -1092,10 +1138,10 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
                 }
             }
 #pragma unroll
-            for (int f = 0; f < 4; ++f) {
+            for (int f = 0; f < NS; ++f) {
                 uint32_t b[4];
                 const float sc = f0[f][st];
-                if constexpr (ggm_narrow<FMT>) {
+                if constexpr (K16 && ggm_narrow<FMT>) {
                     uint32_t lo, hi;
                     wr[CUR][f].bytes2(st, lo, hi);
                     float ql[4], qu[4];
@@ -1108,6 +1154,18 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
                     Pk4gBf16 c0, c1;
                     c0.set(f0[f][2 * st], -32.0f), c1.set(f0[f][2 * st + 1], -32.0f);
                     b[0] = c0.template bytes<0>(lo), b[1] = c0.template bytes<0>(hi), b[2] = c1.template bytes<1>(lo), b[3] = c1.template bytes<1>(hi);
+                } else if constexpr (ORDER) {
+                    uint32_t v0, v1;
+                    wr[CUR][f].in_order(st, v0, v1);
+                    const Pk4gBf16 cv = {sc, c2[f][st]};
+                    if constexpr (ggm_narrow<FMT>) {
+                        float q0[4], q1[4];
+                        pk4g_widen(v0, q0), pk4g_widen(v1, q1);
+                        b[0] = cv.pair(q0[0], q0[1]), b[1] = cv.pair(q0[2], q0[3]), b[2] = cv.pair(q1[0], q1[1]), b[3] = cv.pair(q1[2], q1[3]);
+                    } else {
+                        b[0] = cv.pair((float)(v0 & 0xFFu), (float)((v0 >> 8) & 0xFFu)), b[1] = cv.pair((float)((v0 >> 16) & 0xFFu), (float)(v0 >> 24));
+                        b[2] = cv.pair((float)(v1 & 0xFFu), (float)((v1 >> 8) & 0xFFu)), b[3] = cv.pair((float)((v1 >> 16) & 0xFFu), (float)(v1 >> 24));
+                    }
                 } else if constexpr (NIB) {
                     // plain nibbles (pair pp = nibble pp of each 16-bit half)
                     Pk4gBf16 cv;
@@ -1150,71 +1208,80 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         }
     }
 
-    // the finished tile rows of this wave: all of them (KS = 1), or row tile kq summed over the column group's waves
-    constexpr int FT = KS == 1 ? MT : 1;
-    float4_t fin[FT][4];
+    // the finished tile rows of this wave: all of them (KS = 1), or row tiles FT kq .. + FT - 1 summed over the column group's waves
+    constexpr int FT = KS == 1 ? MT : (MT + KS - 1) / KS;
+    float4_t fin[FT][NS];
     if constexpr (KS == 1) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int f = 0; f < 4; ++f) fin[mt][f] = acc[mt][f];
+            for (int f = 0; f < NS; ++f) fin[mt][f] = acc[mt][f];
     } else {
-        // slot of wave w: [mt][e][lane] x float4 (f = 0..3), 16 KB; the last round's barrier has freed the buffers
-        float4_t *red = (float4_t *)pk4_lds;
+        // slot of wave w: [mt][e][lane] x NS floats; the last round's barrier has freed the buffers
+        typedef float part_t __attribute__((ext_vector_type(NS)));
+        part_t *red = (part_t *)pk4_lds;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                red[((wave * MT + mt) * 4 + e) * 64 + lane] = float4_t{acc[mt][0][e], acc[mt][1][e], acc[mt][2][e], acc[mt][3][e]};
+            for (int e = 0; e < 4; ++e) {
+                part_t v;
+#pragma unroll
+                for (int f = 0; f < NS; ++f) v[f] = acc[mt][f][e];
+                red[((wave * MT + mt) * 4 + e) * 64 + lane] = v;
+            }
         __syncthreads();
 #pragma unroll
-        for (int f = 0; f < 4; ++f) fin[0][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < FT; ++t) {
 #pragma unroll
-        for (int k = 0; k < KS; ++k)  // K order: the same sum whatever the timing
+            for (int f = 0; f < NS; ++f) fin[t][f] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float4_t v = red[(((k * SPW + ws) * MT + min(kq, MT - 1)) * 4 + e) * 64 + lane];
-                fin[0][0][e] += v[0], fin[0][1][e] += v[1], fin[0][2][e] += v[2], fin[0][3][e] += v[3];
-            }
+            for (int k = 0; k < KS; ++k)  // K order: the same sum whatever the timing
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const part_t v = red[(((k * SPW + ws) * MT + min(FT * kq + t, MT - 1)) * 4 + e) * 64 + lane];
+#pragma unroll
+                    for (int f = 0; f < NS; ++f) fin[t][f][e] += v[f];
+                }
+        }
     }
     if (!live || (KS > MT && kq >= MT)) return;
     if (act) {
-        // Fused gate|up layer (ggm_src_row): strip 4 j + f holds gate columns 8 (4 j + f) .. + 7 in lanes ni < 8 and
-        // the up columns they meet in lanes ni + 8.  The two lanes of a pair exchange their four values (row_ror:8)
-        // and finish two outputs each; both factors rounded to bf16 first, as in ggm_epilogue_act.  y is [M, N / 2].
+        // Fused gate|up layer (ggm_src_row): strip NS j + f holds gate columns 8 (NS j + f) .. + 7 in lanes ni < 8 and
+        // the up columns they meet in lanes ni + 8.  The two lanes of a pair exchange their values (row_ror:8) and finish
+        // half of the outputs each; both factors rounded to bf16 first, as in ggm_epilogue_act.  y is [M, N / 2].
         const int hc = N >> 1, p = ni & 7;
         const bool low = ni < 8;
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
+        float bv[NS] = {};
         if (bias) {
 #pragma unroll
-            for (int f = 0; f < 4; ++f) bv[f] = TT::to_f32(bias[(low ? 0 : hc) + 8 * (4 * j + f) + p]);
+            for (int f = 0; f < NS; ++f) bv[f] = TT::to_f32(bias[(low ? 0 : hc) + 8 * (NS * j + f) + p]);
         }
 #pragma unroll
         for (int t = 0; t < FT; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
-                float mine[4], other[4];
+                const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + e;
+                float mine[NS], other[NS];
 #pragma unroll
-                for (int f = 0; f < 4; ++f) {
+                for (int f = 0; f < NS; ++f) {
                     mine[f] = TT::to_f32(TT::from_f32(fin[t][f][e] + bv[f]));
                     other[f] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mine[f]), 0x128, 0xF, 0xF, false));
                 }
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const int f = low ? q : 2 + q;
-                    const float gq = low ? mine[q] : other[2 + q], uq = low ? other[q] : mine[2 + q];
+                for (int q = 0; q < NS / 2; ++q) {
+                    const int f = low ? q : NS / 2 + q;
+                    const float gq = low ? mine[q] : other[NS / 2 + q], uq = low ? other[q] : mine[NS / 2 + q];
                     const uint16_t o = TT::from_f32(mul_f32_rn(act == 1 ? silu_f32(gq) : gelu_tanh_f32(gq), uq));
-                    if (row < M) y[(size_t)row * hc + 8 * (4 * j + f) + p] = o;
+                    if (row < M) y[(size_t)row * hc + 8 * (NS * j + f) + p] = o;
                 }
             }
         return;
     }
-    // row 16 mt + 4 kb + e, column 64 j + 16 f + ni (of the copy)
-    int col[4];
+    // row 16 mt + 4 kb + e, column 16 (NS j + f) + ni (of the copy)
+    int col[NS];
 #pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        const int c = 64 * j + 16 * f + ni;
+    for (int f = 0; f < NS; ++f) {
+        const int c = 16 * (NS * j + f) + ni;
         col[f] = c < N ? ggm_src_row(c, half) : -1;
     }
     if (gridDim.y > 1) {
@@ -1222,27 +1289,27 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         for (int t = 0; t < FT; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
+                const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + e;
                 if (row >= M) continue;
 #pragma unroll
-                for (int f = 0; f < 4; ++f)
+                for (int f = 0; f < NS; ++f)
                     if (col[f] >= 0) part[((size_t)blockIdx.y * M + row) * N + col[f]] = fin[t][f][e];
             }
         return;
     }
-    float bv[4] = {0.f, 0.f, 0.f, 0.f};
+    float bv[NS] = {};
     if (bias) {
 #pragma unroll
-        for (int f = 0; f < 4; ++f) bv[f] = col[f] >= 0 ? TT::to_f32(bias[col[f]]) : 0.f;
+        for (int f = 0; f < NS; ++f) bv[f] = col[f] >= 0 ? TT::to_f32(bias[col[f]]) : 0.f;
     }
 #pragma unroll
     for (int t = 0; t < FT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
+            const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + e;
             if (row >= M) continue;
 #pragma unroll
-            for (int f = 0; f < 4; ++f)
+            for (int f = 0; f < NS; ++f)
                 if (col[f] >= 0) y[(size_t)row * N + col[f]] = TT::from_f32(fin[t][f][e] + bv[f]);
         }
 }
@@ -1517,6 +1584,11 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
 //                       3.5 us + the partials' bytes at 4.2 TB/s.  14336 x 4096 Q4_K at 33 / 128 / 256 rows 31.8 / 57.8 / 86 ->
 //                       20.9 / 30.7 / 53 us (7, 4 and 2 slices), 4096 x 14336 at 64 rows 28.5 -> 23.5 (2 slices)
 //   eight waves         rounds of workgroups (a last one on at most three quarters of the CUs 0.95) x chunks x `wide` + 5
+//   128 rows            rounds of workgroups x (7 + chunks x `wide128`), and of 128 columns x (7 + K rounds of two chunks x `pair128`) with the
+//                       sum of K slices as above; fitted to 4096 x 4096, 4096 x 14336, 14336 x 4096, 2560 x 3072 and 1536 x 6400 at 128 -
+//                       2048 rows in Q4_K, Q8_0, Q6_K and Q3_K.  On 45 other layers of ten formats at 65 - 4000 rows, every form forced
+//                       (130 calls): within 4 % of the fastest at 117, within 10 % at 125; the others are Q2_K and Q3_K calls that
+//                       stay on the file layout
 // (The rounds of eight waves are older than the numbering of tiles without gaps.  With column groups that are no multiple of eight, 36 layers of six
 // formats, 180 calls of 256 - 4000 rows: within 3 % of the faster form at 167, within 8 % at 179.)
 // The file layout's matmul is not ahead of all of these there.  It is for some calls of Q2_K and Q3_K, whose 9 - 32 rows come
@@ -1524,34 +1596,41 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
 // where K or the layer is short (Q2_K, us, file layout / here: 1024 x 5056 at 16 rows 6.9 / 8.8, 4096 x 1024 6.9 / 8.1, 2816 x
 // 6528 10.7 / 11.1; elsewhere 4096 x 4096 at 16, 48, 101, 512 rows 10.0 / 9.2, 15.5 / 13.0, 24 / 17.6, 46 / 32,
 // 14336 x 4096 23 / 16, 38 / 22, 68 / 33, 149 / 99, 9984 x 21056 at 16 rows 61 / 42, Q3_K 79 / 42).  On 71 other layers (K 1024 -
-// 14336, N 512 - 19200, 9 - 2000 rows, 497 calls, every form forced): 0.79 x the file layout's time, none of the 342 calls that come here
-// behind it by 3 %, 454 within 3 % of the fastest form; 12 stay on the file layout by 15 - 42 % of their time (Q3_K 4352 x 896 at 1200
-// rows 54.8, here 38.6; 7168 x 4608 at 500 136.7, here 103.9).
+// 14336, N 512 - 19200, 9 - 2000 rows, 497 calls, every form of 64 rows forced): 0.79 x the file layout's time, none of the 342 calls that
+// come here behind it by 3 %.  With the forms of 128 rows it is ahead from fewer weights above 512 rows (Q3_K 5888 x 512 at 779 rows
+// 30 / 21.5, Q2_K 3072 x 1152 at 656 31.5 / 21.2, Q3_K 2816 x 704 at 704 19.2 / 20.0) and by the bare estimate at 400 tiles (Q2_K
+// 1536 x 5504 at 346 24.6 / 20.8); 31 layers, 124 calls at 49 - 4000 rows: 1.7 % behind the fastest form together, 3.4 % before.
 // Smaller layers compare it with the unsliced forms only, in rounds of 256 workgroups of 64 rows x 512 columns: 0.17 + 1.45 w
 // (1.3 w for the five- and six-bit formats).
 // OXQ_GGUF_GEMM_MIN_M: unset = by cost, 0 = never, n = the eight-wave form from n rows on whatever the cost;
-// OXQ_GGUF_GEMM_KS = 4 | 1: always | never the two-wave form; OXQ_GGUF_GEMM_SLICES = n: that many slices of it.
+// OXQ_GGUF_GEMM_KS = 4 | 1: always | never the two-wave form, 8 | 2: the form of 128 rows and 256 | 128 columns;
+// OXQ_GGUF_GEMM_SLICES = n: that many slices of the two-wave form.
 struct GgmGemmForm {
     int ks, slices;
+    int rows = 64;  // of a workgroup
 };
 struct GgmCost {
-    double chunk, round, wide;
+    double chunk, round, wide, wide128, pair128;
 };
 static GgmCost ggm_cost(int quant) {
     switch (quant) {
-    case OXQ_GGUF_Q4_0: case OXQ_GGUF_Q4_1: case OXQ_GGUF_Q4_K: return {1.45, 2.9, 2.6};
-    case OXQ_GGUF_Q8_0: return {1.6, 2.9, 2.9};
-    case OXQ_GGUF_Q6_K: return {1.75, 3.6, 3.4};
-    case OXQ_GGUF_Q2_K: case OXQ_GGUF_Q3_K: return {0.0, 3.5, 3.2};  // `round`: of 64 rows, below of fewer
-    default: return {1.6, 3.3, 3.0};  // Q5_0, Q5_1, Q5_K
+    case OXQ_GGUF_Q4_0: case OXQ_GGUF_Q4_1: case OXQ_GGUF_Q4_K: return {1.45, 2.9, 2.6, 1.80, 1.94};
+    case OXQ_GGUF_Q8_0: return {1.6, 2.9, 2.9, 1.78, 1.90};
+    case OXQ_GGUF_Q6_K: return {1.75, 3.6, 3.4, 2.15, 2.38};
+    case OXQ_GGUF_Q2_K: case OXQ_GGUF_Q3_K: return {0.0, 3.5, 3.2, 1.90, 2.25};  // `round`: of 64 rows, below of fewer
+    default: return {1.6, 3.3, 3.0, 1.85, 2.04};  // Q5_0, Q5_1, Q5_K
     }
 }
-static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
+// sliced: whether the caller can take K slices, whose partial sums a second launch adds from the workspace.  One that cannot (a fused
+// activation, a copy that lies there itself) chooses among whole sums of 128 rows; slices of 64 rows still win over them, and it
+// then takes another kernel.
+static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype, bool sliced) {
     const int64_t v = tune(ctx, OXQ_TUNE_GGUF_GEMM_MIN_M, -1);
     const bool narrow = ggm_narrow_format(quant);
     if (v == 0 || act_dtype != OXQ_BF16 || !(narrow ? M > 8 : ggm_format(quant) && M > 32)) return {0, 1};
     const int ks = tune(ctx, OXQ_TUNE_GGUF_GEMM_KS, 0);
     if (ks == 4) return {N % 64 == 0 ? 4 : 0, 1};
+    if (ks == 2 || ks == 8) return {ks == 2 ? 2 : 1, 1, 128};
     if (v > 0) return {N % 64 == 0 && M >= v ? 1 : 0, 1};
     const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int64_t row_tiles = ceil_div(M, (int64_t)64), groups = ceil_div(N, (int64_t)64), chunks = K / 128;
@@ -1587,13 +1666,27 @@ static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int6
             if (t < least || given > 0) least = given > 0 ? 0.0 : t, best = {4, (int)S};
         }
     }
+    // 128 rows x 256 | 128 columns a workgroup
+    if (!tune_given(ctx, OXQ_TUNE_GGUF_GEMM_SLICES) && ks == 0 && K < (1 << 22)) {
+        const int64_t row_tiles128 = ceil_div(M, (int64_t)128);
+        const double t8 = std::ceil((double)(ceil_div(N, (int64_t)256) * row_tiles128) / cus) * (7.0 + (double)chunks * c.wide128);
+        if (t8 < least) least = t8, best = {1, 1, 128};
+        const int64_t wgs = ceil_div(N, (int64_t)128) * row_tiles128, most = sliced && N % 4 == 0 ? std::min<int64_t>(ceil_div(chunks, (int64_t)2), 8) : 1;
+        for (int64_t S = 1; S <= most; ++S) {
+            const int64_t rounds = ceil_div(ceil_div(chunks, S), (int64_t)2);
+            if (ceil_div(chunks, 2 * rounds) != S || (S > 1 && (uint64_t)(S * M) * (uint64_t)N * 4 > ctx->workspace_bytes)) continue;
+            double t = std::ceil((double)(wgs * S) / cus) * (7.0 + (double)rounds * c.pair128);
+            if (S > 1) t += 3.5 + ((double)S * 8.0 + 2.0) * (double)M * (double)N / 4.2e6;
+            if (t < least) least = t, best = {2, (int)S, 128};
+        }
+    }
     if (narrow) {
         if (v > 0 || ks || tune(ctx, OXQ_TUNE_GGUF_GEMM_SLICES, 0) > 0) return best;
         const int64_t size = N * K;
         const double file = 6.0 + (double)(row_tiles * 64) * (double)size / 2e8 * (quant == OXQ_GGUF_Q3_K ? 1.15 : 1.0) * (M <= 16 ? 0.55 : M <= 32 ? 0.67 : 1.0);
         bool ahead;
-        if (row_tiles * groups >= 400) ahead = 1.15 * least < file;
-        else if (M > 64) ahead = size >= (M > 128 ? 1 << 22 : 1 << 23);
+        if (row_tiles * groups >= 400) ahead = least < file;
+        else if (M > 64) ahead = size >= (M > 512 ? 1 << 21 : M > 128 ? 1 << 22 : 1 << 23);
         else ahead = K >= 3072 && (size >= 1 << 24 || (size >= 1 << 23 && (K >= 7168 || M > 32)));
         return ahead ? best : GgmGemmForm{0, 1};
     }
@@ -1603,28 +1696,28 @@ static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int6
     if (2.6 + (double)ceil_div(chunks, (int64_t)8) * c.chunk * (ns == 4 ? 2.5 : 1.0) * (int_rounds > 1.0 ? 1.15 * int_rounds : 1.0) < least) best = {-1, 1};
     return best;
 }
-// sliced: whether the caller can take the form whose partial sums a second launch adds (a fused activation cannot)
 bool gguf_gemm_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype, bool sliced) {
-    const GgmGemmForm f = gguf_gemm_form(ctx, quant, M, K, N, act_dtype);
+    const GgmGemmForm f = gguf_gemm_form(ctx, quant, M, K, N, act_dtype, sliced);
     return f.ks > 0 && (sliced || f.slices == 1);
 }
 // rows beyond gguf_mfma_takes that the integer kernel takes in row tiles
 bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
-    return gguf_gemm_form(ctx, quant, M, K, N, act_dtype).ks < 0;
+    return gguf_gemm_form(ctx, quant, M, K, N, act_dtype, true).ks < 0;
 }
 
-template <int FMT, int MT, int KS>
+template <int FMT, int MT, int KS, int NS = 4>
 static int ggm_gemm_go(hipStream_t s, dim3 grid, const GgufProblem &p, float *part, int NG, int RT, int cslice) {
     static LdsGrant grant;  // one per instantiation
     const size_t lds = (size_t)2 * KS * 16 * MT * 256;
-    OXQ_HIP_CHECK(grant.ensure((const void *)ggm_gemm_kernel<FMT, MT, KS>, lds));
-    hipLaunchKernelGGL((ggm_gemm_kernel<FMT, MT, KS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w, (const uint16_t *)p.bias,
+    OXQ_HIP_CHECK(grant.ensure((const void *)ggm_gemm_kernel<FMT, MT, KS, NS>, lds));
+    hipLaunchKernelGGL((ggm_gemm_kernel<FMT, MT, KS, NS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w, (const uint16_t *)p.bias,
                        (uint16_t *)p.y, part, (int)p.M, (int)p.K, (int)p.N, NG, RT, p.act, cslice, (int)p.gate_half);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
 template <int FMT>
-static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, float *part, int NG, int RT, int ks, int cslice) {
+static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, float *part, int NG, int RT, int ks, int cslice, int rows) {
+    if (rows == 128) return ks == 2 ? ggm_gemm_go<FMT, 8, 2, 2>(s, grid, p, part, NG, RT, cslice) : ggm_gemm_go<FMT, 8, 1, 2>(s, grid, p, part, NG, RT, cslice);
     if (ks == 1) return ggm_gemm_go<FMT, 4, 1>(s, grid, p, part, NG, RT, cslice);
     // up to 48 rows: the 64-row tile without its fourth row tile of MFMAs, and of x (14336 x 4096 at 48 rows, us: Q4_K 21.4 ->
     // 20.3, Q6_K 25.9 -> 24.5, Q8_0 23.3 -> 22.2)
@@ -1637,24 +1730,23 @@ static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, floa
 
 // p.w is the matrix-core copy; p.act as for launch_gguf_mfma; p.gate_half: the copy of a fused gate|up layer whose
 // activation this call leaves out
-int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
-    const int rows = 64;
-    GgmGemmForm form = gguf_gemm_form(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);
+int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, bool sliced) {
+    sliced = sliced && !p.act;
+    GgmGemmForm form = gguf_gemm_form(ctx, p.quant, p.M, p.K, p.N, p.act_dtype, sliced);
     if (form.ks <= 0) form = {1, 1};  // a caller that asks for this kernel gets it
-    if (p.act) form.slices = 1;
-    const int ks = form.ks, spw = 8 / ks;
-    const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)64), (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows);
+    if (!sliced) form.slices = 1;
+    const int ks = form.ks, spw = 8 / ks, rows = form.rows;
+    const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)(rows == 128 ? 32 : 64)), (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows);
     const int64_t wgs = ks == 1 ? pk4g_workgroups(RT, NG) : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "gguf prefill matmul: m = %lld exceeds the grid", (long long)p.M);
     const int64_t chunks = p.K / 128;
-    const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)4) * 4) : (int)chunks;
+    const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)ks) * ks) : (int)chunks;
     dim3 grid((unsigned)wgs, (unsigned)form.slices);
-    char name[64];
-    if (form.slices > 1)
-        snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%dk4_s%d", ggm_name(p.quant), rows, spw, form.slices);
-    else
-        snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%d%s%s", ggm_name(p.quant), rows, spw, ks > 1 ? "k4" : "",
-                 p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
+    // the family (eight waves side by side, or K split inside the workgroup too), then the rows where they are not the 64 of its first form
+    char name[64], slices[16] = "";
+    if (form.slices > 1) snprintf(slices, sizeof slices, "_s%d", form.slices);
+    snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r64x%s%s%s%s", ggm_name(p.quant), ks > 1 ? "2k4" : "8", slices, rows == 128 ? "_r128" : "",
+             p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), form.slices, 1, form.slices > 1 ? (size_t)form.slices * p.M * p.N * 4 : 0);
     if (ctx->plan_only) {
         if (form.slices > 1) add_launch(ctx);
@@ -1666,7 +1758,7 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     float *part = (float *)ctx->workspace;
     int rc;
 #define OXQ_GGM(F) \
-    case F: rc = ggm_gemm_go_form<F>(s, grid, p, part, (int)NG, (int)RT, ks, cslice); break
+    case F: rc = ggm_gemm_go_form<F>(s, grid, p, part, (int)NG, (int)RT, ks, cslice, rows); break
     switch (p.quant) {
         OXQ_GGM(OXQ_GGUF_Q4_0);
         OXQ_GGM(OXQ_GGUF_Q8_0);

@@ -1107,7 +1107,7 @@ int oxq_gguf_quant_matmul(oxq_ctx *ctx, void *stream, const oxq_tensor *x,
         if (rc != OXQ_OK) return rc;
         GgufProblem q = p;
         q.w = (const uint8_t *)ctx->workspace;
-        rc = launch_gguf_gemm(ctx, (hipStream_t)stream, q);
+        rc = launch_gguf_gemm(ctx, (hipStream_t)stream, q, false);  // (the partial sums of slices would lie on the copy)
         ctx->plan.launches = 2;
         return rc;
     }
@@ -1134,7 +1134,7 @@ int oxq_gguf_quant_mul_mm(oxq_ctx *ctx, void *stream, const oxq_tensor *x,
         if (rc != OXQ_OK) return rc;
         GgufProblem q = p;
         q.w = (const uint8_t *)ctx->workspace;
-        rc = launch_gguf_gemm(ctx, (hipStream_t)stream, q);
+        rc = launch_gguf_gemm(ctx, (hipStream_t)stream, q, false);  // (the partial sums of slices would lie on the copy)
         ctx->plan.launches = 2;
         return rc;
     }
@@ -2410,7 +2410,7 @@ int oxq_qlinear_forward(oxq_qlinear *l, void *stream, const oxq_tensor *x, const
         p.w = (const uint8_t *)l->mm;
         p.act = l->act;
         if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype, false) && p.N % 64 == 0)
-            return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p);
+            return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p, false);
         return launch_gguf_mfma(l->ctx, (hipStream_t)stream, p);
     }
     OXQ_TRY(check_gguf(l->ctx, decode ? "GgufQuantMatmul" : "GgufQuantMulMM", decode, false, &x2,
@@ -2450,8 +2450,8 @@ static int qlinear_forward_unfused(oxq_qlinear *l, void *stream, const oxq_tenso
 }
 
 // whether `rows` rows of a bf16 layer run whole sums on its matrix-core copy, in the prefill kernel or in row tiles of the
-// integer kernel (a fused gate|up layer then keeps its activation in that kernel's epilogue, and the plain layer takes
-// the same kernel: the same bits)
+// integer kernel (a fused gate|up layer then keeps its activation in that kernel's epilogue; the plain layer takes
+// the same kernel, the same bits, or K slices of it)
 static bool qlinear_prefill_on_copy(const oxq_qlinear *l, int64_t rows) {
     if (l->resident && l->mfma && gguf_mfma_tiles(l->ctx, l->quant, rows, l->in_features, l->out_features, l->out_dtype)) return true;
     return l->resident && l->mfma && l->out_features % 64 == 0 &&
