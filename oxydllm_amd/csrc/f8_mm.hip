@@ -9,12 +9,13 @@
 //   f8_tile_kernel   16 MT rows x NS strips of 16 columns a workgroup; its eight waves split K, each stages its own x and
 //                    weights, no barrier before the sum - up to a few hundred rows of an expert;
 //   f8_gemm_kernel   64 rows x two groups of 64 columns with K split over four waves each (KS = 4, and over workgroups
-//                    where columns are few), or x eight groups (KS = 1).
+//                    where columns are few), or x eight groups (KS = 1);
+//   f8_gemm128_kernel  128 rows x four groups of 32 columns with K split over two waves each, or x eight groups.
 // A strip's rows lie K bytes apart, so loads that fill operands directly touch 16 lines each, one lane at a time: 64
 // cycles of the address unit for 1 KB, and that bound the first version (2.45 us for 64 x 512 x 128 a CU).  Loads now
 // take whole 128-byte (64-byte) runs of a row and turn to operand order through the wave's own LDS: 2.1 us.
 // Measured, us, before (GEMV / staged tiles) -> now: 5632 x 5632 at 1, 33, 96, 256, 1024 rows 11.3 -> 8.3, 22.9 -> 15.9,
-// 31.5 -> 18.4, 52 -> 34, 144 -> 102; 2048 x 5632 at 3, 33, 96 rows 8.5 -> 4.8, 12.5 -> 9.0, 17.0 -> 10.2; 512 x 768 at
+// 31.5 -> 18.4, 52 -> 34, 144 -> 75; 2048 x 5632 at 3, 33, 96 rows 8.5 -> 4.8, 12.5 -> 9.0, 17.0 -> 10.2; 512 x 768 at
 // 33 rows 6.6 -> 3.3.
 // Needs block_r a multiple of 16 (a strip has one scale a chunk), block_c 128 times a power of two; other grids keep
 // blockq_mm.hip.
@@ -28,6 +29,9 @@
 
 namespace oxq {
 
+__device__ __forceinline__ uint32_t f8_pair(float a, float b) {
+    return (uint32_t)BF16Traits::from_f32(a) | ((uint32_t)BF16Traits::from_f32(b) << 16);
+}
 // eight bytes times the scale as four bf16 pairs: exact conversion, one product, one rounding each
 __device__ __forceinline__ void f8_operand(uint32_t w0, uint32_t w1, float s, uint32_t (&b)[4]) {
 #pragma unroll
@@ -192,6 +196,88 @@ __global__ __launch_bounds__(NW * 64) void f8_tile_kernel(const uint16_t *__rest
         }
     }
     pk4n_epilogue<TT, MT, NS, NW, true>(acc, nullptr, y, nullptr, M, N, j, m0, wave, lane);
+}
+
+// The sums of a workgroup's waves: column groups of 16 NS, wave = column group + (8 / KS) x share of K.  All row tiles of this wave
+// (KS = 1), or MT / KS of them summed over the waves of the column group, in K order: the same sum whatever the timing.
+template <int MT, int NS, int KS>
+__device__ __forceinline__ void f8_gemm_finish(float4_t (&acc)[MT][NS], uint16_t *__restrict__ y, float *__restrict__ part, int M, int N,
+                                               int m0, int n0, int wave, int lane, bool live) {
+    static_assert(MT % KS == 0, "the waves of a column group finish as many row tiles each");
+    constexpr int SPW = 8 / KS, FT = MT / KS;
+    extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
+    const int ni = lane & 15, kb = lane >> 4, ws = wave % SPW, kq = wave / SPW;
+    float4_t fin[FT][NS];
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int f = 0; f < NS; ++f) fin[mt][f] = acc[mt][f];
+    } else {
+        // over the buffers of x, once the zeros requested past the last round are in them
+        typedef float part_t __attribute__((ext_vector_type(NS)));
+        pk4g_wait_vmcnt<0>();
+        __syncthreads();
+        part_t *red = (part_t *)pk4_lds;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                part_t v;
+#pragma unroll
+                for (int f = 0; f < NS; ++f) v[f] = acc[mt][f][e];
+                red[((wave * MT + mt) * 4 + e) * 64 + lane] = v;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < FT; ++t) {
+#pragma unroll
+            for (int f = 0; f < NS; ++f) fin[t][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const part_t v = red[(((k * SPW + ws) * MT + FT * kq + t) * 4 + e) * 64 + lane];
+#pragma unroll
+                    for (int f = 0; f < NS; ++f) fin[t][f][e] += v[f];
+                }
+        }
+    }
+    if (!live) return;
+    // row 16 mt + 4 kb + e, column n0 + 16 f + ni
+    // In groups of four columns, one store each: with 2 (4) bytes a lane and store the epilogue of 64 x 512 took 7 us and that of
+    // 128 x 256 as much (512 x 768 at 65 - 2048 rows 20 -> 15 and 18.6 -> 12.4 us a launch).
+    if (N % 4 == 0 && (gridDim.y > 1 || ((uintptr_t)y & 7) == 0)) {
+#pragma unroll
+        for (int t = 0; t < FT; ++t)
+#pragma unroll
+            for (int f = 0; f < NS; ++f) {
+                const int row = m0 + 16 * (FT * kq + t) + 4 * kb + (ni & 3), n = n0 + 16 * f + (ni & 12);
+                const bool there = row < M && n < N;
+                if (gridDim.y > 1) {
+                    const float4_t v = quad_turn32(fin[t][f], lane);
+                    if (there) *(float4_t *)(part + ((size_t)blockIdx.y * M + row) * N + n) = v;
+                } else {
+                    const uint2 v = quad_turn16(f8_pair(fin[t][f][0], fin[t][f][1]), f8_pair(fin[t][f][2], fin[t][f][3]), lane);
+                    if (there) *(uint2 *)(y + (size_t)row * N + n) = v;
+                }
+            }
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < FT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int row = m0 + 16 * (FT * kq + t) + 4 * kb + e;
+            if (row >= M) continue;
+#pragma unroll
+            for (int f = 0; f < NS; ++f) {
+                const int n = n0 + 16 * f + ni;
+                if (n >= N) continue;
+                if (gridDim.y > 1) part[((size_t)blockIdx.y * M + row) * N + n] = fin[t][f][e];
+                else y[(size_t)row * N + n] = BF16Traits::from_f32(fin[t][f][e]);
+            }
+        }
 }
 
 template <int MT, int KS>
@@ -374,51 +460,185 @@ __global__ __launch_bounds__(512) void f8_gemm_kernel(const uint16_t *__restrict
         if (r < NR) chunk(r, std::integral_constant<int, 0>{});
     }
 
-    // the finished tile rows of this wave: all of them (KS = 1), or row tile kq summed over the column group's waves
-    constexpr int FT = KS == 1 ? MT : 1;
-    float4_t fin[FT][4];
+    f8_gemm_finish<MT, 4, KS>(acc, y, part, M, N, m0, n0, wave, lane, live);
+}
+
+// 128 rows, a wave has two strips: a decoded weight serves eight row tiles instead of four (two vector instructions an MFMA), at the
+// price of fragments of x that feed two MFMAs.  KS = 1: 256 columns, KS = 2: 128 with K over the two waves of a column group.
+// What bounds it: LDS, which a round asks for 1.1 of its 1.6 us (40 KB a wave and chunk at 128 bytes a clock; the MFMAs 0.85).
+// us, best of the forms of 64 rows -> 128: 5632 x 5632 at 128 / 400 / 640 / 1024 rows 32 / 68 / 70 / 100 -> 24 / 48 / 50 / 75, 4096 x
+// 4096 at 640 / 1024 53 / 55 -> 38 / 42, 2048 x 5632 at 640 / 1024 34 / 46 -> 24 / 34.  Bits as f8_gemm_kernel's (KS = 1).
+template <int KS>
+__global__ __launch_bounds__(512) void f8_gemm128_kernel(const uint16_t *__restrict__ x, const uint8_t *__restrict__ w,
+                                                         const float *__restrict__ scales, uint16_t *__restrict__ y,
+                                                         float *__restrict__ part, int M, int K, int N, int NG, int RT,
+                                                         int cslice, int block_r, int cshift, int s_cols, int s_rows) {
+    typedef MfmaOps<BF16Traits> Ops;
+    constexpr int MT = 8, NS = 2, SPW = 8 / KS, ROWS = 16 * MT, XBUF = KS * ROWS * 256, XV = ROWS / 4 / SPW, OOB = 0x7FFFFF00;
+    constexpr int RING = 6;  // vector loads of weights and scales between two rounds' loads of x
+    extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ni = lane & 15, kb = lane >> 4;
+    const int ws = wave % SPW, kq = wave / SPW;  // the wave's column group of the workgroup, and its share of K
+    int rt, g;
     if constexpr (KS == 1) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) fin[mt][f] = acc[mt][f];
+        if ((int)blockIdx.x >= RT * NG) return;  // the whole workgroup, before any barrier
+        pk4g_tile_of((int)blockIdx.x, RT, NG, rt, g);
     } else {
-        // over the buffers of x, once the zeros requested past the last round are in them
-        pk4g_wait_vmcnt<0>();
-        __syncthreads();
-        float4_t *red = (float4_t *)pk4_lds;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                red[((wave * MT + mt) * 4 + e) * 64 + lane] = float4_t{acc[mt][0][e], acc[mt][1][e], acc[mt][2][e], acc[mt][3][e]};
-        __syncthreads();
-#pragma unroll
-        for (int f = 0; f < 4; ++f) fin[0][f] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < KS; ++k)  // K order: the same sum whatever the timing
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float4_t v = red[(((k * SPW + ws) * MT + kq) * 4 + e) * 64 + lane];
-                fin[0][0][e] += v[0], fin[0][1][e] += v[1], fin[0][2][e] += v[2], fin[0][3][e] += v[3];
-            }
+        rt = (int)blockIdx.x / NG, g = (int)blockIdx.x % NG;
     }
-    if (!live) return;
-    // row 16 mt + 4 kb + e, column n0 + 16 f + ni
+    const int n0 = 16 * NS * (g * SPW + ws);
+    const bool live = n0 < N;
+    const int m0 = rt * ROWS;
+    const int NC = K >> 7;
+    const int cbeg = (int)blockIdx.y * cslice, cend = min(NC, cbeg + cslice);
+    const int NR = (cend - cbeg + KS - 1) / KS;
+    const int xrows = min(M - m0, ROWS), wrows = live ? min(N - n0, 16 * NS) : 0;
+
+    const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(w, 0u);
+    const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(w + (size_t)(live ? n0 : 0) * K, (uint32_t)wrows * (uint32_t)K);
+    const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(x + (size_t)m0 * K, (uint32_t)xrows * (uint32_t)K * 2u);
+    const __amdgpu_buffer_rsrc_t rs_s = make_rsrc(scales, (uint32_t)(s_rows * s_cols) * 4u);
+    // a chunk of the wave's columns is 4 KB: load q brings rows 8 q + lane / 8 whole, and the wave's own LDS turns them to
+    // operands, the 16-byte pieces of row r swapped by r % 8
+    int voff_w[4], soff_s[NS];
 #pragma unroll
-    for (int t = 0; t < FT; ++t)
+    for (int q = 0; q < 4; ++q) {
+        const int r = 8 * q + (lane >> 3);
+        voff_w[q] = r < wrows ? r * K + (lane & 7) * 16 : OOB;
+    }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = m0 + 16 * (KS == 1 ? t : kq) + 4 * kb + e;
-            if (row >= M) continue;
+    for (int f = 0; f < NS; ++f) soff_s[f] = min((n0 + 16 * f) / block_r, s_rows - 1) * s_cols;
+    unsigned char *wslot = pk4_lds + 2 * XBUF + wave * 4096;
+    const int w_wr = (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
+    int w_rd[2];  // half h of a chunk: two steps
 #pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                const int n = n0 + 16 * f + ni;
-                if (n >= N) continue;
-                if (gridDim.y > 1) part[((size_t)blockIdx.y * M + row) * N + n] = fin[t][f][e];
-                else y[(size_t)row * N + n] = TT::from_f32(fin[t][f][e]);
+    for (int h = 0; h < 2; ++h) w_rd[h] = ni * 128 + (((4 * h + kb) ^ (ni & 7)) << 4);
+    int xo[XV];
+#pragma unroll
+    for (int q = 0; q < XV; ++q) {
+        const int r = 4 * (ws * XV + q) + (lane >> 4);
+        xo[q] = r * K * 2 + (((lane & 15) ^ (r & 15)) << 4);
+    }
+    int a_rd[4];
+#pragma unroll
+    for (int st = 0; st < 4; ++st) a_rd[st] = ni * 256 + ((pk4_x_chunk<1>(st, kb) ^ ni) << 4);
+
+    u32x4_t wr[4], wq[2][NS];  // as loaded; [half][strip]: as operands
+    float sr[2][NS];
+    auto dma_x = [&](int r) {
+        const int i = cbeg + KS * r + kq;
+        const __amdgpu_buffer_rsrc_t rs = i < cend ? rs_x : rs_none;
+#pragma unroll
+        for (int q = 0; q < XV; ++q)
+            pk4g_load_lds16(rs, pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256) + (ws * XV + q) * 1024, xo[q], i * 256);
+    };
+    auto load_w = [&](int i) {
+        const __amdgpu_buffer_rsrc_t rw = i < cend ? rs_w : rs_none;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) wr[q] = __builtin_amdgcn_raw_buffer_load_b128(rw, voff_w[q], i * 128, 0);
+    };
+    auto load_s = [&](int i, float (&s)[NS]) {
+        const __amdgpu_buffer_rsrc_t rs = i < cend ? rs_s : rs_none;
+#pragma unroll
+        for (int f = 0; f < NS; ++f) s[f] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, 0, (soff_s[f] + (i >> cshift)) * 4, 0));
+    };
+    auto put_w = [&](int q) { *(u32x4_t *)(wslot + q * 1024 + w_wr) = wr[q]; };
+    auto get_w = [&](int h, int f) { wq[h][f] = *(const u32x4_t *)(wslot + f * 2048 + w_rd[h]); };
+
+    // The pipeline of f8_gemm_kernel with a group of two products: operands decoded a step ahead, fragments of x read AH groups
+    // ahead, the barrier AH groups before the round's end.  The next chunk's weights go into LDS in step 1 (this chunk's were all
+    // read before it began) and come out by halves in steps 2 and 3, each behind the last decode from the half it replaces.
+    constexpr int GROUPS = 4 * MT, AH = 3;
+    u32x4_t a[4];
+    uint32_t b[2][NS][4];
+    auto read_x = [&](int r, int u) { a[u & 3] = *(const u32x4_t *)(pk4_lds + (r & 1) * XBUF + kq * (ROWS * 256) + (u % MT) * 4096 + a_rd[u / MT]); };
+    auto decode = [&](int st, int f, int pp, const float (&sc)[NS]) {
+        const uint32_t word = wq[st >> 1][f][2 * (st & 1) + (pp >> 1)];
+        const float2_t v = (pp & 1) ? (float2_t)__builtin_amdgcn_cvt_pk_f32_fp8((int)word, true)
+                                    : (float2_t)__builtin_amdgcn_cvt_pk_f32_fp8((int)word, false);
+        b[st & 1][f][pp] = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{v[0] * sc[f], v[1] * sc[f]}, bf16x2_t));
+    };
+
+    dma_x(0);
+    __builtin_amdgcn_sched_barrier(0);  // requests keep this order: the wait counts rely on it
+    load_w(cbeg + kq);
+    load_s(cbeg + kq, sr[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    float4_t acc[MT][NS];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int f = 0; f < NS; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) put_w(q);
+#pragma unroll
+    for (int f = 0; f < NS; ++f) get_w(0, f), get_w(1, f);
+    pk4g_wait_vmcnt<0>();
+    __syncthreads();
+    dma_x(1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(cbeg + KS + kq);
+    load_s(cbeg + KS + kq, sr[1]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < AH; ++u) read_x(0, u);
+#pragma unroll
+    for (int f = 0; f < NS; ++f)
+#pragma unroll
+        for (int pp = 0; pp < 4; ++pp) decode(0, f, pp, sr[0]);
+
+    auto chunk = [&](int r, auto cur_c) {
+        constexpr int CUR = decltype(cur_c)::value;
+        const int i = cbeg + KS * r + kq;  // past the slice (a ragged last round): zeros from both streams
+#pragma unroll
+        for (int u = 0; u < GROUPS; ++u) {
+            const int st = u / MT, mt = u % MT;
+            if (u == GROUPS - AH) {
+                __builtin_amdgcn_sched_barrier(0);
+                pk4g_wait_vmcnt<RING>();  // this wave's part of the next round of x (requested before the weights) is in LDS
+                __syncthreads();          // and every wave holds its last fragment of this round: the buffer is free
+                dma_x(r + 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (u + AH < GROUPS) read_x(r, u + AH);
+            else read_x(r + 1, u + AH - GROUPS);
+            if (st == 1 && mt < 4) put_w(mt);
+            if (st == 2 && mt < NS) get_w(0, mt);
+            if (st == 3 && mt < NS) get_w(1, mt);
+            decode((st + 1) & 3, mt >> 2, mt & 3, sr[st < 3 ? CUR : CUR ^ 1]);
+#pragma unroll
+            for (int f = 0; f < NS; ++f) {
+                uint32_t am[4] = {a[u & 3][0], a[u & 3][1], a[u & 3][2], a[u & 3][3]};
+                acc[mt][f] = Ops::mfma(am, b[st & 1][f], acc[mt][f]);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (st == 1 && mt < 4) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            if (st >= 2 && mt < NS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+            for (int f = 0; f < NS; ++f) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+            }
+            if (mt == MT - 1 && (st == 1 || st == 2)) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (st == 1) load_w(i + 2 * KS);
+                else load_s(i + 2 * KS, sr[CUR]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
+    };
+    {
+        int r = 0;
+        for (; r + 1 < NR; r += 2) {
+            chunk(r, std::integral_constant<int, 0>{});
+            chunk(r + 1, std::integral_constant<int, 1>{});
+        }
+        if (r < NR) chunk(r, std::integral_constant<int, 0>{});
+    }
+    f8_gemm_finish<MT, NS, KS>(acc, y, part, M, N, m0, n0, wave, lane, live);
 }
 
 // ---------------------------------------------------------------------------
@@ -443,14 +663,18 @@ static bool f8_shape_ok(const F8Problem &p) {
 // columns stand between the strips and the 64-column groups (fitted over 512..7168 x 768..7168 at 20..320 rows, 1.15 x the fit:
 // ahead at 163 of 480 points, by 1.28 x there, and behind at none).  Us, without them -> with: 3968 x 3456 at 33, 64, 96 rows
 // 13.1 -> 9.8, 13.3 -> 10.1, 15.1 -> 11.4; 5632 x 5632 at 33 rows 15.7 -> 12.1; 1408 x 2048 at 96 rows 6.7 -> 4.9.
-//   64 rows x 128 columns, K over waves  rounds x (7.5 + 2.6 x rounds of four chunks); K slices add a second launch and
+//   64 rows x 128 columns, K over waves  rounds x (7.5 + 2.45 x rounds of four chunks); K slices add a second launch and
 //                                        the partials' traffic
-//   64 rows x 512 columns                rounds x (7 + 2.3 x chunks)
+//   128 rows x 128 columns, K over waves rounds x (6.7 + 1.75 x rounds of two chunks); K slices likewise
+//   64 rows x 512 columns                rounds x (7 + 2.1 x chunks)
+//   128 rows x 256 columns               rounds x (7.5 + 1.6 x chunks)
+// (The last four fitted again over 40 layers of 512..7168 x 512..7168 at 17..2048 rows, every form forced at each of 160 calls:
+// 0.9 % behind the fastest form together, 148 within 5 %, 157 within 12 %.)
 //   the staged tiles of blockq_mm.hip    from 33 rows and up to K = 2048, where a workgroup of eight waves has too little K
 //                                        to share: several small workgroups a CU win at some shapes
 struct F8Form {
-    int kind, ns, slices;  // kind 0: tiles, 4 | 1: KS of the gemm kernel, -1: blockq_mm.hip
-    int mt = 0;            // tiles of 16 mt rows (0: by the rows at hand)
+    int kind, ns, slices;  // kind 0: tiles, 4 | 1: KS of the gemm kernel of 64 rows, 2: the gemm kernel of 128, -1: blockq_mm.hip
+    int mt = 0;            // tiles of 16 mt rows (0: by the rows at hand); KS of the kernel of 128 rows
 };
 static F8Form f8_form(const oxq_ctx *ctx, const F8Problem &p) {
     const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256, mn = (double)p.M * (double)p.N;
@@ -471,16 +695,29 @@ static F8Form f8_form(const oxq_ctx *ctx, const F8Problem &p) {
     offer(5, 1.4 + std::ceil(pairs * tiles / cus) * (1.15 + 1.8 * per_wave), {0, 2, 1, 2});
     offer(6, 1.4 + std::ceil(pairs * (double)ceil_div(p.M, (int64_t)48) / cus) * (1.7 + 2.0 * per_wave), {0, 2, 1, 3});
     if (p.M <= 32) return best;
+    const auto sum = [&](int64_t S, double us, double rate) { return S > 1 ? us + ((double)S * 8.0 + 2.0) * mn / rate : 0.0; };  // the second launch
     const int64_t rt = ceil_div(p.M, (int64_t)64), wgs = ceil_div(groups, (int64_t)2) * rt;
     const int64_t most = p.N % 4 == 0 ? std::min<int64_t>(ceil_div(chunks, (int64_t)4), 32) : 1;
     for (int64_t S = 1; S <= most; ++S) {
         if (fs > 0 && S != std::min<int64_t>(fs, most)) continue;
         const int64_t rounds = ceil_div(ceil_div(chunks, S), (int64_t)4);
         if (ceil_div(chunks, 4 * rounds) != S || (S > 1 && (uint64_t)(S * p.M) * (uint64_t)p.N * 4 > ctx->workspace_bytes)) continue;
-        offer(4, std::ceil((double)(wgs * S) / cus) * (7.5 + (double)rounds * 2.6) + (S > 1 ? 3.8 + ((double)S * 8.0 + 2.0) * mn / 3.84e6 : 0.0),
+        offer(4, std::ceil((double)(wgs * S) / cus) * (7.5 + (double)rounds * 2.45) + sum(S, 2.5, 4e6),
               {4, 1, (int)S});
     }
-    offer(1, std::ceil((double)(ceil_div(groups, (int64_t)8) * rt) / cus) * (7.0 + (double)chunks * 2.3), {1, 1, 1});
+    offer(1, std::ceil((double)(ceil_div(groups, (int64_t)8) * rt) / cus) * (7.0 + (double)chunks * 2.1), {1, 1, 1});
+    if (p.K < (1 << 22)) {  // 128 rows x 256 | 128 columns
+        const int64_t rt128 = ceil_div(p.M, (int64_t)128), wgs128 = ceil_div(p.N, (int64_t)128) * rt128;
+        offer(9, std::ceil((double)(ceil_div(p.N, (int64_t)256) * rt128) / cus) * (7.5 + (double)chunks * 1.6), {2, 1, 1, 1});
+        const int64_t most2 = p.N % 4 == 0 ? std::min<int64_t>(ceil_div(chunks, (int64_t)2), 8) : 1;
+        for (int64_t S = 1; S <= most2; ++S) {
+            if (fs > 0 && S != std::min<int64_t>(fs, most2)) continue;
+            const int64_t rounds = ceil_div(ceil_div(chunks, S), (int64_t)2);
+            if (ceil_div(chunks, 2 * rounds) != S || (S > 1 && (uint64_t)(S * p.M) * (uint64_t)p.N * 4 > ctx->workspace_bytes)) continue;
+            offer(10, std::ceil((double)(wgs128 * S) / cus) * (6.7 + (double)rounds * 1.75) + sum(S, 1.5, 6e6),
+                  {2, 1, (int)S, 2});
+        }
+    }
     if (p.K <= 2048) offer(8, 4.8 + 0.38 * (double)chunks + mn * 1.0e-6 + mn * (double)p.K * 3.5e-9, {-1, 1, 1});
     return best;
 }
@@ -515,6 +752,18 @@ static int f8_gemm_go(hipStream_t s, dim3 grid, const F8Problem &p, float *part,
     return OXQ_OK;
 }
 
+template <int KS>
+static int f8_gemm128_go(hipStream_t s, dim3 grid, const F8Problem &p, float *part, int NG, int RT, int cslice) {
+    static LdsGrant grant;
+    const size_t lds = (size_t)2 * KS * 128 * 256 + 8 * 4096;
+    OXQ_HIP_CHECK(grant.ensure((const void *)f8_gemm128_kernel<KS>, lds));
+    hipLaunchKernelGGL((f8_gemm128_kernel<KS>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w, p.scales, (uint16_t *)p.y, part,
+                       (int)p.M, (int)p.K, (int)p.N, NG, RT, cslice, (int)p.block_r, __builtin_ctzll((unsigned long long)p.block_c) - 7, (int)p.s_cols,
+                       (int)f8_s_rows(p));
+    OXQ_HIP_CHECK(hipGetLastError());
+    return OXQ_OK;
+}
+
 int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
     const F8Form form = f8_form(ctx, p);
     char name[64];
@@ -529,20 +778,22 @@ int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
         if (mt == 3) return f8_tile_go<3, 4, 12>(s, grid, p);
         return form.ns == 4 ? f8_tile_rows<4>(s, grid, p) : f8_tile_rows<1>(s, grid, p);
     }
-    const int ks = form.kind, spw = 8 / ks;
-    const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)64), (int64_t)spw), RT = ceil_div(p.M, (int64_t)64), chunks = p.K / 128;
+    const bool tall = form.kind == 2;  // 128 rows, 32 columns a wave
+    const int ks = tall ? form.mt : form.kind, spw = 8 / ks, rows = tall ? 128 : 64;
+    const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)(tall ? 32 : 64)), (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows), chunks = p.K / 128;
     const int64_t wgs = ks == 1 ? pk4g_workgroups(RT, NG) : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "f8 matmul: m = %lld exceeds the grid", (long long)p.M);
-    const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)4) * 4) : (int)chunks;
+    const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)ks) * ks) : (int)chunks;
     dim3 grid((unsigned)wgs, (unsigned)form.slices);
-    snprintf(name, sizeof name, "f8_mul_mm_bf16_r64x%d%s", spw, ks > 1 ? "k4" : "");
+    snprintf(name, sizeof name, "f8_mul_mm_bf16_r%dx%d%s", rows, spw, ks == 4 ? "k4" : ks == 2 ? "k2" : "");
     set_plan(ctx, name, grid, dim3(512), form.slices, 1, form.slices > 1 ? (size_t)form.slices * p.M * p.N * 4 : 0);
     if (ctx->plan_only) {
         if (form.slices > 1) add_launch(ctx);
         return OXQ_OK;
     }
     float *part = (float *)ctx->workspace;
-    const int rc = ks == 4 ? f8_gemm_go<4>(s, grid, p, part, (int)NG, (int)RT, cslice) : f8_gemm_go<1>(s, grid, p, part, (int)NG, (int)RT, cslice);
+    const int rc = tall ? (ks == 2 ? f8_gemm128_go<2>(s, grid, p, part, (int)NG, (int)RT, cslice) : f8_gemm128_go<1>(s, grid, p, part, (int)NG, (int)RT, cslice))
+                   : ks == 4 ? f8_gemm_go<4>(s, grid, p, part, (int)NG, (int)RT, cslice) : f8_gemm_go<1>(s, grid, p, part, (int)NG, (int)RT, cslice);
     if (rc != OXQ_OK || form.slices == 1) return rc;
     return launch_splitk_reduce(ctx, s, part, nullptr, p.y, p.M, p.N, form.slices, OXQ_BF16);
 }

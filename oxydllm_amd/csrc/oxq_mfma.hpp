@@ -47,4 +47,46 @@ template <> struct MfmaOps<BF16Traits> {
     }
 };
 
+// An accumulator tile holds four rows of one column a lane; stored like that a store instruction writes 2 bytes a lane in pieces of
+// 32.  These turn the 4 x 4 of a quad of lanes: lane q gets columns 0 .. 3 of row q, one 8 (16) byte store.
+__device__ __forceinline__ uint32_t quad_xor(uint32_t v, std::integral_constant<int, 1>) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);  // quad_perm 1 0 3 2
+}
+__device__ __forceinline__ uint32_t quad_xor(uint32_t v, std::integral_constant<int, 2>) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false);  // quad_perm 2 3 0 1
+}
+// rows 0, 1 and 2, 3 as pairs of 16 bits
+__device__ __forceinline__ uint2 quad_turn16(uint32_t r01, uint32_t r23, int lane) {
+    constexpr std::integral_constant<int, 1> by1{};
+    constexpr std::integral_constant<int, 2> by2{};
+    const uint32_t sel = (lane & 1) ? 0x03020706u : 0x05040100u;  // of the even lane's column, then the odd one's
+    const uint32_t a = perm_b32(quad_xor(r01, by1), r01, sel), b = perm_b32(quad_xor(r23, by1), r23, sel);  // rows q & 1, 2 + (q & 1)
+    const uint32_t got = quad_xor((lane & 2) ? a : b, by2);
+    return (lane & 2) ? uint2{got, b} : uint2{a, got};
+}
+__device__ __forceinline__ float4_t quad_turn32(float4_t v, int lane) {
+    constexpr std::integral_constant<int, 1> by1{};
+    constexpr std::integral_constant<int, 2> by2{};
+    const bool odd = lane & 1, high = lane & 2;
+    uint32_t e[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x = v[i];
+        e[i] = __builtin_bit_cast(uint32_t, x);
+    }
+    uint32_t p[2][2];  // columns q & 2, (q & 2) + 1 of rows q & 1 and 2 + (q & 1)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t mine = odd ? e[2 * h + 1] : e[2 * h], got = quad_xor(odd ? e[2 * h] : e[2 * h + 1], by1);
+        p[h][0] = odd ? got : mine, p[h][1] = odd ? mine : got;
+    }
+    float4_t o;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const uint32_t got = quad_xor(high ? p[0][c] : p[1][c], by2);
+        o[c] = __builtin_bit_cast(float, high ? got : p[0][c]), o[2 + c] = __builtin_bit_cast(float, high ? p[1][c] : got);
+    }
+    return o;
+}
+
 }  // namespace oxq
