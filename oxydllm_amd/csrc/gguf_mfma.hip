@@ -1245,6 +1245,11 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
         }
     }
     if (!live || (KS > MT && kq >= MT)) return;
+    // 128 rows: stores of four columns (a quad of lanes turns its 4 x 4 values; four neighbours of the copy are neighbours of y,
+    // ggm_src_row) where rows of y begin on 8 bytes, not of one: Q4_K 1024 x 8192 at 300 / 2048 rows 14.9 -> 14.3 / 49.4 -> 47.6 us, 4096 x
+    // 14336 at 2048 270 -> 268.  With one row tile a wave, as in the forms of 64 rows, they gain nothing (Q6_K 4096 x 4096 at 300 33.0 / 34.3).
+    const bool by4 = NS == 2 && ((uintptr_t)y & 7) == 0 && N % 4 == 0;
+    const int quad = ni & 3;
     if (act) {
         // Fused gate|up layer (ggm_src_row): strip NS j + f holds gate columns 8 (NS j + f) .. + 7 in lanes ni < 8 and
         // the up columns they meet in lanes ni + 8.  The two lanes of a pair exchange their values (row_ror:8) and finish
@@ -1257,7 +1262,8 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
             for (int f = 0; f < NS; ++f) bv[f] = TT::to_f32(bias[(low ? 0 : hc) + 8 * (NS * j + f) + p]);
         }
 #pragma unroll
-        for (int t = 0; t < FT; ++t)
+        for (int t = 0; t < FT; ++t) {
+            uint32_t o4[4];  // NS = 2
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + e;
@@ -1272,9 +1278,16 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
                     const int f = low ? q : NS / 2 + q;
                     const float gq = low ? mine[q] : other[NS / 2 + q], uq = low ? other[q] : mine[NS / 2 + q];
                     const uint16_t o = TT::from_f32(mul_f32_rn(act == 1 ? silu_f32(gq) : gelu_tanh_f32(gq), uq));
-                    if (row < M) y[(size_t)row * hc + 8 * (NS * j + f) + p] = o;
+                    if constexpr (NS == 2) o4[e] = o;
+                    if (row < M && !by4) y[(size_t)row * hc + 8 * (NS * j + f) + p] = o;
                 }
             }
+            if constexpr (NS == 2) {
+                const uint2 v = quad_turn16(o4[0] | (o4[1] << 16), o4[2] | (o4[3] << 16), lane);
+                const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + quad;
+                if (row < M && by4) *(uint2 *)(y + (size_t)row * hc + 8 * (NS * j + (low ? 0 : 1)) + p - quad) = v;
+            }
+        }
         return;
     }
     // row 16 mt + 4 kb + e, column 16 (NS j + f) + ni (of the copy)
@@ -1286,7 +1299,16 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
     }
     if (gridDim.y > 1) {
 #pragma unroll
-        for (int t = 0; t < FT; ++t)
+        for (int t = 0; t < FT; ++t) {
+            if constexpr (NS == 2) {  // (K slices are a choice of N % 4 == 0 only)
+                const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + quad;
+#pragma unroll
+                for (int f = 0; f < NS; ++f) {
+                    const float4_t v = quad_turn32(fin[t][f], lane);
+                    if (row < M && col[f] >= 0) *(float4_t *)(part + ((size_t)blockIdx.y * M + row) * N + col[f] - quad) = v;
+                }
+                continue;
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + e;
@@ -1295,12 +1317,29 @@ __global__ __launch_bounds__(512) void ggm_gemm_kernel(const uint16_t *__restric
                 for (int f = 0; f < NS; ++f)
                     if (col[f] >= 0) part[((size_t)blockIdx.y * M + row) * N + col[f]] = fin[t][f][e];
             }
+        }
         return;
     }
     float bv[NS] = {};
     if (bias) {
 #pragma unroll
         for (int f = 0; f < NS; ++f) bv[f] = col[f] >= 0 ? TT::to_f32(bias[col[f]]) : 0.f;
+    }
+    if constexpr (NS == 2) {
+        if (by4) {
+#pragma unroll
+            for (int t = 0; t < FT; ++t)
+#pragma unroll
+                for (int f = 0; f < NS; ++f) {
+                    uint32_t o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = TT::from_f32(fin[t][f][e] + bv[f]);
+                    const uint2 v = quad_turn16(o[0] | (o[1] << 16), o[2] | (o[3] << 16), lane);
+                    const int row = m0 + 16 * (KS == 1 ? t : FT * kq + t) + 4 * kb + quad;
+                    if (row < M && col[f] >= 0) *(uint2 *)(y + (size_t)row * N + col[f] - quad) = v;
+                }
+            return;
+        }
     }
 #pragma unroll
     for (int t = 0; t < FT; ++t)

@@ -88,3 +88,27 @@ def test_op_keeps_whole_sums():
     ref = oracle.matmul_nt_f32(round_x(xd.float().cpu().numpy(), oracle.BF16), w)
     for out in (y, z):
         assert_close(out, ref, "op and layer", bf16_out=True)
+
+
+# these forms store groups of four columns where rows of y begin on 8 bytes
+@pytest.mark.parametrize("form", [WIDE, PAIRS])
+@pytest.mark.parametrize("act", [None, ops.ACT_GATED_SILU])
+def test_outputs_off_the_8_byte_grid(form, act):
+    """Columns that are no multiple of four, an output that begins 2 bytes later: a value at a time, the same bits."""
+    fmt, N, K, m = synth.GGUF_Q4_K, 1152, 1024, 70
+    data = synth.gguf_weight(fmt, N, K, seed=11)
+    xd = to_dev(np.random.default_rng(12).standard_normal((m, K)).astype(np.float32), torch.bfloat16)
+    bias = to_dev(((np.arange(N, dtype=np.float32) % 7) - 3) * np.float32(0.5), torch.bfloat16)
+    tune("OXQ_GGUF_GEMM_KS", form)
+    y = ops.QLinear(fmt, to_dev(data), K, N, bias, torch.bfloat16, gate_up_act=act).forward(xd)
+    cols = y.shape[1]
+    room = torch.full((m * cols + 5,), 7.0, dtype=torch.bfloat16, device="cuda")
+    out = room[1:1 + m * cols].view(m, cols)
+    ops.QLinear(fmt, to_dev(data), K, N, bias, torch.bfloat16, gate_up_act=act).forward(xd, out=out)
+    assert "_gemm_bf16" in ops.default_context().last_plan()["kernel"]
+    np.testing.assert_array_equal(bits_of(out), bits_of(y))
+    assert room[0].item() == 7.0 and (room[1 + m * cols:] == 7.0).all()
+    if act is None:
+        less = data.reshape(N, -1)[:N - 6].reshape(-1)
+        z = ops.QLinear(fmt, to_dev(less.copy()), K, N - 6, bias[:N - 6].contiguous(), torch.bfloat16).forward(xd)
+        np.testing.assert_array_equal(bits_of(z), bits_of(y)[:, :N - 6])
