@@ -174,12 +174,15 @@ __device__ __forceinline__ void group_pairs_small(const int32_t *top_idx, const 
 }
 
 // ---------------------------------------------------------------------------
-// group.  Up to 64 pairs: one wave, one pair per lane (group_pairs_small).  Above: 16 waves, wave w
-// owns the pairs [w C, (w + 1) C) and takes them 64 at a time, ranking the lanes that share an expert
-// with ballots exactly as the small form does; its running count per expert lives in its own row of LDS,
-// and the rank inside (wave, expert) is parked in pair_pos.  A scan over (expert, wave) then gives every
-// wave its first position per expert, and a second pass over the pairs writes the lists.  Pair order
-// inside an expert is pair order, whatever the scheduling: every sum here is over integers.
+// group.  Up to 64 pairs: one wave, one pair per lane (group_pairs_small).  Above: a workgroup of 16 waves for every
+// 1024 pairs, a pair per lane.  A wave ranks its lanes with ballots exactly as the small form does and keeps its counts
+// in its own row of LDS; the workgroup counts the experts of all other pairs itself (before its own and after them),
+// and a scan over (expert, wave) gives every wave its first position per expert.  Pair order inside an expert is pair
+// order, whatever the scheduling: every sum here is over integers.
+// What bounds it: a chain of dependent steps (two trips to memory, three barriers), and in one workgroup for all pairs
+// the scattered stores, three a pair, and what it ranks batch by batch: 2060 / 4096 / 16384 / 32768 pairs took 5.7 / 7.8 /
+// 32.6 / 62 us in one workgroup, 4.6 / 4.7 / 6.5 / 8.3 in their own; up to 1024 pairs, one workgroup, 2.9 - 3.0 either way.
+// Every workgroup counting everything costs one LDS addition a lane and 1024 pairs.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void moe_group_kernel(const int32_t *__restrict__ top_idx,
                                                        const float *__restrict__ top_vals, int P, int E,
@@ -190,45 +193,59 @@ __global__ __launch_bounds__(64) void moe_group_kernel(const int32_t *__restrict
     group_pairs_small(top_idx, top_vals, P, E, top_k, group_lds, (int)threadIdx.x, offsets, tokens, weights, pair_pos);
 }
 
-constexpr int GROUP_WAVES = 16;
-__global__ __launch_bounds__(GROUP_WAVES * 64) void moe_group_waves_kernel(
+constexpr int GROUP_WAVES = 16, GROUP_PAIRS = GROUP_WAVES * 64;
+__global__ __launch_bounds__(GROUP_PAIRS) void moe_group_waves_kernel(
     const int32_t *__restrict__ top_idx, const float *__restrict__ top_vals, int P, int E,
     int32_t *__restrict__ offsets, int32_t *__restrict__ tokens, float *__restrict__ weights,
     int32_t *__restrict__ pair_pos, int top_k) {
-    extern __shared__ int32_t group_lds[];  // cnt[GROUP_WAVES][E], then start[E]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    extern __shared__ int32_t group_lds[];  // cnt[GROUP_WAVES][E], before[E], after[E]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int32_t *cnt = group_lds + (size_t)wave * E;
-    int32_t *start = group_lds + (size_t)GROUP_WAVES * E;
-    for (int e = lane; e < E; e += 64) cnt[e] = 0;  // the wave's own row: its LDS accesses stay in order
-    const int C = ((P + GROUP_WAVES * 64 - 1) / (GROUP_WAVES * 64)) * 64;  // pairs per wave, whole batches of 64
-    const int i0 = min(P, wave * C), i1 = min(P, i0 + C);
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const int id_bits = expert_id_bits(E);
-    for (int b = i0; b < i1; b += 64) {
-        const int i = b + lane;
-        const int e = i < i1 ? top_idx[i] : -1;
-        const bool ok = e >= 0 && e < E;  // ids outside [0, E) are dropped
-        const unsigned long long mine = lanes_with_my_expert(e, ok, id_bits);
-        const int r = __builtin_popcountll(mine & below);
-        const int before = ok ? cnt[e] : 0;  // every lane reads before the lowest lane of each expert adds
-        if (ok && r == 0) cnt[e] = before + __builtin_popcountll(mine);
-        const int rank = before + r;
-        if (ok) pair_pos[i] = rank;  // within (wave, expert); made absolute below
+    int32_t *before = group_lds + (size_t)GROUP_WAVES * E, *after = before + E;
+    const int own = (int)blockIdx.x, chunks = (P + GROUP_PAIRS - 1) / GROUP_PAIRS;
+    const int64_t i64 = (int64_t)own * GROUP_PAIRS + tid;
+    const bool mine_in = i64 < P;
+    const int i = (int)i64;
+    const int e = mine_in ? top_idx[i] : -1;
+    const float val = mine_in ? top_vals[i] : 0.0f;
+    for (int x = lane; x < E; x += 64) cnt[x] = 0;  // the wave's own row: its LDS accesses stay in order
+    const bool others = chunks > 1;  // launch-uniform; without others before[] is only written below
+    if (others) {
+        for (int x = tid; x < 2 * E; x += GROUP_PAIRS) before[x] = 0;
+        __syncthreads();
     }
-    __syncthreads();
-    // per expert: exclusive prefix over the waves, total in start[e]
-    for (int e = threadIdx.x; e < E; e += GROUP_WAVES * 64) {
-        int c[GROUP_WAVES], run = 0;
+    // the other chunks' experts, eight loads in flight
+    for (int q0 = 0; others && q0 < chunks; q0 += 8) {
+        int other[8];
 #pragma unroll
-        for (int w = 0; w < GROUP_WAVES; ++w) c[w] = group_lds[(size_t)w * E + e];  // independent reads first
+        for (int u = 0; u < 8; ++u) {
+            const int q = q0 + u;
+            const int64_t j = (int64_t)q * GROUP_PAIRS + tid;
+            other[u] = q != own && j < P ? top_idx[j] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (other[u] >= 0 && other[u] < E) atomicAdd((q0 + u < own ? before : after) + other[u], 1);
+    }
+    const bool ok = e >= 0 && e < E;  // ids outside [0, E) are dropped
+    const unsigned long long mine = lanes_with_my_expert(e, ok, expert_id_bits(E));
+    const int rank = __builtin_popcountll(mine & ((1ull << lane) - 1ull));
+    if (ok && rank == 0) cnt[e] = __builtin_popcountll(mine);
+    __syncthreads();
+    // per expert: exclusive prefix over the chunks before and the waves, total in before[e]
+    for (int x = tid; x < E; x += GROUP_PAIRS) {
+        int c[GROUP_WAVES], run = others ? before[x] : 0;
+#pragma unroll
+        for (int w = 0; w < GROUP_WAVES; ++w) c[w] = group_lds[(size_t)w * E + x];  // independent reads first
 #pragma unroll
         for (int w = 0; w < GROUP_WAVES; ++w) {
-            group_lds[(size_t)w * E + e] = run;
+            group_lds[(size_t)w * E + x] = run;
             run += c[w];
         }
-        start[e] = run;
+        before[x] = others ? run + after[x] : run;
     }
     __syncthreads();
+    int32_t *start = before;
     if (wave == 0) {  // exclusive scan of the totals in expert order, 64 experts per round
         int carry = 0;
         for (int e1 = 0; e1 < E; e1 += 64) {
@@ -242,23 +259,18 @@ __global__ __launch_bounds__(GROUP_WAVES * 64) void moe_group_waves_kernel(
             }
             if (ee < E) {
                 start[ee] = carry + incl - c;
-                offsets[ee] = carry + incl - c;
+                if (own == 0) offsets[ee] = carry + incl - c;
             }
             carry += __shfl(incl, 63, 64);
         }
-        if (lane == 0) offsets[E] = carry;
+        if (lane == 0 && own == 0) offsets[E] = carry;
     }
     __syncthreads();
-    for (int b = i0; b < i1; b += 64) {
-        const int i = b + lane;
-        if (i >= i1) continue;
-        const int e = top_idx[i];
-        if (e < 0 || e >= E) continue;
-        const int pos = start[e] + cnt[e] + pair_pos[i];
-        tokens[pos] = i / top_k;
-        weights[pos] = top_vals[i];
-        pair_pos[i] = pos;
-    }
+    if (!ok) return;
+    const int pos = start[e] + cnt[e] + rank;
+    tokens[pos] = i / top_k;
+    weights[pos] = val;
+    pair_pos[i] = pos;
 }
 
 // ---------------------------------------------------------------------------
@@ -469,14 +481,14 @@ int launch_moe_route(oxq_ctx *ctx, hipStream_t s, const void *logits, int dtype,
 int launch_moe_group(oxq_ctx *ctx, hipStream_t s, const int32_t *top_idx, const float *top_vals, int64_t P, int64_t E,
                      int64_t top_k, int32_t *offsets, int32_t *tokens, float *weights, int32_t *pair_pos) {
     const bool small = P <= 64;
-    dim3 grid(1), block(small ? 64 : GROUP_WAVES * 64);
+    dim3 grid(small ? 1u : (unsigned)ceil_div(P, GROUP_PAIRS)), block(small ? 64 : GROUP_PAIRS);
     set_plan(ctx, "moe_group", grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if (small) {
         hipLaunchKernelGGL(moe_group_kernel, grid, block, 2 * (size_t)E * sizeof(int32_t), s, top_idx, top_vals, (int)P,
                            (int)E, offsets, tokens, weights, pair_pos, (int)top_k);
     } else {
-        const size_t lds = ((size_t)GROUP_WAVES + 1) * (size_t)E * sizeof(int32_t);  // at most 17 KB (256 experts)
+        const size_t lds = ((size_t)GROUP_WAVES + 2) * (size_t)E * sizeof(int32_t);  // at most 18 KB (256 experts)
         hipLaunchKernelGGL(moe_group_waves_kernel, grid, block, lds, s, top_idx, top_vals, (int)P, (int)E, offsets,
                            tokens, weights, pair_pos, (int)top_k);
     }

@@ -465,6 +465,22 @@ def test_moe_group_matches_oracle(T, E, k):
     np.testing.assert_array_equal(rw[pos.ravel()], rvals.ravel())
 
 
+@pytest.mark.parametrize("T,E,k", [(13, 7, 5), (256, 7, 4), (205, 64, 5), (2049, 1, 1), (2300, 130, 8)])
+def test_moe_group_drops_ids_outside_the_experts(T, E, k):
+    """Pairs of an id outside [0, E) reach no list, in the chunk of 1024 pairs that holds them as in the others, and keep
+    their pair_pos; all remaining pairs of one expert stay in order."""
+    say(f"moe group T={T} E={E} k={k} with ids out of range")
+    ids = np.random.default_rng(T).choice([-1, E // 2, E - 1, E, 1 << 20], size=(T, k), p=[.1, .6, .2, .05, .05]).astype(np.int32)
+    vals = np.arange(T * k, dtype=np.float32).reshape(T, k)
+    off, tok, w, pos = (t.cpu().numpy() for t in ops.moe_group(to_dev(ids), to_dev(vals), E))
+    flat = ids.ravel()
+    want = np.concatenate([np.flatnonzero(flat == e) for e in range(E)])
+    np.testing.assert_array_equal(off, np.concatenate([[0], np.cumsum([np.sum(flat == e) for e in range(E)])]))
+    np.testing.assert_array_equal(tok[:len(want)], want // k)
+    np.testing.assert_array_equal(w[:len(want)], vals.ravel()[want])
+    np.testing.assert_array_equal(pos.ravel()[want], np.arange(len(want)))
+
+
 @pytest.mark.parametrize("T,E,k,norm", [(8, 32, 4, True), (1, 32, 4, True), (16, 64, 4, False), (5, 200, 3, True),
                                          (64, 16, 1, True), (13, 256, 5, True), (17, 32, 4, True), (300, 8, 2, False)])
 def test_moe_route_group_equals_the_two_calls(T, E, k, norm):
