@@ -201,6 +201,25 @@ constexpr double PK4_MID_ROUND = 0.31;
 // 16-column strips: the same for a whole round, 0.27 for a last round on at most half of the CUs (4096 x 4096,
 // 4096 x 6144, 8192 x 8192, 14336 x 4096 over 65..2048 rows in both types: 18.7 - 24.4 us a round at K = 4096)
 constexpr double PK4N_MID_ROUND = 0.31, PK4N_MID_PART = 0.27;
+// pk4_mid128_kernel, 128 rows and two strips, one workgroup a CU: a round (f16: a last round on at most 0.7 of the CUs) in the
+// same units.  bf16 takes 31 - 33 us a round at K = 4096 where one of 64 rows takes 22 - 25, f16 28 - 32 against 19 - 20.  Us, best
+// of the other forms -> this: bf16 4096 x 28672 at 65 / 128 / 256 rows 45 / 45 / 75 -> 33 / 34 / 66, 4096 x 14336 at 256 / 512 rows
+// 42 / 72 -> 33 / 65, 3584 x 18944 at 128 / 384 rows 38 / 65 -> 29 / 61; f16 4096 x 28672 at 128 rows 38 -> 32, 4096 x 11008 at 256
+// 37 -> 29.  At 4096 x 28672 and 512 rows 128-row workgroups of eight strips are ahead (bf16 107 against 132).
+// Two rounds and more count 7 % more in bf16 (against three rounds of 64 rows 9344 x 18048 at 236 rows takes 132 against 128, 5120 x
+// 8576 at 487 77 against 75).  Against the forms of eight strips, which add no partial tiles, a short K tells: 1024 x 12544 at 583 rows
+// bf16 28.2 against 25.2, 1152 x 6272 at 994 rows f16 30.9 against 23.0.
+// 16-column strips: a round, and a last one on at most 0.8 of the CUs.  bf16 at K = 4096 takes 31 - 32 and 36 us, f16 30 - 31 and 36; us,
+// best of the other forms -> this: bf16 4096 x 4096 at 768 / 1024 rows 43 / 43 -> 32 / 36, 4096 x 6144 at 384 / 512 42 / 42 -> 32 /
+// 32, 14336 x 4096 at 768 / 1024 124 / 132 -> 94 / 109, 8192 x 8192 at 384 / 512 75 / 78 -> 56 / 65; f16 4096 x 4096 at 768 rows
+// 38 -> 31; 4096 x 6144 at 1024 rows, one and a half rounds, bf16 64 / 65.  Three rounds are behind 128-row workgroups of eight strips
+// (8320 x 6336 at 1913 rows bf16 203 / 187, 5632 x 7552 at 1488 f16 135 / 122).
+struct Pk4Mid128Cost {
+    double full, part, part_upto, more_from, more;  // times `more` beyond `more_from` rounds
+};
+constexpr Pk4Mid128Cost PK4_MID128_BF16 = {0.455, 0.455, 0.7, 1.0, 1.07}, PK4_MID128_F16 = {0.505, 0.45, 0.7, 1.0, 1.04};
+constexpr Pk4Mid128Cost PK4N_MID128_BF16 = {0.52, 0.465, 0.8, 2.0, 1.1}, PK4N_MID128_F16 = {0.57, 0.50, 0.8, 2.0, 1.1};
+constexpr double PK4_MID128_LONG_K = 0.92, PK4_MID128_OVER_K = 314.0;
 
 struct Pk4GemmCost {
     bool pairs64;
@@ -208,7 +227,7 @@ struct Pk4GemmCost {
 };
 // rows of a workgroup (0: the split-K tiles) and the K split inside it (4: pk4_mid_kernel, two strips a workgroup)
 struct Pk4GemmForm {
-    int rows, ks;
+    int rows, ks;  // (128 rows and 4: pk4_mid128_kernel)
     bool light = false;  // 128 rows, and those behind the whole tiles in tiles of 32
 };
 // pk4_mid_kernel at up to 64 rows of 64-column strips, against the one-strip workgroups of pk4_mfma_kernel and
@@ -244,7 +263,8 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     if (p.w.bits == 8 && p.w.strip == 16) return {0, 1};  // (16-column strips are a 4-bit layout)
     const int forced = tune(ctx, OXQ_TUNE_PK4_GEMM_ROWS, 0), forced_ks = tune(ctx, OXQ_TUNE_PK4_GEMM_KS, 0);
     if (p.w.unrounded) return {forced || pk4_fold_prefill(cus, p) ? 64 : 0, 1};
-    if (forced_ks == 4) return {64, 4};
+    const bool can_mid128 = p.w.bits == 4 && pk4_sets(p.w.group_shift) == 1;
+    if (forced_ks == 4) return {forced == 128 && can_mid128 ? 128 : 64, 4};
     const int64_t rest = p.M % 128;
     const bool can_light = p.M > 128 && rest >= 1 && rest <= 32 && p.w.strip != 16 && pk4_sets(p.w.group_shift) == 1;
     if (forced == 32 && can_light) return {128, 1, true};
@@ -291,6 +311,15 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
                          : p.w.strip == 16 ? rounds(w_mid, PK4N_MID_ROUND, PK4N_MID_PART, 0.5)
                                            : std::ceil(w_mid) * PK4_MID_ROUND;
     // (the split-K tiles address the whole of x with 32 bits)
+    const double w_mid128 = (double)(ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)2) * ceil_div(p.M, (int64_t)128)) / cus;
+    const Pk4Mid128Cost &h = p.w.strip == 16 ? (f16 ? PK4N_MID128_F16 : PK4N_MID128_BF16) : (f16 ? PK4_MID128_F16 : PK4_MID128_BF16);
+    const double c_mid128 = !can_mid128 || forced_ks == 1
+                                ? 1e30
+                                : rounds(w_mid128, h.full, h.part, h.part_upto) * (w_mid128 > h.more_from ? h.more : 1.0);
+    const double c_mid128_k = c_mid128 * (PK4_MID128_LONG_K + PK4_MID128_OVER_K / (double)p.w.K);
+    // (against split-K tiles in whole rounds: 3584 x 18944 at 128 rows, 2.3 of them, takes 38 us in bf16, by 2.3 / 8 it would be 28)
+    if (c_mid128_k < c64 && c_mid128_k < c128 && c_mid128_k < c_light && c_mid128 < c_mid &&
+        c_mid128 < std::max(c_split, c.split_lo * std::ceil(tiles) / 8.0)) return {128, 4};
     if (c_split <= c64 && c_split <= c128 && c_split <= c_light && c_split <= c_mid && (uint64_t)p.M * (uint64_t)p.w.K * 2 < (1ull << 31)) return {0, 1};
     if (c_mid < c64 && c_mid < c128 && c_mid < c_light) return {64, 4};
     // (in f16 the 64-row workgroups are ahead at equal estimates: 2048 x 22016 at 1040 rows 98 us against 102)
@@ -328,8 +357,8 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw,
-             form.ks > 1 ? "k4" : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
+    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", form.ks > 1 ? 64 : rows, spw,
+             form.ks > 1 ? (rows == 128 ? "k4_r128" : "k4") : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
              p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
@@ -337,7 +366,7 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (((uintptr_t)p.x | (uintptr_t)p.y) & 15) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: x and y must be 16-byte aligned");
     if (p.bias && ((uintptr_t)p.bias & 7)) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: bias must be 8-byte aligned");
     if (p.w.unrounded) return launch_pk4_gemm_fold(s, grid, p, (int)NG, (int)RT);
-    if (form.ks == 4) return launch_pk4_mid(s, grid, p, (int)NG);
+    if (form.ks == 4) return rows == 128 ? launch_pk4_mid128(s, grid, p, (int)NG) : launch_pk4_mid(s, grid, p, (int)NG);
     if (pk4_sets(p.w.group_shift) > 1) return launch_pk4_gemm_fine(s, grid, p, rows, (int)NG, (int)RT);
     const bool f16 = p.w.dtype == OXQ_F16;
     if (form.light) return f16 ? pk4_gemm_go_light<F16Traits>(s, grid, p, (int)NG, (int)RT) : pk4_gemm_go_light<BF16Traits>(s, grid, p, (int)NG, (int)RT);

@@ -27,6 +27,68 @@ namespace oxq {
 
 constexpr int PK4M_MT = 4, PK4M_KS = 4, PK4M_GROUPS = 2, PK4M_STAGES = 4;
 
+// Stores four rows of a lane's four columns: row row0 + e, fin[e][f] of column group j (64 columns).
+template <typename TT, bool NARROW>
+__device__ __forceinline__ void pk4m_store(const float4_t (&fin)[4], const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
+                                           int M, int N, int j, int ni, int row0, int act) {
+    // columns of fin[e][f]: NARROW 64 j + 16 f + ni, else 64 j + 4 ni + f
+    float bv[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (NARROW) {
+        if (bias) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) bv[f] = TT::to_f32(bias[64 * j + 16 * f + ni]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (row0 + e >= M) continue;
+#pragma unroll
+            for (int f = 0; f < 4; ++f) y[(size_t)(row0 + e) * N + 64 * j + 16 * f + ni] = TT::from_f32(fin[e][f] + bv[f]);
+        }
+        return;
+    }
+    if (act) {
+        // Fused gate|up layer, as in pk4_gemm_kernel: lane ni < 8 holds four gate columns, lane ni + 8 of the same row of
+        // 16 their up columns; they exchange their values and finish two outputs each.  y is [M, N / 2].
+        const int half_n = N >> 1, col = 32 * j + 4 * (ni & 7);
+        const bool low = ni < 8;
+        if (bias) {
+            const uint2 bw = *(const uint2 *)(bias + (low ? 0 : half_n) + col);
+            bv[0] = TT::to_f32((uint16_t)(bw.x & 0xFFFFu)), bv[1] = TT::to_f32((uint16_t)(bw.x >> 16));
+            bv[2] = TT::to_f32((uint16_t)(bw.y & 0xFFFFu)), bv[3] = TT::to_f32((uint16_t)(bw.y >> 16));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float mine[4], other[4];
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                mine[f] = TT::to_f32(TT::from_f32(fin[e][f] + bv[f]));
+                other[f] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mine[f]), 0x128, 0xF, 0xF, false));
+            }
+            uint32_t o[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const float gq = low ? mine[q] : other[2 + q], uq = low ? other[q] : mine[2 + q];
+                o[q] = TT::from_f32(mul_f32_rn(act == 1 ? silu_f32(gq) : gelu_tanh_f32(gq), uq));
+            }
+            if (row0 + e < M) *(uint32_t *)(y + (size_t)(row0 + e) * half_n + col + (low ? 0 : 2)) = o[0] | (o[1] << 16);
+        }
+        return;
+    }
+    if (64 * j + 4 * ni >= N) return;
+    if (bias) {
+        const uint2 bw = *(const uint2 *)(bias + 64 * j + 4 * ni);
+        bv[0] = TT::to_f32((uint16_t)(bw.x & 0xFFFFu)), bv[1] = TT::to_f32((uint16_t)(bw.x >> 16));
+        bv[2] = TT::to_f32((uint16_t)(bw.y & 0xFFFFu)), bv[3] = TT::to_f32((uint16_t)(bw.y >> 16));
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (row0 + e >= M) continue;
+        const uint32_t o0 = TT::from_f32(fin[e][0] + bv[0]), o1 = TT::from_f32(fin[e][1] + bv[1]);
+        const uint32_t o2 = TT::from_f32(fin[e][2] + bv[2]), o3 = TT::from_f32(fin[e][3] + bv[3]);
+        *(uint2 *)(y + (size_t)(row0 + e) * N + 64 * j + 4 * ni) = uint2{o0 | (o1 << 16), o2 | (o3 << 16)};
+    }
+}
+
 // NARROW: the layer is stored in strips of 16 columns; a wave's 64 columns are four neighbouring strips and a strip's
 // block is one 16-byte load a lane whose words are the block's four steps.  SETS: as in pk4_mfma_kernel.
 template <typename TT, int BITS, int SETS, bool NARROW>
@@ -316,63 +378,7 @@ __global__ __launch_bounds__(512) void pk4_mid_kernel(const uint16_t *__restrict
         for (int k = 0; k < KS; ++k)  // K order: the same sum whatever the timing
             fin[e] += red[(((k * SPW + ws_) * MT + kq) * 4 + e) * 64 + lane];
     }
-    const int row0 = m0 + 16 * kq + 4 * kb;
-    // columns of fin[e][f]: NARROW 64 j + 16 f + ni, else 64 j + 4 ni + f
-    float bv[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (NARROW) {
-        if (bias) {
-#pragma unroll
-            for (int f = 0; f < 4; ++f) bv[f] = TT::to_f32(bias[64 * j + 16 * f + ni]);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (row0 + e >= M) continue;
-#pragma unroll
-            for (int f = 0; f < 4; ++f) y[(size_t)(row0 + e) * N + 64 * j + 16 * f + ni] = TT::from_f32(fin[e][f] + bv[f]);
-        }
-        return;
-    }
-    if (act) {
-        // Fused gate|up layer, as in pk4_gemm_kernel: lane ni < 8 holds four gate columns, lane ni + 8 of the same row of
-        // 16 their up columns; they exchange their values and finish two outputs each.  y is [M, N / 2].
-        const int half_n = N >> 1, col = 32 * j + 4 * (ni & 7);
-        const bool low = ni < 8;
-        if (bias) {
-            const uint2 bw = *(const uint2 *)(bias + (low ? 0 : half_n) + col);
-            bv[0] = TT::to_f32((uint16_t)(bw.x & 0xFFFFu)), bv[1] = TT::to_f32((uint16_t)(bw.x >> 16));
-            bv[2] = TT::to_f32((uint16_t)(bw.y & 0xFFFFu)), bv[3] = TT::to_f32((uint16_t)(bw.y >> 16));
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float mine[4], other[4];
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                mine[f] = TT::to_f32(TT::from_f32(fin[e][f] + bv[f]));
-                other[f] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mine[f]), 0x128, 0xF, 0xF, false));
-            }
-            uint32_t o[2];
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const float gq = low ? mine[q] : other[2 + q], uq = low ? other[q] : mine[2 + q];
-                o[q] = TT::from_f32(mul_f32_rn(act == 1 ? silu_f32(gq) : gelu_tanh_f32(gq), uq));
-            }
-            if (row0 + e < M) *(uint32_t *)(y + (size_t)(row0 + e) * half_n + col + (low ? 0 : 2)) = o[0] | (o[1] << 16);
-        }
-        return;
-    }
-    if (64 * j + 4 * ni >= N) return;
-    if (bias) {
-        const uint2 bw = *(const uint2 *)(bias + 64 * j + 4 * ni);
-        bv[0] = TT::to_f32((uint16_t)(bw.x & 0xFFFFu)), bv[1] = TT::to_f32((uint16_t)(bw.x >> 16));
-        bv[2] = TT::to_f32((uint16_t)(bw.y & 0xFFFFu)), bv[3] = TT::to_f32((uint16_t)(bw.y >> 16));
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if (row0 + e >= M) continue;
-        const uint32_t o0 = TT::from_f32(fin[e][0] + bv[0]), o1 = TT::from_f32(fin[e][1] + bv[1]);
-        const uint32_t o2 = TT::from_f32(fin[e][2] + bv[2]), o3 = TT::from_f32(fin[e][3] + bv[3]);
-        *(uint2 *)(y + (size_t)(row0 + e) * N + 64 * j + 4 * ni) = uint2{o0 | (o1 << 16), o2 | (o3 << 16)};
-    }
+    pk4m_store<TT, NARROW>(fin, bias, y, M, N, j, ni, m0 + 16 * kq + 4 * kb, act);
 }
 
 }  // namespace oxq
