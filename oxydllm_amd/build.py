@@ -19,7 +19,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "liboxq_hip.so")
 OBJ_DIR = os.path.join(HERE, "csrc", "build")
 
-SOURCES = ["oxq_api.cpp", "wna16_gemv.hip", "wna16_mfma.hip", "wna16_slab.hip", "wna16_dequant.hip", "awq_transforms.hip", "pk4.hip", "pk4_tile.hip", "pk4_gemm.hip", "pk4_mid.hip", "pk4_mid128.hip", "pk4_fine.hip", "pk4_fold.hip", "gptq_tile.hip",
+SOURCES = ["oxq_api.cpp", "wna16_gemv.hip", "wna16_mfma.hip", "wna16_slab.hip", "wna16_dequant.hip", "awq_transforms.hip", "pk4.hip", "pk4_tile.hip", "pk4_gemm.hip", "pk4_mid.hip", "pk4_mid128.hip", "pk4_midfold.hip", "pk4_fine.hip", "pk4_fold.hip", "gptq_tile.hip",
            "gguf_gemv.hip", "gguf_res.hip", "gguf_mfma.hip", "blockq_mm.hip", "mxfp4_gemv.hip", "mxfp4_gemm.hip", "moe_glue.hip", "f8_block.hip", "f8_mm.hip", "calib.hip",
            "checkpoint_files.cpp"]
 

@@ -248,6 +248,8 @@ int launch_pk4_gemm_fold(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, 
 int launch_pk4_mid(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);
 // 128 rows (pk4_mid128.hip; 4-bit layers with groups of 128 rows and more)
 int launch_pk4_mid128(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);
+// 64 rows, weights not rounded (pk4_midfold.hip)
+int launch_pk4_midfold(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);
 // 49 - 64 rows on a 4-bit layer in 64-column strips (pk4_tile.hip)
 bool pk4_tile64_takes(const Pk4Problem &p, int ks);
 int launch_pk4_tile64(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p);

@@ -246,14 +246,27 @@ static bool pk4_mid_decode(double cus, const Pk4Problem &p) {
 // last): GPTQ 4-bit groups of 64 4096 x 11008 at 256 / 512 / 2048 rows 67.9 / 86.3, 128.6 / 88.7, 493 / 265; groups of 32
 // 4096 x 4096 at 1024 / 2048 rows 100 / 116, 195 / 124; AWQ 8-bit groups of 64 11008 x 4096 at 512 / 1024 rows 131 / 235,
 // 267 / 235 (bf16).
-static bool pk4_fold_prefill(double cus, const Pk4Problem &p) {
+// Between them pk4_midfold_kernel, whole rounds too: a round costs as much as `mid` rounds of tiles (both counted in whole rounds),
+// one of the prefill form then `wide` (the tiles of 8-bit layers are faster in full rounds than the fit above has them).  Us at
+// K = 4096, best of the other two -> this: GPTQ 4-bit groups of 64 N = 4096 at 512 / 1024 rows f16 43 / 85 -> 27 / 50, bf16 44 / 83 -> 29 /
+// 54, N = 11008 at 128 / 256 / 512 f16 33 / 65 / 87 -> 26 / 48 / 74; groups of 32 N = 4096 at 512 rows f16 55 -> 32; 8-bit groups of 64
+// N = 4096 at 512 rows f16 51 -> 29, N = 11008 at 256 bf16 91 -> 63; at 256 rows of N = 4096, two rounds of tiles, f16 21 / 25.  Against the
+// prefill form, which adds no partial tiles, a short K tells (GPTQ 4-bit groups of 128 2048 x 7352 at 515 rows f16 35 / 38).  60 layers of
+// 1024 - 10240 x 600 - 24000, 180 calls at 33 - 2200 rows: 63 came here, 1.31 times as fast.
+static Pk4GemmForm pk4_fold_form(double cus, const Pk4Problem &p, bool mid) {
     static const double unit4[3] = {6.3, 8.0, 9.0}, unit8[3] = {4.8, 5.7, 6.9};  // groups of 128 rows and more, 64, 32
-    const int sets = pk4_sets(p.w.group_shift), i = sets == 1 ? 0 : sets == 2 ? 1 : 2;
+    static const double mid4[2][3] = {{2.08, 2.33, 2.2}, {2.35, 2.55, 2.7}}, wide4[3] = {6.3, 8.0, 8.5};  // f16, bf16
+    static const double mid8[2][3] = {{2.1, 2.13, 2.1}, {2.35, 2.34, 2.35}}, wide8[3] = {5.4, 6.5, 7.3};
+    const int sets = pk4_sets(p.w.group_shift), i = sets == 1 ? 0 : sets == 2 ? 1 : 2, b = p.w.dtype == OXQ_F16 ? 0 : 1;
     // the row tiles address the whole of x with 32 bits and are one grid dimension
-    if ((uint64_t)p.M * (uint64_t)p.w.K * 2 >= (1ull << 31) || ceil_div(p.M, (int64_t)32) > 65535) return true;
-    const int64_t strips = ceil_div(p.w.N, (int64_t)64);
-    const double rounds = std::ceil((double)(ceil_div(strips, (int64_t)PK4G_STRIPS) * ceil_div(p.M, (int64_t)64)) / cus);
-    return rounds * (p.w.bits == 4 ? unit4[i] : unit8[i]) < (double)(strips * ceil_div(p.M, (int64_t)32)) / cus;
+    if ((uint64_t)p.M * (uint64_t)p.w.K * 2 >= (1ull << 31) || ceil_div(p.M, (int64_t)32) > 65535) return {64, 1};
+    const int64_t strips = ceil_div(p.w.N, (int64_t)64), row_tiles = ceil_div(p.M, (int64_t)64);
+    const double rounds = std::ceil((double)(ceil_div(strips, (int64_t)PK4G_STRIPS) * row_tiles) / cus);
+    const double tiles = (double)(strips * ceil_div(p.M, (int64_t)32)) / cus;
+    const double c_mid = std::ceil((double)(ceil_div(strips, (int64_t)2) * row_tiles) / cus) * (p.w.bits == 4 ? mid4 : mid8)[b][i];
+    const double short_k = 0.88 + 500.0 / (double)p.w.K;
+    if (mid && c_mid < std::ceil(tiles) && c_mid * short_k < rounds * (p.w.bits == 4 ? wide4 : wide8)[i]) return {64, 4};
+    return {rounds * (p.w.bits == 4 ? unit4 : unit8)[i] < tiles ? 64 : 0, 1};
 }
 static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     const double cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
@@ -262,7 +275,10 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     if ((uintptr_t)p.bias & 7) return {0, 1};  // (fused gate|up layers only: oxq_api.cpp, prepack_layer)
     if (p.w.bits == 8 && p.w.strip == 16) return {0, 1};  // (16-column strips are a 4-bit layout)
     const int forced = tune(ctx, OXQ_TUNE_PK4_GEMM_ROWS, 0), forced_ks = tune(ctx, OXQ_TUNE_PK4_GEMM_KS, 0);
-    if (p.w.unrounded) return {forced || pk4_fold_prefill(cus, p) ? 64 : 0, 1};
+    if (p.w.unrounded) {
+        if (forced_ks == 4) return {64, 4};
+        return forced ? Pk4GemmForm{64, 1} : pk4_fold_form(cus, p, forced_ks != 1);
+    }
     const bool can_mid128 = p.w.bits == 4 && pk4_sets(p.w.group_shift) == 1;
     if (forced_ks == 4) return {forced == 128 && can_mid128 ? 128 : 64, 4};
     const int64_t rest = p.M % 128;
@@ -365,7 +381,7 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if ((uint64_t)rows * (uint64_t)p.w.K * 2 >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: K too large");
     if (((uintptr_t)p.x | (uintptr_t)p.y) & 15) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: x and y must be 16-byte aligned");
     if (p.bias && ((uintptr_t)p.bias & 7)) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: bias must be 8-byte aligned");
-    if (p.w.unrounded) return launch_pk4_gemm_fold(s, grid, p, (int)NG, (int)RT);
+    if (p.w.unrounded) return form.ks == 4 ? launch_pk4_midfold(s, grid, p, (int)NG) : launch_pk4_gemm_fold(s, grid, p, (int)NG, (int)RT);
     if (form.ks == 4) return rows == 128 ? launch_pk4_mid128(s, grid, p, (int)NG) : launch_pk4_mid(s, grid, p, (int)NG);
     if (pk4_sets(p.w.group_shift) > 1) return launch_pk4_gemm_fine(s, grid, p, rows, (int)NG, (int)RT);
     const bool f16 = p.w.dtype == OXQ_F16;

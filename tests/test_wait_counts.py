@@ -12,10 +12,10 @@ from oxydllm_amd import _lib
 from tests import gpu_code
 
 # Two buffers, the other one filled meanwhile: nothing under way at any barrier.  pk4_mid_kernel: four stages, of which
-# the two after the published one are filled meanwhile, four loads a wave each; pk4_mid128_kernel: five, the published one the next
-# but one, and the same two.
+# the two after the published one are filled meanwhile, four loads a wave each; pk4_mid128_kernel and
+# pk4_midfold_kernel: five, the published one the next but one, and the same two.
 ALLOWED = {"pk4_gemm_kernel": 0, "pk4n_gemm_kernel": 0, "ggm_gemm_kernel": 0, "f8_gemm_kernel": 0, "mxfp4_gemm_kernel": 0,
-           "pk4_mid_kernel": 8, "pk4_mid128_kernel": 8}
+           "pk4_mid_kernel": 8, "pk4_mid128_kernel": 8, "pk4_midfold_kernel": 8}
 
 
 @pytest.fixture(scope="module")
