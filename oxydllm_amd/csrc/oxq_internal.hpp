@@ -246,7 +246,7 @@ int launch_pk4_gemm_fine(hipStream_t s, dim3 grid, const Pk4Problem &p, int rows
 int launch_pk4_gemm_fold(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG, int RT);  // unrounded layers (pk4_fold.hip)
 // 64 rows x two groups of 64 columns a workgroup, K split inside it (pk4_mid.hip)
 int launch_pk4_mid(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);
-// 128 rows (pk4_mid128.hip; 4-bit layers with groups of 128 rows and more)
+// 128 rows (pk4_mid128.hip; 4-bit layers)
 int launch_pk4_mid128(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);
 // 64 rows, weights not rounded (pk4_midfold.hip)
 int launch_pk4_midfold(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG);

@@ -209,6 +209,8 @@ constexpr double PK4N_MID_ROUND = 0.31, PK4N_MID_PART = 0.27;
 // Two rounds and more count 7 % more in bf16 (against three rounds of 64 rows 9344 x 18048 at 236 rows takes 132 against 128, 5120 x
 // 8576 at 487 77 against 75).  Against the forms of eight strips, which add no partial tiles, a short K tells: 1024 x 12544 at 583 rows
 // bf16 28.2 against 25.2, 1152 x 6272 at 994 rows f16 30.9 against 23.0.
+// Groups of 64 and 32 go by the same figures (115 layers, 345 calls at 65 - 2200 rows: 65 came here, 1.27 times as fast, the
+// least 1.05; 4096 x 15488, groups of 64, bf16 at 448 rows 80 -> 72, 8960 x 14720, groups of 32, at 243 100 -> 78).
 // 16-column strips: a round, and a last one on at most 0.8 of the CUs.  bf16 at K = 4096 takes 31 - 32 and 36 us, f16 30 - 31 and 36; us,
 // best of the other forms -> this: bf16 4096 x 4096 at 768 / 1024 rows 43 / 43 -> 32 / 36, 4096 x 6144 at 384 / 512 42 / 42 -> 32 /
 // 32, 14336 x 4096 at 768 / 1024 124 / 132 -> 94 / 109, 8192 x 8192 at 384 / 512 75 / 78 -> 56 / 65; f16 4096 x 4096 at 768 rows
@@ -279,7 +281,7 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
         if (forced_ks == 4) return {64, 4};
         return forced ? Pk4GemmForm{64, 1} : pk4_fold_form(cus, p, forced_ks != 1);
     }
-    const bool can_mid128 = p.w.bits == 4 && pk4_sets(p.w.group_shift) == 1;
+    const bool can_mid128 = p.w.bits == 4;
     if (forced_ks == 4) return {forced == 128 && can_mid128 ? 128 : 64, 4};
     const int64_t rest = p.M % 128;
     const bool can_light = p.M > 128 && rest >= 1 && rest <= 32 && p.w.strip != 16 && pk4_sets(p.w.group_shift) == 1;

@@ -1,4 +1,4 @@
-// pk4_mid128_kernel: 128 rows x two groups of 64 columns a workgroup, for 4-bit layers with groups of 128 rows and more where
+// pk4_mid128_kernel: 128 rows x two groups of 64 columns a workgroup, for 4-bit layers of rounded weights where
 // pk4_mid_kernel (pk4_mid.hpp: the four waves of a column group take every fourth block of K) would run two row tiles.
 //
 // What bounds pk4_mid_kernel is the issue port, and more than half of what it issues turns codes into weights that serve
@@ -19,17 +19,20 @@ namespace oxq {
 constexpr int PK4H_STAGES = 5;
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
-template <typename TT, bool NARROW>
+template <typename TT, int SETS, bool NARROW>
 __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ pw,
                                                          const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                          int M, int K, int N, int NG, int act) {
     typedef MfmaOps<TT> Ops;
     constexpr int MT = PK4M_MT, KS = PK4M_KS, SPW = PK4M_GROUPS, ROWS = 16 * MT, NS = PK4H_STAGES;
-    constexpr int BB = NARROW ? PK4N_BW * 4 : pk4_block_words(4, 1) * 4;
+    constexpr int BB = NARROW ? PK4N_BW * 4 : pk4_block_words(4, SETS) * 4;
     constexpr int TILE = ROWS * 128, STAGE = KS * TILE;  // bytes of x: a wave's unit (64 rows of half a block), a stage
     constexpr bool BF = TT::DTYPE == BF16Traits::DTYPE;
     constexpr bool PAIRED = BF && !NARROW;
-    constexpr int RE = NARROW ? 5 : 3, RO = NARROW ? 4 : 2;  // ring loads in the first and the second half of a block
+    static_assert(!NARROW || SETS == 1, "16-column strips hold groups of 128 rows and more");
+    constexpr int OOB = 0x7FFFFF00;
+    // ring loads in the first and the second half of a block
+    constexpr int RE = NARROW ? 5 : SETS == 4 ? 4 : 3, RO = NARROW ? 4 : SETS == 4 ? 4 : SETS == 2 ? 3 : 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
 
     const int lane = threadIdx.x & 63;
@@ -40,7 +43,7 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
     const int j = g * SPW + ws_;
     const bool live = j < ((N + 63) >> 6);  // wave-uniform: the last workgroup of a layer may have one column group
     const int m0 = rt * 2 * ROWS;
-    const int NB = K >> 7, NR = (NB + KS - 1) / KS;  // blocks; rounds of KS blocks
+    const int NB = SETS > 1 ? (K + 127) >> 7 : K >> 7, NR = (NB + KS - 1) / KS;  // blocks; rounds of KS blocks
 
     const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);
     const __amdgpu_buffer_rsrc_t rs_wl =
@@ -66,22 +69,32 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
         const int r = 8 * (ws_ * MT + q) + (lane >> 3);
         xo[q] = r * K * 2 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
     }
+    // the lanes whose piece of 8 elements lies in the upper half of a half block: of even loads, odd ones the others
+    const bool upper = (lane >> 2) & 1;
     auto dma = [&](int i, int hf, int rh, int slot, int q) {  // load q of a unit of block i
-        const __amdgpu_buffer_rsrc_t rs = i < NB ? (rh ? rs_x1 : rs_x0) : rs_none;
+        // K may end inside the last block, at groups of 32 inside the half: zeros for the pieces past it, not the next row
+        const int left = K - i * 128 - hf * 64;
+        const __amdgpu_buffer_rsrc_t rs = (SETS > 1 ? left > 0 : i < NB) ? (rh ? rs_x1 : rs_x0) : rs_none;
         int rows16 = 32 * K;
         asm volatile("" : "+s"(rows16));
-        pk4g_load_lds16(rs, pk4_lds + slot * STAGE + kq * TILE + ws_ * (MT * 1024) + q * 1024, q < 2 ? xo[q] : xo[q & 1] + rows16,
-                        i * 256 + hf * 128);
+        int off = q < 2 ? xo[q] : xo[q & 1] + rows16;
+        if constexpr (SETS == 4) {
+            // f16: from the first load's offset, one register less - eight rows on, and the piece's half the other one
+            if (q && !BF) off = xo[0] + ((q & 1) ? (upper ? rows16 / 2 - 64 : rows16 / 2 + 64) : 0) + (q >> 1) * rows16;
+            off = left < 64 && upper == !(q & 1) ? OOB : off;
+        }
+        pk4g_load_lds16(rs, pk4_lds + slot * STAGE + kq * TILE + ws_ * (MT * 1024) + q * 1024, off, i * 256 + hf * 128);
     };
-    // fragment of a half block's first step, row tile mt (+ 2048 mt): row ni; the second step's is the neighbouring piece
-    const int a_rd = kq * TILE + ni * 128 + (((pk4_x_chunk<1>(0, kb) & 7) ^ ((ni >> 1) & 7)) << 4);
+    // fragment of a half block's first step, row tile mt (+ 2048 mt): row ni; the second step's is a bit of the piece away
+    constexpr int STEP = SETS == 4 ? 64 : 16;
+    const int a_rd = kq * TILE + ni * 128 + (((pk4_x_chunk<SETS>(0, kb) & 7) ^ ((ni >> 1) & 7)) << 4);
     const NibbleMasks nm = nibble_masks();
 
     // a block of weights by step; 16-column strips: by half block (two of a lane's four words, so that a half's registers are
     // free before the next one's are used) and strip
     u32x4_t wring[NARROW ? 1 : 4];
     u32x2_t wnarrow[2][4];
-    uint32_t zring;
+    uint32_t zring[SETS];
     auto load_w = [&](int i, int st) {
         wring[st] = __builtin_amdgcn_raw_buffer_load_b128(i < NB ? rs_w : rs_none, lane_again() * 16, i * BB + st * 1024, 0);
     };
@@ -92,9 +105,9 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
         for (int f = 0; f < 4; ++f) wnarrow[hf][f] = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rs, at, (f * NB + i) * BB, 0));
     };
     // the pairs of a lane's four columns: lane group f brings those of column (strip) f, pk4_pair_words hands them round
-    auto load_z = [&](int i) {
+    auto load_z = [&](int i, int set) {
         const int l = lane_again(), at = NARROW ? (l >> 4) * (NB * BB) + 1024 + (l & 15) * 4 : 4096 + ((l & 15) * 4 + (l >> 4)) * 4;
-        zring = __builtin_amdgcn_raw_buffer_load_b32(i < NB ? rs_w : rs_none, at, i * BB, 0);
+        zring[set] = __builtin_amdgcn_raw_buffer_load_b32(i < NB ? rs_w : rs_none, at, i * BB + set * 256, 0);
     };
 
     // The compiler orders nothing against the loads into LDS: the waits for them count the younger loads, whose order
@@ -104,7 +117,8 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
 #pragma unroll
     for (int q = 0; q < MT; ++q) dma(kq, 0, 1, 1, q);
     __builtin_amdgcn_sched_barrier(0);
-    load_z(kq);
+#pragma unroll
+    for (int u = 0; u < SETS; ++u) load_z(kq, u);
     if constexpr (NARROW) {
         load_narrow(kq, 0), load_narrow(kq, 1);
     } else {
@@ -134,9 +148,9 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
     uint32_t negzb[4], sp[4];
     Pk4gBf16 cb[4];
     Pk4N<TT> cst[4];
-    auto constants = [&] {  // of the block that the ring holds
+    auto constants = [&](int set) {  // of a group that the ring holds
         uint32_t zv[4];
-        pk4_pair_words(zring, zv);
+        pk4_pair_words(zring[set], zv);
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
             if constexpr (BF) cb[f].set(__builtin_bit_cast(float, zv[f] & 0xFFFF0000u), __builtin_bit_cast(float, zv[f] << 16) + (NARROW ? 0.0f : 128.0f));
@@ -179,14 +193,14 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
     constexpr std::integral_constant<int, 1> P1{};
     u32x4_t a[2][MT];  // fragments of x: the two steps
     auto read_x = [&](int slot, int st) {
-        const unsigned char *from = pk4_lds + ((slot * STAGE + a_rd) ^ (st << 4));
+        const unsigned char *from = pk4_lds + ((slot * STAGE + a_rd) ^ (st ? STEP : 0));
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) a[st][mt] = *(const u32x4_t *)(from + mt * 2048);
     };
     // The first two units, counting as younger only the loads into LDS (the compiler may issue the ring loads behind this wait).
     meet(std::integral_constant<int, 2 * MT>{});
     read_x(0, 0);
-    constants();
+    constants(0);
     pair(0, P0), pair(0, P1);
     __builtin_amdgcn_sched_barrier(0);
 
@@ -224,12 +238,13 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
         };
         if constexpr (RH == 0) {
             if constexpr (!NARROW) load_w(i1, 2 * HF);  // the step that the unit before has left
-            if constexpr (HF == 0) load_z(i1);
+            if constexpr (HF == 0 || SETS > 1) load_z(i1, SETS == 4 ? 2 * HF : HF);  // its group
             dma(i1, HF, RH, free, 0), dma(i1, HF, RH, free, 1);
             read_x(slot, 1);
+            if constexpr (SETS == 4) constants(2 * HF + 1);
             pair(2 * HF + 1, P0);
             multiply(0), multiply(1), multiply(2);
-            order(OXQ_N(2 + MT + (NARROW ? 1 - HF : 2 - HF)), OXQ_N(12), OXQ_N(0), OXQ_N(0), OXQ_N(V));
+            order(OXQ_N(2 + MT + (NARROW ? 1 - HF : SETS > 1 ? 2 : 2 - HF)), OXQ_N(12), OXQ_N(0), OXQ_N(0), OXQ_N(V));
             dma(i1, HF, RH, free, 2);
             pair(2 * HF + 1, P1);
             multiply(3);
@@ -238,16 +253,17 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
             order(OXQ_N(1), OXQ_N(4), OXQ_N(4), OXQ_N(8), OXQ_N(V));
             if constexpr (NARROW) load_narrow(i1, HF);
             else load_w(i1, 2 * HF + 1);
+            if constexpr (SETS == 4) load_z(i1, 2 * HF + 1);
             dma(i1, HF, RH, free, 3);
             multiply(6), multiply(7);
-            order(OXQ_N(NARROW ? 5 : 2), OXQ_N(8), OXQ_N(0), OXQ_N(0), OXQ_N(0));
+            order(OXQ_N(NARROW ? 5 : SETS == 4 ? 3 : 2), OXQ_N(8), OXQ_N(0), OXQ_N(0), OXQ_N(0));
         } else {
             dma(i1, HF, RH, free, 0), dma(i1, HF, RH, free, 1);
             read_x(slot, 1);
             multiply(0), multiply(1);
             order(OXQ_N(2 + MT), OXQ_N(8), OXQ_N(0), OXQ_N(0), OXQ_N(0));
             dma(i1, HF, RH, free, 2);
-            if constexpr (HF == 1) constants();
+            if constexpr (HF == 1 || SETS > 1) constants(HF == 1 ? 0 : SETS / 2);
             pair(2 - 2 * HF, P0);
             multiply(2), multiply(3);
             read_x(next, 0);
@@ -298,21 +314,28 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
     }
 }
 
-template <typename TT, bool NARROW>
+template <typename TT, int SETS, bool NARROW>
 static int mid128_go(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG) {
     static LdsGrant grant;  // one per instantiation
     const size_t lds = (size_t)PK4H_STAGES * PK4M_KS * 16 * PK4M_MT * 128;
-    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_mid128_kernel<TT, NARROW>, lds));
-    hipLaunchKernelGGL((pk4_mid128_kernel<TT, NARROW>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw,
+    OXQ_HIP_CHECK(grant.ensure((const void *)pk4_mid128_kernel<TT, SETS, NARROW>, lds));
+    hipLaunchKernelGGL((pk4_mid128_kernel<TT, SETS, NARROW>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w.pw,
                        (const uint16_t *)p.bias, (uint16_t *)p.y, (int)p.M, (int)p.w.K, (int)p.w.N, NG, p.act);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
+template <typename TT>
+static int mid128_layout(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG) {
+    if (p.w.strip == 16) return mid128_go<TT, 1, true>(s, grid, p, NG);
+    switch (pk4_sets(p.w.group_shift)) {
+    case 1: return mid128_go<TT, 1, false>(s, grid, p, NG);
+    case 2: return mid128_go<TT, 2, false>(s, grid, p, NG);
+    default: return mid128_go<TT, 4, false>(s, grid, p, NG);
+    }
+}
 
 int launch_pk4_mid128(hipStream_t s, dim3 grid, const Pk4Problem &p, int NG) {
-    const bool f16 = p.w.dtype == OXQ_F16;
-    if (p.w.strip == 16) return f16 ? mid128_go<F16Traits, true>(s, grid, p, NG) : mid128_go<BF16Traits, true>(s, grid, p, NG);
-    return f16 ? mid128_go<F16Traits, false>(s, grid, p, NG) : mid128_go<BF16Traits, false>(s, grid, p, NG);
+    return p.w.dtype == OXQ_F16 ? mid128_layout<F16Traits>(s, grid, p, NG) : mid128_layout<BF16Traits>(s, grid, p, NG);
 }
 
 }  // namespace oxq

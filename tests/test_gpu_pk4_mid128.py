@@ -40,3 +40,25 @@ def test_same_bits_as_rows_of_64(pack, dt, K, N, g, strip16):
             plan = layer.ctx.last_plan()
             assert "_r64x2k4_r128" + ("_n16" if strip16 else "") in plan["kernel"] and plan["grid"][0] == -(-m // 128) * -(-N // 128), plan
             np.testing.assert_array_equal(bits_of(got), bits_of(want))
+
+
+# K that ends in a block's first and second half and inside them
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,N,g", [(1216, 320, 64), (2176, 264, 64), (1184, 328, 32), (1376, 192, 32), (4256, 64, 32)])
+def test_groups_inside_a_block(dt, K, N, g):
+    q, z, s = synth.awq_checkpoint(K, N, g, 4, seed=K + N)
+    rng = np.random.default_rng(K * N)
+    bias = to_dev(rng.standard_normal(N).astype(np.float32), dt)
+    x = to_dev(rng.standard_normal((330, K)).astype(np.float32), dt)
+    x[3, K - 1], x[200, 0] = float("inf"), float("nan")
+    tune("OXQ_PK4_GEMM_KS", 4)
+    layer = ops.PackedQuantLinear(4, ops.PACK_OUT, to_dev(q), to_dev(z), to_dev(s, dt), bias, dt)
+    for m in (65, 128, 129, 330):
+        print(f"[case] pk4 128 rows x two strips awq {dt} {K}x{N} g={g} m={m}", flush=True)
+        tune("OXQ_PK4_GEMM_ROWS", 64)
+        want = layer.forward(x[:m])
+        tune("OXQ_PK4_GEMM_ROWS", 128)
+        got = layer.forward(x[:m])
+        plan = layer.ctx.last_plan()
+        assert plan["kernel"].endswith("_r64x2k4_r128"), plan
+        np.testing.assert_array_equal(bits_of(got), bits_of(want))
