@@ -199,7 +199,7 @@ bool pk4_tile64_takes(const Pk4Problem &p, int ks) {
 int launch_pk4_tile64(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     (void)ctx;
     const int NB = (int)(p.w.K / 128);
-    dim3 grid((unsigned)(p.w.N / 64));
+    dim3 grid((unsigned)ceil_div(p.w.N, (int64_t)64));  // the last strip may hold fewer columns
     const bool f16 = p.w.dtype == OXQ_F16;
     if (NB == 32) return f16 ? pk4_tile64_go<F16Traits, 4>(s, grid, p) : pk4_tile64_go<BF16Traits, 4>(s, grid, p);
     if (NB == 40) return f16 ? pk4_tile64_go<F16Traits, 5>(s, grid, p) : pk4_tile64_go<BF16Traits, 5>(s, grid, p);
