@@ -204,23 +204,23 @@ constexpr double PK4N_MID_ROUND = 0.31, PK4N_MID_PART = 0.27;
 // pk4_mid128_kernel, 128 rows and two strips, one workgroup a CU: a round (f16: a last round on at most 0.7 of the CUs) in the
 // same units.  bf16 takes 31 - 33 us a round at K = 4096 where one of 64 rows takes 22 - 25, f16 28 - 32 against 19 - 20.  Us, best
 // of the other forms -> this: bf16 4096 x 28672 at 65 / 128 / 256 rows 45 / 45 / 75 -> 33 / 34 / 66, 4096 x 14336 at 256 / 512 rows
-// 42 / 72 -> 33 / 65, 3584 x 18944 at 128 / 384 rows 38 / 65 -> 29 / 61; f16 4096 x 28672 at 128 rows 38 -> 32, 4096 x 11008 at 256
+// 42 / 72 -> 33 / 65 (the latter left to eight strips, below), 3584 x 18944 at 128 / 384 rows 38 / 65 -> 29 / 61; f16 4096 x 28672 at 128 rows 38 -> 32, 4096 x 11008 at 256
 // 37 -> 29.  At 4096 x 28672 and 512 rows 128-row workgroups of eight strips are ahead (bf16 107 against 132).
-// Two rounds and more count 7 % more in bf16 (against three rounds of 64 rows 9344 x 18048 at 236 rows takes 132 against 128, 5120 x
-// 8576 at 487 77 against 75).  Against the forms of eight strips, which add no partial tiles, a short K tells: 1024 x 12544 at 583 rows
+// Two rounds and more count 11 % more in bf16 (against three rounds of 64 rows 9344 x 18048 at 236 rows takes 132 against 128, 5120 x
+// 8576 at 487 77 against 75; level with a full round of eight strips, where 4096 x 14336 at 512 takes 65 against 72).  Against the forms of eight strips, which add no partial tiles, a short K tells: 1024 x 12544 at 583 rows
 // bf16 28.2 against 25.2, 1152 x 6272 at 994 rows f16 30.9 against 23.0.
 // Groups of 64 and 32 go by the same figures (115 layers, 345 calls at 65 - 2200 rows: 65 came here, 1.27 times as fast, the
 // least 1.05; 4096 x 15488, groups of 64, bf16 at 448 rows 80 -> 72, 8960 x 14720, groups of 32, at 243 100 -> 78).
 // 16-column strips: a round, and a last one on at most 0.8 of the CUs.  bf16 at K = 4096 takes 31 - 32 and 36 us, f16 30 - 31 and 36; us,
 // best of the other forms -> this: bf16 4096 x 4096 at 768 / 1024 rows 43 / 43 -> 32 / 36, 4096 x 6144 at 384 / 512 42 / 42 -> 32 /
 // 32, 14336 x 4096 at 768 / 1024 124 / 132 -> 94 / 109, 8192 x 8192 at 384 / 512 75 / 78 -> 56 / 65; f16 4096 x 4096 at 768 rows
-// 38 -> 31; 4096 x 6144 at 1024 rows, one and a half rounds, bf16 64 / 65.  Three rounds are behind 128-row workgroups of eight strips
-// (8320 x 6336 at 1913 rows bf16 203 / 187, 5632 x 7552 at 1488 f16 135 / 122).
+// 38 -> 31; 4096 x 6144 at 1024 rows, one and a half rounds, bf16 64 / 65.  Two rounds and more are behind the
+// forms of eight strips (5760 x 4480 at 1639 rows bf16 104 / 95, 8320 x 6336 at 1913 203 / 187, 5632 x 7552 at 1488 f16 135 / 122).
 struct Pk4Mid128Cost {
     double full, part, part_upto, more_from, more;  // times `more` beyond `more_from` rounds
 };
-constexpr Pk4Mid128Cost PK4_MID128_BF16 = {0.455, 0.455, 0.7, 1.0, 1.07}, PK4_MID128_F16 = {0.505, 0.45, 0.7, 1.0, 1.04};
-constexpr Pk4Mid128Cost PK4N_MID128_BF16 = {0.52, 0.465, 0.8, 2.0, 1.1}, PK4N_MID128_F16 = {0.57, 0.50, 0.8, 2.0, 1.1};
+constexpr Pk4Mid128Cost PK4_MID128_BF16 = {0.455, 0.455, 0.7, 1.0, 1.11}, PK4_MID128_F16 = {0.505, 0.45, 0.7, 1.0, 1.04};
+constexpr Pk4Mid128Cost PK4N_MID128_BF16 = {0.52, 0.465, 0.8, 1.0, 1.08}, PK4N_MID128_F16 = {0.57, 0.50, 0.8, 1.0, 1.04};
 constexpr double PK4_MID128_LONG_K = 0.92, PK4_MID128_OVER_K = 314.0;
 
 struct Pk4GemmCost {
@@ -371,12 +371,13 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const int rows = form.rows, spw = PK4G_STRIPS / form.ks;
     const int64_t NG = ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)spw), RT = form.light ? p.M / rows : ceil_div(p.M, (int64_t)rows);
     // eight strips a workgroup: in the order of pk4g_tile_of; two strips: row tile by row tile
-    const int64_t wgs = form.ks == 1 ? pk4g_workgroups(RT, NG) + (form.light ? NG : 0) : RT * NG;
+    // (the two-strip forms launch what 64 rows take; those of 128 rows leave the second half idle, last in the launch)
+    const int64_t wgs = form.ks == 1 ? pk4g_workgroups(RT, NG) + (form.light ? NG : 0) : ceil_div(p.M, (int64_t)64) * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", form.ks > 1 ? 64 : rows, spw,
-             form.ks > 1 ? (rows == 128 ? "k4_r128" : "k4") : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
+    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", form.ks > 1 ? 64 : rows, spw,
+             form.ks > 1 ? "k4" : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "", form.ks > 1 && rows == 128 ? "_r128" : "",
              p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
