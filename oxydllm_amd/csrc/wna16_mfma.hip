@@ -693,7 +693,7 @@ bool awq4_mfma_ok(const Wna16Problem &p) {
 }
 
 // The tile-major copy built in the ctx workspace, then the resident-layer kernels on it: two launches (the repack
-// is one pass over the weights: about 45 us at 5120 x 13824, 4-bit).  A caller that holds the layer should hold a
+// is one pass over the weights: 9 us at 4096 x 14336, 4-bit).  A caller that holds the layer should hold a
 // PackedQuantLinear, which repacks once.
 static bool transient_repack_fits(const oxq_ctx *ctx, const Wna16Problem &p) {
     if ((((uintptr_t)p.x | (uintptr_t)p.y) & 15) || ((uintptr_t)p.bias & 7)) return false;
@@ -720,15 +720,23 @@ static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Probl
 }
 
 int launch_wna16_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
-    // Prefill sizes: the resident layout's kernels (x shared in LDS by eight strips, or two with K split inside
-    // the workgroup) run at two to six times the rate of the kernels on the checkpoint layout - 4096 x 14336 at
-    // 2048 rows: 197 (f16) / 216 (bf16) us against 377 / 1313 - which pays for the repack (36 us on that layer) from
-    // a few hundred rows on in f16 (the checkpoint-layout kernel does 0.19 us a row there) and from under a
-    // hundred in bf16 (0.64 us a row): 2048 rows 377 -> 232 and 1313 -> 252 us with the repack included.
-    // The GPTQ kernel on the checkpoint layout holds 0.6 PFLOP/s in both types: the repack pays from 640 rows too
-    // (5120 x 13824 at 2048 rows: 430 / 478 -> 269 / 289 us).
+    // The resident layout's kernels run at two to six times the rate of the kernels on the checkpoint layout, which pays for the
+    // repack (9 us at 4096 x 14336, 4-bit) from few rows on: AWQ in bf16 behind the 16 rows of the slab kernel, in f16 from 33 rows,
+    // on layers of more than 2^24 weights 64, with few columns 128; the GPTQ tile kernel is ahead longer.  Us, checkpoint layout / repack and resident kernel:
+    // AWQ 4-bit bf16 4096 x 14336 at 20 / 64 / 640 rows 46 / 23, 56 / 27, 656 / 110, 4096 x 4096 at 32 28 / 16, 1536 x 2048 at 20 16 / 10;
+    // f16 4096 x 14336 at 32 / 64 / 640 20 / 24, 28 / 27, 189 / 103, 4096 x 4096 at 20 / 32 14 / 14, 21 / 14; GPTQ 4-bit f16 4096 x
+    // 14336 at 160 / 256 41 / 42, 54 / 44, 8192 x 3072 at 256 / 448 24 / 31, 45 / 40, 1536 x 2048 at 448 / 640 9 / 12, 16 / 14; 8-bit 4096 x
+    // 14336 at 256 / 448 64 / 73, 110 / 100; AWQ f16 11008 x 3584 at 90 / 200 29 / 34, 44 / 37.  Up to 16 rows in bf16: AWQ 4-bit 4096 x
+    // 14336 at 9 rows, tile / slab kernel, 43 / 13.
     const bool awq = awq4_mfma_ok(p), gptq = !awq && gptq_tile_ok(p) && tune(ctx, OXQ_TUNE_GPTQ_TILE, 1) != 2;
-    const int64_t repack_from = awq && p.dtype != OXQ_F16 ? 80 : 640;
+    if (awq && p.M <= 16 && wna16_slab_takes(ctx, p)) return launch_wna16_slab(ctx, s, p);
+    const int64_t size = p.K * p.N;
+    const bool f16 = p.dtype == OXQ_F16;
+    int64_t repack_from;
+    if (awq && f16) repack_from = size < (1 << 21) ? 640 : size <= (1 << 24) ? 33 : p.K >= 2 * p.N ? 128 : 64;
+    else if (awq) repack_from = size < (1 << 21) ? 80 : 17;
+    else if (p.bits == 4 && size >= (1 << 25)) repack_from = f16 ? 352 : 256;
+    else repack_from = size > (1 << 24) || (p.bits == 4 && size == (1 << 24)) ? 448 : 640;
     if (p.M >= repack_from && (awq || gptq) && transient_repack_fits(ctx, p)) return launch_transient_repack(ctx, s, p);
     if (awq4_mfma_ok(p) && !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0))
         return p.dtype == OXQ_F16 ? launch_awq4_mfma<F16Traits>(ctx, s, p)

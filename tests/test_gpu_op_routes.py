@@ -1,0 +1,52 @@
+"""The AWQ ops on checkpoint tensors where their kernel changes: one row of ragged columns, bf16 at 9 - 16 rows, and the rows from which the
+tile op builds the tile-major copy for its call."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from oxydllm_amd import ops, synth
+from tests.helpers import assert_close, resident_rounds_weights, round_x, to_dev
+
+pytestmark = pytest.mark.gpu
+DT = {"f16": (oracle.F16, torch.float16), "bf16": (oracle.BF16, torch.bfloat16)}
+
+
+def tensors(K, N, g, bits, dt, tdt):
+    q, z, s = synth.awq_checkpoint(K, N, g, bits, seed=K + N + bits)
+    s_r = oracle.round_through(s, dt)
+    w = oracle.dequantize_awq(q, z, s_r) if bits == 4 else oracle.dequantize_awq8(q, z, s_r)
+    return (to_dev(q), to_dev(z), to_dev(s, tdt)), w
+
+
+@pytest.mark.parametrize("dtn", ["f16", "bf16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("K,N,g", [(1024, 264, 128), (4096, 1096, 64), (2080, 520, 32), (1280, 8200, 128)])
+def test_one_row_of_ragged_columns(dtn, bits, K, N, g):
+    """Weights stay unrounded: outputs are the 64-bit product rounded once, but for those next to a boundary."""
+    dt, tdt = DT[dtn]
+    args, w = tensors(K, N, g, bits, dt, tdt)
+    x = np.random.default_rng(K).standard_normal((1, K)).astype(np.float32)
+    y = (ops.w4a16_matmul if bits == 4 else ops.w8a16_matmul)(to_dev(x, tdt), *args)
+    assert "_slab" in ops.default_context().last_plan()["kernel"]
+    ref = round_x(x, dt).astype(np.float64) @ w.astype(np.float64).T
+    assert (y.cpu() == torch.from_numpy(ref).to(tdt)).double().mean().item() > 0.97
+
+
+@pytest.mark.parametrize("dtn", ["f16", "bf16"])
+@pytest.mark.parametrize("K,N,g,rows", [(1024, 2048, 128, {"f16": 33, "bf16": 17}), (1088, 2056, 64, {"f16": 33, "bf16": 17}),
+                                        (4096, 4104, 128, {"f16": 64, "bf16": 17}), (8224, 2048, 32, {"f16": 128, "bf16": 17})])
+def test_rows_at_the_lines_of_the_rule(dtn, K, N, g, rows):
+    dt, tdt = DT[dtn]
+    args, w = tensors(K, N, g, 4, dt, tdt)
+    x = np.random.default_rng(K).standard_normal((140, K)).astype(np.float32)
+    xd, wr = to_dev(x, tdt), oracle.round_through(w, dt)
+    for m in (9, 16, 17, rows[dtn] - 1, rows[dtn], 140):
+        y = ops.mpp_quant_matmul(xd[:m], *args, 4, ops.PACK_OUT)
+        plan = ops.default_context().last_plan()
+        print(f"[case] awq op {dtn} {K}x{N} g={g} m={m} {plan['kernel']}", flush=True)
+        resident = m >= rows[dtn]
+        slab = "_slab" in plan["kernel"]
+        assert slab == (m <= 16 and dtn == "bf16") and plan["kernel"].startswith("pk4_") == resident, plan
+        unrounded = slab or resident and not resident_rounds_weights(m, dt, False)
+        assert_close(y, oracle.matmul_nt_f32(round_x(x[:m], dt), w if unrounded else wr), f"m{m} {plan['kernel']}")
