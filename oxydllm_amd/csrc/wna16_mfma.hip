@@ -721,8 +721,8 @@ static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Probl
 
 int launch_wna16_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     // The resident layout's kernels run at two to six times the rate of the kernels on the checkpoint layout, which pays for the
-    // repack (9 us at 4096 x 14336, 4-bit) from few rows on: AWQ in bf16 behind the 16 rows of the slab kernel, in f16 from 33 rows,
-    // on layers of more than 2^24 weights 64, with few columns 128; the GPTQ tile kernel is ahead longer.  Us, checkpoint layout / repack and resident kernel:
+    // repack (9 us at 4096 x 14336, 4-bit) from few rows on: AWQ in bf16 behind the 16 rows of the slab kernel, in f16 from 49 rows (up to 48 the
+    // resident kernels fold sums, which make NaN of an infinite x), on layers of more than 2^24 weights 64, with few columns 128; the GPTQ tile kernel is ahead longer.  Us, checkpoint layout / repack and resident kernel:
     // AWQ 4-bit bf16 4096 x 14336 at 20 / 64 / 640 rows 46 / 23, 56 / 27, 656 / 110, 4096 x 4096 at 32 28 / 16, 1536 x 2048 at 20 16 / 10;
     // f16 4096 x 14336 at 32 / 64 / 640 20 / 24, 28 / 27, 189 / 103, 4096 x 4096 at 20 / 32 14 / 14, 21 / 14; GPTQ 4-bit f16 4096 x
     // 14336 at 160 / 256 41 / 42, 54 / 44, 8192 x 3072 at 256 / 448 24 / 31, 45 / 40, 1536 x 2048 at 448 / 640 9 / 12, 16 / 14; 8-bit 4096 x
@@ -733,7 +733,7 @@ int launch_wna16_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     const int64_t size = p.K * p.N;
     const bool f16 = p.dtype == OXQ_F16;
     int64_t repack_from;
-    if (awq && f16) repack_from = size < (1 << 21) ? 640 : size <= (1 << 24) ? 33 : p.K >= 2 * p.N ? 128 : 64;
+    if (awq && f16) repack_from = size < (1 << 21) ? 640 : size <= (1 << 24) ? 49 : p.K >= 2 * p.N ? 128 : 64;
     else if (awq) repack_from = size < (1 << 21) ? 80 : 17;
     else if (p.bits == 4 && size >= (1 << 25)) repack_from = f16 ? 352 : 256;
     else repack_from = size > (1 << 24) || (p.bits == 4 && size == (1 << 24)) ? 448 : 640;

@@ -371,7 +371,7 @@ static int slab_by_shape(hipStream_t s, dim3 grid, const Wna16Problem &p, float 
     // bf16 AWQ tensors that the dot-product kernel takes, as there: NaN for infinite x (the second path's registers cost 4 rows of
     // 4096 x 14336 12.7 -> 13.3 us).  Others (their address counts too) keep the signs that the generic kernel gives.
     if constexpr (TT::DTYPE != F16Traits::DTYPE && !GPTQ) {
-        if (awq_fast_ok(p))
+        if (awq_fast_ok(p) && (p.M <= 8 || p.bits == 8))  // (more rows of 4 bits: the tile kernel's, which keeps the signs)
             return p.bits == 8 ? slab_go<TT, 8, GPTQ, 2, 1, false>(s, grid, p, ws, blocks)
                    : run == 64 ? slab_go<TT, 4, GPTQ, 2, 1, false>(s, grid, p, ws, blocks)
                                : slab_go<TT, 4, GPTQ, 4, 1, false>(s, grid, p, ws, blocks);

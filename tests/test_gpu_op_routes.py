@@ -34,7 +34,7 @@ def test_one_row_of_ragged_columns(dtn, bits, K, N, g):
 
 
 @pytest.mark.parametrize("dtn", ["f16", "bf16"])
-@pytest.mark.parametrize("K,N,g,rows", [(1024, 2048, 128, {"f16": 33, "bf16": 17}), (1088, 2056, 64, {"f16": 33, "bf16": 17}),
+@pytest.mark.parametrize("K,N,g,rows", [(1024, 2048, 128, {"f16": 49, "bf16": 17}), (1088, 2056, 64, {"f16": 49, "bf16": 17}),
                                         (4096, 4104, 128, {"f16": 64, "bf16": 17}), (8224, 2048, 32, {"f16": 128, "bf16": 17})])
 def test_rows_at_the_lines_of_the_rule(dtn, K, N, g, rows):
     dt, tdt = DT[dtn]
@@ -50,3 +50,21 @@ def test_rows_at_the_lines_of_the_rule(dtn, K, N, g, rows):
         assert slab == (m <= 16 and dtn == "bf16") and plan["kernel"].startswith("pk4_") == resident, plan
         unrounded = slab or resident and not resident_rounds_weights(m, dt, False)
         assert_close(y, oracle.matmul_nt_f32(round_x(x[:m], dt), w if unrounded else wr), f"m{m} {plan['kernel']}")
+
+
+@pytest.mark.parametrize("dtn", ["f16", "bf16"])
+@pytest.mark.parametrize("K,N", [(2048, 1032), (1024, 2048)])
+def test_an_infinite_row_keeps_its_signs(dtn, K, N):
+    """One infinite value of x: infinity times a weight, or NaN where the weight is zero, whichever kernel takes the rows."""
+    dt, tdt = DT[dtn]
+    args, w = tensors(K, N, 128, 4, dt, tdt)
+    col = np.argmin((w == 0).sum(axis=0))
+    with np.errstate(invalid="ignore"):
+        want = np.where(w[:, col] == 0, np.nan, np.sign(w[:, col]) * np.inf).astype(np.float32)
+    for m in (9, 16, 17, 48, 49):
+        x = np.random.default_rng(m).standard_normal((m, K)).astype(np.float32)
+        x[m - 1, col] = np.inf
+        y = ops.mpp_quant_matmul(to_dev(x, tdt), *args, 4, ops.PACK_OUT)
+        print(f"[case] infinite row {dtn} {K}x{N} m={m} {ops.default_context().last_plan()['kernel']}", flush=True)
+        np.testing.assert_array_equal(y[m - 1].float().cpu().numpy(), want)
+        assert bool(torch.isfinite(y[:m - 1]).all())
