@@ -67,7 +67,8 @@ namespace oxq {
 // load-time repack
 // ---------------------------------------------------------------------------
 
-constexpr int pk4_repack_parts(int bits) { return bits + 1; }  // 256 words of weights each, and the pairs
+// 256 words of weights each, and a set of pairs each
+constexpr int pk4_repack_parts(int bits, int sets) { return bits + sets; }
 
 template <bool GPTQ, int BITS>
 __device__ __forceinline__ uint32_t src_q(const uint32_t *__restrict__ qw, int k, int col, int N) {
@@ -84,7 +85,9 @@ __device__ __forceinline__ uint32_t src_q(const uint32_t *__restrict__ qw, int k
 // strip's columns are 32 (8-bit: 64) bytes of an AWQ row, and what shares a line of the checkpoint reads it at one time in
 // one place.  What bounds it: the issue of indices and of a nibble's shifts; a thread's four words share the former and their loads.
 // The op that builds a copy for its call, a word a thread strip after strip -> this, us, bf16: AWQ 4-bit 4096 x 8192 at 100 rows 42.8 ->
-// 26.4, 8-bit at 24 40.9 -> 29.7, GPTQ 4-bit 4096 x 8200 at 24 28.2 -> 19.5, 8-bit 38.8 -> 28.7.
+// 26.4, 8-bit at 24 40.9 -> 29.7, GPTQ 4-bit 4096 x 8200 at 24 28.2 -> 19.5, 8-bit 38.8 -> 28.7.  Each set of pairs has a workgroup:
+// four in a row were the last to end on a small layer, groups of 32 (AWQ 2048 x 704 at 971 rows, 8-bit 26.0, now
+// 24.6; 4-bit 16.4, now 14.8; a word a thread 24.9 and 15.5); 4096 x 8192 at 100, GPTQ 4-bit 42.9 -> 35.3, AWQ 8-bit 61 -> 48.
 template <typename TT, bool GPTQ, int BITS, int SETS>
 __global__ __launch_bounds__(256) void pk4_prepack_kernel(const uint32_t *__restrict__ qw,
                                                           const uint32_t *__restrict__ qz,
@@ -93,8 +96,10 @@ __global__ __launch_bounds__(256) void pk4_prepack_kernel(const uint32_t *__rest
                                                           int half) {
     constexpr int PF = 32 / BITS, WL = BITS / 4, BW = pk4_block_words(BITS, SETS);
     const unsigned NB = (unsigned)(K + 127) >> 7, strips = (unsigned)(N + 63) >> 6, quads = (strips + 3) >> 2;
-    const int sh = (int)(blockIdx.x % pk4_repack_parts(BITS)), l = (int)(threadIdx.x & 63);
-    const unsigned at = blockIdx.x / pk4_repack_parts(BITS);
+    constexpr unsigned PARTS = pk4_repack_parts(BITS, SETS);
+    const unsigned at = blockIdx.x / PARTS;
+    // turned by one from block to block: with eight parts the pairs would all fall to the same four XCDs
+    const int sh = (int)((blockIdx.x + at) % PARTS), l = (int)(threadIdx.x & 63);
     const int b = (int)(at / quads), j = (int)(at % quads * 4 + (threadIdx.x >> 6));
     if (j >= (int)strips) return;
     uint32_t *const block = pw + ((size_t)j * NB + b) * BW;
@@ -136,20 +141,17 @@ __global__ __launch_bounds__(256) void pk4_prepack_kernel(const uint32_t *__rest
         return;
     }
     const int ni = l >> 2, f = l & 3, col = pk4_src_col(64 * j + 4 * ni + f, half);
-#pragma unroll
-    for (int set = 0; set < SETS; ++set) {
-        const int row = (b << 7) + set * (128 / SETS), g = row >> gshift;
-        uint32_t word = 0;
-        if (row < K && col < N) {
-            const int c = col % PF;
-            const int slot = (GPTQ || BITS == 8) ? c : ((c >> 1) | ((c & 1) << 2));
-            const uint32_t z = ((qz[(size_t)g * (N / PF) + col / PF] >> (BITS * slot)) & ((1u << BITS) - 1u)) + (GPTQ ? 1u : 0u);
-            const float bf = BITS == 4 ? TT::bias(f) : TT::BYTE_BIAS;
-            const uint32_t nz = TT::from_f32(-((float)z + bf));
-            word = nz | ((uint32_t)sc[(size_t)g * N + col] << 16);
-        }
-        block[1024 * WL + 64 * set + l] = word;
+    const int set = sh - 4 * WL, row = (b << 7) + set * (128 / SETS), g = row >> gshift;
+    uint32_t word = 0;
+    if (row < K && col < N) {
+        const int c = col % PF;
+        const int slot = (GPTQ || BITS == 8) ? c : ((c >> 1) | ((c & 1) << 2));
+        const uint32_t z = ((qz[(size_t)g * (N / PF) + col / PF] >> (BITS * slot)) & ((1u << BITS) - 1u)) + (GPTQ ? 1u : 0u);
+        const float bf = BITS == 4 ? TT::bias(f) : TT::BYTE_BIAS;
+        const uint32_t nz = TT::from_f32(-((float)z + bf));
+        word = nz | ((uint32_t)sc[(size_t)g * N + col] << 16);
     }
+    block[1024 * WL + 64 * set + l] = word;
 }
 
 // ---------------------------------------------------------------------------
@@ -761,7 +763,7 @@ int launch_pk4_prepack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &src, con
     const int sets = pk4_sets(src.group_shift);
     const size_t words = pk4_weight_bytes(K, N, src.bits, sets) / 4;
     const bool gptq = src.pack_dim == OXQ_PACK_IN;
-    const int64_t wide = ceil_div(src.N, (int64_t)256) * ceil_div(src.K, (int64_t)128) * pk4_repack_parts(src.bits);
+    const int64_t wide = ceil_div(src.N, (int64_t)256) * ceil_div(src.K, (int64_t)128) * pk4_repack_parts(src.bits, sets);
     if (dst.strip != 16 && wide > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repack: %lld x %lld exceeds the grid", (long long)src.K, (long long)src.N);
     dim3 grid((unsigned)(dst.strip == 16 ? ceil_div((int64_t)words, 256) : wide)), block(256);
     char name[64];
