@@ -478,11 +478,11 @@ int oxq_qlinear_new(oxq_ctx *ctx, int quant, const oxq_tensor *weight_bytes, int
  * by concatenating their bytes) with gated_silu_fused / gated_gelu_tanh_fused (ffn_kernels.metal:19-160) run in the
  * matmul's epilogue: out_features = 2I, forward writes [.., I] = act(gate(x)) * up(x), bit for bit what
  * oxq_gated_activation gives on the plain layer's output.  Needs a BF16 layer that takes the matrix-core copy (see
- * oxq_qlinear_is_resident below), else OXQ_ERR_UNSUPPORTED.  Every row count runs in one launch: up to 32 rows
- * the integer kernel of the copy; above that, where enough workgroups of 64 rows fill the chip, the copy's prefill
- * kernel (the plain layer takes the same kernel at the same sizes: the same bits); otherwise row tiles of 32 that
- * each read the weights again (with the unrounded weights that the plain layer's tile matmul rounds to bf16) -
- * oxq_mlp_forward sends those row counts (more than OXQ_GGUF_FUSED_ACT_ROWS where the prefill kernel does not take
+ * oxq_qlinear_is_resident below), else OXQ_ERR_UNSUPPORTED.  Up to 32 rows run in the integer kernel of the copy;
+ * above that, where enough workgroups fill the chip, in the copy's prefill kernel (the plain layer takes the same
+ * kernel in the same form at the same sizes: the same bits), in one launch, or in two where K is split over
+ * workgroups of 128 rows and the second adds the partial sums; otherwise in row tiles of 32 that each read the
+ * weights again (with the unrounded weights that the plain layer's tile matmul rounds to bf16) - oxq_mlp_forward sends those row counts (more than OXQ_GGUF_FUSED_ACT_ROWS where the prefill kernel does not take
  * the call) through the plain layer's path and the activation by itself, so that a FeedForward over this layer
  * gives the plain layers' bits at every row count. */
 #define OXQ_GGUF_FUSED_ACT_ROWS 32

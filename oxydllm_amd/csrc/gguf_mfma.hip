@@ -1660,9 +1660,8 @@ static GgmCost ggm_cost(int quant) {
     default: return {1.6, 3.3, 3.0, 1.85, 2.04};  // Q5_0, Q5_1, Q5_K
     }
 }
-// sliced: whether the caller can take K slices, whose partial sums a second launch adds from the workspace.  One that cannot (a fused
-// activation, a copy that lies there itself) chooses among whole sums of 128 rows; slices of 64 rows still win over them, and it
-// then takes another kernel.
+// sliced: whether the caller can take K slices, whose partial sums a second launch adds from the workspace.  One that cannot (a copy
+// that lies there itself) chooses among whole sums of 128 rows; slices of 64 rows still win over them, and it then takes another kernel.
 static GgmGemmForm gguf_gemm_form(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype, bool sliced) {
     const int64_t v = tune(ctx, OXQ_TUNE_GGUF_GEMM_MIN_M, -1);
     const bool narrow = ggm_narrow_format(quant);
@@ -1739,9 +1738,55 @@ bool gguf_gemm_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_
     const GgmGemmForm f = gguf_gemm_form(ctx, quant, M, K, N, act_dtype, sliced);
     return f.ks > 0 && (sliced || f.slices == 1);
 }
+// A fused gate|up layer: the plain layer's form, which keeps its bits - but for slices of 64 rows, whose calls stay in the integer
+// kernel's row tiles (few rows, weights not rounded).  The launch that adds slices of 128 rows runs the activation.
+bool gguf_gemm_takes_act(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
+    const GgmGemmForm f = gguf_gemm_form(ctx, quant, M, K, N, act_dtype, true);
+    return N % 64 == 0 && f.ks > 0 && (f.slices == 1 || f.rows == 128);
+}
 // rows beyond gguf_mfma_takes that the integer kernel takes in row tiles
 bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
     return gguf_gemm_form(ctx, quant, M, K, N, act_dtype, true).ks < 0;
+}
+
+// Adds the K slices of a fused gate|up layer and runs its activation: columns n and hc + n of a row (file order), summed and rounded
+// as splitk_reduce_kernel does it, then act(gate) * up as oxq_gated_activation.  What bounds it: the partials' bytes, as there.  A
+// thread has four outputs.  The fused call, us, whole sums in one launch (which are not the plain layer's bits) -> slices and this: Q4_K
+// 8192 x 4096 at 300 / 512 rows 49.1 / 49.6 -> 42.1 / 46.4, 6144 x 10752 at 74 38.4 -> 29.1, Q6_K 8192 x 4096 at 400 59.9 -> 50.2.  hc is a multiple of 32, and the 8 S M hc bytes of partials fit the workspace: the index fits 32 bits.
+__global__ __launch_bounds__(256) void ggm_act_reduce_kernel(const float *__restrict__ part, const uint16_t *__restrict__ bias,
+                                                             uint16_t *__restrict__ y, unsigned quads, int hc, size_t total, int S, int act) {
+    typedef BF16Traits TT;
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= quads) return;
+    const unsigned row = i / (unsigned)(hc >> 2), n = (i - row * (unsigned)(hc >> 2)) * 4;
+    const float *from = part + (size_t)row * 2 * hc + n;
+    float4_t g = {0.f, 0.f, 0.f, 0.f}, u = g;
+    for (int s0 = 0; s0 < S; s0 += 4) {
+        float4_t vg[4], vu[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float *at = from + (size_t)(s0 + k) * total;
+            vg[k] = s0 + k < S ? *(const float4_t *)at : float4_t{0.f, 0.f, 0.f, 0.f};
+            vu[k] = s0 + k < S ? *(const float4_t *)(at + hc) : float4_t{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) g += vg[k], u += vu[k];  // slice order
+    }
+    uint32_t o[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        float a = g[c], b = u[c];
+        if (bias) a += TT::to_f32(bias[n + c]), b += TT::to_f32(bias[hc + n + c]);
+        a = TT::to_f32(TT::from_f32(a)), b = TT::to_f32(TT::from_f32(b));
+        o[c] = TT::from_f32(mul_f32_rn(act == 1 ? silu_f32(a) : gelu_tanh_f32(a), b));
+    }
+    uint16_t *to = y + (size_t)row * hc + n;
+    if (((uintptr_t)y & 7) == 0) {
+        *(uint2 *)to = uint2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) to[c] = (uint16_t)o[c];
+    }
 }
 
 template <int FMT, int MT, int KS, int NS = 4>
@@ -1769,11 +1814,13 @@ static int ggm_gemm_go_form(hipStream_t s, dim3 grid, const GgufProblem &p, floa
 
 // p.w is the matrix-core copy; p.act as for launch_gguf_mfma; p.gate_half: the copy of a fused gate|up layer whose
 // activation this call leaves out
-int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, bool sliced) {
-    sliced = sliced && !p.act;
+int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &problem, bool sliced) {
+    GgufProblem p = problem;
     GgmGemmForm form = gguf_gemm_form(ctx, p.quant, p.M, p.K, p.N, p.act_dtype, sliced);
     if (form.ks <= 0) form = {1, 1};  // a caller that asks for this kernel gets it
     if (!sliced) form.slices = 1;
+    const int act_after = form.slices > 1 ? p.act : 0;  // (gguf_gemm_takes_act)
+    if (act_after) p.act = 0, p.gate_half = p.N / 2;
     const int ks = form.ks, spw = 8 / ks, rows = form.rows;
     const int64_t NG = ceil_div(ceil_div(p.N, (int64_t)(rows == 128 ? 32 : 64)), (int64_t)spw), RT = ceil_div(p.M, (int64_t)rows);
     const int64_t wgs = ks == 1 ? pk4g_workgroups(RT, NG) : RT * NG;
@@ -1785,7 +1832,7 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, bool sli
     char name[64], slices[16] = "";
     if (form.slices > 1) snprintf(slices, sizeof slices, "_s%d", form.slices);
     snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r64x%s%s%s%s", ggm_name(p.quant), ks > 1 ? "2k4" : "8", slices, rows == 128 ? "_r128" : "",
-             p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
+             problem.act == 1 ? "_silu" : problem.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), form.slices, 1, form.slices > 1 ? (size_t)form.slices * p.M * p.N * 4 : 0);
     if (ctx->plan_only) {
         if (form.slices > 1) add_launch(ctx);
@@ -1813,7 +1860,13 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, bool sli
     }
 #undef OXQ_GGM
     if (rc != OXQ_OK || form.slices == 1) return rc;
-    return launch_splitk_reduce(ctx, s, part, p.bias, p.y, p.M, p.N, form.slices, OXQ_BF16);
+    if (!act_after) return launch_splitk_reduce(ctx, s, part, p.bias, p.y, p.M, p.N, form.slices, OXQ_BF16);
+    add_launch(ctx);
+    const unsigned quads = (unsigned)(p.M * (p.N / 8));
+    hipLaunchKernelGGL(ggm_act_reduce_kernel, dim3((unsigned)ceil_div((int64_t)quads, (int64_t)256)), dim3(256), 0, s, part, (const uint16_t *)p.bias,
+                       (uint16_t *)p.y, quads, (int)(p.N / 2), (size_t)p.M * p.N, form.slices, act_after);
+    OXQ_HIP_CHECK(hipGetLastError());
+    return OXQ_OK;
 }
 
 }  // namespace oxq

@@ -2409,8 +2409,7 @@ int oxq_qlinear_forward(oxq_qlinear *l, void *stream, const oxq_tensor *x, const
         p.bias = l->has_bias ? l->bias.data : nullptr;
         p.w = (const uint8_t *)l->mm;
         p.act = l->act;
-        if (gguf_gemm_takes(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype, false) && p.N % 64 == 0)
-            return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p, false);
+        if (gguf_gemm_takes_act(l->ctx, l->quant, p.M, p.K, p.N, p.act_dtype)) return launch_gguf_gemm(l->ctx, (hipStream_t)stream, p);
         return launch_gguf_mfma(l->ctx, (hipStream_t)stream, p);
     }
     OXQ_TRY(check_gguf(l->ctx, decode ? "GgufQuantMatmul" : "GgufQuantMulMM", decode, false, &x2,
@@ -2449,13 +2448,11 @@ static int qlinear_forward_unfused(oxq_qlinear *l, void *stream, const oxq_tenso
     return qlinear_forward_file_layout(l, stream, p);
 }
 
-// whether `rows` rows of a bf16 layer run whole sums on its matrix-core copy, in the prefill kernel or in row tiles of the
-// integer kernel (a fused gate|up layer then keeps its activation in that kernel's epilogue; the plain layer takes
-// the same kernel, the same bits, or K slices of it)
+// whether `rows` rows of a fused gate|up layer run on its matrix-core copy with the activation, in the prefill kernel or in row tiles
+// of the integer kernel, where the plain layer takes the same kernel in the same form: the same bits
 static bool qlinear_prefill_on_copy(const oxq_qlinear *l, int64_t rows) {
     if (l->resident && l->mfma && gguf_mfma_tiles(l->ctx, l->quant, rows, l->in_features, l->out_features, l->out_dtype)) return true;
-    return l->resident && l->mfma && l->out_features % 64 == 0 &&
-           gguf_gemm_takes(l->ctx, l->quant, rows, l->in_features, l->out_features, l->out_dtype, false);
+    return l->resident && l->mfma && gguf_gemm_takes_act(l->ctx, l->quant, rows, l->in_features, l->out_features, l->out_dtype);
 }
 
 int oxq_qlinear_is_resident(const oxq_qlinear *l, int *resident) {

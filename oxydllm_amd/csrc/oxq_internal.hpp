@@ -285,6 +285,7 @@ int launch_gguf_mfma_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void 
 int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);  // p.w = the copy
 // the prefill kernel on the same copy (csrc/gguf_mfma.hip: ggm_gemm_kernel)
 bool gguf_gemm_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype, bool sliced = true);
+bool gguf_gemm_takes_act(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);  // a fused gate|up layer
 int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, bool sliced = true);  // p.w = the copy; sliced: as it was asked for
 bool gguf_mm_eligible(const oxq_ctx *ctx, const GgufProblem &p);
 int launch_gguf_mm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);

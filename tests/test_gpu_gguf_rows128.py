@@ -71,6 +71,33 @@ def test_slices():
     assert plan["kernel"].endswith("_r128") and plan["split_k"] > 1 and plan["launches"] == 2, plan
 
 
+@pytest.mark.parametrize("fmt,K,I,m,act,biased", [(synth.GGUF_Q4_K, 8192, 2048, 300, ops.ACT_GATED_SILU, True), (synth.GGUF_Q4_K, 8192, 1024, 777, ops.ACT_GATED_GELU_TANH, False),
+                                                  (synth.GGUF_Q8_0, 8192, 1056, 333, ops.ACT_GATED_SILU, True), (synth.GGUF_Q4_K, 6144, 5376, 74, ops.ACT_GATED_SILU, False)])
+def test_fused_activation_where_the_plain_layer_takes_slices(fmt, K, I, m, act, biased):
+    """No form forced: fused layer and FeedForward give the plain layer's bits and the activation's."""
+    wd = to_dev(synth.gguf_weight(fmt, 2 * I, K, seed=I + fmt))
+    bias = to_dev(((np.arange(2 * I, dtype=np.float32) % 9) - 4) * np.float32(0.5), torch.bfloat16) if biased else None
+    xd = to_dev(np.random.default_rng(7).standard_normal((m, K)).astype(np.float32), torch.bfloat16)
+    plain = ops.QLinear(fmt, wd, K, 2 * I, bias, torch.bfloat16)
+    fused = ops.QLinear(fmt, wd, K, 2 * I, bias, torch.bfloat16, gate_up_act=act)
+    both = plain.forward(xd)
+    plan = ops.default_context().last_plan()
+    print(f"[case] gguf fused slices {plan['kernel']} m={m}", flush=True)
+    assert "_gemm_bf16" in plan["kernel"] and plan["split_k"] > 1, plan
+    want = ops.gated_activation(both, act)
+    room = torch.full((m * I + 5,), 7.0, dtype=torch.bfloat16, device="cuda")
+    for out in (None, room[1:1 + m * I].view(m, I)):  # (the second one begins off 8 bytes)
+        y = fused.forward(xd, out=out)
+        got = ops.default_context().last_plan()
+        assert got["split_k"] == plan["split_k"] and got["launches"] == 2 and got["grid"] == plan["grid"], got
+        np.testing.assert_array_equal(bits_of(y), bits_of(want))
+    assert room[0].item() == 7.0 and (room[1 + m * I:] == 7.0).all()
+    if I % 256 == 0:
+        down = ops.QLinear(fmt, to_dev(synth.gguf_weight(fmt, 512, I, seed=3)), I, 512, None, torch.bfloat16)
+        ffn = ops.FeedForward(ops.GATE_UP_FUSED, fused, None, down, I, act)
+        np.testing.assert_array_equal(bits_of(ffn.forward(xd)), bits_of(down.forward(want)))
+
+
 def test_op_keeps_whole_sums():
     """The op's copy lies in the workspace, where the partial sums of slices would go: such a call takes whole sums, where the
     layer, whose copy is its own, takes slices."""
