@@ -11,6 +11,9 @@
 //     step 1 is multiplied, columns 4 .. 7 at the start of the upper rows' step 0, each pair of columns spread over twelve
 //     MFMAs;
 //   - weights come one block ahead, into the registers that the dequant has left (16-column strips: half blocks).
+// (f16, groups of 128, with a column's zero and scale in two registers each: four spilled, and the loop drained its loads once a
+// round.  In the halves of one: 4096 x 28672 at 65 / 128 rows 35.2 / 36.2 -> 32.1 / 33.5 us, 9344 x 18048 at 128 68.5 -> 62.3, 1024 x
+// 12544 at 256 14.6 -> 13.5.)
 // The partial tiles of the four waves meet in LDS 64 rows at a time, added in K order: the bits of pk4_mid_kernel.
 #include "pk4_mid.hpp"
 
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
     };
 
     auto column = [](int n) { return PAIRED ? (n >> 1) | ((n & 1) << 1) : n; };  // the n-th column worked on
-    uint32_t negzb[4], sp[4];
+    uint32_t pairs[4];  // f16: a column's constants in the two halves of a register, which the packed instructions select from
     Pk4gBf16 cb[4];
     Pk4N<TT> cst[4];
     auto constants = [&](int set) {  // of a group that the ring holds
@@ -156,8 +159,12 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
         for (int f = 0; f < 4; ++f) {
             if constexpr (BF) cb[f].set(__builtin_bit_cast(float, zv[f] & 0xFFFF0000u), __builtin_bit_cast(float, zv[f] << 16) + (NARROW ? 0.0f : 128.0f));
             else if constexpr (NARROW) cst[f].prep(zv[f]);
-            else Pk4T<TT>::prep(zv[f], negzb[f], sp[f]);
+            else pairs[f] = zv[f];
         }
+    };
+    auto deq_f16 = [](uint32_t q, uint32_t pair) {  // Pk4T<F16Traits>::deq
+        const half2_t c = __builtin_bit_cast(half2_t, pair), zero = __builtin_shufflevector(c, c, 0, 0), scale = __builtin_shufflevector(c, c, 1, 1);
+        return __builtin_bit_cast(uint32_t, (__builtin_bit_cast(half2_t, q) + zero) * scale);
     };
     uint32_t b[8][4];  // half a block's fragments: (step, column worked on)
     // fragments 2 ph and 2 ph + 1 of step st
@@ -186,7 +193,7 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
 #pragma unroll
                 for (int f = 2 * PH; f < 2 * PH + 2; ++f)
 #pragma unroll
-                    for (int pp = 0; pp < 4; ++pp) b[at + (f & 1)][pp] = Pk4T<TT>::deq(TT::unpack1(wp[pp], f, nm), negzb[f], sp[f]);
+                    for (int pp = 0; pp < 4; ++pp) b[at + (f & 1)][pp] = deq_f16(TT::unpack1(wp[pp], f, nm), pairs[f]);
             }
         }
     };

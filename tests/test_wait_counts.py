@@ -40,6 +40,14 @@ def test_loads_into_lds_are_over_where_a_barrier_publishes_them(found):
         assert len(at) >= 2 and max(at.values()) <= ALLOWED[kernel_of(name)], (name, {hex(a): n for a, n in at.items()})
 
 
+def test_no_form_of_128_rows_or_unrounded_weights_between_decode_and_prefill_uses_scratch(found):
+    """Their registers are full: one too many lies in scratch memory, and its reload waits for every load under way."""
+    checked = {n: c for n, c in found.items() if "pk4_mid128_kernel<" in n or "pk4_midfold_kernel<" in n}
+    assert len(checked) == 20
+    for name, code in checked.items():
+        assert not [a for a, op, *_ in code if op.startswith("scratch_")], name
+
+
 def test_a_load_that_moved_over_its_wait_is_noticed(found):
     """The same code with every counted wait one higher, as if one weight load less came before it."""
     for kernel, allowed in ALLOWED.items():
