@@ -371,13 +371,12 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     const int rows = form.rows, spw = PK4G_STRIPS / form.ks;
     const int64_t NG = ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)spw), RT = form.light ? p.M / rows : ceil_div(p.M, (int64_t)rows);
     // eight strips a workgroup: in the order of pk4g_tile_of; two strips: row tile by row tile
-    // (the two-strip forms launch what 64 rows take; those of 128 rows leave the second half idle, last in the launch)
-    const int64_t wgs = form.ks == 1 ? pk4g_workgroups(RT, NG) + (form.light ? NG : 0) : ceil_div(p.M, (int64_t)64) * NG;
+    const int64_t wgs = form.ks == 1 ? pk4g_workgroups(RT, NG) + (form.light ? NG : 0) : RT * NG;
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", form.ks > 1 ? 64 : rows, spw,
-             form.ks > 1 ? "k4" : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "", form.ks > 1 && rows == 128 ? "_r128" : "",
+    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw,
+             form.ks > 1 ? "k4" : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
              p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;

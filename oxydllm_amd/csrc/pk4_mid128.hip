@@ -46,7 +46,6 @@ __global__ __launch_bounds__(512) void pk4_mid128_kernel(const uint16_t *__restr
     const int j = g * SPW + ws_;
     const bool live = j < ((N + 63) >> 6);  // wave-uniform: the last workgroup of a layer may have one column group
     const int m0 = rt * 2 * ROWS;
-    if (m0 >= M) return;  // the launch has the workgroups of 64-row tiles: the last ones, idle
     const int NB = SETS > 1 ? (K + 127) >> 7 : K >> 7, NR = (NB + KS - 1) / KS;  // blocks; rounds of KS blocks
 
     const __amdgpu_buffer_rsrc_t rs_none = make_rsrc(pw, 0u);

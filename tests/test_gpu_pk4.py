@@ -250,7 +250,7 @@ def test_prefill_two_strips_with_k_split(kind, dtn, K, N, g, strip16):
 
 def test_prefill_takes_over_where_it_fills_the_chip():
     """With the switches at their defaults a 4096 x 14336 layer moves from the split-K tiles (one row tile) to
-    workgroups of two strips with K split inside (128 rows: 224 of them), then to 64-row and 128-row workgroups of
+    workgroups of two strips with K split inside (128 rows: 224 of them; 256 rows: as many of 128), then to 64-row and 128-row workgroups of
     eight strips as m grows (512 rows are 224 workgroups of 64 rows, 1000 rows 224 of 128), OXQ_PK4_GEMM_MIN_M = 0
     keeps the split-K tiles, and the two agree within the tolerance of one f16 rounding of y."""
     K, N, g = 4096, 14336, 128
@@ -258,7 +258,7 @@ def test_prefill_takes_over_where_it_fills_the_chip():
     layer = layer_of(trip, pack_dim, oracle.F16, None)
     rng = np.random.default_rng(5)
     xd = to_dev(rng.standard_normal((1000, K)).astype(np.float32), torch.float16)
-    for m, kern in [(64, "pk4_mfma_f16_mt4"), (128, "pk4_gemm_f16_r64x2k4"), (256, "pk4_gemm_f16_r64x2k4"), (512, "pk4_gemm_f16_r64x8"),
+    for m, kern in [(64, "pk4_mfma_f16_mt4"), (128, "pk4_gemm_f16_r64x2k4"), (256, "pk4_gemm_f16_r128x2k4"), (512, "pk4_gemm_f16_r64x8"),
                     (1000, "pk4_gemm_f16_r128x8")]:
         say(f"pk4 prefill rule m={m}")
         y = layer.forward(xd[:m])

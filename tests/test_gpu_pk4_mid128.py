@@ -38,7 +38,7 @@ def test_same_bits_as_rows_of_64(pack, dt, K, N, g, strip16):
             tune("OXQ_PK4_GEMM_ROWS", 128)
             got = layer.forward(x[:m])
             plan = layer.ctx.last_plan()
-            assert "_r64x2k4" + ("_n16" if strip16 else "") + "_r128" in plan["kernel"] and plan["grid"][0] == -(-m // 64) * -(-N // 128), plan
+            assert "_r128x2k4" + ("_n16" if strip16 else "") in plan["kernel"] and plan["grid"][0] == -(-m // 128) * -(-N // 128), plan
             np.testing.assert_array_equal(bits_of(got), bits_of(want))
 
 
@@ -60,5 +60,5 @@ def test_groups_inside_a_block(dt, K, N, g):
         tune("OXQ_PK4_GEMM_ROWS", 128)
         got = layer.forward(x[:m])
         plan = layer.ctx.last_plan()
-        assert plan["kernel"].endswith("_r64x2k4_r128"), plan
+        assert plan["kernel"].endswith("_r128x2k4") and plan["grid"][0] == -(-m // 128) * -(-N // 128), plan
         np.testing.assert_array_equal(bits_of(got), bits_of(want))
