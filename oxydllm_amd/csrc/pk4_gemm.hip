@@ -204,11 +204,17 @@ constexpr double PK4N_MID_ROUND = 0.31, PK4N_MID_PART = 0.27;
 // pk4_mid128_kernel, 128 rows and two strips, one workgroup a CU: a round (f16: a last round on at most 0.7 of the CUs) in the
 // same units.  bf16 takes 31 - 33 us a round at K = 4096 where one of 64 rows takes 22 - 25, f16 28 - 32 against 19 - 20.  Us, best
 // of the other forms -> this: bf16 4096 x 28672 at 65 / 128 / 256 rows 45 / 45 / 75 -> 33 / 34 / 66, 4096 x 14336 at 256 / 512 rows
-// 42 / 72 -> 33 / 65 (the latter left to eight strips, below), 3584 x 18944 at 128 / 384 rows 38 / 65 -> 29 / 61; f16 4096 x 28672 at 128 rows 38 -> 32, 4096 x 11008 at 256
-// 37 -> 29.  At 4096 x 28672 and 512 rows 128-row workgroups of eight strips are ahead (bf16 107 against 132).
-// Two rounds and more count 11 % more in bf16 (against three rounds of 64 rows 9344 x 18048 at 236 rows takes 132 against 128, 5120 x
-// 8576 at 487 77 against 75; level with a full round of eight strips, where 4096 x 14336 at 512 takes 65 against 72).  Against the forms of eight strips, which add no partial tiles, a short K tells: 1024 x 12544 at 583 rows
-// bf16 28.2 against 25.2, 1152 x 6272 at 994 rows f16 30.9 against 23.0.
+// 42 / 72 -> 33 / 65, 3584 x 18944 at 128 / 384 rows 38 / 65 -> 29 / 60; f16 4096 x 28672 at 128 rows 43 -> 34, 4096 x 11008 at 256
+// 39 -> 32.  At 4096 x 28672 and 512 rows 128-row workgroups of eight strips are ahead (bf16 107 against 132).
+// Beyond one round it counts 11 % more in bf16, and 7 % where K is long (from 3968 in up to two rounds, groups of 64 in any; groups of
+// 32 at any K).  Us, the form of eight strips -> this at 118 calls of other layers that lie between the two figures: groups of 128 in up to two rounds
+// 4096 x 14336 at 448 / 512 rows 70 / 74 -> 65 / 67, 3968 x 20992 at 286 69 -> 68, 4480 x 14464 at 461 79 -> 76, but 3840 x 7424 at 953
+// 67 / 71, 3328 x 10048 at 630 59 / 61; in three 7936 x 13888 at 856 181 / 195, 7040 x 11328 at 994 162 / 168; groups of 64 3968 x 16320 at 492
+// 75 -> 71, 8960 x 9920 at 1059 231 -> 209, but 3200 x 15936 at 489 63 / 68; groups of 32 3456 x 14272 at 477 71 -> 65, 7808 x 17088 at
+// 1137 397 -> 335.  Against three rounds of 64 rows 9344 x 18048 at 236 rows takes 132 against 128, 5120 x 8576 at 487 77 against 75.  Against
+// the forms of eight strips, which add no partial tiles, a short K tells: 1024 x 12544 at 583 rows bf16 28.2 against 25.2, 1152 x 6272 at
+// 994 rows f16 30.9 against 23.0.  (f16: figures 7 % lower, what its kernel has gained since they were fitted, choose no better: 2.1 % behind the
+// fastest form together over ten layers, 80 calls, 1.9 % with these.)
 // Groups of 64 and 32 go by the same figures (115 layers, 345 calls at 65 - 2200 rows: 65 came here, 1.27 times as fast, the
 // least 1.05; 4096 x 15488, groups of 64, bf16 at 448 rows 80 -> 72, 8960 x 14720, groups of 32, at 243 100 -> 78).
 // 16-column strips: a round, and a last one on at most 0.8 of the CUs.  bf16 at K = 4096 takes 31 - 32 and 36 us, f16 30 - 31 and 36; us,
@@ -222,6 +228,7 @@ struct Pk4Mid128Cost {
 constexpr Pk4Mid128Cost PK4_MID128_BF16 = {0.455, 0.455, 0.7, 1.0, 1.11}, PK4_MID128_F16 = {0.505, 0.45, 0.7, 1.0, 1.04};
 constexpr Pk4Mid128Cost PK4N_MID128_BF16 = {0.52, 0.465, 0.8, 1.0, 1.08}, PK4N_MID128_F16 = {0.57, 0.50, 0.8, 1.0, 1.04};
 constexpr double PK4_MID128_LONG_K = 0.92, PK4_MID128_OVER_K = 314.0;
+constexpr double PK4_MID128_BF16_MORE_LONG_K = 1.07;  // 64-column strips
 
 struct Pk4GemmCost {
     bool pairs64;
@@ -331,9 +338,12 @@ static Pk4GemmForm pk4_gemm_form(const oxq_ctx *ctx, const Pk4Problem &p) {
     // (the split-K tiles address the whole of x with 32 bits)
     const double w_mid128 = (double)(ceil_div(ceil_div(p.w.N, (int64_t)64), (int64_t)2) * ceil_div(p.M, (int64_t)128)) / cus;
     const Pk4Mid128Cost &h = p.w.strip == 16 ? (f16 ? PK4N_MID128_F16 : PK4N_MID128_BF16) : (f16 ? PK4_MID128_F16 : PK4_MID128_BF16);
+    const int sets = pk4_sets(p.w.group_shift);
+    const bool long_k = !f16 && p.w.strip != 16 && (sets == 4 || (p.w.K >= 3968 && (sets == 2 || w_mid128 <= 2.0)));
     const double c_mid128 = !can_mid128 || forced_ks == 1
                                 ? 1e30
-                                : rounds(w_mid128, h.full, h.part, h.part_upto) * (w_mid128 > h.more_from ? h.more : 1.0);
+                                : rounds(w_mid128, h.full, h.part, h.part_upto) *
+                                      (w_mid128 <= h.more_from ? 1.0 : long_k ? PK4_MID128_BF16_MORE_LONG_K : h.more);
     const double c_mid128_k = c_mid128 * (PK4_MID128_LONG_K + PK4_MID128_OVER_K / (double)p.w.K);
     // (against split-K tiles in whole rounds: 3584 x 18944 at 128 rows, 2.3 of them, takes 38 us in bf16, by 2.3 / 8 it would be 28)
     if (c_mid128_k < c64 && c_mid128_k < c128 && c_mid128_k < c_light && c_mid128 < c_mid &&

@@ -428,8 +428,8 @@ def test_layers_validate_like_reference(lib, ctx):
     # of eight strips would leave most of the chip idle, then row tiles of 64 or 128 x eight strips, whichever needs
     # the cheaper rounds of 256 workgroups
     for rows, kern, wgs in [(64, "pk4_mfma_bf16_mt4", None), (65, "pk4_gemm_bf16_r64x2k4", 2 * 112),
-                            (256, "pk4_gemm_bf16_r128x2k4", 2 * 112), (384, "pk4_gemm_bf16_r64x2k4", 6 * 112), (448, "pk4_gemm_bf16_r64x8", 7 * 28),
-                            (512, "pk4_gemm_bf16_r64x8", 4 * 64),
+                            (256, "pk4_gemm_bf16_r128x2k4", 2 * 112), (384, "pk4_gemm_bf16_r64x2k4", 6 * 112), (448, "pk4_gemm_bf16_r128x2k4", 4 * 112),
+                            (512, "pk4_gemm_bf16_r128x2k4", 4 * 112),
                             (768, "pk4_gemm_bf16_r128x8", 6 * 28), (1000, "pk4_gemm_bf16_r128x8", 4 * 64),
                             (1536, "pk4_gemm_bf16_r64x8", 3 * 4 * 64), (1537, "pk4_gemm_bf16_r64x8", 3 * 4 * 64 + 28),
                             (2100, "pk4_gemm_bf16_r128x8", 2 * 4 * 64 + 28),
