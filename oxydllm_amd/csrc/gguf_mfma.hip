@@ -1828,10 +1828,10 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &problem, bo
     const int64_t chunks = p.K / 128;
     const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)ks) * ks) : (int)chunks;
     dim3 grid((unsigned)wgs, (unsigned)form.slices);
-    // the family (eight waves side by side, or K split inside the workgroup too), then the rows where they are not the 64 of its first form
+    // rows x column groups of the workgroup, and the waves that share K inside it
     char name[64], slices[16] = "";
     if (form.slices > 1) snprintf(slices, sizeof slices, "_s%d", form.slices);
-    snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r64x%s%s%s%s", ggm_name(p.quant), ks > 1 ? "2k4" : "8", slices, rows == 128 ? "_r128" : "",
+    snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%d%s%s%s", ggm_name(p.quant), rows, spw, ks == 4 ? "k4" : ks == 2 ? "k2" : "", slices,
              problem.act == 1 ? "_silu" : problem.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), form.slices, 1, form.slices > 1 ? (size_t)form.slices * p.M * p.N * 4 : 0);
     if (ctx->plan_only) {

@@ -384,7 +384,7 @@ def test_feed_forward_validates_and_plans(lib, ctx):
     assert rc == 0, err(lib)
     elems = C.c_int64()
     assert lib.oxq_mlp_scratch_elems(m, 2, C.byref(elems)) == 0 and elems.value == 2 * 3 * I
-    for rows, kern in [(2, "gguf_q4k_mfma_bf16_mt1"), (100, "gguf_q4k_gemm_bf16_r64x2k4_s")]:  # the down projection ran last
+    for rows, kern in [(2, "gguf_q4k_mfma_bf16_mt1"), (100, "gguf_q4k_gemm_bf16_r128x4k2_s")]:  # the down projection ran last
         assert lib.oxq_mlp_forward(m, None, C.byref(fake((rows, H), BF16)), C.byref(fake((rows * 3 * I,), BF16)),
                                    C.byref(fake((rows, H), BF16))) == 0, err(lib)
         assert plan(lib, ctx).kernel.decode().startswith(kern), plan(lib, ctx).kernel
@@ -485,12 +485,12 @@ def test_layers_validate_like_reference(lib, ctx):
     for m_rows, kern in [(1, "gguf_q4k_mfma_bf16_mt1"), (2, "gguf_q4k_mfma_bf16_mt1"),
                          (4, "gguf_q4k_mfma_bf16_mt1"), (8, "gguf_q4k_mfma_bf16_mt1"),
                          (16, "gguf_q4k_mfma_bf16_mt1"), (32, "gguf_q4k_mfma_bf16_mt2"), (33, "gguf_q4k_gemm_bf16_r64x2k4_s8"),
-                         # more rows: the prefill kernels on the layer's copy - 32 pairs of column groups x row tiles of
-                         # 64 with K split inside the workgroup and, where those leave CUs idle, over K slices of
-                         # workgroups, and eight groups of 512 columns x row tiles once those fill the chip
+                         # more rows: the prefill kernels on the layer's copy - 32 groups of 128 columns x row tiles of
+                         # 64, then of 128, with K split inside the workgroup and, where those leave CUs idle, over K slices of
+                         # workgroups, and sixteen groups of 256 columns x row tiles of 128 once those fill the chip
                          (128, "gguf_q4k_gemm_bf16_r64x2k4_s4"), (256, "gguf_q4k_gemm_bf16_r64x2k4"),
-                         (1024, "gguf_q4k_gemm_bf16_r64x2k4"), (2048, "gguf_q4k_gemm_bf16_r64x8"),
-                         (4096, "gguf_q4k_gemm_bf16_r64x8")]:
+                         (1024, "gguf_q4k_gemm_bf16_r128x4k2"), (2048, "gguf_q4k_gemm_bf16_r128x8"),
+                         (4096, "gguf_q4k_gemm_bf16_r128x8")]:
         assert lib.oxq_qlinear_forward(q, None, C.byref(fake((m_rows, 4096), BF16)),
                                        C.byref(fake((m_rows, 4096), BF16))) == 0, err(lib)
         p = plan(lib, ctx)

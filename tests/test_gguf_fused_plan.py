@@ -26,7 +26,7 @@ def test_same_form_as_the_plain_layer(fmt):
                     p = plan.last_plan()
                     seen.append((p["kernel"], tuple(p["grid"]), p["split_k"], p["workspace_bytes"]))
                 (kernel, *form), got = seen
-                if "_gemm_" not in kernel or ("_r128" not in kernel and form[1] > 1):  # slices of 64 rows: row tiles of the integer kernel
+                if "_gemm_" not in kernel or ("_r128x" not in kernel and form[1] > 1):  # slices of 64 rows: row tiles of the integer kernel
                     assert "_gemm_" not in got[0], (K, N, m, seen)
                     continue
                 assert got == (kernel + "_silu", *form), (K, N, m, seen)

@@ -10,6 +10,7 @@ from tests.helpers import assert_close, bits_of, round_x, to_dev, tune
 pytestmark = pytest.mark.gpu
 
 WIDE, PAIRS = 8, 2  # OXQ_GGUF_GEMM_KS: 256 columns; 128 columns, K over two waves
+NAME = {WIDE: "_r128x8", PAIRS: "_r128x4k2"}
 FMTS = [synth.GGUF_Q4_K, synth.GGUF_Q8_0, synth.GGUF_Q5_1, synth.GGUF_Q6_K, synth.GGUF_Q2_K, synth.GGUF_Q3_K]
 
 
@@ -33,7 +34,7 @@ def test_rows_at_the_edges(fmt, N, K):
             print(f"[case] gguf 128 rows {name} N={N} K={K} m={m} form={form}", flush=True)
             y = layer.forward(xd[:m])
             plan = ops.default_context().last_plan()
-            assert plan["kernel"].endswith("_r128") and plan["launches"] == 1, plan
+            assert plan["kernel"].endswith(NAME[form]) and plan["launches"] == 1, plan
             assert_close(y, ref[:m], f"gguf 128 rows {name} m={m}", bf16_out=True)
             if first is None:
                 first = bits_of(y)
@@ -53,7 +54,7 @@ def test_fused_activation(fmt, form):
     fused = ops.QLinear(fmt, wd, K, 2 * I, bias, torch.bfloat16, gate_up_act=ops.ACT_GATED_SILU)
     for m in (40, 150):
         y = fused.forward(xd[:m])
-        assert ops.default_context().last_plan()["kernel"].endswith("_r128_silu")
+        assert ops.default_context().last_plan()["kernel"].endswith(NAME[form] + "_silu")
         np.testing.assert_array_equal(bits_of(y), bits_of(ops.gated_activation(plain.forward(xd[:m]), ops.ACT_GATED_SILU)))
 
 
@@ -68,7 +69,7 @@ def test_slices():
     print(f"[case] gguf 128 rows in slices {plan['kernel']}", flush=True)
     ref = oracle.matmul_nt_f32(round_x(x, oracle.BF16), oracle.round_through(oracle.dequantize_gguf(fmt, data, N, K), oracle.BF16))
     assert_close(y, ref, plan["kernel"], bf16_out=True)
-    assert plan["kernel"].endswith("_r128") and plan["split_k"] > 1 and plan["launches"] == 2, plan
+    assert f"{NAME[PAIRS]}_s" in plan["kernel"] and plan["split_k"] > 1 and plan["launches"] == 2, plan
 
 
 @pytest.mark.parametrize("fmt,K,I,m,act,biased", [(synth.GGUF_Q4_K, 8192, 2048, 300, ops.ACT_GATED_SILU, True), (synth.GGUF_Q4_K, 8192, 1024, 777, ops.ACT_GATED_GELU_TANH, False),

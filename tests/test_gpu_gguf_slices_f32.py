@@ -163,7 +163,7 @@ def test_prefill_rows_of_few_columns(fmt, N, K):
         say(f"gguf slices {synth.GGUF_NAMES[fmt]} N={N} K={K} m={m} {plan['kernel']} x {plan['split_k']}")
         whole = "_mfma_bf16_mt2" in plan["kernel"]  # row tiles of the integer kernel: the weights unrounded
         assert plan["launches"] == (2 if plan["split_k"] > 1 else 1) and (slices is None or plan["split_k"] > 1), plan
-        assert whole or "_gemm_bf16_r64x" in plan["kernel"], plan
+        assert whole or "_gemm_bf16_r" in plan["kernel"], plan
         ref = oracle.matmul_nt_f32(round_x(x, oracle.BF16), w if whole else wr, round_x(bias, oracle.BF16))
         assert_close(y, ref, f"{synth.GGUF_NAMES[fmt]} m={m}", bf16_out=True)
     for m in (1, 17, 32):  # the integer kernel on a ragged last strip
