@@ -182,7 +182,12 @@ __device__ __forceinline__ void group_pairs_small(const int32_t *top_idx, const 
 // What bounds it: a chain of dependent steps (two trips to memory, three barriers), and in one workgroup for all pairs
 // the scattered stores, three a pair, and what it ranks batch by batch: 2060 / 4096 / 16384 / 32768 pairs took 5.7 / 7.8 /
 // 32.6 / 62 us in one workgroup, 4.6 / 4.7 / 6.5 / 8.3 in their own; up to 1024 pairs, one workgroup, 2.9 - 3.0 either way.
-// Every workgroup counting everything costs one LDS addition a lane and 1024 pairs.
+// Every workgroup counting everything costs one LDS addition a lane and 1024 pairs; the additions of a wave to one count come one
+// after the other, and workgroups times pairs is the square of the pairs.  So beyond GROUP_ONE batches (MANY) there are
+// at most GROUP_MOST workgroups, of neighbouring batches, and a wave's lanes add to eight copies of a count.  Us, evenly spread ids
+// over 32 experts / all pairs of one: one workgroup for all 131072 pairs 180 / 128, one a batch 20 / 113, MANY 18 / 21; 1048576 1895 /
+// 1399, 414 / 3520, 133 / 137; 4194304 7542 / 5573, 6100 / 56200, 501 / 527.  At 36000 one a batch 8.6 / 34, MANY 8.3 / 8.9; at 16384
+// evenly spread ids lose 0.4 to the copies.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void moe_group_kernel(const int32_t *__restrict__ top_idx,
                                                        const float *__restrict__ top_vals, int P, int E,
@@ -193,84 +198,106 @@ __global__ __launch_bounds__(64) void moe_group_kernel(const int32_t *__restrict
     group_pairs_small(top_idx, top_vals, P, E, top_k, group_lds, (int)threadIdx.x, offsets, tokens, weights, pair_pos);
 }
 
-constexpr int GROUP_WAVES = 16, GROUP_PAIRS = GROUP_WAVES * 64;
+constexpr int GROUP_WAVES = 16, GROUP_PAIRS = GROUP_WAVES * 64, GROUP_ONE = 32, GROUP_MOST = 256;
+// ints of LDS: a row of counts a wave, start and one more array, and MANY the copies of the counts before and from the own pairs on
+constexpr size_t group_lds_ints(int64_t E, bool many) { return (size_t)(GROUP_WAVES + 2) * E + (many ? 2 * 8 * (size_t)(E + 1) : 0); }
+template <bool MANY>
 __global__ __launch_bounds__(GROUP_PAIRS) void moe_group_waves_kernel(
     const int32_t *__restrict__ top_idx, const float *__restrict__ top_vals, int P, int E,
     int32_t *__restrict__ offsets, int32_t *__restrict__ tokens, float *__restrict__ weights,
-    int32_t *__restrict__ pair_pos, int top_k) {
-    extern __shared__ int32_t group_lds[];  // cnt[GROUP_WAVES][E], before[E], after[E]
+    int32_t *__restrict__ pair_pos, int top_k, int batches) {
+    constexpr int COPIES = MANY ? 8 : 1;
+    extern __shared__ int32_t group_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int32_t *cnt = group_lds + (size_t)wave * E;
-    int32_t *before = group_lds + (size_t)GROUP_WAVES * E, *after = before + E;
-    const int own = (int)blockIdx.x, chunks = (P + GROUP_PAIRS - 1) / GROUP_PAIRS;
-    const int64_t i64 = (int64_t)own * GROUP_PAIRS + tid;
-    const bool mine_in = i64 < P;
-    const int i = (int)i64;
-    const int e = mine_in ? top_idx[i] : -1;
-    const float val = mine_in ? top_vals[i] : 0.0f;
+    int32_t *start = group_lds + (size_t)GROUP_WAVES * E, *base = start + E;  // base: MANY only
+    const int stride = MANY ? E + 1 : E;  // of copies, in different banks
+    int32_t *before = MANY ? base + E : start, *after = before + COPIES * stride;  // without MANY `after` is where base would be
+    const int chunks = (int)(((int64_t)P + GROUP_PAIRS - 1) / GROUP_PAIRS);
+    const int first = MANY ? (int)blockIdx.x * batches : (int)blockIdx.x, last = MANY ? min(chunks, first + batches) : first + 1;
+    int64_t at = (int64_t)first * GROUP_PAIRS + tid;
+    int e = at < P ? top_idx[at] : -1;
+    float val = at < P ? top_vals[at] : 0.0f;
     for (int x = lane; x < E; x += 64) cnt[x] = 0;  // the wave's own row: its LDS accesses stay in order
-    const bool others = chunks > 1;  // launch-uniform; without others before[] is only written below
+    const bool others = MANY || chunks > 1;  // launch-uniform; without others before[] is only written below
     if (others) {
-        for (int x = tid; x < 2 * E; x += GROUP_PAIRS) before[x] = 0;
+        for (int x = tid; x < 2 * COPIES * stride; x += GROUP_PAIRS) before[x] = 0;
         __syncthreads();
     }
-    // the other chunks' experts, eight loads in flight
+    // the other chunks' experts (MANY: all), eight loads in flight
     for (int q0 = 0; others && q0 < chunks; q0 += 8) {
         int other[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const int q = q0 + u;
             const int64_t j = (int64_t)q * GROUP_PAIRS + tid;
-            other[u] = q != own && j < P ? top_idx[j] : -1;
+            other[u] = (MANY || q != first) && j < P ? top_idx[j] : -1;
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            if (other[u] >= 0 && other[u] < E) atomicAdd((q0 + u < own ? before : after) + other[u], 1);
+            if (other[u] >= 0 && other[u] < E) atomicAdd((q0 + u < first ? before : after) + (tid & (COPIES - 1)) * stride + other[u], 1);
     }
-    const bool ok = e >= 0 && e < E;  // ids outside [0, E) are dropped
-    const unsigned long long mine = lanes_with_my_expert(e, ok, expert_id_bits(E));
-    const int rank = __builtin_popcountll(mine & ((1ull << lane) - 1ull));
-    if (ok && rank == 0) cnt[e] = __builtin_popcountll(mine);
-    __syncthreads();
-    // per expert: exclusive prefix over the chunks before and the waves, total in before[e]
-    for (int x = tid; x < E; x += GROUP_PAIRS) {
-        int c[GROUP_WAVES], run = others ? before[x] : 0;
+    for (int q = first;;) {
+        const bool ok = e >= 0 && e < E;  // ids outside [0, E) are dropped
+        const unsigned long long mine = lanes_with_my_expert(e, ok, expert_id_bits(E));
+        const int rank = __builtin_popcountll(mine & ((1ull << lane) - 1ull));
+        if (ok && rank == 0) cnt[e] = __builtin_popcountll(mine);
+        __syncthreads();
+        // per expert: exclusive prefix over the pairs before and the waves; in the first batch the total in start[e]
+        for (int x = tid; x < E; x += GROUP_PAIRS) {
+            int c[GROUP_WAVES], run = 0, total = 0;
+            if (q != first) {
+                run = base[x];
+            } else if (others) {
 #pragma unroll
-        for (int w = 0; w < GROUP_WAVES; ++w) c[w] = group_lds[(size_t)w * E + x];  // independent reads first
-#pragma unroll
-        for (int w = 0; w < GROUP_WAVES; ++w) {
-            group_lds[(size_t)w * E + x] = run;
-            run += c[w];
-        }
-        before[x] = others ? run + after[x] : run;
-    }
-    __syncthreads();
-    int32_t *start = before;
-    if (wave == 0) {  // exclusive scan of the totals in expert order, 64 experts per round
-        int carry = 0;
-        for (int e1 = 0; e1 < E; e1 += 64) {
-            const int ee = e1 + lane;
-            const int c = ee < E ? start[ee] : 0;
-            int incl = c;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int t = __shfl_up(incl, off, 64);
-                if (lane >= off) incl += t;
+                for (int w = 0; w < COPIES; ++w) run += before[w * stride + x], total += MANY ? after[w * stride + x] : 0;
+                if (MANY) total += run;
             }
-            if (ee < E) {
-                start[ee] = carry + incl - c;
-                if (own == 0) offsets[ee] = carry + incl - c;
+#pragma unroll
+            for (int w = 0; w < GROUP_WAVES; ++w) c[w] = group_lds[(size_t)w * E + x];  // independent reads first
+#pragma unroll
+            for (int w = 0; w < GROUP_WAVES; ++w) {
+                group_lds[(size_t)w * E + x] = run;
+                run += c[w];
             }
-            carry += __shfl(incl, 63, 64);
+            if (MANY) base[x] = run;
+            if (q == first) start[x] = MANY ? total : others ? run + after[x] : run;
         }
-        if (lane == 0 && own == 0) offsets[E] = carry;
+        __syncthreads();
+        if (q == first) {
+            if (wave == 0) {  // exclusive scan of the totals in expert order, 64 experts per round
+                int carry = 0;
+                for (int e1 = 0; e1 < E; e1 += 64) {
+                    const int ee = e1 + lane;
+                    const int c = ee < E ? start[ee] : 0;
+                    int incl = c;
+#pragma unroll
+                    for (int off = 1; off < 64; off <<= 1) {
+                        const int t = __shfl_up(incl, off, 64);
+                        if (lane >= off) incl += t;
+                    }
+                    if (ee < E) {
+                        start[ee] = carry + incl - c;
+                        if (first == 0) offsets[ee] = carry + incl - c;
+                    }
+                    carry += __shfl(incl, 63, 64);
+                }
+                if (lane == 0 && first == 0) offsets[E] = carry;
+            }
+            __syncthreads();
+        }
+        if (ok) {
+            const int pos = start[e] + cnt[e] + rank;
+            tokens[pos] = (int)at / top_k;
+            weights[pos] = val;
+            pair_pos[at] = pos;
+        }
+        if (!MANY || ++q == last) break;
+        for (int x = lane; x < E; x += 64) cnt[x] = 0;
+        at += GROUP_PAIRS;
+        e = at < P ? top_idx[at] : -1;
+        val = at < P ? top_vals[at] : 0.0f;
     }
-    __syncthreads();
-    if (!ok) return;
-    const int pos = start[e] + cnt[e] + rank;
-    tokens[pos] = i / top_k;
-    weights[pos] = val;
-    pair_pos[i] = pos;
 }
 
 // ---------------------------------------------------------------------------
@@ -481,16 +508,18 @@ int launch_moe_route(oxq_ctx *ctx, hipStream_t s, const void *logits, int dtype,
 int launch_moe_group(oxq_ctx *ctx, hipStream_t s, const int32_t *top_idx, const float *top_vals, int64_t P, int64_t E,
                      int64_t top_k, int32_t *offsets, int32_t *tokens, float *weights, int32_t *pair_pos) {
     const bool small = P <= 64;
-    dim3 grid(small ? 1u : (unsigned)ceil_div(P, GROUP_PAIRS)), block(small ? 64 : GROUP_PAIRS);
+    const int64_t chunks = ceil_div(P, (int64_t)GROUP_PAIRS), batches = ceil_div(chunks, (int64_t)GROUP_MOST);
+    const bool many = chunks > GROUP_ONE;
+    dim3 grid(small ? 1u : (unsigned)ceil_div(chunks, std::max<int64_t>(batches, 1))), block(small ? 64 : GROUP_PAIRS);
     set_plan(ctx, "moe_group", grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if (small) {
         hipLaunchKernelGGL(moe_group_kernel, grid, block, 2 * (size_t)E * sizeof(int32_t), s, top_idx, top_vals, (int)P,
                            (int)E, offsets, tokens, weights, pair_pos, (int)top_k);
     } else {
-        const size_t lds = ((size_t)GROUP_WAVES + 2) * (size_t)E * sizeof(int32_t);  // at most 18 KB (256 experts)
-        hipLaunchKernelGGL(moe_group_waves_kernel, grid, block, lds, s, top_idx, top_vals, (int)P, (int)E, offsets,
-                           tokens, weights, pair_pos, (int)top_k);
+        const size_t lds = group_lds_ints(E, many) * sizeof(int32_t);  // at most 34 KB (256 experts)
+        hipLaunchKernelGGL(many ? moe_group_waves_kernel<true> : moe_group_waves_kernel<false>, grid, block, lds, s, top_idx, top_vals, (int)P, (int)E,
+                           offsets, tokens, weights, pair_pos, (int)top_k, (int)batches);
     }
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;

@@ -465,10 +465,11 @@ def test_moe_group_matches_oracle(T, E, k):
     np.testing.assert_array_equal(rw[pos.ravel()], rvals.ravel())
 
 
-@pytest.mark.parametrize("T,E,k", [(13, 7, 5), (256, 7, 4), (205, 64, 5), (2049, 1, 1), (2300, 130, 8)])
+@pytest.mark.parametrize("T,E,k", [(13, 7, 5), (256, 7, 4), (205, 64, 5), (2049, 1, 1), (2300, 130, 8), (9000, 70, 5),
+                                   (70001, 33, 4), (131073, 256, 2)])
 def test_moe_group_drops_ids_outside_the_experts(T, E, k):
-    """Pairs of an id outside [0, E) reach no list, in the chunk of 1024 pairs that holds them as in the others, and keep
-    their pair_pos; all remaining pairs of one expert stay in order."""
+    """Pairs of an id outside [0, E) reach no list, in the batch of 1024 pairs that holds them as in the others, and keep
+    their pair_pos; all remaining pairs of one expert stay in order.  (The last two: several batches a workgroup.)"""
     say(f"moe group T={T} E={E} k={k} with ids out of range")
     ids = np.random.default_rng(T).choice([-1, E // 2, E - 1, E, 1 << 20], size=(T, k), p=[.1, .6, .2, .05, .05]).astype(np.int32)
     vals = np.arange(T * k, dtype=np.float32).reshape(T, k)
