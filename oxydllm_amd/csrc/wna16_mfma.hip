@@ -701,11 +701,7 @@ static bool transient_repack_fits(const oxq_ctx *ctx, const Wna16Problem &p) {
            !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0) &&
            ((pk4_weight_bytes(p.K, p.N, p.bits, pk4_sets(p.group_shift)) + 255) & ~(size_t)255) <= ctx->workspace_bytes;
 }
-static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
-    Pk4Weights w{(uint32_t *)ctx->workspace, nullptr, p.K, p.N, p.group_shift, p.dtype, p.bits, 0,
-                   p.pack_dim == OXQ_PACK_IN ? 32 : 16, 64, pk4_unrounded(p)};
-    int rc = launch_pk4_prepack(ctx, s, p, w);
-    if (rc != OXQ_OK) return rc;
+static Pk4Problem transient_problem(const oxq_ctx *ctx, const Wna16Problem &p) {
     Pk4Problem q;
     q.x = p.x;
     q.bias = p.bias;
@@ -713,31 +709,47 @@ static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Probl
     q.M = p.M;
     q.act = 0;
     q.no_split = 1;  // the workspace holds the copy: no room for K slices' partials
-    q.w = w;
+    q.w = Pk4Weights{(uint32_t *)ctx->workspace, nullptr, p.K, p.N, p.group_shift, p.dtype, p.bits, 0,
+                     p.pack_dim == OXQ_PACK_IN ? 32 : 16, 64, pk4_unrounded(p)};
+    return q;
+}
+static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
+    const Pk4Problem q = transient_problem(ctx, p);
+    int rc = launch_pk4_prepack(ctx, s, p, q.w);
+    if (rc != OXQ_OK) return rc;
     rc = launch_pk4_forward(ctx, s, q);
     ctx->plan.launches = 2;
     return rc;
 }
 
+// GPTQ tensors that the tile kernel takes (workgroups of 64 rows x 64 columns): it is ahead while these are one round of CUs.  From two
+// rounds the copy is, where its prefill forms take the call (8-bit in f16: unless a last round of two or three is nearly full), in 4 bits
+// from six row tiles on (bf16 layers of 2^25 weights: four), in 8 bits from seven.  Below 3/4 of 2^24 weights, and at most everywhere,
+// 640 rows.  Us, tile kernel / repack and resident kernel: 4-bit f16 4096 x 4096 at 256 / 512 / 576 rows 16.8 / 23.8, 28.2 / 27.9, 38.9 /
+// 34.5, 8192 x 2048 at 448 / 576 25.2 / 30.1, 44.9 / 36.0, 4096 x 14336 at 448 91 / 74, bf16 at 256 59 / 47; 8-bit f16 4096 x 14336 at
+// 512 116 / 99, 8192 x 3072 at 448 52 / 48, 6528 x 6464 at 400, 2.76 rounds, 84 / 89, bf16 92 / 89, 4096 x 5120 at 448, left to the split-K
+// tiles, 44 / 53.  On 147 other layers (8232 calls of 100 - 1500 rows) against 640 rows everywhere: 34 slower by 3 % and more, 2.5 % less time.
+static bool gptq_repack_pays(const oxq_ctx *ctx, const Wna16Problem &p) {
+    if (p.M >= 640) return true;
+    const int64_t size = p.K * p.N, least = 3 << 22, row_tiles = ceil_div(p.M, (int64_t)64);
+    const double w = (double)(row_tiles * (p.N / 64)) / (ctx->num_cus > 0 ? ctx->num_cus : 256), rounds = std::ceil(w);
+    if (size < least || rounds < 2.0) return false;
+    if (p.bits == 4 ? row_tiles < (p.dtype != OXQ_F16 && size >= (1 << 25) ? 4 : 6) : row_tiles < 7 || (p.dtype == OXQ_F16 && rounds < 4.0 && w > 0.9 * rounds)) return false;
+    return pk4_gemm_takes(ctx, transient_problem(ctx, p));
+}
+
 int launch_wna16_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
-    // The resident layout's kernels run at two to six times the rate of the kernels on the checkpoint layout, which pays for the
-    // repack (9 us at 4096 x 14336, 4-bit) from few rows on: AWQ in bf16 behind the 16 rows of the slab kernel, in f16 from 49 rows (up to 48 the
-    // resident kernels fold sums, which make NaN of an infinite x), on layers of more than 2^24 weights 64, with few columns 128; the GPTQ tile kernel is ahead longer.  Us, checkpoint layout / repack and resident kernel:
-    // AWQ 4-bit bf16 4096 x 14336 at 20 / 64 / 640 rows 46 / 23, 56 / 27, 656 / 110, 4096 x 4096 at 32 28 / 16, 1536 x 2048 at 20 16 / 10;
-    // f16 4096 x 14336 at 32 / 64 / 640 20 / 24, 28 / 27, 189 / 103, 4096 x 4096 at 20 / 32 14 / 14, 21 / 14; GPTQ 4-bit f16 4096 x
-    // 14336 at 160 / 256 41 / 42, 54 / 44, 8192 x 3072 at 256 / 448 24 / 31, 45 / 40, 1536 x 2048 at 448 / 640 9 / 12, 16 / 14; 8-bit 4096 x
-    // 14336 at 256 / 448 64 / 73, 110 / 100; AWQ f16 11008 x 3584 at 90 / 200 29 / 34, 44 / 37.  Up to 16 rows in bf16: AWQ 4-bit 4096 x
-    // 14336 at 9 rows, tile / slab kernel, 43 / 13.
+    // The resident layout's kernels run at two to six times the rate of the AWQ kernels on the checkpoint layout, which pays for the
+    // repack (9 us at 4096 x 14336, 4-bit) from few rows on: in bf16 behind the 16 rows of the slab kernel, in f16 from 49 rows (up to
+    // 48 the resident kernels fold sums, which make NaN of an infinite x), on layers of more than 2^24 weights 64, with few columns
+    // 128.  Us, checkpoint layout / repack and resident kernel: bf16 4096 x 14336 at 20 / 64 / 640 rows 46 / 23, 56 / 27, 656 / 110, 4096 x
+    // 4096 at 32 28 / 16, 1536 x 2048 at 20 16 / 10; f16 4096 x 14336 at 32 / 64 / 640 20 / 24, 28 / 27, 189 / 103, 4096 x 4096 at 20 / 32
+    // 14 / 14, 21 / 14, 11008 x 3584 at 90 / 200 29 / 34, 44 / 37.  Up to 16 rows in bf16: 4096 x 14336 at 9 rows, tile / slab kernel, 43 / 13.
     const bool awq = awq4_mfma_ok(p), gptq = !awq && gptq_tile_ok(p) && tune(ctx, OXQ_TUNE_GPTQ_TILE, 1) != 2;
     if (awq && p.M <= 16 && wna16_slab_takes(ctx, p)) return launch_wna16_slab(ctx, s, p);
     const int64_t size = p.K * p.N;
-    const bool f16 = p.dtype == OXQ_F16;
-    int64_t repack_from;
-    if (awq && f16) repack_from = size < (1 << 21) ? 640 : size <= (1 << 24) ? 49 : p.K >= 2 * p.N ? 128 : 64;
-    else if (awq) repack_from = size < (1 << 21) ? 80 : 17;
-    else if (p.bits == 4 && size >= (1 << 25)) repack_from = f16 ? 352 : 256;
-    else repack_from = size > (1 << 24) || (p.bits == 4 && size == (1 << 24)) ? 448 : 640;
-    if (p.M >= repack_from && (awq || gptq) && transient_repack_fits(ctx, p)) return launch_transient_repack(ctx, s, p);
+    const int64_t awq_from = p.dtype != OXQ_F16 ? (size < (1 << 21) ? 80 : 17) : size < (1 << 21) ? 640 : size <= (1 << 24) ? 49 : p.K >= 2 * p.N ? 128 : 64;
+    if ((awq ? p.M >= awq_from : gptq && gptq_repack_pays(ctx, p)) && transient_repack_fits(ctx, p)) return launch_transient_repack(ctx, s, p);
     if (awq4_mfma_ok(p) && !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0))
         return p.dtype == OXQ_F16 ? launch_awq4_mfma<F16Traits>(ctx, s, p)
                                   : launch_awq4_mfma<BF16Traits>(ctx, s, p);

@@ -1,5 +1,5 @@
-"""The AWQ ops on checkpoint tensors where their kernel changes: one row of ragged columns, bf16 at 9 - 16 rows, and the rows from which the
-tile op builds the tile-major copy for its call."""
+"""The ops on checkpoint tensors where their kernel changes: AWQ, one row of ragged columns and bf16 at 9 - 16 rows; AWQ and GPTQ, the rows
+from which the tile op builds the tile-major copy for its call."""
 import numpy as np
 import pytest
 import torch
@@ -50,6 +50,28 @@ def test_rows_at_the_lines_of_the_rule(dtn, K, N, g, rows):
         assert slab == (m <= 16 and dtn == "bf16") and plan["kernel"].startswith("pk4_") == resident, plan
         unrounded = slab or resident and not resident_rounds_weights(m, dt, False)
         assert_close(y, oracle.matmul_nt_f32(round_x(x[:m], dt), w if unrounded else wr), f"m{m} {plan['kernel']}")
+
+
+# (rows that stay on the tile kernel, rows of a copy): one round of the tile kernel's workgroups, and the row tiles the rule asks for
+@pytest.mark.parametrize("bits,dtn,K,N,edges", [
+    (4, "f16", 3072, 4096, ((320, 321),)), (4, "f16", 8192, 2048, ((448, 513), (512, 513))), (4, "f16", 4096, 8192, ((320, 321),)),
+    (4, "bf16", 4096, 8192, ((192, 193),)), (4, "bf16", 3072, 4032, ((639, 640),)), (8, "f16", 8192, 3072, ((384, 385), (577, 640))),
+    (8, "f16", 3072, 4160, ((384, 385), (449, 577))), (8, "bf16", 1920, 6592, ((384, 385),))])
+def test_rows_at_the_lines_of_the_gptq_rule(bits, dtn, K, N, edges):
+    dt, tdt = DT[dtn]
+    q, z, s = synth.gptq_checkpoint(K, N, 128, bits, seed=K + N + bits)
+    s_r = oracle.round_through(s, dt)
+    w = oracle.round_through(oracle.dequantize_gptq(q, z, s_r, bits), dt)
+    x = np.random.default_rng(K).standard_normal((max(m for pair in edges for m in pair), K)).astype(np.float32)
+    xd, args = to_dev(x, tdt), (to_dev(q), to_dev(z), to_dev(s, tdt))
+    ref = oracle.matmul_nt_f32(round_x(x, dt), w)
+    for pair in edges:
+        for m, copied in zip(pair, (False, True)):
+            y = ops.mpp_quant_matmul(xd[:m], *args, bits, ops.PACK_IN)
+            plan = ops.default_context().last_plan()
+            print(f"[case] gptq op {bits} {dtn} {K}x{N} m={m} {plan['kernel']}", flush=True)
+            assert plan["kernel"].startswith(f"pk{bits}_" if copied else f"gptq{bits}_tile_"), plan
+            assert_close(y, ref[:m], f"m{m} {plan['kernel']}")
 
 
 @pytest.mark.parametrize("dtn", ["f16", "bf16"])
