@@ -1099,7 +1099,7 @@ int oxq_gguf_quant_matmul(oxq_ctx *ctx, void *stream, const oxq_tensor *x,
     // Prefill sizes without a cached copy: the matrix-core copy built in the ctx workspace (one pass over the
     // blocks: 10 us for 4096 x 4096 Q4_K), then its prefill kernel, which runs at 1.5 - 1.8 x the tile matmul on the
     // file layout - ahead from about a thousand rows.  Two launches.
-    if (!ctx->plan_only && p.act_dtype == OXQ_BF16 && p.M >= 1024 && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
+    if (p.act_dtype == OXQ_BF16 && p.M >= 1024 && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
         gguf_mfma_eligible(ctx, quant, p.K, p.N) && gguf_gemm_takes(ctx, quant, p.M, p.K, p.N, p.act_dtype, false) &&
         ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 1) == 0 &&
         ((gguf_mfma_bytes(quant, p.K, p.N) + 255) & ~(size_t)255) <= ctx->workspace_bytes) {
@@ -1126,7 +1126,7 @@ int oxq_gguf_quant_mul_mm(oxq_ctx *ctx, void *stream, const oxq_tensor *x,
     // Prefill sizes without a cached copy: the matrix-core copy built in the ctx workspace (one pass over the
     // blocks: 10 us for 4096 x 4096 Q4_K), then its prefill kernel, which runs at 1.5 - 1.8 x the tile matmul on the
     // file layout - ahead from about a thousand rows.  Two launches.
-    if (!ctx->plan_only && p.act_dtype == OXQ_BF16 && p.M >= 1024 && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
+    if (p.act_dtype == OXQ_BF16 && p.M >= 1024 && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
         gguf_mfma_eligible(ctx, quant, p.K, p.N) && gguf_gemm_takes(ctx, quant, p.M, p.K, p.N, p.act_dtype, false) &&
         ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 1) == 0 &&
         ((gguf_mfma_bytes(quant, p.K, p.N) + 255) & ~(size_t)255) <= ctx->workspace_bytes) {

@@ -697,7 +697,7 @@ bool awq4_mfma_ok(const Wna16Problem &p) {
 // PackedQuantLinear, which repacks once.
 static bool transient_repack_fits(const oxq_ctx *ctx, const Wna16Problem &p) {
     if ((((uintptr_t)p.x | (uintptr_t)p.y) & 15) || ((uintptr_t)p.bias & 7)) return false;
-    return p.M > 8 && pk4_eligible(p) && !ctx->plan_only && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
+    return p.M > 8 && pk4_eligible(p) && tune(ctx, OXQ_TUNE_TRANSIENT_REPACK, 1) &&
            !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0) &&
            ((pk4_weight_bytes(p.K, p.N, p.bits, pk4_sets(p.group_shift)) + 255) & ~(size_t)255) <= ctx->workspace_bytes;
 }

@@ -210,6 +210,12 @@ def test_maybe_mpp_declines_like_reference(lib, ctx):
     assert call(fake((64, 4096), F16, contiguous=False), fake((64, 14336), F16)) == 0
     assert taken.value == 0
     assert call(fake((64, 4096), F16), fake((64, 14336), F16)) == 0 and taken.value == 1
+    # the tile-major copy, built in the workspace, and the resident layers' kernel on it
+    p = plan(lib, ctx)
+    assert p.kernel.decode() == "pk4_mfma_f16_mt4" and p.grid[0] == 224 and p.split_k == 1 and p.launches == 2
+    assert lib.oxq_ctx_set_tuning(ctx, b"OXQ_TRANSIENT_REPACK", 0) == 0
+    assert call(fake((64, 4096), F16), fake((64, 14336), F16)) == 0 and taken.value == 1
+    assert lib.oxq_ctx_reset_tuning(ctx, b"OXQ_TRANSIENT_REPACK") == 0
     p = plan(lib, ctx)
     assert p.kernel.decode() == "awq4_mfma_pipe_f16_mt4" and p.grid[0] == 28 and p.grid[2] == 1
     assert p.launches == 2 and p.workspace_bytes == p.split_k * 64 * 14336 * 4

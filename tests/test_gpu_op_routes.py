@@ -90,3 +90,31 @@ def test_an_infinite_row_keeps_its_signs(dtn, K, N):
         print(f"[case] infinite row {dtn} {K}x{N} m={m} {ops.default_context().last_plan()['kernel']}", flush=True)
         np.testing.assert_array_equal(y[m - 1].float().cpu().numpy(), want)
         assert bool(torch.isfinite(y[:m - 1]).all())
+
+
+def test_a_plan_only_context_reports_what_runs():
+    """Calls that build a copy of their tensors and calls next to them."""
+    plans = ops.Context(plan_only=True)
+
+    def same(name, call, bits_out):
+        seen = []
+        for ctx in (plans, ops.default_context()):
+            call(ctx)
+            seen.append({k: v for k, v in ctx.last_plan().items()})
+        print(f"[case] plan only {name} {seen[1]['kernel']}", flush=True)
+        assert seen[0] == seen[1], name
+        assert seen[0]["kernel"].startswith(bits_out), seen[0]
+
+    K, N = 2048, 1024
+    for dtn, (dt, tdt) in DT.items():
+        args, _ = tensors(K, N, 128, 4, dt, tdt)
+        q, z, s = synth.gptq_checkpoint(K, N, 128, 8, seed=1)
+        gargs = (to_dev(q), to_dev(z), to_dev(s, tdt))
+        for m in (16, 17, 49, 64, 640):
+            x = torch.zeros(m, K, dtype=tdt, device="cuda")
+            same(f"awq {dtn} {m}", lambda c: ops.mpp_quant_matmul(x, *args, 4, ops.PACK_OUT, ctx=c), ("awq4", "pk4"))
+            same(f"gptq {dtn} {m}", lambda c: ops.mpp_quant_matmul(x, *gargs, 8, ops.PACK_IN, ctx=c), ("gptq8", "pk8"))
+    wd = to_dev(synth.gguf_weight(synth.GGUF_Q4_K, N, K, seed=2))
+    for m in (1023, 1024):
+        x = torch.zeros(m, K, dtype=torch.bfloat16, device="cuda")
+        same(f"gguf {m}", lambda c: ops.gguf_quant_mul_mm(x, wd, K, N, synth.GGUF_Q4_K, ctx=c), "gguf_q4k_")
