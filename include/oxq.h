@@ -482,9 +482,10 @@ int oxq_qlinear_new(oxq_ctx *ctx, int quant, const oxq_tensor *weight_bytes, int
  * above that, where enough workgroups fill the chip, in the copy's prefill kernel (the plain layer takes the same
  * kernel in the same form at the same sizes: the same bits), in one launch, or in two where K is split over
  * workgroups of 128 rows and the second adds the partial sums; otherwise in row tiles of 32 that each read the
- * weights again (with the unrounded weights that the plain layer's tile matmul rounds to bf16) - oxq_mlp_forward sends those row counts (more than OXQ_GGUF_FUSED_ACT_ROWS where the prefill kernel does not take
- * the call) through the plain layer's path and the activation by itself, so that a FeedForward over this layer
- * gives the plain layers' bits at every row count. */
+ * weights again (with the unrounded weights that the plain layer's tile matmul rounds to bf16) - oxq_mlp_forward
+ * sends those row counts (more than OXQ_GGUF_FUSED_ACT_ROWS where the prefill kernel does not take the call) through
+ * the plain layer's path and the activation by itself, so that a FeedForward over this layer gives the plain layers'
+ * bits at every row count. */
 #define OXQ_GGUF_FUSED_ACT_ROWS 32
 int oxq_qlinear_new_gate_up(oxq_ctx *ctx, int quant, const oxq_tensor *weight_bytes, int64_t in_features,
                             int64_t out_features, const oxq_tensor *bias_or_null, int act, int out_dtype,

@@ -465,7 +465,8 @@ __global__ __launch_bounds__(512) void f8_gemm_kernel(const uint16_t *__restrict
 
 // 128 rows, a wave has two strips: a decoded weight serves eight row tiles instead of four (two vector instructions an MFMA), at the
 // price of fragments of x that feed two MFMAs.  KS = 1: 256 columns, KS = 2: 128 with K over the two waves of a column group.
-// What bounds it: LDS, which a round asks for 1.1 of its 1.6 us (40 KB a wave and chunk at 128 bytes a clock; the MFMAs 0.85).
+// What bounds it: issue.  At 5632 x 5632 and 1024 rows the MFMAs take 55 % of the time, with 2.4 other vector instructions each, and reads
+// of LDS 38 %, at the 256 bytes a clock that a loop of 16-byte reads reaches (K over two waves, 640 rows: 43 % and 32 %).
 // us, best of the forms of 64 rows -> 128: 5632 x 5632 at 128 / 400 / 640 / 1024 rows 32 / 68 / 70 / 100 -> 24 / 48 / 50 / 75, 4096 x
 // 4096 at 640 / 1024 53 / 55 -> 38 / 42, 2048 x 5632 at 640 / 1024 34 / 46 -> 24 / 34.  Bits as f8_gemm_kernel's (KS = 1).
 template <int KS>

@@ -998,8 +998,9 @@ __global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) vo
 // launch adds them in slice order.  half: a fused gate|up layer without its activation - columns go back to the
 // file's order (ggm_src_row).
 // NS = 2, MT = 8: 128 rows, a wave has two strips.  What bounds the form above is the conversion's vector instructions, 5 - 7 an
-// MFMA at four row tiles a weight; here a weight serves eight, at the price of LDS, whose fragment then feeds two MFMAs instead of
-// four.  (Four strips do not fit: 128 accumulators beside two ring halves.)  KS = 1: 256 columns, 143 - 161 registers; KS = 2: 128
+// MFMA at four row tiles a weight; here a weight serves eight (Q4_K 4.1, Q6_K 4.8 an MFMA; the MFMAs take 45 and 37 % of the time),
+// at the price of LDS, whose fragment then feeds two MFMAs instead of four (reads, without conflicts: 22 and 19 %).  (Four strips do
+// not fit: 128 accumulators beside two ring halves.)  KS = 1: 256 columns, 143 - 161 registers; KS = 2: 128
 // columns, the two waves of a column group take every other chunk and finish four row tiles each - for launches that 256 columns
 // leave CUs idle in.  us, best of the forms of 64 rows -> 128: Q4_K 4096 x 4096 at 520 / 1024 / 2048 rows 55 / 56 / 91 -> 39 / 42 / 71,
 // 4096 x 14336 at 256 / 1024 / 2048 56 / 179 / 345 -> 41 / 136 / 262, 14336 x 4096 at 777 164 -> 122; Q8_0 4096 x 14336 at 2048
@@ -1752,7 +1753,8 @@ bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_
 // Adds the K slices of a fused gate|up layer and runs its activation: columns n and hc + n of a row (file order), summed and rounded
 // as splitk_reduce_kernel does it, then act(gate) * up as oxq_gated_activation.  What bounds it: the partials' bytes, as there.  A
 // thread has four outputs.  The fused call, us, whole sums in one launch (which are not the plain layer's bits) -> slices and this: Q4_K
-// 8192 x 4096 at 300 / 512 rows 49.1 / 49.6 -> 42.1 / 46.4, 6144 x 10752 at 74 38.4 -> 29.1, Q6_K 8192 x 4096 at 400 59.9 -> 50.2.  hc is a multiple of 32, and the 8 S M hc bytes of partials fit the workspace: the index fits 32 bits.
+// 8192 x 4096 at 300 / 512 rows 49.1 / 49.6 -> 42.1 / 46.4, 6144 x 10752 at 74 38.4 -> 29.1, Q6_K 8192 x 4096 at 400 59.9 -> 50.2.
+// hc is a multiple of 32, and the 8 S M hc bytes of partials fit the workspace: the index fits 32 bits.
 __global__ __launch_bounds__(256) void ggm_act_reduce_kernel(const float *__restrict__ part, const uint16_t *__restrict__ bias,
                                                              uint16_t *__restrict__ y, unsigned quads, int hc, size_t total, int S, int act) {
     typedef BF16Traits TT;

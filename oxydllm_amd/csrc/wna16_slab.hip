@@ -1,5 +1,6 @@
 // The checkpoint layouts (AWQ, quant_kernels.metal:3349-3499; GPTQ) at few rows of x on the matrix cores: up to 16, AWQ
-// 4-bit in f16 up to 8.
+// 4-bit in f16 up to 8 (from nine rows its tile kernel has the calls, though not by its time: 4096 x 4096 at 9 / 16 rows, tile kernel /
+// this one, 10.5 / 8.7, 12.7 / 9.9 us, 4096 x 14336 13.9 / 12.6, 15.3 / 15.1, 8192 x 1024 11.3 / 8.9, 12.0 / 9.7).
 //
 // An AWQ word holds 8 (8-bit: 4) columns of one row of K.  A lane takes 16 columns - two (four) neighbouring words - of
 // eight consecutive rows: nibble slot s of its words, row by row, is the B operand of one MFMA step for one column, and
