@@ -722,6 +722,19 @@ static int launch_transient_repack(oxq_ctx *ctx, hipStream_t s, const Wna16Probl
     return rc;
 }
 
+// AWQ 4-bit tensors in f16: from 49 rows (up to 48 the resident kernels fold sums, which make NaN of an infinite x), on layers of more
+// than 2^24 weights 64, of less than 2^21 640.  The copy leaves no workspace for slices of K, which the checkpoint-layout kernels
+// take: up to three row tiles of 64 a long K keeps those, half as long again with groups of 64 and 32, where they are slower.  Us,
+// checkpoint layout / repack and resident kernel: 4096 x 14336 at 32 / 64 / 640 rows 20 / 24, 28 / 27, 189 / 103, 4096 x 4096 at 20 / 32
+// 14 / 14, 21 / 14; 6912 x 5024 at 64 23 / 30, 12928 x 7320 at 64 / 200 34 / 55, 91 / 77, 12800 x 2488 at 128 29 / 39, groups of 64 8960 x
+// 9552 at 64 39 / 50.  On 150 layers that the lines were not drawn from 1213 calls of 49 - 639 rows come here, in 0.73 of the checkpoint
+// layout's time, 27 of them behind it by 3 % and more (14208 x 928 at 300 rows 30 / 39, 4480 x 13912 at 64 28 / 32).
+static bool awq_f16_repack_pays(const Wna16Problem &p) {
+    const int64_t size = p.K * p.N, row_tiles = ceil_div(p.M, (int64_t)64), most_k = 3072 + 1536 * row_tiles;
+    if (p.M < (size < (1 << 21) ? 640 : size <= (1 << 24) ? 49 : 64)) return false;
+    return row_tiles > 3 || p.K < (p.group_size >= 128 ? most_k : most_k + most_k / 2);
+}
+
 // GPTQ tensors that the tile kernel takes (workgroups of 64 rows x 64 columns): it is ahead while these are one round of CUs.  From two
 // rounds the copy is, where its prefill forms take the call (8-bit in f16: unless a last round of two or three is nearly full), in 4 bits
 // from six row tiles on (bf16 layers of 2^25 weights: four), in 8 bits from seven.  Below 3/4 of 2^24 weights, and at most everywhere,
@@ -740,16 +753,13 @@ static bool gptq_repack_pays(const oxq_ctx *ctx, const Wna16Problem &p) {
 
 int launch_wna16_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     // The resident layout's kernels run at two to six times the rate of the AWQ kernels on the checkpoint layout, which pays for the
-    // repack (9 us at 4096 x 14336, 4-bit) from few rows on: in bf16 behind the 16 rows of the slab kernel, in f16 from 49 rows (up to
-    // 48 the resident kernels fold sums, which make NaN of an infinite x), on layers of more than 2^24 weights 64, with few columns
-    // 128.  Us, checkpoint layout / repack and resident kernel: bf16 4096 x 14336 at 20 / 64 / 640 rows 46 / 23, 56 / 27, 656 / 110, 4096 x
-    // 4096 at 32 28 / 16, 1536 x 2048 at 20 16 / 10; f16 4096 x 14336 at 32 / 64 / 640 20 / 24, 28 / 27, 189 / 103, 4096 x 4096 at 20 / 32
-    // 14 / 14, 21 / 14, 11008 x 3584 at 90 / 200 29 / 34, 44 / 37.  Up to 16 rows in bf16: 4096 x 14336 at 9 rows, tile / slab kernel, 43 / 13.
+    // repack (9 us at 4096 x 14336, 4-bit) from few rows on: in bf16 behind the 16 rows of the slab kernel (4096 x 14336 at 9 rows, tile /
+    // slab kernel, 43 / 13), in f16 as awq_f16_repack_pays says.  Us, checkpoint layout / repack and resident kernel, bf16: 4096 x 14336 at
+    // 20 / 64 / 640 rows 46 / 23, 56 / 27, 656 / 110, 4096 x 4096 at 32 28 / 16, 1536 x 2048 at 20 16 / 10.
     const bool awq = awq4_mfma_ok(p), gptq = !awq && gptq_tile_ok(p) && tune(ctx, OXQ_TUNE_GPTQ_TILE, 1) != 2;
     if (awq && p.M <= 16 && wna16_slab_takes(ctx, p)) return launch_wna16_slab(ctx, s, p);
-    const int64_t size = p.K * p.N;
-    const int64_t awq_from = p.dtype != OXQ_F16 ? (size < (1 << 21) ? 80 : 17) : size < (1 << 21) ? 640 : size <= (1 << 24) ? 49 : p.K >= 2 * p.N ? 128 : 64;
-    if ((awq ? p.M >= awq_from : gptq && gptq_repack_pays(ctx, p)) && transient_repack_fits(ctx, p)) return launch_transient_repack(ctx, s, p);
+    const bool awq_pays = p.dtype == OXQ_F16 ? awq_f16_repack_pays(p) : p.M >= (p.K * p.N < (1 << 21) ? 80 : 17);
+    if ((awq ? awq_pays : gptq && gptq_repack_pays(ctx, p)) && transient_repack_fits(ctx, p)) return launch_transient_repack(ctx, s, p);
     if (awq4_mfma_ok(p) && !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0))
         return p.dtype == OXQ_F16 ? launch_awq4_mfma<F16Traits>(ctx, s, p)
                                   : launch_awq4_mfma<BF16Traits>(ctx, s, p);

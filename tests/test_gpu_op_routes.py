@@ -35,13 +35,15 @@ def test_one_row_of_ragged_columns(dtn, bits, K, N, g):
 
 @pytest.mark.parametrize("dtn", ["f16", "bf16"])
 @pytest.mark.parametrize("K,N,g,rows", [(1024, 2048, 128, {"f16": 49, "bf16": 17}), (1088, 2056, 64, {"f16": 49, "bf16": 17}),
-                                        (4096, 4104, 128, {"f16": 64, "bf16": 17}), (8224, 2048, 32, {"f16": 128, "bf16": 17})])
+                                        (4096, 4104, 128, {"f16": 64, "bf16": 17}), (8224, 2048, 32, {"f16": 65, "bf16": 17}),
+                                        (4608, 512, 128, {"f16": 65, "bf16": 17}), (6144, 1032, 128, {"f16": 129, "bf16": 17}),
+                                        (9280, 520, 64, {"f16": 129, "bf16": 17}), (7680, 520, 128, {"f16": 193, "bf16": 17})])
 def test_rows_at_the_lines_of_the_rule(dtn, K, N, g, rows):
     dt, tdt = DT[dtn]
     args, w = tensors(K, N, g, 4, dt, tdt)
-    x = np.random.default_rng(K).standard_normal((140, K)).astype(np.float32)
+    x = np.random.default_rng(K).standard_normal((200, K)).astype(np.float32)
     xd, wr = to_dev(x, tdt), oracle.round_through(w, dt)
-    for m in (9, 16, 17, rows[dtn] - 1, rows[dtn], 140):
+    for m in (9, 16, 17, rows[dtn] - 1, rows[dtn], 200):
         y = ops.mpp_quant_matmul(xd[:m], *args, 4, ops.PACK_OUT)
         plan = ops.default_context().last_plan()
         print(f"[case] awq op {dtn} {K}x{N} g={g} m={m} {plan['kernel']}", flush=True)
