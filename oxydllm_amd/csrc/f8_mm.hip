@@ -666,11 +666,14 @@ static bool f8_shape_ok(const F8Problem &p) {
 // 13.1 -> 9.8, 13.3 -> 10.1, 15.1 -> 11.4; 5632 x 5632 at 33 rows 15.7 -> 12.1; 1408 x 2048 at 96 rows 6.7 -> 4.9.
 //   64 rows x 128 columns, K over waves  rounds x (7.5 + 2.45 x rounds of four chunks); K slices add a second launch and
 //                                        the partials' traffic
-//   128 rows x 128 columns, K over waves rounds x (6.7 + 1.75 x rounds of two chunks); K slices likewise
+//   128 rows x 128 columns, K over waves 6.4 + rounds x (1.2 + 1.6 x rounds of two chunks) + 0.36 x those, of the CUs in use; K slices likewise
 //   64 rows x 512 columns                rounds x (7 + 2.1 x chunks)
 //   128 rows x 256 columns               rounds x (7.5 + 1.6 x chunks)
 // (The last four fitted again over 40 layers of 512..7168 x 512..7168 at 17..2048 rows, every form forced at each of 160 calls:
-// 0.9 % behind the fastest form together, 148 within 5 %, 157 within 12 %.)
+// 0.9 % behind the fastest form together, 148 within 5 %, 157 within 12 %.  That of 128 rows x 128 columns, fitted there without a term of
+// its own for slices, took 57 of 2592 calls of 520 other layers that a form without 128 rows ends 4 - 38 % earlier, all of long K and few columns
+// (7296 x 640 at 218 rows 18.9 / 13.6 us, 7936 x 1792 at 157 21.9 / 17.2); fitted on half of those layers, 5 of 2592, the most 9 %, and 1.7 %
+// behind the fastest form together.)
 //   the staged tiles of blockq_mm.hip    from 33 rows and up to K = 2048, where a workgroup of eight waves has too little K
 //                                        to share: several small workgroups a CU win at some shapes
 struct F8Form {
@@ -715,8 +718,8 @@ static F8Form f8_form(const oxq_ctx *ctx, const F8Problem &p) {
             if (fs > 0 && S != std::min<int64_t>(fs, most2)) continue;
             const int64_t rounds = ceil_div(ceil_div(chunks, S), (int64_t)2);
             if (ceil_div(chunks, 2 * rounds) != S || (S > 1 && (uint64_t)(S * p.M) * (uint64_t)p.N * 4 > ctx->workspace_bytes)) continue;
-            offer(10, std::ceil((double)(wgs128 * S) / cus) * (6.7 + (double)rounds * 1.75) + sum(S, 1.5, 6e6),
-                  {2, 1, (int)S, 2});
+            const double w = (double)(wgs128 * S) / cus;
+            offer(10, 6.4 + std::ceil(w) * (1.2 + (double)rounds * 1.6) + w * (double)rounds * 0.36 + sum(S, 1.3, 4.3e6), {2, 1, (int)S, 2});
         }
     }
     if (p.K <= 2048) offer(8, 4.8 + 0.38 * (double)chunks + mn * 1.0e-6 + mn * (double)p.K * 3.5e-9, {-1, 1, 1});
