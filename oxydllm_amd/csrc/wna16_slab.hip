@@ -353,8 +353,9 @@ bool wna16_slab_takes(const oxq_ctx *ctx, const Wna16Problem &p) {
         if (p.M == 1 && p.K % 128 == 0 && p.group_size >= 128) return false;
         return p.M >= 3 || p.K * p.N >= (1 << 23);
     }
-    // (one row that the dot-product kernel refuses, ragged columns: 4096 x 8200 bf16 4-bit 21.9 -> 13.2 us, 8-bit 30.4 -> 15.3)
-    if (p.M == 1) return p.group_size < 64 || !awq_fast_ok(p) || (p.bits == 4 && slab_tiles(p) <= cus);
+    // (one row that the dot-product kernel refuses, ragged columns: 4096 x 8200 bf16 4-bit 21.9 -> 13.2 us, 8-bit 30.4 -> 15.3; groups of 64
+    // and a short K stay with the generic kernel, 8-bit 960 x 4776 7.7 / 8.5, 320 x 6192 6.9 / 8.3, but 1088 x 3472 8.0 / 7.1)
+    if (p.M == 1) return p.group_size < 64 || (!awq_fast_ok(p) && (p.group_size >= 128 || p.K >= 1024)) || (p.bits == 4 && slab_tiles(p) <= cus);
     return p.bits == 8 || p.dtype != OXQ_F16 || p.group_size < 128 || 2 * slab_tiles(p) >= 64;
 }
 

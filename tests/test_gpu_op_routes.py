@@ -21,14 +21,15 @@ def tensors(K, N, g, bits, dt, tdt):
 
 @pytest.mark.parametrize("dtn", ["f16", "bf16"])
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("K,N,g", [(1024, 264, 128), (4096, 1096, 64), (2080, 520, 32), (1280, 8200, 128)])
+@pytest.mark.parametrize("K,N,g", [(1024, 264, 128), (4096, 1096, 64), (2080, 520, 32), (1280, 8200, 128), (960, 1096, 64), (1024, 1096, 64)])
 def test_one_row_of_ragged_columns(dtn, bits, K, N, g):
     """Weights stay unrounded: outputs are the 64-bit product rounded once, but for those next to a boundary."""
     dt, tdt = DT[dtn]
     args, w = tensors(K, N, g, bits, dt, tdt)
     x = np.random.default_rng(K).standard_normal((1, K)).astype(np.float32)
     y = (ops.w4a16_matmul if bits == 4 else ops.w8a16_matmul)(to_dev(x, tdt), *args)
-    assert "_slab" in ops.default_context().last_plan()["kernel"]
+    short = bits == 8 and g == 64 and K < 1024  # the generic kernel
+    assert ("_slab" in ops.default_context().last_plan()["kernel"]) != short
     ref = round_x(x, dt).astype(np.float64) @ w.astype(np.float64).T
     assert (y.cpu() == torch.from_numpy(ref).to(tdt)).double().mean().item() > 0.97
 
