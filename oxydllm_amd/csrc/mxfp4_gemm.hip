@@ -201,22 +201,22 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {  // one hard
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{lo, hi}, bf16x2_t));
 }
 
-// One tile: RT x 32 rows of x (pairs m0 .. m_end - 1 of one expert) by eight groups of 32 columns, a wave each, in
+// One tile: RT x 32 rows of x (pairs m0 .. m_end - 1 of one expert) by NW groups of 32 columns, a wave each, in
 // 32 x 32 x 16 MFMAs over units of 64 elements of K (two blocks).
-template <int RT>
+template <int RT, int NW>
 __device__ __forceinline__ void mxw_tile(unsigned char *lds, const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw,
                                          const unsigned char *__restrict__ ps, const uint16_t *__restrict__ bias,
                                          uint16_t *__restrict__ y, const int32_t *__restrict__ token_ids, int K, int N, int NG,
                                          uint32_t x_bytes, int swiglu, float limit, int e, int c0, int m0, int m_end) {
     constexpr int NS = MXW_STAGES, D = MXW_RING;
-    constexpr int XL = (RT + 1) / 2;              // loads of x a wave issues a unit, 8 rows each (past the tile: zeros)
-    constexpr int STAGE = XL * MXG_WAVES * 1024;  // bytes of x: a unit
+    constexpr int XL = (4 * RT + NW - 1) / NW;    // loads of x a wave issues a unit, 8 rows each (past the tile: zeros)
+    constexpr int STAGE = XL * NW * 1024;         // bytes of x: a unit
     constexpr int OOB = 0x7FFFFF00;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n32 = lane & 31, h = lane >> 5, ni = lane & 15;
-    const int j = c0 * MXG_WAVES + wave;          // the wave's 32 columns: tiles 2 j and 2 j + 1 of 16 weight rows
+    const int j = c0 * NW + wave;                 // the wave's 32 columns: tiles 2 j and 2 j + 1 of 16 weight rows
     const int ntiles = N >> 4, nb = K >> 5, NU = (nb + 1) >> 1;
     const int live_tiles = min(2, ntiles - 2 * j);  // wave-uniform; <= 0: a wave past the last tile
     const bool live = live_tiles > 0;
@@ -359,11 +359,11 @@ __device__ __forceinline__ void mxw_tile(unsigned char *lds, const uint16_t *__r
         }
 }
 
-__global__ __launch_bounds__(512, 4) void mxfp4_wide_kernel(const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw,
-                                                            const unsigned char *__restrict__ ps, const uint16_t *__restrict__ bias,
-                                                            uint16_t *__restrict__ y, const int32_t *__restrict__ offsets,
-                                                            const int32_t *__restrict__ token_ids, int K, int N, int NG, int E,
-                                                            int col_groups, int tiles_bound, uint32_t x_bytes, int swiglu, float limit) {
+template <int NW>
+__device__ __forceinline__ void mxw_workgroup(const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw, const unsigned char *__restrict__ ps,
+                                              const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, const int32_t *__restrict__ offsets,
+                                              const int32_t *__restrict__ token_ids, int K, int N, int NG, int E, int col_groups, int tiles_bound,
+                                              uint32_t x_bytes, int swiglu, float limit) {
     extern __shared__ __attribute__((aligned(16))) unsigned char mxg_lds[];
     const int id = ((int)blockIdx.z * (int)gridDim.y + (int)blockIdx.y) * (int)gridDim.x + (int)blockIdx.x;
     if (id >= tiles_bound * col_groups) return;
@@ -411,12 +411,34 @@ __global__ __launch_bounds__(512, 4) void mxfp4_wide_kernel(const uint16_t *__re
     const int u0 = t * small + min(t, more), rt = small + (t < more ? 1 : 0);
     const int m0 = pairs0 + 32 * u0, m_end = min(pairs1, m0 + 32 * rt);
     auto go = [&](auto rt_c) {
-        mxw_tile<decltype(rt_c)::value>(mxg_lds, x, pw, ps, bias, y, token_ids, K, N, NG, x_bytes, swiglu, limit, e, c, m0, m_end);
+        mxw_tile<decltype(rt_c)::value, NW>(mxg_lds, x, pw, ps, bias, y, token_ids, K, N, NG, x_bytes, swiglu, limit, e, c, m0, m_end);
     };
     if (rt == 4) go(std::integral_constant<int, 4>{});
     else if (rt == 3) go(std::integral_constant<int, 3>{});
     else if (rt == 2) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, 1>{});
+}
+
+__global__ __launch_bounds__(512, 4) void mxfp4_wide_kernel(const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw,
+                                                            const unsigned char *__restrict__ ps, const uint16_t *__restrict__ bias,
+                                                            uint16_t *__restrict__ y, const int32_t *__restrict__ offsets,
+                                                            const int32_t *__restrict__ token_ids, int K, int N, int NG, int E,
+                                                            int col_groups, int tiles_bound, uint32_t x_bytes, int swiglu, float limit) {
+    mxw_workgroup<MXG_WAVES>(x, pw, ps, bias, y, offsets, token_ids, K, N, NG, E, col_groups, tiles_bound, x_bytes, swiglu, limit);
+}
+
+// Twelve waves, one workgroup a CU: where its workgroups of 384 columns are at most one a CU and those of 256 are more.  Then some CUs
+// hold two of the latter and the others one, and the launch lasts as long as 512 columns; 27 % of the time of the 2880 x 2880 experts at
+// 515 tokens their CUs stood idle.  us, 256 columns a workgroup -> 384, pairs an expert 3 / 16 / 64: 32 experts of 2880 x 2880 (K x N)
+// 31.7 / 31.8 / 51.9 -> 26.3 / 26.0 / 44.8, of 2560 x 2752 25.0 / 26.9 / 45.3 -> 19.8 / 23.8 / 39.3, 64 of 3456 x 1088 31.7 / 32.1 / 55.8 ->
+// 25.6 / 26.1 / 46.0.  In two rounds it is behind (5760 columns 58.3 / 87.6 -> 59.5 / 91.3 at 16 / 64 pairs): nothing covers its prologue.
+constexpr int MXG_WAVES12 = 12;
+__global__ __launch_bounds__(768, 3) void mxfp4_wide12_kernel(const uint16_t *__restrict__ x, const unsigned char *__restrict__ pw,
+                                                              const unsigned char *__restrict__ ps, const uint16_t *__restrict__ bias,
+                                                              uint16_t *__restrict__ y, const int32_t *__restrict__ offsets,
+                                                              const int32_t *__restrict__ token_ids, int K, int N, int NG, int E,
+                                                              int col_groups, int tiles_bound, uint32_t x_bytes, int swiglu, float limit) {
+    mxw_workgroup<MXG_WAVES12>(x, pw, ps, bias, y, offsets, token_ids, K, N, NG, E, col_groups, tiles_bound, x_bytes, swiglu, limit);
 }
 
 // Takes the grouped problem from three pairs an expert on average (below, the decode kernel's passes of four tokens
@@ -433,14 +455,16 @@ int mxfp4_gemm_form(const oxq_ctx *ctx, int64_t n_pairs, int64_t E, int64_t K, i
     return avg <= 12 ? 16 : avg < 96 ? 32 : avg < 200 ? 64 : 128;
 }
 
+template <int NW>
 static int mxfp4_wide_go(hipStream_t s, dim3 grid, const Mxfp4Problem &p, int NG, uint32_t x_bytes) {
-    static LdsGrant grant;
-    const size_t lds = (size_t)MXW_STAGES * MXW_ROWS * 128;
-    OXQ_HIP_CHECK(grant.ensure((const void *)mxfp4_wide_kernel, lds));
+    static LdsGrant grant;  // one per instantiation
+    constexpr auto kernel = NW == MXG_WAVES12 ? mxfp4_wide12_kernel : mxfp4_wide_kernel;
+    const size_t lds = (size_t)MXW_STAGES * ((MXW_ROWS / 8 + NW - 1) / NW) * NW * 1024;
+    OXQ_HIP_CHECK(grant.ensure((const void *)kernel, lds));
     const int64_t bound = p.n_pairs / MXW_ROWS + p.n_experts;
-    hipLaunchKernelGGL(mxfp4_wide_kernel, grid, dim3(512), lds, s, (const uint16_t *)p.x, (const unsigned char *)p.blocks,
+    hipLaunchKernelGGL(kernel, grid, dim3(NW * 64), lds, s, (const uint16_t *)p.x, (const unsigned char *)p.blocks,
                        (const unsigned char *)p.scales, (const uint16_t *)p.bias, (uint16_t *)p.y, p.expert_offsets, p.token_ids,
-                       (int)p.K, (int)p.N, NG, (int)p.n_experts, (int)ceil_div(p.N, 32 * MXG_WAVES), (int)bound, x_bytes, p.swiglu, p.swiglu_limit);
+                       (int)p.K, (int)p.N, NG, (int)p.n_experts, (int)ceil_div(p.N, 32 * NW), (int)bound, x_bytes, p.swiglu, p.swiglu_limit);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
@@ -468,18 +492,23 @@ int launch_mxfp4_res_gemm(oxq_ctx *ctx, hipStream_t s, const Mxfp4Problem &p) {
     // the faster ones where K is long and the wide kernel's workgroups of 256 columns do not fill two places a compute unit (32
     // experts x 2880 x 2880 at 24 / 48 / 96 tokens 32.2 / 34.1 / 34.6 against 34.6 / 36.4 / 36.7 us; 5760 x 2880, which fills
     // them, 60.5 / 63.6 / 63.6 against 57.6 / 60.6 / 61.6; 64 experts x 1024 x 1024 at 64 tokens 16.8 against 9.4).
-    const int64_t places = 2 * (ctx->num_cus > 0 ? ctx->num_cus : 256);
-    const bool narrow = rows == 16 && p.K >= 2048 && ceil_div(p.N, 32 * MXG_WAVES) * p.n_experts < places;
+    const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    // (up to 96 pairs an expert, few of which then hold more than one tile of rows)
+    const bool wide12 = !tune_given(ctx, OXQ_TUNE_MXFP4_GEMM_ROWS) && p.n_pairs <= 96 * p.n_experts &&
+                        ceil_div(p.N, 32 * MXG_WAVES12) * p.n_experts <= cus && ceil_div(p.N, 32 * MXG_WAVES) * p.n_experts > cus;
+    const bool narrow = !wide12 && rows == 16 && p.K >= 2048 && ceil_div(p.N, 32 * MXG_WAVES) * p.n_experts < 2 * cus;
     dim3 grid((unsigned)ceil_div(p.N / 16, (int64_t)4 * MXG_WAVES), (unsigned)ytiles, narrow ? 1 : 2);
+    if (wide12) grid = dim3((unsigned)ceil_div(p.N, 32 * MXG_WAVES12), (unsigned)ytiles);
     char name[64];
-    snprintf(name, sizeof name, "mxfp4_experts_gemm_bf16_r%dx8%s", rows, p.swiglu ? "_swiglu" : "");
-    set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
+    snprintf(name, sizeof name, "mxfp4_experts_gemm_bf16_r%dx%d%s", rows, wide12 ? MXG_WAVES12 : MXG_WAVES, p.swiglu ? "_swiglu" : "");
+    set_plan(ctx, name, grid, dim3(wide12 ? 64 * MXG_WAVES12 : 512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     const uint64_t x_bytes = (uint64_t)p.M * (uint64_t)p.K * 2u;
     if (x_bytes >= (1ull << 31)) return fail(OXQ_ERR_UNSUPPORTED, "mxfp4 experts prefill: x of %llu bytes exceeds 2 GiB", (unsigned long long)x_bytes);
     if ((uintptr_t)p.x & 15) return fail(OXQ_ERR_UNSUPPORTED, "mxfp4 experts prefill: x must be 16-byte aligned");
     if ((uintptr_t)p.y & 3) return fail(OXQ_ERR_UNSUPPORTED, "mxfp4 experts prefill: out must be 4-byte aligned");
-    return narrow ? mxfp4_gemm_go(s, grid, p, NC, NG, (uint32_t)x_bytes) : mxfp4_wide_go(s, grid, p, NG, (uint32_t)x_bytes);
+    if (wide12) return mxfp4_wide_go<MXG_WAVES12>(s, grid, p, NG, (uint32_t)x_bytes);
+    return narrow ? mxfp4_gemm_go(s, grid, p, NC, NG, (uint32_t)x_bytes) : mxfp4_wide_go<MXG_WAVES>(s, grid, p, NG, (uint32_t)x_bytes);
 }
 
 }  // namespace oxq
