@@ -15,8 +15,8 @@
 // cycles of the address unit for 1 KB, and that bound the first version (2.45 us for 64 x 512 x 128 a CU).  Loads now
 // take whole 128-byte (64-byte) runs of a row and turn to operand order through the wave's own LDS: 2.1 us.
 // Measured, us, before (GEMV / staged tiles) -> now: 5632 x 5632 at 1, 33, 96, 256, 1024 rows 11.3 -> 8.3, 22.9 -> 15.9,
-// 31.5 -> 18.4, 52 -> 34, 144 -> 75; 2048 x 5632 at 3, 33, 96 rows 8.5 -> 4.8, 12.5 -> 9.0, 17.0 -> 10.2; 512 x 768 at
-// 33 rows 6.6 -> 3.3.
+// 31.5 -> 18.4, 52 -> 34, 144 -> 75; 2048 x 5632 at 3, 33, 96 rows 8.5 -> 4.8, 12.5 -> 7.0, 17.0 -> 10.0; 512 x 768 at
+// 33 rows 6.6 -> 3.0.
 // Needs block_r a multiple of 16 (a strip has one scale a chunk), block_c 128 times a power of two; other grids keep
 // blockq_mm.hip.
 #include "oxq_device.hpp"
@@ -43,17 +43,27 @@ __device__ __forceinline__ void f8_operand(uint32_t w0, uint32_t w1, float s, ui
     }
 }
 
+template <int N, typename F> __device__ __forceinline__ void each(F f) {  // f(0) .. f(N - 1), constants
+    if constexpr (N > 1) each<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+}
+
 // XQ: loads of x a chunk (four rows each).  RD chunks in flight a wave: what hides the cache's latency; two or three are
 // what the registers hold (48 rows: 256 registers, one chunk of x; the LDS slots fill the CU's 160 KB).
-template <int MT, int NS, int NW, int XQ>
+// NL > 0: no wave has more than NL chunks and none fewer than NL - 1, all of them requested at once; 0: a loop.  A load that brings
+// nothing (past a wave's last chunk) takes its turn in the address unit as any other, and a kernel's instructions come from memory
+// anew at each launch: with a body for each number of chunks neither a load nor a jump is left over.  us, one loop with such loads for
+// all -> now: 5632 x 2816 (N x K) at 1 / 8 / 16 rows 5.8 / 6.6 / 7.9 -> 5.5 / 6.0 / 6.8, 5632 x 2048 at 24 / 48 / 96 / 144 6.8 / 7.8 / 10.6 / 16.6 ->
+// 6.1 / 7.2 / 10.0 / 15.5, 768 x 512 at 33 3.3 -> 3.0; with bodies for all of them in one kernel 1 and 3 rows were 2 - 6 % behind.
+template <int MT, int NS, int NW, int XQ, int NL>
 __global__ __launch_bounds__(NW * 64) void f8_tile_kernel(const uint16_t *__restrict__ x, const uint8_t *__restrict__ w,
                                                           const float *__restrict__ scales, uint16_t *__restrict__ y,
                                                           int M, int K, int N, int block_r, int cshift, int s_cols, int s_rows) {
     typedef BF16Traits TT;
     typedef MfmaOps<TT> Ops;
     constexpr int ROWS = 16 * MT, AQ = XQ, SLOT = ROWS * 256, WSLOT = NS * 2048, OOB = 0x7FFFFF00;
-    constexpr int RD = NS > 1 ? 2 : 3;       // chunks in flight a wave
-    constexpr int XD = MT == 3 ? 1 : RD;     // and of x, which comes from L2 (48 rows: the registers allow one)
+    constexpr int RD = NL > 0 ? NL : NS > 1 ? 2 : 3;  // chunks in flight a wave
+    constexpr int XD = MT == 3 ? 1 : RD;              // and of x, which comes from L2 (48 rows: the registers allow one)
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
 
     const int lane = threadIdx.x & 63;
@@ -125,11 +135,6 @@ __global__ __launch_bounds__(NW * 64) void f8_tile_kernel(const uint16_t *__rest
         }
         __builtin_amdgcn_sched_barrier(0);  // chunks are requested in the order they are used
     };
-#pragma unroll
-    for (int d = 0; d < RD; ++d) {
-        if (d < XD) request_x(d, ar[d]);
-        request(d, wr[d], sr[d]);
-    }
 
     float4_t acc[MT][NS];
 #pragma unroll
@@ -137,15 +142,18 @@ __global__ __launch_bounds__(NW * 64) void f8_tile_kernel(const uint16_t *__rest
 #pragma unroll
         for (int f = 0; f < NS; ++f) acc[mt][f] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    auto chunk = [&](int i, auto cur_c, bool more) {
+    // placed: x lies in the slot.  more: request chunk i + RD; next: x of chunk i + 1
+    auto chunk = [&](int i, auto cur_c, bool placed, auto more_c, auto next_c) {
         constexpr int CUR = decltype(cur_c)::value;
+        if (!placed) {
 #pragma unroll
-        for (int q = 0; q < AQ; ++q) *(u32x4_t *)(slot + q * 1024 + a_wr[q & 3]) = ar[CUR % XD][q];
+            for (int q = 0; q < AQ; ++q) *(u32x4_t *)(slot + q * 1024 + a_wr[q & 3]) = ar[CUR % XD][q];
+        }
 #pragma unroll
         for (int f = 0; f < NS; ++f)
 #pragma unroll
             for (int h = 0; h < 2; ++h) *(u32x4_t *)(wslot + f * 2048 + h * 1024 + w_wr) = wr[CUR][f][h];
-        if constexpr (XD == 1) {
+        if constexpr (XD == 1 && next_c.value) {
             request_x(i + 1, ar[0]);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -171,29 +179,57 @@ __global__ __launch_bounds__(NW * 64) void f8_tile_kernel(const uint16_t *__rest
             }
             if constexpr (MT == 3) __builtin_amdgcn_sched_barrier(0);  // no operands of the next step early: no registers for them
         }
-        if (more) {
+        if constexpr (more_c.value) {
             if constexpr (XD > 1) request_x(i + RD, ar[CUR]);
             request(i + RD, wr[CUR], sr[CUR]);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    {
-        int i = 0;
-        if constexpr (RD == 2) {
-            for (; i + 1 < nloc; i += 2) {
-                chunk(i, std::integral_constant<int, 0>{}, true);
-                chunk(i + 1, std::integral_constant<int, 1>{}, true);
+    if constexpr (NL > 0) {
+        // 48 rows have registers for one chunk of x: the first goes straight into its slot, so that the second is under way beside it
+        // (us: 5632 x 2048 at 33 / 48 rows 7.2 / 7.5 -> 7.0 / 7.2; 48 rows x 64 columns of two chunks, 96 rows, 10.0 -> 10.15, stay).
+        constexpr bool DMA = MT == 3 && (NS == 2 || NL == 1);
+        if constexpr (DMA) {
+            static_assert(NL <= 2 && AQ == 4 * MT, "one chunk in the slot, one in registers; whole slots");
+            if (nloc > 0) {
+#pragma unroll
+                for (int q = 0; q < AQ; ++q) {  // lane 16 kb + ni fills piece ni of row r: that of the columns ni ^ (r % 16)
+                    const int r = 4 * q + kb;
+                    pk4g_load_lds16(rs_x, slot + q * 1024, r < xrows ? r * K * 2 + ((ni ^ (r & 15)) << 4) : OOB, cc0 * 256);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (i < nloc) chunk(i, std::integral_constant<int, 0>{}, false);
-        } else {
-            for (; i + 2 < nloc; i += 3) {
-                chunk(i, std::integral_constant<int, 0>{}, true);
-                chunk(i + 1, std::integral_constant<int, 1>{}, true);
-                chunk(i + 2, std::integral_constant<int, 2>{}, true);
-            }
-            if (i < nloc) chunk(i, std::integral_constant<int, 0>{}, false);
-            if (i + 1 < nloc) chunk(i + 1, std::integral_constant<int, 1>{}, false);
         }
+        each<NL>([&](auto s_c) {
+            constexpr int S = decltype(s_c)::value;
+            const int i = nloc - NL + S;
+            if (S == 0 && i < 0) return;
+            if (XD > 1 || (i > 0) == DMA) request_x(i, ar[S % XD]);
+            request(i, wr[S], sr[S]);
+        });
+        each<NL>([&](auto s_c) {
+            constexpr int S = decltype(s_c)::value;
+            const int i = nloc - NL + S;
+            if (S == 0 && i < 0) return;
+            if constexpr (DMA) {
+                pk4g_wait_vmcnt<(NL - 1 - S) * (AQ + 3 * NS)>();  // the first chunk is here, the second under way
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            chunk(i, s_c, DMA && i == 0, std::false_type{}, std::integral_constant<bool, (!DMA && S + 1 < NL)>{});
+        });
+    } else {
+#pragma unroll
+        for (int d = 0; d < RD; ++d) {
+            if (d < XD) request_x(d, ar[d]);
+            request(d, wr[d], sr[d]);
+        }
+        int i = 0;
+        for (; i + RD < nloc; i += RD)
+            each<RD>([&](auto s_c) { chunk(i + s_c.value, s_c, false, std::true_type{}, std::true_type{}); });
+        each<RD>([&](auto s_c) {
+            constexpr int S = decltype(s_c)::value;
+            if (i + S < nloc) chunk(i + S, s_c, false, std::false_type{}, std::integral_constant<bool, (S + 1 < RD)>{});
+        });
     }
     pk4n_epilogue<TT, MT, NS, NW, true>(acc, nullptr, y, nullptr, M, N, j, m0, wave, lane);
 }
@@ -728,21 +764,25 @@ static F8Form f8_form(const oxq_ctx *ctx, const F8Problem &p) {
 
 bool f8_direct_takes(const oxq_ctx *ctx, const F8Problem &p) { return f8_shape_ok(p) && f8_form(ctx, p).kind >= 0; }
 
-template <int MT, int NS, int XQ>
-static int f8_tile_go(hipStream_t s, dim3 grid, const F8Problem &p) {
+template <int MT, int NS, int XQ, int NL>
+static int f8_tile_launch(hipStream_t s, dim3 grid, const F8Problem &p) {
     static LdsGrant grant;
+    constexpr auto kernel = f8_tile_kernel<MT, NS, 8, XQ, NL>;
     const size_t lds = (size_t)8 * (MT * 4096 + NS * 2048);
-    OXQ_HIP_CHECK(grant.ensure((const void *)f8_tile_kernel<MT, NS, 8, XQ>, lds));
-    hipLaunchKernelGGL((f8_tile_kernel<MT, NS, 8, XQ>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w, p.scales, (uint16_t *)p.y,
+    OXQ_HIP_CHECK(grant.ensure((const void *)kernel, lds));
+    hipLaunchKernelGGL(kernel, grid, dim3(512), lds, s, (const uint16_t *)p.x, p.w, p.scales, (uint16_t *)p.y,
                        (int)p.M, (int)p.K, (int)p.N, (int)p.block_r, __builtin_ctzll((unsigned long long)p.block_c) - 7, (int)p.s_cols, (int)f8_s_rows(p));
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
-template <int NS>
-static int f8_tile_rows(hipStream_t s, dim3 grid, const F8Problem &p) {
-    if (p.M > 16) return f8_tile_go<2, NS, 8>(s, grid, p);
-    if (p.M > 8) return f8_tile_go<1, NS, 4>(s, grid, p);
-    return p.M > 4 ? f8_tile_go<1, NS, 2>(s, grid, p) : f8_tile_go<1, NS, 1>(s, grid, p);
+template <int MT, int NS, int XQ>
+static int f8_tile_go(hipStream_t s, dim3 grid, const F8Problem &p) {
+    const int64_t most = ceil_div(p.K / 128, (int64_t)8);  // chunks a wave
+    if (most <= 1) return f8_tile_launch<MT, NS, XQ, 1>(s, grid, p);
+    if (most == 2) return f8_tile_launch<MT, NS, XQ, 2>(s, grid, p);
+    if constexpr (NS == 1)
+        if (most == 3) return f8_tile_launch<MT, NS, XQ, 3>(s, grid, p);
+    return f8_tile_launch<MT, NS, XQ, 0>(s, grid, p);
 }
 template <int KS>
 static int f8_gemm_go(hipStream_t s, dim3 grid, const F8Problem &p, float *part, int NG, int RT, int cslice) {
@@ -779,8 +819,10 @@ int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
         set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
         if (ctx->plan_only) return OXQ_OK;
         if (form.ns == 2) return mt == 3 ? f8_tile_go<3, 2, 12>(s, grid, p) : f8_tile_go<2, 2, 8>(s, grid, p);
-        if (mt == 3) return f8_tile_go<3, 4, 12>(s, grid, p);
-        return form.ns == 4 ? f8_tile_rows<4>(s, grid, p) : f8_tile_rows<1>(s, grid, p);
+        if (form.ns == 4) return mt == 3 ? f8_tile_go<3, 4, 12>(s, grid, p) : f8_tile_go<2, 4, 8>(s, grid, p);
+        if (p.M > 16) return f8_tile_go<2, 1, 8>(s, grid, p);
+        if (p.M > 8) return f8_tile_go<1, 1, 4>(s, grid, p);
+        return p.M > 4 ? f8_tile_go<1, 1, 2>(s, grid, p) : f8_tile_go<1, 1, 1>(s, grid, p);
     }
     const bool tall = form.kind == 2;  // 128 rows, 32 columns a wave
     const int ks = tall ? form.mt : form.kind, spw = 8 / ks, rows = tall ? 128 : 64;
