@@ -423,7 +423,7 @@ static int launch_mm_src(oxq_ctx *ctx, hipStream_t s, MmArgs &a, const char *nam
     dim3 grid((unsigned)ceil_div(a.N, MM_BN), (unsigned)ytiles, (unsigned)pl.ks);
     char name[64];
     hilo = hilo && mt == 1 && SRC::HAS_RESIDUE;
-    snprintf(name, sizeof name, "%s_mul_mm_bf16_mt%d%s", name_prefix, mt, hilo ? "_f32w" : "");
+    plan_name(name, sizeof name, "%s_mul_mm_bf16_mt%d%s", name_prefix, mt, hilo ? "_f32w" : "");
     set_plan(ctx, name, grid, dim3(256), pl.ks, 1, pl.ks > 1 ? (size_t)pl.ks * a.M * a.N * 4 : 0);
     if (ctx->plan_only) {
         if (pl.ks > 1) add_launch(ctx);

@@ -128,7 +128,7 @@ int launch_calib_upfront(oxq_ctx *ctx, hipStream_t s, const uint8_t *src, uint64
     const int nl = (int)(span / ((uint64_t)waves * 1024));
     dim3 grid((unsigned)workgroups), block((unsigned)waves * 64);
     char name[48];
-    snprintf(name, sizeof name, "calib_upfront_%dw_%dl%s", waves, nl, nontemporal ? "_nt" : "");
+    plan_name(name, sizeof name, "calib_upfront_%dw_%dl%s", waves, nl, nontemporal ? "_nt" : "");
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
 #define OXQ_UF(NLv)                                                                                              \
@@ -204,7 +204,7 @@ int launch_calib_two_streams(oxq_ctx *ctx, hipStream_t s, const uint8_t *w, uint
     const int nl = (int)(span / 8192);
     dim3 grid((unsigned)workgroups), block(768);
     char name[48];
-    snprintf(name, sizeof name, "calib_two_streams_%d", which);
+    plan_name(name, sizeof name, "calib_two_streams_%d", which);
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     const size_t lds = 4 * 16384;

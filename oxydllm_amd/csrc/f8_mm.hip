@@ -815,7 +815,7 @@ int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
         const int mt = form.mt ? form.mt : p.M > 16 ? 2 : 1;
         dim3 grid((unsigned)ceil_div(p.N, (int64_t)16 * form.ns), 1, (unsigned)ceil_div(p.M, (int64_t)16 * mt));
         if (grid.z > 65535) return fail(OXQ_ERR_UNSUPPORTED, "f8 matmul: m = %lld exceeds the grid", (long long)p.M);
-        snprintf(name, sizeof name, "f8_mul_mm_bf16_mt%d%s", mt, form.ns == 4 ? "_n64" : form.ns == 2 ? "_n32" : "");
+        plan_name(name, sizeof name, "f8_mul_mm_bf16_mt%d%s", mt, form.ns == 4 ? "_n64" : form.ns == 2 ? "_n32" : "");
         set_plan(ctx, name, grid, dim3(512), 1, 1, 0);
         if (ctx->plan_only) return OXQ_OK;
         if (form.ns == 2) return mt == 3 ? f8_tile_go<3, 2, 12>(s, grid, p) : f8_tile_go<2, 2, 8>(s, grid, p);
@@ -831,7 +831,7 @@ int launch_f8_direct(oxq_ctx *ctx, hipStream_t s, const F8Problem &p) {
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "f8 matmul: m = %lld exceeds the grid", (long long)p.M);
     const int cslice = form.slices > 1 ? (int)(ceil_div(ceil_div(chunks, (int64_t)form.slices), (int64_t)ks) * ks) : (int)chunks;
     dim3 grid((unsigned)wgs, (unsigned)form.slices);
-    snprintf(name, sizeof name, "f8_mul_mm_bf16_r%dx%d%s", rows, spw, ks == 4 ? "k4" : ks == 2 ? "k2" : "");
+    plan_name(name, sizeof name, "f8_mul_mm_bf16_r%dx%d%s", rows, spw, ks == 4 ? "k4" : ks == 2 ? "k2" : "");
     set_plan(ctx, name, grid, dim3(512), form.slices, 1, form.slices > 1 ? (size_t)form.slices * p.M * p.N * 4 : 0);
     if (ctx->plan_only) {
         if (form.slices > 1) add_launch(ctx);

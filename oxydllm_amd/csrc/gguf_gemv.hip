@@ -469,7 +469,7 @@ int launch_gguf_gemv(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     const int pass = use_lds ? mb : 8;  // rows of x a launch
     const uint32_t chunks = (uint32_t)ceil_div(p.M, pass);
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_gemv_%s%s", fmt_name(p.quant), bf ? "bf16" : "f32", use_lds ? "_lds" : "");
+    plan_name(name, sizeof name, "gguf_%s_gemv_%s%s", fmt_name(p.quant), bf ? "bf16" : "f32", use_lds ? "_lds" : "");
     dim3 grid((unsigned)(use_lds ? ceil_div(p.N, rpwg) : ceil_div(p.N, 4))), block(use_lds && rpwg >= 16 ? 1024 : use_lds && rpwg >= 8 ? 512 : 256);
     set_plan(ctx, name, grid, block, 1, chunks, 0);
     if (ctx->plan_only) return OXQ_OK;
@@ -508,7 +508,7 @@ int launch_gguf_dequant(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p, float
     const size_t units = (size_t)N * (K >> 5);
     dim3 grid((unsigned)ceil_div((int64_t)units, 256)), block(256);
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_dequant", fmt_name(p.quant));
+    plan_name(name, sizeof name, "gguf_%s_dequant", fmt_name(p.quant));
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
 #define OXQ_DQ(F) \

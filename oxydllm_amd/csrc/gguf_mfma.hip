@@ -1424,7 +1424,7 @@ int launch_gguf_mfma_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_
     const size_t threads = (size_t)ceil_div(N, 16) * (K / 128) * 64;
     dim3 grid((unsigned)ceil_div((int64_t)threads, 256)), block(256);
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_mfma_repack", ggm_name(quant));
+    plan_name(name, sizeof name, "gguf_%s_mfma_repack", ggm_name(quant));
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     switch (quant) {
@@ -1449,7 +1449,7 @@ int launch_gguf_mfma_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void 
     const size_t threads = (size_t)ceil_div(N, 16) * (K / 128) * 64;
     dim3 grid((unsigned)ceil_div((int64_t)threads, 256)), block(256);
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_mfma_dequant", ggm_name(quant));
+    plan_name(name, sizeof name, "gguf_%s_mfma_dequant", ggm_name(quant));
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     switch (quant) {
@@ -1582,7 +1582,7 @@ int launch_gguf_mfma(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p) {
     const int nw = (chunks < 16 || chunks >= 64 || mt == 2 || ns == 4 || f32 || !one_round || tune(ctx, OXQ_TUNE_GGR_WAVES, 16) == 8) ? 8 : 16;
     dim3 grid((unsigned)ceil_div(p.N, (int64_t)16 * ns), 1, (unsigned)ceil_div(p.M, (int64_t)tile * mt));
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_mfma_%s_mt%d%s%s", ggm_name(p.quant), f32 ? "f32" : "bf16", mt, ns == 4 ? "_n64" : "", p.act ? "_act" : "");
+    plan_name(name, sizeof name, "gguf_%s_mfma_%s_mt%d%s%s", ggm_name(p.quant), f32 ? "f32" : "bf16", mt, ns == 4 ? "_n64" : "", p.act ? "_act" : "");
     set_plan(ctx, name, grid, dim3(nw * 64), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if (!f32 && p.act_dtype != OXQ_BF16) return fail(OXQ_ERR_UNSUPPORTED, "gguf matrix-core matmul: activations must be BF16 or F32");
@@ -1833,7 +1833,7 @@ int launch_gguf_gemm(oxq_ctx *ctx, hipStream_t s, const GgufProblem &problem, bo
     // rows x column groups of the workgroup, and the waves that share K inside it
     char name[64], slices[16] = "";
     if (form.slices > 1) snprintf(slices, sizeof slices, "_s%d", form.slices);
-    snprintf(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%d%s%s%s", ggm_name(p.quant), rows, spw, ks == 4 ? "k4" : ks == 2 ? "k2" : "", slices,
+    plan_name(name, sizeof name, "gguf_%s_gemm_bf16_r%dx%d%s%s%s", ggm_name(p.quant), rows, spw, ks == 4 ? "k4" : ks == 2 ? "k2" : "", slices,
              problem.act == 1 ? "_silu" : problem.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), form.slices, 1, form.slices > 1 ? (size_t)form.slices * p.M * p.N * 4 : 0);
     if (ctx->plan_only) {

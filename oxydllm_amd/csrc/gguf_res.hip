@@ -720,7 +720,7 @@ int launch_gguf_res_repack(oxq_ctx *ctx, hipStream_t s, int quant, const uint8_t
     const size_t threads = (size_t)(N / 16) * (K / 128) * 64;
     dim3 grid((unsigned)ceil_div((int64_t)threads, 256)), block(256);
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_repack", ggr_name(quant));
+    plan_name(name, sizeof name, "gguf_%s_repack", ggr_name(quant));
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
 #define OXQ_GR(F) \
@@ -747,7 +747,7 @@ int launch_gguf_res_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void *
     const size_t threads = (size_t)(N / 16) * (K / 128) * 64;
     dim3 grid((unsigned)ceil_div((int64_t)threads, 256)), block(256);
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_res_dequant", ggr_name(quant));
+    plan_name(name, sizeof name, "gguf_%s_res_dequant", ggr_name(quant));
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
 #define OXQ_GR(F) \
@@ -796,7 +796,7 @@ int launch_gguf_res_gemv(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p0) {
     const int64_t cap = tune(ctx, OXQ_TUNE_GGR_GRID, nw == 8 ? 512 : 256);
     dim3 grid((unsigned)std::min<int64_t>(p0.N / 16, cap > 0 ? cap : p0.N / 16));
     char name[64];
-    snprintf(name, sizeof name, "gguf_%s_res_gemv_%s_m%d", ggr_name(p0.quant), p0.act_dtype == OXQ_BF16 ? "bf16" : "f32", mb);
+    plan_name(name, sizeof name, "gguf_%s_res_gemv_%s_m%d", ggr_name(p0.quant), p0.act_dtype == OXQ_BF16 ? "bf16" : "f32", mb);
     set_plan(ctx, name, grid, dim3(nw * 64), 1, (uint32_t)ceil_div(p0.M, 4), 0);
     if (ctx->plan_only) return OXQ_OK;
     if (!gguf_res_takes(p0.K, p0.M, p0.act_dtype)) return fail(OXQ_ERR_UNSUPPORTED, "gguf resident gemv: m = %lld", (long long)p0.M);

@@ -373,7 +373,7 @@ int launch_gptq_tile(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     dim3 grid((unsigned)(p.N / 64), (unsigned)ceil_div(p.M, 16 * mt), (unsigned)ks);
     const size_t ws_bytes = ks > 1 ? (size_t)ks * p.M * p.N * 4 : 0;
     char name[64];
-    snprintf(name, sizeof name, "gptq%d_tile_%s_mt%d", p.bits, p.dtype == OXQ_F16 ? "f16" : "bf16", mt);
+    plan_name(name, sizeof name, "gptq%d_tile_%s_mt%d", p.bits, p.dtype == OXQ_F16 ? "f16" : "bf16", mt);
     set_plan(ctx, name, grid, dim3(512), ks, 1, ws_bytes);
     if (ctx->plan_only) {
         if (ks > 1) add_launch(ctx);

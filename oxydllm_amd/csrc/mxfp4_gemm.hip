@@ -500,7 +500,7 @@ int launch_mxfp4_res_gemm(oxq_ctx *ctx, hipStream_t s, const Mxfp4Problem &p) {
     dim3 grid((unsigned)ceil_div(p.N / 16, (int64_t)4 * MXG_WAVES), (unsigned)ytiles, narrow ? 1 : 2);
     if (wide12) grid = dim3((unsigned)ceil_div(p.N, 32 * MXG_WAVES12), (unsigned)ytiles);
     char name[64];
-    snprintf(name, sizeof name, "mxfp4_experts_gemm_bf16_r%dx%d%s", rows, wide12 ? MXG_WAVES12 : MXG_WAVES, p.swiglu ? "_swiglu" : "");
+    plan_name(name, sizeof name, "mxfp4_experts_gemm_bf16_r%dx%d%s", rows, wide12 ? MXG_WAVES12 : MXG_WAVES, p.swiglu ? "_swiglu" : "");
     set_plan(ctx, name, grid, dim3(wide12 ? 64 * MXG_WAVES12 : 512), 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     const uint64_t x_bytes = (uint64_t)p.M * (uint64_t)p.K * 2u;

@@ -701,7 +701,7 @@ int launch_mxfp4_res_gemv(oxq_ctx *ctx, hipStream_t s, const Mxfp4Problem &p) {
     constexpr int WR = 8, NWV = 4;
     dim3 grid((unsigned)ceil_div(p.N / 16, NWV), (unsigned)p.n_experts), block(NWV * 64);
     char name[64];
-    snprintf(name, sizeof name, "mxfp4_experts_gemv_bf16_t%d%s", MTOK, p.swiglu ? "_swiglu" : "");
+    plan_name(name, sizeof name, "mxfp4_experts_gemv_bf16_t%d%s", MTOK, p.swiglu ? "_swiglu" : "");
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if ((uintptr_t)p.x & 15) return fail(OXQ_ERR_UNSUPPORTED, "mxfp4 experts: x must be 16-byte aligned");
@@ -759,7 +759,7 @@ int launch_mxfp4_gemv(oxq_ctx *ctx, hipStream_t s, const Mxfp4Problem &p) {
         if (variant == 0 && lds <= 128 * 1024 && p.K % 32 == 0) {
             dim3 grid((unsigned)ceil_div(p.N, 4 * 16 * FR), grouped ? (unsigned)p.n_experts : 1u), block(256);
             char name[64];
-            snprintf(name, sizeof name, "%s_mfma_t%d%s", grouped ? "mxfp4_moe_gemv_bf16" : "mxfp4_gemv_bf16", mtok,
+            plan_name(name, sizeof name, "%s_mfma_t%d%s", grouped ? "mxfp4_moe_gemv_bf16" : "mxfp4_gemv_bf16", mtok,
                      p.swiglu ? "_swiglu" : "");
             set_plan(ctx, name, grid, block, 1, 1, 0);
             if (ctx->plan_only) return OXQ_OK;
@@ -780,7 +780,7 @@ int launch_mxfp4_gemv(oxq_ctx *ctx, hipStream_t s, const Mxfp4Problem &p) {
     if (use_lds) {
         dim3 grid((unsigned)ceil_div(p.N, 4 * RW), grouped ? (unsigned)p.n_experts : 1u), block(256);
         char name[64];
-        snprintf(name, sizeof name, "%s_lds_m%d", grouped ? "mxfp4_moe_gemv_bf16" : "mxfp4_gemv_bf16", mb);
+        plan_name(name, sizeof name, "%s_lds_m%d", grouped ? "mxfp4_moe_gemv_bf16" : "mxfp4_gemv_bf16", mb);
         set_plan(ctx, name, grid, block, 1, 1, 0);
         if (ctx->plan_only) return OXQ_OK;
         if (((uintptr_t)p.blocks & 15) || ((uintptr_t)p.x & 15) || (p.K % 8))

@@ -5,7 +5,9 @@
 #include "oxq_internal.hpp"
 #include "oxq_bench.h"
 
+#include <cstdarg>
 #include <cstdlib>
+#include <cstring>
 #include <new>
 #include <vector>
 
@@ -34,11 +36,34 @@ const char *dtype_name(int dtype) {
     }
 }
 
+void plan_name(char *buf, size_t n, const char *fmt, ...) {
+    va_list ap;
+    va_start(ap, fmt);
+    char *out = buf, *const end = buf + n - 1;
+    for (; *fmt && out < end; ++fmt) {
+        if (*fmt != '%') {
+            *out++ = *fmt;
+        } else if (*++fmt == 's') {
+            for (const char *t = va_arg(ap, const char *); *t && out < end; ++t) *out++ = *t;
+        } else {  // 'd'
+            const int v = va_arg(ap, int);
+            unsigned u = v < 0 ? 0u - (unsigned)v : (unsigned)v;
+            char digits[12];
+            int k = 0;
+            do digits[k++] = (char)('0' + u % 10); while (u /= 10);
+            if (v < 0) digits[k++] = '-';
+            while (k > 0 && out < end) *out++ = digits[--k];
+        }
+    }
+    va_end(ap);
+    *out = 0;
+}
+
 void set_plan(oxq_ctx *ctx, const char *kernel, dim3 grid, dim3 block, uint32_t split_k,
               uint32_t launches, uint64_t ws_bytes) {
     oxq_plan &pl = ctx->plan;
     memset(&pl, 0, sizeof pl);
-    snprintf(pl.kernel, sizeof pl.kernel, "%s", kernel);
+    memcpy(pl.kernel, kernel, strnlen(kernel, sizeof pl.kernel - 1));
     pl.grid[0] = grid.x; pl.grid[1] = grid.y; pl.grid[2] = grid.z;
     pl.block[0] = block.x; pl.block[1] = block.y; pl.block[2] = block.z;
     pl.split_k = split_k;
@@ -48,13 +73,16 @@ void set_plan(oxq_ctx *ctx, const char *kernel, dim3 grid, dim3 block, uint32_t 
 
 void add_launch(oxq_ctx *ctx) { ctx->plan.launches++; }
 
-static void dims_str(const oxq_tensor *t, char *buf, size_t n) {
-    size_t off = 0;
-    off += snprintf(buf + off, n - off, "[");
-    for (int i = 0; i < t->rank && off < n; ++i)
-        off += snprintf(buf + off, n - off, "%s%lld", i ? ", " : "", (long long)t->dims[i]);
-    if (off < n) snprintf(buf + off, n - off, "]");
-}
+// "[2, 3]", where a message is composed (snprintf on calls that succeed took a microsecond of an op's host time)
+struct DimsStr {
+    char s[96];
+    explicit DimsStr(const oxq_tensor *t) {
+        size_t off = (size_t)snprintf(s, sizeof s, "[");
+        for (int i = 0; i < t->rank && off < sizeof s; ++i)
+            off += snprintf(s + off, sizeof s - off, "%s%lld", i ? ", " : "", (long long)t->dims[i]);
+        if (off < sizeof s) snprintf(s + off, sizeof s - off, "]");
+    }
+};
 
 // Basic descriptor sanity + residency.  `op` prefixes the message.
 static int check_tensor(const oxq_ctx *ctx, const char *op, const char *what, const oxq_tensor *t) {
@@ -106,17 +134,15 @@ static int check_wna16(oxq_ctx *ctx, const char *op, Wna16Kind kind, const oxq_t
     OXQ_TRY(check_tensor(ctx, op, "qzeros", qzeros));
     OXQ_TRY(check_tensor(ctx, op, "scales", scales));
     OXQ_TRY(check_tensor(ctx, op, "out", out));
-    char b0[96], b1[96];
 
     int64_t m = 1, in_features = 0;
     if (kind != KIND_DEQUANT) {
         if (!x->contiguous) return fail(OXQ_ERR_CONTIGUOUS, "%s: x must be contiguous", op);
-        dims_str(x, b0, sizeof b0);
-        if (x->rank != 2) return fail(OXQ_ERR_SHAPE, "%s: x must be 2-D [m, in], got %s", op, b0);
+        if (x->rank != 2) return fail(OXQ_ERR_SHAPE, "%s: x must be 2-D [m, in], got %s", op, DimsStr(x).s);
         if (kind == KIND_GEMV && !(x->dims[0] >= 1 && x->dims[0] <= 8))
             return fail(OXQ_ERR_M_RANGE,
-                        "%s: x must be [m, in] with m in 1..=8 (decode GEMV path), got %s", op, b0);
-        if (x->dims[0] < 1) return fail(OXQ_ERR_SHAPE, "%s: x has no rows, got %s", op, b0);
+                        "%s: x must be [m, in] with m in 1..=8 (decode GEMV path), got %s", op, DimsStr(x).s);
+        if (x->dims[0] < 1) return fail(OXQ_ERR_SHAPE, "%s: x has no rows, got %s", op, DimsStr(x).s);
         m = x->dims[0];
         in_features = x->dims[1];
     } else if (!qweight->contiguous) {
@@ -137,8 +163,7 @@ static int check_wna16(oxq_ctx *ctx, const char *op, Wna16Kind kind, const oxq_t
     if (pack_dim == OXQ_PACK_OUT) {
         const int64_t qw_in = qweight->dims[0], packed_out = qweight->dims[1];
         if (qzeros->rank != 2 || qzeros->dims[0] != groups || qzeros->dims[1] != packed_out) {
-            dims_str(qzeros, b0, sizeof b0);
-            return fail(OXQ_ERR_SHAPE, "%s: qzeros shape %s != [%lld, %lld]", op, b0,
+            return fail(OXQ_ERR_SHAPE, "%s: qzeros shape %s != [%lld, %lld]", op, DimsStr(qzeros).s,
                         (long long)groups, (long long)packed_out);
         }
         // AwqShape::new_bits (metal_ops.rs:1434-1458)
@@ -155,8 +180,7 @@ static int check_wna16(oxq_ctx *ctx, const char *op, Wna16Kind kind, const oxq_t
             return fail(OXQ_ERR_SHAPE, "%s: qweight dim1 %lld != scales out_features %lld", op,
                         (long long)qw_out, (long long)out_features);
         if (qzeros->rank != 2 || qzeros->dims[0] != groups || qzeros->dims[1] * pf != out_features) {
-            dims_str(qzeros, b0, sizeof b0);
-            return fail(OXQ_ERR_SHAPE, "%s: qzeros shape %s != [%lld, %lld]", op, b0,
+            return fail(OXQ_ERR_SHAPE, "%s: qzeros shape %s != [%lld, %lld]", op, DimsStr(qzeros).s,
                         (long long)groups, (long long)(out_features / pf));
         }
         // GptqShape::new_bits (metal_ops.rs:1923-1943)
@@ -173,13 +197,12 @@ static int check_wna16(oxq_ctx *ctx, const char *op, Wna16Kind kind, const oxq_t
     if (kind != KIND_DEQUANT && in_features != K)
         return fail(OXQ_ERR_SHAPE, "%s: x in_features %lld != weight in_features %lld", op,
                     (long long)in_features, (long long)K);
-    dims_str(out, b1, sizeof b1);
     if (kind == KIND_DEQUANT) {
         if (out->rank != 2 || out->dims[0] != K || out->dims[1] != out_features)
-            return fail(OXQ_ERR_SHAPE, "%s: output shape %s != [%lld, %lld]", op, b1, (long long)K,
+            return fail(OXQ_ERR_SHAPE, "%s: output shape %s != [%lld, %lld]", op, DimsStr(out).s, (long long)K,
                         (long long)out_features);
     } else if (out->rank != 2 || out->dims[0] != m || out->dims[1] != out_features) {
-        return fail(OXQ_ERR_SHAPE, "%s: output shape %s != [%lld, %lld]", op, b1, (long long)m,
+        return fail(OXQ_ERR_SHAPE, "%s: output shape %s != [%lld, %lld]", op, DimsStr(out).s, (long long)m,
                     (long long)out_features);
     }
     if (!out->contiguous) return fail(OXQ_ERR_CONTIGUOUS, "%s: out must be contiguous", op);
@@ -259,7 +282,6 @@ static int check_gguf(oxq_ctx *ctx, const char *op, bool decode, bool dequant, c
     if (!dequant) OXQ_TRY(check_tensor(ctx, op, "x", x));
     OXQ_TRY(check_tensor(ctx, op, "weight_bytes", w));
     OXQ_TRY(check_tensor(ctx, op, "out", out));
-    char b0[96];
     int act = OXQ_F32;
     int64_t m = 1;
     if (!dequant) {
@@ -286,15 +308,13 @@ static int check_gguf(oxq_ctx *ctx, const char *op, bool decode, bool dequant, c
         if (decode && !(m >= 1 && m <= 8))
             return fail(OXQ_ERR_M_RANGE, "%s (%s): m %lld out of [1, 8]", op, qn, (long long)m);
         if (!x->contiguous) return fail(OXQ_ERR_CONTIGUOUS, "%s (%s): x must be contiguous", op, qn);
-        dims_str(x, b0, sizeof b0);
         if (x->rank != 2 || x->dims[1] != in_features || m < 1)
-            return fail(OXQ_ERR_SHAPE, "%s (%s): x shape %s != [%s, %lld]", op, qn, b0,
+            return fail(OXQ_ERR_SHAPE, "%s (%s): x shape %s != [%s, %lld]", op, qn, DimsStr(x).s,
                         decode ? "m" : "M", (long long)in_features);
     }
-    dims_str(out, b0, sizeof b0);
     const int64_t o0 = dequant ? out_features : m, o1 = dequant ? in_features : out_features;
     if (out->rank != 2 || out->dims[0] != o0 || out->dims[1] != o1 || !out->contiguous)
-        return fail(OXQ_ERR_SHAPE, "%s (%s): output shape %s != [%lld, %lld]", op, qn, b0,
+        return fail(OXQ_ERR_SHAPE, "%s (%s): output shape %s != [%lld, %lld]", op, qn, DimsStr(out).s,
                     (long long)o0, (long long)o1);
     const int64_t expected = out_features * (in_features / be) * bb;
     if (numel(w) != expected || !w->contiguous)
@@ -325,7 +345,6 @@ static int check_mxfp4(oxq_ctx *ctx, const char *op, bool dequant, const oxq_ten
     OXQ_TRY(check_tensor(ctx, op, "blocks", blocks));
     OXQ_TRY(check_tensor(ctx, op, "scales", scales));
     OXQ_TRY(check_tensor(ctx, op, "out", out));
-    char b0[96];
     if (!dequant && (out->dtype != OXQ_BF16 || x->dtype != OXQ_BF16))
         return fail(OXQ_ERR_DTYPE, "%s: x/out must be BF16, got %s/%s", op, dtype_name(x->dtype),
                     dtype_name(out->dtype));
@@ -344,9 +363,8 @@ static int check_mxfp4(oxq_ctx *ctx, const char *op, bool dequant, const oxq_ten
     int64_t m = 1;
     if (!dequant) {
         if (!x->contiguous) return fail(OXQ_ERR_CONTIGUOUS, "%s: x must be contiguous", op);
-        dims_str(x, b0, sizeof b0);
         if (x->rank != 2 || x->dims[1] != k || x->dims[0] < 1)
-            return fail(OXQ_ERR_SHAPE, "%s: x shape %s != [m, %lld]", op, b0, (long long)k);
+            return fail(OXQ_ERR_SHAPE, "%s: x shape %s != [m, %lld]", op, DimsStr(x).s, (long long)k);
         m = x->dims[0];
     }
     if (k > INT32_MAX || n > INT32_MAX) return fail(OXQ_ERR_SHAPE, "%s: dimension exceeds 2^31-1", op);
@@ -1374,10 +1392,8 @@ static int check_f8(oxq_ctx *ctx, const char *op, const oxq_tensor *x, const oxq
         if (x->dtype != OXQ_BF16) return fail(OXQ_ERR_DTYPE, "%s: x must be BF16, got %s", op, dtype_name(x->dtype));
         if (!x->contiguous) return fail(OXQ_ERR_CONTIGUOUS, "%s: x must be contiguous", op);
         if (x->rank != 2 || x->dims[1] != cols || x->dims[0] == 0 || (decode && x->dims[0] > 8)) {
-            char b0[96];
-            dims_str(x, b0, sizeof b0);
             return fail(decode && x->rank == 2 && x->dims[1] == cols ? OXQ_ERR_M_RANGE : OXQ_ERR_SHAPE,
-                        "%s: x shape %s incompatible with in_features %lld%s", op, b0, (long long)cols,
+                        "%s: x shape %s incompatible with in_features %lld%s", op, DimsStr(x).s, (long long)cols,
                         decode ? " (m must be 1..=8)" : "");
         }
         m = x->dims[0];
@@ -1431,10 +1447,8 @@ int oxq_mxfp4_matmul(oxq_ctx *ctx, void *stream, const oxq_tensor *x, const oxq_
                      const oxq_tensor *scales, int64_t k, int64_t n, const oxq_tensor *out) {
     Mxfp4Problem p;
     OXQ_TRY(check_mxfp4(ctx, "Mxfp4Matmul", false, x, blocks, scales, k, n, 0, out, &p));
-    char b0[96];
-    dims_str(out, b0, sizeof b0);
     if (out->rank != 2 || out->dims[0] != p.M || out->dims[1] != n || !out->contiguous)
-        return fail(OXQ_ERR_SHAPE, "Mxfp4Matmul: output shape %s != [%lld, %lld]", b0,
+        return fail(OXQ_ERR_SHAPE, "Mxfp4Matmul: output shape %s != [%lld, %lld]", DimsStr(out).s,
                     (long long)p.M, (long long)n);
     return launch_mxfp4_gemv(ctx, (hipStream_t)stream, p);
 }

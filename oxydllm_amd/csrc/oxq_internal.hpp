@@ -103,6 +103,8 @@ inline int tune(const oxq_ctx *ctx, oxq_tune_key key, int dflt) {
 }
 inline bool tune_given(const oxq_ctx *ctx, oxq_tune_key key) { return ctx->tuning[key] != OXQ_TUNE_UNSET; }
 
+// A kernel's name for a plan, %s and %d only: every call formats one, and snprintf took a tenth of a small call's host time.
+void plan_name(char *buf, size_t n, const char *fmt, ...) __attribute__((format(printf, 3, 4)));
 void set_plan(oxq_ctx *ctx, const char *kernel, dim3 grid, dim3 block, uint32_t split_k,
               uint32_t launches, uint64_t ws_bytes);
 void add_launch(oxq_ctx *ctx);

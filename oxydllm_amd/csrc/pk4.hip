@@ -767,7 +767,7 @@ int launch_pk4_prepack(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &src, con
     if (dst.strip != 16 && wide > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repack: %lld x %lld exceeds the grid", (long long)src.K, (long long)src.N);
     dim3 grid((unsigned)(dst.strip == 16 ? ceil_div((int64_t)words, 256) : wide)), block(256);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_prepack_%s%s", src.bits, gptq ? "gptq" : "awq", dst.strip == 16 ? "_n16" : "");
+    plan_name(name, sizeof name, "pk%d_prepack_%s%s", src.bits, gptq ? "gptq" : "awq", dst.strip == 16 ? "_n16" : "");
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if (dst.strip == 16) {
@@ -806,7 +806,7 @@ int launch_pk4_dequant(oxq_ctx *ctx, hipStream_t s, const Pk4Weights &w, void *o
     const size_t words = (size_t)ceil_div(w.N, 64) * (size_t)ceil_div(w.K, 128) * 256 * (size_t)w.bits;  // weights of whole blocks
     dim3 grid((unsigned)ceil_div((int64_t)words, 256)), block(256);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_dequant_%s", w.bits, w.dtype == OXQ_F16 ? "f16" : "bf16");
+    plan_name(name, sizeof name, "pk%d_dequant_%s", w.bits, w.dtype == OXQ_F16 ? "f16" : "bf16");
     set_plan(ctx, name, grid, block, 1, 1, 0);
     if (ctx->plan_only) return OXQ_OK;
     if (w.strip == 16) {
@@ -1190,7 +1190,7 @@ static int launch_pk4n_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p)
                         (M <= 8 || (M <= 16 && ceil_div(bslice, 16) <= 4));
     const bool w16 = nfront || (ns == 1 && M <= 2 && tune(ctx, OXQ_TUNE_PK4N_W16, NB >= 64));
     char name[64];
-    snprintf(name, sizeof name, "pk4_mfma_%s_mt%d%s_n16x%d%s", p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows_mt,
+    plan_name(name, sizeof name, "pk4_mfma_%s_mt%d%s_n16x%d%s", p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows_mt,
              (fold || ns == 1) ? "_gs" : "", ns, pk4_by_name(mt, rows_mt));
     set_plan(ctx, name, grid, dim3(w16 ? 1024 : 512), ks, 1, ks > 1 ? (size_t)ks * M * N * 4 : 0);
     if (ctx->plan_only) {
@@ -1274,7 +1274,7 @@ int launch_pk4_forward(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
         else
             front = (front_mode != 2 && bslice == 32 && ks == 1) ? 1 : (bslice % 8 == 0 && share8 <= 8 && share8 != 7) ? 2 : 0;
     }
-    snprintf(name, sizeof name, "pk%d_mfma_%s_mt%d%s%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows_mt,
+    plan_name(name, sizeof name, "pk%d_mfma_%s_mt%d%s%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows_mt,
              fold ? "_gs" : "", sets == 2 ? "_g64" : sets == 4 ? "_g32" : "", front == 1 ? "_front" : front == 2 ? "_line" : "",
              pk4_by_name(mt, rows_mt), p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(front == 1 ? 1024 : 512), ks, 1, ks > 1 ? (size_t)ks * M * p.w.N * 4 : 0);

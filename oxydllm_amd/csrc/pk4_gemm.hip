@@ -385,7 +385,7 @@ int launch_pk4_gemm(oxq_ctx *ctx, hipStream_t s, const Pk4Problem &p) {
     if (wgs > 0x7FFFFFFF) return fail(OXQ_ERR_UNSUPPORTED, "repacked matmul: m = %lld exceeds the grid", (long long)p.M);
     dim3 grid((unsigned)wgs);
     char name[64];
-    snprintf(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw,
+    plan_name(name, sizeof name, "pk%d_gemm_%s_r%dx%d%s%s%s%s", p.w.bits, p.w.dtype == OXQ_F16 ? "f16" : "bf16", rows, spw,
              form.ks > 1 ? "k4" : form.light ? "r32" : "", p.w.unrounded ? "_gs" : "", p.w.strip == 16 ? "_n16" : "",
              p.act == 1 ? "_silu" : p.act == 2 ? "_gelu" : "");
     set_plan(ctx, name, grid, dim3(512), 1, 1, 0);

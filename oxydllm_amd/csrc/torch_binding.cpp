@@ -251,7 +251,7 @@ at::Tensor empty_rows(const at::Tensor &x, int64_t width) {
 }
 
 // One resident 4096 x 4096 4-bit layer at one row of f16, called back to back without waiting: 12.2 us through
-// Python-built descriptors, 4.9 us here (4.1 with the caller's output tensor; the kernel alone takes 3.6 us, torch's
+// Python-built descriptors, 4.5 us here (3.7 with the caller's output tensor; the kernel alone takes 3.6 us, torch's
 // own zero_() 3.8 us a call).  The six outputs and one launch of moe_route_group: 27.8 -> 8.5 us.
 PyObject *layer_call(PyObject *self, PyObject *const *args, size_t nargsf, PyObject *kwnames) {
     OXQ_BODY_BEGIN

@@ -735,7 +735,7 @@ static int launch_awq_fast_t(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p,
     dim3 block(WPG * GPB * 64);
     const uint64_t ws_bytes = S > 1 ? (uint64_t)S * p.M * p.N * 4 : 0;
     char name[64];
-    snprintf(name, sizeof name, "awq%d_gemv_fast_%s_m%d_w%d_g%dx%d_r%d_p%d", BITS,
+    plan_name(name, sizeof name, "awq%d_gemv_fast_%s_m%d_w%d_g%dx%d_r%d_p%d", BITS,
              TT::DTYPE == 1 ? "f16" : "bf16", MB, WPL, WPG, GPB, RPW, PS);
     set_plan(ctx, name, grid, block, S, 1, ws_bytes);
     if (ctx->plan_only) {
@@ -829,7 +829,7 @@ static int launch_generic_t(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) 
     dim3 grid((unsigned)tiles, (unsigned)S), block(256);
     const uint64_t ws_bytes = S > 1 ? (uint64_t)S * p.M * p.N * 4 : 0;
     char name[64];
-    snprintf(name, sizeof name, "%s_gemv_generic_w%d_%s_m%d", awq ? "awq" : "gptq", BITS,
+    plan_name(name, sizeof name, "%s_gemv_generic_w%d_%s_m%d", awq ? "awq" : "gptq", BITS,
              TT::DTYPE == 1 ? "f16" : "bf16", mb);
     set_plan(ctx, name, grid, block, S, 1, ws_bytes);
     // the stand-alone reduce handles 4 outputs per thread
@@ -889,7 +889,7 @@ static int launch_gptq_fast(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) 
     dim3 grid((unsigned)slabs, (unsigned)S), block(512);
     const uint64_t ws_bytes = S > 1 ? (uint64_t)S * p.M * p.N * 4 : 0;
     char name[64];
-    snprintf(name, sizeof name, "gptq%d_gemv_fast_%s_m%d", BITS, TT::DTYPE == 1 ? "f16" : "bf16", mb);
+    plan_name(name, sizeof name, "gptq%d_gemv_fast_%s_m%d", BITS, TT::DTYPE == 1 ? "f16" : "bf16", mb);
     set_plan(ctx, name, grid, block, S, 1, ws_bytes);
     const int fused = splitk_fused(ctx, S);
     if (ctx->plan_only) {

@@ -606,7 +606,7 @@ static int launch_awq4_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) 
         }
         dim3 grid((unsigned)(ctiles * S), 1, (unsigned)mtiles), block(256);
         const uint64_t ws_bytes = S > 1 ? (uint64_t)S * M * N * 4 : 0;
-        snprintf(name, sizeof name, "awq4_mfma_ksplit_%s_mt%d", dt, mt);
+        plan_name(name, sizeof name, "awq4_mfma_ksplit_%s_mt%d", dt, mt);
         set_plan(ctx, name, grid, block, S, 1, ws_bytes);
         if (ctx->plan_only) {
             if (S > 1) add_launch(ctx);
@@ -648,7 +648,7 @@ static int launch_awq4_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) 
     dim3 grid((unsigned)ctiles, (unsigned)S, (unsigned)mtiles), block(256);
     const uint64_t ws_bytes = S > 1 ? (uint64_t)S * M * N * 4 : 0;
     const bool pipe = variant != 3 && p.group_size >= 128 && kslice2 % 128 == 0 && K % 128 == 0;
-    snprintf(name, sizeof name, "awq4_mfma%s_%s_mt%d", pipe ? "_pipe" : "", dt, mt);
+    plan_name(name, sizeof name, "awq4_mfma%s_%s_mt%d", pipe ? "_pipe" : "", dt, mt);
     set_plan(ctx, name, grid, block, S, 1, ws_bytes);
     if (ctx->plan_only) {
         if (S > 1) add_launch(ctx);

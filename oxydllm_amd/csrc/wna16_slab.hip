@@ -405,7 +405,7 @@ int launch_wna16_slab(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     const uint64_t ws_bytes = S > 1 ? (uint64_t)S * p.M * p.N * 4 : 0;
     const bool f16 = p.dtype == OXQ_F16, gptq = p.pack_dim == OXQ_PACK_IN;
     char name[64];
-    snprintf(name, sizeof name, "%s%d_gemv_fast_%s_m%d_slab%d%s", gptq ? "gptq" : "awq", p.bits, f16 ? "f16" : "bf16", (int)p.M, run,
+    plan_name(name, sizeof name, "%s%d_gemv_fast_%s_m%d_slab%d%s", gptq ? "gptq" : "awq", p.bits, f16 ? "f16" : "bf16", (int)p.M, run,
              p.group_size >= 128 ? "" : p.group_size == 64 ? "_g64" : "_g32");
     set_plan(ctx, name, grid, dim3(SLAB_WAVES * 64), S, 1, ws_bytes);
     if (!ctx->plan_only) {
