@@ -499,8 +499,18 @@ __global__ __launch_bounds__(NW * 64) void pk4n_mfma_kernel(const uint16_t *__re
 
     u32x4_t afirst[AQ];
     load_a(0, afirst);
+    // The last two blocks by themselves, requesting nothing behind them - but where the instructions of two more bodies, which come
+    // from memory anew at each launch, count for more than the loads: one folded row tile, f16 at one tile and at four.  us, one loop ->
+    // ends: bf16 14336 x 4096 at 20 / 64 rows 14.6 / 21.4 -> 14.1 / 20.7, 5120 x 5120 at 40 / 64 13.3 / 15.2 -> 12.8 / 14.6, 2048 x 2048 at 20 / 64
+    // 6.5 / 6.9 -> 6.2 / 6.6, f16 8192 x 8192 at 20 16.0 -> 15.0; left alone f16 4096 x 4096 at 20 7.6 / 7.8, 14336 x 4096 at 64 20.4 / 21.2.
+    constexpr bool ENDS = RD == 2 && (DUAL ? MT == 2 || MT == 3 : MT > 1 || !GS);
+    const bool odd = nloc & 1;  // the last block has ring half 1
+    if (ENDS && odd) {
+        load_w(0, wr[1], zr[1 % ZD]);
+    } else {
 #pragma unroll
-    for (int d = 0; d + 1 < RD; ++d) load_w(d, wr[d], zr[d % ZD]);
+        for (int d = 0; d + 1 < RD; ++d) load_w(d, wr[d], zr[d % ZD]);
+    }
     if constexpr (ZD == 1) load_z(0, zr[0]);
     load_a(1, aring);
 
@@ -516,11 +526,13 @@ __global__ __launch_bounds__(NW * 64) void pk4n_mfma_kernel(const uint16_t *__re
 
     store_a(afirst);
 
-    // one block: its weights are in ring half CUR; the next block is requested into the other half first
-    auto block = [&](int i, auto cur_c) {
-        constexpr int CUR = decltype(cur_c)::value, NXT = (CUR + RD - 1) % RD;
+    // one block: its weights are in ring half CUR; the next block is requested into the other half first.  AFTER: blocks known to follow
+    // (2: two, or as many as it takes), behind which nothing is requested: a load from the empty descriptor takes its turn in the
+    // address unit as any other, and what follows waits for the registers it writes (64 rows: sixteen loads of x a block).
+    auto block = [&](int i, auto cur_c, auto after_c) {
+        constexpr int CUR = decltype(cur_c)::value, NXT = (CUR + RD - 1) % RD, AFTER = decltype(after_c)::value;
         constexpr int ZC = CUR % ZD, ZN = NXT % ZD;
-        load_w(i + RD - 1, wr[NXT], zr[ZN]);
+        if constexpr (AFTER > 0) load_w(i + RD - 1, wr[NXT], zr[ZN]);
         float4_t tmp[GS ? MT : 1][NS], tmp1[GS ? MT : 1], tmpb[(GS && DUAL) ? MT : 1];
         Pk4N<TT> cst[(GS && !EXACT) ? 1 : NS];
         constexpr bool WIDEN = !GS && TT::DTYPE == BF16Traits::DTYPE;
@@ -532,7 +544,7 @@ __global__ __launch_bounds__(NW * 64) void pk4n_mfma_kernel(const uint16_t *__re
 #pragma unroll
             for (int f = 0; f < NS; ++f) cst[f].prep(zr[ZC][f]);
         }
-        if constexpr (ZD == 1) load_z(i + 1, zr[0]);
+        if constexpr (ZD == 1 && AFTER > 0) load_z(i + 1, zr[0]);
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             uint32_t a[MT][4];
@@ -568,6 +580,7 @@ __global__ __launch_bounds__(NW * 64) void pk4n_mfma_kernel(const uint16_t *__re
                     if (DUAL) tmpb[mt] = Ops::mfma(a[mt], biases, fresh ? zero4 : tmpb[mt]);
                 }
             }
+            if constexpr (MT >= 3 && AFTER < 2) __builtin_amdgcn_sched_barrier(0);  // no operands of the next step early: no registers for them
         }
         if (GS) {  // y += s * ((sum - biased row sum) - z * row sum), all f32
 #pragma unroll
@@ -588,30 +601,41 @@ __global__ __launch_bounds__(NW * 64) void pk4n_mfma_kernel(const uint16_t *__re
                     }
             }
         }
-        store_a(aring);
-        load_a(i + 2, aring);
+        if constexpr (AFTER > 0) store_a(aring);
+        if constexpr (AFTER > 1) load_a(i + 2, aring);
         // the requests for the block after next stay here: sunk to their use in the next block (which the
         // scheduler does in some single-tile instantiations to save registers) they would be waited for at
         // once (bf16, 16 rows, 14336 x 4096: 13.0 -> 10.7 us).  The larger tiles schedule better without.
-        if constexpr (MT == 1) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (MT == 1 || AFTER == 1) __builtin_amdgcn_sched_barrier(0);
     };
     {
+        const std::integral_constant<int, 0> c0;
+        const std::integral_constant<int, 1> c1;
+        const std::integral_constant<int, 2> c2;
         int i = 0;
-        if constexpr (RD == 2) {
-            for (; i + 1 < nloc; i += 2) {
-                block(i, std::integral_constant<int, 0>{});
-                block(i + 1, std::integral_constant<int, 1>{});
+        if constexpr (ENDS) {
+            if (odd && nloc > 1) block(i++, c1, c2);
+            for (; i + 2 < nloc; i += 2) {
+                block(i, c0, c2);
+                block(i + 1, c1, c2);
             }
-            if (i < nloc) block(i, std::integral_constant<int, 0>{});
+            if (nloc > 1) block(nloc - 2, c0, c1);
+            if (nloc > 0) block(nloc - 1, c1, c0);
+        } else if constexpr (RD == 2) {
+            for (; i + 1 < nloc; i += 2) {
+                block(i, c0, c2);
+                block(i + 1, c1, c2);
+            }
+            if (i < nloc) block(i, c0, c2);
         } else {
             static_assert(RD == 3, "the loop below is unrolled for a ring of three");
             for (; i + 2 < nloc; i += 3) {
-                block(i, std::integral_constant<int, 0>{});
-                block(i + 1, std::integral_constant<int, 1>{});
-                block(i + 2, std::integral_constant<int, 2>{});
+                block(i, c0, c2);
+                block(i + 1, c1, c2);
+                block(i + 2, c2, c2);
             }
-            if (i < nloc) block(i, std::integral_constant<int, 0>{});
-            if (i + 1 < nloc) block(i + 1, std::integral_constant<int, 1>{});
+            if (i < nloc) block(i, c0, c2);
+            if (i + 1 < nloc) block(i + 1, c1, c2);
         }
     }
 

@@ -241,6 +241,9 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
     for (int u = 0; u < UF; ++u) {
         const int i = i0 + u;
         if (u > 0 && i >= nloc) break;
+        // Straight-line code knows its last block, behind which nothing is requested: a load from the empty descriptor takes its turn
+        // in the address unit as any other, and what follows waits for the registers it writes.
+        const bool last = NBLK > 0 && i + 1 >= NBLK;
         float4_t tmp[GS ? MT : 1][4], tmps[GS ? MT : 1];  // per-block integer sums of the GS form
         // the tile form's constants of a set, and the request for the next block's
         auto constants = [&](int set) {
@@ -251,13 +254,13 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
                 if constexpr (WIDEN) cb[f].set(__builtin_bit_cast(float, zv[f] & 0xFFFF0000u), __builtin_bit_cast(float, zv[f] << 16) + 128.0f);
                 else Pk4T<TT>::prep(zv[f], negzb[f], sp[f]);
             }
-            load_z(i + 1, set);
+            if (!last) load_z(i + 1, set);
         };
         // the folded form: y += s * (sum - (bias + z) * rowsum), all f32
         auto fold = [&](int set) {
             uint32_t zv[4];
             pk4_pair_words(zring[set], zv);
-            load_z(i + 1, set);
+            if (!last) load_z(i + 1, set);
 #pragma unroll
             for (int f = 0; f < 4; ++f) {
                 const float sf = TT::to_f32((uint16_t)(zv[f] >> 16));
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
             // Refill this ring slot after its last use, so that the new block can land in the same registers
             // (requested while the old value is live it lands in others, copied at the loop's end behind a wait
             // for the request): 17 / 33 / 48 rows f16 9.96 / 12.76 / 13.57 -> 9.85 / 12.57 / 13.44 us.
-            load_w(i + 1, st, wring[st]);
+            if (!last) load_w(i + 1, st, wring[st]);
             if constexpr (PLACED) __builtin_amdgcn_sched_barrier(0x106);
             if (GS && (st + 1) % SPS == 0) fold(st / SPS);
         }
@@ -342,8 +345,10 @@ __global__ __launch_bounds__(512) void pk4_mfma_kernel(const uint16_t *__restric
         // fragments of the current block held in registers instead), its reload comes late in the block and
         // is waited for at the next block's start.
         if constexpr (PLACED) __builtin_amdgcn_sched_barrier(0);
-        store_a(aring);
-        load_a(i + 2, aring);
+        if (!last) {
+            store_a(aring);
+            if (NBLK == 0 || i + 2 < NBLK) load_a(i + 2, aring);
+        }
         // two and four row tiles as straight-line code: the requests for the block after next stay at the block's
         // end (four tiles at 64 rows, same box: f16 16.54 -> 16.37 us, bf16 18.42 -> 17.90; three tiles the same
         // either way)
