@@ -740,10 +740,10 @@ constexpr int ggm_waves = FMT == OXQ_GGUF_Q6_K && MT == 1 && XQ == 1 && NW == 8 
 // f32 results keep what the sums hold, so a chunk's steps are summed by themselves before they join the wave's sum: added to it
 // one by one, 4 - 16 roundings a chunk at the size of the whole sum, the formats with a minimum were 1.4 - 1.8 x as far from
 // 64 bits as the vector kernels at K = 14336 (Q4_K at 8 rows 1.7e-7 against 1.25e-7; now 1.0e-7, at up to 2.5 % of the time).
-template <int FMT, int MT, int XQ, int NW, int NS, bool XF32 = false>
-__global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) void ggm_kernel(
-    const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
-    float *__restrict__ ws, int M, int K, int N, int cslice, int act) {
+// NL > 0 (ggm_short_kernel): no wave has more than NL chunks, all of them requested at once; 0: a loop.
+template <int FMT, int MT, int XQ, int NW, int NS, bool XF32, int NL>
+__device__ __forceinline__ void ggm_body(const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw, const uint16_t *__restrict__ bias,
+                                         uint16_t *__restrict__ y, float *__restrict__ ws, int M, int K, int N, int cslice, int act) {
     constexpr bool ONE = XF32 && XQ == 1;
     static_assert(!XF32 || XQ == 2 * MT || (ONE && MT == 1), "two loads a lane bring four rows' chunk of f32");
     constexpr int TROWS = XF32 ? 4 * MT : 16 * MT;  // rows of x a tile takes
@@ -755,7 +755,7 @@ __global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) vo
     constexpr int ROWS = 16 * MT, AQ = XQ, SLOT = ROWS * 256, OOB = 0x7FFFFF00, NSTEP = C::NSTEP;
     // chunks in flight a wave: three (4096 x 4096 at one row, Q8_0: 5.06 us with three, 5.87 with two); two
     // where a workgroup takes four strips, whose quants are four times the registers
-    constexpr int RD = NS > 1 ? 2 : 3;
+    constexpr int RD = NL > 0 ? NL : NS > 1 ? 2 : 3;
     constexpr bool K16 = NSTEP == 8;  // steps of 16 elements
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
 
@@ -827,8 +827,14 @@ __global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) vo
         for (int f = 0; f < NS; ++f) w[f].request(rw, lane, ni, c, (int)(f * strip_bytes));
         __builtin_amdgcn_sched_barrier(0);  // chunks are requested in the order they are used
     };
+    if constexpr (NL > 0) {  // the last chunk has the last set, whatever their number
 #pragma unroll
-    for (int d = 0; d < RD; ++d) request(d, wr[d], ar[d]);
+        for (int d = 0; d < RD; ++d)
+            if (nloc - RD + d >= 0) request(nloc - RD + d, wr[d], ar[d]);
+    } else {
+#pragma unroll
+        for (int d = 0; d < RD; ++d) request(d, wr[d], ar[d]);
+    }
 
     float4_t acc[MT][NS];
 #pragma unroll
@@ -954,22 +960,37 @@ __global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) vo
         if (more) request(i + RD, wr[CUR], ar[CUR]);
         __builtin_amdgcn_sched_barrier(0);  // one chunk's operands in the registers at a time
     };
-    {
+    // A load that brings nothing (past a wave's last chunk) takes its turn in the address unit as any other: none but at the loop's
+    // start.  us, the last round of chunks in the loop -> behind it: 6144 x 4096 at 1 / 6 / 16 rows Q4_K 5.9 / 6.7 / 11.4 -> 5.3 / 5.8 / 7.6, Q6_K
+    // 8.1 / 8.5 / 15.0 -> 6.8 / 7.1 / 9.2, 3072 x 8192 at 6 / 24 Q4_K 6.6 / 15.2 -> 5.8 / 12.3, Q8_0 9.1 / 16.5 -> 7.2 / 13.3; four strips, 2048 x 16384
+    // at 1 / 32 Q4_K 8.2 / 13.1 -> 7.4 / 11.5, 4096 x 14336 at 1 / 32 11.2 / 19.1 -> 10.7 / 18.3.
+    const std::integral_constant<int, 0> c0;
+    const std::integral_constant<int, 1> c1;
+    const std::integral_constant<int, 2> c2;
+    if constexpr (NL > 0) {
+        static_assert(NL <= 2, "two chunks at most");
+        if constexpr (NL == 2) {
+            if (nloc > 1) chunk(nloc - 2, c0, false);
+        }
+        if (nloc > 0) chunk(nloc - 1, std::integral_constant<int, NL - 1>{}, false);
+    } else {
         int i = 0;
         if constexpr (RD == 2) {
-            for (; i + 1 < nloc; i += 2) {
-                chunk(i, std::integral_constant<int, 0>{}, true);
-                chunk(i + 1, std::integral_constant<int, 1>{}, true);
+            for (; i + 2 < nloc; i += 2) {
+                chunk(i, c0, true);
+                chunk(i + 1, c1, true);
             }
-            if (i < nloc) chunk(i, std::integral_constant<int, 0>{}, false);
+            if (i < nloc) chunk(i, c0, false);
+            if (i + 1 < nloc) chunk(i + 1, c1, false);
         } else {
-            for (; i + 2 < nloc; i += 3) {
-                chunk(i, std::integral_constant<int, 0>{}, true);
-                chunk(i + 1, std::integral_constant<int, 1>{}, true);
-                chunk(i + 2, std::integral_constant<int, 2>{}, true);
+            for (; i + 3 < nloc; i += 3) {
+                chunk(i, c0, true);
+                chunk(i + 1, c1, true);
+                chunk(i + 2, c2, true);
             }
-            if (i < nloc) chunk(i, std::integral_constant<int, 0>{}, false);
-            if (i + 1 < nloc) chunk(i + 1, std::integral_constant<int, 1>{}, false);
+            if (i < nloc) chunk(i, c0, false);
+            if (i + 1 < nloc) chunk(i + 1, c1, false);
+            if (i + 2 < nloc) chunk(i + 2, c2, false);
         }
     }
     if constexpr (XF32) ggm_epilogue_f32<MT, NS, NW>(acc, (const float *)bias, (float *)y, M, N, j, m0, wave, lane);
@@ -979,6 +1000,20 @@ __global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) vo
             return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) == 0x7F800000u ? ggm_narrow_dot<FMT>(pw, x + (size_t)m * K, n, K) : v;
         });
     else pk4n_epilogue<TT, MT, NS, NW, true>(acc, bias, y, ws, M, N, j, m0, wave, lane);
+}
+
+template <int FMT, int MT, int XQ, int NW, int NS, bool XF32 = false>
+__global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) void ggm_kernel(
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
+    float *__restrict__ ws, int M, int K, int N, int cslice, int act) {
+    ggm_body<FMT, MT, XQ, NW, NS, XF32, 0>(x, pw, bias, y, ws, M, K, N, cslice, act);
+}
+// The same for up to NL chunks a wave, without the loop's code to jump over: a kernel's instructions come from memory anew at each launch.
+template <int FMT, int MT, int XQ, int NW, int NS, bool XF32, int NL>
+__global__ __launch_bounds__(NW * 64, (ggm_waves<FMT, MT, XQ, NW, NS, XF32>)) void ggm_short_kernel(
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ pw, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
+    float *__restrict__ ws, int M, int K, int N, int cslice, int act) {
+    ggm_body<FMT, MT, XQ, NW, NS, XF32, NL>(x, pw, bias, y, ws, M, K, N, cslice, act);
 }
 
 // ---------------------------------------------------------------------------
@@ -1467,25 +1502,29 @@ int launch_gguf_mfma_dequant(oxq_ctx *ctx, hipStream_t s, int quant, const void 
     return OXQ_OK;
 }
 
-template <int FMT, int MT, int XQ, int NW, int NS>
-static int ggm_go(hipStream_t s, dim3 grid, const GgufProblem &p, float *ws, int cslice) {
+template <int FMT, int MT, int XQ, int NW, int NS, bool XF32, int NL>
+static int ggm_launch(hipStream_t s, dim3 grid, const GgufProblem &p, float *ws, int cslice) {
     static LdsGrant lds_grant;  // one per instantiation
+    constexpr auto kernel = [] {
+        if constexpr (NL > 0) return &ggm_short_kernel<FMT, MT, XQ, NW, NS, XF32, NL>;
+        else return &ggm_kernel<FMT, MT, XQ, NW, NS, XF32>;
+    }();
     const size_t lds = (size_t)NW * MT * 4096;
-    OXQ_HIP_CHECK(lds_grant.ensure((const void *)ggm_kernel<FMT, MT, XQ, NW, NS>, lds));
-    hipLaunchKernelGGL((ggm_kernel<FMT, MT, XQ, NW, NS>), grid, dim3(NW * 64), lds, s, (const uint16_t *)p.x, p.w,
-                       (const uint16_t *)p.bias, (uint16_t *)p.y, ws, (int)p.M, (int)p.K, (int)p.N, cslice, p.act);
+    OXQ_HIP_CHECK(lds_grant.ensure((const void *)kernel, lds));
+    hipLaunchKernelGGL(kernel, grid, dim3(NW * 64), lds, s, (const uint16_t *)p.x, p.w, (const uint16_t *)p.bias, (uint16_t *)p.y, ws,
+                       (int)p.M, (int)p.K, (int)p.N, cslice, p.act);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
+template <int FMT, int MT, int XQ, int NW, int NS, bool XF32 = false>
+static int ggm_go(hipStream_t s, dim3 grid, const GgufProblem &p, float *ws, int cslice) {
+    if (cslice <= NW) return ggm_launch<FMT, MT, XQ, NW, NS, XF32, 1>(s, grid, p, ws, cslice);
+    if (cslice <= 2 * NW) return ggm_launch<FMT, MT, XQ, NW, NS, XF32, 2>(s, grid, p, ws, cslice);
+    return ggm_launch<FMT, MT, XQ, NW, NS, XF32, 0>(s, grid, p, ws, cslice);
+}
 template <int FMT, int MT, int XQ, int NW, int NS>
 static int ggm_f32_go(hipStream_t s, dim3 grid, const GgufProblem &p, int cslice) {
-    static LdsGrant lds_grant;
-    const size_t lds = (size_t)NW * MT * 4096;
-    OXQ_HIP_CHECK(lds_grant.ensure((const void *)ggm_kernel<FMT, MT, XQ, NW, NS, true>, lds));
-    hipLaunchKernelGGL((ggm_kernel<FMT, MT, XQ, NW, NS, true>), grid, dim3(NW * 64), lds, s, (const uint16_t *)p.x, p.w,
-                       (const uint16_t *)p.bias, (uint16_t *)p.y, nullptr, (int)p.M, (int)p.K, (int)p.N, cslice, 0);
-    OXQ_HIP_CHECK(hipGetLastError());
-    return OXQ_OK;
+    return ggm_go<FMT, MT, XQ, NW, NS, true>(s, grid, p, nullptr, cslice);
 }
 template <int FMT>
 static int ggm_f32_by_shape(hipStream_t s, dim3 grid, const GgufProblem &p, int cslice, int mt, int ns) {
