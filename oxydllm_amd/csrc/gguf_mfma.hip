@@ -1433,21 +1433,28 @@ bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int ac
 bool gguf_mfma_alone(const oxq_ctx *ctx, int quant, int act_dtype) {
     return !ggm_narrow_format(quant) && (act_dtype == OXQ_BF16 || tune(ctx, OXQ_TUNE_GGUF_MFMA, 1) == 2);
 }
-// f32 rows of a layer that has both copies: the vector GEMV's arithmetic grows with the rows and is slow on many short
-// strips; the matrix cores take four rows as one.  us on the rotated / the matrix-core copy, Q4_K, 1 / 2 / 4 / 8 rows:
-// 4096 x 4096 4.2 / 5.0 / 6.5 / 12.7 against 4.5 / 5.2 / 5.5 / 7.8, 14336 x 4096 10.7 / 13.3 / 17.8 / 35.2 against 10.0 / 11.7 /
-// 11.7 / 19.2, 2048 x 8192 6.5 / 8.0 / 10.9 / 21.2 against 4.7 / 5.1 / 5.3 / 7.2 (Q6_K: 7.1 / 8.7 against 7.2 / 7.3).
-bool gguf_f32_on_mfma(const oxq_ctx *ctx, int64_t M, int64_t K, int64_t N) {
-    const bool many = ceil_div(N, (int64_t)16) > (ctx->num_cus > 0 ? ctx->num_cus : 256);
-    return M >= 3 || (M == 2 ? many || K >= 8192 : many && K <= 2048);
+// f32 rows of a layer that has both copies: the vector GEMV's arithmetic grows with the rows, and it is slow on many short strips, on
+// a K that leaves its sixteen waves little or three chunks each, of which it works off four; the matrix cores take four rows as
+// one.  us on the rotated / the matrix-core copy, Q4_K, 1 / 2 / 4 / 8 rows: 4096 x 4096 4.5 / 5.2 / 6.5 / 12.7 against 4.7 / 5.6 / 5.9 / 8.7,
+// 14336 x 4096 11.5 / 14.1 / 17.8 / 35.2 against 11.0 / 13.7 / 15.1 / 22.0.  1 / 2 rows: 1024 x 4096 4.4 / 5.2 against 3.3 / 3.3 (Q6_K 4.5 / 5.5 against
+// 3.6 / 3.7), 1536 x 4096 4.4 / 5.2 against 3.5 / 3.7, 2048 x 4096 4.3 / 5.0 against 4.0 / 4.3 (Q6_K 4.4 / 5.2 against 4.5 / 4.8, Q4_1 4.0 / 4.8
+// against 4.5 / 4.5), 3072 x 8192 7.2 / 8.9 against 5.9 / 7.0, 4096 x 8192 7.6 / 9.3 against 7.3 / 8.7 (Q6_K 8.7 against 9.5), 6144 x 4096
+// 6.7 / 8.2 against 5.7 / 7.0 (Q6_K 7.9 / 8.8 against 7.1 / 8.4), 5120 x 4096 5.6 / 6.8 against 5.3 / 6.3 (Q4_1 5.3 / 6.3 against 5.8 / 6.3).
+bool gguf_f32_on_mfma(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N) {
+    if (M >= 3) return true;
+    const bool many = ceil_div(N, (int64_t)16) > (ctx->num_cus > 0 ? ctx->num_cus : 256), three = K > 4096 && K <= 6144;
+    const bool pairs = quant == OXQ_GGUF_Q4_1 || quant == OXQ_GGUF_Q5_1;
+    if (M == 2) return many || K <= 2048 || K >= 8192 || (three && !pairs);
+    return K < 2048 || (many && K <= 3072) || ((K == 2048 || three) && quant != OXQ_GGUF_Q6_K && !pairs) || (three && K > 5120);
 }
 // Rows of a layer that holds both copies: whether they run on the matrix-core one.  Q2_K and Q3_K, us on the rotated / the
 // matrix-core copy: 4096 x 4096 bf16 3 rows 6.7 / 5.2, 2 rows 5.0 / 5.2 (Q3_K 5.6 / 5.4), 1024 x 5056 2 rows 7.2 / 3.8, 14336 x 4096
-// 13.4 / 11.8; f32 3 rows 6.5 / 6.5, 18.2 / 15.9 at 14336 x 4096, 8 rows 12.8 / 9.6, 36 / 26, but 2 rows 12.6 / 15.9.
+// 14.3 / 12.5, 6144 x 4096 8.4 / 6.5, 2048 x 4096 5.1 / 4.1; f32 3 rows 6.5 / 6.5, 18.2 / 15.9 at 14336 x 4096, 8 rows 12.8 / 9.6, 36 / 26, but
+// 2 rows 12.6 / 15.9.
 bool gguf_rows_on_mfma(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype) {
     const bool many = ceil_div(N, (int64_t)16) > (ctx->num_cus > 0 ? ctx->num_cus : 256);
-    if (ggm_narrow_format(quant)) return act_dtype == OXQ_BF16 ? M >= 3 || (M == 2 && (many || quant == OXQ_GGUF_Q3_K)) : M >= 3 && M <= 8;
-    return act_dtype == OXQ_BF16 || gguf_f32_on_mfma(ctx, M, K, N);
+    if (ggm_narrow_format(quant)) return act_dtype == OXQ_BF16 ? M >= 3 || (M == 2 && (many || K <= 3072 || K > 4096 || quant == OXQ_GGUF_Q3_K)) : M >= 3 && M <= 8;
+    return act_dtype == OXQ_BF16 || gguf_f32_on_mfma(ctx, quant, M, K, N);
 }
 size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N) {
     if (quant == OXQ_GGUF_Q3_K) return (size_t)N * (size_t)(K / 256) * 114;  // its scales are a byte each

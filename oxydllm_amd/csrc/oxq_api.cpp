@@ -876,7 +876,7 @@ static bool wcache_forward_gguf(oxq_ctx *ctx, hipStream_t s, const GgufProblem &
     if (!ctx->wcache_limit || ctx->plan_only) return false;
     const bool rotated = gguf_res_eligible(p.quant, p.K, p.N);
     const bool mfma = p.quant != OXQ_GGUF_Q2_K && p.quant != OXQ_GGUF_Q3_K && gguf_mfma_layer(ctx, p.quant, p.K, p.N, p.act_dtype) &&
-                      (gguf_mfma_alone(ctx, p.quant, p.act_dtype) || !rotated || gguf_f32_on_mfma(ctx, p.M, p.K, p.N));
+                      (gguf_mfma_alone(ctx, p.quant, p.act_dtype) || !rotated || gguf_f32_on_mfma(ctx, p.quant, p.M, p.K, p.N));
     if (!mfma && !rotated) return false;
     const bool gemm = mfma && gguf_gemm_takes(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);  // prefill sizes, same copy
     const bool tiles = mfma && gguf_mfma_tiles(ctx, p.quant, p.M, p.K, p.N, p.act_dtype);

@@ -276,7 +276,7 @@ bool gguf_mfma_eligible(const oxq_ctx *ctx, int quant, int64_t K, int64_t N);
 bool gguf_mfma_layer(const oxq_ctx *ctx, int quant, int64_t K, int64_t N, int act_dtype);
 bool gguf_mfma_alone(const oxq_ctx *ctx, int quant, int act_dtype);
 size_t gguf_mfma_bytes(int quant, int64_t K, int64_t N);
-bool gguf_f32_on_mfma(const oxq_ctx *ctx, int64_t M, int64_t K, int64_t N);
+bool gguf_f32_on_mfma(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N);
 bool gguf_rows_on_mfma(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);
 bool gguf_mfma_tiles(const oxq_ctx *ctx, int quant, int64_t M, int64_t K, int64_t N, int act_dtype);
 bool gguf_mfma_takes(const oxq_ctx *ctx, int quant, int64_t M, int64_t N, int act_dtype);

@@ -189,3 +189,31 @@ def test_ffn_without_room_for_the_fused_activation(fmt, slices):
     want = down.forward(ops.gated_activation(plain.forward(x), ops.ACT_GATED_SILU))
     got = ops.FeedForward(ops.GATE_UP_FUSED, fused, None, down, inter).forward(x)
     np.testing.assert_array_equal(bits_of(got), bits_of(want))
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("N,K,rows", [(1024, 1024, (1, 2)), (592, 1792, (1, 2)), (512, 2048, (2,)), (256, 5376, (1,)), (4112, 3072, (1, 2))])
+def test_one_and_two_f32_rows_where_the_matrix_cores_take_them(fmt, N, K, rows):
+    """Beside the layer without the matrix-core copy: both within 4e-7 of 64 bits, and not further from it; the same infinities."""
+    data = to_dev(synth.gguf_weight(fmt, N, K, seed=N + K + fmt))
+    plain = ops.Context()
+    tune("OXQ_GGUF_MFMA", 0, plain)
+    layer, former = ops.QLinear(fmt, data, K, N, None, torch.float32), ops.QLinear(fmt, data, K, N, None, torch.float32, ctx=plain)
+    w = layer.dequantize().double()
+    try:
+        for m in rows:
+            err = []
+            for ly, ctx, name in ((layer, ops.default_context(), "_mfma_f32_mt1"), (former, plain, "_res_gemv_f32")):
+                x = torch.from_numpy(np.random.default_rng(K + m).standard_normal((m, K)).astype(np.float32)).cuda()
+                say(f"gguf f32 {synth.GGUF_NAMES[fmt]} N={N} K={K} m={m} {name}")
+                y = ly.forward(x)
+                assert name in ctx.last_plan()["kernel"], ctx.last_plan()
+                ref = x.double() @ w.T
+                err.append(((y.double() - ref).norm() / ref.norm()).item())
+            assert err[0] < 4e-7 and err[0] <= 1.1 * err[1], (m, err)  # (a draw of a few hundred outputs scatters by a few per cent)
+            x = torch.from_numpy(np.random.default_rng(m).standard_normal((m, K)).astype(np.float32)).cuda()
+            x[0, 77], x[m - 1, K - 3] = float("inf"), -float("inf") if m == 2 else 1.0
+            got, want = layer.forward(x), former.forward(x)
+            assert torch.equal(torch.nan_to_num(got, 0.0, 1.0, -1.0), torch.nan_to_num(want, 0.0, 1.0, -1.0)), "infinities"
+    finally:
+        plain.close()
