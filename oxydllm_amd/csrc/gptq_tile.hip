@@ -52,7 +52,9 @@ template <int BITS> struct GptqDeq<BF16Traits, BITS> {
     }
 };
 
-template <typename TT, int BITS, int MT, int PER, int D, bool FOLD>
+// PER: blocks of a wave, as straight-line code; 0: a loop of two; -1: the same with a last one behind it, which costs registers (4-bit f16 of one
+// row tile 161 for 126, and a workgroup of two a CU), for odd numbers.  WHOLE: of all eight waves of every slice.
+template <typename TT, int BITS, int MT, int PER, int D, bool FOLD, bool WHOLE>
 __global__ __launch_bounds__(512) void gptq_tile_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ qw,
                                                         const uint32_t *__restrict__ qz,
                                                         const uint16_t *__restrict__ sc,
@@ -66,8 +68,9 @@ __global__ __launch_bounds__(512) void gptq_tile_kernel(const uint16_t *__restri
     // One row tile in straight-line code: the wave's whole share of x is put into LDS before the first block
     // (2 PER stages a wave), requested ahead of the weights.  Otherwise x travels by half blocks through two
     // stages a wave, and every request for it queues behind the weights requested before it.
-    constexpr bool XFRONT = MT == 1 && PER > 0;
-    constexpr int NSTAGE = XFRONT ? 2 * PER : 2;
+    constexpr int LINE = PER > 0 ? PER : 0;
+    constexpr bool XFRONT = MT == 1 && LINE;
+    constexpr int NSTAGE = XFRONT ? 2 * LINE : 2;
     constexpr uint32_t OOB = 0x80000000u;
     constexpr int WAUX = MT <= 2 ? 2 : 0;  // up to 32 rows one workgroup reads a strip's weights, once: nontemporal
     extern __shared__ __attribute__((aligned(16))) unsigned char pk4_lds[];
@@ -81,9 +84,9 @@ __global__ __launch_bounds__(512) void gptq_tile_kernel(const uint16_t *__restri
     const int NBS = (NBT + (int)gridDim.z - 1) / (int)gridDim.z;
     const int s0 = blockIdx.z * NBS;
     const int NB = s0 + NBS < NBT ? NBS : NBT - s0;   // blocks of this slice
-    const int per = PER ? PER : (NB + 7) >> 3;  // PER: K / 128 = 8 PER, one slice (launcher)
+    const int per = LINE ? LINE : (NBS + 7) >> 3;  // (LINE: that number)
     const int b0 = s0 + wave * per;
-    const int b1 = b0 + per < s0 + NB ? b0 + per : s0 + NB;
+    const int b1 = WHOLE || b0 + per < s0 + NB ? b0 + per : s0 + NB;
     unsigned char *slot = pk4_lds + wave * NSTAGE * STAGE;
 
     const int wrow = N * 4;  // bytes a word row
@@ -261,7 +264,9 @@ __global__ __launch_bounds__(512) void gptq_tile_kernel(const uint16_t *__restri
 
     // D register sets of weights in a ring, D - 1 blocks requested ahead.
     WB w[D];
-    if (XFRONT) {
+    if (LINE && !WHOLE && b0 >= b1) {
+        // no block for this wave
+    } else if (XFRONT) {
         // x of the whole share first (the vector-memory counter runs in issue order: what is needed first is
         // requested first), then the weights; x is in LDS by the time the first block's weights arrive
         u32x4_t xa[NSTAGE][XL];
@@ -269,10 +274,11 @@ __global__ __launch_bounds__(512) void gptq_tile_kernel(const uint16_t *__restri
         for (int st = 0; st < NSTAGE; ++st)
 #pragma unroll
             for (int i = 0; i < XL; ++i)
-                xa[st][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_x, (int)(xo0 + (uint32_t)i * xstep), (b0 * 2 + st) * 128, 0);
+                xa[st][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_x, (int)(xo0 + (uint32_t)i * xstep + (WHOLE || b0 + st / 2 < b1 ? 0u : OOB)),
+                                                                 (b0 * 2 + st) * 128, 0);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < D - 1 && i < PER; ++i) load_w(b0 + i, w[i]);
+        for (int i = 0; i < D - 1 && i < LINE; ++i) load_w(b0 + i, w[i]);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int st = 0; st < NSTAGE; ++st) {
@@ -281,26 +287,34 @@ __global__ __launch_bounds__(512) void gptq_tile_kernel(const uint16_t *__restri
             stage_x(st);
         }
 #pragma unroll
-        for (int i = 0; i < PER; ++i) block_xfront(i, w[i % D], b0 + i + D - 1, w[(i + D - 1) % D], i + D - 1 < PER);
-    } else if (PER) {
-        // K = 8 PER blocks: straight-line code, every wave PER blocks; D = PER requests a wave's whole share
-        // before it waits for any of it
+        for (int i = 0; i < LINE; ++i) block_xfront(i, w[i % D], b0 + i + D - 1, w[(i + D - 1) % D], i + D - 1 < LINE);
+    } else if (LINE) {
+        // straight-line code; D = PER requests a wave's whole share before it waits for any of it
         load_x(b0, 0);
 #pragma unroll
-        for (int i = 0; i < D - 1 && i < PER; ++i) load_w(b0 + i, w[i]);
+        for (int i = 0; i < D - 1 && i < LINE; ++i) load_w(b0 + i, w[i]);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < PER; ++i) block(b0 + i, w[i % D], b0 + i + D - 1, w[(i + D - 1) % D], i + D - 1 < PER);
+        for (int i = 0; i < LINE; ++i) block(b0 + i, w[i % D], b0 + i + D - 1, w[(i + D - 1) % D], i + D - 1 < LINE);
     } else if (b0 < b1) {
         // any K: a loop whose body is D blocks, so that every set keeps its registers (a rotating ring would
-        // be copied at the loop's end, and a copy waits for the load behind it); blocks past the share
-        // are zeros
+        // be copied at the loop's end, and a copy waits for the load behind it)
         load_x(b0, 0);
 #pragma unroll
         for (int i = 0; i < D - 1; ++i) load_w(b0 + i, w[i]);
-        for (int b = b0; b < b1; b += D) {
-#pragma unroll
-            for (int i = 0; i < D; ++i) block(b + i, w[i], b + i + D - 1, w[(i + D - 1) % D], true);
+        static_assert(LINE || D == 2, "the loops below");
+        if constexpr (PER < 0) {
+            int b = b0;
+            for (; b + 1 < b1; b += 2) {
+                block(b, w[0], b + 1, w[1 % D], true);
+                block(b + 1, w[1 % D], b + 2, w[0], true);
+            }
+            if (b < b1) block(b, w[0], b, w[1 % D], false);
+        } else {  // (a block past the share is zeros)
+            for (int b = b0; b < b1; b += 2) {
+                block(b, w[0], b + 1, w[1 % D], true);
+                block(b + 1, w[1 % D], b + 2, w[0], true);
+            }
         }
     }
     __syncthreads();  // the partial tiles go where other waves' x stages were
@@ -319,39 +333,61 @@ bool gptq_tile_ok(const Wna16Problem &p) {
     return true;
 }
 
-template <typename TT, int BITS, int MT, int PER, int D>
+template <typename TT, int BITS, int MT, int PER, int D, bool WHOLE = false>
 static int gptq_tile_go(hipStream_t s, dim3 grid, const Wna16Problem &p, float *ws) {
     constexpr bool FOLD = MT <= 2;
     // 8 partial tiles of 16 MT x 64 f32; the x stages are as large, or 2 PER stages of 2 KB a wave when x goes first
-    const size_t lds = MT == 1 && PER > 2 ? (size_t)8 * 2 * PER * 2048 : (size_t)8 * MT * 4096;
+    const size_t lds = MT == 1 && PER > 1 ? (size_t)8 * 2 * PER * 2048 : (size_t)8 * MT * 4096;
     static LdsGrant lds_grant;
-    OXQ_HIP_CHECK(lds_grant.ensure((const void *)gptq_tile_kernel<TT, BITS, MT, PER, D, FOLD>, lds));
-    hipLaunchKernelGGL((gptq_tile_kernel<TT, BITS, MT, PER, D, FOLD>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.qweight,
+    OXQ_HIP_CHECK(lds_grant.ensure((const void *)gptq_tile_kernel<TT, BITS, MT, PER, D, FOLD, WHOLE>, lds));
+    hipLaunchKernelGGL((gptq_tile_kernel<TT, BITS, MT, PER, D, FOLD, WHOLE>), grid, dim3(512), lds, s, (const uint16_t *)p.x, p.qweight,
                        p.qzeros, (const uint16_t *)p.scales, (const uint16_t *)p.bias, (uint16_t *)p.y, ws, (int)p.M,
                        (int)p.K, (int)p.N, p.group_shift);
     OXQ_HIP_CHECK(hipGetLastError());
     return OXQ_OK;
 }
 
-// Weight ring: as deep as the registers beside the accumulators and the x half block allow.  K = 4096 and
-// 5120 (4 or 5 blocks a wave) run as straight-line code.
+// Weight ring: as deep as the registers beside the accumulators and the x half block allow.  Up to five blocks a wave run as straight-
+// line code.  The loop, which takes two at a time and requested two more, had shares of one, two and three blocks too, and multiplied
+// zeros where they were odd.
 template <typename TT, int BITS, int MT>
-static int gptq_tile_per(hipStream_t s, dim3 grid, int per, const Wna16Problem &p, float *ws) {
+static int gptq_tile_per(hipStream_t s, dim3 grid, int per, bool whole, const Wna16Problem &p, float *ws) {
     constexpr bool f16 = TT::DTYPE == 1;
     constexpr int DMAX = BITS == 4 ? (MT == 1 ? 5 : MT == 2 ? 4 : 2) : (MT == 1 ? (f16 ? 4 : 3) : MT == 2 ? 3 : 2);
-    if (per == 4) return gptq_tile_go<TT, BITS, MT, 4, (DMAX < 4 ? DMAX : 4)>(s, grid, p, ws);
-    if (per == 5) return gptq_tile_go<TT, BITS, MT, 5, (DMAX < 5 ? DMAX : 5)>(s, grid, p, ws);
-    return gptq_tile_go<TT, BITS, MT, 0, 2>(s, grid, p, ws);
+    constexpr int D5 = f16 && BITS == 4 && MT == 2 ? 3 : DMAX < 5 ? DMAX : 5;  // (four: registers in scratch memory, 5120 x 13824 at 24 rows 17.6 us)
+    switch (per) {
+    case 1: return gptq_tile_go<TT, BITS, MT, 1, 1>(s, grid, p, ws);
+    case 2: return gptq_tile_go<TT, BITS, MT, 2, 2>(s, grid, p, ws);
+    case 3: return gptq_tile_go<TT, BITS, MT, 3, (DMAX < 3 ? DMAX : 3)>(s, grid, p, ws);
+    case 4: return gptq_tile_go<TT, BITS, MT, 4, (DMAX < 4 ? DMAX : 4), true>(s, grid, p, ws);
+    case 5:
+        return whole ? gptq_tile_go<TT, BITS, MT, 5, D5, true>(s, grid, p, ws)
+                     : gptq_tile_go<TT, BITS, MT, 5, D5>(s, grid, p, ws);
+    case -1: return gptq_tile_go<TT, BITS, MT, -1, 2>(s, grid, p, ws);
+    default: return gptq_tile_go<TT, BITS, MT, 0, 2>(s, grid, p, ws);
+    }
 }
 
 template <typename TT, int BITS>
-static int gptq_tile_mt(hipStream_t s, dim3 grid, int mt, const Wna16Problem &p, float *ws) {
-    const int64_t NB = p.K / 128;
-    const int per = grid.z == 1 && NB % 8 == 0 ? (int)(NB / 8) : 0;  // straight-line code: one slice of 32 or 40 blocks
+static int gptq_tile_mt(hipStream_t s, dim3 grid, int mt, const Wna16Problem &p, float *ws, int64_t cus) {
+    // Blocks of a wave, as the kernel deals them; 0, -1: the loops.  It has the registers and the LDS of fewer requests, so that several of up to
+    // two row tiles' workgroups share a CU, which is ahead from three blocks where there is more than one round of them; and four
+    // blocks of seven waves (28 of a slice) are no faster in a line.
+    // us, before (a loop in steps of two; 32 and 40 blocks in a line, whatever the rounds) -> now, 4-bit f16 unless said:
+    //   one block       4096 x 4096 (four slices) at 8 / 64 rows 8.2 / 13.7 -> 7.0 / 11.0, 8192 x 1024 7.6 / 12.3 -> 6.4 / 9.8, 8-bit 8.6 / 14.0 -> 7.3 / 10.5
+    //   two             2048 x 8192 at 8 / 24 5.8 / 7.4 -> 5.3 / 7.1, 2048 x 28672 at 4 10.6 (loop) / 9.0
+    //   three           11008 x 4096 (four slices) at 8 / 24 / 64 11.1 / 14.1 / 20.5 -> 10.1 / 12.8 / 18.4
+    //   five            4608 x 6144 at 8 / 24 / 64 9.9 / 12.8 / 17.0 -> 8.8 / 11.5 / 14.9
+    //   line / loop     4096 x 28672 at 4 / 24 17.7 / 16.7, 24.1 / 23.1, bf16 at 4 17.8 / 15.7, 5120 x 18944 at 4 / 24 19.8 / 17.2, 31.2 / 25.1, 3584 x 18944 at 8
+    //                   15.2 / 13.3; 14336 x 4096 (four slices) at 16 / 24 12.2 / 11.7, 15.2 / 14.6
+    const int64_t blocks = ceil_div(p.K / 128, (int64_t)grid.z), share = ceil_div(blocks, (int64_t)8);
+    const bool rounds = (int64_t)grid.x * grid.y * grid.z > cus;
+    const bool whole = blocks == 8 * share && blocks * (int64_t)grid.z == p.K / 128;
+    const int per = share <= 2 || (share <= 5 && (mt == 4 || !rounds) && (share != 4 || whole)) ? (int)share : share % 2 ? -1 : 0;
     switch (mt) {
-    case 1: return gptq_tile_per<TT, BITS, 1>(s, grid, per, p, ws);
-    case 2: return gptq_tile_per<TT, BITS, 2>(s, grid, per, p, ws);
-    default: return gptq_tile_per<TT, BITS, 4>(s, grid, per, p, ws);
+    case 1: return gptq_tile_per<TT, BITS, 1>(s, grid, per, whole, p, ws);
+    case 2: return gptq_tile_per<TT, BITS, 2>(s, grid, per, whole, p, ws);
+    default: return gptq_tile_per<TT, BITS, 4>(s, grid, per, whole, p, ws);
     }
 }
 
@@ -384,9 +420,10 @@ int launch_gptq_tile(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
                     ctx->workspace_bytes);
     float *ws = (float *)ctx->workspace;
     const bool f16 = p.dtype == OXQ_F16;
+    const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     int rc;
-    if (p.bits == 4) rc = f16 ? gptq_tile_mt<F16Traits, 4>(s, grid, mt, p, ws) : gptq_tile_mt<BF16Traits, 4>(s, grid, mt, p, ws);
-    else rc = f16 ? gptq_tile_mt<F16Traits, 8>(s, grid, mt, p, ws) : gptq_tile_mt<BF16Traits, 8>(s, grid, mt, p, ws);
+    if (p.bits == 4) rc = f16 ? gptq_tile_mt<F16Traits, 4>(s, grid, mt, p, ws, cus) : gptq_tile_mt<BF16Traits, 4>(s, grid, mt, p, ws, cus);
+    else rc = f16 ? gptq_tile_mt<F16Traits, 8>(s, grid, mt, p, ws, cus) : gptq_tile_mt<BF16Traits, 8>(s, grid, mt, p, ws, cus);
     if (rc != OXQ_OK || ks == 1) return rc;
     return launch_splitk_reduce(ctx, s, ws, p.bias, p.y, p.M, p.N, ks, p.dtype);
 }
