@@ -393,14 +393,28 @@ static int gptq_tile_mt(hipStream_t s, dim3 grid, int mt, const Wna16Problem &p,
 
 // K slices for a layer of few strips: as many as bring the launch to about one workgroup a CU, at least
 // 8 blocks (one a wave) each; their f32 partial tiles are added in slice order by a second launch.
+// From 24 blocks on, where three slices have one to two blocks a wave in place of three or four.  us, one slice / three, at 4 / 24 / 64 rows:
+// 3072 x 3072 f16 6.4 / 6.2, 9.2 / 7.5, 12.0 / 9.9, 8-bit bf16 10.2 / 7.3, 12.6 / 8.7, 15.5 / 10.7; 3840 x 2560 f16 at 2 / 24 / 64 7.4 / 7.0, 11.0 /
+// 8.7, 14.1 / 11.5.  Two slices (tiles of more than a third of the CUs) of 24 - 31 blocks are ahead but for 4-bit weights of up to 16 rows
+// (3072 x 3072 6.4 / 6.9, 8-bit 9.6 / 8.2); 23 blocks and fewer gain in 8 bits alone (2560 x 2560 at 24 rows 10.5 / 9.2, 4-bit
+// at 4 rows 6.2 / 6.9) and stay whole.  These slices are taken where the ctx workspace holds them.
 int gptq_tile_slices(const oxq_ctx *ctx, const Wna16Problem &p) {
     const int mt = p.M > 32 ? 4 : (int)((p.M + 15) / 16);
     const int64_t tiles = (p.N / 64) * ceil_div(p.M, 16 * mt), NB = p.K / 128;
     int ks = 1;
-    if (tiles <= 96 && NB >= 32) ks = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tiles, NB / 8));
-    else if (tiles <= 128 && NB >= 64) ks = 2;  // half a round of workgroups and a long K
+    if (tiles <= 96 && NB >= 24) {
+        ks = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tiles, NB / 8));
+        if (NB < 32 && ((ks < 3 && p.bits == 4 && mt == 1) || (uint64_t)ks * p.M * p.N * 4 > ctx->workspace_bytes)) ks = 1;
+    } else if (tiles <= 128 && NB >= 64) ks = 2;  // half a round of workgroups and a long K
     ks = tune(ctx, OXQ_TUNE_GPTQ_TILE_KS, ks);
     return (int)std::max<int64_t>(1, std::min<int64_t>(ks, NB));
+}
+
+// One row of a layer of few strips: launch_wna16_gemv has the figures.
+bool gptq_tile_one_row(const oxq_ctx *ctx, const Wna16Problem &p) {
+    if (p.M != 1 || p.K * p.N >= (1 << 24) || (p.bits == 8 && p.K > 2048 && p.K < 4096)) return false;
+    const int ks = gptq_tile_slices(ctx, p);
+    return ks == 1 || (uint64_t)ks * p.N * 4 <= ctx->workspace_bytes;
 }
 
 int launch_gptq_tile(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {

@@ -259,6 +259,7 @@ int launch_wna16_gemv(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p);
 bool awq4_mfma_ok(const Wna16Problem &p);
 bool gptq_tile_ok(const Wna16Problem &p);
 int launch_gptq_tile(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p);
+bool gptq_tile_one_row(const oxq_ctx *ctx, const Wna16Problem &p);
 int launch_wna16_mfma(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p);
 int launch_wna16_dequant(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p, void *out_kn);
 int launch_gguf_gemv(oxq_ctx *ctx, hipStream_t s, const GgufProblem &p);

@@ -930,13 +930,16 @@ int launch_wna16_gemv(oxq_ctx *ctx, hipStream_t s, const Wna16Problem &p) {
     // GPTQ words feed the matrix cores as they are stored (gptq_tile.hip): 64-column strips, K inside the
     // workgroup (layers of few strips: K slices and the slice-ordered sum), the same time for 1 - 16 rows where
     // the dot-product kernel's arithmetic grows with the rows.  Like that kernel it never rounds a dequantized
-    // weight at these row counts.  A single row of a layer of few strips stays with the dot-product kernel
-    // (4096 x 4096: 7.1 against 7.3 us; 8-bit also two rows: 8.4 against 9.0); from there on the tile kernel
-    // is ahead (14336 x 4096 at 2 / 8 rows: 10.5 / 10.7 against 11.2 / 21.0 us).
+    // weight at these row counts.  On layers of few strips it is ahead from two rows on (14336 x 4096 at 2 / 8 rows: 10.5 /
+    // 10.7 against 11.2 / 21.0 us; 8-bit: four: the kernel of two and three subtracts the zero point from each weight, so that
+    // an infinity of x comes out as one where this kernel, which like that of one row takes it off the sum, gives NaN).  One row is
+    // ahead on fewer than 2^24 weights, in 8 bits not between 17 and 31 blocks of K.  us, dot-product kernel / tile kernel: 1024 x 512
+    // 5.3 / 3.3, 2048 x 2048 6.7 / 4.9, 3072 x 3072 6.9 / 6.0, 3968 x 4096 7.6 / 7.1, 14336 x 1024 10.0 / 6.9; 8-bit 2048 x 2048 6.6 / 6.2,
+    // 8192 x 1024 10.3 / 6.6, 2304 x 5120 7.4 / 8.2, 3584 x 3072 7.2 / 7.8.  From 2^24 on it is level (14336 x 4096: 10.8 / 11.1).
     if (gptq_tile_ok(p) && !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0)) {
         const int v = tune(ctx, OXQ_TUNE_GPTQ_TILE, 1);
-        const bool wide = p.N >= 96 * 64;
-        if (v == 2 || (v == 1 && (wide || p.M >= (p.bits == 4 ? 2 : 4)))) return launch_gptq_tile(ctx, s, p);
+        const bool wide = p.N >= 96 * 64, enough = p.M >= (p.bits == 4 ? 2 : 4);
+        if (v == 2 || (v == 1 && (wide || enough || gptq_tile_one_row(ctx, p)))) return launch_gptq_tile(ctx, s, p);
     }
     if (gptq_fast_ok(p) && !tune(ctx, OXQ_TUNE_FORCE_GENERIC, 0)) {
         if (p.bits == 4)
